@@ -4,21 +4,15 @@
 //   kq  = MUL_MAT(K F16, q)            ggml_compute_forward_mul_mat with vec_dot_type F16: q is converted to F16, f32 accumulate
 //   p   = SOFT_MAX_EXT(kq, mask, scale) ggml_compute_forward_soft_max_f32 (ggml.c:13783): max, expf, sum, scale by 1/sum
 //   kqv = MUL_MAT(V^T F16, p)          p converted to F16, f32 accumulate
-// with the SAME rounding points (q and p rounded to F16, K / V F16, f32 accumulation) - only the f32 summation order
-// differs. The per-token kernel (attn_decode_kernel) needs O(n_tokens^2) scalar work: 9.2 ms per layer for a 2048-token
+// with q and p rounded to F16, K / V F16, f32 accumulation. The per-token kernel (attn_decode_kernel) needs O(n_tokens^2) scalar work: 9.2 ms per layer for a 2048-token
 // prompt on the 70B shape, more than all GEMMs of the layer together.
 //
-// Design. One workgroup = 128 consecutive query tokens of one head, 4 waves x 32 queries. Everything is computed
-// TRANSPOSED so that a query is a COLUMN of the MFMA result: S^T = K Q^T (keys x queries) and O^T = V^T P^T. In the
-// 32x32 accumulator layout a lane then holds 16 keys of ONE query (column = lane & 31), so the softmax row statistics are
-// in-lane reductions plus one exchange with the partner lane (lane ^ 32), and P^T comes out of the accumulator in exactly
-// the order the next MFMA wants its B operand (again with one partner exchange) - no LDS round trip, no LDS at all.
-// K rows ([key][dh] F16) and V^T rows ([dh][key] F16, the reference's transposed V cache) are both "k-contiguous" MFMA A
-// operands and are read straight from global memory (the 4 waves of a workgroup and the 8 query heads of a KV group share
-// them through L1 / L2). Two passes over the keys, because p must be rounded to F16 AFTER the division by the full row
-// sum, exactly like the reference: pass 1 = row max and sum (online), pass 2 = recompute S, p = exp(s - max) / sum -> F16,
-// accumulate O. FLOPs: 3 x (n_q x n_kv x dh x 2) / 2 per head.
+// Design. Everything is computed TRANSPOSED so that a query is a COLUMN of the MFMA result: S^T = K Q^T (keys x queries) and O^T = V^T P^T. In the 32x32 accumulator layout a lane
+// then holds 16 keys of ONE query (column = lane & 31): the softmax statistics are in-lane reductions plus one exchange with the partner lane (lane ^ 32), and P^T never leaves the
+// registers. attn_prompt_kernel serves the transposed V cache of the default graphs, attn_rowmajor_kernel the row-major one of the flash-attention graphs.
 #include "pm355_device.h"
+#include "pm355_dense.h"
+#include "pm355_kernels.h"
 #include "pm355_layer_ops.h"
 
 namespace {
@@ -33,24 +27,17 @@ struct PfP {
     // ggml-graph mode (mask != nullptr; pm355_attn_prefill_masked): every query attends cells [0, n_kv) with the additive F32 KQ_mask
     // row of its token (0 / -inf; llama_set_inputs src/llama.cpp:17379-17420) instead of the causal rule "cell <= position"
     const float * mask; long mask_stride; int n_kv;
-    // flash-attention graphs (FLASH_ATTN_EXT, llm_build_kqv src/llama.cpp:10075-10095): v_rowmajor = the V cache is [n_ctx][Hkv*DH] like K
-    // (the V^T operand is then gathered with 2-byte loads: a lane needs 8 consecutive keys of ONE channel); mask_f16 = the mask rows are
-    // F16. P is rounded to F16 here as well (it is an MFMA operand; the reference keeps it f32 and rounds its F16 accumulator instead).
-    int v_rowmajor, mask_f16;
+    int mask_f16;                                // the mask rows are F16
     _Float16 * out_h;                            // optional: the result as F16 [T][H*DH] (activations of the wo GEMM) instead of `out`
 };
 
-// key index (inside a 32-key tile) of accumulator register r in lane-half h: C[row = (r&3) + 8 (r>>2) + 4 h][col]
-__device__ __forceinline__ int acc_row(int r, int h) { return (r & 3) + 8 * (r >> 2) + 4 * h; }
-
-// K and V tiles (32 keys) travel global -> registers -> LDS once per WORKGROUP and are double-buffered: the loads of tile j+1 are in
-// flight while the four waves multiply tile j out of LDS (round 2; before, every wave loaded its own copy straight into MFMA operands,
-// 213 + 80 registers = one wave per SIMD and nothing to hide the L2 latency behind: 8.3 us per key tile, 1.14 ms per layer for a
-// 2048-token prompt of the 70B shape). Row strides are padded so that the fragment reads (lane = key / channel, 16 bytes) are
-// conflict-free: K rows DH + 8 halves (68 dwords: lane i -> bank 4 i), V^T rows 40 halves (20 dwords: 16 lanes cover the 64 banks once).
-// A row-major V cache (flash-attention graphs) is transposed on its way into LDS.
+// Flash-attention graphs (FLASH_ATTN_EXT, llm_build_kqv src/llama.cpp:10075-10095): V cache [n_ctx][Hkv*DH] like K, always masked. One workgroup = 128 queries of one head, 4 waves x
+// 32. K and V tiles (32 keys) travel global -> registers -> LDS once per workgroup, double-buffered; V is transposed on its way. Row strides are padded so that the fragment reads
+// (lane = key / channel, 16 bytes) are conflict-free: K rows DH + 8 halves (68 dwords: lane i -> bank 4 i), V^T rows 40 halves (20 dwords: 16 lanes cover the 64 banks once). Two
+// passes over the keys, because p is rounded to F16 after the division by the full row sum: pass 1 = row max and sum (online), pass 2 = recompute S, p = exp(s - max) / sum -> F16,
+// accumulate O. P is rounded to F16 here as well (it is an MFMA operand; the reference keeps it f32 and rounds its F16 accumulator instead).
 template <int DH>
-__global__ __launch_bounds__(256, 2) void attn_prefill_kernel(PfP p) {
+__global__ __launch_bounds__(256, 2) void attn_rowmajor_kernel(PfP p) {
     constexpr int KK = DH / 16;                  // k-steps of the S^T MFMAs
     constexpr int DT = DH / 32;                  // 32-row tiles of O^T
     constexpr int KS = DH + 8, VS = 40;          // LDS row strides (halves)
@@ -61,24 +48,15 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(PfP p) {
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int col = lane & 31, hf = lane >> 5;
     const int h = blockIdx.y, hk = h / (p.H / p.Hkv);
-    const int seq = p.seq_ptr ? *p.seq_ptr : 0;
-    const int pos0 = p.mask ? 0 : p.pos0_ptr[seq];
     const long krow = (long) p.Hkv * DH;
-    const uint16_t * kc = p.kc + (long) seq * p.seq_stride + (long) hk * DH;          // K[key][Hkv*DH]
-    const uint16_t * vc = p.vc + (long) seq * p.seq_stride + (p.v_rowmajor ? (long) hk * DH : (long) hk * DH * p.n_ctx); // V^T[hk*DH + e][n_ctx] / V[key][Hkv*DH]
-    // causal mode: the LAST query blocks attend the most keys - they are dispatched first (longest-processing-time order) so that the
-    // short ones fill the tail
-    const int qb = p.mask ? (int) blockIdx.x : (int) (gridDim.x - 1 - blockIdx.x);
+    const uint16_t * kc = p.kc + (long) hk * DH, * vc = p.vc + (long) hk * DH;         // K, V [key][Hkv*DH]
+    const int qb = (int) blockIdx.x;
     const int tq0 = qb * 128 + wave * 32;                                              // first query token of this wave
     const bool wave_live = tq0 < p.T;
     const int tq = min(tq0 + col, p.T - 1);                                            // this lane's query (clamped)
-    const int qpos = pos0 + tq;                                                        // attends keys 0 .. qpos
-    const int last = pos0 + min(tq0 + 31, p.T - 1);                                    // wave-uniform causal limit
-    const int n_tiles = !wave_live ? 0 : (p.mask ? (p.n_kv + 31) / 32 : last / 32 + 1);
-    // the workgroup walks the tiles its LAST live wave needs (every wave takes part in the staging and the barriers)
-    const int n_wg = p.mask ? (p.n_kv + 31) / 32 : (pos0 + min(qb * 128 + 127, p.T - 1)) / 32 + 1;
-    const float * mrow = (p.mask && !p.mask_f16) ? p.mask + (long) tq * p.mask_stride : nullptr;
-    const uint16_t * mrow16 = (p.mask && p.mask_f16) ? (const uint16_t *) p.mask + (long) tq * p.mask_stride : nullptr;
+    const int n_wg = (p.n_kv + 31) / 32, n_tiles = wave_live ? n_wg : 0;                // (every wave takes part in the staging and the barriers)
+    const float * mrow = !p.mask_f16 ? p.mask + (long) tq * p.mask_stride : nullptr;
+    const uint16_t * mrow16 = p.mask_f16 ? (const uint16_t *) p.mask + (long) tq * p.mask_stride : nullptr;
 
     // ---- staging: global -> registers (fetch) -> LDS (put)
     u32x4 kg[NU], vg[NU];
@@ -92,9 +70,8 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(PfP p) {
     auto fetch_v = [&](int j) __attribute__((always_inline)) {
 #pragma unroll
         for (int i = 0; i < NU; ++i) {
-            const int u = tid + 256 * i;
-            if (!p.v_rowmajor) { const int row = u >> 2, unit = u & 3; vg[i] = *(const u32x4 *) (vc + (long) row * p.n_ctx + j * 32 + 8 * unit); }
-            else { const int key = min(j * 32 + u / UPR, p.n_ctx - 1), piece = u % UPR; vg[i] = *(const u32x4 *) (vc + (long) key * krow + 8 * piece); }
+            const int u = tid + 256 * i, key = min(j * 32 + u / UPR, p.n_ctx - 1), piece = u % UPR;
+            vg[i] = *(const u32x4 *) (vc + (long) key * krow + 8 * piece);
         }
     };
     auto put_k = [&](int b) __attribute__((always_inline)) {
@@ -104,14 +81,10 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(PfP p) {
     auto put_v = [&](int b) __attribute__((always_inline)) {
 #pragma unroll
         for (int i = 0; i < NU; ++i) {
-            const int u = tid + 256 * i;
-            if (!p.v_rowmajor) *(u32x4 *) (vs[b] + (u >> 2) * VS + 8 * (u & 3)) = vg[i];
-            else {                                                       // V[key][8 piece .. +8] -> V^T rows 8 piece .. +8, column key
-                const int key = u / UPR, piece = u % UPR;
-                uint16_t * d = (uint16_t *) vs[b] + (8 * piece) * VS + key;
+            const int u = tid + 256 * i, key = u / UPR, piece = u % UPR;      // V[key][8 piece .. +8] -> V^T rows 8 piece .. +8, column key
+            uint16_t * d = (uint16_t *) vs[b] + (8 * piece) * VS + key;
 #pragma unroll
-                for (int e = 0; e < 4; ++e) { d[(2 * e) * VS] = (uint16_t) (vg[i][e] & 0xFFFF); d[(2 * e + 1) * VS] = (uint16_t) (vg[i][e] >> 16); }
-            }
+            for (int e = 0; e < 4; ++e) { d[(2 * e) * VS] = (uint16_t) (vg[i][e] & 0xFFFF); d[(2 * e + 1) * VS] = (uint16_t) (vg[i][e] >> 16); }
         }
     };
 
@@ -133,9 +106,8 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(PfP p) {
         const _Float16 * kr = ks[b] + col * KS + 8 * hf;
 #pragma unroll
         for (int kk = 0; kk < KK; ++kk) acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(*(const half8 *) (kr + 16 * kk), qf[kk], acc, 0, 0, 0);
-        if (mrow || mrow16) {
 #pragma unroll
-            for (int g = 0; g < 4; ++g) {                            // registers 4g .. 4g+3 = keys j*32 + 8g + 4hf .. +4: one float4 of the mask row
+        for (int g = 0; g < 4; ++g) {                            // registers 4g .. 4g+3 = keys j*32 + 8g + 4hf .. +4: one float4 of the mask row
                 const int k0 = j * 32 + 8 * g + 4 * hf;
                 float4 mv = float4{-INFINITY, -INFINITY, -INFINITY, -INFINITY};
                 if (k0 + 3 < p.n_kv) {
@@ -145,13 +117,6 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(PfP p) {
                 s[4 * g + 0] = acc[4 * g + 0] * p.scale + mv.x; s[4 * g + 1] = acc[4 * g + 1] * p.scale + mv.y;
                 s[4 * g + 2] = acc[4 * g + 2] * p.scale + mv.z; s[4 * g + 3] = acc[4 * g + 3] * p.scale + mv.w;
             }
-            return;
-        }
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-            const int k = j * 32 + acc_row(r, hf);
-            s[r] = k <= qpos ? acc[r] * p.scale : -INFINITY;        // soft_max_ext: x * scale (+ causal mask = -inf)
-        }
     };
 
     // ---- pass 1: row max and sum of exp (online within the lane, merged with the partner lane at the end)
@@ -236,22 +201,218 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(PfP p) {
     }
     // ---- O^T[dh = 32 d + acc_row(r, hf)][query = col] -> out[t][h*DH + dh]
     if (wave_live && tq0 + col < p.T) {
-        if (p.out_h) {
-            _Float16 * orow = p.out_h + ((long) tq * p.H + h) * DH;
-#pragma unroll
-            for (int d = 0; d < DT; ++d)
-#pragma unroll
-                for (int g = 0; g < 4; ++g)
-                    *(half4 *) (orow + 32 * d + 8 * g + 4 * hf) = half4{(_Float16) o[d][4 * g], (_Float16) o[d][4 * g + 1], (_Float16) o[d][4 * g + 2], (_Float16) o[d][4 * g + 3]};
-        } else {
         float * orow = p.out + ((long) tq * p.H + h) * DH;
 #pragma unroll
         for (int d = 0; d < DT; ++d)
 #pragma unroll
             for (int g = 0; g < 4; ++g)
                 *(float4 *) (orow + 32 * d + 8 * g + 4 * hf) = float4{o[d][4 * g], o[d][4 * g + 1], o[d][4 * g + 2], o[d][4 * g + 3]};
+    }
+}
+
+// ---- the default graphs' layout: V transposed ---------------------------------------------------------------------------------------------------------------------------------
+// One workgroup = QW * 32 consecutive queries of one head; QW query waves x KW = 8 / QW key groups. Per stage KS keys of K ([KS][DH]) and V^T ([DH][KS]) travel by LDS-DMA
+// (double-buffered, 16-byte chunks XOR-swizzled on the source side so that the sixteen lanes a fragment read serves hit sixteen bank groups); key group kw multiplies keys
+// kw * KT .. + KT of every stage and keeps an online softmax of its own, the groups are merged through LDS at the end. Rows of a K tile are read with bits 2 and 3 of the row
+// index swapped: the accumulators of S^T then ARE the B operand of the P.V product.
+// ONE pass over the keys: the probabilities are rounded to F16 before the division by their sum (which adds the unrounded ones), where the reference rounds behind it - the same
+// relative error per probability (2^-12; smaller where p would be subnormal), without the second K.q product and the second exponential of every score: 2.0e-4 of the result from
+// float64 with two passes, 1.6e-4 with one.
+// Bound by the LDS reads of the fragments (32 queries per wave: 32 KiB per 64 keys and wave at ~80 bytes per cycle and CU, about the time of the 32 matrix instructions) and the
+// exponentials beside them. Against the two-pass form with 4 waves x 32 queries, 32-key tiles through registers: 6001 tokens x 32 heads 870 -> 393 us (752 TFLOP/s), 512 x 64 behind
+// 1024 cached cells 102 -> 38, 101 x 32 behind 300 29.8 -> 11.7, 2048 x 32 144 -> 55.
+template <int DH, int QW, int KS, bool MASK>
+__global__ __launch_bounds__(512, 2) void attn_prompt_kernel(PfP p) {
+    constexpr int KW = 8 / QW, KT = KS / KW, ST = KT / 32;            // keys per wave and stage, 32-key score tiles
+    constexpr int KK = DH / 16, DT = DH / 32, CK = DH / 8, CV = KS / 8;      // k-steps of a score tile, output tiles, 16-byte chunks per K row / V^T row
+    constexpr int STAGE = KS * DH * 4, OS = DH + 4;
+    constexpr float NONE = -1e30f, LOG2E = 1.4426950408889634f;
+    static_assert(KT % 32 == 0, "whole score tiles");
+    extern __shared__ __attribute__((aligned(1024))) char smem[];
+    const int wave = __builtin_amdgcn_readfirstlane((int) threadIdx.x >> 6), lane = threadIdx.x & 63, lr = lane & 31, hf = lane >> 5;
+    const int qw = wave % QW, kw = wave / QW;
+    // an XCD (blockIdx % 8) keeps to its share of the heads: the query heads of a KV head meet in one L2. Tiles with the most keys first: the short ones fill the tail
+    int h, tile;
+    const int n_tiles = (p.T + QW * 32 - 1) / (QW * 32);
+    if (p.H % 8 == 0) { const int per = p.H / 8, j = blockIdx.x >> 3; h = (blockIdx.x & 7) * per + j % per; tile = j / per; }
+    else { h = blockIdx.x % p.H; tile = blockIdx.x / p.H; }
+    tile = n_tiles - 1 - tile;
+    const int hk = h / (p.H / p.Hkv);
+    const int seq = p.seq_ptr ? *p.seq_ptr : 0;
+    const int pos0 = MASK ? 0 : p.pos0_ptr[seq];
+    const long krow = (long) p.Hkv * DH;
+    const uint16_t * kc = p.kc + (long) seq * p.seq_stride + (long) hk * DH;                     // K[key][Hkv*DH]
+    const uint16_t * vc = p.vc + (long) seq * p.seq_stride + (long) hk * DH * p.n_ctx;           // V^T[hk*DH + e][n_ctx]
+    const int tq0 = tile * QW * 32 + qw * 32;                                                    // first query of this wave
+    const bool live = tq0 < p.T;
+    const int tq = min(tq0 + lr, p.T - 1), qpos = pos0 + tq;
+    const int w_first = pos0 + tq0, w_last = pos0 + min(tq0 + 31, p.T - 1);                      // the wave's first and last query
+    const int n_keys = MASK ? p.n_kv : pos0 + min(tile * QW * 32 + QW * 32, p.T);                // cells the workgroup's last query sees
+    const int n_it = (n_keys + KS - 1) / KS;
+
+    const uint32_t lds0 = (uint32_t) (uintptr_t) (__attribute__((address_space(3))) char *) smem;
+    auto request = [&](int it, int stage) __attribute__((always_inline)) {
+        const char * kb = (const char *) (kc + (long) it * KS * krow), * vb = (const char *) vc;
+        const int key0 = it * KS, kmax = p.n_ctx - 1 - key0, vmax = p.n_ctx - 8 - key0;          // (cells behind the cache: its last ones, masked)
+#pragma unroll
+        for (int i = 0; i < KS * DH * 2 / 8192; ++i) {
+            const int o = (wave + i * 8) * 64 + lane, row = o / CK, ch = o % CK;
+            pm_dma16(kb, (uint32_t) min(row, kmax) * (uint32_t) (krow * 2) + (uint32_t) (ch ^ (CK == 8 ? (row >> 1) & 7 : row & 15)) * 16u, lds0 + stage * STAGE + (wave + i * 8) * 1024);
+        }
+#pragma unroll
+        for (int i = 0; i < KS * DH * 2 / 8192; ++i) {
+            const int o = (wave + i * 8) * 64 + lane, row = o / CV, ch = o % CV;
+            const int key = key0 + min((ch ^ (CV == 8 ? (row >> 1) & 7 : row & 15)) * 8, vmax);
+            pm_dma16(vb, (uint32_t) row * (uint32_t) (p.n_ctx * 2) + (uint32_t) key * 2u, lds0 + stage * STAGE + KS * DH * 2 + (wave + i * 8) * 1024);
+        }
+    };
+    request(0, 0);
+
+    // Q^T as B operand: lane (query lr, hf) holds q[query][16 kk + 8 hf .. + 8], rounded to F16 like the reference
+    half8 q[KK];
+    {
+        const float * qr = p.q + ((long) tq * p.H + h) * DH + 8 * hf;
+#pragma unroll
+        for (int kk = 0; kk < KK; ++kk) {
+            const float4 a = *(const float4 *) (qr + 16 * kk), b = *(const float4 *) (qr + 16 * kk + 4);
+            q[kk] = half8{(_Float16) a.x, (_Float16) a.y, (_Float16) a.z, (_Float16) a.w, (_Float16) b.x, (_Float16) b.y, (_Float16) b.z, (_Float16) b.w};
         }
     }
+    const float * mrow = (const float *) p.mask + (long) tq * p.mask_stride;
+    const uint16_t * mrow16 = (const uint16_t *) p.mask + (long) tq * p.mask_stride;
+    float16v o[DT];
+#pragma unroll
+    for (int d = 0; d < DT; ++d)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) o[d][r] = 0.0f;
+    float m = NONE, l = 0.0f;
+    const float c = p.scale * LOG2E;
+    const int kr = (lr & ~12) | ((lr & 4) << 1) | ((lr & 8) >> 1);
+    for (int it = 0; it < n_it; ++it) {
+        const int stage = it & 1;
+        pm_vm_drain();
+        __syncthreads();
+        if (it + 1 < n_it) request(it + 1, stage ^ 1);
+        const int key0 = it * KS + kw * KT;
+        if (!live || key0 >= (MASK ? p.n_kv : w_last + 1)) continue;
+        const char * ks = smem + stage * STAGE, * vs = ks + KS * DH * 2;
+        float16v s[ST];
+#pragma unroll
+        for (int t = 0; t < ST; ++t)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) s[t][r] = 0.0f;
+#pragma unroll
+        for (int kk = 0; kk < KK; ++kk)
+#pragma unroll
+            for (int t = 0; t < ST; ++t) {
+                const int row = kw * KT + t * 32 + kr;
+                const half8 k = *(const half8 *) (ks + row * (DH * 2) + ((kk * 2 + hf) ^ (CK == 8 ? (row >> 1) & 7 : row & 15)) * 16);
+                s[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(k, q[kk], s[t], 0, 0, 0);
+            }
+        float mx = NONE;
+        if (MASK) {
+#pragma unroll
+            for (int t = 0; t < ST; ++t)
+#pragma unroll
+                for (int g = 0; g < 4; ++g) {                     // registers 4 g .. + 4 = keys 16 (g >> 1) + 8 hf + 4 (g & 1) .. + 4
+                    const int k0 = key0 + t * 32 + 16 * (g >> 1) + 8 * hf + 4 * (g & 1);
+                    float4 mv = float4{-INFINITY, -INFINITY, -INFINITY, -INFINITY};
+                    if (k0 + 3 < p.n_kv) {
+                        if (!p.mask_f16) mv = *(const float4 *) (mrow + k0);
+                        else { const u32x2 mh = *(const u32x2 *) (mrow16 + k0); mv = float4{h2f((uint16_t) (mh[0] & 0xFFFF)), h2f((uint16_t) (mh[0] >> 16)), h2f((uint16_t) (mh[1] & 0xFFFF)), h2f((uint16_t) (mh[1] >> 16))}; }
+                    }
+                    s[t][4 * g + 0] = fmaf(mv.x, LOG2E, s[t][4 * g + 0] * c); s[t][4 * g + 1] = fmaf(mv.y, LOG2E, s[t][4 * g + 1] * c);
+                    s[t][4 * g + 2] = fmaf(mv.z, LOG2E, s[t][4 * g + 2] * c); s[t][4 * g + 3] = fmaf(mv.w, LOG2E, s[t][4 * g + 3] * c);
+                }
+        } else if (key0 + KT - 1 > w_first) {                     // (keys that some query of the wave does not see)
+#pragma unroll
+            for (int t = 0; t < ST; ++t)
+#pragma unroll
+                for (int r = 0; r < 16; ++r)
+                    if (key0 + t * 32 + 16 * (r >> 3) + 8 * hf + (r & 7) > qpos) s[t][r] = -INFINITY;
+        }
+#pragma unroll
+        for (int t = 0; t < ST; ++t)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) mx = fmaxf(mx, s[t][r]);
+        mx = fmaxf(mx, __shfl_xor(mx, 32));
+        if (!MASK) mx = fmaxf(mx * c, NONE);                      // (scores are scaled where the exponent is formed; scale > 0)
+        const float mn = fmaxf(m, mx);
+        if (__any(mn > m)) {
+            const float corr = __builtin_amdgcn_exp2f(m - mn);
+            l *= corr; m = mn;
+#pragma unroll
+            for (int d = 0; d < DT; ++d)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) o[d][r] *= corr;
+        }
+        half8 pr[2 * ST];
+#pragma unroll
+        for (int t = 0; t < ST; ++t)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const float e = __builtin_amdgcn_exp2f(MASK ? s[t][r] - m : fmaf(s[t][r], c, -m));
+                l += e;
+                pr[2 * t + (r >> 3)][r & 7] = (_Float16) e;
+            }
+#pragma unroll
+        for (int j = 0; j < 2 * ST; ++j)
+#pragma unroll
+            for (int d = 0; d < DT; ++d) {
+                const int row = d * 32 + lr, ch = kw * (KT / 8) + 2 * j + hf;
+                const half8 v = *(const half8 *) (vs + row * (KS * 2) + (ch ^ (CV == 8 ? (row >> 1) & 7 : row & 15)) * 16);
+                o[d] = __builtin_amdgcn_mfma_f32_32x32x16_f16(v, pr[j], o[d], 0, 0, 0);
+            }
+    }
+    l += __shfl_xor(l, 32);
+    __syncthreads();                                              // (the stages become the exchange of the results)
+    float * ex = (float *) smem, * ml = ex + 8 * 32 * OS;         // [wave][query][DH + 4], [wave][query]{m, l}
+    float f = 1.0f / l;
+    if (KW > 1) {
+        if (hf == 0) { ml[(wave * 32 + lr) * 2] = m; ml[(wave * 32 + lr) * 2 + 1] = l; }
+        __syncthreads();
+        float M = NONE, L = 0.0f;
+#pragma unroll
+        for (int g = 0; g < KW; ++g) M = fmaxf(M, ml[((g * QW + qw) * 32 + lr) * 2]);
+#pragma unroll
+        for (int g = 0; g < KW; ++g) L += ml[((g * QW + qw) * 32 + lr) * 2 + 1] * __builtin_amdgcn_exp2f(ml[((g * QW + qw) * 32 + lr) * 2] - M);
+        f = __builtin_amdgcn_exp2f(m - M) / L;
+    }
+    // O^T[d][query]: queries are columns; through LDS, then a wave stores whole rows
+#pragma unroll
+    for (int d = 0; d < DT; ++d)
+#pragma unroll
+        for (int g = 0; g < 4; ++g)
+            *(float4 *) (ex + (wave * 32 + lr) * OS + d * 32 + 8 * g + 4 * hf) = float4{o[d][4 * g] * f, o[d][4 * g + 1] * f, o[d][4 * g + 2] * f, o[d][4 * g + 3] * f};
+    __syncthreads();
+    constexpr int RL = DH / 4, RP = 64 / RL;                       // lanes per row (4 values each), rows per pass
+    for (int r = kw * (32 / KW) + lane / RL; r < (kw + 1) * (32 / KW); r += RP) {
+        if (tq0 + r >= p.T) break;
+        float4 a = *(const float4 *) (ex + (qw * 32 + r) * OS + 4 * (lane % RL));
+#pragma unroll
+        for (int g = 1; g < KW; ++g) {
+            const float4 b = *(const float4 *) (ex + ((g * QW + qw) * 32 + r) * OS + 4 * (lane % RL));
+            a.x += b.x; a.y += b.y; a.z += b.z; a.w += b.w;
+        }
+        const long at = ((long) (tq0 + r) * p.H + h) * DH + 4 * (lane % RL);
+        if (p.out_h) *(half4 *) (p.out_h + at) = half4{(_Float16) a.x, (_Float16) a.y, (_Float16) a.z, (_Float16) a.w};
+        else *(float4 *) (p.out + at) = a;
+    }
+}
+
+template <int DH, int QW, int KS, bool MASK> void launch_prompt(const PfP & p, hipStream_t st) {
+    constexpr size_t stages = 2 * (size_t) KS * DH * 4, ex = (size_t) 8 * 32 * (DH + 4) * 4 + 8 * 32 * 2 * 4, lds = stages > ex ? stages : ex;
+    pm_allow_big_lds((const void *) attn_prompt_kernel<DH, QW, KS, MASK>, lds);
+    hipLaunchKernelGGL((attn_prompt_kernel<DH, QW, KS, MASK>), dim3((p.T + QW * 32 - 1) / (QW * 32) * p.H), dim3(512), lds, st, p);
+}
+// Which tile: a CU holds one workgroup. 256 queries share a stage where that still makes two rounds of workgroups (2048 tokens x 64 heads: 102 us, 110 with 128 queries; x 32 heads
+// = one round whose longest tile decides: 80 against 57); 128 queries where they make one (512 x 64 behind 1024 cached: 38 against 50 with 64); below that 64 queries with four key
+// groups each (101 x 32 behind 300: 11.7 against 14.9).
+template <int DH, bool MASK> void launch_prompt_dh(const PfP & p, hipStream_t st) {
+    const int cus = pm_device_cus();
+    if ((p.T + 255) / 256 * p.H >= 2 * cus) launch_prompt<DH, 8, 64, MASK>(p, st);
+    else if ((p.T + 127) / 128 * p.H >= cus) launch_prompt<DH, 4, 128, MASK>(p, st);
+    else launch_prompt<DH, 2, 128, MASK>(p, st);
 }
 
 } // namespace
@@ -263,10 +424,16 @@ int pm_launch_attn_prefill(const float * q, const void * kc, const void * vc, co
     if ((dh != 64 && dh != 128) || n_ctx % 32 || n_tok < 1) return -1;
     if (mask && (n_kv < 1 || n_kv > n_ctx || n_kv % 4 || mask_stride % 4)) return -1;
     if ((v_rowmajor || mask_f16) && !mask) return -1;                 // the flash-attention form exists in ggml-graph mode only
-    PfP p = {q, (const uint16_t *) kc, (const uint16_t *) vc, pos0, seq, seq_stride, out, n_tok, H, Hkv, n_ctx, scale, mask, mask_stride, n_kv,
-             v_rowmajor ? 1 : 0, mask_f16 ? 1 : 0, (_Float16 *) out_f16};
-    const dim3 grid((n_tok + 127) / 128, H);
-    if (dh == 128) hipLaunchKernelGGL(attn_prefill_kernel<128>, grid, dim3(256), 0, st, p);
-    else           hipLaunchKernelGGL(attn_prefill_kernel<64>, grid, dim3(256), 0, st, p);
+    PfP p = {q, (const uint16_t *) kc, (const uint16_t *) vc, pos0, seq, seq_stride, out, n_tok, H, Hkv, n_ctx, scale, mask, mask_stride, n_kv, mask_f16 ? 1 : 0, (_Float16 *) out_f16};
+    if (v_rowmajor) {
+        if (out_f16 || seq) return -1;
+        const dim3 grid((n_tok + 127) / 128, H);
+        if (dh == 128) hipLaunchKernelGGL(attn_rowmajor_kernel<128>, grid, dim3(256), 0, st, p);
+        else           hipLaunchKernelGGL(attn_rowmajor_kernel<64>, grid, dim3(256), 0, st, p);
+    } else if (dh == 128) {
+        if (mask) launch_prompt_dh<128, true>(p, st); else launch_prompt_dh<128, false>(p, st);
+    } else {
+        if (mask) launch_prompt_dh<64, true>(p, st); else launch_prompt_dh<64, false>(p, st);
+    }
     return 0;
 }

@@ -307,9 +307,12 @@ const int MMQ_MIN_TOKENS = 3;                           // (3 columns cost the m
 // integer kernel (profiles/r06_small_batch.txt; round 5's 256-token tiles: 3 x slower, profiles/r05_small_batch_crossover.txt). PM355_MMQ_MAX_TOKENS = 16 .. 64
 // moves the crossover (the F16 path is the prompt's parity tier: activations not re-quantized)
 const int MMQ_MAX_TOKENS = [] { const char * e = getenv("PM355_MMQ_MAX_TOKENS"); const int v = e ? atoi(e) : 0; return v >= 16 && v <= 64 ? v : 32; }();
-// small batches from this size on attend through the prompt path's matrix-core kernel (attn_prefill.hip: one workgroup per head, the same rounding points);
-// below it one workgroup per (head, token) (attn_cached.hip). 70B layer at 16 / 24 / 32 tokens: 190.1 / 219.1 / 229.9 -> 188.9 / 214.0 / 217.0 us
+// small batches of at least so many tokens, or that attend at least so many cells, take the prompt path's matrix-core kernel (attn_prefill.hip); the others one workgroup per
+// (head, token) (attn_cached.hip). Layer of the 70B shape, 2 / 8 / 15 tokens: behind 120 cells 134.0 / 158.0 / 176.5 us with the workgroups per token, 133.7 / 157.4 / 170.7 on the matrix
+// cores; behind 300 141.6 / 165.3 / 188.7 against 136.4 / 159.5 / 172.2, behind 3000 194 / 249 / 358 against 162 / 185 / 200; of the 8B shape behind 30 cells 67.5 / 84.0 / 89.6 against
+// 69.8 / 86.4 / 92.0, behind 300 76.3 / 91.7 / 99.3 against 72.4 / 89.1 / 94.5
 const int SMALL_ATTN_MFMA_MIN = [] { const char * e = getenv("PM355_SMALL_ATTN_MFMA_MIN"); return e ? atoi(e) : 16; }();
+const int SMALL_ATTN_MFMA_CELLS = 192;
 const int MMQ_MULTI_MIN_TOKENS = 2;       // the fused wq | wk | wv and ffn_gate | ffn_up launches already win at 2 tokens (3 / 4 mat-vec launches otherwise)
 // the table output of the Q8_K quantizers, when this batch size takes the small-batch mat-mul (mmq_i8.hip)
 pm_q8k_tables mmq_tables(const pm_window * m, int K, int T, hipStream_t st) {
@@ -820,8 +823,7 @@ int run_window(pm_window * m, const int32_t * d_tokens, const float * d_x_in, in
                                 (const float *) m->rope_freqs.d, T, H, Hkv, dh, hp.n_ctx, m->rope, st, 1);
         // (a shape attn_cached refuses - head_dim other than 64 / 128 / 256, scores beyond 150 KiB of LDS - falls back to attn_decode, which rounds q to
         //  F16 itself: the pre-rounded rows give it the same bits as raw ones, tests/test_gpu_ops.py::test_small_batch_attention_fallback_...)
-        // (from SMALL_ATTN_MFMA_MIN tokens on: the prompt path's matrix-core kernel - 12 us per layer at 32 tokens against 26 for 2048 small workgroups)
-        if (!(T >= SMALL_ATTN_MFMA_MIN && pm_launch_attn_prefill(m->q, L.kc, L.vc, m->d_pos, m->d_ctl, kv_stride, m->att, T, H, Hkv, dh, hp.n_ctx, kq_scale, st) == 0))
+        if (!((T >= SMALL_ATTN_MFMA_MIN || m->h_pos[m->h_seq] + T >= SMALL_ATTN_MFMA_CELLS) && pm_launch_attn_prefill(m->q, L.kc, L.vc, m->d_pos, m->d_ctl, kv_stride, m->att, T, H, Hkv, dh, hp.n_ctx, kq_scale, st) == 0))
         if (pm_launch_attn_cached(m->q, L.kc, L.vc, m->d_pos, m->d_ctl, kv_stride, m->att, H, Hkv, dh, hp.n_ctx, kq_scale, st, nullptr, nullptr, 0, 0, 0, T) &&
             pm_launch_attn_decode(m->q, L.kc, L.vc, m->d_pos, m->d_ctl, kv_stride, m->att, T, H, Hkv, dh, hp.n_ctx, kq_scale, st))
             return seterr(m, PM355_E_RANGE, "decode: n_ctx too large for the decode-attention kernel");

@@ -441,6 +441,44 @@ def test_attn_prefill_mfma_vs_exact(P, oracle, n_past, T, dh):
             assert np.abs(out[t, h] - want).max() <= 2e-3 * np.abs(want).max() + 1e-4, (t, h)
 
 
+@pytest.mark.parametrize("H,Hkv,dh,T,past,mask", [
+    (8, 2, 128, 1, 0, None), (8, 2, 64, 31, 1, None), (6, 3, 128, 33, 95, None), (8, 8, 64, 65, 127, None), (8, 1, 128, 130, 30, None),      # 64 queries per workgroup
+    (64, 8, 128, 500, 12, None), (256, 32, 64, 128, 1, None),                                                                           # 128
+    (128, 8, 64, 1000, 23, None), (128, 8, 128, 1021, 0, None),                                                                          # 256
+    (8, 2, 128, 40, 60, "f32"), (8, 2, 64, 40, 60, "f16"), (64, 8, 128, 500, 12, "f16"), (128, 8, 64, 1000, 24, "f32")])
+def test_attn_prefill_tiles_against_float64(P, H, Hkv, dh, T, past, mask):
+    """Every tile choice of the one-pass kernel (64 / 128 / 256 queries per workgroup), tokens and keys around the tile edges, caches that end on half a stage, both mask types.
+    Bound: every probability is rounded to F16 once (2^-11 of itself at most), so an output is off by 2^-11 sum p |v|; a tenth of it again for the f32 scores and sums."""
+    import ctypes as C
+    from prima_cpp_amd import lib as L
+    torch = P.torch
+    n = past + T
+    n_ctx = -(-n // 32) * 32
+    g = torch.Generator(device="cuda").manual_seed(n + dh)
+    q = torch.randn((T, H, dh), generator=g, device="cuda") * 2
+    K = torch.randn((n_ctx, Hkv, dh), generator=g, device="cuda").half()
+    V = torch.randn((Hkv, dh, n_ctx), generator=g, device="cuda").half()
+    sc = 1.0 / np.sqrt(dh)
+    seen = torch.arange(n, device="cuda")[None] <= torch.arange(T, device="cuda")[:, None] + past
+    if mask is None:
+        out = P.attn_prefill(q.view(T, -1), K, V, past, H, Hkv, dh, n_ctx, sc).view(T, H, dh)
+    else:                                                  # cells at random, the query's own always; n_kv a multiple of 4 as the graphs have it
+        seen &= torch.rand((T, n), generator=g, device="cuda") < 0.7
+        seen[torch.arange(T), torch.arange(T) + past] = True
+        n_kv = -(-n // 4) * 4
+        m = torch.full((T, n_kv), -np.inf, device="cuda", dtype=torch.float32 if mask == "f32" else torch.float16)
+        m[:, :n][seen] = 0
+        out = torch.empty((T, H, dh), device="cuda")
+        f = L.declare("pm355_attn_prefill_masked_ex", C.c_int, [C.c_void_p] * 4 + [C.c_int64, C.c_void_p] + [C.c_int] * 6 + [C.c_float, C.c_int, C.c_void_p])
+        L.check(f(L.ptr(q), L.ptr(K), L.ptr(V), L.ptr(m), n_kv, L.ptr(out), T, H, Hkv, dh, n_ctx, n_kv, float(sc), 0 if mask == "f32" else 2, L.stream_ptr()), "masked")
+    for h in range(0, H, max(1, H // 8)):
+        k, v = K[:n, h * Hkv // H].double(), V[h * Hkv // H, :, :n].double()
+        p = ((q[:, h].half().double() @ k.T) * sc).masked_fill(~seen, -np.inf).softmax(-1)
+        off = (out[:, h].double() - p @ v.T).abs()
+        bound = 1.1 * 2.0 ** -11 * (p @ v.abs().T) + 1e-6
+        assert bool((off <= bound).all()), (h, float((off / bound).max()))
+
+
 @pytest.mark.parametrize("dh", [64, 128])
 @pytest.mark.parametrize("n_past", [0, 5, 255, 256, 700, 1023])
 def test_attn_decode_split_equals_single_workgroup_kernel(P, n_past, dh):
