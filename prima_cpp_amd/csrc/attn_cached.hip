@@ -20,9 +20,9 @@
 namespace {
 
 // this token's (cos, sin) per rotation pair: one launch per token serves every layer's wq | wk | wv epilogue
-__global__ __launch_bounds__(128) void rope_table_kernel(RopeP r, const int32_t * pos_ptr, const int32_t * seq_ptr, const float * freq_factors, float * tab) {
-    const int seq = seq_ptr ? *seq_ptr : 0;
-    const int pos = pos_ptr[seq] + (int) blockIdx.x;             // (blockIdx.x: token of a small batch, its table n_dims floats further on)
+__global__ __launch_bounds__(128) void rope_table_kernel(RopeP r, const int32_t * pos_ptr, const int32_t * seq_ptr, const float * freq_factors, float * tab, int rows) {
+    // (blockIdx.x: token of a small batch, its table n_dims floats further on)
+    const int pos = rows ? pos_ptr[blockIdx.x] : pos_ptr[seq_ptr ? *seq_ptr : 0] + (int) blockIdx.x;
     tab += (size_t) blockIdx.x * r.n_dims;
     for (int pair = threadIdx.x; pair < r.n_dims / 2; pair += blockDim.x) {
         float c, s;
@@ -70,8 +70,8 @@ __global__ __launch_bounds__(256) void attn_cached_kernel(AttnP a_in) {
         int seq = 0, n_kv;
         if (a.dyn) n_kv = uniform_const_ptr(a.dyn)[1];
         else {
-            seq = a.seq_ptr ? uniform_const_ptr(a.seq_ptr)[0] : 0;
-            n_kv = uniform_const_ptr(a.pos0_ptr)[seq] + 1 + a.tok;
+            seq = a.seq_ptr ? uniform_const_ptr(a.seq_ptr)[a.rows ? a.tok : 0] : 0;
+            n_kv = uniform_const_ptr(a.pos0_ptr)[a.rows ? a.tok : seq] + 1 + (a.rows ? 0 : a.tok);
         }
         // (short path: a lane owns a key and reads whole V^T chunks of KPP cells - only where the cache holds at least 64 cells per row; a smaller
         //  n_ctx takes the general body below, whose loads are bounded by n_kv)
@@ -147,18 +147,18 @@ __global__ __launch_bounds__(256) void attn_cached_kernel(AttnP a_in) {
 
 } // namespace
 
-void pm_launch_rope_table(const pm_rope_cfg & c, const int32_t * pos, const int32_t * seq, const float * freq_factors, float * tab, hipStream_t st, int n_tok) {
+void pm_launch_rope_table(const pm_rope_cfg & c, const int32_t * pos, const int32_t * seq, const float * freq_factors, float * tab, hipStream_t st, int n_tok, int rows) {
     RopeP r;
     r.n_dims = c.n_dims; r.mode = c.mode; r.n_ctx_orig = c.n_ctx_orig; r.theta_scale = c.theta_scale;
     r.freq_scale = c.freq_scale; r.ext_factor = c.ext_factor; r.attn_factor = c.attn_factor; r.corr0 = c.corr0; r.corr1 = c.corr1;
-    hipLaunchKernelGGL(rope_table_kernel, dim3(n_tok < 1 ? 1 : n_tok), dim3(128), 0, st, r, pos, seq, freq_factors, tab);
+    hipLaunchKernelGGL(rope_table_kernel, dim3(n_tok < 1 ? 1 : n_tok), dim3(128), 0, st, r, pos, seq, freq_factors, tab, rows);
 }
 
 // q = rotated, F16-rounded query rows; caches already hold this token. Same arguments as pm_launch_attn_rope_fused otherwise.
 int pm_launch_attn_cached(const float * q, void * kc, void * vc, const int32_t * pos0, const int32_t * seq, long seq_stride, float * out,
                           int H, int Hkv, int dh, int n_ctx, float scale, hipStream_t st, const int32_t * dyn, const void * mask,
-                          int max_keys, int v_rowmajor, int mask_f16, int n_tok) {
-    if ((dh != 64 && dh != 128 && dh != 256) || n_ctx % 8 || n_tok < 1 || (n_tok > 1 && dyn)) return -1;
+                          int max_keys, int v_rowmajor, int mask_f16, int n_tok, int rows) {
+    if ((dh != 64 && dh != 128 && dh != 256) || n_ctx % 8 || n_tok < 1 || (n_tok > 1 && dyn) || (rows && (dyn || !seq || !pos0))) return -1;
     const size_t lds = (size_t) (4 * dh + (v_rowmajor ? 2048 : 256) + (max_keys > 0 ? ((max_keys + 7) & ~7) : n_ctx) + 8) * 4;
     if (lds > 150 * 1024) return -1;
     RopeP r = {};
@@ -167,7 +167,7 @@ int pm_launch_attn_cached(const float * q, void * kc, void * vc, const int32_t *
     auto launch = [&](auto kern) {
         if (lds > 48 * 1024) (void) hipFuncSetAttribute((const void *) kern, hipFuncAttributeMaxDynamicSharedMemorySize, 150 * 1024);
         AttnP a = {q, nullptr, nullptr, (uint16_t *) kc, (uint16_t *) vc, pos0, seq, seq_stride, nullptr, out, H, Hkv, n_ctx, scale, r, dyn,
-                   (const float *) mask, mask_f16, pm_ts_next_slot()};
+                   (const float *) mask, mask_f16, pm_ts_next_slot(), 0, rows};
         hipLaunchKernelGGL(kern, dim3(H, n_tok), dim3(256), lds, st, a);
     };
     if (v_rowmajor) {

@@ -37,6 +37,7 @@ struct AttnP {
     int mask_f16;
     unsigned long long * ts;                 // measurement builds (-DPM_TS)
     int tok;                                 // engine mode, cached form: token index of a multi-token launch (position = pos0 + tok; q / out rows are advanced by the kernel)
+    int rows;                                // ... with a sequence and a position of its own per token: seq_ptr[tok], pos0_ptr[tok]
 };
 __device__ __forceinline__ float attn_mask_at(const void * mask, int f16, int i) {
     if (!mask) return 0.0f;
@@ -115,13 +116,14 @@ __device__ __forceinline__ void attn_rope_body(const AttnP & a, int h, char * sm
     };
     int seq = 0, pos, slot, n_kv;                // rope position, cache cell of this token, cells attended = [0, n_kv)
     int pv = 0, sv = 0;
-    if (seq_ptr) { pv = pos0_ptr[lane]; sv = *seq_ptr; } else pv = pos0_ptr[0];     // (the engine's position table has 64 entries)
+    if (CACHED && a.rows) { pv = pos0_ptr[a.tok]; sv = seq_ptr[a.tok]; }
+    else if (seq_ptr) { pv = pos0_ptr[lane]; sv = *seq_ptr; } else pv = pos0_ptr[0];     // (the engine's position table has 64 entries)
     int dyn0 = 0, dyn1 = 0;
     if (a.dyn) { const PM_G int32_t * dyn = (const PM_G int32_t *) a.dyn; dyn0 = dyn[0]; dyn1 = dyn[1]; }
     if (seq_stride == 0 || !seq_ptr) first_loads(kc, vc);
     if (seq_ptr) {
         seq = __builtin_amdgcn_readfirstlane(sv);
-        pos = __builtin_amdgcn_readlane(pv, seq) + a.tok;
+        pos = CACHED && a.rows ? __builtin_amdgcn_readfirstlane(pv) : __builtin_amdgcn_readlane(pv, seq) + a.tok;
         slot = pos; n_kv = pos + 1;
     } else {
         pos = __builtin_amdgcn_readfirstlane(pv) + a.tok;

@@ -29,6 +29,7 @@ struct PfP {
     const float * mask; long mask_stride; int n_kv;
     int mask_f16;                                // the mask rows are F16
     _Float16 * out_h;                            // optional: the result as F16 [T][H*DH] (activations of the wo GEMM) instead of `out`
+    const int32_t * tiles; int n_tiles;          // optional: tiles {row, queries, position, sequence} of several sequences; else consecutive tokens from pos0 on
 };
 
 // Flash-attention graphs (FLASH_ATTN_EXT, llm_build_kqv src/llama.cpp:10075-10095): V cache [n_ctx][Hkv*DH] like K, always masked. One workgroup = 128 queries of one head, 4 waves x
@@ -233,21 +234,21 @@ __global__ __launch_bounds__(512, 2) void attn_prompt_kernel(PfP p) {
     const int qw = wave % QW, kw = wave / QW;
     // an XCD (blockIdx % 8) keeps to its share of the heads: the query heads of a KV head meet in one L2. Tiles with the most keys first: the short ones fill the tail
     int h, tile;
-    const int n_tiles = (p.T + QW * 32 - 1) / (QW * 32);
     if (p.H % 8 == 0) { const int per = p.H / 8, j = blockIdx.x >> 3; h = (blockIdx.x & 7) * per + j % per; tile = j / per; }
     else { h = blockIdx.x % p.H; tile = blockIdx.x / p.H; }
-    tile = n_tiles - 1 - tile;
+    tile = p.n_tiles - 1 - tile;
     const int hk = h / (p.H / p.Hkv);
-    const int seq = p.seq_ptr ? *p.seq_ptr : 0;
-    const int pos0 = MASK ? 0 : p.pos0_ptr[seq];
+    int row0 = tile * QW * 32, nq = min(QW * 32, p.T - row0), pos0 = 0, seq = 0;                 // the workgroup's first row, its queries, the first one's position
+    if (!MASK && p.tiles) { row0 = p.tiles[4 * tile]; nq = p.tiles[4 * tile + 1]; pos0 = p.tiles[4 * tile + 2]; seq = p.tiles[4 * tile + 3]; }
+    else { seq = p.seq_ptr ? *p.seq_ptr : 0; if (!MASK) pos0 = p.pos0_ptr[seq] + row0; }
     const long krow = (long) p.Hkv * DH;
     const uint16_t * kc = p.kc + (long) seq * p.seq_stride + (long) hk * DH;                     // K[key][Hkv*DH]
     const uint16_t * vc = p.vc + (long) seq * p.seq_stride + (long) hk * DH * p.n_ctx;           // V^T[hk*DH + e][n_ctx]
-    const int tq0 = tile * QW * 32 + qw * 32;                                                    // first query of this wave
-    const bool live = tq0 < p.T;
-    const int tq = min(tq0 + lr, p.T - 1), qpos = pos0 + tq;
-    const int w_first = pos0 + tq0, w_last = pos0 + min(tq0 + 31, p.T - 1);                      // the wave's first and last query
-    const int n_keys = MASK ? p.n_kv : pos0 + min(tile * QW * 32 + QW * 32, p.T);                // cells the workgroup's last query sees
+    const int q0 = qw * 32, tq0 = row0 + q0;                                                     // first query of this wave: in the workgroup, and its row
+    const bool live = q0 < nq;
+    const int qi = min(q0 + lr, nq - 1), tq = row0 + qi, qpos = pos0 + qi;
+    const int w_first = pos0 + q0, w_last = pos0 + min(q0 + 31, nq - 1);                         // positions of the wave's first and last query
+    const int n_keys = MASK ? p.n_kv : pos0 + nq;                                                // cells the workgroup's last query sees
     const int n_it = (n_keys + KS - 1) / KS;
 
     const uint32_t lds0 = (uint32_t) (uintptr_t) (__attribute__((address_space(3))) char *) smem;
@@ -387,7 +388,7 @@ __global__ __launch_bounds__(512, 2) void attn_prompt_kernel(PfP p) {
     __syncthreads();
     constexpr int RL = DH / 4, RP = 64 / RL;                       // lanes per row (4 values each), rows per pass
     for (int r = kw * (32 / KW) + lane / RL; r < (kw + 1) * (32 / KW); r += RP) {
-        if (tq0 + r >= p.T) break;
+        if (q0 + r >= nq) break;
         float4 a = *(const float4 *) (ex + (qw * 32 + r) * OS + 4 * (lane % RL));
 #pragma unroll
         for (int g = 1; g < KW; ++g) {
@@ -400,40 +401,48 @@ __global__ __launch_bounds__(512, 2) void attn_prompt_kernel(PfP p) {
     }
 }
 
-template <int DH, int QW, int KS, bool MASK> void launch_prompt(const PfP & p, hipStream_t st) {
+template <int DH, int QW, int KS, bool MASK> void launch_prompt(PfP p, hipStream_t st) {
+    if (!p.tiles) p.n_tiles = (p.T + QW * 32 - 1) / (QW * 32);
     constexpr size_t stages = 2 * (size_t) KS * DH * 4, ex = (size_t) 8 * 32 * (DH + 4) * 4 + 8 * 32 * 2 * 4, lds = stages > ex ? stages : ex;
     pm_allow_big_lds((const void *) attn_prompt_kernel<DH, QW, KS, MASK>, lds);
-    hipLaunchKernelGGL((attn_prompt_kernel<DH, QW, KS, MASK>), dim3((p.T + QW * 32 - 1) / (QW * 32) * p.H), dim3(512), lds, st, p);
+    hipLaunchKernelGGL((attn_prompt_kernel<DH, QW, KS, MASK>), dim3(p.n_tiles * p.H), dim3(512), lds, st, p);
 }
 // Which tile: a CU holds one workgroup. 256 queries share a stage where that still makes two rounds of workgroups (2048 tokens x 64 heads: 102 us, 110 with 128 queries; x 32 heads
 // = one round whose longest tile decides: 80 against 57); 128 queries where they make one (512 x 64 behind 1024 cached: 38 against 50 with 64); below that 64 queries with four key
 // groups each (101 x 32 behind 300: 11.7 against 14.9).
-template <int DH, bool MASK> void launch_prompt_dh(const PfP & p, hipStream_t st) {
+int tile_of(int n_tok, int H) {
     const int cus = pm_device_cus();
-    if ((p.T + 255) / 256 * p.H >= 2 * cus) launch_prompt<DH, 8, 64, MASK>(p, st);
-    else if ((p.T + 127) / 128 * p.H >= cus) launch_prompt<DH, 4, 128, MASK>(p, st);
+    return (n_tok + 255) / 256 * H >= 2 * cus ? 256 : (n_tok + 127) / 128 * H >= cus ? 128 : 64;
+}
+template <int DH, bool MASK> void launch_prompt_dh(const PfP & p, int tile_q, hipStream_t st) {
+    if (tile_q == 256) launch_prompt<DH, 8, 64, MASK>(p, st);
+    else if (tile_q == 128) launch_prompt<DH, 4, 128, MASK>(p, st);
     else launch_prompt<DH, 2, 128, MASK>(p, st);
 }
 
 } // namespace
 
+int pm_attn_prefill_tile(int n_tok, int H) { return tile_of(n_tok, H); }
+
 // n_ctx % 32 == 0 and head_dim 64 / 128 only (callers fall back to the per-token kernel otherwise)
 int pm_launch_attn_prefill(const float * q, const void * kc, const void * vc, const int32_t * pos0, const int32_t * seq,
                            long seq_stride, float * out, int n_tok, int H, int Hkv, int dh, int n_ctx, float scale, hipStream_t st,
-                           const float * mask, long mask_stride, int n_kv, int v_rowmajor, int mask_f16, void * out_f16) {
+                           const float * mask, long mask_stride, int n_kv, int v_rowmajor, int mask_f16, void * out_f16, const int32_t * tiles, int n_tiles, int tile_q) {
     if ((dh != 64 && dh != 128) || n_ctx % 32 || n_tok < 1) return -1;
     if (mask && (n_kv < 1 || n_kv > n_ctx || n_kv % 4 || mask_stride % 4)) return -1;
     if ((v_rowmajor || mask_f16) && !mask) return -1;                 // the flash-attention form exists in ggml-graph mode only
-    PfP p = {q, (const uint16_t *) kc, (const uint16_t *) vc, pos0, seq, seq_stride, out, n_tok, H, Hkv, n_ctx, scale, mask, mask_stride, n_kv, mask_f16 ? 1 : 0, (_Float16 *) out_f16};
+    PfP p = {q, (const uint16_t *) kc, (const uint16_t *) vc, pos0, seq, seq_stride, out, n_tok, H, Hkv, n_ctx, scale, mask, mask_stride, n_kv, mask_f16 ? 1 : 0, (_Float16 *) out_f16, tiles, n_tiles};
+    if (tiles && (mask || n_tiles < 1)) return -1;
+    if (!tiles) tile_q = tile_of(n_tok, H);
     if (v_rowmajor) {
         if (out_f16 || seq) return -1;
         const dim3 grid((n_tok + 127) / 128, H);
         if (dh == 128) hipLaunchKernelGGL(attn_rowmajor_kernel<128>, grid, dim3(256), 0, st, p);
         else           hipLaunchKernelGGL(attn_rowmajor_kernel<64>, grid, dim3(256), 0, st, p);
     } else if (dh == 128) {
-        if (mask) launch_prompt_dh<128, true>(p, st); else launch_prompt_dh<128, false>(p, st);
+        if (mask) launch_prompt_dh<128, true>(p, tile_q, st); else launch_prompt_dh<128, false>(p, tile_q, st);
     } else {
-        if (mask) launch_prompt_dh<64, true>(p, st); else launch_prompt_dh<64, false>(p, st);
+        if (mask) launch_prompt_dh<64, true>(p, tile_q, st); else launch_prompt_dh<64, false>(p, tile_q, st);
     }
     return 0;
 }

@@ -106,6 +106,10 @@ struct pm_window : pm355_model {
     std::vector<StepGraph> graphs;
     // batches: open sequences (a sequence holds one KV slab), their last greedy token on the device, and the hidden rows of a portion whose logits are asked for
     std::vector<char> seq_open; int32_t * d_last = nullptr; float * rows = nullptr;
+    // a pass over rows of several sequences (batch): every row's position and sequence in device memory, tiles for the matrix-core attention; rag is set while one is launched
+    struct Ragged { const int32_t * pos, * seq, * tiles; int n_tiles, tile_q, max_cells; bool singles; };
+    const Ragged * rag = nullptr; int32_t * d_rows = nullptr; float * head_lg = nullptr;
+    int batch_rows(const pm355_batch_entry * e, int n, float * d_logits, int32_t * d_argmax, hipStream_t st, bool * served);
 
     ~pm_window() override;
     int set_tensor(int kind, int layer, int type, const void * host, size_t nbytes) override;
@@ -313,6 +317,7 @@ const int MMQ_MAX_TOKENS = [] { const char * e = getenv("PM355_MMQ_MAX_TOKENS");
 // 69.8 / 86.4 / 92.0, behind 300 76.3 / 91.7 / 99.3 against 72.4 / 89.1 / 94.5
 const int SMALL_ATTN_MFMA_MIN = [] { const char * e = getenv("PM355_SMALL_ATTN_MFMA_MIN"); return e ? atoi(e) : 16; }();
 const int SMALL_ATTN_MFMA_CELLS = 192;
+constexpr int HEAD_ROWS = 32;            // rows of a batch that go through the head at once (what one pass of the integer mat-mul takes)
 const int MMQ_MULTI_MIN_TOKENS = 2;       // the fused wq | wk | wv and ffn_gate | ffn_up launches already win at 2 tokens (3 / 4 mat-vec launches otherwise)
 // the table output of the Q8_K quantizers, when this batch size takes the small-batch mat-mul (mmq_i8.hip)
 pm_q8k_tables mmq_tables(const pm_window * m, int K, int T, hipStream_t st) {
@@ -604,6 +609,20 @@ int run_layers_fused(pm_window * m, const float * cur, float * d_x_out, const fl
     return 0;
 }
 
+// batches up to MMQ_MAX_TOKENS take the small-batch path (8-bit activations) unless its per-token attention kernel cannot hold n_ctx scores in LDS, or one of the layer's large matrices
+// has a type neither small-batch path serves: then up to SMALL_PLAIN_MAX
+constexpr int SMALL_PLAIN_MAX = 15;
+bool small_path(const pm_window * m, const Layer & L, int T) {
+    bool ok = !m->no_mmq && (size_t) (m->hp.head_dim + m->hp.n_ctx) * 4 <= 150 * 1024;
+    for (int k : {PM355_T_WQ, PM355_T_WO, PM355_T_FFN_GATE, PM355_T_FFN_UP, PM355_T_FFN_DOWN}) {
+        // Q4_K / Q5_K / Q6_K and (round 4) Q8_0 - Qwen2.5-72B's ffn_down: 29568 % 256 != 0, src/llama.cpp:19547 - on the integer matrix cores
+        // (mmq_i8.hip; Q8_0 with Q8_0 activations = ggml_vec_dot_q8_0_q8_0's arithmetic); a Q8_0 shape it does not serve falls back to the multi-column mat-vec
+        const bool served = pm_mmq_i8_check(L.t[k].type, (int) L.t[k].K, (int) L.t[k].N, T < 1 ? 1 : (T > MMQ_MAX_TOKENS ? MMQ_MAX_TOKENS : T)) == 0;
+        ok = ok && (served || L.t[k].type == PM_Q8_0);
+    }
+    return ok;
+}
+
 // x_in -> x_out for layers [lo, hi); positions from device memory d_pos (pos of token 0)
 int run_window(pm_window * m, const int32_t * d_tokens, const float * d_x_in, int T, float * d_x_out,
                float * d_logits, int32_t * d_argmax, hipStream_t st) {
@@ -625,7 +644,24 @@ int run_window(pm_window * m, const int32_t * d_tokens, const float * d_x_in, in
     // are written here, once for all layers
     const bool small_epi = T >= MMQ_MULTI_MIN_TOKENS && T <= 32 && T <= MMQ_MAX_TOKENS && !m->no_fuse && !m->no_mmq && !m->no_multi && !m->no_small_epi && m->qkv_epi && m->rope_tab &&
                            m->rope.mode == 0 && m->hi > m->lo;
-    if (small_epi) pm_launch_rope_table(m->rope, m->d_pos, m->d_ctl, (const float *) m->rope_freqs.d, m->rope_tab, st, T);
+    // positions and sequences: consecutive tokens of the current sequence from d_pos on, or (rg) every row its own
+    const pm_window::Ragged * rg = m->rag;
+    const int32_t * d_pos = rg ? rg->pos : m->d_pos, * d_seq = rg ? rg->seq : m->d_ctl;
+    const long kv_stride = (long) hp.n_ctx * Hkv * dh;
+    auto rope_store = [&](const Layer & L, int round_q) {
+        pm_launch_rope_kv_store(m->q, m->k, m->v, m->q, nullptr, L.kc, L.vc, d_pos, d_seq, kv_stride, (const float *) m->rope_freqs.d, T, H, Hkv, dh, hp.n_ctx, m->rope, st, round_q, rg ? 1 : 0);
+    };
+    auto attend_mfma = [&](const Layer & L, float * out, void * out_f16) {
+        return pm_launch_attn_prefill(m->q, L.kc, L.vc, d_pos, d_seq, kv_stride, out, T, H, Hkv, dh, hp.n_ctx, kq_scale, st, nullptr, 0, 0, 0, 0, out_f16,
+                                      rg ? rg->tiles : nullptr, rg ? rg->n_tiles : 0, rg ? rg->tile_q : 0);
+    };
+    // one workgroup per (head, token); a shape attn_cached refuses - head_dim other than 64 / 128 / 256, scores beyond 150 KiB of LDS - falls back to attn_decode, which rounds q to
+    // F16 itself: the pre-rounded rows give it the same bits as raw ones, tests/test_gpu_ops.py::test_small_batch_attention_fallback_...
+    auto attend_rows = [&](const Layer & L) {
+        const int rc = pm_launch_attn_cached(m->q, L.kc, L.vc, d_pos, d_seq, kv_stride, m->att, H, Hkv, dh, hp.n_ctx, kq_scale, st, nullptr, nullptr, rg ? rg->max_cells : 0, 0, 0, T, rg ? 1 : 0);
+        return rc && !rg ? pm_launch_attn_decode(m->q, L.kc, L.vc, d_pos, d_seq, kv_stride, m->att, T, H, Hkv, dh, hp.n_ctx, kq_scale, st) : rc;
+    };
+    if (small_epi) pm_launch_rope_table(m->rope, d_pos, d_seq, (const float *) m->rope_freqs.d, m->rope_tab, st, T, rg ? 1 : 0);
     if (T == 1 && !m->no_fuse) {
         m->flash_cells = attn_regime(m); m->long_ctx = m->flash_cells != 0;
         // ---- single token: every activation transform is fused into a mat-vec prologue / epilogue, 5 launches per layer
@@ -653,15 +689,7 @@ int run_window(pm_window * m, const int32_t * d_tokens, const float * d_x_in, in
     for (int il = m->lo; il < m->hi; ++il) {
         Layer Lv = layer_acquire(m, il, st); Layer & L = Lv;
         const Tensor * qkv[3] = {&L.t[PM355_T_WQ], &L.t[PM355_T_WK], &L.t[PM355_T_WV]};
-        // batches up to MMQ_MAX_TOKENS take the small-batch path below unless its per-token attention kernel cannot hold n_ctx scores in LDS
-        const bool small_attn_ok = (size_t) (dh + hp.n_ctx) * 4 <= 150 * 1024;
-        bool small_ok = !m->no_mmq && small_attn_ok;              // ... and unless one of the layer's large matrices has a type neither small-batch path serves
-        for (int k : {PM355_T_WQ, PM355_T_WO, PM355_T_FFN_GATE, PM355_T_FFN_UP, PM355_T_FFN_DOWN}) {
-            // Q4_K / Q5_K / Q6_K and (round 4) Q8_0 - Qwen2.5-72B's ffn_down: 29568 % 256 != 0, src/llama.cpp:19547 - on the integer matrix cores
-            // (mmq_i8.hip; Q8_0 with Q8_0 activations = ggml_vec_dot_q8_0_q8_0's arithmetic); a Q8_0 shape it does not serve falls back to the multi-column mat-vec
-            const bool served = pm_mmq_i8_check(L.t[k].type, (int) L.t[k].K, (int) L.t[k].N, T < 1 ? 1 : (T > MMQ_MAX_TOKENS ? MMQ_MAX_TOKENS : T)) == 0;
-            small_ok = small_ok && (served || L.t[k].type == PM_Q8_0);
-        }
+        const bool small_ok = small_path(m, L, T);
         // prompts: every large matrix the integer kernel serves (Q4_K / Q6_K, K % 1024 == 0) runs on Q8_K activations with the CPU reference's
         // arithmetic; wv alone may stay on the F16 GEMM (Llama-3-70B Q4_K_M: Q5_K in half the layers, src/llama.cpp:19360-19373)
         bool big_ok = T > MMQ_MAX_TOKENS && !m->no_fuse && !m->no_big && m->tab_big && m->h2;
@@ -688,11 +716,8 @@ int run_window(pm_window * m, const int32_t * d_tokens, const float * d_x_in, in
             (void) hipEventRecord(m->side_b, m->side);
             (void) hipStreamWaitEvent(st, m->side_b, 0);
             if (rc) return seterr(m, PM355_E_UNSUPPORTED, "prefill: qkv mat-mul (integer matrix cores)");
-            const long kvs = (long) hp.n_ctx * Hkv * dh;
-            pm_launch_rope_kv_store(m->q, m->k, m->v, m->q, nullptr, L.kc, L.vc, m->d_pos, m->d_ctl, kvs,
-                                    (const float *) m->rope_freqs.d, T, H, Hkv, dh, hp.n_ctx, m->rope, st);
-            if (pm_launch_attn_prefill(m->q, L.kc, L.vc, m->d_pos, m->d_ctl, kvs, m->att, T, H, Hkv, dh, hp.n_ctx, kq_scale, st) &&
-                pm_launch_attn_decode(m->q, L.kc, L.vc, m->d_pos, m->d_ctl, kvs, m->att, T, H, Hkv, dh, hp.n_ctx, kq_scale, st))
+            rope_store(L, 0);
+            if (attend_mfma(L, m->att, nullptr) && (rg || pm_launch_attn_decode(m->q, L.kc, L.vc, d_pos, d_seq, kv_stride, m->att, T, H, Hkv, dh, hp.n_ctx, kq_scale, st)))
                 return seterr(m, PM355_E_RANGE, "prefill: n_ctx too large for the attention kernel");
             pm_launch_quantize_q8k(m->att, m->aq_k, Eq, T, st, TB(Eq));
             float * x_mid = (cur == bufs[0]) ? bufs[1] : bufs[0];
@@ -707,7 +732,7 @@ int run_window(pm_window * m, const int32_t * d_tokens, const float * d_x_in, in
             cur = x_next;
             continue;
         }
-        if (T > (small_ok ? MMQ_MAX_TOKENS : 15) && !m->no_fuse) {
+        if (T > (small_ok ? MMQ_MAX_TOKENS : SMALL_PLAIN_MAX) && !m->no_fuse) {
             // ---- prefill: batched GEMMs on the MFMA matrix cores (mmq.hip), f32 activations
             // F16 plumbing: the producers of GEMM activations write them as F16 (the rounding the GEMM's own conversion pass would apply) into
             // the engine's scratch - xn / att in place of their f32 forms, h = silu(gate) * up into h2: no conversion launches, half the bytes
@@ -728,13 +753,11 @@ int run_window(pm_window * m, const int32_t * d_tokens, const float * d_x_in, in
                 rc = pm_launch_gemm_q_multi(qkvj, 3, nullptr, m->xn, E, T, st);
             }
             if (rc) return seterr(m, PM355_E_UNSUPPORTED, "prefill: qkv gemm");
-            const long kvs = (long) hp.n_ctx * Hkv * dh;
-            pm_launch_rope_kv_store(m->q, m->k, m->v, m->q, nullptr, L.kc, L.vc, m->d_pos, m->d_ctl, kvs,
-                                    (const float *) m->rope_freqs.d, T, H, Hkv, dh, hp.n_ctx, m->rope, st);
+            rope_store(L, 0);
             bool att_h = true;
-            if (pm_launch_attn_prefill(m->q, L.kc, L.vc, m->d_pos, m->d_ctl, kvs, nullptr, T, H, Hkv, dh, hp.n_ctx, kq_scale, st, nullptr, 0, 0, 0, 0, m->att)) {
+            if (attend_mfma(L, nullptr, m->att)) {
                 att_h = false;
-                if (pm_launch_attn_decode(m->q, L.kc, L.vc, m->d_pos, m->d_ctl, kvs, m->att, T, H, Hkv, dh, hp.n_ctx, kq_scale, st))
+                if (rg || pm_launch_attn_decode(m->q, L.kc, L.vc, d_pos, d_seq, kv_stride, m->att, T, H, Hkv, dh, hp.n_ctx, kq_scale, st))
                     return seterr(m, PM355_E_RANGE, "prefill: n_ctx too large for the attention kernel");
             }
             float * x_mid = (cur == bufs[0]) ? bufs[1] : bufs[0];
@@ -779,8 +802,8 @@ int run_window(pm_window * m, const int32_t * d_tokens, const float * d_x_in, in
         };
         // RoPE + KV store in the epilogue of the wq | wk | wv launch (NORM rope; the tokens' cos / sin tables were written once for this step): no
         // rope_kv_store launch. PM355_SMALL_ROPE_EPI=0: the separate launch
-        const long kv_stride = (long) hp.n_ctx * Hkv * dh;
-        const pm_qkv_epi qe = {m->rope_tab, m->d_pos, m->d_ctl, nullptr, kv_stride, L.kc, L.vc, Hkv, dh, hp.n_ctx, m->rope.n_dims, 0, 0};
+        pm_qkv_epi qe = {m->rope_tab, d_pos, d_seq, nullptr, kv_stride, L.kc, L.vc, Hkv, dh, hp.n_ctx, m->rope.n_dims, 0, 0};
+        qe.rows = rg ? 1 : 0;
         const pm_qkv_epi * epi = small_epi ? &qe : nullptr;
         bool rope_done = false;
         const Tensor & wq_ = L.t[PM355_T_WQ], & wk_ = L.t[PM355_T_WK], & wv_ = L.t[PM355_T_WV];
@@ -818,14 +841,9 @@ int run_window(pm_window * m, const int32_t * d_tokens, const float * d_x_in, in
         if (!fused_attn) {
         // q rotated AND rounded to F16, every token's K row / V column stored: the attention of a small batch then is the single-token kernel over
         // cached cells, one workgroup per (head, token) (attn_cached.hip: one barrier up to 64 cells; 11 -> ~4 us per layer at 2..8 tokens)
-        if (!rope_done)
-        pm_launch_rope_kv_store(m->q, m->k, m->v, m->q, nullptr, L.kc, L.vc, m->d_pos, m->d_ctl, kv_stride,
-                                (const float *) m->rope_freqs.d, T, H, Hkv, dh, hp.n_ctx, m->rope, st, 1);
-        // (a shape attn_cached refuses - head_dim other than 64 / 128 / 256, scores beyond 150 KiB of LDS - falls back to attn_decode, which rounds q to
-        //  F16 itself: the pre-rounded rows give it the same bits as raw ones, tests/test_gpu_ops.py::test_small_batch_attention_fallback_...)
-        if (!((T >= SMALL_ATTN_MFMA_MIN || m->h_pos[m->h_seq] + T >= SMALL_ATTN_MFMA_CELLS) && pm_launch_attn_prefill(m->q, L.kc, L.vc, m->d_pos, m->d_ctl, kv_stride, m->att, T, H, Hkv, dh, hp.n_ctx, kq_scale, st) == 0))
-        if (pm_launch_attn_cached(m->q, L.kc, L.vc, m->d_pos, m->d_ctl, kv_stride, m->att, H, Hkv, dh, hp.n_ctx, kq_scale, st, nullptr, nullptr, 0, 0, 0, T) &&
-            pm_launch_attn_decode(m->q, L.kc, L.vc, m->d_pos, m->d_ctl, kv_stride, m->att, T, H, Hkv, dh, hp.n_ctx, kq_scale, st))
+        if (!rope_done) rope_store(L, 1);
+        const bool mfma = rg ? rg->max_cells >= SMALL_ATTN_MFMA_CELLS : T >= SMALL_ATTN_MFMA_MIN || m->h_pos[m->h_seq] + T >= SMALL_ATTN_MFMA_CELLS;
+        if (!(mfma && attend_mfma(L, m->att, nullptr) == 0) && attend_rows(L))
             return seterr(m, PM355_E_RANGE, "decode: n_ctx too large for the decode-attention kernel");
         }
         const Tensor * wo[1] = {&L.t[PM355_T_WO]};
@@ -932,7 +950,7 @@ pm_window::~pm_window() {
     for (auto & L : m->layers) { for (auto & t : L.t) if (t.d) (void) hipFree(t.d); if (L.kc) (void) hipFree(L.kc); if (L.vc) (void) hipFree(L.vc); }
     Tensor * g[4] = {&m->tok_embd, &m->out_norm, &m->output, &m->rope_freqs};
     for (auto t : g) if (t->d) (void) hipFree(t->d);
-    void * s[] = {m->x, m->x1, m->q, m->k, m->v, m->att, m->h, m->h2, m->logits, m->xn, m->aq_k, m->aq_0, m->d_pos, m->d_tok, m->d_ctl, m->split_scratch, m->rope_tab, m->tab_big, m->ss, m->att_tk, m->d_last, m->rows};
+    void * s[] = {m->x, m->x1, m->q, m->k, m->v, m->att, m->h, m->h2, m->logits, m->xn, m->aq_k, m->aq_0, m->d_pos, m->d_tok, m->d_ctl, m->split_scratch, m->rope_tab, m->tab_big, m->ss, m->att_tk, m->d_last, m->rows, m->d_rows, m->head_lg};
     for (auto p : s) if (p) (void) hipFree(p);
     pm355_uploader_free(m->up);
     if (m->cap_stream) (void) hipStreamDestroy(m->cap_stream);
@@ -1254,7 +1272,12 @@ int pm_window::finalize_pool(int max_tokens_, int n_seq_, int64_t pool_tokens) {
     if (!(flags & PM355_HAS_EMBD) || !(flags & PM355_HAS_HEAD)) return seterr(this, PM355_E_UNSUPPORTED, "finalize_pool: batches need the embedding and the head");
     const int rc = finalize(max_tokens_, n_seq_);
     if (rc) return rc;
-    return hipMalloc((void **) &rows, (size_t) max_tokens * hp.n_embd * 4 + 256) == hipSuccess ? 0 : seterr(this, PM355_E_NOMEM, "finalize_pool: hidden rows");
+    const size_t T = max_tokens;
+    for (void * p : {(void *) rows, (void *) d_rows, (void *) head_lg}) if (p) (void) hipFree(p);
+    rows = head_lg = nullptr; d_rows = nullptr;
+    // (tables of a pass, pm_launch_batch_rows: 3 integers per row, 4 per tile, 2 per sequence, 1 per wanted row, 2 per kept token)
+    return hipMalloc((void **) &rows, T * hp.n_embd * 4 + 256) == hipSuccess && hipMalloc((void **) &d_rows, 12 * T * 4 + 256) == hipSuccess &&
+           hipMalloc((void **) &head_lg, (size_t) std::min(max_tokens, HEAD_ROWS) * hp.n_vocab * 4 + 256) == hipSuccess ? 0 : seterr(this, PM355_E_NOMEM, "finalize_pool: hidden rows");
 }
 int pm_window::seq_new() {
     if (!finalized) return seterr(this, PM355_E_SHAPE, "seq_new: model not finalized");
@@ -1272,6 +1295,105 @@ int pm_window::pool_info(pm355_pool_info * o) {
     for (char c : seq_open) if (!c) { ++o->free_pages; ++o->free_seqs; }
     return 0;
 }
+// All entries as rows of common passes: the weights are read once per pass instead of once per sequence (eight sequences of the 8B shape, eight layers and
+// head: prompts of 12..24 tokens and twelve steps 47.0 ms one sequence after another, 14.0 ms as common passes). A portion keeps the arithmetic that it has alone - up to 32 tokens 8-bit activations, beyond 16-bit ones -
+// whatever shares the step with it: the longer portions (a sequence's first ones) go first, then the short ones. served = false and nothing done where a pass does not take rows of
+// several sequences.
+int pm_window::batch_rows(const pm355_batch_entry * e, int n, float * d_logits, int32_t * d_argmax, hipStream_t st, bool * served) {
+    pm_window * m = this;
+    *served = false;
+    const int dh = hp.head_dim, V = hp.n_vocab;
+    if (no_fuse || hi <= lo || (dh != 64 && dh != 128) || hp.n_ctx % 32 || max_tokens < 2) return 0;      // (what the matrix-core attention takes)
+    int small = MMQ_MAX_TOKENS;
+    for (auto & L : layers) if (!small_path(this, L, MMQ_MAX_TOKENS)) small = SMALL_PLAIN_MAX;
+    small = std::min(small, max_tokens);
+    struct Want { int row, out; };                                                                          // row of the pass, row of the outputs
+    struct Pass { std::vector<int32_t> tok, pos, seq, ent, keep; std::vector<Want> want; int cap = 0, max_cells = 0; bool singles = true; };
+    std::vector<Pass> passes;
+    for (int longer = 1; longer >= 0; --longer) {
+        auto mine = [&](int T) { return (T > small) == (longer != 0); };
+        int64_t total = 0, done = 0;
+        for (int i = 0; i < n; ++i)
+            for (int off = 0; off < e[i].n_tokens; off += max_tokens) { const int T = std::min(max_tokens, e[i].n_tokens - off); if (mine(T)) total += T; }
+        const int64_t k = (total + (longer ? max_tokens : small) - 1) / (longer ? max_tokens : small);     // passes of equal size: a longer portion's piece stays above `small` rows
+        int64_t at = 0;
+        for (int i = 0, out0 = 0; i < n; out0 += e[i].n_want, ++i)
+            for (int p0 = 0; p0 < e[i].n_tokens; p0 += max_tokens) {
+                const int p1 = std::min(p0 + max_tokens, e[i].n_tokens);
+                if (!mine(p1 - p0)) continue;
+                for (int off = p0; off < p1;) {
+                    if (!at || (int) passes.back().tok.size() == passes.back().cap) { passes.emplace_back(); passes.back().cap = (int) (total * (at + 1) / k - total * at / k); ++at; }
+                    Pass & p = passes.back();
+                    const int row = (int) p.tok.size(), T = std::min(p.cap - row, p1 - off), pos0 = h_pos[e[i].seq] + off;
+                    for (int t = 0; t < T; ++t) { p.tok.push_back(e[i].tokens ? e[i].tokens[off + t] : -1); p.pos.push_back(pos0 + t); p.seq.push_back(e[i].seq); }
+                    p.ent.push_back(e[i].seq); p.ent.push_back(pos0 + T);
+                    p.max_cells = std::max(p.max_cells, pos0 + T); p.singles = p.singles && T == 1;
+                    for (int j = 0; j < e[i].n_want; ++j) if (e[i].want[j] >= off && e[i].want[j] < off + T) p.want.push_back({row + e[i].want[j] - off, out0 + j});
+                    if (d_argmax && e[i].n_want && off + T == e[i].n_tokens) { p.keep.push_back(e[i].seq); p.keep.push_back(out0 + e[i].n_want - 1); }
+                    off += T; done += T;
+                }
+            }
+        if (done != total) return 0;
+    }
+    for (Pass & p : passes) if (p.want.size() > p.tok.size()) return 0;                                     // (a row asked for several times)
+    *served = true;
+    for (Pass & p : passes) {
+        const int T = (int) p.tok.size(), W = (int) p.want.size();
+        const int tile_q = pm_attn_prefill_tile(T, hp.n_head);
+        struct Tile { int32_t row, n, pos, seq; };
+        std::vector<Tile> tl;
+        for (int r = 0; r < T;) {
+            int r1 = r + 1;
+            while (r1 < T && r1 - r < tile_q && p.seq[r1] == p.seq[r]) ++r1;
+            tl.push_back({r, r1 - r, p.pos[r], p.seq[r]});
+            r = r1;
+        }
+        std::stable_sort(tl.begin(), tl.end(), [](const Tile & a, const Tile & b) { return a.pos + a.n < b.pos + b.n; });      // (the kernel takes them from the end: most keys first)
+        std::stable_sort(p.want.begin(), p.want.end(), [](const Want & a, const Want & b) { return a.out < b.out; });
+        std::vector<int32_t> blk;
+        blk.reserve(12 * (size_t) T);
+        auto put = [&](const int32_t * v, size_t k) { const int at = (int) blk.size(); blk.insert(blk.end(), v, v + k); return at; };
+        put(p.tok.data(), T); const int at_pos = put(p.pos.data(), T), at_seq = put(p.seq.data(), T), at_tiles = put((const int32_t *) tl.data(), 4 * tl.size());
+        const int at_ent = put(p.ent.data(), p.ent.size()), at_want = (int) blk.size();
+        for (const Want & w : p.want) blk.push_back(w.row);
+        const int at_keep = put(p.keep.data(), p.keep.size());
+        const pm_batch_layout lay = {T, at_seq, at_ent, (int) p.ent.size() / 2, (int) blk.size()};
+        if (pm_launch_batch_rows(d_rows, blk.data(), lay, d_last, d_pos, d_ctl, st)) return seterr(m, PM355_E_HIP, "batch: table upload");
+        const Ragged r = {d_rows + at_pos, d_rows + at_seq, d_rows + at_tiles, (int) tl.size(), tile_q, p.max_cells, p.singles};
+        int rc;
+        if (T == 1) {                                                                                      // (one row is a step of its own, and that sequence's)
+            rc = decode(p.seq[0], d_rows, nullptr, 1, p.pos[0], W ? rows : nullptr, nullptr, nullptr, st);
+            if (!rc) rc = set_seq_pos(p.seq[0], p.pos[0] + 1, st);
+        } else {
+            rag = &r;
+            rc = run_window(m, d_rows, nullptr, T, W ? rows : nullptr, nullptr, nullptr, st);
+            rag = nullptr;
+        }
+        if (rc) return rc;
+        for (size_t k = 0; k < p.ent.size(); k += 2) h_pos[p.ent[k]] = p.ent[k + 1];
+        h_seq = p.ent[p.ent.size() - 2];
+        for (int w = 0; w < W;) {                                           // rows whose outputs are neighbours go through the head together
+            int w1 = w + 1;
+            while (w1 < W && w1 - w < std::min(max_tokens, HEAD_ROWS) && p.want[w1].out == p.want[w1 - 1].out + 1) ++w1;
+            const int k = w1 - w, o = p.want[w].out;
+            float * lg = d_logits ? d_logits + (size_t) o * V : head_lg;
+            if (k == 1) rc = run_head(m, rows + (size_t) p.want[w].row * hp.n_embd, lg, d_argmax ? d_argmax + o : nullptr, st);
+            else {
+                if (!output.d || !out_norm.d) return seterr(m, PM355_E_UNSUPPORTED, "head: output / output_norm missing");
+                const Tensor * ow[1] = {&output};
+                pm_launch_gather_rows(rows, d_rows + at_want + w, k, hp.n_embd, x1, st);
+                const ActQ a = norm_quantize_for(m, x1, (const float *) out_norm.d, hp.n_embd, k, ow, 1, st);
+                bool prepped = false;
+                if (matmul_small(m, output, a, k, lg, nullptr, nullptr, prepped, st)) return seterr(m, PM355_E_UNSUPPORTED, "head: lm_head mat-mul");
+                if (d_argmax) pm_launch_argmax(lg, V, d_argmax + o, nullptr, st, k);
+            }
+            if (rc) return rc;
+            w = w1;
+        }
+        if (!p.keep.empty()) pm_launch_keep_last(d_argmax, d_rows + at_keep, (int) p.keep.size() / 2, d_last, st);
+    }
+    return hip_ok() ? 0 : seterr(m, PM355_E_HIP, "batch: kernel launch failed");
+}
 int pm_window::batch(const pm355_batch_entry * e, int n, float * d_logits, int32_t * d_argmax, hipStream_t st) {
     pm_window * m = this;
     if (!finalized || !rows) return seterr(m, PM355_E_SHAPE, "batch: finalize_pool first");
@@ -1282,6 +1404,11 @@ int pm_window::batch(const pm355_batch_entry * e, int n, float * d_logits, int32
         for (int j = 0; j < i; ++j) if (e[j].seq == e[i].seq) return seterr(m, PM355_E_SHAPE, "batch: a sequence appears twice");
         for (int j = 0; j < e[i].n_want; ++j) if (e[i].want[j] < 0 || e[i].want[j] >= e[i].n_tokens) return seterr(m, PM355_E_RANGE, "batch: want outside the portion");
         for (int j = 0; e[i].tokens && j < e[i].n_tokens; ++j) if (e[i].tokens[j] < 0 || e[i].tokens[j] >= hp.n_vocab) return seterr(m, PM355_E_RANGE, "batch: token id outside the vocabulary");
+    }
+    if (n > 1) {
+        bool served = false;
+        const int rc = batch_rows(e, n, d_logits, d_argmax, st, &served);
+        if (served) return rc;
     }
     size_t row = 0;
     for (int i = 0; i < n; ++i) {

@@ -11,6 +11,7 @@
 //   add / silu_mul / scale / cpy  the elementwise nodes of build_llama (ggml.c:9002, :11581, :10077)
 // All are HBM/latency-bound byte movers; positions (pos) are read from DEVICE memory so that a captured
 // hipGraph can be replayed for every token without re-recording.
+#include <cstring>
 #include "pm355_device.h"
 #include "pm355_kernels.h"
 #include "pm355_layer_ops.h"
@@ -78,10 +79,10 @@ __global__ __launch_bounds__(64) void rope_kv_store_kernel(const float * q, cons
                                                            uint16_t * kc, uint16_t * vc,
                                                            const int32_t * pos0_ptr, const int32_t * seq_ptr, long seq_stride,
                                                            const float * freq_factors,
-                                                           int H, int Hkv, int dh, int n_ctx, RopeP r, int round_q) {
+                                                           int H, int Hkv, int dh, int n_ctx, RopeP r, int round_q, int rows) {
     const int head = blockIdx.x, t = blockIdx.y, lane = threadIdx.x;
-    const int seq = seq_ptr ? *seq_ptr : 0;              // multi-sequence: one KV slab and one position per sequence
-    const int pos = pos0_ptr[seq] + t;
+    const int seq = seq_ptr ? seq_ptr[rows ? t : 0] : 0;              // multi-sequence: one KV slab and one position per sequence (rows: both per token)
+    const int pos = rows ? pos0_ptr[t] : pos0_ptr[seq] + t;
     kc += (long) seq * seq_stride; vc += (long) seq * seq_stride;
     const bool is_q = head < H;
     const int hh = is_q ? head : head - H;
@@ -241,7 +242,8 @@ __global__ __launch_bounds__(256) void attn_rope_fused_kernel(AttnP a) {
 // ------------------------------------------------------------------------------------------------
 // argmax over n floats, first maximum wins. Single workgroup of 1024 threads.
 // ------------------------------------------------------------------------------------------------
-__global__ __launch_bounds__(1024) void argmax_kernel(const float * x, int n, int32_t * out_idx, float * out_val) {
+__global__ __launch_bounds__(1024) void argmax_kernel(const float * x, int n, int32_t * out_idx, float * out_val) {      // blockIdx.x: row of n
+    x += (size_t) blockIdx.x * n; out_idx += blockIdx.x;
     __shared__ float bv[16];
     __shared__ int bi[16];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -272,7 +274,7 @@ __global__ __launch_bounds__(1024) void argmax_kernel(const float * x, int n, in
         // nothing compared greater than -inf (every logit NaN or -inf): index 0, like llama_sampler_greedy's loop that starts from entry 0
         // (src/llama-sampling.cpp:390-397) - never an out-of-range id that the next step would use as an embedding row
         *out_idx = (idx < 0 || idx >= n) ? 0 : idx;
-        if (out_val) *out_val = best;
+        if (out_val) out_val[blockIdx.x] = best;
     }
 }
 
@@ -302,6 +304,24 @@ __global__ void advance_kernel(int32_t * pos, int32_t * ctl, int by, int rotate)
     if (rotate) ctl[0] = (s + rotate) % ctl[1];
 }
 __global__ void set_i32_kernel(int32_t * p, int v) { *p = v; }
+// The tables of a pass over rows of several sequences: integers that travel as kernel arguments (up to 960: no staging copy, nothing of the caller's outlives the call) or are in
+// place already, tokens that are taken from the device (-1: the sequence's last greedy token), and the sequences' positions behind the pass.
+struct BatchInts { int32_t v[960]; };
+__global__ __launch_bounds__(256) void batch_rows_kernel(BatchInts a, int n, int32_t * blk, pm_batch_layout l, const int32_t * last, int32_t * pos, int32_t * ctl) {
+    for (int i = threadIdx.x; i < n; i += 256) blk[i] = a.v[i];
+    __syncthreads();
+    for (int t = threadIdx.x; t < l.T; t += 256) if (blk[t] < 0) blk[t] = last[blk[l.seq + t]];
+    for (int i = threadIdx.x; i < l.n_entries; i += 256) pos[blk[l.entries + 2 * i]] = blk[l.entries + 2 * i + 1];
+    if (threadIdx.x == 0) ctl[0] = blk[l.entries + 2 * (l.n_entries - 1)];
+}
+__global__ __launch_bounds__(256) void gather_rows_kernel(const float * x, const int32_t * at, int K, float * y) {
+    const int i = (int) (blockIdx.x * 256 + threadIdx.x);
+    if (4 * i < K) *(float4 *) (y + (size_t) blockIdx.y * K + 4 * i) = *(const float4 *) (x + (size_t) at[blockIdx.y] * K + 4 * i);
+}
+__global__ __launch_bounds__(64) void keep_last_kernel(const int32_t * argmax, const int32_t * pairs, int n, int32_t * last) {      // pairs {sequence, row of argmax}
+    const int i = (int) (blockIdx.x * 64 + threadIdx.x);
+    if (i < n) last[pairs[2 * i]] = argmax[pairs[2 * i + 1]];
+}
 __global__ void set_i32x2_kernel(int32_t * p, int a, int b) { p[0] = a; p[1] = b; }
 
 // ---- launchers -------------------------------------------------------------------------------------
@@ -323,12 +343,12 @@ void pm_rope_params(pm_rope_cfg & c) {
 void pm_launch_rope_kv_store(const float * q, const float * k, const float * v, float * q_out, float * k_out_f32,
                              void * kc, void * vc, const int32_t * pos0, const int32_t * seq, long seq_stride,
                              const float * freq_factors,
-                             int n_tok, int H, int Hkv, int dh, int n_ctx, const pm_rope_cfg & c, hipStream_t st, int round_q) {
+                             int n_tok, int H, int Hkv, int dh, int n_ctx, const pm_rope_cfg & c, hipStream_t st, int round_q, int rows) {
     RopeP r;
     r.n_dims = c.n_dims; r.mode = c.mode; r.n_ctx_orig = c.n_ctx_orig; r.theta_scale = c.theta_scale;
     r.freq_scale = c.freq_scale; r.ext_factor = c.ext_factor; r.attn_factor = c.attn_factor; r.corr0 = c.corr0; r.corr1 = c.corr1;
     hipLaunchKernelGGL(rope_kv_store_kernel, dim3(H + Hkv, n_tok), dim3(64), 0, st,
-                       q, k, v, q_out, k_out_f32, (uint16_t *) kc, (uint16_t *) vc, pos0, seq, seq_stride, freq_factors, H, Hkv, dh, n_ctx, r, round_q);
+                       q, k, v, q_out, k_out_f32, (uint16_t *) kc, (uint16_t *) vc, pos0, seq, seq_stride, freq_factors, H, Hkv, dh, n_ctx, r, round_q, rows);
 }
 
 int pm_launch_attn_decode(const float * q, const void * kc, const void * vc, const int32_t * pos0,
@@ -372,8 +392,22 @@ int pm_launch_attn_rope_fused(const float * q, const float * k, const float * v,
     return 0;
 }
 
-void pm_launch_argmax(const float * x, int n, int32_t * idx, float * val, hipStream_t st) {
-    hipLaunchKernelGGL(argmax_kernel, dim3(1), dim3(1024), 0, st, x, n, idx, val);
+void pm_launch_argmax(const float * x, int n, int32_t * idx, float * val, hipStream_t st, int rows) {
+    hipLaunchKernelGGL(argmax_kernel, dim3(rows), dim3(1024), 0, st, x, n, idx, val);
+}
+int pm_launch_batch_rows(int32_t * blk, const int32_t * host, const pm_batch_layout & l, const int32_t * last, int32_t * pos, int32_t * ctl, hipStream_t st) {
+    BatchInts a;
+    const bool fits = l.n_ints <= (int) (sizeof(a.v) / 4);
+    if (fits) std::memcpy(a.v, host, (size_t) l.n_ints * 4);
+    else if (hipMemcpyAsync(blk, host, (size_t) l.n_ints * 4, hipMemcpyHostToDevice, st) != hipSuccess) return -1;
+    hipLaunchKernelGGL(batch_rows_kernel, dim3(1), dim3(256), 0, st, a, fits ? l.n_ints : 0, blk, l, last, pos, ctl);
+    return 0;
+}
+void pm_launch_gather_rows(const float * x, const int32_t * at, int n, int K, float * y, hipStream_t st) {
+    hipLaunchKernelGGL(gather_rows_kernel, dim3((K / 4 + 255) / 256, n), dim3(256), 0, st, x, at, K, y);
+}
+void pm_launch_keep_last(const int32_t * argmax, const int32_t * pairs, int n, int32_t * last, hipStream_t st) {
+    hipLaunchKernelGGL(keep_last_kernel, dim3((n + 63) / 64), dim3(64), 0, st, argmax, pairs, n, last);
 }
 void pm_launch_add(const float * a, const float * b, float * y, long n, long nb, hipStream_t st) {
     hipLaunchKernelGGL(add_kernel, dim3((unsigned) ((n + 255) / 256)), dim3(256), 0, st, a, b, y, n, nb);

@@ -65,7 +65,7 @@ struct MmqP {
     // F16-rounded f32 into its y, k -> the F16 K-cache row of cell pos + t, v -> the transposed F16 V cache - what rope_kv_store_kernel (layer_ops.hip) does in a
     // launch of its own, the same expressions (ggml_compute_forward_rope_f32 ggml.c:14224-14237; llm_build_kv_store src/llama.cpp:9688-9716).
     // e_role[j]: 1 q, 2 k, 3 v (single-job launches: e_role[0]). Workgroup row slices start on even rows then.
-    int e_on, e_role[3]; const float * e_tab; const int32_t * e_pos, * e_seq; long e_seq_stride; uint16_t * e_kc, * e_vc; int e_dh, e_nctx, e_nrot, e_kvdim;
+    int e_on, e_role[3]; const float * e_tab; const int32_t * e_pos, * e_seq; long e_seq_stride; uint16_t * e_kc, * e_vc; int e_dh, e_nctx, e_nrot, e_kvdim, e_rows;   // e_rows: e_pos[t], e_seq[t] per token
 };
 
 __device__ __forceinline__ long pk(uint32_t a, uint32_t b) { return (long) (((uint64_t) b << 32) | a); }
@@ -554,8 +554,8 @@ __device__ __forceinline__ void mmq_i8_body(const MmqP & p, const int w, const i
                 const float sp = __shfl_xor(s, 1);                      // the pair's other row: the neighbouring lane (r0 even), same token
                 if (live) {
                     const int role = j == 0 ? p.e_role[0] : j == 1 ? p.e_role[1] : p.e_role[2];
-                    const int seq = p.e_seq ? *p.e_seq : 0;
-                    const int pos = p.e_pos[seq] + t;
+                    const int seq = p.e_seq ? p.e_seq[p.e_rows ? t : 0] : 0;
+                    const int pos = p.e_rows ? p.e_pos[t] : p.e_pos[seq] + t;
                     const long kv_off = (long) seq * p.e_seq_stride;
                     if (role == 3) p.e_vc[kv_off + (long) lr * p.e_nctx + pos] = f2h(s);
                     else {
@@ -868,7 +868,7 @@ bool fill_epi(MmqP & p, const pm_qkv_epi * e, int r0, int r1, int r2) {
     if (e->neox || e->v_rowmajor || e->dyn || !e->tab || !e->pos || !e->kc || !e->vc || e->dh < 2 || (e->dh & 1) || (e->n_rot & 1)) return false;
     p.e_on = 1; p.e_role[0] = r0; p.e_role[1] = r1; p.e_role[2] = r2;
     p.e_tab = e->tab; p.e_pos = e->pos; p.e_seq = e->seq; p.e_seq_stride = e->seq_stride; p.e_kc = (uint16_t *) e->kc; p.e_vc = (uint16_t *) e->vc;
-    p.e_dh = e->dh; p.e_nctx = e->n_ctx; p.e_nrot = e->n_rot; p.e_kvdim = e->Hkv * e->dh;
+    p.e_dh = e->dh; p.e_nctx = e->n_ctx; p.e_nrot = e->n_rot; p.e_kvdim = e->Hkv * e->dh; p.e_rows = e->rows;
     return true;
 }
 }  // namespace

@@ -94,6 +94,7 @@ struct pm_qkv_epi {
     // attention launch and its boundary disappear. att_ticket: Hkv counters (zeroed once, monotonic), att_err: watchdog word (a bounded wait gave up).
     // Position-pointer mode only (pos != null, dyn == null); -7 when the shape is not served (then launch pm_launch_attn_cached as before)
     float * att_out; unsigned * att_ticket; int * att_err; float kq_scale; int n_head, att_max_keys;
+    int rows;                           // small batches: pos[t] and seq[t] are token t's
 };
 struct pm_gemv_fused {
     int K; int njobs;

@@ -16,7 +16,7 @@ void pm_launch_rope_kv_store(const float * q, const float * k, const float * v, 
                              void * kc, void * vc, const int32_t * pos0, const int32_t * seq, long seq_stride,
                              const float * freq_factors,
                              int n_tok, int H, int Hkv, int dh, int n_ctx, const pm_rope_cfg & c, hipStream_t st,
-                             int round_q = 0);       // q_out rounded to F16 (what MUL_MAT(k, q) does to its src1): the form pm_launch_attn_cached reads
+                             int round_q = 0, int rows = 0);       // rows: pos0[t] and seq[t] are token t's. round_q: q_out rounded to F16 (what MUL_MAT(k, q) does to its src1): the form pm_launch_attn_cached reads
 int  pm_launch_attn_decode(const float * q, const void * kc, const void * vc, const int32_t * pos0,
                            const int32_t * seq, long seq_stride, float * out,
                            int n_tok, int H, int Hkv, int dh, int n_ctx, float scale, hipStream_t st);
@@ -44,7 +44,9 @@ int  pm_launch_attn_prefill(const float * q, const void * kc, const void * vc, c
                             long seq_stride, float * out, int n_tok, int H, int Hkv, int dh, int n_ctx, float scale, hipStream_t st,
                             const float * mask = nullptr, long mask_stride = 0, int n_kv = 0,   // mask != null: ggml-graph mode (cells [0, n_kv) + additive mask row per token)
                             int v_rowmajor = 0, int mask_f16 = 0,                              // flash-attention graphs: row-major V cache, F16 mask rows
-                            void * out_f16 = nullptr);                                         // result as F16 (activations of the wo GEMM) instead of `out`
+                            void * out_f16 = nullptr,                                          // result as F16 (activations of the wo GEMM) instead of `out`
+                            const int32_t * tiles = nullptr, int n_tiles = 0, int tile_q = 0);  // device int32 {row, queries, position, sequence} per tile of up to tile_q queries
+int  pm_attn_prefill_tile(int n_tok, int H);      // queries per tile for a batch of this size: 64, 128 or 256
 int  pm_launch_attn_rope_fused(const float * q, const float * k, const float * v, void * kc, void * vc,
                                 const int32_t * pos0, const int32_t * seq, long seq_stride, const float * freq_factors,
                                 float * out, int H, int Hkv, int dh, int n_ctx, float scale, const pm_rope_cfg & c, hipStream_t st,
@@ -53,11 +55,11 @@ int  pm_launch_attn_rope_fused(const float * q, const float * k, const float * v
 // (tab[2 i], tab[2 i + 1] for rotation pair i; position = pos[seq ? *seq : 0]) and the attention over cells that are all cached
 // (q = rotated, F16-rounded; attn_cached.hip). Remaining arguments as pm_launch_attn_rope_fused.
 void pm_launch_rope_table(const pm_rope_cfg & c, const int32_t * pos, const int32_t * seq, const float * freq_factors, float * tab, hipStream_t st,
-                          int n_tok = 1);    // n_tok > 1: tables of the tokens pos .. pos + n_tok - 1, n_dims floats each
+                          int n_tok = 1, int rows = 0);    // n_tok > 1: tables of the tokens pos .. pos + n_tok - 1 (rows: pos[t]), n_dims floats each
 int  pm_launch_attn_cached(const float * q, void * kc, void * vc, const int32_t * pos0, const int32_t * seq, long seq_stride, float * out,
                            int H, int Hkv, int dh, int n_ctx, float scale, hipStream_t st, const int32_t * dyn = nullptr,
                            const void * mask = nullptr, int max_keys = 0, int v_rowmajor = 0, int mask_f16 = 0,
-                           int n_tok = 1);          // n_tok > 1 (engine mode): token t of a small batch attends cells [0, pos0 + t], q / out rows t
+                           int n_tok = 1, int rows = 0);    // n_tok > 1 (engine mode): token t of a small batch attends cells [0, pos0 + t] (rows: [0, pos0[t]] of sequence seq[t]), q / out rows t
 // ggml-graph mode of the two launchers above: dyn = device int32[2] {cache cell the token is stored in, cells attended}, the RoPE
 // position is pos0[0], mask = additive KQ-mask row [cells attended] (f32, or F16 with mask_f16) or null; v_rowmajor = the V cache is
 // [n_ctx][n_embd_v_gqa] (flash-attention graphs) instead of transposed, with flash-attention rounding points; max_keys (> 0) sizes the fused kernel's LDS score
@@ -72,7 +74,12 @@ int  pm_launch_q8_token_prep(const float * q, const float * k, const float * v, 
 int  pm_launch_attn_q8_token(const float * q, const float * k, const float * v, void * kc, void * vc, const int32_t * pos, const int32_t * dyn,
                              const void * mask, int mask_f16, const float * ff, float * out, int H, int Hkv, int dh, int n_ctx, float scale,
                              const pm_rope_cfg & c, int k_q8, int v_q8, int max_keys, hipStream_t st);
-void pm_launch_argmax(const float * x, int n, int32_t * idx, float * val, hipStream_t st);
+void pm_launch_argmax(const float * x, int n, int32_t * idx, float * val, hipStream_t st, int rows = 1);
+// a pass over T rows of several sequences: block of int32 = tokens [T] | positions [T] | sequences [T] | ... ; offsets in integers. entries: {sequence, position behind the pass}
+struct pm_batch_layout { int T, seq, entries, n_entries, n_ints; };
+int  pm_launch_batch_rows(int32_t * blk, const int32_t * host, const pm_batch_layout & l, const int32_t * last, int32_t * pos, int32_t * ctl, hipStream_t st);
+void pm_launch_gather_rows(const float * x, const int32_t * at, int n, int K, float * y, hipStream_t st);                  // y[i] = x[at[i]], K % 4 == 0
+void pm_launch_keep_last(const int32_t * argmax, const int32_t * pairs, int n, int32_t * last, hipStream_t st);             // last[pairs[i].sequence] = argmax[pairs[i].row]
 void pm_launch_add(const float * a, const float * b, float * y, long n, long nb, hipStream_t st);
 void pm_launch_mul(const float * a, const float * b, float * y, long n, long nb, hipStream_t st);
 void pm_launch_silu_mul(const float * g, const float * u, float * y, long n, hipStream_t st);

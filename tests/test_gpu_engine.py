@@ -462,3 +462,52 @@ def test_attention_tail_decode_is_bit_identical(E, monkeypatch, arch):
         w.close()
     for i, ((h0, l0), (h1, l1)) in enumerate(zip(*outs)):
         assert np.array_equal(h0, h1) and np.array_equal(l0, l1), i
+
+
+@pytest.mark.parametrize("arch,max_tokens,n_ctx", [(0, 64, 96), (1, 64, 96), (0, 7, 64), (0, 40, 288), (0, 2, 64), (0, 64, 72)])
+def test_batches_of_several_sequences_equal_one_sequence_at_a_time(E, arch, max_tokens, n_ctx):
+    """pm355_model_batch over several sequences runs their rows in common passes: prompts of unequal length (single tokens, odd ones, longer than 32 - the 16-bit arithmetic -, cut by
+    max_tokens), decoded tokens taken on the device, rows wanted out of order, twice or not at all; behind 192 cells the attention changes kernels; n_ctx = 72 takes the sequences one by
+    one. Against the same portions given alone: the same arithmetic with other summation orders, so 8-bit roundings may turn (the bound of the oracle comparisons above)."""
+    torch = E.torch
+    rng = np.random.default_rng(7 + max_tokens)
+    d = tiny_model(rng, arch=arch, n_layer=2, n_embd=256, n_head=4, n_head_kv=2, n_ff=512, n_vocab=320, n_ctx=n_ctx, rope_freqs=arch == 0)
+    lens = [1, 3, 17, 38, 5] if n_ctx < 200 else [200, 3, 17, 38, 190]
+    ws = []
+    for _ in range(2):
+        w = E.Window(_hp(d), n_ctx=n_ctx)
+        w.load_desc(d)
+        w.finalize_pool(max_tokens, len(lens), len(lens) * n_ctx)
+        ws.append((w, [w.seq_new() for _ in lens]))
+    (w, seqs), (w1, seqs1) = ws
+    toks = [rng.integers(0, 320, n + 8).astype(np.int32) for n in lens]
+    steps = [[(i, toks[i][:n], [n - 1] if i != 2 else [n - 1, 0, n - 1]) for i, n in enumerate(lens)],
+             [(4, None, [0]), (0, toks[0][lens[0]:lens[0] + 2], []), (3, None, [0]), (1, toks[1][3:4], [0])],
+             [(2, None, [0]), (4, None, [0])],
+             [(0, toks[0][:1], [0]), (1, None, [0]), (2, toks[2][:1], [0]), (3, toks[3][:1], [0])],
+             [(3, None, [0])]]
+    last = {}
+    for entries in steps:
+        rows = sum(len(x[2]) for x in entries)
+        lg, am = torch.full((rows, 320), float("nan"), device="cuda"), torch.full((rows,), -1, dtype=torch.int32, device="cuda")
+        w.batch([(seqs[i], t, want) for i, t, want in entries], logits=lg, argmax=am)
+        lg1, at = torch.empty((rows, 320), device="cuda"), 0
+        for i, t, want in entries:
+            w1.batch([(seqs1[i], np.array([last[i]], dtype=np.int32) if t is None else t, want)], logits=lg1[at:at + len(want)], argmax=None)
+            at += len(want)
+            if want:
+                last[i] = int(am[at - 1])
+        a, b = lg.double().cpu().numpy(), lg1.double().cpu().numpy()
+        assert (am.cpu().numpy() == a.argmax(-1)).all()
+        for r in range(rows):
+            assert ((a[r] - b[r]) ** 2).sum() < 1e-3 * (b[r] ** 2).sum(), (r, ((a[r] - b[r]) ** 2).sum() / (b[r] ** 2).sum())
+        assert [w.seq_len(s) for s in seqs] == [w1.seq_len(s) for s in seqs1]
+    # the device's own counters are where the sequences are: a single step behind the batches
+    tok, out, out1 = torch.tensor([5], dtype=torch.int32, device="cuda"), torch.empty(320, device="cuda"), torch.empty(320, device="cuda")
+    for m, s, o in ((w, seqs, out), (w1, seqs1, out1)):
+        m.set_seq(s[1])
+        m.step(token=tok, logits=o)
+    a, b = out.double().cpu().numpy(), out1.double().cpu().numpy()
+    assert ((a - b) ** 2).sum() < 1e-3 * (b ** 2).sum()
+    w.close()
+    w1.close()
