@@ -109,6 +109,8 @@ struct pm_window : pm355_model {
     // a pass over rows of several sequences (batch): every row's position and sequence in device memory, tiles for the matrix-core attention; rag is set while one is launched
     struct Ragged { const int32_t * pos, * seq, * tiles; int n_tiles, tile_q, max_cells; bool singles; };
     const Ragged * rag = nullptr; int32_t * d_rows = nullptr; float * head_lg = nullptr;
+    uint64_t * am_part = nullptr;                 // argmax scratch of up to HEAD_ROWS rows
+    int adv = 0, rot = 0;                         // what the launch that ends a step still does to the position counters (step_body; the argmax does it on its way)
     int batch_rows(const pm355_batch_entry * e, int n, float * d_logits, int32_t * d_argmax, hipStream_t st, bool * served);
 
     ~pm_window() override;
@@ -403,7 +405,10 @@ int run_head(pm_window * m, const float * x_row, float * d_logits, int32_t * d_a
         ActQ a = norm_quantize_for(m, x_row, (const float *) m->out_norm.d, m->hp.n_embd, 1, ow, 1, st);
         if (gemv(m->output, nullptr, a, 1, lg, nullptr, nullptr, st)) return seterr(m, PM355_E_UNSUPPORTED, "head: lm_head gemv");
     }
-    if (d_argmax) pm_launch_argmax(lg, m->hp.n_vocab, d_argmax, nullptr, st);
+    if (d_argmax) {
+        pm_launch_argmax(lg, m->hp.n_vocab, d_argmax, nullptr, st, 1, m->am_part, m->adv || m->rot ? m->d_pos : nullptr, m->d_ctl, m->adv, m->rot);
+        m->adv = m->rot = 0;
+    }
     return 0;
 }
 
@@ -507,7 +512,7 @@ int attn_regime(const pm_window * m) {
     return (int) (b > m->hp.n_ctx ? m->hp.n_ctx : b);
 }
 
-// the single-token layer sequence (5 launches per layer)
+// the single-token layer sequence (5 launches per layer); the token's cos / sin table is there (m->rope_tab) where the window has one
 // *n_ss_end: number of partials the LAST layer's ffn_down left in m->ss + 256 for the sum of squares of the window's output row (0: none)
 int run_layers_fused(pm_window * m, const float * cur, float * d_x_out, const float ** cur_out, hipStream_t st, int * n_ss_end = nullptr) {
     const pm355_hparams & hp = m->hp;
@@ -518,7 +523,6 @@ int run_layers_fused(pm_window * m, const float * cur, float * d_x_out, const fl
     // (NEOX rope - build_qwen2 - where every workgroup's slice of wq / wk holds both halves of its rotation pairs: pm_launch_gemv_fused tells)
     bool epi = m->qkv_epi && m->rope_tab && (m->rope.mode == 0 || m->rope.mode == 2) &&
                (!m->long_ctx || (m->use_flash && m->attn_mfma && H / Hkv <= 8 && pm_attn_flash_cached_ok(H, Hkv, dh, hp.n_ctx) == 0));
-    if (epi) pm_launch_rope_table(m->rope, m->d_pos, m->d_ctl, (const float *) m->rope_freqs.d, m->rope_tab, st);
     bool tail = epi && !m->long_ctx && m->attn_tail && m->att_tk && Hkv <= 64;
     double * ss_wo = (m->use_ss && m->ss) ? m->ss : nullptr, * ss_dn = ss_wo ? m->ss + 256 : nullptr;
     int n_wo = 0, n_dn = 0;                           // partials the previous wo / ffn_down launch left (0: the consumer reduces the row itself)
@@ -634,7 +638,6 @@ int run_window(pm_window * m, const int32_t * d_tokens, const float * d_x_in, in
     const float * cur = d_x_in;
     if (d_tokens) {
         if (!(m->flags & PM355_HAS_EMBD) || !m->tok_embd.d) return seterr(m, PM355_E_UNSUPPORTED, "decode: tokens given but window has no tok_embd");
-        pm_launch_embed(m->tok_embd.type, m->tok_embd.d, E, d_tokens, T, m->x, st);
         cur = m->x;
     }
     if (!cur) return seterr(m, PM355_E_SHAPE, "decode: neither tokens nor x_in");
@@ -661,7 +664,10 @@ int run_window(pm_window * m, const int32_t * d_tokens, const float * d_x_in, in
         const int rc = pm_launch_attn_cached(m->q, L.kc, L.vc, d_pos, d_seq, kv_stride, m->att, H, Hkv, dh, hp.n_ctx, kq_scale, st, nullptr, nullptr, rg ? rg->max_cells : 0, 0, 0, T, rg ? 1 : 0);
         return rc && !rg ? pm_launch_attn_decode(m->q, L.kc, L.vc, d_pos, d_seq, kv_stride, m->att, T, H, Hkv, dh, hp.n_ctx, kq_scale, st) : rc;
     };
-    if (small_epi) pm_launch_rope_table(m->rope, d_pos, d_seq, (const float *) m->rope_freqs.d, m->rope_tab, st, T, rg ? 1 : 0);
+    // the tokens' rows, and with them the cos / sin tables that the wq | wk | wv epilogues of all layers read
+    const bool one = T == 1 && !m->no_fuse, tab = (one ? m->qkv_epi && m->rope_tab : small_epi) && m->hi > m->lo;
+    if (d_tokens) pm_launch_embed(m->tok_embd.type, m->tok_embd.d, E, d_tokens, T, m->x, st, &m->rope, d_pos, d_seq, (const float *) m->rope_freqs.d, tab ? m->rope_tab : nullptr, rg ? 1 : 0);
+    else if (tab) pm_launch_rope_table(m->rope, d_pos, d_seq, (const float *) m->rope_freqs.d, m->rope_tab, st, T, rg ? 1 : 0);
     if (T == 1 && !m->no_fuse) {
         m->flash_cells = attn_regime(m); m->long_ctx = m->flash_cells != 0;
         // ---- single token: every activation transform is fused into a mat-vec prologue / epilogue, 5 launches per layer
@@ -674,7 +680,6 @@ int run_window(pm_window * m, const int32_t * d_tokens, const float * d_x_in, in
         }
         if (eng) {
             // ---- ... or, where served, ALL layers as one persistent launch (decode_engine.hip): cos / sin table, the first norm's sum of squares, the engine
-            pm_launch_rope_table(m->rope, m->d_pos, m->d_ctl, (const float *) m->rope_freqs.d, m->rope_tab, st);
             pm_launch_sumsq_row(cur, E, eng->ss_in0, st);
 #if PM_EXPERIMENTS
             if (pm_eng_plan_launch(eng->plan, st)) return seterr(m, PM355_E_HIP, "decode: engine launch");
@@ -950,7 +955,7 @@ pm_window::~pm_window() {
     for (auto & L : m->layers) { for (auto & t : L.t) if (t.d) (void) hipFree(t.d); if (L.kc) (void) hipFree(L.kc); if (L.vc) (void) hipFree(L.vc); }
     Tensor * g[4] = {&m->tok_embd, &m->out_norm, &m->output, &m->rope_freqs};
     for (auto t : g) if (t->d) (void) hipFree(t->d);
-    void * s[] = {m->x, m->x1, m->q, m->k, m->v, m->att, m->h, m->h2, m->logits, m->xn, m->aq_k, m->aq_0, m->d_pos, m->d_tok, m->d_ctl, m->split_scratch, m->rope_tab, m->tab_big, m->ss, m->att_tk, m->d_last, m->rows, m->d_rows, m->head_lg};
+    void * s[] = {m->x, m->x1, m->q, m->k, m->v, m->att, m->h, m->h2, m->logits, m->xn, m->aq_k, m->aq_0, m->d_pos, m->d_tok, m->d_ctl, m->split_scratch, m->rope_tab, m->tab_big, m->ss, m->att_tk, m->d_last, m->rows, m->d_rows, m->head_lg, m->am_part};
     for (auto p : s) if (p) (void) hipFree(p);
     pm355_uploader_free(m->up);
     if (m->cap_stream) (void) hipStreamDestroy(m->cap_stream);
@@ -1056,7 +1061,8 @@ int pm_window::finalize(int max_tokens_, int n_seq_) {
               A((void **) &m->rope_tab, (size_t) hp.head_dim * 4 * 32) &&      // cos / sin tables of up to 32 tokens (small-batch epilogue)
               A((void **) &m->ss, 2 * 256 * sizeof(double)) &&
               A((void **) &m->att_tk, 65 * 4) && A((void **) &m->d_last, 64 * 4);
-    if (ok) (void) hipMemset(m->att_tk, 0, 65 * 4);
+    ok = ok && A((void **) &m->am_part, PM_ARGMAX_SCRATCH);
+    if (ok) { (void) hipMemset(m->att_tk, 0, 65 * 4); (void) hipMemset(m->am_part, 0, PM_ARGMAX_SCRATCH); }
     if (ok && T > MMQ_MAX_TOKENS && !m->no_big) ok = A((void **) &m->tab_big, pm_mmq_big_table_bytes((int) ((maxK + 255) / 256 * 256), (int) T));
     if (!ok) return seterr(m, PM355_E_NOMEM, "finalize: scratch");
     if (hp.n_head / hp.n_head_kv <= 8 && (hp.head_dim == 64 || hp.head_dim == 128) &&
@@ -1126,8 +1132,8 @@ int pm_window::set_seq_pos(int seq, int pos, hipStream_t st) {
     if (seq >= m->n_seq) return seterr(m, PM355_E_RANGE, "set_seq_pos: seq >= n_seq");
     if (pos < 0 || pos > m->hp.n_ctx) return seterr(m, PM355_E_RANGE, "set_seq_pos: position outside [0, n_ctx]");
     // values travel as kernel arguments: capture-safe, no host buffer lifetime to manage
-    if (seq < 0) { pm_launch_set_i32(m->d_ctl, 0, (hipStream_t) st); seq = 0; m->h_seq = 0; }
-    pm_launch_set_i32(m->d_pos + seq, pos, (hipStream_t) st);
+    if (seq < 0) { seq = 0; m->h_seq = 0; pm_launch_set_i32_pair(m->d_ctl, 0, m->d_pos, pos, (hipStream_t) st); }
+    else pm_launch_set_i32(m->d_pos + seq, pos, (hipStream_t) st);
     m->h_pos[seq] = pos;
     return 0;
 }
@@ -1153,9 +1159,10 @@ int pm_window::decode(int seq, const int32_t * d_tokens, const float * d_x_in, i
     if (!m->finalized) return seterr(m, PM355_E_SHAPE, "decode: model not finalized");
     if (T < 1 || T > m->max_tokens) return seterr(m, PM355_E_RANGE, "decode: n_tokens exceeds finalize(max_tokens)");
     if (pos0 < 0 || pos0 + T > m->hp.n_ctx) return seterr(m, PM355_E_RANGE, "decode: position outside n_ctx");
-    int rc = set_seq_pos(seq, pos0, st);
-    if (!rc && seq >= 0) rc = set_seq(seq, st);
-    if (rc) return rc;
+    if (seq >= m->n_seq) return seterr(m, PM355_E_RANGE, "decode: bad sequence id");
+    const int s = seq < 0 ? 0 : seq;
+    pm_launch_set_i32_pair(m->d_ctl, s, m->d_pos + s, pos0, st);
+    m->h_pos[s] = pos0; m->h_seq = s;
     return run_window(m, d_tokens, d_x_in, T, d_x_out, d_logits, d_argmax, st);
 }
 extern "C" int pm355_small_batch_max_tokens(void) { return MMQ_MAX_TOKENS; }
@@ -1171,7 +1178,11 @@ static int step_body(pm_window * m, const int32_t * d_token, const float * d_x_i
         if (rc) return rc;
         rc = run_window(m, d_token, nullptr, 1, d_x_out, nullptr, nullptr, st);
     } else {
+        m->adv = advance; m->rot = rotate;
         rc = run_window(m, d_token, d_token ? nullptr : d_x_in, 1, d_x_out, d_logits, d_argmax, st);
+        const bool done = (advance || rotate) && !m->adv && !m->rot;          // (the argmax launch moved them)
+        m->adv = m->rot = 0;
+        if (rc || done) return rc;
     }
     if (rc) return rc;
     if (advance || rotate) pm_launch_advance(m->d_pos, m->d_ctl, advance, rotate, st);
@@ -1385,7 +1396,7 @@ int pm_window::batch_rows(const pm355_batch_entry * e, int n, float * d_logits, 
                 const ActQ a = norm_quantize_for(m, x1, (const float *) out_norm.d, hp.n_embd, k, ow, 1, st);
                 bool prepped = false;
                 if (matmul_small(m, output, a, k, lg, nullptr, nullptr, prepped, st)) return seterr(m, PM355_E_UNSUPPORTED, "head: lm_head mat-mul");
-                if (d_argmax) pm_launch_argmax(lg, V, d_argmax + o, nullptr, st, k);
+                if (d_argmax) pm_launch_argmax(lg, V, d_argmax + o, nullptr, st, k, am_part);
             }
             if (rc) return rc;
             w = w1;

@@ -11,10 +11,12 @@
 //   add / silu_mul / scale / cpy  the elementwise nodes of build_llama (ggml.c:9002, :11581, :10077)
 // All are HBM/latency-bound byte movers; positions (pos) are read from DEVICE memory so that a captured
 // hipGraph can be replayed for every token without re-recording.
+#include <algorithm>
 #include <cstring>
 #include "pm355_device.h"
 #include "pm355_kernels.h"
 #include "pm355_layer_ops.h"
+#include "attn_device.h"
 
 // ------------------------------------------------------------------------------------------------
 // generic element dequantization from the HBM layouts (slow path: embedding row lookup only)
@@ -57,12 +59,27 @@ __device__ float pm_dequant_elem(int type, const uint8_t * row, int K, int i) {
     return 0.0f;
 }
 
-__global__ __launch_bounds__(256) void embed_rows_kernel(int type, const uint8_t * table, long row_bytes, int K,
-                                                         const int32_t * tokens, int n_tok, float * out) {
+// The rows of a batch's tokens, four values per thread. tab != null: the grid has a column of workgroups more, which write the tokens' (cos, sin) tables
+// (pm_launch_rope_table) - two launches of ~4.5 us at the front of a decoded token whose work is a microsecond become one.
+__global__ __launch_bounds__(256) void embed_rows_kernel(int type, const uint8_t * table, long row_bytes, int K, const int32_t * tokens, float * out,
+                                                         RopeP r, const int32_t * pos_ptr, const int32_t * seq_ptr, const float * freq_factors, float * tab, int rows) {
     const int t = blockIdx.y;
-    const int i = blockIdx.x * 256 + threadIdx.x;
-    if (t >= n_tok || i >= K) return;
-    out[(long) t * K + i] = pm_dequant_elem(type, table + (long) tokens[t] * row_bytes, K, i);
+    if (tab && blockIdx.x == gridDim.x - 1) {
+        const int pos = rows ? pos_ptr[t] : pos_ptr[seq_ptr ? *seq_ptr : 0] + t;
+        for (int pair = threadIdx.x; pair < r.n_dims / 2; pair += 256) {
+            float c, s;
+            rope_cs(r, (float) pos, pair, freq_factors, c, s);
+            tab[(size_t) t * r.n_dims + 2 * pair] = c; tab[(size_t) t * r.n_dims + 2 * pair + 1] = s;
+        }
+        return;
+    }
+    const int i = 4 * (int) (blockIdx.x * 256 + threadIdx.x);
+    if (i >= K) return;
+    const uint8_t * row = table + (long) tokens[t] * row_bytes;
+    float * o = out + (long) t * K + i;
+    if ((K & 3) == 0 && ((uintptr_t) out & 15) == 0)
+        *(float4 *) o = float4{pm_dequant_elem(type, row, K, i), pm_dequant_elem(type, row, K, i + 1), pm_dequant_elem(type, row, K, i + 2), pm_dequant_elem(type, row, K, i + 3)};
+    else for (int e = 0; e < 4 && i + e < K; ++e) o[e] = pm_dequant_elem(type, row, K, i + e);
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -70,8 +87,6 @@ __global__ __launch_bounds__(256) void embed_rows_kernel(int type, const uint8_t
 // theta is built by the reference's running product (theta *= theta_scale per pair) so that the f32
 // rounding sequence is identical; cosf/sinf are the device libm (<= 2 ulp from glibc).
 // ------------------------------------------------------------------------------------------------
-#include "attn_device.h"
-
 // q: [n_tok][H*dh] f32 (rotated in place into q_out), k: [n_tok][Hkv*dh], v: [n_tok][Hkv*dh]
 // K cache: f16 [n_ctx][Hkv*dh]; V cache: f16 [Hkv*dh][n_ctx] (transposed, as in the reference without flash-attn)
 __global__ __launch_bounds__(64) void rope_kv_store_kernel(const float * q, const float * k, const float * v,
@@ -240,10 +255,15 @@ __global__ __launch_bounds__(256) void attn_rope_fused_kernel(AttnP a) {
 }
 
 // ------------------------------------------------------------------------------------------------
-// argmax over n floats, first maximum wins. Single workgroup of 1024 threads.
+// argmax over n floats, first maximum wins. Workgroups of 1024 threads: one, or (part != null) gridDim.x per row whose results meet in the last one to arrive. One workgroup over
+// the 128256 logits of the Llama-3 vocabulary is bound by its own loads in flight: 15.3 us; thirty-two take 5.8. The last one also moves the step's position counters
+// (pos != null): a launch of one thread less per token.
 // ------------------------------------------------------------------------------------------------
-__global__ __launch_bounds__(1024) void argmax_kernel(const float * x, int n, int32_t * out_idx, float * out_val) {      // blockIdx.x: row of n
-    x += (size_t) blockIdx.x * n; out_idx += blockIdx.x;
+__global__ __launch_bounds__(1024) void argmax_kernel(const float * x, int n, int32_t * out_idx, float * out_val, uint64_t * part, int32_t * pos, int32_t * ctl, int by, int rotate) {
+    const int row = blockIdx.y, nb = gridDim.x, n_all = n;
+    x += (size_t) row * n; out_idx += row;
+    const int per = ((n + nb - 1) / nb + 3) & ~3, x0 = min((int) blockIdx.x * per, n);           // this workgroup's values [x0, x0 + n)
+    x += x0; n = min(per, n - x0);
     __shared__ float bv[16];
     __shared__ int bi[16];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -269,12 +289,38 @@ __global__ __launch_bounds__(1024) void argmax_kernel(const float * x, int n, in
     }
     if (lane == 0) { bv[wave] = best; bi[wave] = idx; }
     __syncthreads();
-    if (tid == 0) {
-        for (int w = 1; w < 16; ++w) if (bv[w] > best || (bv[w] == best && bi[w] < idx)) { best = bv[w]; idx = bi[w]; }
+    if (wave) return;
+    if (lane < 16) { best = bv[lane]; idx = bi[lane] == 0x7fffffff ? bi[lane] : bi[lane] + x0; } else { best = -INFINITY; idx = 0x7fffffff; }
+    auto across = [&]() __attribute__((always_inline)) {
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) { const float ov = __shfl_xor(best, off); const int oi = __shfl_xor(idx, off); take(ov, oi); }
+    };
+    across();
+    if (nb > 1) {
+        // partial results out (value | index), then a ticket (in front of the partials); the last workgroup of the row merges and re-arms it
+        unsigned * ticket = (unsigned *) part + row;
+        part += PM_ARGMAX_ROWS / 2 + (size_t) row * nb;
+        int last = 0;
+        if (lane == 0) {
+            __hip_atomic_store(part + blockIdx.x, (uint64_t) __float_as_uint(best) << 32 | (uint32_t) idx, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            last = __hip_atomic_fetch_add(ticket, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) == (unsigned) nb - 1;
+        }
+        if (!__shfl(last, 0)) return;
+        const uint64_t v = lane < nb ? __hip_atomic_load(part + lane, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : (uint64_t) 0xff800000u << 32 | 0x7fffffffu;
+        best = __uint_as_float((uint32_t) (v >> 32)); idx = (int) (uint32_t) v;
+        across();
+        if (lane == 0) __hip_atomic_store(ticket, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    if (lane == 0) {
         // nothing compared greater than -inf (every logit NaN or -inf): index 0, like llama_sampler_greedy's loop that starts from entry 0
         // (src/llama-sampling.cpp:390-397) - never an out-of-range id that the next step would use as an embedding row
-        *out_idx = (idx < 0 || idx >= n) ? 0 : idx;
-        if (out_val) out_val[blockIdx.x] = best;
+        *out_idx = (idx < 0 || idx >= n_all) ? 0 : idx;
+        if (out_val) out_val[row] = best;
+        if (pos) {
+            const int s = ctl[0];
+            pos[s] += by;
+            if (rotate) ctl[0] = (s + rotate) % ctl[1];
+        }
     }
 }
 
@@ -322,12 +368,19 @@ __global__ __launch_bounds__(64) void keep_last_kernel(const int32_t * argmax, c
     const int i = (int) (blockIdx.x * 64 + threadIdx.x);
     if (i < n) last[pairs[2 * i]] = argmax[pairs[2 * i + 1]];
 }
+__global__ void set_i32_pair_kernel(int32_t * p, int a, int32_t * q, int b) { *p = a; *q = b; }
 __global__ void set_i32x2_kernel(int32_t * p, int a, int b) { p[0] = a; p[1] = b; }
 
 // ---- launchers -------------------------------------------------------------------------------------
-void pm_launch_embed(int type, const void * table, int K, const int32_t * tokens, int n_tok, float * out, hipStream_t st) {
-    hipLaunchKernelGGL(embed_rows_kernel, dim3((K + 255) / 256, n_tok), dim3(256), 0, st,
-                       type, (const uint8_t *) table, (long) pm_weight_row_stride(type, K), K, tokens, n_tok, out);
+void pm_launch_embed(int type, const void * table, int K, const int32_t * tokens, int n_tok, float * out, hipStream_t st, const pm_rope_cfg * c, const int32_t * pos, const int32_t * seq,
+                     const float * freq_factors, float * tab, int rows) {
+    RopeP r = {};
+    if (tab) {
+        r.n_dims = c->n_dims; r.mode = c->mode; r.n_ctx_orig = c->n_ctx_orig; r.theta_scale = c->theta_scale;
+        r.freq_scale = c->freq_scale; r.ext_factor = c->ext_factor; r.attn_factor = c->attn_factor; r.corr0 = c->corr0; r.corr1 = c->corr1;
+    }
+    hipLaunchKernelGGL(embed_rows_kernel, dim3((K + 1023) / 1024 + (tab ? 1 : 0), n_tok), dim3(256), 0, st,
+                       type, (const uint8_t *) table, (long) pm_weight_row_stride(type, K), K, tokens, out, r, pos, seq, freq_factors, tab, rows);
 }
 
 void pm_rope_params(pm_rope_cfg & c) {
@@ -392,8 +445,9 @@ int pm_launch_attn_rope_fused(const float * q, const float * k, const float * v,
     return 0;
 }
 
-void pm_launch_argmax(const float * x, int n, int32_t * idx, float * val, hipStream_t st, int rows) {
-    hipLaunchKernelGGL(argmax_kernel, dim3(rows), dim3(1024), 0, st, x, n, idx, val);
+void pm_launch_argmax(const float * x, int n, int32_t * idx, float * val, hipStream_t st, int rows, uint64_t * part, int32_t * pos, int32_t * ctl, int by, int rotate) {
+    const int nb = part ? std::min(PM_ARGMAX_PARTS, (n + 4095) / 4096) : 1;               // (a workgroup per 4096 values: a row of a small vocabulary stays with one)
+    hipLaunchKernelGGL(argmax_kernel, dim3(nb, rows), dim3(1024), 0, st, x, n, idx, val, part, pos, ctl, by, rotate);
 }
 int pm_launch_batch_rows(int32_t * blk, const int32_t * host, const pm_batch_layout & l, const int32_t * last, int32_t * pos, int32_t * ctl, hipStream_t st) {
     BatchInts a;
@@ -423,6 +477,9 @@ void pm_launch_scale(const float * a, float * y, float s, long n, hipStream_t st
 }
 void pm_launch_set_i32(int32_t * p, int v, hipStream_t st) {
     hipLaunchKernelGGL(set_i32_kernel, dim3(1), dim3(1), 0, st, p, v);
+}
+void pm_launch_set_i32_pair(int32_t * p, int a, int32_t * q, int b, hipStream_t st) {
+    hipLaunchKernelGGL(set_i32_pair_kernel, dim3(1), dim3(1), 0, st, p, a, q, b);
 }
 void pm_launch_set_i32x2(int32_t * p, int a, int b, hipStream_t st) {
     hipLaunchKernelGGL(set_i32x2_kernel, dim3(1), dim3(1), 0, st, p, a, b);

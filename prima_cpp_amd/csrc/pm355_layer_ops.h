@@ -11,7 +11,9 @@ struct pm_rope_cfg {
 };
 void pm_rope_params(pm_rope_cfg & c);
 
-void pm_launch_embed(int type, const void * table, int K, const int32_t * tokens, int n_tok, float * out, hipStream_t st);
+// tab != null: also the tokens' cos / sin tables (pm_launch_rope_table, same arguments) in the same launch
+void pm_launch_embed(int type, const void * table, int K, const int32_t * tokens, int n_tok, float * out, hipStream_t st, const pm_rope_cfg * c = nullptr, const int32_t * pos = nullptr,
+                     const int32_t * seq = nullptr, const float * freq_factors = nullptr, float * tab = nullptr, int rows = 0);
 void pm_launch_rope_kv_store(const float * q, const float * k, const float * v, float * q_out, float * k_out_f32,
                              void * kc, void * vc, const int32_t * pos0, const int32_t * seq, long seq_stride,
                              const float * freq_factors,
@@ -74,7 +76,11 @@ int  pm_launch_q8_token_prep(const float * q, const float * k, const float * v, 
 int  pm_launch_attn_q8_token(const float * q, const float * k, const float * v, void * kc, void * vc, const int32_t * pos, const int32_t * dyn,
                              const void * mask, int mask_f16, const float * ff, float * out, int H, int Hkv, int dh, int n_ctx, float scale,
                              const pm_rope_cfg & c, int k_q8, int v_q8, int max_keys, hipStream_t st);
-void pm_launch_argmax(const float * x, int n, int32_t * idx, float * val, hipStream_t st, int rows = 1);
+// part: PM_ARGMAX_SCRATCH bytes, zeroed once, for up to PM_ARGMAX_ROWS rows: a row is shared by up to PM_ARGMAX_PARTS workgroups; pos != null (one row): the launch ends with pm_launch_advance's work
+constexpr int PM_ARGMAX_PARTS = 32, PM_ARGMAX_ROWS = 64;
+constexpr size_t PM_ARGMAX_SCRATCH = (size_t) PM_ARGMAX_ROWS * (4 + PM_ARGMAX_PARTS * 8);
+void pm_launch_argmax(const float * x, int n, int32_t * idx, float * val, hipStream_t st, int rows = 1, uint64_t * part = nullptr, int32_t * pos = nullptr, int32_t * ctl = nullptr,
+                      int by = 0, int rotate = 0);
 // a pass over T rows of several sequences: block of int32 = tokens [T] | positions [T] | sequences [T] | ... ; offsets in integers. entries: {sequence, position behind the pass}
 struct pm_batch_layout { int T, seq, entries, n_entries, n_ints; };
 int  pm_launch_batch_rows(int32_t * blk, const int32_t * host, const pm_batch_layout & l, const int32_t * last, int32_t * pos, int32_t * ctl, hipStream_t st);
@@ -85,6 +91,7 @@ void pm_launch_mul(const float * a, const float * b, float * y, long n, long nb,
 void pm_launch_silu_mul(const float * g, const float * u, float * y, long n, hipStream_t st);
 void pm_launch_scale(const float * a, float * y, float s, long n, hipStream_t st);
 void pm_launch_set_i32(int32_t * p, int v, hipStream_t st);
+void pm_launch_set_i32_pair(int32_t * p, int a, int32_t * q, int b, hipStream_t st);      // *p = a, *q = b
 void pm_launch_advance(int32_t * pos, int32_t * ctl, int by, int rotate, hipStream_t st);
 void pm_launch_fill_random_blocks(int type, void * dst, int64_t K, int64_t nrows, uint64_t seed, float scale, hipStream_t st);
 void pm_launch_fill_random_f32(float * dst, int64_t n, uint64_t seed, float mean, float amp, hipStream_t st);

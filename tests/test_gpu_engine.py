@@ -511,3 +511,53 @@ def test_batches_of_several_sequences_equal_one_sequence_at_a_time(E, arch, max_
     assert ((a - b) ** 2).sum() < 1e-3 * (b ** 2).sum()
     w.close()
     w1.close()
+
+
+@pytest.mark.parametrize("n_vocab", [320, 4097, 20011, 140001])
+def test_greedy_token_is_the_first_of_equal_maxima_over_many_workgroups(E, n_vocab):
+    """result_norm + lm_head + argmax: rows of the vocabulary are shared by up to 32 workgroups; equal rows of the head (equal logits to the bit) in several of their parts - the first one
+    wins; a token that ends a step also moves the position counter."""
+    torch = E.torch
+    rng = np.random.default_rng(n_vocab)
+    d = tiny_model(rng, n_layer=1, n_vocab=320, n_ctx=32, rope_freqs=True)
+    w = E.Window(dict(_hp(d), n_vocab=n_vocab), n_ctx=32)
+    from _bind import rand_blocks, row_size
+    for name, kind in (("attn_norm", E.T_ATTN_NORM), ("wq", E.T_WQ), ("wk", E.T_WK), ("wv", E.T_WV), ("wo", E.T_WO), ("ffn_norm", E.T_FFN_NORM), ("ffn_gate", E.T_FFN_GATE),
+                       ("ffn_up", E.T_FFN_UP), ("ffn_down", E.T_FFN_DOWN)):
+        t = getattr(d, name)[0]
+        k, n = dict(attn_norm=(256, 1), wq=(256, 256), wk=(256, 128), wv=(256, 128), wo=(256, 256), ffn_norm=(256, 1), ffn_gate=(256, 512), ffn_up=(256, 512), ffn_down=(512, 256))[name]
+        w._chk(w.lib.pm355_model_set_tensor(w.h, kind, 0, t.type, t.data, E.L.row_size(t.type, k) * n), name)
+    rs = row_size(Q4_K, 256)
+    emb, head = rand_blocks(Q4_K, 512, 256, rng), rand_blocks(Q4_K, n_vocab, 256, rng).reshape(n_vocab, rs)
+    w.set_tensor(E.T_TOK_EMBD, -1, Q4_K, np.resize(emb, n_vocab * rs))
+    w.set_tensor(E.T_OUT_NORM, -1, E.F32, np.ones(256, dtype=np.float32))
+    w.set_tensor(E.T_OUTPUT, -1, Q4_K, head)
+    w.finalize(max_tokens=1)
+    lg, am = torch.empty(n_vocab, device="cuda"), torch.empty(1, dtype=torch.int32, device="cuda")
+    x = torch.randn((1, 256), generator=torch.Generator(device="cuda").manual_seed(1), device="cuda")
+    w.head(x, logits=lg, argmax=am)
+    assert int(am) == int((lg == lg.max()).nonzero()[0])
+    best = int(am)
+    for at in sorted({0, n_vocab // 3, 2 * n_vocab // 3, n_vocab - 1} - {best}, reverse=True):       # the same row again, each time further in front or behind
+        head[at] = head[best]
+        w.set_tensor(E.T_OUTPUT, -1, Q4_K, head)
+        torch.cuda.synchronize()                           # (the uploader's stream)
+        w.head(x, logits=lg, argmax=am)
+        top = (lg == lg.max()).nonzero()[:, 0]
+        assert at in top.tolist() and best in top.tolist() and int(am) == int(top[0])
+    tok = torch.zeros(1, dtype=torch.int32, device="cuda")
+    w.set_pos(0)
+    outs = []
+    for i in range(3):                                     # captured once, replayed: the position moves on its own
+        tok.fill_(3 + i)
+        w.step(token=tok, logits=lg, argmax=am)
+        torch.cuda.synchronize()
+        outs.append(lg.clone())
+        assert int(am) == int((lg == lg.max()).nonzero()[0])
+    for pos in (1, 0):                                     # without the argmax: the same token behind the same single one, and behind none
+        w.set_pos(pos)
+        tok.fill_(4)
+        w.step(token=tok, logits=lg)
+        torch.cuda.synchronize()
+        assert torch.equal(lg, outs[1]) == (pos == 1)
+    w.close()
