@@ -13,7 +13,7 @@
 // (profiles/r02_small_batch_probe.txt); this kernel streams the weights ONCE per 32 tokens and does the products on the matrix cores.
 //
 // Mapping (one MFMA = 32 tokens x 32 weight rows x 32 k for Q4_K / Q5_K = one 32-weight sub-block; x 16 k for Q6_K = one 16-weight group):
-//   A operand = activations: lane (t = lane % 32, g = lane / 32) holds 16 (8) consecutive int8 of token t
+//   A operand = activations: lane (t = lane % 32, g = lane / 32) holds 16 (8) consecutive int8 of token t (up to 16 tokens: several sub-blocks share a register, ActSrc)
 //   B operand = weights    : lane (r = lane % 32, g)            holds the same k of weight row r
 //   result                 : lane (r, g) holds, for ITS OWN row r, tokens 8 (v / 4) + 4 g + v % 4, v = 0..15
 // so the per-row sub-block scale / min / d of a K-quant are lane-local scalars when the i32 tile is scaled (one v_mad_i32_i24 per result;
@@ -103,6 +103,12 @@ template <> struct Rows<true> {           // several matrices: a lane's rows may
 // s_waitcnt vmcnt bookkeeping then assumes the loads behind it may not have been issued: the wait for THIS step's activations also waited for
 // the NEXT step's whole weight tile (ISA: vmcnt(14) where 31 loads were in flight), i.e. the prefetch overlapped half a step. Buffer loads
 // instead: unconditional instructions, the lanes without a token carry an out-of-range offset, return 0 and touch no memory.
+//
+// A 32 x 32 product has 32 token rows; up to 8 (16) tokens would leave three quarters (half) of the operand's lanes empty. They carry OTHER sub-blocks instead: operand lane
+// r = R q + t, R = 2 NV rows per sub-block, holds token t's bytes of sub-block P i + q (P = 16 / NV sub-blocks per register). The product with the weights of sub-block P i + q is
+// right in the rows R q .. R q + R - 1, i.e. in the result registers NV q .. NV q + NV - 1, and nobody reads the others. One load brings what P loads of half-empty lanes did: 2 (4)
+// loads per super-block instead of 8 and as many registers less. At 8 tokens these loads were 10 of the 60 us of a 57344 x 8192 Q4_K launch (the vector memory path is paid per
+// instruction): 57.4 -> 51.6 us on weights out of memory.
 struct ActSrc {
     __amdgpu_buffer_rsrc_t rx, rb; uint32_t xo, bo;        // xo / bo: this lane's byte offset into the operand-ordered activations / the group-sum table (or out of range)
     // sub-block s of super-block sb: lane (t, g) gets the 16 bytes k = 32 s + 16 g .. + 15 of token t (one coalesced kilobyte per wave and 32 tokens)
@@ -119,7 +125,7 @@ template <int TYPE> struct MT;
 template <> struct MT<PM_Q4_K> {
     static constexpr int QA = 0, QB = 32 * PITCH, HD = 64 * PITCH, WAVE_LDS = 64 * PITCH + 32 * PITCH_H;
     struct B { u32x4 qa[4], qb[4], h; };
-    struct A { u32x4 q[8]; f16x8 bs; };
+    template <int NV> struct A { u32x4 q[NV / 2]; f16x8 bs; };
     // part n of a step's tile (4 parts: rows rr + 8 n of both nibble streams; part 0 also the headers)
     template <class RW>
     static __device__ __forceinline__ void issue_b_part(B & b, const RW & rw, int nb, int pr, int lane, int n) {
@@ -139,13 +145,13 @@ template <> struct MT<PM_Q4_K> {
     }
     // sub-block s (32 weights) = the 16 bytes at 32 s + 16 g of the super-block
     template <int NV>
-    static __device__ __forceinline__ void issue_a(A & a, const ActSrc & x, int sb) {
+    static __device__ __forceinline__ void issue_a(A<NV> & a, const ActSrc & x, int sb) {
 #pragma unroll
-        for (int s = 0; s < 8; ++s) a.q[s] = x.ld_sub(sb, s);
+        for (int i = 0; i < NV / 2; ++i) a.q[i] = x.ld_sub(sb, i * (16 / NV));
         a.bs = x.ld_bs(sb);
     }
     template <int NV, class F>
-    static __device__ __forceinline__ void compute(const A & a, const uint8_t * L, int sbi, int r, int g, const float * yd_lds, int /*t_off*/, f32x16 & out, F && between) {
+    static __device__ __forceinline__ void compute(const A<NV> & a, const uint8_t * L, int sbi, int r, int g, const float * yd_lds, int /*t_off*/, f32x16 & out, F && between) {
         const u32x4 hd = *(const u32x4 *) (L + HD + r * PITCH_H + sbi * 16);
         const i32x16 zero = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
         i32x16 isum = zero;
@@ -164,12 +170,12 @@ template <> struct MT<PM_Q4_K> {
             between(j);
             const u32x4 w = *(const u32x4 *) (L + (g ? QB : QA) + r * PITCH + (4 * sbi + j) * 16);
             const int sc0 = (int) ((sc4[(2 * j) >> 2] >> (8 * ((2 * j) & 3))) & 0xFFu), sc1 = (int) ((sc4[(2 * j + 1) >> 2] >> (8 * ((2 * j + 1) & 3))) & 0xFFu);
-            i32x16 acc = mfma_i8x32(a.q[2 * j], w & 0x0F0F0F0Fu, zero);                    // one 32-k MFMA = one 32-weight sub-block
+            i32x16 acc = mfma_i8x32(a.q[2 * j / (16 / NV)], w & 0x0F0F0F0Fu, zero);                    // one 32-k MFMA = one 32-weight sub-block
 #pragma unroll
-            for (int v = 0; v < NV; ++v) { isum[v] = __mul24(sc0, acc[v]) + isum[v]; asm volatile("" : "+v"(isum[v])); }   // (keeps it ONE v_mad_i32_i24:
-            acc = mfma_i8x32(a.q[2 * j + 1], (w >> 4) & 0x0F0F0F0Fu, zero);                //  the re-associated mul, mul, add3 form is 1.5 instructions per term)
+            for (int v = 0; v < NV; ++v) { isum[v] = __mul24(sc0, acc[NV * (2 * j % (16 / NV)) + v]) + isum[v]; asm volatile("" : "+v"(isum[v])); }   // (keeps it ONE v_mad_i32_i24:
+            acc = mfma_i8x32(a.q[(2 * j + 1) / (16 / NV)], (w >> 4) & 0x0F0F0F0Fu, zero);                //  the re-associated mul, mul, add3 form is 1.5 instructions per term)
 #pragma unroll
-            for (int v = 0; v < NV; ++v) { isum[v] = __mul24(sc1, acc[v]) + isum[v]; asm volatile("" : "+v"(isum[v])); }
+            for (int v = 0; v < NV; ++v) { isum[v] = __mul24(sc1, acc[NV * ((2 * j + 1) % (16 / NV)) + v]) + isum[v]; asm volatile("" : "+v"(isum[v])); }
         }
         const f32x16 fz = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
         const f32x16 ms = __builtin_amdgcn_mfma_f32_32x32x16_f16(a.bs, bm, fz, 0, 0, 0);   // sum_s min_s * (bsum[2s] + bsum[2s+1]), exact
@@ -192,7 +198,7 @@ template <> struct MT<PM_Q4_K> {
 template <> struct MT<PM_Q5_K> {
     static constexpr int RP = 368, WAVE_LDS = 32 * RP;
     struct B { u32x4 c[11]; };
-    struct A { u32x4 q[8]; f16x8 bs; };
+    template <int NV> struct A { u32x4 q[NV / 2]; f16x8 bs; };
     template <class RW>
     static __device__ __forceinline__ void issue_b_part(B & b, const RW & rw, int nb, int pr, int lane, int n) {
 #pragma unroll
@@ -210,13 +216,13 @@ template <> struct MT<PM_Q5_K> {
         }
     }
     template <int NV>
-    static __device__ __forceinline__ void issue_a(A & a, const ActSrc & x, int sb) {
+    static __device__ __forceinline__ void issue_a(A<NV> & a, const ActSrc & x, int sb) {
 #pragma unroll
-        for (int s = 0; s < 8; ++s) a.q[s] = x.ld_sub(sb, s);
+        for (int i = 0; i < NV / 2; ++i) a.q[i] = x.ld_sub(sb, i * (16 / NV));
         a.bs = x.ld_bs(sb);
     }
     template <int NV, class F>
-    static __device__ __forceinline__ void compute(const A & a, const uint8_t * L, int sbi, int r, int g, const float * yd_lds, int /*t_off*/, f32x16 & out, F && between) {
+    static __device__ __forceinline__ void compute(const A<NV> & a, const uint8_t * L, int sbi, int r, int g, const float * yd_lds, int /*t_off*/, f32x16 & out, F && between) {
         const uint8_t * blk = L + r * RP + sbi * 176;
         const u32x4 hd = *(const u32x4 *) blk;
         const u32x4 qh = *(const u32x4 *) (blk + 16 + 16 * g);       // bit s of byte l: fifth bit of weight l of sub-block s (l = 16 g + i)
@@ -232,12 +238,12 @@ template <> struct MT<PM_Q5_K> {
             between(j);
             const u32x4 w = *(const u32x4 *) (blk + 48 + 32 * j + 16 * g);
             const int sc0 = (int) ((sc4[(2 * j) >> 2] >> (8 * ((2 * j) & 3))) & 0xFFu), sc1 = (int) ((sc4[(2 * j + 1) >> 2] >> (8 * ((2 * j + 1) & 3))) & 0xFFu);
-            i32x16 acc = mfma_i8x32(a.q[2 * j], (w & 0x0F0F0F0Fu) | (((qh >> (2 * j)) & 0x01010101u) << 4), zero);
+            i32x16 acc = mfma_i8x32(a.q[2 * j / (16 / NV)], (w & 0x0F0F0F0Fu) | (((qh >> (2 * j)) & 0x01010101u) << 4), zero);
 #pragma unroll
-            for (int v = 0; v < NV; ++v) { isum[v] = __mul24(sc0, acc[v]) + isum[v]; asm volatile("" : "+v"(isum[v])); }
-            acc = mfma_i8x32(a.q[2 * j + 1], ((w >> 4) & 0x0F0F0F0Fu) | (((qh >> (2 * j + 1)) & 0x01010101u) << 4), zero);
+            for (int v = 0; v < NV; ++v) { isum[v] = __mul24(sc0, acc[NV * (2 * j % (16 / NV)) + v]) + isum[v]; asm volatile("" : "+v"(isum[v])); }
+            acc = mfma_i8x32(a.q[(2 * j + 1) / (16 / NV)], ((w >> 4) & 0x0F0F0F0Fu) | (((qh >> (2 * j + 1)) & 0x01010101u) << 4), zero);
 #pragma unroll
-            for (int v = 0; v < NV; ++v) { isum[v] = __mul24(sc1, acc[v]) + isum[v]; asm volatile("" : "+v"(isum[v])); }
+            for (int v = 0; v < NV; ++v) { isum[v] = __mul24(sc1, acc[NV * ((2 * j + 1) % (16 / NV)) + v]) + isum[v]; asm volatile("" : "+v"(isum[v])); }
         }
         const f32x16 fz = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
         const f32x16 ms = __builtin_amdgcn_mfma_f32_32x32x16_f16(a.bs, bm, fz, 0, 0, 0);
@@ -258,7 +264,7 @@ template <> struct MT<PM_Q5_K> {
 template <> struct MT<PM_Q6_K> {
     static constexpr int LA = 0, LB = 32 * PITCH, QH = 64 * PITCH, SC = 96 * PITCH, DD = SC + 32 * PITCH_H, WAVE_LDS = DD + 128;
     struct B { u32x4 la[4], lb[4], qh[4], s; uint16_t d; };
-    struct A { u32x4 q[8]; f16x8 bs; };       // as loaded: lane (t, g) holds the WHOLE 16-weight group 2 s + g of sub-block s (operand(): the halves the 16-k products need)
+    template <int NV> struct A { u32x4 q[NV / 2]; f16x8 bs; };       // as loaded: lane (t, g) holds the WHOLE 16-weight group 2 s + g of sub-block s (operand(): the halves the 16-k products need)
     template <class RW>
     static __device__ __forceinline__ void issue_b_part(B & b, const RW & rw, int nb, int pr, int lane, int n) {
         const uint32_t u = (uint32_t) min(8 * pr + (lane & 7), 4 * nb - 1), sb = (uint32_t) min(2 * pr + (lane & 1), nb - 1);
@@ -281,9 +287,9 @@ template <> struct MT<PM_Q6_K> {
     }
     // 16-weight group G = the 8 bytes at 16 G + 8 g of the super-block
     template <int NV>
-    static __device__ __forceinline__ void issue_a(A & a, const ActSrc & x, int sb) {
+    static __device__ __forceinline__ void issue_a(A<NV> & a, const ActSrc & x, int sb) {
 #pragma unroll
-        for (int s = 0; s < 8; ++s) a.q[s] = x.ld_sub(sb, s);
+        for (int i = 0; i < NV / 2; ++i) a.q[i] = x.ld_sub(sb, i * (16 / NV));
         a.bs = x.ld_bs(sb);
     }
     // A operand of the 16-k product over group G: lane (t, g) needs bytes 8 g .. 8 g + 7 of group G. The lane pair (t, 0) / (t, 1) holds groups
@@ -296,14 +302,14 @@ template <> struct MT<PM_Q6_K> {
         }
     }
     template <int NV, class F>
-    static __device__ __forceinline__ void compute(const A & a, const uint8_t * L, int sbi, int r, int g, const float * yd_lds, int /*t_off*/, f32x16 & out, F && between) {
+    static __device__ __forceinline__ void compute(const A<NV> & a, const uint8_t * L, int sbi, int r, int g, const float * yd_lds, int /*t_off*/, f32x16 & out, F && between) {
         const u32x4 s16 = *(const u32x4 *) (L + SC + r * PITCH_H + sbi * 16);
         const float d = h2f(*(const uint16_t *) (L + DD + (sbi * 32 + r) * 2));
         const i32x16 zero = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
         i32x16 isum = zero;
-        u32x2 aop[16];                                   // (the swaps work in place on the registers of a.q)
+        u32x2 aop[NV];                                   // (the swaps work in place on the registers of a.q)
 #pragma unroll
-        for (int s = 0; s < 8; ++s) operands(a.q[s], aop[2 * s], aop[2 * s + 1]);
+        for (int i = 0; i < NV / 2; ++i) operands(a.q[i], aop[2 * i], aop[2 * i + 1]);
 #pragma unroll
         for (int hh = 0; hh < 2; ++hh)
 #pragma unroll
@@ -321,9 +327,11 @@ template <> struct MT<PM_Q6_K> {
                 for (int c = 0; c < 4; ++c) {
                     const int G = 8 * hh + 2 * c + v2;                                   // group index inside the super-block = scale index
                     const int sc = (int) (int8_t) (s16[G >> 2] >> (8 * (G & 3)));
-                    const i32x16 acc = mfma_i8(pk(aop[G][0], aop[G][1]), pk(qv[c][0], qv[c][1]), zero);
+                    constexpr int P = 16 / NV;                                           // sub-blocks G / 2 per operand register
+                    const u32x2 op = aop[2 * ((G >> 1) / P) + (G & 1)];
+                    const i32x16 acc = mfma_i8(pk(op[0], op[1]), pk(qv[c][0], qv[c][1]), zero);
 #pragma unroll
-                    for (int v = 0; v < NV; ++v) { isum[v] = __mul24(sc, acc[v]) + isum[v]; if constexpr (NV < 16) asm volatile("" : "+v"(isum[v])); }   // |acc| <= 16*63*127 (NV = 16: the barrier costs 100 B of spills)
+                    for (int v = 0; v < NV; ++v) { isum[v] = __mul24(sc, acc[NV * ((G >> 1) % P) + v]) + isum[v]; if constexpr (NV < 16) asm volatile("" : "+v"(isum[v])); }   // |acc| <= 16*63*127 (NV = 16: the barrier costs 100 B of spills)
                 }
             }
         // sum_G scale_G * bsum_G (the -32 offset of every weight): B slot s of lane group g = scale[2 s + g]
@@ -353,7 +361,7 @@ template <> struct MT<PM_Q6_K> {
 template <> struct MT<PM_Q8_0> {
     static constexpr int QA = 0, QB = 32 * PITCH, HD = 64 * PITCH, DS = HD + 32 * PITCH_H, WAVE_LDS = DS + 1024;
     struct B { u32x4 qa[4], qb[4], h, ds; };
-    struct A { u32x4 q[4]; };
+    template <int NV> struct A { u32x4 q[NV / 4]; };
     // (ds: the ACTIVATION scales of the step's 8 blocks, [block][32 token slots] f32 = 1 KiB per wave and step, travel with the weight tile into the wave's
     //  LDS image - held in registers per result token they cost 32 VGPRs per operand set and the 16-token form spilled)
     template <class RW>
@@ -375,12 +383,12 @@ template <> struct MT<PM_Q8_0> {
         *(u32x4 *) (L + DS + lane * 16) = b.ds;
     }
     template <int NV>
-    static __device__ __forceinline__ void issue_a(A & a, const ActSrc & x, int sb) {
+    static __device__ __forceinline__ void issue_a(A<NV> & a, const ActSrc & x, int sb) {
 #pragma unroll
-        for (int j = 0; j < 4; ++j) a.q[j] = x.ld_blk(4 * sb + j);
+        for (int i = 0; i < NV / 4; ++i) a.q[i] = x.ld_blk(4 * sb + i * (16 / NV));
     }
     template <int NV, class F>
-    static __device__ __forceinline__ void compute(const A & a, const uint8_t * L, int sbi, int r, int g, const float *, int t_off, f32x16 & out, F && between) {
+    static __device__ __forceinline__ void compute(const A<NV> & a, const uint8_t * L, int sbi, int r, int g, const float *, int t_off, f32x16 & out, F && between) {
         const i32x16 zero = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
         const u32x2 d4 = *(const u32x2 *) (L + HD + r * PITCH_H + sbi * 8);              // this row's four block scales (f16)
         const float * ds = (const float *) (L + DS) + t_off;                             // (16-token passes over a 32-slot table start at slot t_off)
@@ -390,12 +398,12 @@ template <> struct MT<PM_Q8_0> {
             const u32x4 w = *(const u32x4 *) (L + (g ? QB : QA) + r * PITCH + (4 * sbi + j) * 16);
             const uint32_t hb = (d4[j >> 1] >> (16 * (j & 1))) & 0xFFFFu;
             const float dw = (hb & 0x7C00u) == 0x7C00u ? 0.0f : h2f((uint16_t) hb);       // (a block past the row: whatever the padding holds, times zero)
-            const i32x16 acc = mfma_i8x32(a.q[j], w, zero);
+            const i32x16 acc = mfma_i8x32(a.q[j / (16 / NV)], w, zero);
 #pragma unroll
             for (int q = 0; q < NV / 4; ++q) {
                 const f32x4 yd = *(const f32x4 *) (ds + (4 * sbi + j) * 32 + 8 * q + 4 * g);
 #pragma unroll
-                for (int i = 0; i < 4; ++i) out[4 * q + i] = fmaf((float) acc[4 * q + i], dw * yd[i], out[4 * q + i]);
+                for (int i = 0; i < 4; ++i) out[4 * q + i] = fmaf((float) acc[NV * (j % (16 / NV)) + 4 * q + i], dw * yd[i], out[4 * q + i]);
             }
         }
     }
@@ -428,19 +436,21 @@ __device__ __forceinline__ void mmq_i8_body(const MmqP & p, const int w, const i
 #endif
     uint8_t * L = stage + wave * M::WAVE_LDS;
     const int r = lane & 31, g = lane >> 5;
-    const bool act = NV == 16 ? true : r < p.T;                                     // token slots >= T: operand bytes are don't-care (scale row 0, never stored)
+    constexpr int RT = 2 * NV;                                                      // operand rows per sub-block
+    const int tq = r / RT, tt = r % RT;                                              // this lane's sub-block of a register, and its token
+    const bool act = NV == 16 ? true : tt < p.T, act_b = NV == 16 ? true : r < p.T; // token slots >= T: operand bytes are don't-care (scale row 0, never stored)
     ActSrc xs;
     xs.rx = __builtin_amdgcn_make_buffer_rsrc((void *) p.qT, 0, Q80 ? nbw * 1024 : nsb * 8192, 0x00020000);
     xs.rb = __builtin_amdgcn_make_buffer_rsrc((void *) p.bsT, 0, Q80 ? nbw * 128 : nsb * 1024 + 512, 0x00020000);   // (+ t_off slots of the last super-block: inside the table allocation)
-    xs.xo = act ? (uint32_t) ((32 * g + r + p.t_off) * 16) : 0x80000000u;
-    xs.bo = Q80 ? (uint32_t) (16 * lane) : act ? (uint32_t) ((lane + p.t_off) * 16) : 0x80000000u;   // (Q8_0: lane l carries 16 bytes of the step's [8 blocks][32 slots] activation scales)
+    xs.xo = act ? (uint32_t) (tq * 1024 + (32 * g + tt + p.t_off) * 16) : 0x80000000u;
+    xs.bo = Q80 ? (uint32_t) (16 * lane) : act_b ? (uint32_t) ((lane + p.t_off) * 16) : 0x80000000u;   // (Q8_0: lane l carries 16 bytes of the step's [8 blocks][32 slots] activation scales)
     Rows<MJ> rw;
-    // (round 6, measured and rejected: TWO weight tiles in flight per wave - a second register set, the steps taking the sets alternately. The forms with the
-    //  registers for it, Q4_K up to 8 tokens, went from 170 to 248 VGPRs and - with the look-ahead past the last step made cheap - from 36.7 to 38.5 us on
-    //  ffn_gate, 16.5 to 17.6 on wq, 160.5 to 165.7 us per 70B layer: the streaming part of a launch already runs at 6.3 TB/s, what a launch pays is its
-    //  fixed ~8 us - profiles/r06_small_batch.txt)
+    // (measured and rejected, again with the registers that the packed activations free: TWO weight tiles in flight per wave, the activations of the next step in front of them -
+    //  57344 x 8192 Q4_K at 8 tokens 53.0 -> 55.1 us, Q6_K 98.0 -> 102.4; and two workgroups that share a row group's K where 128 row groups leave half the chip idle - 4096 x 14336
+    //  Q6_K 24.7 -> 22.8 us, but Q4_K 14.3 -> 16.3 and 4096 x 8192 11.6 -> 13.1: the exchange costs what the second half of the chip saves. What Q6_K launches lose is memory traffic:
+    //  1.36 x the weights' bytes, the scale and d lines of a row tail are fetched again for every step)
     typename M::B R;
-    typename M::A A0 = {}, A1 = {};                              // (inactive token lanes keep these zeros)
+    typename M::template A<NV> A0 = {}, A1 = {};                 // (inactive token lanes keep these zeros)
     // a step's weight tile goes out in FOUR parts. Issued in one burst (13 x 1 KiB per wave, 100 KB per CU) the wave sat in the issue itself until the
     // CU's miss queues had taken the whole tile - and only then started on the tile it holds: load time and compute time added up
     // (ffn_down Q6_K, 8 tokens: 41 us stream + 19 us compute + 12 fixed = 70). One part in front of every quarter of the first super-block's
@@ -518,12 +528,12 @@ __device__ __forceinline__ void mmq_i8_body(const MmqP & p, const int w, const i
                     if constexpr (SPREAD && !(ABL & 2)) { __builtin_amdgcn_sched_barrier(0); issue_b_part(Rc, prn, n); __builtin_amdgcn_sched_barrier(0); }
                 };
                 if constexpr (!(ABL & 4)) M::template compute<NV>(A0, L, 0, r, g, dTl + sb0 * 32, p.t_off, out, part);
-                else { for (int s_ = 0; s_ < 8; ++s_) asm volatile("" :: "v"(A0.q[s_])); asm volatile("" :: "v"(A0.bs)); asm volatile("" :: "v"(*(const u32x4 *) (L + 16 * lane))); }
+                else { for (int s_ = 0; s_ < NV / 2; ++s_) asm volatile("" :: "v"(A0.q[s_])); asm volatile("" :: "v"(A0.bs)); asm volatile("" :: "v"(*(const u32x4 *) (L + 16 * lane))); }
                 __builtin_amdgcn_sched_barrier(0);
                 if constexpr (!(ABL & 1)) M::template issue_a<NV>(A0, xs, min(2 * prn, nsb - 1));
                 __builtin_amdgcn_sched_barrier(0);
                 if constexpr (!(ABL & 4)) M::template compute<NV>(A1, L, 1, r, g, dTl + (2 * pr + 1 < nsb ? sb1 : nsb) * 32, p.t_off, out, [](int) {});
-                else { for (int s_ = 0; s_ < 8; ++s_) asm volatile("" :: "v"(A1.q[s_])); asm volatile("" :: "v"(A1.bs)); asm volatile("" :: "v"(*(const u32x4 *) (L + 16 * lane + 1024))); }
+                else { for (int s_ = 0; s_ < NV / 2; ++s_) asm volatile("" :: "v"(A1.q[s_])); asm volatile("" :: "v"(A1.bs)); asm volatile("" :: "v"(*(const u32x4 *) (L + 16 * lane + 1024))); }
                 __builtin_amdgcn_sched_barrier(0);
             };
             for (int pr = pb; pr < pe; pr += pstep) step(R, pr);
@@ -593,7 +603,7 @@ template <int TA, int TB, int NV, bool EPI = false>
 __global__ __launch_bounds__(BLOCK, 2) void mmq_i8_dual_kernel(MmqP2 pp) {
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
     if ((int) blockIdx.x < pp.ga) mmq_i8_body<TA, NV, 0, true, EPI>(pp.a, (int) blockIdx.x, pp.ga, smem);
-    else mmq_i8_body<TB, NV, 0, TB == PM_Q6_K, EPI>(pp.b, (int) blockIdx.x - pp.ga, (int) gridDim.x - pp.ga, smem);   // (Q6_K: the one-job multi-job form - no spills at 16 tokens)
+    else mmq_i8_body<TB, NV, 0, TB == PM_Q6_K, EPI>(pp.b, (int) blockIdx.x - pp.ga, (int) gridDim.x - pp.ga, smem);
 }
 
 // prologue: per super-block, the activation group sums as F16 in A-operand order and the transposed activation scales
@@ -849,13 +859,7 @@ int pm_launch_mmq_i8(int type, const void * W, const void * xq, const float * x_
         if (type == PM_Q4_K) { if (tn <= 8) go(mmq_i8_kernel<PM_Q4_K, 4>); else if (tn <= 16) go(mmq_i8_kernel<PM_Q4_K, 8>); else go(mmq_i8_kernel<PM_Q4_K, 16>); }
         else if (type == PM_Q5_K) { if (tn <= 8) go(mmq_i8_kernel<PM_Q5_K, 4>); else go(mmq_i8_kernel<PM_Q5_K, 8>); }
         else if (tn <= 8)    go(mmq_i8_kernel<PM_Q6_K, 4>);
-        else if (tn <= 16) {
-            // the 16-token Q6_K form with wave-uniform row addressing spills 44 B per lane; the one with per-lane row pointers (the multi-job form) does not
-            // (249 registers): a launch of ONE job in that form
-            p.njobs = 1; p.y_stride = N;
-            for (int j = 0; j < 3; ++j) { p.Wj[j] = p.W; p.yj[j] = p.y; p.bj[j] = p.bias; p.nj[j] = N; p.start[j] = j == 0 ? 0 : N; }
-            go(mmq_i8_kernel<PM_Q6_K, 8, 0, true>);
-        }
+        else if (tn <= 16)   go(mmq_i8_kernel<PM_Q6_K, 8>);
         else                 go(mmq_i8_kernel<PM_Q6_K, 16>);
     }
     return 0;
