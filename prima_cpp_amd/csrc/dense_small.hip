@@ -304,6 +304,124 @@ template <typename T, int NT, int RM, int SRC, int EXP> __global__ __launch_boun
     } while (EXP == SORTED && t0 < n_tok);
 }
 
+// The same product over ONE bf16 matrix for up to 8 tokens: workgroups that stay (two per CU) take the row tiles blockIdx.x, + gridDim.x, .. one after another. A workgroup per
+// tile copies all activations for every 8 or 16 rows - six tokens of 4096 values are 48 KB against 64 KB of weights -, behind a barrier, and has nothing on its way while it
+// starts and while it adds up; what bounds the product is the read of the weights. Here the load groups of all tiles are one sequence, two of them in flight, the next one
+// requested right behind the products that free its registers, also across the end of a tile. TP = 4 or 8: the activations of that many tokens are copied to LDS once, by DMA and
+// by the wave that multiplies them (a wave has every 8th 64-k block of all rows: no barrier). TP = 0: they do not fit and ride in the load groups; 16 rows share them, one workgroup
+// per CU with twice the registers. The bias rides there too (loads return in order: one of its own would wait for the weights in flight).
+// Weights from memory, in us before / now: 14336 x 4096 3 tokens 27.9 / 22.5, 6 30.4 / 22.7 (5.2 TB/s); 4096 x 14336 6 tokens 33.2 / 24.3; 32000 x 4096 6 tokens 59 / 45.7 (5.7 TB/s);
+// 28672 x 8192 5 tokens 133 / 77 (6.1 TB/s). Taken back: two sum buffers in turn for one barrier less (spills at RM = 2, 32000 x 2048 25.1 -> 26.6).
+template <int RM, int TP> __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(TP == 0 && RM == 2 ? 2 : 4))) void dense_rows_kernel(SmallP p, int tiles) {
+    constexpr int U = TP ? 8 / RM : 4, NL = U * (RM + (TP ? 0 : 1)) + 1, ROWS = 8 * RM;            // 64-k blocks and loads of a group
+    extern __shared__ __attribute__((aligned(16))) char smem[];
+    float * red = (float *) smem;                                                                  // [8 waves][RM][16 columns][16 rows]
+    const int wave = __builtin_amdgcn_readfirstlane((int) threadIdx.x >> 6), lane = threadIdx.x & 63, lr = lane & 15, g = lane >> 4;
+    const int nblk = p.K >> 6, mine = (nblk - wave + 7) >> 3, ng = mine > U ? (mine + U - 1) / U : 1;      // 64-k blocks wave, wave + 8, .. ; load groups per tile
+    const int my_tiles = (tiles - (int) blockIdx.x + (int) gridDim.x - 1) / (int) gridDim.x, total = my_tiles * ng;
+    const uint16_t * W = (const uint16_t *) p.W;
+    const uint32_t at = (uint32_t) ((lr >> 3) * 32 + g * 8), tok = (lr & 7) < p.T ? lr & 7 : p.T - 1;
+    uint32_t w_off[RM];
+#pragma unroll
+    for (int m = 0; m < RM; ++m) w_off[m] = ((uint32_t) (m * 8 + (lr & 7)) * (uint32_t) p.K + at) * 2;
+    // the element of a tile that this thread stores: rows fastest, a token's rows are one segment
+    const int o_row = threadIdx.x % ROWS, o_tok = threadIdx.x / ROWS;
+    // this wave's blocks of the activations: [block][TP tokens][8 pieces of 16 bytes, piece p in place p ^ token / 2]
+    char * xs = smem + 8 * RM * 1024 + (size_t) wave * ((nblk + 7) >> 3) * (TP * 128);
+    if constexpr (TP != 0) {
+        constexpr int PER = 8 / TP;                                                                // blocks per request
+        const int t = lane >> 3 & (TP - 1), b = lane >> 3 >> (TP == 8 ? 3 : 2);
+        const uint32_t src = ((uint32_t) t * (uint32_t) p.lda + (uint32_t) (((lane & 7) ^ (t >> 1)) * 8)) * 2 + (uint32_t) (wave + b * 8) * 128, dst = (uint32_t) (uintptr_t) (__attribute__((address_space(3))) char *) xs;
+        for (int i = 0; i < mine; i += PER)
+            if (t < p.T && i + b < mine) pm_dma16(p.act, src + (uint32_t) i * 1024, dst + (uint32_t) i * (TP * 128));
+    }
+    const char * x_at = xs + (TP ? (tok * 128 + (((lr >> 3) * 4 + g) ^ (tok >> 1)) * 16) : 0);
+    const uint32_t x_off = (tok * (uint32_t) p.lda + at) * 2;
+    const __amdgpu_buffer_rsrc_t rb = __builtin_amdgcn_make_buffer_rsrc((void *) p.bias, 0, p.bias ? p.n_store * 4 : 0, 0x00020000);
+    struct Group { u32x4 w[U][RM], x[TP ? 1 : U]; float bias; };
+    int l_tile = (int) blockIdx.x, l_grp = 0;                                                      // the next group to be requested
+    auto load = [&](Group & a) __attribute__((always_inline)) {
+        const uint16_t * at_tile = W + (size_t) l_tile * ROWS * p.K;
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            // past the end of a row: out of the bounds of an empty buffer, no traffic (the last block again would be waited for)
+            const int i = l_grp * U + u, in = i < mine, soff = in ? (wave + i * 8) * 128 : 0;
+            if (TP == 0) {
+                const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc((void *) p.act, 0, in ? ((p.T - 1) * p.lda + p.K) * 2 : 0, 0x00020000);
+                a.x[TP ? 0 : u] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rx, (int) x_off, soff, 0));
+            }
+            const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc((void *) at_tile, 0, in ? ROWS * p.K * 2 : 0, 0x00020000);
+#pragma unroll
+            for (int m = 0; m < RM; ++m) a.w[u][m] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rw, (int) w_off[m], soff, 2));      // (2: streamed past the caches)
+        }
+        a.bias = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rb, (l_tile * ROWS + o_row) * 4, 0, 0));       // (past n_store, without a bias: 0)
+        if (++l_grp == ng) { l_grp = 0; l_tile += gridDim.x; }
+    };
+    Group ga, gb;
+    load(ga);
+    if (total > 1) load(gb);
+    // the activations are in LDS (a wave reads its own blocks only), the weights on their way
+    if constexpr (TP != 0) {
+        if (total > 1) asm volatile("s_waitcnt vmcnt(%0)" : : "n"(2 * NL) : "memory");
+        else asm volatile("s_waitcnt vmcnt(%0)" : : "n"(NL) : "memory");
+    }
+    f32x4 acc[RM];
+#pragma unroll
+    for (int m = 0; m < RM; ++m) acc[m] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    int c_tile = (int) blockIdx.x, c_grp = 0;              // the group that is multiplied
+    auto step = [&](const Group & a) __attribute__((always_inline)) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int i = c_grp * U + u;
+            // (read on every path: a register that may still be on its way would be waited for where it is loaded again)
+            if (TP == 0) asm volatile("" : : "v"(a.x[TP ? 0 : u]));
+#pragma unroll
+            for (int m = 0; m < RM; ++m) asm volatile("" : : "v"(a.w[u][m]));
+            if (i >= mine) continue;
+            const u32x4 x = TP ? *(const u32x4 *) (x_at + i * (TP * 128)) : a.x[TP ? 0 : u];
+#pragma unroll
+            for (int m = 0; m < RM; ++m) acc[m] = Frag<uint16_t>::mma(a.w[u][m], x, acc[m]);
+        }
+        const float bias = a.bias;
+        asm volatile("" : : "v"(bias));
+        if (++c_grp < ng) return;
+        c_grp = 0;
+        // (the wait states between a product and the store that reads it, spelled out as in the kernel above)
+#pragma unroll
+        for (int m = 0; m < RM; ++m) asm volatile("" : "+v"(acc[m]));
+        asm volatile("s_nop 15\n\ts_nop 3");
+#pragma unroll
+        for (int m = 0; m < RM; ++m) asm volatile("" : "+v"(acc[m]));
+#pragma unroll
+        for (int m = 0; m < RM; ++m) { *(f32x4 *) (red + ((wave * RM + m) * 16 + lr) * 16 + g * 4) = acc[m]; acc[m] = f32x4{0.0f, 0.0f, 0.0f, 0.0f}; }
+        __syncthreads();
+        const int row = c_tile * ROWS + o_row;
+        if (o_tok < p.T && row < p.n_store) {
+            float v = 0.0f;
+#pragma unroll
+            for (int w = 0; w < 8; ++w) { const float * q = red + ((w * RM + o_row / 8) * 16 + o_tok) * 16 + o_row % 8; v += q[0]; v += q[8 * 16 + 8]; }
+            st_type(p.y, (size_t) o_tok * p.ldy + row, p.y_type, act_apply(p.act_fn, v + bias));
+        }
+        c_tile += gridDim.x;
+        __syncthreads();
+    };
+    if (total == 1) { step(ga); return; }
+    int left = total - 2;
+    for (; left > 1; left -= 2) { step(ga); load(ga); step(gb); load(gb); }
+    step(ga);
+    if (left) { load(ga); step(gb); step(ga); }
+    else step(gb);
+}
+size_t rows_lds(int rm, int tp, int K) { return (size_t) 8 * rm * 1024 + (size_t) (K / 64 + 7) / 8 * 8 * tp * 128; }
+template <int RM, int TP> int launch_rows(const SmallP & p, int N, hipStream_t st) {
+    const int tiles = N / (8 * RM), cus = pm_device_cus();
+    const size_t lds = rows_lds(RM, TP, p.K);
+    const int per = TP == 0 && RM == 2 || lds > 80 * 1024 ? 1 : 2, grid = tiles < per * cus ? tiles : per * cus;
+    pm_allow_big_lds((const void *) dense_rows_kernel<RM, TP>, lds);
+    hipLaunchKernelGGL((dense_rows_kernel<RM, TP>), dim3(grid), dim3(512), lds, st, p, tiles);
+    return 0;
+}
+
 template <typename T, int NT, int RM, int SRC, int EXP = DENSE> int launch(const SmallP & p, int N, int y, hipStream_t st) {
     constexpr bool LINE = sizeof(T) == 2 && SRC != 0;
     constexpr int rows = (LINE ? 8 : 16) * RM, toks = (LINE ? 8 : 16) * NT;
@@ -326,6 +444,16 @@ template <typename T> int launch_type(const pm_dense_args & a, const SmallP & p,
         if constexpr (sizeof(T) == 2) if (rm == 2) return a.T == 1 ? launch<T, 1, 2, 1>(p, N, 0, st) : a.T == 2 ? launch<T, 1, 2, 2>(p, N, 0, st) : launch<T, 1, 2, 4>(p, N, 0, st);
         return a.T == 1 ? launch<T, 1, 1, 1>(p, N, 0, st) : a.T == 2 ? launch<T, 1, 1, 2>(p, N, 0, st) : launch<T, 1, 1, 4>(p, N, 0, st);
     }
+    // One matrix, up to 8 tokens: the workgroups that stay, with the activations in LDS where they fit (150 KB: 16 bytes per value for 5..8 tokens, 8 for less), from memory above that
+    // (5 tokens of 4096 values, 14336 rows: 22.7 us against 27 from memory). One token of shorter rows stays with a workgroup per tile, which has less to do before its first and after
+    // its last weight (32000 x 2048: 23.6 us against 25.1, 4096 x 5120: 10.2 / 10.9; the other way round from 6144 values: 5120 x 6144 16.8 / 15.2, 2048 x 8192 10.3 / 9.0)
+    if constexpr (sizeof(T) == 2)
+        if (a.T <= 8 && !a.group && !a.merge && (a.T > 1 || a.K >= 6144) && (int64_t) p.T * p.lda < (1 << 28) && a.K < (1 << 26)) {
+            const int tp = a.T <= 4 ? 4 : 8;
+            if (rows_lds(rm, tp, a.K) > 150 * 1024) return launch_rows<2, 0>(p, N, st);
+            if (tp == 4) return rm == 1 ? launch_rows<1, 4>(p, N, st) : launch_rows<2, 4>(p, N, st);
+            return rm == 1 ? launch_rows<1, 8>(p, N, st) : launch_rows<2, 8>(p, N, st);
+        }
     if constexpr (sizeof(T) == 2)
         if (a.T <= 8 && (size_t) a.T * (a.K * 2 + 16) <= LDS_ACT) return rm == 1 ? launch<T, 1, 1, -1>(p, N, 0, st) : launch<T, 1, 2, -1>(p, N, 0, st);
     const bool wide = N / 32 >= 512;

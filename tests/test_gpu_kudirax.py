@@ -118,6 +118,27 @@ def test_dense_mul_mat(dtype, T, K, N, n_store):
         assert (y[:, n_store:] == 7.0).all()               # nothing beyond the wanted columns is touched
 
 
+# waves without a block (K < 512), a last load group that is not full, one group per tile and several, activations in LDS for 4 and 8 tokens and from memory, one workgroup per CU
+# and two, more tiles than workgroups (not a multiple), a stored row count that ends inside a tile
+@pytest.mark.parametrize("T,K,n_store", [(2, 64, 33), (3, 704, 1030), (8, 704, 9001), (5, 2048, 16421), (4, 4096, 8260), (7, 4096, 12300), (8, 5120, 4100), (4, 5120, 8194), (1, 6144, 700),
+                                         (8, 8192, 2100), (8, 9216, 2500), (6, 9728, 8300), (4, 18496, 1100), (1, 20480, 4110)])
+def test_dense_mul_mat_few_tokens_over_many_rows(T, K, n_store):
+    import prima_cpp_amd.ops as O
+    N = (n_store + 63) // 64 * 64
+    g = torch.Generator(device="cuda").manual_seed(T + K)
+    w = (torch.randn(N, K, generator=g, device="cuda") / K ** 0.5).bfloat16()
+    x = torch.randn(T, K + 64, generator=g, device="cuda").bfloat16()[:, :K]
+    b = torch.randn(N, generator=g, device="cuda")
+    ref = x.double() @ w.double().T
+    for bias, act, ydt in ((None, 0, torch.float32), (b, 1, torch.bfloat16)):
+        y = torch.full((T, N), 7.0, dtype=ydt, device="cuda")
+        O.dense_mul_mat(w, x, y, n_store=n_store, bias=bias, act=act)
+        want = ref if bias is None else (ref + b.double()).clamp(min=0) ** 2
+        tol = 2e-6 * K ** 0.5 if ydt == torch.float32 else 1e-2
+        assert ((y.double() - want)[:, :n_store].abs() <= tol * (1 + want[:, :n_store].abs())).all()
+        assert (y[:, n_store:] == 7.0).all()
+
+
 @pytest.mark.parametrize("tiles", [(2048, 2048), (300, 4096)])
 def test_dense_mul_mat_large_tiles(tiles):
     """shapes whose grid takes the 256 x 256 tiles, ragged in both directions"""
