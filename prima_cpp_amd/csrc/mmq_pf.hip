@@ -24,6 +24,7 @@
 // measured ~1e-6).
 #include "pm355_device.h"
 #include "pm355_kernels.h"
+#include "attn_tail_device.h"
 #include <stdlib.h>
 #include <stdio.h>
 #include <mutex>
@@ -72,6 +73,63 @@ template <> struct PfT<PM_Q6_K> { static constexpr int NSTREAM = 3, EXTRA = 512;
 // Q8_0 (row-SoA qa[K/32][16] | qb[K/32][16] | half d[K/32]): slots of 64 k = one k-step (two blocks: 1 KiB of qa, 1 KiB of qb per wave), requested two steps ahead
 template <> struct PfT<PM_Q8_0> { static constexpr int NSTREAM = 2, EXTRA = 0; };
 template <int TYPE> constexpr int pf_wave_bytes() { return 2 * PfT<TYPE>::NSTREAM * 1024 + 1024 + PfT<TYPE>::EXTRA; }
+
+// 8 weights -> one A operand: 16-k slice j of 64-k step ks (may be a run-time value) of 128-k piece mm of a super-block. Written stage by stage over the four independent half2
+// chains (and - perm - add - fma): a dependent vector instruction issues ~8-10 cycles after its producer, four chains side by side hide that
+template <int TYPE> __device__ __forceinline__ half8 pf_dequant(const u32x2 ql, const u32x2 qh, const int mm, const int ks, const int j, const half2v mul, const half2v add) {
+    uint32_t v[2];
+    half2v t[4];
+    if (TYPE == PM_Q8_0) {
+        // int8 x -> byte x ^ 0x80 = x + 128 -> F16 1024 + 128 + x (exact) -> - 1152 -> * d: one rounding, dequantize_row_q8_0's d * x (ggml-quants.c:1616)
+        const half2v bias = half2v{(_Float16) -1152.0f, (_Float16) -1152.0f};
+#pragma unroll
+        for (int c = 0; c < 2; ++c) v[c] = ql[c] ^ 0x80808080u;
+#pragma unroll
+        for (int c = 0; c < 2; ++c) { t[2 * c] = h2(__builtin_amdgcn_perm(0x64646464u, v[c], 0x05010400u)); t[2 * c + 1] = h2(__builtin_amdgcn_perm(0x64646464u, v[c], 0x07030602u)); }
+#pragma unroll
+        for (int c = 0; c < 4; ++c) t[c] = t[c] + bias;
+#pragma unroll
+        for (int c = 0; c < 4; ++c) t[c] = t[c] * mul;
+    } else if (TYPE == PM_Q4_K || TYPE == PM_Q5_K) {
+        const bool hi = j >> 1;                            // slices 2, 3: the unit's second sub-block = high nibbles
+        const half2v bias = hi ? half2v{(_Float16) -64.0f, (_Float16) -64.0f} : half2v{(_Float16) -1024.0f, (_Float16) -1024.0f};
+        uint32_t ex[2] = {hi ? 0x54545454u : 0x64646464u, hi ? 0x54545454u : 0x64646464u};   // F16 exponent byte: 64 + m / 16 (m = nibble << 4) / 1024 + m
+#pragma unroll
+        for (int c = 0; c < 2; ++c) v[c] = ql[c] & (hi ? 0xF0F0F0F0u : 0x0F0F0F0Fu);
+        if (TYPE == PM_Q5_K) {
+            // the 5th bit (bit s of the qh bytes, s = sub-block): low nibbles - bit 4 of the value byte; high nibbles (value byte = q << 4, ulp 1/16) - it is
+            // mantissa bit 8 = bit 0 of the half's HIGH byte, which v_perm takes from the exponent operand
+            const int sb = 4 * mm + 2 * ks + (j >> 1);
+#pragma unroll
+            for (int c = 0; c < 2; ++c) {
+                const uint32_t bit = (qh[c] >> sb) & 0x01010101u;
+                if (hi) ex[c] |= bit; else v[c] |= bit << 4;
+            }
+        }
+#pragma unroll
+        for (int c = 0; c < 2; ++c) { t[2 * c] = h2(__builtin_amdgcn_perm(ex[c], v[c], 0x05010400u)); t[2 * c + 1] = h2(__builtin_amdgcn_perm(ex[c], v[c], 0x07030602u)); }
+#pragma unroll
+        for (int c = 0; c < 4; ++c) t[c] = t[c] + bias;
+#pragma unroll
+        for (int c = 0; c < 4; ++c) t[c] = pk_fma(t[c], mul, add);
+    } else {
+        const half2v bias = half2v{(_Float16) -1056.0f, (_Float16) -1056.0f};  // 1024 + q - 32
+        uint32_t lo4[2], hi2[2];
+#pragma unroll
+        for (int c = 0; c < 2; ++c) lo4[c] = (ql[c] >> (4 * ks)) & 0x0F0F0F0Fu;
+#pragma unroll
+        for (int c = 0; c < 2; ++c) hi2[c] = (j >> 1 ? (qh[c] >> (4 * ks)) << 2 : (qh[c] >> (4 * ks)) << 4) & 0x30303030u;
+#pragma unroll
+        for (int c = 0; c < 2; ++c) v[c] = lo4[c] | hi2[c];
+#pragma unroll
+        for (int c = 0; c < 2; ++c) { t[2 * c] = h2(__builtin_amdgcn_perm(0x64646464u, v[c], 0x05010400u)); t[2 * c + 1] = h2(__builtin_amdgcn_perm(0x64646464u, v[c], 0x07030602u)); }
+#pragma unroll
+        for (int c = 0; c < 4; ++c) t[c] = t[c] + bias;
+#pragma unroll
+        for (int c = 0; c < 4; ++c) t[c] = t[c] * mul;
+    }
+    return __builtin_bit_cast(half8, u32x4{u2(t[0]), u2(t[1]), u2(t[2]), u2(t[3])});
+}
 
 // the k loop + epilogue of one workgroup tile: rows [n0, n0 + 256) of job jb, tokens [t0, t0 + 32 NT)
 // role: 0 plain; 1 / 2 = the gate / up half of a PAIR tile (waves 0-3 multiply ffn_gate's rows [n0, n0 + 128), waves 4-7 the same rows of ffn_up; the gate
@@ -194,64 +252,7 @@ __device__ __forceinline__ void pf_body(const PfP & p, const PfJob & jb, const i
             mul = half2v{dd, dd};
         }
     };
-    // 8 weights of slice i -> one A operand. Written stage by stage over the four independent half2 chains (and - perm - add - fma): a dependent vector
-    // instruction issues ~8-10 cycles after its producer, four chains side by side hide that
-    auto dequant = [&](const Raw & w, int i) __attribute__((always_inline)) {
-        const int ks = (i >> 2) & 1, j = i & 3;
-        uint32_t v[2];
-        half2v t[4];
-        if (Q8) {
-            // int8 x -> byte x ^ 0x80 = x + 128 -> F16 1024 + 128 + x (exact) -> - 1152 -> * d: one rounding, dequantize_row_q8_0's d * x (ggml-quants.c:1616)
-            const half2v bias = half2v{(_Float16) -1152.0f, (_Float16) -1152.0f};
-#pragma unroll
-            for (int c = 0; c < 2; ++c) v[c] = w.ql[c] ^ 0x80808080u;
-#pragma unroll
-            for (int c = 0; c < 2; ++c) { t[2 * c] = h2(__builtin_amdgcn_perm(0x64646464u, v[c], 0x05010400u)); t[2 * c + 1] = h2(__builtin_amdgcn_perm(0x64646464u, v[c], 0x07030602u)); }
-#pragma unroll
-            for (int c = 0; c < 4; ++c) t[c] = t[c] + bias;
-#pragma unroll
-            for (int c = 0; c < 4; ++c) t[c] = t[c] * mul;
-        } else if (K45) {
-            const bool hi = j >> 1;                            // slices 2, 3: the unit's second sub-block = high nibbles
-            const half2v bias = hi ? half2v{(_Float16) -64.0f, (_Float16) -64.0f} : half2v{(_Float16) -1024.0f, (_Float16) -1024.0f};
-            uint32_t ex[2] = {hi ? 0x54545454u : 0x64646464u, hi ? 0x54545454u : 0x64646464u};   // F16 exponent byte: 64 + m / 16 (m = nibble << 4) / 1024 + m
-#pragma unroll
-            for (int c = 0; c < 2; ++c) v[c] = w.ql[c] & (hi ? 0xF0F0F0F0u : 0x0F0F0F0Fu);
-            if (TYPE == PM_Q5_K) {
-                // the 5th bit (bit s of the qh bytes, s = sub-block): low nibbles - bit 4 of the value byte; high nibbles (value byte = q << 4, ulp 1/16) - it is
-                // mantissa bit 8 = bit 0 of the half's HIGH byte, which v_perm takes from the exponent operand
-                const int sb = i >> 1;
-#pragma unroll
-                for (int c = 0; c < 2; ++c) {
-                    const uint32_t bit = (w.qh[c] >> sb) & 0x01010101u;
-                    if (hi) ex[c] |= bit; else v[c] |= bit << 4;
-                }
-            }
-#pragma unroll
-            for (int c = 0; c < 2; ++c) { t[2 * c] = h2(__builtin_amdgcn_perm(ex[c], v[c], 0x05010400u)); t[2 * c + 1] = h2(__builtin_amdgcn_perm(ex[c], v[c], 0x07030602u)); }
-#pragma unroll
-            for (int c = 0; c < 4; ++c) t[c] = t[c] + bias;
-#pragma unroll
-            for (int c = 0; c < 4; ++c) t[c] = pk_fma(t[c], mul, add);
-        } else {
-            const int g = 2 * ks + (j >> 1);
-            const half2v bias = half2v{(_Float16) -1056.0f, (_Float16) -1056.0f};  // 1024 + q - 32
-            uint32_t lo4[2], hi2[2];
-#pragma unroll
-            for (int c = 0; c < 2; ++c) lo4[c] = ks ? (w.ql[c] >> 4) & 0x0F0F0F0Fu : w.ql[c] & 0x0F0F0F0Fu;
-#pragma unroll
-            for (int c = 0; c < 2; ++c) hi2[c] = g == 0 ? (w.qh[c] << 4) & 0x30303030u : g == 1 ? (w.qh[c] << 2) & 0x30303030u : g == 2 ? w.qh[c] & 0x30303030u : (w.qh[c] >> 2) & 0x30303030u;
-#pragma unroll
-            for (int c = 0; c < 2; ++c) v[c] = lo4[c] | hi2[c];
-#pragma unroll
-            for (int c = 0; c < 2; ++c) { t[2 * c] = h2(__builtin_amdgcn_perm(0x64646464u, v[c], 0x05010400u)); t[2 * c + 1] = h2(__builtin_amdgcn_perm(0x64646464u, v[c], 0x07030602u)); }
-#pragma unroll
-            for (int c = 0; c < 4; ++c) t[c] = t[c] + bias;
-#pragma unroll
-            for (int c = 0; c < 4; ++c) t[c] = t[c] * mul;
-        }
-        return __builtin_bit_cast(half8, u32x4{u2(t[0]), u2(t[1]), u2(t[2]), u2(t[3])});
-    };
+    auto dequant = [&](const Raw & w, int i) __attribute__((always_inline)) { return pf_dequant<TYPE>(w.ql, w.qh, (i >> 3) & 1, (i >> 2) & 1, i & 3, mul, add); };
 
     float16v acc[NT];
 #pragma unroll
@@ -473,9 +474,270 @@ __device__ __forceinline__ void pf_body(const PfP & p, const PfJob & jb, const i
     }
 }
 
+// ---- one round of workgroups (NT = 2 / 4): 128 rows x 32 NT tokens per workgroup, wave (g, kk) = rows [32 g, + 32) x the kk-th 64 k of every 128-k step ----
+// Few tokens leave little to multiply between two barriers. The loop above - 256 rows, two barriers per 16-k slice - spent 860 cycles on a slice of 128 tokens (128 of them in
+// MFMAs), half of them in barriers with nothing else left in it, and a launch had 16-64 tiles whose last K slice then read all slabs and stored 16-byte pieces of 32 token rows
+// by itself (14 of the 34 us of a 4096 x 4096 launch). Here: one barrier per 128 k; both halves of a step are multiplied side by side and added up through LDS at the end (half the
+// slabs of a K split for the same number of workgroups); three activation buffers, weights requested 2 to 4 steps ahead; tiles of 128 rows, so that twice as many
+// workgroups share the reduction; results cross LDS once more and are stored as whole 128-byte pieces of a token row.
+// What bounds it: the DMA of 41 KB of operands per 128 x 128 x 128 products (0.73 of a step's 1.2 us by itself) next to a step's 0.87 us of LDS reads, dequantization and MFMAs.
+// Llama-3-8B's launches at 101 tokens, Q4_K, us before / now: wq | wk | wv 37 / 24, wo 34 / 23, ffn_gate | ffn_up 61 / 50, ffn_down 54 / 36.6. Taken back: 64 rows and a quarter of the
+// k per wave (half the LDS reads: no change, 1-2 us more for the longer merge); two activation buffers instead of three (2-10 % slower).
+template <int TYPE> constexpr int mid_slot() { return TYPE == PM_Q8_0 ? 4096 : PfT<TYPE>::NSTREAM * 1024; }           // 128 k of 32 rows
+template <int TYPE> constexpr int mid_ahead() { return TYPE == PM_Q8_0 ? 2 : TYPE == PM_Q6_K ? 3 : 4; }               // weights are requested this many steps ahead (what LDS has room for)
+template <int TYPE> constexpr int mid_group_bytes() { return (mid_ahead<TYPE>() + 1) * mid_slot<TYPE>() + 2048 + (TYPE == PM_Q5_K ? 4096 : TYPE == PM_Q6_K ? 1024 : 0); }   // + four headers, four qh, two groups of d
+template <int N> __device__ __forceinline__ void mid_wait() { asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" : : "n"(N) : "memory"); }
+
+template <int TYPE, int NT>
+__device__ __forceinline__ void mid_body(const PfP & p, const PfJob & jb, const int n0, const int t0, uint8_t * smem, const int role, const int ks, const int S, const int tile_id) {
+    constexpr int HB = NT * 32 * 128, BBUF = 2 * HB;           // activations: 32 NT tokens x 64 halfs, two of them per step
+    constexpr int SLOT = mid_slot<TYPE>(), AG = mid_group_bytes<TYPE>(), NH = NT / 2, AHEAD = mid_ahead<TYPE>(), HDR = (AHEAD + 1) * SLOT, XTRA = HDR + 2048;
+    constexpr bool K45 = TYPE == PM_Q4_K || TYPE == PM_Q5_K, Q8 = TYPE == PM_Q8_0;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), g = wave & 3, kk = wave >> 2;       // (waves w and w + 4 share a SIMD)
+    const int r = lane & 31, h = lane >> 5;
+    const int K = p.K, nsteps = K / 128, nb = (K + 255) / 256;  // (Q8_0 rows may end on half a super-block: one step)
+    uint8_t * const ag = smem + 3 * BBUF + g * AG;              // the row group's weights: slots of the steps in turn, header of super-block b % 4
+    const uint32_t lds0 = (uint32_t) (uintptr_t) (__attribute__((address_space(3))) uint8_t *) smem, ag_l = lds0 + 3 * BBUF + g * AG;
+    const uint8_t * const Wg = jb.W;
+    const int nw = n0 + 32 * (role ? g & 1 : g);                // first row of this wave
+    const uint32_t wrow = (uint32_t) min(nw + r, jb.N - 1) * (uint32_t) jb.row_stride;
+    const uint8_t * const Xg = (const uint8_t *) p.Xh;
+    uint32_t xsrc[2 * NT];                                      // instruction q: 64-k half q / NT, token rows 8 (g + 4 (q % NT)) .. + 8 (swizzled as above)
+#pragma unroll
+    for (int q = 0; q < 2 * NT; ++q) {
+        const int t = 8 * (g + 4 * (q % NT)) + (lane >> 3);
+        xsrc[q] = (uint32_t) min(t0 + t, p.T - 1) * (uint32_t) (2 * K) + 128u * (uint32_t) (q / NT) + 16u * (uint32_t) ((lane & 7) ^ ((t >> 1) & 7));
+    }
+    const uint32_t boff0 = (uint32_t) (kk * HB + r * 128 + ((h ^ ((r >> 1) & 7)) << 4));
+    const uint32_t aoff = (uint32_t) (r * 16 + 8 * h);
+
+    // Requests return in order, and weights come from memory, activations mostly from L2: the waves of the first half request the weights, MID_AHEAD steps ahead, those of the
+    // second half the activations, one step ahead (with both behind one counter every weight was waited for after two steps)
+    // part u (0..3) of step s's requests
+    auto issue_A = [&](int s, uint32_t sl, bool even, int u) __attribute__((always_inline)) {
+        const uint32_t sc = (uint32_t) min(s, nsteps - 1);
+        const int b = s >> 1;
+        const uint32_t bc = (uint32_t) min(b, nb - 1);
+        if (u < SLOT / 1024) {                                  // stream u
+            uint32_t off;
+            if (Q8) off = (u & 1 ? (uint32_t) K / 2u : 0u) + (4u * sc + 2u * (uint32_t) (u >> 1) + (uint32_t) h) * 16u;       // blocks 2 k + h of k-step k = 2 s + u / 2, stream qa / qb
+            else if (TYPE == PM_Q5_K) off = (sc >> 1) * 176u + 48u + (sc & 1u) * 64u + 32u * (uint32_t) h + 16u * (uint32_t) u;
+            else off = 16u * (uint32_t) h + 32u * sc + (uint32_t) u * (uint32_t) nb * 64u;
+            dma16(Wg, wrow + off, ag_l + sl + u * 1024);
+        }
+        if (even && u == 3) {
+            const uint32_t off = TYPE == PM_Q4_K ? (uint32_t) nb * 128u + bc * 16u : TYPE == PM_Q5_K ? bc * 176u : Q8 ? (uint32_t) K + bc * 16u : pm_q6k_sc_off((uint32_t) nb, bc);
+            if (h == 0) dma16(Wg, wrow + off, ag_l + HDR + (b & 3) * 512);
+        }
+        if (even && u == 2) {
+            if (TYPE == PM_Q5_K) dma16(Wg, wrow + bc * 176u + 16u + 16u * (uint32_t) h, ag_l + XTRA + (b & 3) * 1024);
+            // (the d's of a group of eight super-blocks: with every one of them, the same bytes again)
+            if (TYPE == PM_Q6_K && h == 0) dma16(Wg, wrow + pm_q6k_d_off((uint32_t) nb, (uint32_t) (8 * min(b >> 3, (nb - 1) >> 3))), ag_l + XTRA + ((b >> 3) & 1) * 512);
+        }
+    };
+    auto issue_B = [&](int s, uint32_t bb, int u) __attribute__((always_inline)) {
+        const uint32_t sc = (uint32_t) min(s, nsteps - 1);
+#pragma unroll
+        for (int v = 0; v < NH; ++v) { const int q = NH * u + v; dma16(Xg, xsrc[q] + sc * 256u, lds0 + bb + (q / NT) * HB + (g + 4 * (q % NT)) * 1024); }
+    };
+    // end of an even / odd step: the next one's weights (all but those of the MID_AHEAD - 1 steps behind it) and activations are there, this wave's LDS reads are through
+    auto settle = [&](bool even) __attribute__((always_inline)) {
+        constexpr int W = SLOT / 1024, E = TYPE == PM_Q5_K || TYPE == PM_Q6_K ? 2 : 1;
+        if (kk) mid_wait<2 * NT>();
+        else if (even) mid_wait<(AHEAD - 1) * W + AHEAD / 2 * E>();
+        else mid_wait<(AHEAD - 1) * W + (AHEAD - 1) / 2 * E>();
+        __builtin_amdgcn_s_barrier();
+    };
+
+    float16v acc[NT];
+#pragma unroll
+    for (int jt = 0; jt < NT; ++jt)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) acc[jt][e] = 0.0f;
+    // the 4 slices of this wave's half of the step in buffer bb / slot sl: 128-k half mm of super-block b
+    // a quarter of the step's requests behind each slice's MFMAs (an issue blocks the wave for 60-180 cycles: in front of the step they were 0.4 of its 1.25 us)
+    auto multiply = [&](int b, int mm, uint32_t bb, uint32_t sl, auto && request) __attribute__((always_inline)) {
+        half8 bf[2][NT], af[2];
+        auto read_B = [&](int j) __attribute__((always_inline)) {
+#pragma unroll
+            for (int jt = 0; jt < NT; ++jt) bf[j & 1][jt] = *(const half8 *) (smem + bb + jt * 4096 + (boff0 ^ (uint32_t) (j << 5)));
+        };
+        u32x4 hd = {0, 0, 0, 0};
+        uint16_t d6 = 0;
+        const uint8_t * hp = ag + HDR + (b & 3) * 512 + r * 16;
+        if (K45) hd = *(const u32x4 *) hp;
+        else hd[0] = *(const uint32_t *) (hp + (2 * mm + kk) * 4);                            // the 4 scales (Q6_K), the 2 d's (Q8_0) of this wave's 64 k
+        if (TYPE == PM_Q6_K) d6 = *(const uint16_t *) (ag + XTRA + ((b >> 3) & 1) * 512 + r * 16 + (b & 7) * 2);
+        const uint8_t * ap = ag + sl + aoff;
+        u32x2 ql[4], qh[2] = {{0, 0}, {0, 0}};
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            if (Q8) ql[j] = *(const u32x2 *) (ap + kk * 2048 + (j & 1) * 1024 + (j >> 1) * 512);
+            else if (K45) { if (j < 2) ql[j] = *(const u32x2 *) (ap + j * 1024 + kk * 512); else ql[j] = ql[j - 2]; }   // (slices 2, 3: the high nibbles)
+            else ql[j] = *(const u32x2 *) (ap + (j >> 1) * 1024 + (j & 1) * 512);
+        }
+        if (TYPE == PM_Q5_K)
+#pragma unroll
+            for (int v = 0; v < 2; ++v) qh[v] = *(const u32x2 *) (ag + XTRA + (b & 3) * 1024 + v * 512 + aoff);
+        if (TYPE == PM_Q6_K)
+#pragma unroll
+            for (int v = 0; v < 2; ++v) qh[v] = *(const u32x2 *) (ap + 2048 + v * 512);
+        half2v mul = {0, 0}, add = {0, 0};
+        auto operand = [&](int j) __attribute__((always_inline)) {
+            if (K45 && (j & 1) == 0) {
+                const int sh = 8 * (2 * kk + (j >> 1));                                       // 32-weight sub-block 4 mm + 2 kk + j / 2
+                const uint32_t a = hd[1] >> sh, m = hd[2] >> sh, c = hd[3] >> sh;
+                const int sc = (int) (mm ? (c & 0x0Fu) | ((a & 0xC0u) >> 2) : a & 63u), mn = (int) (mm ? ((c >> 4) & 0x0Fu) | ((m & 0xC0u) >> 2) : m & 63u);
+                const _Float16 ds = (_Float16) (h2f((uint16_t) (hd[0] & 0xFFFF)) * (float) sc), ms = (_Float16) (h2f((uint16_t) (hd[0] >> 16)) * (float) mn);
+                mul = half2v{ds, ds}; add = half2v{(_Float16) -ms, (_Float16) -ms};
+            } else if (TYPE == PM_Q6_K) {
+                const _Float16 dd = (_Float16) (h2f(d6) * (float) (int) (int8_t) (hd[0] >> (8 * j)));
+                mul = half2v{dd, dd};
+            } else if (Q8 && (j & 1) == 0) {
+                const _Float16 dd = __builtin_bit_cast(_Float16, (uint16_t) (hd[0] >> (16 * (j >> 1))));
+                mul = half2v{dd, dd};
+            }
+            af[j & 1] = pf_dequant<TYPE>(ql[j], qh[j & 1], mm, kk, j, mul, add);
+        };
+        read_B(0);
+        operand(0);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            if (j < 3) { read_B(j + 1); operand(j + 1); }
+#pragma unroll
+            for (int jt = 0; jt < NT; ++jt) acc[jt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[j & 1], bf[j & 1][jt], acc[jt], 0, 0, 0);
+            request(j);
+        }
+    };
+
+    // split K: slice ks of S takes the super-blocks [b0, b1)
+    const int b0 = (int) ((long) ks * nb / S), b1 = (int) ((long) (ks + 1) * nb / S);
+    uint32_t bb = 0, bn = BBUF, bw = 2 * BBUF, sl = 0, sw = AHEAD * SLOT;       // buffers of steps s, s + 1, s + 2, slots of steps s and s + AHEAD
+    auto request = [&](int s, bool even, int u) __attribute__((always_inline)) { if (kk) issue_B(s + 2, bw, u); else issue_A(s + AHEAD, sw, AHEAD & 1 ? !even : even, u); };
+    auto turn = [&] __attribute__((always_inline)) { const uint32_t t = bb; bb = bn; bn = bw; bw = t; sw = sl; sl = sl == AHEAD * SLOT ? 0 : sl + SLOT; };
+#pragma unroll
+    for (int u = 0; u < 8; ++u) if (kk) issue_B(2 * b0 + (u >> 2), u & 4 ? bn : bb, u & 3);
+#pragma unroll
+    for (int w = 0; w < AHEAD; ++w)
+#pragma unroll
+        for (int u = 0; u < 4; ++u) if (!kk) issue_A(2 * b0 + w, w * SLOT, (w & 1) == 0, u);
+    settle(false);
+    for (int b = b0; b < b1; ++b) {
+        multiply(b, 0, bb, sl, [&](int u) __attribute__((always_inline)) { request(2 * b, true, u); });
+        settle(true);
+        turn();
+        if (Q8 && 2 * b + 1 >= nsteps) break;
+        multiply(b, 1, bb, sl, [&](int u) __attribute__((always_inline)) { request(2 * b + 1, false, u); });
+        settle(false);
+        turn();
+    }
+    mid_wait<0>();                                             // (the last steps' look-ahead still lands in the buffers)
+    __syncthreads();
+    // ---- the two halves of K: every wave keeps its rows' tokens [32 NH kk, + 32 NH) and takes the partner's sums of them
+    f32x4 * const xl = (f32x4 *) smem;
+    float16v own[NH];
+#pragma unroll
+    for (int i = 0; i < NH; ++i) {
+        const float16v give = kk ? acc[i] : acc[NH + i];
+        own[i] = kk ? acc[NH + i] : acc[i];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) xl[((wave * NH + i) * 4 + q) * 64 + lane] = f32x4{give[4 * q], give[4 * q + 1], give[4 * q + 2], give[4 * q + 3]};
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < NH; ++i)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const f32x4 o = xl[(((wave ^ 4) * NH + i) * 4 + q) * 64 + lane];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) own[i][4 * q + e] += o[e];
+        }
+    __syncthreads();
+    // ---- split K: slabs, ticket, the last arriver adds them up in slice order (as above). The slabs are written through and read past the caches: a release of everything this
+    //      XCD's L2 holds cost more than the hand-over. Four slabs are on their way at a time (one by one: a trip to memory each, 10 us at S = 8)
+    if (S > 1) {
+        constexpr int TILE = 8 * NH * 4 * 64, Q = NH * 4;
+        const __amdgpu_buffer_rsrc_t rs = coh_rsrc((f32x4 *) p.ws + (size_t) tile_id * S * TILE);
+        const uint32_t at = (uint32_t) ((wave * Q) * 64 + lane) * 16u;
+#pragma unroll
+        for (int q = 0; q < Q; ++q)
+            __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, f32x4{own[q / 4][4 * (q % 4)], own[q / 4][4 * (q % 4) + 1], own[q / 4][4 * (q % 4) + 2], own[q / 4][4 * (q % 4) + 3]}), rs,
+                                                   (int) (at + (uint32_t) ks * (TILE * 16u) + (uint32_t) q * 1024u), 0, 17);
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();
+        if (tid == 0) *(volatile unsigned *) smem = __hip_atomic_fetch_add(p.cnt + tile_id, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __syncthreads();
+        if (*(volatile unsigned *) smem != (unsigned) (S - 1)) return;
+        if (tid == 0) __hip_atomic_store(p.cnt + tile_id, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+        for (int i = 0; i < NH; ++i)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) own[i][e] = 0.0f;
+        for (int u = 0; u < S; u += 4) {
+            u32x4 v[4][Q];
+#pragma unroll
+            for (int w = 0; w < 4; ++w)
+#pragma unroll
+                for (int q = 0; q < Q; ++q) v[w][q] = coh_ld16u(rs, at + (uint32_t) min(u + w, S - 1) * (TILE * 16u) + (uint32_t) q * 1024u);
+#pragma unroll
+            for (int w = 0; w < 4; ++w) {
+                if (u + w >= S) break;
+#pragma unroll
+                for (int q = 0; q < Q; ++q)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) own[q / 4][4 * (q % 4) + e] += __builtin_bit_cast(f32x4, v[w][q])[e];
+            }
+        }
+        __syncthreads();                                        // (the ticket word is tile memory)
+    }
+    // ---- pair tiles: the gate waves park their sums in LDS (same lane, same register index as the up wave that needs them)
+    if (role) {
+        if (role == 1) {
+#pragma unroll
+            for (int i = 0; i < NH; ++i)
+#pragma unroll
+                for (int q = 0; q < 4; ++q) xl[(((2 * kk + (g & 1)) * NH + i) * 4 + q) * 64 + lane] = f32x4{own[i][4 * q], own[i][4 * q + 1], own[i][4 * q + 2], own[i][4 * q + 3]};
+        }
+        __syncthreads();
+        if (role == 1) return;
+#pragma unroll
+        for (int i = 0; i < NH; ++i)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const f32x4 gg = xl[(((2 * kk + (g & 1)) * NH + i) * 4 + q) * 64 + lane];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) own[i][4 * q + e] *= gg[e] / (1.0f + expf(-gg[e]));
+            }
+    }
+    // ---- epilogue: C[row = (e & 3) + 8 (e >> 2) + 4 h][token = r] crosses a wave-private LDS tile [token][32 rows + 4]; 8 lanes then hold a token's 32 rows
+    uint8_t * const xe = smem + 8 * NH * 4096 + wave * (32 * 144);
+#pragma unroll
+    for (int i = 0; i < NH; ++i) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) *(f32x4 *) (xe + r * 144 + (8 * q + 4 * h) * 4) = f32x4{own[i][4 * q], own[i][4 * q + 1], own[i][4 * q + 2], own[i][4 * q + 3]};
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const int tr = 8 * q + (lane >> 3), t = t0 + 32 * (kk * NH + i) + tr, n = nw + (lane & 7) * 4;
+            f32x4 v = *(const f32x4 *) (xe + tr * 144 + (lane & 7) * 16);
+            if (t >= p.T || n >= jb.N) continue;                // (N is a multiple of 4)
+            const long o = (long) t * jb.ldy + n;
+            if (jb.bias) v += ld_g((const f32x4 *) (jb.bias + n));
+            if (jb.resid) v += ld_g((const f32x4 *) (jb.resid + o));
+            if (jb.silu_gate) {
+                const f32x4 gg = ld_g((const f32x4 *) (jb.silu_gate + o));
+#pragma unroll
+                for (int e = 0; e < 4; ++e) v[e] *= gg[e] / (1.0f + expf(-gg[e]));
+            }
+            if (jb.Yh) *(PM_G half4v *) (jb.Yh + o) = half4v{(_Float16) v[0], (_Float16) v[1], (_Float16) v[2], (_Float16) v[3]};
+            else *(PM_G f32x4 *) (jb.Y + o) = v;
+        }
+    }
+}
+
 // block id -> (row tile, token tile): XCD x = id % 8 takes the row tiles x, x + 8, ..; its consecutive slots sweep the token tiles of one row tile, so the
 // workgroups that run together on an XCD share a few row tiles of weights and the activation k-slices in its L2 (mmq_big.hip's mapping)
-template <int TA, int TB, int NT, int EXP = 0>
+template <int TA, int TB, int NT, bool MID = false, int EXP = 0>
 __global__ __launch_bounds__(PF_NTHR) void gemm_pf_kernel(PfP p) {
     extern __shared__ __attribute__((aligned(1024))) uint8_t pf_smem[];
     const int id = (int) blockIdx.x, x = id & 7;
@@ -489,22 +751,31 @@ __global__ __launch_bounds__(PF_NTHR) void gemm_pf_kernel(PfP p) {
     const int tile_n = x + 8 * (slot / p.nt_t), tile_t = slot % p.nt_t;
     PfJob jb = p.job[0];                                       // (selected field by field with static indices: a run-time index would put the table into scratch)
     int n0, role = 0;
-    if (p.pair) {                                              // 128-row tiles of job 0 (waves 0-3) and job 1 (waves 4-7)
-        role = 1 + __builtin_amdgcn_readfirstlane((int) (threadIdx.x >> 8));
+    constexpr int ROWS = MID ? 128 : 256;
+    if (p.pair) {                                              // ROWS / 2-row tiles of job 0 (waves 0-3; mid_body: row groups 0, 1) and job 1
+        role = 1 + __builtin_amdgcn_readfirstlane((int) (MID ? (threadIdx.x >> 7) & 1 : threadIdx.x >> 8));
         if (role == 2) jb = p.job[1];
-        n0 = tile_n * 128;
+        n0 = tile_n * (ROWS / 2);
     } else {
 #pragma unroll
         for (int q = 1; q < PF_MAX_JOBS; ++q) if (q < p.njobs && tile_n >= p.job[q].tile0) jb = p.job[q];
-        n0 = (tile_n - jb.tile0) * 256;
+        n0 = (tile_n - jb.tile0) * ROWS;
     }
     const int t0 = tile_t * 32 * NT;
     const int tile_id = (slot - p.full) * 8 + x;                 // (split tiles only: slab and counter index)
-    if (TA == TB || jb.type == TA) pf_body<TA, NT, EXP>(p, jb, n0, t0, pf_smem, role, ks, S, tile_id);
-    else pf_body<TB, NT, EXP>(p, jb, n0, t0, pf_smem, role, ks, S, tile_id);
+    if constexpr (!MID) {
+        if (TA == TB || jb.type == TA) pf_body<TA, NT, EXP>(p, jb, n0, t0, pf_smem, role, ks, S, tile_id);
+        else pf_body<TB, NT, EXP>(p, jb, n0, t0, pf_smem, role, ks, S, tile_id);
+    } else {
+        if (TA == TB || jb.type == TA) mid_body<TA, NT>(p, jb, n0, t0, pf_smem, role, ks, S, tile_id);
+        else mid_body<TB, NT>(p, jb, n0, t0, pf_smem, role, ks, S, tile_id);
+    }
 }
 
-template <int TA, int TB, int NT> constexpr size_t pf_lds_bytes() { return (size_t) 3 * NT * 32 * 128 + (size_t) 8 * (pf_wave_bytes<TA>() > pf_wave_bytes<TB>() ? pf_wave_bytes<TA>() : pf_wave_bytes<TB>()); }
+template <int TA, int TB, int NT, bool MID = false> constexpr size_t pf_lds_bytes() {
+    if (!MID) return (size_t) 3 * NT * 32 * 128 + (size_t) 8 * (pf_wave_bytes<TA>() > pf_wave_bytes<TB>() ? pf_wave_bytes<TA>() : pf_wave_bytes<TB>());
+    return (size_t) 6 * NT * 32 * 128 + (size_t) 4 * (mid_group_bytes<TA>() > mid_group_bytes<TB>() ? mid_group_bytes<TA>() : mid_group_bytes<TB>());
+}
 
 void pf_allow_lds(const void * kern, size_t lds) {
     struct E { const void * k; int dev; };
@@ -554,7 +825,7 @@ int pm_gemm_pf_check(int type, int K, int N, int T) {
     return 0;
 }
 
-// The launch geometry of `tiles` row tiles (256 rows; pair launches: 128 rows of each matrix) x T tokens over K on a device of `cus` CUs in 8 XCDs - host
+// The launch geometry of `tiles` row tiles (256 rows, 128 where mid_body runs; pair launches: half of that of each matrix) x T tokens over K on a device of `cus` CUs in 8 XCDs - host
 // arithmetic only (tests/test_gemm_plan.py plans the layer shapes without a device). nt: 32-token sub-tiles per workgroup tile (2 / 4 / 8 = 64 / 128 / 256
 // tokens: a dequantized operand serves nt MFMAs; smaller tiles only where the batch has no more tokens). Few tiles - wo / ffn_down / wq | wk | wv at the
 // reference's default n_ubatch 512 (common/common.h:178) are 64-80 tiles for 256 CUs - are split along K: S slices per tile, the slice count that minimises
@@ -599,6 +870,17 @@ int pm_launch_gemm_pf(const pm_gemm_pf_job * jobs, int njobs, const void * xh, i
 int pm_launch_gemm_pf_ex(const pm_gemm_pf_job * jobs, int njobs, const void * xh, int K, int T, int pair, hipStream_t st) {
     if (njobs < 1 || njobs > PF_MAX_JOBS || !jobs || !xh) return -2;
     if (pair && (njobs != 2 || jobs[0].type != jobs[1].type || jobs[0].N != jobs[1].N || jobs[0].bias || jobs[0].resid || jobs[1].silu_gate)) return -2;
+    static const int force_nt = [] { const char * e = getenv("PM355_GEMM_PF_NT"); return e ? atoi(e) : 0; }();
+    const int cus = pm_device_cus();
+    // mid_body where its 128-row tiles are one round of workgroups: there a launch is its fixed costs and its K split. us, pf_body / mid_body, Q4_K: 4096 x 4096 101 tokens 28.9 / 22.0,
+    // 256 55.8 / 26.6, 512 60.1 / 35.7; 32768 x 4096 (256 tiles) 128 tokens 66 / 52. With more tiles the 256-row tiles' fewer bytes per product win: 40960 x 4096 (320) 101 tokens 65.8 / 70,
+    // 128256 x 4096 (Q6_K) 209 / 235; and with a long K over more than 256 tokens: 8192 x 28672 512 tokens 264 / 287 (256: 168 / 153; K = 8192 512 tokens: 109 / 89)
+    const int mid_nt = T <= 64 ? 2 : 4;
+    long mid_wgs = 0;
+    for (int j = 0; j < njobs && !(pair && j); ++j) mid_wgs += (jobs[j].N + (pair ? 63 : 127)) / (pair ? 64 : 128);
+    mid_wgs *= (T + 32 * mid_nt - 1) / (32 * mid_nt);
+    const bool mid = !force_nt && mid_wgs <= cus && (T <= 256 || K <= 16384);
+    const int rows = mid ? 128 : 256;
     PfP p = {};
     p.pair = pair ? 1 : 0;
     int tiles = 0, ta = jobs[0].type, tb = jobs[0].type;
@@ -609,28 +891,26 @@ int pm_launch_gemm_pf_ex(const pm_gemm_pf_job * jobs, int njobs, const void * xh
         PfJob & o = p.job[j];
         o.W = (const uint8_t *) jobs[j].W; o.Y = jobs[j].Y; o.Yh = (_Float16 *) jobs[j].Yh; o.bias = jobs[j].bias; o.resid = jobs[j].resid; o.silu_gate = jobs[j].silu_gate;
         o.row_stride = (long) pm_weight_row_stride(jobs[j].type, K); o.ldy = jobs[j].ldy ? jobs[j].ldy : jobs[j].N; o.type = jobs[j].type; o.N = jobs[j].N; o.tile0 = tiles;
-        tiles += (jobs[j].N + 255) / 256;
+        tiles += (jobs[j].N + rows - 1) / rows;
     }
-    if (pair) tiles = (jobs[0].N + 127) / 128;
+    if (pair) tiles = (jobs[0].N + rows / 2 - 1) / (rows / 2);
     if (ta > tb) { const int t = ta; ta = tb; tb = t; }       // (Q4_K, Q6_K) in that order
     static const int grp = [] { const char * e = getenv("PM355_GEMM_PF_GROUP"); return e ? atoi(e) : 0; }();
     p.grp = grp;
     p.njobs = njobs; p.nt_n = tiles; p.Xh = (const _Float16 *) xh; p.K = K; p.T = T;
-    static const int force_nt = [] { const char * e = getenv("PM355_GEMM_PF_NT"); return e ? atoi(e) : 0; }();
     static const int force_s = [] { const char * e = getenv("PM355_GEMM_PF_SPLITK"); return e ? atoi(e) : 0; }();
     static const bool no_mixed = [] { const char * e = getenv("PM355_GEMM_PF_MIXED"); return e && e[0] == '0'; }();
-    const int cus = pm_device_cus();
     // 256-token tiles (a dequantized operand serves 8 MFMAs; 128-token tiles only where the batch has no more tokens). Few tiles - wo / ffn_down / wq | wk | wv
     // at the reference's default n_ubatch 512 (common/common.h:178) are 64-80 tiles for 256 CUs - are split along K: S slices per tile, the slice count that
     // minimises  rounds of workgroups x (super-blocks per slice + ~3 for prologue, slab traffic and the reducer's pass)
     pm_gemm_pf_plan_t pl;
-    pm_gemm_pf_plan(tiles, K, T, cus, force_nt, force_s, no_mixed ? 0 : 1, &pl);
+    pm_gemm_pf_plan(tiles, K, T, cus, mid ? mid_nt : force_nt, force_s, no_mixed ? 0 : 1, &pl);
     const int nt = pl.nt, S = pl.splitk, full = pl.full, maxL = ((tiles + 7) / 8) * pl.nt_t;
     p.nt_t = pl.nt_t;
     p.splitk = S; p.full = full;
     const int split_slots = maxL - full;                       // per XCD
     if (S > 1) {
-        const size_t slab = (size_t) 8 * nt * 4 * 64 * 16, need = 65536 + (size_t) 8 * split_slots * S * slab;
+        const size_t slab = (size_t) (mid ? 4 : 8) * nt * 4 * 64 * 16, need = 65536 + (size_t) 8 * split_slots * S * slab;
         if ((size_t) 8 * split_slots > 16384) return -2;
         uint8_t * w = pf_workspace(st, need);
         if (!w) return -3;
@@ -648,9 +928,9 @@ int pm_launch_gemm_pf_ex(const pm_gemm_pf_job * jobs, int njobs, const void * xh
         if (!tr) (void) hipMalloc((void **) &tr, 42 * 8);
         p.trace = tr;
         switch (exp_sw) {
-#define PF_AB(E) case E: go(gemm_pf_kernel<PM_Q4_K, PM_Q4_K, 8, E>, pf_lds_bytes<PM_Q4_K, PM_Q4_K, 8>()); return 0;
+#define PF_AB(E) case E: go(gemm_pf_kernel<PM_Q4_K, PM_Q4_K, 8, false, E>, pf_lds_bytes<PM_Q4_K, PM_Q4_K, 8>()); return 0;
             PF_AB(3) PF_AB(4) PF_AB(8) PF_AB(16) PF_AB(24) PF_AB(27)
-#define PF_TR(E) case 128 + E: go(gemm_pf_kernel<PM_Q4_K, PM_Q4_K, 8, 128 + E>, pf_lds_bytes<PM_Q4_K, PM_Q4_K, 8>()); break;
+#define PF_TR(E) case 128 + E: go(gemm_pf_kernel<PM_Q4_K, PM_Q4_K, 8, false, 128 + E>, pf_lds_bytes<PM_Q4_K, PM_Q4_K, 8>()); break;
             PF_TR(0) PF_TR(3) PF_TR(8) PF_TR(16) PF_TR(24) PF_TR(27)
 #undef PF_TR
             default: return -2;
@@ -666,7 +946,7 @@ int pm_launch_gemm_pf_ex(const pm_gemm_pf_job * jobs, int njobs, const void * xh
         return 0;
     }
 #endif
-#define PF_GO(A, B) (nt == 8 ? go(gemm_pf_kernel<A, B, 8>, pf_lds_bytes<A, B, 8>()) : nt == 4 ? go(gemm_pf_kernel<A, B, 4>, pf_lds_bytes<A, B, 4>()) : go(gemm_pf_kernel<A, B, 2>, pf_lds_bytes<A, B, 2>()))
+#define PF_GO(A, B) (mid ? nt == 4 ? go(gemm_pf_kernel<A, B, 4, true>, pf_lds_bytes<A, B, 4, true>()) : go(gemm_pf_kernel<A, B, 2, true>, pf_lds_bytes<A, B, 2, true>()) : nt == 8 ? go(gemm_pf_kernel<A, B, 8>, pf_lds_bytes<A, B, 8>()) : nt == 4 ? go(gemm_pf_kernel<A, B, 4>, pf_lds_bytes<A, B, 4>()) : go(gemm_pf_kernel<A, B, 2>, pf_lds_bytes<A, B, 2>()))
     if (ta == tb) { if (ta == PM_Q4_K) PF_GO(PM_Q4_K, PM_Q4_K); else if (ta == PM_Q5_K) PF_GO(PM_Q5_K, PM_Q5_K); else if (ta == PM_Q8_0) PF_GO(PM_Q8_0, PM_Q8_0); else PF_GO(PM_Q6_K, PM_Q6_K); }
     else if (ta == PM_Q8_0 || tb == PM_Q8_0) return -1;      // (Q8_0 only as a launch of its own: ffn_down of the files whose n_ff is no multiple of 256)
     else if (ta == PM_Q4_K && tb == PM_Q5_K) PF_GO(PM_Q4_K, PM_Q5_K);

@@ -697,6 +697,35 @@ def test_prompt_gemm_jobs_one_launch(P, oracle, types, T):
         assert nm < 1e-6, (t, nm)
 
 
+# one and several token tiles of 64 and 128 tokens, rows that end inside a 128-row tile and inside a wave's 32, fewer steps of K than are requested ahead, K slices (8 super-blocks and
+# more), for Q8_0 a last step that is half a super-block (in a slice and without one); 256 tiles, the last launch of one round, and 258, which the 256-row tiles take
+@pytest.mark.parametrize("t", QUANT_TYPES)
+@pytest.mark.parametrize("K,N,T", [(512, 132, 33), (768, 260, 64), (512, 4, 65), (4096, 388, 128), (2304, 128, 129), (1024, 1028, 257), (512, 32768, 40), (512, 33024, 40)])
+def test_prompt_gemm_tiles_of_128_rows(P, oracle, t, K, N, T):
+    """Against the general tiles (the same rows in a launch of more than 256 tiles): the operands are the same F16 numbers, so the results differ by the order of f32 sums only - at most
+    2 K 2^-24 sum |w x| between two orders; and against the exact f64 product of the dequantized weights."""
+    torch = P.torch
+    rng = np.random.default_rng(K + N + T)
+    if t == Q8_0:
+        K = {512: 640, 768: 896, 2304: 2176, 4096: 4224}.get(K, K)
+    uniq = min(N, 516)
+    blocks = rand_blocks(t, uniq, K, rng, scale=1.0).reshape(uniq, -1)
+    rows = lambda n: np.concatenate([blocks] * (n // uniq + 1))[:n].reshape(-1)
+    x = rng.normal(0, 1, (T, K)).astype(np.float32)
+    xd = _dev(P, x)
+    w, big = P.upload_weight(t, rows(N), K, N), P.upload_weight(t, rows(33024), K, 33024)
+    got = P.mul_mat_mfma(w, xd)
+    assert torch.equal(got, P.mul_mat_mfma(w, xd))
+    Wf = torch.from_numpy(np.stack([oracle.dequantize_row(t, b, K) for b in blocks]).astype(np.float64)).cuda()
+    xx = xd.double()
+    bound = 2 * K * 2.0 ** -24 * (xx.abs() @ Wf.abs().T)
+    assert ((P.mul_mat_mfma(big, xd)[:, :uniq].double() - got[:, :uniq].double()).abs() <= bound).all()
+    exact = xx @ Wf.T
+    for at in range(0, N - uniq + 1, uniq):
+        nm = ((got[:, at:at + uniq].double() - exact) ** 2).sum() / (exact ** 2).sum()
+        assert nm < 1e-6, (at, float(nm))
+
+
 @pytest.mark.parametrize("t", [Q4_K, Q5_K, Q6_K])
 @pytest.mark.parametrize("K,N,T", [(1024, 384, 200), (2048, 132, 64), (512, 256, 257)])
 def test_prompt_gemm_pair_tiles_silu_gate_times_up(P, oracle, t, K, N, T):
