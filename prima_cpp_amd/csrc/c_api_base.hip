@@ -12,6 +12,12 @@ int pm_api_fail(int code, const char * what, hipError_t e) {
     snprintf(g_err, sizeof(g_err), "%s%s%s", what, e != hipSuccess ? ": " : "", e != hipSuccess ? hipGetErrorString(e) : "");
     return code;
 }
+int pm_device_cus() {
+    static int cus[16] = {};
+    const int dv = pm_cur_dev();
+    if (!cus[dv]) { hipDeviceProp_t pr; cus[dv] = hipGetDeviceProperties(&pr, dv) == hipSuccess ? pr.multiProcessorCount : 256; }
+    return cus[dv];
+}
 #define HIP_TRY(expr) do { hipError_t e_ = (expr); if (e_ != hipSuccess) return pm_api_fail(PM355_E_HIP, #expr, e_); } while (0)
 static inline hipStream_t S(pm355_stream_t s) { return (hipStream_t) s; }
 

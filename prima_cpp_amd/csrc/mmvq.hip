@@ -136,13 +136,6 @@ bool type_ok(int t) { return t == PM_Q4_K || t == PM_Q5_K || t == PM_Q6_K || t =
 
 } // namespace
 
-static int g_num_cus_dev[16] = {};
-static int num_cus() {
-    const int dv = pm_cur_dev();
-    if (!g_num_cus_dev[dv]) { hipDeviceProp_t pr; g_num_cus_dev[dv] = hipGetDeviceProperties(&pr, dv) == hipSuccess ? pr.multiProcessorCount : 256; }
-    return g_num_cus_dev[dv];
-}
-
 int pm_gemv_units_per_row(int type, int64_t K) { return (int) (K / nv_of(type)); }
 
 // Validates a fused job list and fills the kernel argument block. ta <= tb are the (at most two) quant types in the
@@ -173,7 +166,7 @@ int pmv::gemv_fill(const pm_gemv_fused & a, int grid_fixed, GemvP & p, int & ta_
         if (ta != PM_Q4_K || (tb != PM_Q6_K && tb != PM_Q5_K)) return -1;
     }
     // one workgroup of 16 waves per CU; every workgroup takes an equal slice of the rows of EVERY job
-    int grid = grid_fixed > 0 ? grid_fixed : (1024 / PM_GEMV_BLOCK) * num_cus();
+    int grid = grid_fixed > 0 ? grid_fixed : (1024 / PM_GEMV_BLOCK) * pm_device_cus();
     long tot_rows = 0;
     for (int j = 0; j < a.njobs; ++j) tot_rows += a.job[j].N;
     int rows_cap = PM_MAX_ROWS_PER_WG;
@@ -233,8 +226,6 @@ int pmv::gemv_fill(const pm_gemv_fused & a, int grid_fixed, GemvP & p, int & ta_
     ta_out = ta; tb_out = tb; pair_out = pair; lds_out = lds; grid_out = grid;
     return 0;
 }
-
-int pm_device_cus() { return num_cus(); }
 
 int pm_gemv_fused_check(const pm_gemv_fused & a) {
     GemvP p; int ta, tb, grid; bool pair; size_t lds;
