@@ -386,6 +386,22 @@ def test_rope_kv_store_vs_oracle(P, oracle, mode, with_ff):
     assert not kc_h[:pos0].any() and not kc_h[pos0 + T:].any() and not vc_h[:, :pos0].any() and not vc_h[:, pos0 + T:].any()
 
 
+@pytest.mark.parametrize("T,H,Hkv,dh,n_dims,mode,ff", [(256, 8, 2, 128, 128, 0, True), (257, 3, 1, 64, 64, 2, False), (300, 5, 5, 96, 64, 0, False), (319, 4, 2, 256, 128, 2, True)])
+def test_rope_kv_store_of_a_prompt_equals_small_batches(P, T, H, Hkv, dh, n_dims, mode, ff):
+    """256 tokens and more take a workgroup per token and turned tiles of V: the same bits as batches of fewer, and nothing written beside them"""
+    torch = P.torch
+    g = torch.Generator(device="cuda").manual_seed(T)
+    q, k, v = (torch.randn(T, n * dh, generator=g, device="cuda") for n in (H, Hkv, Hkv))
+    f = 1 + torch.rand(dh // 2, generator=g, device="cuda") if ff else None
+    kw = dict(freq_factors=f, mode=mode, freq_base=500000.0, n_dims=n_dims)
+    n_ctx, pos0 = 384, 37
+    one, many = ([torch.zeros(n_ctx * Hkv * dh, dtype=torch.int16, device="cuda") for _ in range(2)] for _ in range(2))
+    got = P.rope_kv_store(q, k, v, *one, pos0, H, Hkv, dh, n_ctx, **kw)
+    parts = [P.rope_kv_store(q[i:i + 160], k[i:i + 160], v[i:i + 160], *many, pos0 + i, H, Hkv, dh, n_ctx, **kw) for i in range(0, T, 160)]
+    assert all(torch.equal(a, torch.cat(b)) for a, b in zip(got, zip(*parts)))
+    assert all(torch.equal(a, b) for a, b in zip(one, many))
+
+
 @pytest.mark.parametrize("n_past,T", [(0, 1), (5, 1), (63, 1), (200, 3), (0, 4)])
 def test_attn_decode_vs_oracle(P, oracle, n_past, T):
     """Same rounding points as the reference (q and p rounded to F16, F16 K/V): compare with an exact numpy
