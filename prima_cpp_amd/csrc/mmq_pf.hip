@@ -872,14 +872,13 @@ int pm_launch_gemm_pf_ex(const pm_gemm_pf_job * jobs, int njobs, const void * xh
     if (pair && (njobs != 2 || jobs[0].type != jobs[1].type || jobs[0].N != jobs[1].N || jobs[0].bias || jobs[0].resid || jobs[1].silu_gate)) return -2;
     static const int force_nt = [] { const char * e = getenv("PM355_GEMM_PF_NT"); return e ? atoi(e) : 0; }();
     const int cus = pm_device_cus();
-    // mid_body where its 128-row tiles are one round of workgroups: there a launch is its fixed costs and its K split. us, pf_body / mid_body, Q4_K: 4096 x 4096 101 tokens 28.9 / 22.0,
-    // 256 55.8 / 26.6, 512 60.1 / 35.7; 32768 x 4096 (256 tiles) 128 tokens 66 / 52. With more tiles the 256-row tiles' fewer bytes per product win: 40960 x 4096 (320) 101 tokens 65.8 / 70,
-    // 128256 x 4096 (Q6_K) 209 / 235; and with a long K over more than 256 tokens: 8192 x 28672 512 tokens 264 / 287 (256: 168 / 153; K = 8192 512 tokens: 109 / 89)
+    // mid_body for up to 128 tokens where its 128-row tiles are one round of workgroups: there a launch is its fixed costs and its K split. us, pf_body / mid_body, Q4_K: 4096 x 4096
+    // 101 tokens 28.9 / 22.0, 4096 x 14336 50.4 / 35.7, 32768 x 4096 (256 tiles) 128 tokens 66 / 52. With more tiles the 256-row tiles' fewer bytes per product win: 40960 x 4096 (320)
+    // 101 tokens 65.8 / 70, 128256 x 4096 (Q6_K) 209 / 235
     const int mid_nt = T <= 64 ? 2 : 4;
     long mid_wgs = 0;
     for (int j = 0; j < njobs && !(pair && j); ++j) mid_wgs += (jobs[j].N + (pair ? 63 : 127)) / (pair ? 64 : 128);
-    mid_wgs *= (T + 32 * mid_nt - 1) / (32 * mid_nt);
-    const bool mid = !force_nt && mid_wgs <= cus && (T <= 256 || K <= 16384);
+    const bool mid = !force_nt && T <= 128 && mid_wgs <= cus;
     const int rows = mid ? 128 : 256;
     PfP p = {};
     p.pair = pair ? 1 : 0;
