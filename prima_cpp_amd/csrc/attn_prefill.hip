@@ -250,6 +250,8 @@ __global__ __launch_bounds__(512, 2) void attn_prompt_kernel(PfP p) {
     const int w_first = pos0 + q0, w_last = pos0 + min(q0 + 31, nq - 1);                         // positions of the wave's first and last query
     const int n_keys = MASK ? p.n_kv : pos0 + nq;                                                // cells the workgroup's last query sees
     const int n_it = (n_keys + KS - 1) / KS;
+    // cells this wave's queries see together
+    const int seen = MASK ? p.n_kv : w_last + 1;
 
     const uint32_t lds0 = (uint32_t) (uintptr_t) (__attribute__((address_space(3))) char *) smem;
     auto request = [&](int it, int stage) __attribute__((always_inline)) {
@@ -295,7 +297,7 @@ __global__ __launch_bounds__(512, 2) void attn_prompt_kernel(PfP p) {
         __syncthreads();
         if (it + 1 < n_it) request(it + 1, stage ^ 1);
         const int key0 = it * KS + kw * KT;
-        if (!live || key0 >= (MASK ? p.n_kv : w_last + 1)) continue;
+        if (!live || key0 >= seen) continue;
         const char * ks = smem + stage * STAGE, * vs = ks + KS * DH * 2;
         float16v s[ST];
 #pragma unroll
@@ -317,11 +319,13 @@ __global__ __launch_bounds__(512, 2) void attn_prompt_kernel(PfP p) {
 #pragma unroll
                 for (int g = 0; g < 4; ++g) {                     // registers 4 g .. + 4 = keys 16 (g >> 1) + 8 hf + 4 (g & 1) .. + 4
                     const int k0 = key0 + t * 32 + 16 * (g >> 1) + 8 * hf + 4 * (g & 1);
-                    float4 mv = float4{-INFINITY, -INFINITY, -INFINITY, -INFINITY};
-                    if (k0 + 3 < p.n_kv) {
-                        if (!p.mask_f16) mv = *(const float4 *) (mrow + k0);
-                        else { const u32x2 mh = *(const u32x2 *) (mrow16 + k0); mv = float4{h2f((uint16_t) (mh[0] & 0xFFFF)), h2f((uint16_t) (mh[0] >> 16)), h2f((uint16_t) (mh[1] & 0xFFFF)), h2f((uint16_t) (mh[1] >> 16))}; }
+                    if (k0 >= p.n_kv) {                           // (n_kv is a multiple of 4; whatever a cell behind n_kv holds, its score does not count)
+                        s[t][4 * g + 0] = s[t][4 * g + 1] = s[t][4 * g + 2] = s[t][4 * g + 3] = -INFINITY;
+                        continue;
                     }
+                    float4 mv;
+                    if (!p.mask_f16) mv = *(const float4 *) (mrow + k0);
+                    else { const u32x2 mh = *(const u32x2 *) (mrow16 + k0); mv = float4{h2f((uint16_t) (mh[0] & 0xFFFF)), h2f((uint16_t) (mh[0] >> 16)), h2f((uint16_t) (mh[1] & 0xFFFF)), h2f((uint16_t) (mh[1] >> 16))}; }
                     s[t][4 * g + 0] = fmaf(mv.x, LOG2E, s[t][4 * g + 0] * c); s[t][4 * g + 1] = fmaf(mv.y, LOG2E, s[t][4 * g + 1] * c);
                     s[t][4 * g + 2] = fmaf(mv.z, LOG2E, s[t][4 * g + 2] * c); s[t][4 * g + 3] = fmaf(mv.w, LOG2E, s[t][4 * g + 3] * c);
                 }
@@ -356,14 +360,28 @@ __global__ __launch_bounds__(512, 2) void attn_prompt_kernel(PfP p) {
                 l += e;
                 pr[2 * t + (r >> 3)][r & 7] = (_Float16) e;
             }
+        // cells behind the last attended one: a probability of 0 does not undo what they hold (0 x NaN), so they become zeros in LDS. Every wave of a key group writes the same bytes and
+        // waits for its own only
+        if (key0 + KT > n_keys)
+            for (int i = lane; i < DH * (KT / 8); i += 64) {
+                const int row = i / (KT / 8), ch = i % (KT / 8), n = n_keys - (key0 + 8 * ch);      // n: attended cells of the chunk
+                u32x4 * at = (u32x4 *) (smem + stage * STAGE + KS * DH * 2 + row * (KS * 2) + ((kw * (KT / 8) + ch) ^ (CV == 8 ? (row >> 1) & 7 : row & 15)) * 16);
+                if (n >= 8) continue;
+                u32x4 v = *at;
 #pragma unroll
-        for (int j = 0; j < 2 * ST; ++j)
+                for (int e = 0; e < 4; ++e) v[e] &= n >= 2 * e + 2 ? 0xFFFFFFFFu : n == 2 * e + 1 ? 0xFFFFu : 0u;
+                *at = v;
+            }
+#pragma unroll
+        for (int j = 0; j < 2 * ST; ++j) {
+            if (ST > 1 && j == 2 && key0 + 32 >= seen) break;      // (nor do the later tokens' cells belong to the queries of this wave)
 #pragma unroll
             for (int d = 0; d < DT; ++d) {
                 const int row = d * 32 + lr, ch = kw * (KT / 8) + 2 * j + hf;
                 const half8 v = *(const half8 *) (vs + row * (KS * 2) + (ch ^ (CV == 8 ? (row >> 1) & 7 : row & 15)) * 16);
                 o[d] = __builtin_amdgcn_mfma_f32_32x32x16_f16(v, pr[j], o[d], 0, 0, 0);
             }
+        }
     }
     l += __shfl_xor(l, 32);
     __syncthreads();                                              // (the stages become the exchange of the results)

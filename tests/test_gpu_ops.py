@@ -495,6 +495,43 @@ def test_attn_prefill_tiles_against_float64(P, H, Hkv, dh, T, past, mask):
         assert bool((off <= bound).all()), (h, float((off / bound).max()))
 
 
+def _masked_attention(P, q, K, V, m, n_kv, H, Hkv, dh, n_ctx, sc):
+    import ctypes as C
+    from prima_cpp_amd import lib as L
+    out = P.torch.empty((q.shape[0], H, dh), device="cuda")
+    f = L.declare("pm355_attn_prefill_masked_ex", C.c_int, [C.c_void_p] * 4 + [C.c_int64, C.c_void_p] + [C.c_int] * 6 + [C.c_float, C.c_int, C.c_void_p])
+    L.check(f(L.ptr(q), L.ptr(K), L.ptr(V), L.ptr(m), m.shape[1], L.ptr(out), q.shape[0], H, Hkv, dh, n_ctx, n_kv, float(sc), 0 if m.dtype == P.torch.float32 else 2, L.stream_ptr()), "masked")
+    return out
+
+
+@pytest.mark.parametrize("junk", [float("nan"), float("inf")])
+@pytest.mark.parametrize("H,Hkv,dh,T,past,n_kv", [
+    (8, 2, 128, 40, 3, None), (8, 2, 64, 70, 30, None), (64, 8, 128, 512, 33, None), (128, 8, 64, 1000, 29, None), (128, 8, 128, 1021, 0, None),
+    (8, 2, 128, 40, 0, 60), (8, 2, 64, 33, 0, 96), (64, 8, 128, 512, 32, 544), (64, 8, 64, 512, 32, 548), (128, 8, 128, 1000, 0, 1012)])
+def test_attn_prefill_does_not_look_behind_the_attended_cells(P, H, Hkv, dh, T, past, n_kv, junk):
+    """Cells behind the last attended one - of the causal form, and of n_kv with a mask - may hold anything: the same bits as with zeros there. Every tile, counts that end inside a stage of
+    keys, inside 32 and inside 8 of them"""
+    torch = P.torch
+    n = n_kv or past + T
+    n_ctx = -(-n // 32) * 32 + 64
+    g = torch.Generator(device="cuda").manual_seed(n + dh)
+    q = torch.randn((T, H * dh), generator=g, device="cuda")
+    outs = []
+    for fill in (0.0, junk):
+        g.manual_seed(n)
+        K = torch.randn((n_ctx, Hkv, dh), generator=g, device="cuda").half()
+        V = torch.randn((Hkv, dh, n_ctx), generator=g, device="cuda").half()
+        K[n:], V[:, :, n:] = fill, fill
+        if n_kv is None:
+            outs.append(P.attn_prefill(q, K, V, past, H, Hkv, dh, n_ctx, dh ** -0.5))
+            continue
+        hidden = torch.arange(n_kv, device="cuda")[None] > torch.arange(T, device="cuda")[:, None] + past
+        for dt in (torch.float32, torch.float16):
+            outs.append(_masked_attention(P, q, K, V, torch.zeros((T, n_kv), device="cuda", dtype=dt).masked_fill_(hidden, -np.inf), n_kv, H, Hkv, dh, n_ctx, dh ** -0.5))
+    assert all(bool(o.isfinite().all()) for o in outs)
+    assert all(torch.equal(o, w) for o, w in zip(outs[len(outs) // 2:], outs))
+
+
 @pytest.mark.parametrize("dh", [64, 128])
 @pytest.mark.parametrize("n_past", [0, 5, 255, 256, 700, 1023])
 def test_attn_decode_split_equals_single_workgroup_kernel(P, n_past, dh):
