@@ -273,11 +273,14 @@ __global__ __launch_bounds__(512, 2) void attn_prompt_kernel(PfP p) {
 
     // Q^T as B operand: lane (query lr, hf) holds q[query][16 kk + 8 hf .. + 8], rounded to F16 like the reference
     half8 q[KK];
+    // (times the sign of the scale: hidden scores are -inf in front of the positive factor c)
     {
         const float * qr = p.q + ((long) tq * p.H + h) * DH + 8 * hf;
+        const float sg = p.scale == 0.0f ? 0.0f : copysignf(1.0f, p.scale);
 #pragma unroll
         for (int kk = 0; kk < KK; ++kk) {
-            const float4 a = *(const float4 *) (qr + 16 * kk), b = *(const float4 *) (qr + 16 * kk + 4);
+            float4 a = *(const float4 *) (qr + 16 * kk), b = *(const float4 *) (qr + 16 * kk + 4);
+            a.x *= sg; a.y *= sg; a.z *= sg; a.w *= sg; b.x *= sg; b.y *= sg; b.z *= sg; b.w *= sg;
             q[kk] = half8{(_Float16) a.x, (_Float16) a.y, (_Float16) a.z, (_Float16) a.w, (_Float16) b.x, (_Float16) b.y, (_Float16) b.z, (_Float16) b.w};
         }
     }
@@ -289,7 +292,7 @@ __global__ __launch_bounds__(512, 2) void attn_prompt_kernel(PfP p) {
 #pragma unroll
         for (int r = 0; r < 16; ++r) o[d][r] = 0.0f;
     float m = NONE, l = 0.0f;
-    const float c = p.scale * LOG2E;
+    const float c = p.scale == 0.0f ? LOG2E : fabsf(p.scale) * LOG2E;
     const int kr = (lr & ~12) | ((lr & 4) << 1) | ((lr & 8) >> 1);
     for (int it = 0; it < n_it; ++it) {
         const int stage = it & 1;
@@ -341,7 +344,7 @@ __global__ __launch_bounds__(512, 2) void attn_prompt_kernel(PfP p) {
 #pragma unroll
             for (int r = 0; r < 16; ++r) mx = fmaxf(mx, s[t][r]);
         mx = fmaxf(mx, __shfl_xor(mx, 32));
-        if (!MASK) mx = fmaxf(mx * c, NONE);                      // (scores are scaled where the exponent is formed; scale > 0)
+        if (!MASK) mx = fmaxf(mx * c, NONE);                      // (scores are scaled where the exponent is formed; c > 0)
         const float mn = fmaxf(m, mx);
         if (__any(mn > m)) {
             const float corr = __builtin_amdgcn_exp2f(m - mn);

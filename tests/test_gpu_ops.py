@@ -532,6 +532,25 @@ def test_attn_prefill_does_not_look_behind_the_attended_cells(P, H, Hkv, dh, T, 
     assert all(torch.equal(o, w) for o, w in zip(outs[len(outs) // 2:], outs))
 
 
+@pytest.mark.parametrize("scale", [-0.09, 0.0])
+@pytest.mark.parametrize("H,Hkv,dh,T,past", [(8, 2, 128, 40, 60), (64, 8, 64, 300, 12)])
+def test_attn_prefill_scales_that_are_not_positive(P, H, Hkv, dh, T, past, scale):
+    """hidden cells stay hidden whatever the sign of the scale; the bound of test_attn_prefill_tiles_against_float64"""
+    torch = P.torch
+    n = past + T
+    n_ctx = -(-n // 32) * 32
+    g = torch.Generator(device="cuda").manual_seed(n)
+    q = torch.randn((T, H, dh), generator=g, device="cuda")
+    K = torch.randn((n_ctx, Hkv, dh), generator=g, device="cuda").half()
+    V = torch.randn((Hkv, dh, n_ctx), generator=g, device="cuda").half()
+    out = P.attn_prefill(q.view(T, -1), K, V, past, H, Hkv, dh, n_ctx, scale).view(T, H, dh)
+    hidden = torch.arange(n, device="cuda")[None] > torch.arange(T, device="cuda")[:, None] + past
+    for h in range(H):
+        k, v = K[:n, h * Hkv // H].double(), V[h * Hkv // H, :, :n].double()
+        p = ((q[:, h].half().double() @ k.T) * scale).masked_fill(hidden, -np.inf).softmax(-1)
+        assert bool(((out[:, h].double() - p @ v.T).abs() <= 1.1 * 2.0 ** -11 * (p @ v.abs().T) + 1e-6).all()), h
+
+
 @pytest.mark.parametrize("dh", [64, 128])
 @pytest.mark.parametrize("n_past", [0, 5, 255, 256, 700, 1023])
 def test_attn_decode_split_equals_single_workgroup_kernel(P, n_past, dh):
