@@ -227,7 +227,10 @@ __global__ __launch_bounds__(512, 2) void attn_prompt_kernel(PfP p) {
     constexpr int KW = 8 / QW, KT = KS / KW, ST = KT / 32;            // keys per wave and stage, 32-key score tiles
     constexpr int KK = DH / 16, DT = DH / 32, CK = DH / 8, CV = KS / 8;      // k-steps of a score tile, output tiles, 16-byte chunks per K row / V^T row
     constexpr int STAGE = KS * DH * 4, OS = DH + 4;
-    constexpr float NONE = -1e30f, LOG2E = 1.4426950408889634f;
+    constexpr float LOG2E = 1.4426950408889634f;
+    // the maxima below are in units of log2, with a mask in natural units - a mask entry times log2 e may overflow (the lowest f32 value), which would hide a cell that a row of such
+    // entries attends - and start from the lowest value there is
+    constexpr float NONE = MASK ? -INFINITY : -1e30f, UNIT = MASK ? LOG2E : 1.0f;
     static_assert(KT % 32 == 0, "whole score tiles");
     extern __shared__ __attribute__((aligned(1024))) char smem[];
     const int wave = __builtin_amdgcn_readfirstlane((int) threadIdx.x >> 6), lane = threadIdx.x & 63, lr = lane & 31, hf = lane >> 5;
@@ -292,7 +295,7 @@ __global__ __launch_bounds__(512, 2) void attn_prompt_kernel(PfP p) {
 #pragma unroll
         for (int r = 0; r < 16; ++r) o[d][r] = 0.0f;
     float m = NONE, l = 0.0f;
-    const float c = p.scale == 0.0f ? LOG2E : fabsf(p.scale) * LOG2E;
+    const float sc = p.scale == 0.0f ? 1.0f : fabsf(p.scale), c = sc * LOG2E;
     const int kr = (lr & ~12) | ((lr & 4) << 1) | ((lr & 8) >> 1);
     for (int it = 0; it < n_it; ++it) {
         const int stage = it & 1;
@@ -329,8 +332,8 @@ __global__ __launch_bounds__(512, 2) void attn_prompt_kernel(PfP p) {
                     float4 mv;
                     if (!p.mask_f16) mv = *(const float4 *) (mrow + k0);
                     else { const u32x2 mh = *(const u32x2 *) (mrow16 + k0); mv = float4{h2f((uint16_t) (mh[0] & 0xFFFF)), h2f((uint16_t) (mh[0] >> 16)), h2f((uint16_t) (mh[1] & 0xFFFF)), h2f((uint16_t) (mh[1] >> 16))}; }
-                    s[t][4 * g + 0] = fmaf(mv.x, LOG2E, s[t][4 * g + 0] * c); s[t][4 * g + 1] = fmaf(mv.y, LOG2E, s[t][4 * g + 1] * c);
-                    s[t][4 * g + 2] = fmaf(mv.z, LOG2E, s[t][4 * g + 2] * c); s[t][4 * g + 3] = fmaf(mv.w, LOG2E, s[t][4 * g + 3] * c);
+                    s[t][4 * g + 0] = fmaf(s[t][4 * g + 0], sc, mv.x); s[t][4 * g + 1] = fmaf(s[t][4 * g + 1], sc, mv.y);
+                    s[t][4 * g + 2] = fmaf(s[t][4 * g + 2], sc, mv.z); s[t][4 * g + 3] = fmaf(s[t][4 * g + 3], sc, mv.w);
                 }
         } else if (key0 + KT - 1 > w_first) {                     // (keys that some query of the wave does not see)
 #pragma unroll
@@ -345,9 +348,9 @@ __global__ __launch_bounds__(512, 2) void attn_prompt_kernel(PfP p) {
             for (int r = 0; r < 16; ++r) mx = fmaxf(mx, s[t][r]);
         mx = fmaxf(mx, __shfl_xor(mx, 32));
         if (!MASK) mx = fmaxf(mx * c, NONE);                      // (scores are scaled where the exponent is formed; c > 0)
-        const float mn = fmaxf(m, mx);
+        const float mn = fmaxf(m, mx), mr = MASK && mn == -INFINITY ? 0.0f : mn;      // (nothing visible so far: every exponent below is -inf)
         if (__any(mn > m)) {
-            const float corr = __builtin_amdgcn_exp2f(m - mn);
+            const float corr = __builtin_amdgcn_exp2f((m - mr) * UNIT);
             l *= corr; m = mn;
 #pragma unroll
             for (int d = 0; d < DT; ++d)
@@ -359,7 +362,7 @@ __global__ __launch_bounds__(512, 2) void attn_prompt_kernel(PfP p) {
         for (int t = 0; t < ST; ++t)
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
-                const float e = __builtin_amdgcn_exp2f(MASK ? s[t][r] - m : fmaf(s[t][r], c, -m));
+                const float e = __builtin_amdgcn_exp2f(MASK ? (s[t][r] - mr) * LOG2E : fmaf(s[t][r], c, -m));
                 l += e;
                 pr[2 * t + (r >> 3)][r & 7] = (_Float16) e;
             }
@@ -397,8 +400,8 @@ __global__ __launch_bounds__(512, 2) void attn_prompt_kernel(PfP p) {
 #pragma unroll
         for (int g = 0; g < KW; ++g) M = fmaxf(M, ml[((g * QW + qw) * 32 + lr) * 2]);
 #pragma unroll
-        for (int g = 0; g < KW; ++g) L += ml[((g * QW + qw) * 32 + lr) * 2 + 1] * __builtin_amdgcn_exp2f(ml[((g * QW + qw) * 32 + lr) * 2] - M);
-        f = __builtin_amdgcn_exp2f(m - M) / L;
+        for (int g = 0; g < KW; ++g) L += ml[((g * QW + qw) * 32 + lr) * 2 + 1] * __builtin_amdgcn_exp2f((ml[((g * QW + qw) * 32 + lr) * 2] - M) * UNIT);
+        f = __builtin_amdgcn_exp2f((m - M) * UNIT) / L;
     }
     // O^T[d][query]: queries are columns; through LDS, then a wave stores whole rows
 #pragma unroll

@@ -551,6 +551,32 @@ def test_attn_prefill_scales_that_are_not_positive(P, H, Hkv, dh, T, past, scale
         assert bool(((out[:, h].double() - p @ v.T).abs() <= 1.1 * 2.0 ** -11 * (p @ v.abs().T) + 1e-6).all()), h
 
 
+@pytest.mark.parametrize("H,Hkv,dh,T,n_kv", [(8, 2, 128, 40, 100), (64, 8, 128, 500, 512), (128, 8, 64, 1000, 1024)])
+@pytest.mark.parametrize("lowest", [float(np.finfo(np.float32).min), -1e32, float(np.finfo(np.float16).min)])
+def test_attn_prefill_masks_of_the_lowest_value(P, H, Hkv, dh, T, n_kv, lowest):
+    """Masks that hide with the lowest finite value of their type: cells beside visible ones weigh nothing, and a row of which every cell is hidden that way attends all of them like the sum of
+    score and mask says (the f32 sums are all the same number where the mask's step is larger than the scores; the F16 one leaves steps of 2^-8, so 2^-9 of every weight more in the bound)"""
+    torch = P.torch
+    f16 = lowest > -1e5
+    g = torch.Generator(device="cuda").manual_seed(n_kv)
+    q = torch.randn((T, H, dh), generator=g, device="cuda")
+    K = torch.randn((n_kv + 28, Hkv, dh), generator=g, device="cuda").half()[:-(-n_kv // 32) * 32].contiguous()
+    n_ctx = K.shape[0]
+    V = torch.randn((Hkv, dh, n_ctx), generator=g, device="cuda").half()
+    m = torch.zeros((T, n_kv), device="cuda").masked_fill_(torch.rand((T, n_kv), generator=g, device="cuda") < 0.3, lowest)
+    m[::3] = lowest
+    m = m.half() if f16 else m
+    sc = dh ** -0.5
+    out = _masked_attention(P, q.view(T, -1), K, V, m, n_kv, H, Hkv, dh, n_ctx, sc)
+    for h in range(0, H, max(1, H // 8)):
+        k, v = K[:n_kv, h * Hkv // H].double(), V[h * Hkv // H, :, :n_kv].double()
+        s = ((q[:, h].half().double() @ k.T) * sc + m.double()).float() if not f16 else (q[:, h].half().double() @ k.T) * sc + m.double()
+        p = s.double().softmax(-1)
+        bound = (1.1 * 2.0 ** -11 + (2.0 * 2.0 ** -9 if f16 else 0.0)) * (p @ v.abs().T) + 1e-6
+        off = (out[:, h].double() - p @ v.T).abs()
+        assert bool((off <= bound).all()), (h, float((off / bound).nan_to_num(1e9).max()))
+
+
 @pytest.mark.parametrize("dh", [64, 128])
 @pytest.mark.parametrize("n_past", [0, 5, 255, 256, 700, 1023])
 def test_attn_decode_split_equals_single_workgroup_kernel(P, n_past, dh):
