@@ -109,8 +109,8 @@ struct pm_window : pm355_model {
     // a pass over rows of several sequences (batch): every row's position and sequence in device memory, tiles for the matrix-core attention; rag is set while one is launched
     struct Ragged { const int32_t * pos, * seq, * tiles; int n_tiles, tile_q, max_cells; bool singles; };
     const Ragged * rag = nullptr; int32_t * d_rows = nullptr; float * head_lg = nullptr;
-    uint64_t * am_part = nullptr;                 // argmax scratch of up to HEAD_ROWS rows
-    int adv = 0, rot = 0;                         // what the launch that ends a step still does to the position counters (step_body; the argmax does it on its way)
+    uint64_t * am_part = nullptr;                 // argmax scratch of up to HEAD_ROWS rows: one user at a time, like the window's activations
+    struct Advance { int by, rotate; };           // what the launch that ends a step still does to the position counters (step_body; the argmax does it on its way and clears this)
     int batch_rows(const pm355_batch_entry * e, int n, float * d_logits, int32_t * d_argmax, hipStream_t st, bool * served);
 
     ~pm_window() override;
@@ -392,8 +392,10 @@ int gemv_f32(pm_window * m, const Tensor * const * ws, const Tensor * const * w2
     return pm_launch_gemv_fused(f, st);
 }
 
-// result_norm + lm_head (+ greedy argmax) on ONE hidden row (build_llama's last sub-graph, src/llama.cpp:11191-11215)
-int run_head(pm_window * m, const float * x_row, float * d_logits, int32_t * d_argmax, hipStream_t st, const double * ss_in = nullptr, int n_ss_in = 0) {
+// result_norm + lm_head (+ greedy argmax) on ONE hidden row (build_llama's last sub-graph, src/llama.cpp:11191-11215). alone: nothing of the window is shared with launches on other
+// streams (the caller's logits and index, no layers in front): the argmax then stays with one workgroup, whose partials need no scratch
+int run_head(pm_window * m, const float * x_row, float * d_logits, int32_t * d_argmax, hipStream_t st, const double * ss_in = nullptr, int n_ss_in = 0, pm_window::Advance * adv = nullptr,
+             bool alone = false) {
     if (!m->output.d || !m->out_norm.d) return seterr(m, PM355_E_UNSUPPORTED, "head: output / output_norm missing");
     const Tensor * ow[1] = {&m->output};
     float * lg = d_logits ? d_logits : m->logits;
@@ -406,8 +408,9 @@ int run_head(pm_window * m, const float * x_row, float * d_logits, int32_t * d_a
         if (gemv(m->output, nullptr, a, 1, lg, nullptr, nullptr, st)) return seterr(m, PM355_E_UNSUPPORTED, "head: lm_head gemv");
     }
     if (d_argmax) {
-        pm_launch_argmax(lg, m->hp.n_vocab, d_argmax, nullptr, st, 1, m->am_part, m->adv || m->rot ? m->d_pos : nullptr, m->d_ctl, m->adv, m->rot);
-        m->adv = m->rot = 0;
+        const bool move = adv && (adv->by || adv->rotate);
+        pm_launch_argmax(lg, m->hp.n_vocab, d_argmax, nullptr, st, 1, alone ? nullptr : m->am_part, move ? m->d_pos : nullptr, m->d_ctl, move ? adv->by : 0, move ? adv->rotate : 0);
+        if (move) *adv = {0, 0};
     }
     return 0;
 }
@@ -629,7 +632,7 @@ bool small_path(const pm_window * m, const Layer & L, int T) {
 
 // x_in -> x_out for layers [lo, hi); positions from device memory d_pos (pos of token 0)
 int run_window(pm_window * m, const int32_t * d_tokens, const float * d_x_in, int T, float * d_x_out,
-               float * d_logits, int32_t * d_argmax, hipStream_t st) {
+               float * d_logits, int32_t * d_argmax, hipStream_t st, pm_window::Advance * adv = nullptr) {
     (void) hipGetLastError();
     const pm355_hparams & hp = m->hp;
     const int E = hp.n_embd, H = hp.n_head, Hkv = hp.n_head_kv, dh = hp.head_dim, F = hp.n_ff;
@@ -909,7 +912,7 @@ int run_window(pm_window * m, const int32_t * d_tokens, const float * d_x_in, in
     }
     if (d_x_out && cur != d_x_out) (void) hipMemcpyAsync(d_x_out, cur, (size_t) T * E * 4, hipMemcpyDeviceToDevice, st);
     if ((d_logits || d_argmax) && (m->flags & PM355_HAS_HEAD)) {
-        int rc = run_head(m, cur + (size_t) (T - 1) * E, d_logits, d_argmax, st, n_ss_head ? ss_head : nullptr, n_ss_head);
+        int rc = run_head(m, cur + (size_t) (T - 1) * E, d_logits, d_argmax, st, n_ss_head ? ss_head : nullptr, n_ss_head, adv, m->hi == m->lo);
         if (rc) return rc;
     }
     return hip_ok() ? 0 : seterr(m, PM355_E_HIP, "decode: kernel launch failed");
@@ -1148,7 +1151,7 @@ int pm_window::head(const float * d_x_row, float * d_logits, int32_t * d_argmax,
     pm_window * m = this;
     if (!m->finalized || !(m->flags & PM355_HAS_HEAD)) return seterr(m, PM355_E_UNSUPPORTED, "head: window has no head");
     (void) hipGetLastError();
-    int rc = run_head(m, d_x_row, d_logits, d_argmax, (hipStream_t) st);
+    int rc = run_head(m, d_x_row, d_logits, d_argmax, (hipStream_t) st, nullptr, 0, nullptr, true);
     if (rc) return rc;
     return hip_ok() ? 0 : seterr(m, PM355_E_HIP, "head: kernel launch failed");
 }
@@ -1178,11 +1181,9 @@ static int step_body(pm_window * m, const int32_t * d_token, const float * d_x_i
         if (rc) return rc;
         rc = run_window(m, d_token, nullptr, 1, d_x_out, nullptr, nullptr, st);
     } else {
-        m->adv = advance; m->rot = rotate;
-        rc = run_window(m, d_token, d_token ? nullptr : d_x_in, 1, d_x_out, d_logits, d_argmax, st);
-        const bool done = (advance || rotate) && !m->adv && !m->rot;          // (the argmax launch moved them)
-        m->adv = m->rot = 0;
-        if (rc || done) return rc;
+        pm_window::Advance adv = {advance, rotate};
+        rc = run_window(m, d_token, d_token ? nullptr : d_x_in, 1, d_x_out, d_logits, d_argmax, st, &adv);
+        advance = adv.by; rotate = adv.rotate;                                // (0 where the argmax launch moved them)
     }
     if (rc) return rc;
     if (advance || rotate) pm_launch_advance(m->d_pos, m->d_ctl, advance, rotate, st);

@@ -303,7 +303,8 @@ __global__ __launch_bounds__(256) void attn_rope_fused_kernel(AttnP a) {
 
 // ------------------------------------------------------------------------------------------------
 // argmax over n floats, first maximum wins. Workgroups of 1024 threads: one, or (part != null) gridDim.x per row whose results meet in the last one to arrive. One workgroup over
-// the 128256 logits of the Llama-3 vocabulary is bound by its own loads in flight: 15.3 us; thirty-two take 5.8. The last one also moves the step's position counters
+// the 128256 logits of the Llama-3 vocabulary is bound by its own loads in flight: 15.3 us; thirty-two take 5.8. part (tickets and partials) serves one launch at a time, so callers that
+// may be on several streams at once pass null and stay with one workgroup. The last one also moves the step's position counters
 // (pos != null): a launch of one thread less per token.
 // ------------------------------------------------------------------------------------------------
 __global__ __launch_bounds__(1024) void argmax_kernel(const float * x, int n, int32_t * out_idx, float * out_val, uint64_t * part, int32_t * pos, int32_t * ctl, int by, int rotate) {

@@ -561,3 +561,39 @@ def test_greedy_token_is_the_first_of_equal_maxima_over_many_workgroups(E, n_voc
         torch.cuda.synchronize()
         assert torch.equal(lg, outs[1]) == (pos == 1)
     w.close()
+
+
+def test_heads_on_two_streams(E):
+    """the head on the caller's own logits and index shares nothing between calls: two streams at once, a vocabulary of many workgroups"""
+    torch = E.torch
+    rng = np.random.default_rng(14)
+    n_vocab = 131072
+    d = tiny_model(rng, n_layer=1, n_vocab=320, n_ctx=32)
+    w = E.Window(dict(_hp(d), n_vocab=n_vocab), lo=0, hi=0, flags=E.HAS_HEAD, n_ctx=32)
+    w._chk(w.lib.pm355_model_set_tensor(w.h, E.T_OUT_NORM, -1, d.out_norm.type, d.out_norm.data, 256 * 4), "out_norm")
+    w.fill_tensor(E.T_OUTPUT, -1, Q4_K, 5, 1.0)
+    w.finalize(max_tokens=1)
+    x = torch.randn((2, 256), generator=torch.Generator(device="cuda").manual_seed(2), device="cuda")
+    want = []
+    for r in range(2):
+        lg = torch.empty(n_vocab, device="cuda")
+        w.head(x[r:r + 1], logits=lg)
+        want.append(int((lg == lg.max()).nonzero()[0]))
+    assert want[0] != want[1]
+    n, streams, graphs = 100, [torch.cuda.Stream() for _ in range(2)], []
+    lg, am = torch.empty((2, n_vocab), device="cuda"), torch.full((2, n), -1, dtype=torch.int32, device="cuda")
+    torch.cuda.synchronize()
+    for r, st in enumerate(streams):                       # (captured: back to back on the device)
+        graphs.append(torch.cuda.CUDAGraph())
+        with torch.cuda.graph(graphs[r], stream=st):
+            for i in range(n):
+                w.head(x[r:r + 1], logits=lg[r], argmax=am[r, i:])
+    for _ in range(5):
+        am.fill_(-1)
+        torch.cuda.synchronize()
+        for g, st in zip(graphs, streams):
+            with torch.cuda.stream(st):
+                g.replay()
+        torch.cuda.synchronize()
+        assert [int(am[r].ne(want[r]).sum()) for r in range(2)] == [0, 0]
+    w.close()
