@@ -1369,21 +1369,18 @@ int pm_window::batch_rows(const pm355_batch_entry * e, int n, float * d_logits, 
         const int at_ent = put(p.ent.data(), p.ent.size()), at_want = (int) blk.size();
         for (const Want & w : p.want) blk.push_back(w.row);
         const int at_keep = put(p.keep.data(), p.keep.size());
-        const pm_batch_layout lay = {T, at_seq, at_ent, (int) p.ent.size() / 2, (int) blk.size()};
-        if (pm_launch_batch_rows(d_rows, blk.data(), lay, d_last, d_pos, d_ctl, st)) return seterr(m, PM355_E_HIP, "batch: table upload");
+        const pm_batch_layout lay = {T, at_seq, at_ent, (int) p.ent.size() / 2, at_keep, (int) p.keep.size() / 2, (int) blk.size()};
+        if (pm_launch_batch_rows(d_rows, blk.data(), lay, d_last, st)) return seterr(m, PM355_E_HIP, "batch: table upload");
         const Ragged r = {d_rows + at_pos, d_rows + at_seq, d_rows + at_tiles, (int) tl.size(), tile_q, p.max_cells, p.singles};
         int rc;
         if (T == 1) {                                                                                      // (one row is a step of its own, and that sequence's)
             rc = decode(p.seq[0], d_rows, nullptr, 1, p.pos[0], W ? rows : nullptr, nullptr, nullptr, st);
-            if (!rc) rc = set_seq_pos(p.seq[0], p.pos[0] + 1, st);
         } else {
             rag = &r;
             rc = run_window(m, d_rows, nullptr, T, W ? rows : nullptr, nullptr, nullptr, st);
             rag = nullptr;
         }
         if (rc) return rc;
-        for (size_t k = 0; k < p.ent.size(); k += 2) h_pos[p.ent[k]] = p.ent[k + 1];
-        h_seq = p.ent[p.ent.size() - 2];
         for (int w = 0; w < W;) {                                           // rows whose outputs are neighbours go through the head together
             int w1 = w + 1;
             while (w1 < W && w1 - w < std::min(max_tokens, HEAD_ROWS) && p.want[w1].out == p.want[w1 - 1].out + 1) ++w1;
@@ -1402,7 +1399,9 @@ int pm_window::batch_rows(const pm355_batch_entry * e, int n, float * d_logits, 
             if (rc) return rc;
             w = w1;
         }
-        if (!p.keep.empty()) pm_launch_keep_last(d_argmax, d_rows + at_keep, (int) p.keep.size() / 2, d_last, st);
+        pm_launch_batch_end(d_rows, lay, d_argmax, d_last, d_pos, d_ctl, st);
+        for (size_t k = 0; k < p.ent.size(); k += 2) h_pos[p.ent[k]] = p.ent[k + 1];
+        h_seq = p.ent[p.ent.size() - 2];
     }
     return hip_ok() ? 0 : seterr(m, PM355_E_HIP, "batch: kernel launch failed");
 }

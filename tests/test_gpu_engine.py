@@ -597,3 +597,32 @@ def test_heads_on_two_streams(E):
         torch.cuda.synchronize()
         assert [int(am[r].ne(want[r]).sum()) for r in range(2)] == [0, 0]
     w.close()
+
+
+def test_a_refused_batch_leaves_the_positions(E):
+    """the head is refused (the window has none yet): the sequences stay where they were, on the host and on the device"""
+    torch = E.torch
+    rng = np.random.default_rng(13)
+    d = tiny_model(rng, n_layer=1, n_embd=256, n_head=4, n_head_kv=2, n_ff=512, n_vocab=320, n_ctx=64)
+    toks = rng.integers(0, 320, (2, 6)).astype(np.int32)
+    outs = []
+    for head in (True, False):
+        w = E.Window(_hp(d), n_ctx=64)
+        w.flags = E.HAS_EMBD | (E.HAS_HEAD if head else 0)  # (the wrapper's: what it loads)
+        w.load_desc(d)
+        w.finalize_pool(16, 2, 128)
+        s = [w.seq_new() for _ in range(2)]
+        if not head:
+            with pytest.raises(E.L.PM355Error, match="head"):
+                _batch(E, w, [(q, t, (5,)) for q, t in zip(s, toks)])
+            assert [w.seq_len(q) for q in s] == [0, 0]
+            w._chk(w.lib.pm355_model_set_tensor(w.h, E.T_OUT_NORM, -1, d.out_norm.type, d.out_norm.data, 256 * 4), "out_norm")
+            w._chk(w.lib.pm355_model_set_tensor(w.h, E.T_OUTPUT, -1, d.output.type, d.output.data, E.L.row_size(d.output.type, 256) * 320), "output")
+            torch.cuda.synchronize()
+        lg = torch.empty(320, device="cuda")
+        for q in s:
+            w.set_seq(q)
+            w.step(token=torch.from_numpy(toks[q][:1]).cuda(), logits=lg, use_graph=False)
+            outs.append(lg.clone())
+        w.close()
+    assert torch.equal(outs[0], outs[2]) and torch.equal(outs[1], outs[3])
