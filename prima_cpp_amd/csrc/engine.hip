@@ -1338,7 +1338,10 @@ int pm_window::batch_rows(const pm355_batch_entry * e, int n, float * d_logits, 
                     Pass & p = passes.back();
                     const int row = (int) p.tok.size(), T = std::min(p.cap - row, p1 - off), pos0 = h_pos[e[i].seq] + off;
                     for (int t = 0; t < T; ++t) { p.tok.push_back(e[i].tokens ? e[i].tokens[off + t] : -1); p.pos.push_back(pos0 + t); p.seq.push_back(e[i].seq); }
-                    p.ent.push_back(e[i].seq); p.ent.push_back(pos0 + T);
+                    size_t at_ent = 0;                                                                      // (pieces of one sequence may meet in a pass: one position per sequence)
+                    while (at_ent < p.ent.size() && p.ent[at_ent] != e[i].seq) at_ent += 2;
+                    if (at_ent == p.ent.size()) { p.ent.push_back(e[i].seq); p.ent.push_back(0); }
+                    p.ent[at_ent + 1] = pos0 + T;
                     p.max_cells = std::max(p.max_cells, pos0 + T); p.singles = p.singles && T == 1;
                     for (int j = 0; j < e[i].n_want; ++j) if (e[i].want[j] >= off && e[i].want[j] < off + T) p.want.push_back({row + e[i].want[j] - off, out0 + j});
                     if (d_argmax && e[i].n_want && off + T == e[i].n_tokens) { p.keep.push_back(e[i].seq); p.keep.push_back(out0 + e[i].n_want - 1); }

@@ -626,3 +626,27 @@ def test_a_refused_batch_leaves_the_positions(E):
             outs.append(lg.clone())
         w.close()
     assert torch.equal(outs[0], outs[2]) and torch.equal(outs[1], outs[3])
+
+
+@pytest.mark.parametrize("n_vocab", [320, 4099])
+def test_positions_behind_a_portion_cut_into_passes(E, n_vocab):
+    """20 tokens with scratch for 8: pieces of one sequence that meet in a pass; a step behind them continues where the sequence ends (the device's counter), and so does the next portion"""
+    torch = E.torch
+    rng = np.random.default_rng(15)
+    d = tiny_model(rng, n_layer=2, n_embd=512, n_head=8, n_head_kv=2, n_ff=1024, n_vocab=n_vocab, n_ctx=64, rope_freqs=True)
+    toks = rng.integers(0, n_vocab, (3, 21)).astype(np.int32)
+    outs = []
+    for together in (True, False):
+        w = _pool_window(E, d, 64, 8, 3)
+        s = [w.seq_new() for _ in range(3)]
+        entries = [(q, t[:n], ()) for q, t, n in zip(s, toks, (20, 20, 13))]
+        for e in [entries] if together else [[x] for x in entries]:
+            w.batch(e)
+        lg = torch.empty((3, n_vocab), device="cuda")
+        for i, q in enumerate(s):
+            w.set_seq(q)
+            w.step(token=torch.from_numpy(toks[i][-1:]).cuda(), logits=lg[i], use_graph=False)
+        outs.append(lg.double().cpu().numpy())
+        w.close()
+    for a, b in zip(*outs):
+        assert ((a - b) ** 2).sum() < 1e-3 * (b ** 2).sum()
