@@ -563,6 +563,21 @@ def test_greedy_token_is_the_first_of_equal_maxima_over_many_workgroups(E, n_voc
     w.close()
 
 
+def _pool_window(E, d, n_ctx, max_tokens, n_seq, n_vocab=None):
+    w = E.Window(dict(_hp(d), n_vocab=n_vocab or d.n_vocab), n_ctx=n_ctx)
+    w.load_desc(d)
+    w.finalize_pool(max_tokens, n_seq, n_seq * n_ctx)
+    return w
+
+
+def _batch(E, w, entries, argmax=False):
+    """logits of the wanted rows (and greedy tokens) of one batch"""
+    rows = sum(len(e[2]) for e in entries)
+    lg, am = E.torch.full((rows, w.n_vocab), float("nan"), device="cuda"), E.torch.full((rows,), -1, dtype=E.torch.int32, device="cuda")
+    w.batch(entries, logits=lg, argmax=am if argmax else None)
+    return (lg, am) if argmax else lg
+
+
 def test_heads_on_two_streams(E):
     """the head on the caller's own logits and index shares nothing between calls: two streams at once, a vocabulary of many workgroups"""
     torch = E.torch
