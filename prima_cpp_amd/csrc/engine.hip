@@ -1372,7 +1372,7 @@ int pm_window::batch_rows(const pm355_batch_entry * e, int n, float * d_logits, 
         const int at_ent = put(p.ent.data(), p.ent.size()), at_want = (int) blk.size();
         for (const Want & w : p.want) blk.push_back(w.row);
         const int at_keep = put(p.keep.data(), p.keep.size());
-        const pm_batch_layout lay = {T, at_seq, at_ent, (int) p.ent.size() / 2, at_keep, (int) p.keep.size() / 2, (int) blk.size()};
+        const pm_batch_layout lay = {T, at_seq, at_ent, (int) p.ent.size() / 2, at_keep, (int) p.keep.size() / 2, (int) blk.size(), e[n - 1].seq};
         if (pm_launch_batch_rows(d_rows, blk.data(), lay, d_last, st)) return seterr(m, PM355_E_HIP, "batch: table upload");
         const Ragged r = {d_rows + at_pos, d_rows + at_seq, d_rows + at_tiles, (int) tl.size(), tile_q, p.max_cells, p.singles};
         int rc;
@@ -1404,7 +1404,7 @@ int pm_window::batch_rows(const pm355_batch_entry * e, int n, float * d_logits, 
         }
         pm_launch_batch_end(d_rows, lay, d_argmax, d_last, d_pos, d_ctl, st);
         for (size_t k = 0; k < p.ent.size(); k += 2) h_pos[p.ent[k]] = p.ent[k + 1];
-        h_seq = p.ent[p.ent.size() - 2];
+        h_seq = e[n - 1].seq;
     }
     return hip_ok() ? 0 : seterr(m, PM355_E_HIP, "batch: kernel launch failed");
 }

@@ -410,11 +410,11 @@ __global__ __launch_bounds__(256) void gather_rows_kernel(const float * x, const
     const int i = (int) (blockIdx.x * 256 + threadIdx.x);
     if (4 * i < K) *(float4 *) (y + (size_t) blockIdx.y * K + 4 * i) = *(const float4 *) (x + (size_t) at[blockIdx.y] * K + 4 * i);
 }
-// The end of a pass, behind everything that could still be refused: positions of its sequences, the last one of them current, and greedy tokens where the next step's embedding finds them
+// The end of a pass, behind everything that could still be refused: positions of its sequences, the batch's last sequence current, and greedy tokens where the next step's embedding finds them
 __global__ __launch_bounds__(256) void batch_end_kernel(const int32_t * blk, pm_batch_layout l, const int32_t * argmax, int32_t * last, int32_t * pos, int32_t * ctl) {
     for (int i = threadIdx.x; i < l.n_entries; i += 256) pos[blk[l.entries + 2 * i]] = blk[l.entries + 2 * i + 1];
     for (int i = threadIdx.x; i < l.n_keep; i += 256) last[blk[l.keep + 2 * i]] = argmax[blk[l.keep + 2 * i + 1]];
-    if (threadIdx.x == 0) ctl[0] = blk[l.entries + 2 * (l.n_entries - 1)];
+    if (threadIdx.x == 0) ctl[0] = l.current;
 }
 __global__ void set_i32_pair_kernel(int32_t * p, int a, int32_t * q, int b) { *p = a; *q = b; }
 __global__ void set_i32x2_kernel(int32_t * p, int a, int b) { p[0] = a; p[1] = b; }

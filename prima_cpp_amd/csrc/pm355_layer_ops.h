@@ -82,8 +82,8 @@ constexpr size_t PM_ARGMAX_SCRATCH = (size_t) PM_ARGMAX_ROWS * (4 + PM_ARGMAX_PA
 void pm_launch_argmax(const float * x, int n, int32_t * idx, float * val, hipStream_t st, int rows = 1, uint64_t * part = nullptr, int32_t * pos = nullptr, int32_t * ctl = nullptr,
                       int by = 0, int rotate = 0);
 // a pass over T rows of several sequences: block of int32 = tokens [T] | positions [T] | sequences [T] | ... ; offsets in integers. entries: {sequence, position behind the pass};
-// keep: {sequence, row of argmax}. batch_rows in front of the pass, batch_end behind it: pos[sequence] = position, last[sequence] = argmax[row], ctl[0] = the last entry's sequence
-struct pm_batch_layout { int T, seq, entries, n_entries, keep, n_keep, n_ints; };
+// keep: {sequence, row of argmax}. batch_rows in front of the pass, batch_end behind it: pos[sequence] = position, last[sequence] = argmax[row], ctl[0] = current
+struct pm_batch_layout { int T, seq, entries, n_entries, keep, n_keep, n_ints, current; };
 int  pm_launch_batch_rows(int32_t * blk, const int32_t * host, const pm_batch_layout & l, const int32_t * last, hipStream_t st);
 void pm_launch_batch_end(const int32_t * blk, const pm_batch_layout & l, const int32_t * argmax, int32_t * last, int32_t * pos, int32_t * ctl, hipStream_t st);
 void pm_launch_gather_rows(const float * x, const int32_t * at, int n, int K, float * y, hipStream_t st);                  // y[i] = x[at[i]], K % 4 == 0

@@ -665,3 +665,22 @@ def test_positions_behind_a_portion_cut_into_passes(E, n_vocab):
         w.close()
     for a, b in zip(*outs):
         assert ((a - b) ** 2).sum() < 1e-3 * (b ** 2).sum()
+
+
+@pytest.mark.parametrize("lens", [(3, 40), (40, 3), (3, 4), (1, 1)])
+def test_the_last_portion_of_a_batch_is_the_current_sequence(E, lens):
+    """whichever pass it ran in"""
+    torch = E.torch
+    rng = np.random.default_rng(16)
+    d = tiny_model(rng, n_layer=1, n_embd=256, n_head=4, n_head_kv=2, n_ff=512, n_vocab=320, n_ctx=64)
+    w = _pool_window(E, d, 64, 64, 3)
+    s = [w.seq_new() for _ in lens]
+    w.batch([(q, rng.integers(0, 320, n), ()) for q, n in zip(s, lens)])
+    a, b = torch.empty(320, device="cuda"), torch.empty(320, device="cuda")
+    w.step(token=torch.tensor([7], dtype=torch.int32, device="cuda"), logits=a, use_graph=False)
+    assert [w.seq_len(q) for q in s] == [lens[0], lens[1] + 1]
+    w.set_seq_pos(s[1], lens[1])
+    w.set_seq(s[1])
+    w.step(token=torch.tensor([7], dtype=torch.int32, device="cuda"), logits=b, use_graph=False)
+    assert torch.equal(a, b)
+    w.close()
