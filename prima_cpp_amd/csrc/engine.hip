@@ -1308,26 +1308,28 @@ int pm_window::pool_info(pm355_pool_info * o) {
     return 0;
 }
 // All entries as rows of common passes: the weights are read once per pass instead of once per sequence (eight sequences of the 8B shape, eight layers and
-// head: prompts of 12..24 tokens and twelve steps 47.0 ms one sequence after another, 14.0 ms as common passes). A portion keeps the arithmetic that it has alone - up to 32 tokens 8-bit activations, beyond 16-bit ones -
-// whatever shares the step with it: the longer portions (a sequence's first ones) go first, then the short ones. served = false and nothing done where a pass does not take rows of
-// several sequences.
+// head: prompts of 12..24 tokens and twelve steps 47.0 ms one sequence after another, 14.0 ms as common passes). A portion keeps the arithmetic that it has alone - up to 32 tokens 8-bit
+// activations, beyond 16-bit ones; up to 15 where a layer has no 8-bit path, and between the two either, layer by layer - whatever shares the step with it: portions meet in passes of
+// their own tier, the longer ones (a sequence's first) first. served = false and nothing done where a pass does not take rows of several sequences.
 int pm_window::batch_rows(const pm355_batch_entry * e, int n, float * d_logits, int32_t * d_argmax, hipStream_t st, bool * served) {
     pm_window * m = this;
     *served = false;
     const int dh = hp.head_dim, V = hp.n_vocab;
     if (no_fuse || hi <= lo || (dh != 64 && dh != 128) || hp.n_ctx % 32 || max_tokens < 2) return 0;      // (what the matrix-core attention takes)
-    int small = MMQ_MAX_TOKENS;
-    for (auto & L : layers) if (!small_path(this, L, MMQ_MAX_TOKENS)) small = SMALL_PLAIN_MAX;
-    small = std::min(small, max_tokens);
+    bool every = true, any = false;
+    for (auto & L : layers) { const bool s8 = small_path(this, L, MMQ_MAX_TOKENS); every = every && s8; any = any || s8; }
+    std::vector<int> tier;                                                                                 // the longest portion of each tier
+    for (int t : {every ? 0 : SMALL_PLAIN_MAX, any ? MMQ_MAX_TOKENS : 0, max_tokens}) if (t > (tier.empty() ? 0 : tier.back()) && (tier.empty() || tier.back() < max_tokens)) tier.push_back(std::min(t, max_tokens));
     struct Want { int row, out; };                                                                          // row of the pass, row of the outputs
     struct Pass { std::vector<int32_t> tok, pos, seq, ent, keep; std::vector<Want> want; int cap = 0, max_cells = 0; bool singles = true; };
     std::vector<Pass> passes;
-    for (int longer = 1; longer >= 0; --longer) {
-        auto mine = [&](int T) { return (T > small) == (longer != 0); };
+    for (int tr = (int) tier.size() - 1; tr >= 0; --tr) {
+        const int above = tr ? tier[tr - 1] : 0, most = tier[tr];
+        auto mine = [&](int T) { return T > above && T <= most; };
         int64_t total = 0, done = 0;
         for (int i = 0; i < n; ++i)
             for (int off = 0; off < e[i].n_tokens; off += max_tokens) { const int T = std::min(max_tokens, e[i].n_tokens - off); if (mine(T)) total += T; }
-        const int64_t k = (total + (longer ? max_tokens : small) - 1) / (longer ? max_tokens : small);     // passes of equal size: a longer portion's piece stays above `small` rows
+        const int64_t k = (total + most - 1) / most;                                                       // passes of equal size: more than `above` rows, like every portion of the tier
         int64_t at = 0;
         for (int i = 0, out0 = 0; i < n; out0 += e[i].n_want, ++i)
             for (int p0 = 0; p0 < e[i].n_tokens; p0 += max_tokens) {

@@ -684,3 +684,20 @@ def test_the_last_portion_of_a_batch_is_the_current_sequence(E, lens):
     w.step(token=torch.tensor([7], dtype=torch.int32, device="cuda"), logits=b, use_graph=False)
     assert torch.equal(a, b)
     w.close()
+
+
+def test_portions_keep_their_tier_where_only_some_layers_have_an_8_bit_path(E):
+    """ffn_down of 65536 columns, Q6_K in the first layer and Q4_K in the second: Q4_K has the integer small-batch product, Q6_K has none. Portions of 16..32 tokens then run one layer on 16-bit and one on 8-bit activations; two of them in
+    one step do as well, in passes of their size: the same bits as alone."""
+    rng = np.random.default_rng(12)
+    d = tiny_model(rng, n_layer=2, n_embd=512, n_head=8, n_head_kv=2, n_ff=65536, n_vocab=320, n_ctx=256, types=dict(attn_v=Q4_K))
+    toks = rng.integers(0, 320, (2, 220)).astype(np.int32)
+    w = _pool_window(E, d, 256, 64, 4)
+    s = [w.seq_new() for _ in range(4)]
+    for i, q in enumerate(s):
+        w.batch([(q, toks[i % 2, 20:], ())])
+    toks = toks[:, :20]
+    alone = [_batch(E, w, [(s[i], toks[i], (19,))]) for i in range(2)]
+    both = _batch(E, w, [(s[2 + i], toks[i], (19,)) for i in range(2)])
+    assert E.torch.equal(both, E.torch.cat(alone))
+    w.close()
