@@ -106,8 +106,9 @@ struct pm_window : pm355_model {
     std::vector<StepGraph> graphs;
     // batches: open sequences (a sequence holds one KV slab), their last greedy token on the device, and the hidden rows of a portion whose logits are asked for
     std::vector<char> seq_open; int32_t * d_last = nullptr; float * rows = nullptr;
-    // a pass over rows of several sequences (batch): every row's position and sequence in device memory, tiles for the matrix-core attention; rag is set while one is launched
-    struct Ragged { const int32_t * pos, * seq, * tiles; int n_tiles, tile_q, max_cells; bool singles; };
+    // a pass over rows of several sequences (batch): every row's position and sequence in device memory; rag is set while one is launched. Attention: rows [0, n_rows) see at most max_cells
+    // cells and have a workgroup per head and row, the rows behind them are the first n_tiles tiles of the matrix-core kernel (all_tiles: those of all rows)
+    struct Ragged { const int32_t * pos, * seq, * tiles; int n_tiles, all_tiles, tile_q, n_rows, max_cells; };
     const Ragged * rag = nullptr; int32_t * d_rows = nullptr; float * head_lg = nullptr;
     uint64_t * am_part = nullptr;                 // argmax scratch of up to HEAD_ROWS rows: one user at a time, like the window's activations
     struct Advance { int by, rotate; };           // what the launch that ends a step still does to the position counters (step_body; the argmax does it on its way and clears this)
@@ -319,6 +320,7 @@ const int MMQ_MAX_TOKENS = [] { const char * e = getenv("PM355_MMQ_MAX_TOKENS");
 // 69.8 / 86.4 / 92.0, behind 300 76.3 / 91.7 / 99.3 against 72.4 / 89.1 / 94.5
 const int SMALL_ATTN_MFMA_MIN = [] { const char * e = getenv("PM355_SMALL_ATTN_MFMA_MIN"); return e ? atoi(e) : 16; }();
 const int SMALL_ATTN_MFMA_CELLS = 192;
+bool small_attn_mfma(int T, int past) { return T >= SMALL_ATTN_MFMA_MIN || past + T >= SMALL_ATTN_MFMA_CELLS; }
 constexpr int HEAD_ROWS = 32;            // rows of a batch that go through the head at once (what one pass of the integer mat-mul takes)
 const int MMQ_MULTI_MIN_TOKENS = 2;       // the fused wq | wk | wv and ffn_gate | ffn_up launches already win at 2 tokens (3 / 4 mat-vec launches otherwise)
 // the table output of the Q8_K quantizers, when this batch size takes the small-batch mat-mul (mmq_i8.hip)
@@ -657,14 +659,14 @@ int run_window(pm_window * m, const int32_t * d_tokens, const float * d_x_in, in
     auto rope_store = [&](const Layer & L, int round_q) {
         pm_launch_rope_kv_store(m->q, m->k, m->v, m->q, nullptr, L.kc, L.vc, d_pos, d_seq, kv_stride, (const float *) m->rope_freqs.d, T, H, Hkv, dh, hp.n_ctx, m->rope, st, round_q, rg ? 1 : 0);
     };
-    auto attend_mfma = [&](const Layer & L, float * out, void * out_f16) {
+    auto attend_mfma = [&](const Layer & L, float * out, void * out_f16, bool all = true) {
         return pm_launch_attn_prefill(m->q, L.kc, L.vc, d_pos, d_seq, kv_stride, out, T, H, Hkv, dh, hp.n_ctx, kq_scale, st, nullptr, 0, 0, 0, 0, out_f16,
-                                      rg ? rg->tiles : nullptr, rg ? rg->n_tiles : 0, rg ? rg->tile_q : 0);
+                                      rg ? rg->tiles : nullptr, rg ? (all ? rg->all_tiles : rg->n_tiles) : 0, rg ? rg->tile_q : 0);
     };
     // one workgroup per (head, token); a shape attn_cached refuses - head_dim other than 64 / 128 / 256, scores beyond 150 KiB of LDS - falls back to attn_decode, which rounds q to
     // F16 itself: the pre-rounded rows give it the same bits as raw ones, tests/test_gpu_ops.py::test_small_batch_attention_fallback_...
     auto attend_rows = [&](const Layer & L) {
-        const int rc = pm_launch_attn_cached(m->q, L.kc, L.vc, d_pos, d_seq, kv_stride, m->att, H, Hkv, dh, hp.n_ctx, kq_scale, st, nullptr, nullptr, rg ? rg->max_cells : 0, 0, 0, T, rg ? 1 : 0);
+        const int rc = pm_launch_attn_cached(m->q, L.kc, L.vc, d_pos, d_seq, kv_stride, m->att, H, Hkv, dh, hp.n_ctx, kq_scale, st, nullptr, nullptr, rg ? rg->max_cells : 0, 0, 0, rg ? rg->n_rows : T, rg ? 1 : 0);
         return rc && !rg ? pm_launch_attn_decode(m->q, L.kc, L.vc, d_pos, d_seq, kv_stride, m->att, T, H, Hkv, dh, hp.n_ctx, kq_scale, st) : rc;
     };
     // the tokens' rows, and with them the cos / sin tables that the wq | wk | wv epilogues of all layers read
@@ -850,8 +852,8 @@ int run_window(pm_window * m, const int32_t * d_tokens, const float * d_x_in, in
         // q rotated AND rounded to F16, every token's K row / V column stored: the attention of a small batch then is the single-token kernel over
         // cached cells, one workgroup per (head, token) (attn_cached.hip: one barrier up to 64 cells; 11 -> ~4 us per layer at 2..8 tokens)
         if (!rope_done) rope_store(L, 1);
-        const bool mfma = rg ? rg->max_cells >= SMALL_ATTN_MFMA_CELLS : T >= SMALL_ATTN_MFMA_MIN || m->h_pos[m->h_seq] + T >= SMALL_ATTN_MFMA_CELLS;
-        if (!(mfma && attend_mfma(L, m->att, nullptr) == 0) && attend_rows(L))
+        const bool mfma = !rg && small_attn_mfma(T, m->h_pos[m->h_seq]);
+        if (rg ? (rg->n_rows && attend_rows(L)) || (rg->n_tiles && attend_mfma(L, m->att, nullptr, false)) : !(mfma && attend_mfma(L, m->att, nullptr) == 0) && attend_rows(L))
             return seterr(m, PM355_E_RANGE, "decode: n_ctx too large for the decode-attention kernel");
         }
         const Tensor * wo[1] = {&L.t[PM355_T_WO]};
@@ -1309,8 +1311,9 @@ int pm_window::pool_info(pm355_pool_info * o) {
 }
 // All entries as rows of common passes: the weights are read once per pass instead of once per sequence (eight sequences of the 8B shape, eight layers and
 // head: prompts of 12..24 tokens and twelve steps 47.0 ms one sequence after another, 14.0 ms as common passes). A portion keeps the arithmetic that it has alone - up to 32 tokens 8-bit
-// activations, beyond 16-bit ones; up to 15 where a layer has no 8-bit path, and between the two either, layer by layer - whatever shares the step with it: portions meet in passes of
-// their own tier, the longer ones (a sequence's first) first. served = false and nothing done where a pass does not take rows of several sequences.
+// activations, beyond 16-bit ones; up to 15 where a layer has no 8-bit path, and between the two either, layer by layer; probabilities rounded before or behind their division - whatever
+// shares the step with it: portions meet in passes of their own tier, the longer ones (a sequence's first) first, and a row's attention is chosen by its own portion and history. served =
+// false and nothing done where a pass does not take rows of several sequences.
 int pm_window::batch_rows(const pm355_batch_entry * e, int n, float * d_logits, int32_t * d_argmax, hipStream_t st, bool * served) {
     pm_window * m = this;
     *served = false;
@@ -1320,66 +1323,85 @@ int pm_window::batch_rows(const pm355_batch_entry * e, int n, float * d_logits, 
     for (auto & L : layers) { const bool s8 = small_path(this, L, MMQ_MAX_TOKENS); every = every && s8; any = any || s8; }
     std::vector<int> tier;                                                                                 // the longest portion of each tier
     for (int t : {every ? 0 : SMALL_PLAIN_MAX, any ? MMQ_MAX_TOKENS : 0, max_tokens}) if (t > (tier.empty() ? 0 : tier.back()) && (tier.empty() || tier.back() < max_tokens)) tier.push_back(std::min(t, max_tokens));
-    struct Want { int row, out; };                                                                          // row of the pass, row of the outputs
-    struct Pass { std::vector<int32_t> tok, pos, seq, ent, keep; std::vector<Want> want; int cap = 0, max_cells = 0; bool singles = true; };
+    struct Piece { int entry, off, T, pos0, out0; bool tiles; };                                           // tokens [off, off + T) of an entry, whose first wanted row is out0
+    struct Pass { std::vector<Piece> piece; int cap = 0, T = 0; };
+    // attention of a portion of T tokens as it has it alone: one pass over the keys on the matrix cores, or a workgroup per head and token (whose scores are in LDS: 4 bytes a cell)
+    auto in_tiles = [&](int T, int past) { return (T == 1 ? split_scratch && past >= split_min : small_attn_mfma(T, past)) || past + T > 32768; };
     std::vector<Pass> passes;
     for (int tr = (int) tier.size() - 1; tr >= 0; --tr) {
         const int above = tr ? tier[tr - 1] : 0, most = tier[tr];
         auto mine = [&](int T) { return T > above && T <= most; };
-        int64_t total = 0, done = 0;
+        int64_t total = 0;
         for (int i = 0; i < n; ++i)
             for (int off = 0; off < e[i].n_tokens; off += max_tokens) { const int T = std::min(max_tokens, e[i].n_tokens - off); if (mine(T)) total += T; }
         const int64_t k = (total + most - 1) / most;                                                       // passes of equal size: more than `above` rows, like every portion of the tier
         int64_t at = 0;
         for (int i = 0, out0 = 0; i < n; out0 += e[i].n_want, ++i)
             for (int p0 = 0; p0 < e[i].n_tokens; p0 += max_tokens) {
-                const int p1 = std::min(p0 + max_tokens, e[i].n_tokens);
+                const int p1 = std::min(p0 + max_tokens, e[i].n_tokens), past = h_pos[e[i].seq];
                 if (!mine(p1 - p0)) continue;
                 for (int off = p0; off < p1;) {
-                    if (!at || (int) passes.back().tok.size() == passes.back().cap) { passes.emplace_back(); passes.back().cap = (int) (total * (at + 1) / k - total * at / k); ++at; }
+                    if (!at || passes.back().T == passes.back().cap) { passes.emplace_back(); passes.back().cap = (int) (total * (at + 1) / k - total * at / k); ++at; }
                     Pass & p = passes.back();
-                    const int row = (int) p.tok.size(), T = std::min(p.cap - row, p1 - off), pos0 = h_pos[e[i].seq] + off;
-                    for (int t = 0; t < T; ++t) { p.tok.push_back(e[i].tokens ? e[i].tokens[off + t] : -1); p.pos.push_back(pos0 + t); p.seq.push_back(e[i].seq); }
-                    size_t at_ent = 0;                                                                      // (pieces of one sequence may meet in a pass: one position per sequence)
-                    while (at_ent < p.ent.size() && p.ent[at_ent] != e[i].seq) at_ent += 2;
-                    if (at_ent == p.ent.size()) { p.ent.push_back(e[i].seq); p.ent.push_back(0); }
-                    p.ent[at_ent + 1] = pos0 + T;
-                    p.max_cells = std::max(p.max_cells, pos0 + T); p.singles = p.singles && T == 1;
-                    for (int j = 0; j < e[i].n_want; ++j) if (e[i].want[j] >= off && e[i].want[j] < off + T) p.want.push_back({row + e[i].want[j] - off, out0 + j});
-                    if (d_argmax && e[i].n_want && off + T == e[i].n_tokens) { p.keep.push_back(e[i].seq); p.keep.push_back(out0 + e[i].n_want - 1); }
-                    off += T; done += T;
+                    const int T = std::min(p.cap - p.T, p1 - off);
+                    p.piece.push_back({i, off, T, past + off, out0, in_tiles(p1 - p0, past + p0)});
+                    p.T += T; off += T;
                 }
             }
-        if (done != total) return 0;
     }
-    for (Pass & p : passes) if (p.want.size() > p.tok.size()) return 0;                                     // (a row asked for several times)
+    struct Want { int row, out; };                                                                          // row of the pass, row of the outputs
+    auto wanted = [&](const Piece & c, auto && f) { for (int j = 0; j < e[c.entry].n_want; ++j) if (e[c.entry].want[j] >= c.off && e[c.entry].want[j] < c.off + c.T) f(e[c.entry].want[j] - c.off, c.out0 + j); };
+    for (const Pass & p : passes) {
+        int w = 0;
+        for (const Piece & c : p.piece) wanted(c, [&](int, int) { ++w; });
+        if (w > p.T) return 0;                                                                              // (a row asked for several times)
+    }
     *served = true;
     for (Pass & p : passes) {
-        const int T = (int) p.tok.size(), W = (int) p.want.size();
-        const int tile_q = pm_attn_prefill_tile(T, hp.n_head);
+        const int T = p.T;
+        std::vector<int32_t> tok, pos, seq, ent, keep;
+        std::vector<Want> want;
+        int n_rows = 0, max_cells = 0;
+        std::stable_sort(p.piece.begin(), p.piece.end(), [](const Piece & a, const Piece & b) { return a.tiles < b.tiles; });      // (every row is stored before any attends: their order is free)
+        for (const Piece & c : p.piece) {
+            const pm355_batch_entry & x = e[c.entry];
+            const int row = (int) tok.size();
+            for (int t = 0; t < c.T; ++t) { tok.push_back(x.tokens ? x.tokens[c.off + t] : -1); pos.push_back(c.pos0 + t); seq.push_back(x.seq); }
+            if (!c.tiles) { n_rows += c.T; max_cells = std::max(max_cells, c.pos0 + c.T); }
+            size_t at_ent = 0;                                                                              // (pieces of one sequence may meet in a pass: one position per sequence)
+            while (at_ent < ent.size() && ent[at_ent] != x.seq) at_ent += 2;
+            if (at_ent == ent.size()) { ent.push_back(x.seq); ent.push_back(0); }
+            ent[at_ent + 1] = std::max(ent[at_ent + 1], c.pos0 + c.T);
+            wanted(c, [&](int t, int out) { want.push_back({row + t, out}); });
+            if (d_argmax && x.n_want && c.off + c.T == x.n_tokens) { keep.push_back(x.seq); keep.push_back(c.out0 + x.n_want - 1); }
+        }
+        const int W = (int) want.size(), tile_q = pm_attn_prefill_tile(T, hp.n_head);
         struct Tile { int32_t row, n, pos, seq; };
         std::vector<Tile> tl;
+        int n_tiles = 0;
         for (int r = 0; r < T;) {
             int r1 = r + 1;
-            while (r1 < T && r1 - r < tile_q && p.seq[r1] == p.seq[r]) ++r1;
-            tl.push_back({r, r1 - r, p.pos[r], p.seq[r]});
+            while (r1 < T && r1 != n_rows && r1 - r < tile_q && seq[r1] == seq[r] && pos[r1] == pos[r1 - 1] + 1) ++r1;
+            tl.push_back({r, r1 - r, pos[r], seq[r]});
+            if (r >= n_rows) ++n_tiles;
             r = r1;
         }
-        std::stable_sort(tl.begin(), tl.end(), [](const Tile & a, const Tile & b) { return a.pos + a.n < b.pos + b.n; });      // (the kernel takes them from the end: most keys first)
-        std::stable_sort(p.want.begin(), p.want.end(), [](const Want & a, const Want & b) { return a.out < b.out; });
+        std::rotate(tl.begin(), tl.end() - n_tiles, tl.end());
+        std::stable_sort(tl.begin(), tl.begin() + n_tiles, [](const Tile & a, const Tile & b) { return a.pos + a.n < b.pos + b.n; });      // (the kernel takes them from the end: most keys first)
+        std::stable_sort(want.begin(), want.end(), [](const Want & a, const Want & b) { return a.out < b.out; });
         std::vector<int32_t> blk;
         blk.reserve(12 * (size_t) T);
         auto put = [&](const int32_t * v, size_t k) { const int at = (int) blk.size(); blk.insert(blk.end(), v, v + k); return at; };
-        put(p.tok.data(), T); const int at_pos = put(p.pos.data(), T), at_seq = put(p.seq.data(), T), at_tiles = put((const int32_t *) tl.data(), 4 * tl.size());
-        const int at_ent = put(p.ent.data(), p.ent.size()), at_want = (int) blk.size();
-        for (const Want & w : p.want) blk.push_back(w.row);
-        const int at_keep = put(p.keep.data(), p.keep.size());
-        const pm_batch_layout lay = {T, at_seq, at_ent, (int) p.ent.size() / 2, at_keep, (int) p.keep.size() / 2, (int) blk.size(), e[n - 1].seq};
+        put(tok.data(), T); const int at_pos = put(pos.data(), T), at_seq = put(seq.data(), T), at_tiles = put((const int32_t *) tl.data(), 4 * tl.size());
+        const int at_ent = put(ent.data(), ent.size()), at_want = (int) blk.size();
+        for (const Want & w : want) blk.push_back(w.row);
+        const int at_keep = put(keep.data(), keep.size());
+        const pm_batch_layout lay = {T, at_seq, at_ent, (int) ent.size() / 2, at_keep, (int) keep.size() / 2, (int) blk.size(), e[n - 1].seq};
         if (pm_launch_batch_rows(d_rows, blk.data(), lay, d_last, st)) return seterr(m, PM355_E_HIP, "batch: table upload");
-        const Ragged r = {d_rows + at_pos, d_rows + at_seq, d_rows + at_tiles, (int) tl.size(), tile_q, p.max_cells, p.singles};
+        const Ragged r = {d_rows + at_pos, d_rows + at_seq, d_rows + at_tiles, n_tiles, (int) tl.size(), tile_q, n_rows, max_cells};
         int rc;
         if (T == 1) {                                                                                      // (one row is a step of its own, and that sequence's)
-            rc = decode(p.seq[0], d_rows, nullptr, 1, p.pos[0], W ? rows : nullptr, nullptr, nullptr, st);
+            rc = decode(seq[0], d_rows, nullptr, 1, pos[0], W ? rows : nullptr, nullptr, nullptr, st);
         } else {
             rag = &r;
             rc = run_window(m, d_rows, nullptr, T, W ? rows : nullptr, nullptr, nullptr, st);
@@ -1388,10 +1410,10 @@ int pm_window::batch_rows(const pm355_batch_entry * e, int n, float * d_logits, 
         if (rc) return rc;
         for (int w = 0; w < W;) {                                           // rows whose outputs are neighbours go through the head together
             int w1 = w + 1;
-            while (w1 < W && w1 - w < std::min(max_tokens, HEAD_ROWS) && p.want[w1].out == p.want[w1 - 1].out + 1) ++w1;
-            const int k = w1 - w, o = p.want[w].out;
+            while (w1 < W && w1 - w < std::min(max_tokens, HEAD_ROWS) && want[w1].out == want[w1 - 1].out + 1) ++w1;
+            const int k = w1 - w, o = want[w].out;
             float * lg = d_logits ? d_logits + (size_t) o * V : head_lg;
-            if (k == 1) rc = run_head(m, rows + (size_t) p.want[w].row * hp.n_embd, lg, d_argmax ? d_argmax + o : nullptr, st);
+            if (k == 1) rc = run_head(m, rows + (size_t) want[w].row * hp.n_embd, lg, d_argmax ? d_argmax + o : nullptr, st);
             else {
                 if (!output.d || !out_norm.d) return seterr(m, PM355_E_UNSUPPORTED, "head: output / output_norm missing");
                 const Tensor * ow[1] = {&output};
@@ -1405,7 +1427,7 @@ int pm_window::batch_rows(const pm355_batch_entry * e, int n, float * d_logits, 
             w = w1;
         }
         pm_launch_batch_end(d_rows, lay, d_argmax, d_last, d_pos, d_ctl, st);
-        for (size_t k = 0; k < p.ent.size(); k += 2) h_pos[p.ent[k]] = p.ent[k + 1];
+        for (size_t k = 0; k < ent.size(); k += 2) h_pos[ent[k]] = ent[k + 1];
         h_seq = e[n - 1].seq;
     }
     return hip_ok() ? 0 : seterr(m, PM355_E_HIP, "batch: kernel launch failed");
