@@ -107,8 +107,9 @@ struct pm_window : pm355_model {
     // batches: open sequences (a sequence holds one KV slab), their last greedy token on the device, and the hidden rows of a portion whose logits are asked for
     std::vector<char> seq_open; int32_t * d_last = nullptr; float * rows = nullptr;
     // a pass over rows of several sequences (batch): every row's position and sequence in device memory; rag is set while one is launched. Attention: rows [0, n_rows) see at most max_cells
-    // cells and have a workgroup per head and row, the rows behind them are the first n_tiles tiles of the matrix-core kernel (all_tiles: those of all rows)
-    struct Ragged { const int32_t * pos, * seq, * tiles; int n_tiles, all_tiles, tile_q, n_rows, max_cells; };
+    // cells and have a workgroup per head and row, the last n_long rows (sequence and position on the host too) a key-split launch each, the rows between are the first n_tiles tiles of the
+    // matrix-core kernel (all_tiles: those of all rows)
+    struct Ragged { const int32_t * pos, * seq, * tiles; int n_tiles, all_tiles, tile_q, n_rows, max_cells, n_long; const int32_t * h_pos, * h_seq; };
     const Ragged * rag = nullptr; int32_t * d_rows = nullptr; float * head_lg = nullptr;
     uint64_t * am_part = nullptr;                 // argmax scratch of up to HEAD_ROWS rows: one user at a time, like the window's activations
     struct Advance { int by, rotate; };           // what the launch that ends a step still does to the position counters (step_body; the argmax does it on its way and clears this)
@@ -509,12 +510,18 @@ bool engine_eligible(const pm_window * m) {
 
 // which single-token attention path the current sequence takes: 0 = one workgroup per head; else the cells the long-context grid is
 // sized for (power-of-two bucket >= position + 1, capped at n_ctx) - also the key of the captured step graph
-int attn_regime(const pm_window * m) {
-    const int pos = m->h_pos[m->h_seq];
-    if (!m->split_scratch || pos < m->split_min) return 0;
+int flash_bucket(const pm_window * m, int pos) {
     long b = 1024;
     while (b < (long) pos + 2) b *= 2;
     return (int) (b > m->hp.n_ctx ? m->hp.n_ctx : b);
+}
+int attn_regime(const pm_window * m) {
+    const int pos = m->h_pos[m->h_seq];
+    return !m->split_scratch || pos < m->split_min ? 0 : flash_bucket(m, pos);
+}
+// long contexts on the matrix cores, the keys split over workgroups (attn_flash_mfma.hip)
+bool flash_mfma_ok(const pm_window * m) {
+    return m->split_scratch && m->use_flash && m->attn_mfma && m->hp.n_head / m->hp.n_head_kv <= 8 && pm_attn_flash_cached_ok(m->hp.n_head, m->hp.n_head_kv, m->hp.head_dim, m->hp.n_ctx) == 0;
 }
 
 // the single-token layer sequence (5 launches per layer); the token's cos / sin table is there (m->rope_tab) where the window has one
@@ -527,7 +534,7 @@ int run_layers_fused(pm_window * m, const float * cur, float * d_x_out, const fl
     // rope + KV store in the QKV epilogue: NORM-mode rope, one-workgroup-per-head attention regime
     // (NEOX rope - build_qwen2 - where every workgroup's slice of wq / wk holds both halves of its rotation pairs: pm_launch_gemv_fused tells)
     bool epi = m->qkv_epi && m->rope_tab && (m->rope.mode == 0 || m->rope.mode == 2) &&
-               (!m->long_ctx || (m->use_flash && m->attn_mfma && H / Hkv <= 8 && pm_attn_flash_cached_ok(H, Hkv, dh, hp.n_ctx) == 0));
+               (!m->long_ctx || flash_mfma_ok(m));
     bool tail = epi && !m->long_ctx && m->attn_tail && m->att_tk && Hkv <= 64;
     double * ss_wo = (m->use_ss && m->ss) ? m->ss : nullptr, * ss_dn = ss_wo ? m->ss + 256 : nullptr;
     int n_wo = 0, n_dn = 0;                           // partials the previous wo / ffn_down launch left (0: the consumer reduces the row itself)
@@ -668,6 +675,16 @@ int run_window(pm_window * m, const int32_t * d_tokens, const float * d_x_in, in
     auto attend_rows = [&](const Layer & L) {
         const int rc = pm_launch_attn_cached(m->q, L.kc, L.vc, d_pos, d_seq, kv_stride, m->att, H, Hkv, dh, hp.n_ctx, kq_scale, st, nullptr, nullptr, rg ? rg->max_cells : 0, 0, 0, rg ? rg->n_rows : T, rg ? 1 : 0);
         return rc && !rg ? pm_launch_attn_decode(m->q, L.kc, L.vc, d_pos, d_seq, kv_stride, m->att, T, H, Hkv, dh, hp.n_ctx, kq_scale, st) : rc;
+    };
+    auto attend_long = [&](const Layer & L, int r) {
+        const long slab = (long) rg->h_seq[r] * kv_stride;
+        return pm_launch_attn_flash_cached(m->q + (size_t) r * Eq, (uint16_t *) L.kc + slab, (uint16_t *) L.vc + slab, rg->pos + r, nullptr, 0, m->att + (size_t) r * Eq, m->split_scratch, H, Hkv, dh,
+                                           hp.n_ctx, kq_scale, st, nullptr, nullptr, 0, flash_bucket(m, rg->h_pos[r]));
+    };
+    auto attend_ragged = [&](const Layer & L) {
+        if ((rg->n_rows && attend_rows(L)) || (rg->n_tiles && attend_mfma(L, m->att, nullptr, false))) return -1;
+        for (int r = T - rg->n_long; r < T; ++r) if (attend_long(L, r)) return -1;
+        return 0;
     };
     // the tokens' rows, and with them the cos / sin tables that the wq | wk | wv epilogues of all layers read
     const bool one = T == 1 && !m->no_fuse, tab = (one ? m->qkv_epi && m->rope_tab : small_epi) && m->hi > m->lo;
@@ -853,7 +870,7 @@ int run_window(pm_window * m, const int32_t * d_tokens, const float * d_x_in, in
         // cached cells, one workgroup per (head, token) (attn_cached.hip: one barrier up to 64 cells; 11 -> ~4 us per layer at 2..8 tokens)
         if (!rope_done) rope_store(L, 1);
         const bool mfma = !rg && small_attn_mfma(T, m->h_pos[m->h_seq]);
-        if (rg ? (rg->n_rows && attend_rows(L)) || (rg->n_tiles && attend_mfma(L, m->att, nullptr, false)) : !(mfma && attend_mfma(L, m->att, nullptr) == 0) && attend_rows(L))
+        if (rg ? attend_ragged(L) : !(mfma && attend_mfma(L, m->att, nullptr) == 0) && attend_rows(L))
             return seterr(m, PM355_E_RANGE, "decode: n_ctx too large for the decode-attention kernel");
         }
         const Tensor * wo[1] = {&L.t[PM355_T_WO]};
@@ -1323,7 +1340,8 @@ int pm_window::batch_rows(const pm355_batch_entry * e, int n, float * d_logits, 
     for (auto & L : layers) { const bool s8 = small_path(this, L, MMQ_MAX_TOKENS); every = every && s8; any = any || s8; }
     std::vector<int> tier;                                                                                 // the longest portion of each tier
     for (int t : {every ? 0 : SMALL_PLAIN_MAX, any ? MMQ_MAX_TOKENS : 0, max_tokens}) if (t > (tier.empty() ? 0 : tier.back()) && (tier.empty() || tier.back() < max_tokens)) tier.push_back(std::min(t, max_tokens));
-    struct Piece { int entry, off, T, pos0, out0; bool tiles; };                                           // tokens [off, off + T) of an entry, whose first wanted row is out0
+    enum { ROWS, TILES, LONG };                                                                            // attention, in the order of a pass's rows
+    struct Piece { int entry, off, T, pos0, out0, att; };                                                  // tokens [off, off + T) of an entry, whose first wanted row is out0
     struct Pass { std::vector<Piece> piece; int cap = 0, T = 0; };
     // attention of a portion of T tokens as it has it alone: one pass over the keys on the matrix cores, or a workgroup per head and token (whose scores are in LDS: 4 bytes a cell)
     auto in_tiles = [&](int T, int past) { return (T == 1 ? split_scratch && past >= split_min : small_attn_mfma(T, past)) || past + T > 32768; };
@@ -1344,11 +1362,37 @@ int pm_window::batch_rows(const pm355_batch_entry * e, int n, float * d_logits, 
                     if (!at || passes.back().T == passes.back().cap) { passes.emplace_back(); passes.back().cap = (int) (total * (at + 1) / k - total * at / k); ++at; }
                     Pass & p = passes.back();
                     const int T = std::min(p.cap - p.T, p1 - off);
-                    p.piece.push_back({i, off, T, past + off, out0, in_tiles(p1 - p0, past + p0)});
+                    p.piece.push_back({i, off, T, past + off, out0, in_tiles(p1 - p0, past + p0) ? TILES : ROWS});
                     p.T += T; off += T;
                 }
             }
     }
+    // Single tokens behind long histories. A tile has one workgroup per head walk all keys; the key-split kernel that such a token takes alone spreads them over the chip, but is a launch per
+    // token. The longest histories go there as far as that is the shorter sum (us): 9.3 + 1.07 per 1000 cells a launch, against 3 + 10.5 per 1000 cells of the longest history left or 13 of
+    // what a compute unit gets of all of them. Both round the probabilities in front of their division. Two layers of the 70B shape, us per step, one sequence after another / tiles /
+    // this rule: two sequences of 1500 cells 458 / 294 / 298, 6000 474 / 372 / 322, 12000 489 / 494 / 339, 32000 549 / 1044 / 403; eight of 6000 1929 / 607 / 559, of 32000 2208 / 1889 / 847; the 8B shape,
+    // two of 12000 262 / 363 / 210, eight of 32000 1295 / 1019 / 695
+    if (flash_mfma_ok(this))
+        for (Pass & p : passes) {
+            std::vector<Piece *> one;
+            double cells = 0, most = 0;                                                                      // of the tiles: all of them, the most of one
+            for (Piece & c : p.piece) {
+                if (c.att != TILES) continue;
+                if (c.T == 1) one.push_back(&c); else most = std::max(most, (double) (c.pos0 + c.T));
+                cells += (double) ((c.T + 63) / 64) * (c.pos0 + c.T);
+            }
+            std::sort(one.begin(), one.end(), [](const Piece * a, const Piece * b) { return a->pos0 > b->pos0; });
+            double split = 0, best = 1e30;
+            size_t n_best = 0;
+            for (size_t k = 0;; ++k) {
+                const double left = std::max(most, k < one.size() ? one[k]->pos0 + 1.0 : 0.0), tiles = left > 0 ? 3.0 + std::max(0.0105 * left, 0.013 * cells * hp.n_head / pm_device_cus()) : 0.0;
+                if (split + tiles < best) { best = split + tiles; n_best = k; }
+                if (k == one.size()) break;
+                split += 9.3 + 0.00107 * one[k]->pos0;
+                cells -= one[k]->pos0 + 1.0;
+            }
+            for (size_t k = 0; k < n_best; ++k) one[k]->att = LONG;
+        }
     struct Want { int row, out; };                                                                          // row of the pass, row of the outputs
     auto wanted = [&](const Piece & c, auto && f) { for (int j = 0; j < e[c.entry].n_want; ++j) if (e[c.entry].want[j] >= c.off && e[c.entry].want[j] < c.off + c.T) f(e[c.entry].want[j] - c.off, c.out0 + j); };
     for (const Pass & p : passes) {
@@ -1361,13 +1405,14 @@ int pm_window::batch_rows(const pm355_batch_entry * e, int n, float * d_logits, 
         const int T = p.T;
         std::vector<int32_t> tok, pos, seq, ent, keep;
         std::vector<Want> want;
-        int n_rows = 0, max_cells = 0;
-        std::stable_sort(p.piece.begin(), p.piece.end(), [](const Piece & a, const Piece & b) { return a.tiles < b.tiles; });      // (every row is stored before any attends: their order is free)
+        int n_rows = 0, max_cells = 0, n_long = 0;
+        std::stable_sort(p.piece.begin(), p.piece.end(), [](const Piece & a, const Piece & b) { return a.att < b.att; });      // (every row is stored before any attends: their order is free)
         for (const Piece & c : p.piece) {
             const pm355_batch_entry & x = e[c.entry];
             const int row = (int) tok.size();
             for (int t = 0; t < c.T; ++t) { tok.push_back(x.tokens ? x.tokens[c.off + t] : -1); pos.push_back(c.pos0 + t); seq.push_back(x.seq); }
-            if (!c.tiles) { n_rows += c.T; max_cells = std::max(max_cells, c.pos0 + c.T); }
+            n_long += c.att == LONG;
+            if (c.att == ROWS) { n_rows += c.T; max_cells = std::max(max_cells, c.pos0 + c.T); }
             size_t at_ent = 0;                                                                              // (pieces of one sequence may meet in a pass: one position per sequence)
             while (at_ent < ent.size() && ent[at_ent] != x.seq) at_ent += 2;
             if (at_ent == ent.size()) { ent.push_back(x.seq); ent.push_back(0); }
@@ -1381,12 +1426,12 @@ int pm_window::batch_rows(const pm355_batch_entry * e, int n, float * d_logits, 
         int n_tiles = 0;
         for (int r = 0; r < T;) {
             int r1 = r + 1;
-            while (r1 < T && r1 != n_rows && r1 - r < tile_q && seq[r1] == seq[r] && pos[r1] == pos[r1 - 1] + 1) ++r1;
+            while (r1 < T && r1 != n_rows && r1 < T - n_long && r1 - r < tile_q && seq[r1] == seq[r] && pos[r1] == pos[r1 - 1] + 1) ++r1;
             tl.push_back({r, r1 - r, pos[r], seq[r]});
-            if (r >= n_rows) ++n_tiles;
+            n_tiles += r >= n_rows && r < T - n_long;
             r = r1;
         }
-        std::rotate(tl.begin(), tl.end() - n_tiles, tl.end());
+        std::rotate(tl.begin(), tl.end() - n_tiles - n_long, tl.end());
         std::stable_sort(tl.begin(), tl.begin() + n_tiles, [](const Tile & a, const Tile & b) { return a.pos + a.n < b.pos + b.n; });      // (the kernel takes them from the end: most keys first)
         std::stable_sort(want.begin(), want.end(), [](const Want & a, const Want & b) { return a.out < b.out; });
         std::vector<int32_t> blk;
@@ -1398,7 +1443,7 @@ int pm_window::batch_rows(const pm355_batch_entry * e, int n, float * d_logits, 
         const int at_keep = put(keep.data(), keep.size());
         const pm_batch_layout lay = {T, at_seq, at_ent, (int) ent.size() / 2, at_keep, (int) keep.size() / 2, (int) blk.size(), e[n - 1].seq};
         if (pm_launch_batch_rows(d_rows, blk.data(), lay, d_last, st)) return seterr(m, PM355_E_HIP, "batch: table upload");
-        const Ragged r = {d_rows + at_pos, d_rows + at_seq, d_rows + at_tiles, n_tiles, (int) tl.size(), tile_q, n_rows, max_cells};
+        const Ragged r = {d_rows + at_pos, d_rows + at_seq, d_rows + at_tiles, n_tiles, (int) tl.size(), tile_q, n_rows, max_cells, n_long, pos.data(), seq.data()};
         int rc;
         if (T == 1) {                                                                                      // (one row is a step of its own, and that sequence's)
             rc = decode(seq[0], d_rows, nullptr, 1, pos[0], W ? rows : nullptr, nullptr, nullptr, st);

@@ -723,3 +723,29 @@ def test_a_portion_does_not_depend_on_the_histories_beside_it(E, arch):
     for other in (250, 420):
         assert all(E.torch.equal(x, y) for x, y in zip(got[other], got[5])), other
     assert E.torch.equal(got[5][-1], got[5][-2])
+
+
+def test_single_tokens_behind_long_histories_share_a_pass(E):
+    """Decoded tokens behind 3, 350, 1500 and 2900 cells in one pass: a workgroup per head, tiles of the matrix-core kernel and the key-split kernel side by side, wanted rows out of order.
+    Against the same tokens one sequence at a time (the same arithmetic, other summation orders: the bound of the comparisons above), step by step."""
+    torch = E.torch
+    rng = np.random.default_rng(17)
+    lens = [2900, 3, 1500, 350, 2870]
+    d = tiny_model(rng, n_layer=2, n_embd=512, n_head=8, n_head_kv=2, n_ff=1024, n_vocab=320, n_ctx=2944, rope_freqs=True)
+    toks = rng.integers(0, 320, (len(lens), 2944)).astype(np.int32)
+    ws = []
+    for _ in range(2):
+        w = _pool_window(E, d, 2944, 512, len(lens))
+        s = [w.seq_new() for _ in lens]
+        for i, n in enumerate(lens):
+            w.batch([(s[i], toks[i, :n], ())])
+        ws.append((w, s))
+    for step in range(4):
+        (w, s), (w1, s1) = ws
+        some = [i for i in range(len(lens)) if not (step == 2 and i == 1)]
+        a = _batch(E, w, [(s[i], toks[i, lens[i] + step:lens[i] + step + 1], (0,)) for i in some]).double()
+        b = torch.cat([_batch(E, w1, [(s1[i], toks[i, lens[i] + step:lens[i] + step + 1], (0,))]) for i in some]).double()
+        off = (a - b).square().sum(-1) / b.square().sum(-1)
+        assert bool((off < 1e-3).all()), (step, off.tolist())
+    for w, _ in ws:
+        w.close()
