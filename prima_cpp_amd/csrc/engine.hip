@@ -1441,37 +1441,40 @@ int pm_window::batch_rows(const pm355_batch_entry * e, int n, float * d_logits, 
         const int at_ent = put(ent.data(), ent.size()), at_want = (int) blk.size();
         for (const Want & w : want) blk.push_back(w.row);
         const int at_keep = put(keep.data(), keep.size());
-        const pm_batch_layout lay = {T, at_seq, at_ent, (int) ent.size() / 2, at_keep, (int) keep.size() / 2, (int) blk.size(), e[n - 1].seq};
-        if (pm_launch_batch_rows(d_rows, blk.data(), lay, d_last, st)) return seterr(m, PM355_E_HIP, "batch: table upload");
+        const pm_batch_layout lay = {T, at_seq, at_ent, (int) ent.size() / 2, (int) blk.size(), e[n - 1].seq};
+        if (pm_launch_batch_rows(d_rows, blk.data(), lay, d_last, d_pos, d_ctl, st)) return seterr(m, PM355_E_HIP, "batch: table upload");
         const Ragged r = {d_rows + at_pos, d_rows + at_seq, d_rows + at_tiles, n_tiles, (int) tl.size(), tile_q, n_rows, max_cells, n_long, pos.data(), seq.data()};
         int rc;
         if (T == 1) {                                                                                      // (one row is a step of its own, and that sequence's)
             rc = decode(seq[0], d_rows, nullptr, 1, pos[0], W ? rows : nullptr, nullptr, nullptr, st);
+            if (!rc) pm_launch_set_i32_pair(d_pos + seq[0], pos[0] + 1, d_ctl, e[n - 1].seq, st);
         } else {
             rag = &r;
             rc = run_window(m, d_rows, nullptr, T, W ? rows : nullptr, nullptr, nullptr, st);
             rag = nullptr;
         }
-        if (rc) return rc;
-        for (int w = 0; w < W;) {                                           // rows whose outputs are neighbours go through the head together
+        for (int w = 0; w < W && !rc;) {                                    // rows whose outputs are neighbours go through the head together
             int w1 = w + 1;
             while (w1 < W && w1 - w < std::min(max_tokens, HEAD_ROWS) && want[w1].out == want[w1 - 1].out + 1) ++w1;
             const int k = w1 - w, o = want[w].out;
             float * lg = d_logits ? d_logits + (size_t) o * V : head_lg;
             if (k == 1) rc = run_head(m, rows + (size_t) want[w].row * hp.n_embd, lg, d_argmax ? d_argmax + o : nullptr, st);
             else {
-                if (!output.d || !out_norm.d) return seterr(m, PM355_E_UNSUPPORTED, "head: output / output_norm missing");
+                if (!output.d || !out_norm.d) { rc = seterr(m, PM355_E_UNSUPPORTED, "head: output / output_norm missing"); break; }
                 const Tensor * ow[1] = {&output};
                 pm_launch_gather_rows(rows, d_rows + at_want + w, k, hp.n_embd, x1, st);
                 const ActQ a = norm_quantize_for(m, x1, (const float *) out_norm.d, hp.n_embd, k, ow, 1, st);
                 bool prepped = false;
-                if (matmul_small(m, output, a, k, lg, nullptr, nullptr, prepped, st)) return seterr(m, PM355_E_UNSUPPORTED, "head: lm_head mat-mul");
-                if (d_argmax) pm_launch_argmax(lg, V, d_argmax + o, nullptr, st, k, am_part);
+                if (matmul_small(m, output, a, k, lg, nullptr, nullptr, prepped, st)) rc = seterr(m, PM355_E_UNSUPPORTED, "head: lm_head mat-mul");
+                else if (d_argmax) pm_launch_argmax(lg, V, d_argmax + o, nullptr, st, k, am_part);
             }
-            if (rc) return rc;
             w = w1;
         }
-        pm_launch_batch_end(d_rows, lay, d_argmax, d_last, d_pos, d_ctl, st);
+        if (rc) {                                                           // (refused: the device's positions are the host's again)
+            for (size_t k = 0; k < ent.size(); k += 2) pm_launch_set_i32_pair(d_pos + ent[k], h_pos[ent[k]], d_ctl, h_seq, st);
+            return rc;
+        }
+        if (!keep.empty()) pm_launch_keep_last(d_argmax, d_rows + at_keep, (int) keep.size() / 2, d_last, st);
         for (size_t k = 0; k < ent.size(); k += 2) h_pos[ent[k]] = ent[k + 1];
         h_seq = e[n - 1].seq;
     }

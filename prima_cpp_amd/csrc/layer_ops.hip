@@ -399,22 +399,23 @@ __global__ void advance_kernel(int32_t * pos, int32_t * ctl, int by, int rotate)
 }
 __global__ void set_i32_kernel(int32_t * p, int v) { *p = v; }
 // The tables of a pass over rows of several sequences: integers that travel as kernel arguments (up to 960: no staging copy, nothing of the caller's outlives the call) or are in
-// place already, and tokens that are taken from the device (-1: the sequence's last greedy token).
+// place already, tokens that are taken from the device (-1: the sequence's last greedy token), and the sequences' positions behind the pass (a launch of their own at its end cost 2-4 us
+// a step; the caller takes them back where the pass is refused).
 struct BatchInts { int32_t v[960]; };
-__global__ __launch_bounds__(256) void batch_rows_kernel(BatchInts a, int n, int32_t * blk, pm_batch_layout l, const int32_t * last) {
+__global__ __launch_bounds__(256) void batch_rows_kernel(BatchInts a, int n, int32_t * blk, pm_batch_layout l, const int32_t * last, int32_t * pos, int32_t * ctl) {
     for (int i = threadIdx.x; i < n; i += 256) blk[i] = a.v[i];
     __syncthreads();
     for (int t = threadIdx.x; t < l.T; t += 256) if (blk[t] < 0) blk[t] = last[blk[l.seq + t]];
+    for (int i = threadIdx.x; i < l.n_entries; i += 256) pos[blk[l.entries + 2 * i]] = blk[l.entries + 2 * i + 1];
+    if (threadIdx.x == 0) ctl[0] = l.current;
 }
 __global__ __launch_bounds__(256) void gather_rows_kernel(const float * x, const int32_t * at, int K, float * y) {
     const int i = (int) (blockIdx.x * 256 + threadIdx.x);
     if (4 * i < K) *(float4 *) (y + (size_t) blockIdx.y * K + 4 * i) = *(const float4 *) (x + (size_t) at[blockIdx.y] * K + 4 * i);
 }
-// The end of a pass, behind everything that could still be refused: positions of its sequences, the batch's last sequence current, and greedy tokens where the next step's embedding finds them
-__global__ __launch_bounds__(256) void batch_end_kernel(const int32_t * blk, pm_batch_layout l, const int32_t * argmax, int32_t * last, int32_t * pos, int32_t * ctl) {
-    for (int i = threadIdx.x; i < l.n_entries; i += 256) pos[blk[l.entries + 2 * i]] = blk[l.entries + 2 * i + 1];
-    for (int i = threadIdx.x; i < l.n_keep; i += 256) last[blk[l.keep + 2 * i]] = argmax[blk[l.keep + 2 * i + 1]];
-    if (threadIdx.x == 0) ctl[0] = l.current;
+__global__ __launch_bounds__(64) void keep_last_kernel(const int32_t * argmax, const int32_t * pairs, int n, int32_t * last) {      // pairs {sequence, row of argmax}
+    const int i = (int) (blockIdx.x * 64 + threadIdx.x);
+    if (i < n) last[pairs[2 * i]] = argmax[pairs[2 * i + 1]];
 }
 __global__ void set_i32_pair_kernel(int32_t * p, int a, int32_t * q, int b) { *p = a; *q = b; }
 __global__ void set_i32x2_kernel(int32_t * p, int a, int b) { p[0] = a; p[1] = b; }
@@ -503,19 +504,19 @@ void pm_launch_argmax(const float * x, int n, int32_t * idx, float * val, hipStr
     const int nb = part ? std::min(PM_ARGMAX_PARTS, (n + 4095) / 4096) : 1;               // (a workgroup per 4096 values: a row of a small vocabulary stays with one)
     hipLaunchKernelGGL(argmax_kernel, dim3(nb, rows), dim3(1024), 0, st, x, n, idx, val, part, pos, ctl, by, rotate);
 }
-int pm_launch_batch_rows(int32_t * blk, const int32_t * host, const pm_batch_layout & l, const int32_t * last, hipStream_t st) {
+int pm_launch_batch_rows(int32_t * blk, const int32_t * host, const pm_batch_layout & l, const int32_t * last, int32_t * pos, int32_t * ctl, hipStream_t st) {
     BatchInts a;
     const bool fits = l.n_ints <= (int) (sizeof(a.v) / 4);
     if (fits) std::memcpy(a.v, host, (size_t) l.n_ints * 4);
     else if (hipMemcpyAsync(blk, host, (size_t) l.n_ints * 4, hipMemcpyHostToDevice, st) != hipSuccess) return -1;
-    hipLaunchKernelGGL(batch_rows_kernel, dim3(1), dim3(256), 0, st, a, fits ? l.n_ints : 0, blk, l, last);
+    hipLaunchKernelGGL(batch_rows_kernel, dim3(1), dim3(256), 0, st, a, fits ? l.n_ints : 0, blk, l, last, pos, ctl);
     return 0;
 }
 void pm_launch_gather_rows(const float * x, const int32_t * at, int n, int K, float * y, hipStream_t st) {
     hipLaunchKernelGGL(gather_rows_kernel, dim3((K / 4 + 255) / 256, n), dim3(256), 0, st, x, at, K, y);
 }
-void pm_launch_batch_end(const int32_t * blk, const pm_batch_layout & l, const int32_t * argmax, int32_t * last, int32_t * pos, int32_t * ctl, hipStream_t st) {
-    hipLaunchKernelGGL(batch_end_kernel, dim3(1), dim3(256), 0, st, blk, l, argmax, last, pos, ctl);
+void pm_launch_keep_last(const int32_t * argmax, const int32_t * pairs, int n, int32_t * last, hipStream_t st) {
+    hipLaunchKernelGGL(keep_last_kernel, dim3((n + 63) / 64), dim3(64), 0, st, argmax, pairs, n, last);
 }
 void pm_launch_add(const float * a, const float * b, float * y, long n, long nb, hipStream_t st) {
     hipLaunchKernelGGL(add_kernel, dim3((unsigned) ((n + 255) / 256)), dim3(256), 0, st, a, b, y, n, nb);

@@ -81,12 +81,12 @@ constexpr int PM_ARGMAX_PARTS = 32, PM_ARGMAX_ROWS = 64;
 constexpr size_t PM_ARGMAX_SCRATCH = (size_t) PM_ARGMAX_ROWS * (4 + PM_ARGMAX_PARTS * 8);
 void pm_launch_argmax(const float * x, int n, int32_t * idx, float * val, hipStream_t st, int rows = 1, uint64_t * part = nullptr, int32_t * pos = nullptr, int32_t * ctl = nullptr,
                       int by = 0, int rotate = 0);
-// a pass over T rows of several sequences: block of int32 = tokens [T] | positions [T] | sequences [T] | ... ; offsets in integers. entries: {sequence, position behind the pass};
-// keep: {sequence, row of argmax}. batch_rows in front of the pass, batch_end behind it: pos[sequence] = position, last[sequence] = argmax[row], ctl[0] = current
-struct pm_batch_layout { int T, seq, entries, n_entries, keep, n_keep, n_ints, current; };
-int  pm_launch_batch_rows(int32_t * blk, const int32_t * host, const pm_batch_layout & l, const int32_t * last, hipStream_t st);
-void pm_launch_batch_end(const int32_t * blk, const pm_batch_layout & l, const int32_t * argmax, int32_t * last, int32_t * pos, int32_t * ctl, hipStream_t st);
+// a pass over T rows of several sequences: block of int32 = tokens [T] | positions [T] | sequences [T] | ... ; offsets in integers. entries: {sequence, position behind the pass}; ctl[0] =
+// current
+struct pm_batch_layout { int T, seq, entries, n_entries, n_ints, current; };
+int  pm_launch_batch_rows(int32_t * blk, const int32_t * host, const pm_batch_layout & l, const int32_t * last, int32_t * pos, int32_t * ctl, hipStream_t st);
 void pm_launch_gather_rows(const float * x, const int32_t * at, int n, int K, float * y, hipStream_t st);                  // y[i] = x[at[i]], K % 4 == 0
+void pm_launch_keep_last(const int32_t * argmax, const int32_t * pairs, int n, int32_t * last, hipStream_t st);             // last[pairs[i].sequence] = argmax[pairs[i].row]
 void pm_launch_add(const float * a, const float * b, float * y, long n, long nb, hipStream_t st);
 void pm_launch_mul(const float * a, const float * b, float * y, long n, long nb, hipStream_t st);
 void pm_launch_silu_mul(const float * g, const float * u, float * y, long n, hipStream_t st);
