@@ -1442,7 +1442,7 @@ int pm_window::batch_rows(const pm355_batch_entry * e, int n, float * d_logits, 
         for (const Want & w : want) blk.push_back(w.row);
         const int at_keep = put(keep.data(), keep.size());
         const pm_batch_layout lay = {T, at_seq, at_ent, (int) ent.size() / 2, (int) blk.size(), e[n - 1].seq};
-        if (pm_launch_batch_rows(d_rows, blk.data(), lay, d_last, d_pos, d_ctl, st)) return seterr(m, PM355_E_HIP, "batch: table upload");
+        pm_launch_batch_rows(d_rows, blk.data(), lay, d_last, d_pos, d_ctl, st);
         const Ragged r = {d_rows + at_pos, d_rows + at_seq, d_rows + at_tiles, n_tiles, (int) tl.size(), tile_q, n_rows, max_cells, n_long, pos.data(), seq.data()};
         int rc;
         if (T == 1) {                                                                                      // (one row is a step of its own, and that sequence's)

@@ -398,12 +398,15 @@ __global__ void advance_kernel(int32_t * pos, int32_t * ctl, int by, int rotate)
     if (rotate) ctl[0] = (s + rotate) % ctl[1];
 }
 __global__ void set_i32_kernel(int32_t * p, int v) { *p = v; }
-// The tables of a pass over rows of several sequences: integers that travel as kernel arguments (up to 960: no staging copy, nothing of the caller's outlives the call) or are in
-// place already, tokens that are taken from the device (-1: the sequence's last greedy token), and the sequences' positions behind the pass (a launch of their own at its end cost 2-4 us
-// a step; the caller takes them back where the pass is refused).
+// The tables of a pass over rows of several sequences: integers that travel as kernel arguments (no staging copy, nothing of the caller's is read behind the call, also where the pass is
+// captured), more than 960 of them by several launches. The last one takes tokens from the device (-1: the sequence's last greedy token) and moves the sequences' positions behind the pass
+// (a launch of its own at the end cost 2-4 us a step; the caller takes them back where the pass is refused).
 struct BatchInts { int32_t v[960]; };
-__global__ __launch_bounds__(256) void batch_rows_kernel(BatchInts a, int n, int32_t * blk, pm_batch_layout l, const int32_t * last, int32_t * pos, int32_t * ctl) {
-    for (int i = threadIdx.x; i < n; i += 256) blk[i] = a.v[i];
+__global__ __launch_bounds__(256) void batch_ints_kernel(BatchInts a, int32_t * blk) {
+    for (int i = threadIdx.x; i < 960; i += 256) blk[i] = a.v[i];
+}
+__global__ __launch_bounds__(256) void batch_rows_kernel(BatchInts a, int n, int at, int32_t * blk, pm_batch_layout l, const int32_t * last, int32_t * pos, int32_t * ctl) {
+    for (int i = threadIdx.x; i < n; i += 256) blk[at + i] = a.v[i];
     __syncthreads();
     for (int t = threadIdx.x; t < l.T; t += 256) if (blk[t] < 0) blk[t] = last[blk[l.seq + t]];
     for (int i = threadIdx.x; i < l.n_entries; i += 256) pos[blk[l.entries + 2 * i]] = blk[l.entries + 2 * i + 1];
@@ -504,13 +507,16 @@ void pm_launch_argmax(const float * x, int n, int32_t * idx, float * val, hipStr
     const int nb = part ? std::min(PM_ARGMAX_PARTS, (n + 4095) / 4096) : 1;               // (a workgroup per 4096 values: a row of a small vocabulary stays with one)
     hipLaunchKernelGGL(argmax_kernel, dim3(nb, rows), dim3(1024), 0, st, x, n, idx, val, part, pos, ctl, by, rotate);
 }
-int pm_launch_batch_rows(int32_t * blk, const int32_t * host, const pm_batch_layout & l, const int32_t * last, int32_t * pos, int32_t * ctl, hipStream_t st) {
+void pm_launch_batch_rows(int32_t * blk, const int32_t * host, const pm_batch_layout & l, const int32_t * last, int32_t * pos, int32_t * ctl, hipStream_t st) {
     BatchInts a;
-    const bool fits = l.n_ints <= (int) (sizeof(a.v) / 4);
-    if (fits) std::memcpy(a.v, host, (size_t) l.n_ints * 4);
-    else if (hipMemcpyAsync(blk, host, (size_t) l.n_ints * 4, hipMemcpyHostToDevice, st) != hipSuccess) return -1;
-    hipLaunchKernelGGL(batch_rows_kernel, dim3(1), dim3(256), 0, st, a, fits ? l.n_ints : 0, blk, l, last, pos, ctl);
-    return 0;
+    constexpr int N = sizeof(a.v) / 4;
+    int at = 0;
+    for (; l.n_ints - at > N; at += N) {
+        std::memcpy(a.v, host + at, sizeof(a.v));
+        hipLaunchKernelGGL(batch_ints_kernel, dim3(1), dim3(256), 0, st, a, blk + at);
+    }
+    std::memcpy(a.v, host + at, (size_t) (l.n_ints - at) * 4);
+    hipLaunchKernelGGL(batch_rows_kernel, dim3(1), dim3(256), 0, st, a, l.n_ints - at, at, blk, l, last, pos, ctl);
 }
 void pm_launch_gather_rows(const float * x, const int32_t * at, int n, int K, float * y, hipStream_t st) {
     hipLaunchKernelGGL(gather_rows_kernel, dim3((K / 4 + 255) / 256, n), dim3(256), 0, st, x, at, K, y);

@@ -84,7 +84,7 @@ void pm_launch_argmax(const float * x, int n, int32_t * idx, float * val, hipStr
 // a pass over T rows of several sequences: block of int32 = tokens [T] | positions [T] | sequences [T] | ... ; offsets in integers. entries: {sequence, position behind the pass}; ctl[0] =
 // current
 struct pm_batch_layout { int T, seq, entries, n_entries, n_ints, current; };
-int  pm_launch_batch_rows(int32_t * blk, const int32_t * host, const pm_batch_layout & l, const int32_t * last, int32_t * pos, int32_t * ctl, hipStream_t st);
+void pm_launch_batch_rows(int32_t * blk, const int32_t * host, const pm_batch_layout & l, const int32_t * last, int32_t * pos, int32_t * ctl, hipStream_t st);
 void pm_launch_gather_rows(const float * x, const int32_t * at, int n, int K, float * y, hipStream_t st);                  // y[i] = x[at[i]], K % 4 == 0
 void pm_launch_keep_last(const int32_t * argmax, const int32_t * pairs, int n, int32_t * last, hipStream_t st);             // last[pairs[i].sequence] = argmax[pairs[i].row]
 void pm_launch_add(const float * a, const float * b, float * y, long n, long nb, hipStream_t st);

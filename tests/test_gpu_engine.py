@@ -749,3 +749,42 @@ def test_single_tokens_behind_long_histories_share_a_pass(E):
         assert bool((off < 1e-3).all()), (step, off.tolist())
     for w, _ in ws:
         w.close()
+
+
+def test_large_batches_of_several_sequences(E):
+    """Portions of up to 600 tokens in passes of 512 rows: tables of more than one launch's arguments, rope + store by token with a position and a sequence per row, tiles of 64 and 128
+    queries, argmax over rows that several workgroups share (odd vocabulary: rows that do not start on 16 bytes). Against one sequence at a time; then the same captured on a stream and
+    replayed after the host's arrays are gone."""
+    torch = E.torch
+    rng = np.random.default_rng(18)
+    lens, V, n_ctx = [600, 33, 290, 431, 50], 4099, 640
+    d = tiny_model(rng, n_layer=2, n_embd=1024, n_head=16, n_head_kv=4, n_ff=1024, n_vocab=V, n_ctx=n_ctx, rope_freqs=True)
+    toks = [rng.integers(0, V, n).astype(np.int32) for n in lens]
+    st = torch.cuda.Stream()
+    with torch.cuda.stream(st):
+        w, w1 = (_pool_window(E, d, n_ctx, 512, len(lens)) for _ in range(2))
+        s, s1 = ([m.seq_new() for _ in lens] for m in (w, w1))
+        lg, am = _batch(E, w, [(q, t, (len(t) - 1, len(t) - 7)) for q, t in zip(s, toks)], argmax=True)
+        lg1 = torch.cat([_batch(E, w1, [(q, t, (len(t) - 1, len(t) - 7))]) for q, t in zip(s1, toks)])
+        assert torch.equal(am.long(), lg.argmax(-1))
+        off = (lg - lg1).double().square().sum(-1) / lg1.double().square().sum(-1)
+        assert bool((off < 1e-3).all()), off.tolist()
+        assert [w.seq_len(q) for q in s] == lens
+        for q in s:
+            w.seq_free(q)
+        s = [w.seq_new() for _ in lens]
+        out = torch.zeros((2 * len(lens), V), device="cuda")
+        g = torch.cuda.CUDAGraph()
+        torch.cuda.synchronize()
+        with torch.cuda.graph(g, stream=st, capture_error_mode="relaxed"):
+            w.batch([(q, t.copy(), (len(t) - 1, len(t) - 7)) for q, t in zip(s, toks)], logits=out)
+        junk = [np.full(1 << 16, 0x7f7f7f7f, dtype=np.int32) for _ in range(64)]      # (what the call allocated is someone else's by now)
+        for _ in range(3):
+            out.zero_()
+            g.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(out, lg)
+            torch.cuda.synchronize()
+        del junk
+    w.close()
+    w1.close()
