@@ -788,3 +788,32 @@ def test_large_batches_of_several_sequences(E):
         del junk
     w.close()
     w1.close()
+
+
+@pytest.mark.parametrize("arch,types,n_vocab", [(0, dict(attn_v=Q4_K), 320), (0, dict(attn_v=Q6_K), 4099), (0, {}, 320), (1, dict(attn_v=Q6_K), 4099), (0, dict(attn_v=Q4_K, output=Q4_K), 8197)])
+def test_shared_passes_on_the_integer_products(E, arch, types, n_vocab):
+    """Matrices of 512 columns and more take the integer small-batch products, with rope and KV store in the epilogue of wq | wk | wv (one launch for three matrices of a type, two parts for
+    another wv, NEOX in a launch of its own), and the head the same for neighbouring rows: passes of 3, 8, 9, 17, 26 and 32 rows of several sequences against one sequence at a time."""
+    torch = E.torch
+    rng = np.random.default_rng(19 + arch)
+    d = tiny_model(rng, arch=arch, n_layer=2, n_embd=1024, n_head=8, n_head_kv=2, n_ff=1536, n_vocab=n_vocab, n_ctx=224, types=types, rope_freqs=arch == 0)
+    w, w1 = (_pool_window(E, d, 224, 64, 4) for _ in range(2))
+    s, s1 = ([m.seq_new() for _ in range(4)] for m in (w, w1))
+    for ns in ((1, 2, 0, 0), (3, 2, 1, 2), (1, 4, 3, 1), (5, 1, 9, 2), (8, 8, 2, 8), (14, 1, 16, 1), (32, 20, 12, 32), (31, 3, 40, 1), (1, 1, 1, 1), (1, 0, 1, 1)):
+        entries = [(i, rng.integers(0, n_vocab, n).astype(np.int32), range(n - 1, max(n - 5, -1), -1) if i % 2 else (n - 1,)) for i, n in enumerate(ns) if n]
+        a, am = _batch(E, w, [(s[i], t, want) for i, t, want in entries], argmax=True)
+        b = torch.cat([_batch(E, w1, [(s1[i], t, want)]) for i, t, want in entries]).double()
+        off = (a - b).square().sum(-1) / b.square().sum(-1)
+        assert bool((off < 1e-3).all()), (ns, off.tolist())
+        assert torch.equal(am.long(), a.argmax(-1))
+    # equal rows of the head in several workgroups' parts: the first one wins in every row
+    if n_vocab > 4096:
+        best, k = int(am[0]), E.L.row_size(d.output.type, 1024)
+        head = np.ctypeslib.as_array((np.ctypeslib.ctypes.c_uint8 * (k * n_vocab)).from_address(d.output.data)).reshape(n_vocab, k)
+        head[[7, n_vocab - 1]] = head[best]
+        w._chk(w.lib.pm355_model_set_tensor(w.h, E.T_OUTPUT, -1, d.output.type, d.output.data, k * n_vocab), "output")
+        torch.cuda.synchronize()
+        a, am = _batch(E, w, [(s[i], t, want) for i, t, want in entries], argmax=True)
+        assert torch.equal(a[:, 7], a[:, -1]) and am.tolist() == a.cpu().numpy().argmax(-1).tolist() and 7 in am.tolist()
+    w.close()
+    w1.close()
