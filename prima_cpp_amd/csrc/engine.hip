@@ -318,9 +318,9 @@ const int MMQ_MAX_TOKENS = [] { const char * e = getenv("PM355_MMQ_MAX_TOKENS");
 // small batches of at least so many tokens, or that attend at least so many cells, take the prompt path's matrix-core kernel (attn_prefill.hip); the others one workgroup per
 // (head, token) (attn_cached.hip). Layer of the 70B shape, 2 / 8 / 15 tokens: behind 120 cells 134.0 / 158.0 / 176.5 us with the workgroups per token, 133.7 / 157.4 / 170.7 on the matrix
 // cores; behind 300 141.6 / 165.3 / 188.7 against 136.4 / 159.5 / 172.2, behind 3000 194 / 249 / 358 against 162 / 185 / 200; of the 8B shape behind 30 cells 67.5 / 84.0 / 89.6 against
-// 69.8 / 86.4 / 92.0, behind 300 76.3 / 91.7 / 99.3 against 72.4 / 89.1 / 94.5
-const int SMALL_ATTN_MFMA_MIN = [] { const char * e = getenv("PM355_SMALL_ATTN_MFMA_MIN"); return e ? atoi(e) : 16; }();
-const int SMALL_ATTN_MFMA_CELLS = 192;
+// 69.8 / 86.4 / 92.0, behind 300 76.3 / 91.7 / 99.3 against 72.4 / 89.1 / 94.5. PM355_SMALL_ATTN_MFMA_MIN = n: from n tokens on, whatever the cells
+const char * const SMALL_ATTN_ENV = getenv("PM355_SMALL_ATTN_MFMA_MIN");
+const int SMALL_ATTN_MFMA_MIN = SMALL_ATTN_ENV ? atoi(SMALL_ATTN_ENV) : 16, SMALL_ATTN_MFMA_CELLS = SMALL_ATTN_ENV ? INT32_MAX : 192;
 bool small_attn_mfma(int T, int past) { return T >= SMALL_ATTN_MFMA_MIN || past + T >= SMALL_ATTN_MFMA_CELLS; }
 constexpr int HEAD_ROWS = 32;            // rows of a batch that go through the head at once (what one pass of the integer mat-mul takes)
 const int MMQ_MULTI_MIN_TOKENS = 2;       // the fused wq | wk | wv and ffn_gate | ffn_up launches already win at 2 tokens (3 / 4 mat-vec launches otherwise)
@@ -1297,7 +1297,7 @@ int pm_window::generate(int32_t * d_io, int pos0, int n_steps, int use_graph, hi
     return 0;
 }
 
-// ---- batches: every entry is a portion of one open sequence; a sequence holds one KV slab of n_ctx cells, portions run one after another ----------------------
+// ---- batches: every entry is a portion of one open sequence; a sequence holds one KV slab of n_ctx cells, portions of similar length share passes ----------------------
 int pm_window::finalize_pool(int max_tokens_, int n_seq_, int64_t pool_tokens) {
     if (pool_tokens > (int64_t) n_seq_ * hp.n_ctx) return seterr(this, PM355_E_RANGE, "finalize_pool: more tokens than n_seq slabs of n_ctx cells hold");
     if (!(flags & PM355_HAS_EMBD) || !(flags & PM355_HAS_HEAD)) return seterr(this, PM355_E_UNSUPPORTED, "finalize_pool: batches need the embedding and the head");
@@ -1328,9 +1328,9 @@ int pm_window::pool_info(pm355_pool_info * o) {
 }
 // All entries as rows of common passes: the weights are read once per pass instead of once per sequence (eight sequences of the 8B shape, eight layers and
 // head: prompts of 12..24 tokens and twelve steps 47.0 ms one sequence after another, 14.0 ms as common passes). A portion keeps the arithmetic that it has alone - up to 32 tokens 8-bit
-// activations, beyond 16-bit ones; up to 15 where a layer has no 8-bit path, and between the two either, layer by layer; probabilities rounded before or behind their division - whatever
-// shares the step with it: portions meet in passes of their own tier, the longer ones (a sequence's first) first, and a row's attention is chosen by its own portion and history. served =
-// false and nothing done where a pass does not take rows of several sequences.
+// activations, beyond 16-bit ones; up to 15 where a layer has no 8-bit path, and between the two either, layer by layer - whatever shares the step with it: portions meet in passes of
+// their own tier, the longer ones (a sequence's first) first, and the attention of a portion is chosen by the cells that it attends itself. served = false and nothing done where a pass does
+// not take rows of several sequences.
 int pm_window::batch_rows(const pm355_batch_entry * e, int n, float * d_logits, int32_t * d_argmax, hipStream_t st, bool * served) {
     pm_window * m = this;
     *served = false;
@@ -1343,8 +1343,11 @@ int pm_window::batch_rows(const pm355_batch_entry * e, int n, float * d_logits, 
     enum { ROWS, TILES, LONG };                                                                            // attention, in the order of a pass's rows
     struct Piece { int entry, off, T, pos0, out0, att; };                                                  // tokens [off, off + T) of an entry, whose first wanted row is out0
     struct Pass { std::vector<Piece> piece; int cap = 0, T = 0; };
-    // attention of a portion of T tokens as it has it alone: one pass over the keys on the matrix cores, or a workgroup per head and token (whose scores are in LDS: 4 bytes a cell)
-    auto in_tiles = [&](int T, int past) { return (T == 1 ? split_scratch && past >= split_min : small_attn_mfma(T, past)) || past + T > 32768; };
+    // attention of a portion of T tokens: one pass over the keys on the matrix cores, or a workgroup per head and token (whose scores are in LDS: 4 bytes a cell). Alone, 16 tokens and more take
+    // the matrix cores behind any history, and a single one behind 320 cells: they then round the probabilities in front of their division where a shared pass rounds behind it, or the other
+    // way round, 2^-11 of each. Held to the same kernel here, short prompts pay for it (eight prompts of 12..24 tokens of the 8B shape: a tile launch of 8.5 us where the rows take 4; with twelve
+    // steps behind 13.41 instead of 13.22 ms)
+    auto in_tiles = [&](int T, int past) { return past + T > 32768 || (SMALL_ATTN_ENV ? small_attn_mfma(T, past) : past + T >= SMALL_ATTN_MFMA_CELLS); };
     std::vector<Pass> passes;
     for (int tr = (int) tier.size() - 1; tr >= 0; --tr) {
         const int above = tr ? tier[tr - 1] : 0, most = tier[tr];

@@ -705,24 +705,21 @@ def test_portions_keep_their_tier_where_only_some_layers_have_an_8_bit_path(E):
 
 @pytest.mark.parametrize("arch", [0, 1])
 def test_a_portion_does_not_depend_on_the_histories_beside_it(E, arch):
-    """A sequence's rows next to short and to long histories: the pass has the same rows, so the same products, and the attention of a row is chosen by its own sequence - equal bits. And
-    twenty tokens next to a single one as twenty tokens alone: the products of 17 to 32 rows sum alike."""
+    """A sequence's rows next to short and to long histories: the pass has the same rows, so the same products, and the attention of a row is chosen by its own sequence - equal bits"""
     rng = np.random.default_rng(3 + arch)
     d = tiny_model(rng, arch=arch, n_layer=2, n_embd=512, n_head=8, n_head_kv=2, n_ff=1024, n_vocab=320, n_ctx=448, types=dict(attn_v=Q6_K))
     toks = rng.integers(0, 320, 448).astype(np.int32)
     got = {}
     for other in (5, 250, 420):                            # cells of the sequence beside them
         w = _pool_window(E, d, 448, 64, 4)
-        a, b, c, e = (w.seq_new() for _ in range(4))
+        a, b, c = (w.seq_new() for _ in range(3))
         w.batch([(a, toks[:10], ())])
         w.batch([(b, toks[:other], ())])
         got[other] = [_batch(E, w, [(a, toks[i:i + 1], (0,)), (b, toks[i:i + 1], (0,))])[0] for i in range(10, 14)]
         got[other].append(_batch(E, w, [(c, toks[:20], (19,)), (b, toks[:1], ())]))
-        got[other].append(_batch(E, w, [(e, toks[:20], (19,))]))
         w.close()
     for other in (250, 420):
         assert all(E.torch.equal(x, y) for x, y in zip(got[other], got[5])), other
-    assert E.torch.equal(got[5][-1], got[5][-2])
 
 
 def test_single_tokens_behind_long_histories_share_a_pass(E):
