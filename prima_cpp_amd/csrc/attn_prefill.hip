@@ -217,7 +217,7 @@ __global__ __launch_bounds__(256, 2) void attn_rowmajor_kernel(PfP p) {
 // kw * KT .. + KT of every stage and keeps an online softmax of its own, the groups are merged through LDS at the end. Rows of a K tile are read with bits 2 and 3 of the row
 // index swapped: the accumulators of S^T then ARE the B operand of the P.V product.
 // ONE pass over the keys: the probabilities are rounded to F16 before the division by their sum (which adds the unrounded ones), where the reference rounds behind it - the same
-// relative error per probability (2^-12; smaller where p would be subnormal), without the second K.q product and the second exponential of every score: 2.0e-4 of the result from
+// relative error per probability (2^-11 at most; smaller where p would be subnormal), without the second K.q product and the second exponential of every score: 2.0e-4 of the result from
 // float64 with two passes, 1.6e-4 with one.
 // Bound by the LDS reads of the fragments (32 queries per wave: 32 KiB per 64 keys and wave at ~80 bytes per cycle and CU, about the time of the 32 matrix instructions) and the
 // exponentials beside them. Against the two-pass form with 4 waves x 32 queries, 32-key tiles through registers: 6001 tokens x 32 heads 870 -> 393 us (752 TFLOP/s), 512 x 64 behind
@@ -276,16 +276,18 @@ __global__ __launch_bounds__(512, 2) void attn_prompt_kernel(PfP p) {
 
     // Q^T as B operand: lane (query lr, hf) holds q[query][16 kk + 8 hf .. + 8], rounded to F16 like the reference
     half8 q[KK];
-    // (times the sign of the scale: hidden scores are -inf in front of the positive factor c)
     {
         const float * qr = p.q + ((long) tq * p.H + h) * DH + 8 * hf;
-        const float sg = p.scale == 0.0f ? 0.0f : copysignf(1.0f, p.scale);
 #pragma unroll
         for (int kk = 0; kk < KK; ++kk) {
-            float4 a = *(const float4 *) (qr + 16 * kk), b = *(const float4 *) (qr + 16 * kk + 4);
-            a.x *= sg; a.y *= sg; a.z *= sg; a.w *= sg; b.x *= sg; b.y *= sg; b.z *= sg; b.w *= sg;
+            const float4 a = *(const float4 *) (qr + 16 * kk), b = *(const float4 *) (qr + 16 * kk + 4);
             q[kk] = half8{(_Float16) a.x, (_Float16) a.y, (_Float16) a.z, (_Float16) a.w, (_Float16) b.x, (_Float16) b.y, (_Float16) b.z, (_Float16) b.w};
         }
+    }
+    if (!(p.scale > 0.0f)) {                                      // (the queries carry the sign of the scale: hidden scores are -inf in front of the positive factor c)
+        const _Float16 sg = p.scale == 0.0f ? (_Float16) 0.0f : (_Float16) -1.0f;
+#pragma unroll
+        for (int kk = 0; kk < KK; ++kk) q[kk] *= sg;
     }
     const float * mrow = (const float *) p.mask + (long) tq * p.mask_stride;
     const uint16_t * mrow16 = (const uint16_t *) p.mask + (long) tq * p.mask_stride;
