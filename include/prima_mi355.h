@@ -247,16 +247,17 @@ PM355_API size_t pm355_attn_split_scratch_floats(int n_head, int head_dim, int n
 PM355_API int pm355_attn_decode_split(const float * q_rot, const void * k_cache, const void * v_cache, const int32_t * d_pos0,
                                       float * out, float * scratch, int n_head, int n_head_kv, int head_dim, int n_ctx,
                                       float kq_scale, pm355_stream_t stream);
-/* the same chain for a multi-token (prefill) batch on the MFMA matrix cores: causal, two passes over the keys so that p is
- * rounded to F16 after the division by the full row sum like the reference (prima_cpp_amd/csrc/attn_prefill.hip).
- * head_dim 64 or 128, n_ctx % 32 == 0. Same arguments and result layout as pm355_attn_decode. */
+/* the same chain for a multi-token (prefill) batch on the MFMA matrix cores: causal, one pass over the keys; the probabilities are rounded to F16
+ * in front of their division by the row sum, where the reference rounds behind it (prima_cpp_amd/csrc/attn_prefill.hip; the same 2^-11 of each).
+ * head_dim 64 or 128, n_ctx % 32 == 0. Same arguments and result layout as pm355_attn_decode. Cells behind the last query's position may hold anything. */
 PM355_API int pm355_attn_prefill(const float * q, const void * k_cache, const void * v_cache, const int32_t * d_pos0,
                                  float * out, int n_tokens, int n_head, int n_head_kv, int head_dim, int n_ctx,
                                  float kq_scale, pm355_stream_t stream);
 /* ggml-graph form of pm355_attn_prefill: the node chain MUL_MAT(k, q) SOFT_MAX(kq, KQ_mask, scale) MUL_MAT(v, kq) PERMUTE CONT of
  * llm_build_kqv (src/llama.cpp:10062-10148) for a multi-token batch. q = the ROTATED queries [n_tokens][n_head*head_dim] f32, the caches
  * already hold the batch; every query attends cells [0, n_kv) with its row of the additive F32 KQ_mask [n_kv per row, mask_stride floats
- * apart] (any mask the reference builds, not just causal). */
+ * apart] (any mask the reference builds, not just causal; the lowest finite value of the mask's type hides like -inf where anything else is visible). Cells
+ * behind n_kv may hold anything. */
 PM355_API int pm355_attn_prefill_masked(const float * q, const void * k_cache, const void * v_cache, const float * mask, int64_t mask_stride,
                                         float * out, int n_tokens, int n_head, int n_head_kv, int head_dim, int n_ctx, int n_kv,
                                         float kq_scale, pm355_stream_t stream);
@@ -509,7 +510,8 @@ PM355_API pm355_model * pm355_model_new_stack(const pm355_stack_desc * d);
  * pm355_model_finalize_pool: cache for n_seq open sequences that hold at most pool_tokens tokens together (each rounded up to whole pages; layer windows: one slab of
  * n_ctx cells per sequence instead) and scratch for max_tokens tokens at once (longer batches run in pieces).
  * pm355_model_batch: one step over the entries - prompt portions of any length next to single decoded tokens - all of them in one pass where the architecture has a
- * batched step (layer-described models). d_logits: f32 [wanted rows][n_vocab] in the order of entries and of `want`; d_argmax: int32 per wanted row (greedy token,
+ * batched step (layer-described models), in passes of portions of similar length for layer windows (a portion keeps the precision that it has alone; head_dim 64 / 128, n_ctx % 32 == 0, else
+ * one after another). d_logits: f32 [wanted rows][n_vocab] in the order of entries and of `want`; d_argmax: int32 per wanted row (greedy token,
  * first maximum); either may be NULL. tokens: host pointer; NULL = one token, the sequence's last greedy token, taken on the device. Asynchronous; the host arrays may
  * be reused on return. Errors are detected before anything is changed: PM355_E_NOMEM when the pages do not suffice. */
 typedef struct { int32_t seq, n_tokens; const int32_t * tokens; int32_t n_want; const int32_t * want; } pm355_batch_entry;
@@ -576,8 +578,8 @@ PM355_API int pm355_model_decode_seq(pm355_model * m, int seq, const int32_t * d
                                      float * d_x_out, float * d_logits, int32_t * d_argmax, pm355_stream_t stream);
 PM355_API int pm355_model_n_embd(const pm355_model * m);
 PM355_API int pm355_model_n_seq(const pm355_model * m);          /* KV slabs the window was finalized for (pm355_model_finalize_seqs) */
-/* Launch geometry of the prompt GEMM (pm355_mul_mat_q_mfma and friends) for n_row_tiles tiles of 256 weight rows (pair launches: 128 rows of each matrix) x
- * n_tokens x K on a device of n_cus CUs in 8 XCDs - host arithmetic only, no device needed (the reference's counterpart is the stream-k / tile choice of
+/* Launch geometry of the prompt GEMM (pm355_mul_mat_q_mfma and friends) for n_row_tiles tiles of weight rows (pair launches: half of a tile of each matrix) x
+ * n_tokens x K. A tile is 256 rows; 128 rows up to 128 tokens where the launch then has at most n_cus tiles; geometry on a device of n_cus CUs in 8 XCDs - host arithmetic only, no device needed (the reference's counterpart is the stream-k / tile choice of
  * ggml-cuda/mmq.cuh:2583-2700). out5 = {tokens per tile (64 / 128 / 256), token tiles, K slices of a split tile, whole-tile slots per XCD in front of the split
  * ones (0: every tile is split, or none when slices == 1), workgroups launched}. allow_tail_split = 0: the uniform split only. */
 PM355_API int pm355_gemm_plan(int64_t n_row_tiles, int64_t K, int64_t n_tokens, int n_cus, int allow_tail_split, int32_t * out5);

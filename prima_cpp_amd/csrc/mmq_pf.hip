@@ -512,8 +512,8 @@ __device__ __forceinline__ void mid_body(const PfP & p, const PfJob & jb, const 
     const uint32_t boff0 = (uint32_t) (kk * HB + r * 128 + ((h ^ ((r >> 1) & 7)) << 4));
     const uint32_t aoff = (uint32_t) (r * 16 + 8 * h);
 
-    // Requests return in order, and weights come from memory, activations mostly from L2: the waves of the first half request the weights, MID_AHEAD steps ahead, those of the
-    // second half the activations, one step ahead (with both behind one counter every weight was waited for after two steps)
+    // Requests return in order, and weights come from memory, activations mostly from L2: the waves of the first half request the weights, AHEAD steps ahead, those of the
+    // second half the activations, two steps ahead (with both behind one counter every weight was waited for after two steps)
     // part u (0..3) of step s's requests
     auto issue_A = [&](int s, uint32_t sl, bool even, int u) __attribute__((always_inline)) {
         const uint32_t sc = (uint32_t) min(s, nsteps - 1);
@@ -541,7 +541,7 @@ __device__ __forceinline__ void mid_body(const PfP & p, const PfJob & jb, const 
 #pragma unroll
         for (int v = 0; v < NH; ++v) { const int q = NH * u + v; dma16(Xg, xsrc[q] + sc * 256u, lds0 + bb + (q / NT) * HB + (g + 4 * (q % NT)) * 1024); }
     };
-    // end of an even / odd step: the next one's weights (all but those of the MID_AHEAD - 1 steps behind it) and activations are there, this wave's LDS reads are through
+    // end of an even / odd step: the next one's weights (all but those of the AHEAD - 1 steps behind it) and activations are there, this wave's LDS reads are through
     auto settle = [&](bool even) __attribute__((always_inline)) {
         constexpr int W = SLOT / 1024, E = TYPE == PM_Q5_K || TYPE == PM_Q6_K ? 2 : 1;
         if (kk) mid_wait<2 * NT>();
@@ -874,7 +874,9 @@ int pm_launch_gemm_pf_ex(const pm_gemm_pf_job * jobs, int njobs, const void * xh
     const int cus = pm_device_cus();
     // mid_body for up to 128 tokens where its 128-row tiles are one round of workgroups: there a launch is its fixed costs and its K split. us, pf_body / mid_body, Q4_K: 4096 x 4096
     // 101 tokens 28.9 / 22.0, 4096 x 14336 50.4 / 35.7, 32768 x 4096 (256 tiles) 128 tokens 66 / 52. With more tiles the 256-row tiles' fewer bytes per product win: 40960 x 4096 (320)
-    // 101 tokens 65.8 / 70, 128256 x 4096 (Q6_K) 209 / 235
+    // 101 tokens 65.8 / 70, 128256 x 4096 (Q6_K) 209 / 235. Beyond 128 tokens mid_body is still the faster one (4096 x 4096: 256 tokens 55.8 / 26.6, 512 60 / 36) and not taken for its
+    // results: it adds the halves of every 128 k in another order, and tokens decoded behind such a prompt then differ from those behind pf_body's by up to 3 % of their logits (eight layers of
+    // the 8B shape; their 8-bit roundings turn), although neither is nearer to 64 bits
     const int mid_nt = T <= 64 ? 2 : 4;
     long mid_wgs = 0;
     for (int j = 0; j < njobs && !(pair && j); ++j) mid_wgs += (jobs[j].N + (pair ? 63 : 127)) / (pair ? 64 : 128);

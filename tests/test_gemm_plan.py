@@ -75,6 +75,17 @@ def test_layer_shapes_of_the_baseline_models():
     assert p["tile_tokens"] == 64 and p["nt_t"] == 1 and p["S"] == 8
 
 
+@pytest.mark.parametrize("rows,K,T,S", [((4096, 1024, 1024), 4096, 101, 4), ((4096,), 4096, 101, 4), ((4096,), 14336, 101, 8), ((14336, 14336), 4096, 101, 1), ((8192,), 8192, 64, 4), ((132,), 512, 33, 1)])
+def test_launches_of_128_row_tiles(rows, K, T, S):
+    """Up to 128 tokens, launches with at most one 128-row tile per CU are planned on those tiles (of every matrix of the launch; a pair launch: 64 rows of each): Llama-3-8B's at 101 tokens"""
+    tiles = -(-rows[0] // 64) if rows == (14336, 14336) else sum(-(-n // 128) for n in rows)
+    assert tiles <= CUS
+    p = plan(tiles, K, T)
+    assert p["tile_tokens"] == (64 if T <= 64 else 128) and p["nt_t"] == 1 and p["S"] == S and p["full"] == 0
+    cov = coverage(tiles, p)
+    assert len(cov) == tiles and all(sorted(sl) == [(k, S) for k in range(S)] for sl in cov.values())
+
+
 def test_bad_arguments_are_refused():
     lib = L.load()
     lib.pm355_gemm_plan.restype = C.c_int

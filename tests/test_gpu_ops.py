@@ -795,8 +795,9 @@ def test_prompt_gemm_jobs_one_launch(P, oracle, types, T):
         assert nm < 1e-6, (t, nm)
 
 
-# token tiles of 64 and 128 tokens and the first counts beyond, rows that end inside a 128-row tile and inside a wave's 32, fewer steps of K than are requested ahead, K slices (8 super-blocks and
-# more), for Q8_0 a last step that is half a super-block (in a slice and without one); 256 tiles, the last launch of one round, and 258, which the 256-row tiles take
+# token tiles of 64 and 128 tokens, rows that end inside a 128-row tile and inside a wave's 32, fewer steps of K than are requested ahead, K slices (8 super-blocks and more), for Q8_0 a last
+# step that is half a super-block (in a slice and without one); 256 tiles, the last launch of one round, and 258, which the 256-row tiles take, as they take the first counts beyond 128 tokens
+# (129 and 257: the general tiles against themselves, other slices of K)
 @pytest.mark.parametrize("t", QUANT_TYPES)
 @pytest.mark.parametrize("K,N,T", [(512, 132, 33), (768, 260, 64), (512, 4, 65), (4096, 388, 128), (2304, 128, 129), (1024, 1028, 257), (512, 32768, 40), (512, 33024, 40)])
 def test_prompt_gemm_tiles_of_128_rows(P, oracle, t, K, N, T):
