@@ -416,7 +416,7 @@ size_t rows_lds(int rm, int tp, int K) { return (size_t) 8 * rm * 1024 + (size_t
 template <int RM, int TP> int launch_rows(const SmallP & p, int N, hipStream_t st) {
     const int tiles = N / (8 * RM), cus = pm_device_cus();
     const size_t lds = rows_lds(RM, TP, p.K);
-    const int per = TP == 0 && RM == 2 || lds > 80 * 1024 ? 1 : 2, grid = tiles < per * cus ? tiles : per * cus;
+    const int per = (TP == 0 && RM == 2) || lds > 80 * 1024 ? 1 : 2, grid = tiles < per * cus ? tiles : per * cus;
     pm_allow_big_lds((const void *) dense_rows_kernel<RM, TP>, lds);
     hipLaunchKernelGGL((dense_rows_kernel<RM, TP>), dim3(grid), dim3(512), lds, st, p, tiles);
     return 0;
@@ -446,9 +446,10 @@ template <typename T> int launch_type(const pm_dense_args & a, const SmallP & p,
     }
     // One matrix, up to 8 tokens: the workgroups that stay, with the activations in LDS where they fit (150 KB: 16 bytes per value for 5..8 tokens, 8 for less), from memory above that
     // (5 tokens of 4096 values, 14336 rows: 22.7 us against 27 from memory). One token of shorter rows stays with a workgroup per tile, which has less to do before its first and after
-    // its last weight (32000 x 2048: 23.6 us against 25.1, 4096 x 5120: 10.2 / 10.9; the other way round from 6144 values: 5120 x 6144 16.8 / 15.2, 2048 x 8192 10.3 / 9.0)
+    // its last weight (32000 x 2048: 23.6 us against 25.1, 4096 x 5120: 10.2 / 10.9; the other way round from 6144 values: 5120 x 6144 16.8 / 15.2, 2048 x 8192 10.3 / 9.0). DMA and buffer loads
+    // of 16 bytes want operands that start on 16 bytes
     if constexpr (sizeof(T) == 2)
-        if (a.T <= 8 && !a.group && !a.merge && (a.T > 1 || a.K >= 6144) && (int64_t) p.T * p.lda < (1 << 28) && a.K < (1 << 26)) {
+        if (a.T <= 8 && (((uintptr_t) p.W | (uintptr_t) p.act) & 15) == 0 && !a.group && !a.merge && (a.T > 1 || a.K >= 6144) && (int64_t) p.T * p.lda < (1 << 28) && a.K < (1 << 26)) {
             const int tp = a.T <= 4 ? 4 : 8;
             if (rows_lds(rm, tp, a.K) > 150 * 1024) return launch_rows<2, 0>(p, N, st);
             if (tp == 4) return rm == 1 ? launch_rows<1, 4>(p, N, st) : launch_rows<2, 4>(p, N, st);

@@ -139,6 +139,18 @@ def test_dense_mul_mat_few_tokens_over_many_rows(T, K, n_store):
         assert (y[:, n_store:] == 7.0).all()
 
 
+@pytest.mark.parametrize("T,K,off_x,off_w", [(3, 1024, 4, 0), (8, 4096, 1, 0), (1, 8192, 0, 4), (5, 9216, 2, 2)])
+def test_dense_mul_mat_of_operands_that_do_not_start_on_16_bytes(T, K, off_x, off_w):
+    import prima_cpp_amd.ops as O
+    g = torch.Generator(device="cuda").manual_seed(T + K)
+    w = (torch.randn(192 * K + 8, generator=g, device="cuda") / K ** 0.5).bfloat16()[off_w:off_w + 192 * K].view(192, K)
+    x = torch.randn(T * (K + 64) + 8, generator=g, device="cuda").bfloat16()[off_x:off_x + T * (K + 64)].view(T, K + 64)[:, :K]
+    y = torch.zeros(T, 192, device="cuda")
+    O.dense_mul_mat(w, x, y)
+    want = x.double() @ w.double().T
+    assert ((y.double() - want).abs() <= 2e-6 * K ** 0.5 * (1 + want.abs())).all()
+
+
 @pytest.mark.parametrize("tiles", [(2048, 2048), (300, 4096)])
 def test_dense_mul_mat_large_tiles(tiles):
     """shapes whose grid takes the 256 x 256 tiles, ragged in both directions"""
