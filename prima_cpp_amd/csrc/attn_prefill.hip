@@ -222,7 +222,8 @@ __global__ __launch_bounds__(256, 2) void attn_rowmajor_kernel(PfP p) {
 // Bound by the LDS reads of the fragments (32 queries per wave: 32 KiB per 64 keys and wave at ~80 bytes per cycle and CU, about the time of the 32 matrix instructions) and the
 // exponentials beside them. Against the two-pass form with 4 waves x 32 queries, 32-key tiles through registers: 6001 tokens x 32 heads 870 -> 393 us (752 TFLOP/s), 512 x 64 behind
 // 1024 cached cells 102 -> 38, 101 x 32 behind 300 29.8 -> 11.7, 2048 x 32 144 -> 55.
-template <int DH, int QW, int KS, bool MASK>
+// PLAIN: caches that do not start on 16 bytes, by loads and LDS stores instead of DMA
+template <int DH, int QW, int KS, bool MASK, bool PLAIN = false>
 __global__ __launch_bounds__(512, 2) void attn_prompt_kernel(PfP p) {
     constexpr int KW = 8 / QW, KT = KS / KW, ST = KT / 32;            // keys per wave and stage, 32-key score tiles
     constexpr int KK = DH / 16, DT = DH / 32, CK = DH / 8, CV = KS / 8;      // k-steps of a score tile, output tiles, 16-byte chunks per K row / V^T row
@@ -257,19 +258,23 @@ __global__ __launch_bounds__(512, 2) void attn_prompt_kernel(PfP p) {
     const int seen = MASK ? p.n_kv : w_last + 1;
 
     const uint32_t lds0 = (uint32_t) (uintptr_t) (__attribute__((address_space(3))) char *) smem;
+    auto bring = [&](const char * base, uint32_t off, int to) __attribute__((always_inline)) {
+        if constexpr (PLAIN) { u32x4 v; __builtin_memcpy(&v, base + off, 16); *(u32x4 *) (smem + to + lane * 16) = v; }
+        else pm_dma16(base, off, lds0 + to);
+    };
     auto request = [&](int it, int stage) __attribute__((always_inline)) {
         const char * kb = (const char *) (kc + (long) it * KS * krow), * vb = (const char *) vc;
         const int key0 = it * KS, kmax = p.n_ctx - 1 - key0, vmax = p.n_ctx - 8 - key0;          // (cells behind the cache: its last ones, masked)
 #pragma unroll
         for (int i = 0; i < KS * DH * 2 / 8192; ++i) {
             const int o = (wave + i * 8) * 64 + lane, row = o / CK, ch = o % CK;
-            pm_dma16(kb, (uint32_t) min(row, kmax) * (uint32_t) (krow * 2) + (uint32_t) (ch ^ (CK == 8 ? (row >> 1) & 7 : row & 15)) * 16u, lds0 + stage * STAGE + (wave + i * 8) * 1024);
+            bring(kb, (uint32_t) min(row, kmax) * (uint32_t) (krow * 2) + (uint32_t) (ch ^ (CK == 8 ? (row >> 1) & 7 : row & 15)) * 16u, stage * STAGE + (wave + i * 8) * 1024);
         }
 #pragma unroll
         for (int i = 0; i < KS * DH * 2 / 8192; ++i) {
             const int o = (wave + i * 8) * 64 + lane, row = o / CV, ch = o % CV;
             const int key = key0 + min((ch ^ (CV == 8 ? (row >> 1) & 7 : row & 15)) * 8, vmax);
-            pm_dma16(vb, (uint32_t) row * (uint32_t) (p.n_ctx * 2) + (uint32_t) key * 2u, lds0 + stage * STAGE + KS * DH * 2 + (wave + i * 8) * 1024);
+            bring(vb, (uint32_t) row * (uint32_t) (p.n_ctx * 2) + (uint32_t) key * 2u, stage * STAGE + KS * DH * 2 + (wave + i * 8) * 1024);
         }
     };
     request(0, 0);
@@ -433,11 +438,11 @@ __global__ __launch_bounds__(512, 2) void attn_prompt_kernel(PfP p) {
     }
 }
 
-template <int DH, int QW, int KS, bool MASK> void launch_prompt(PfP p, hipStream_t st) {
+template <int DH, int QW, int KS, bool MASK, bool PLAIN = false> void launch_prompt(PfP p, hipStream_t st) {
     if (!p.tiles) p.n_tiles = (p.T + QW * 32 - 1) / (QW * 32);
     constexpr size_t stages = 2 * (size_t) KS * DH * 4, ex = (size_t) 8 * 32 * (DH + 4) * 4 + 8 * 32 * 2 * 4, lds = stages > ex ? stages : ex;
-    pm_allow_big_lds((const void *) attn_prompt_kernel<DH, QW, KS, MASK>, lds);
-    hipLaunchKernelGGL((attn_prompt_kernel<DH, QW, KS, MASK>), dim3(p.n_tiles * p.H), dim3(512), lds, st, p);
+    pm_allow_big_lds((const void *) attn_prompt_kernel<DH, QW, KS, MASK, PLAIN>, lds);
+    hipLaunchKernelGGL((attn_prompt_kernel<DH, QW, KS, MASK, PLAIN>), dim3(p.n_tiles * p.H), dim3(512), lds, st, p);
 }
 // Which tile: a CU holds one workgroup. 256 queries share a stage where that still makes two rounds of workgroups (2048 tokens x 64 heads: 102 us, 110 with 128 queries; x 32 heads
 // = one round whose longest tile decides: 80 against 57); 128 queries where they make one (512 x 64 behind 1024 cached: 38 against 50 with 64); below that 64 queries with four key
@@ -447,7 +452,8 @@ int tile_of(int n_tok, int H) {
     return (n_tok + 255) / 256 * H >= 2 * cus ? 256 : (n_tok + 127) / 128 * H >= cus ? 128 : 64;
 }
 template <int DH, bool MASK> void launch_prompt_dh(const PfP & p, int tile_q, hipStream_t st) {
-    if (tile_q == 256) launch_prompt<DH, 8, 64, MASK>(p, st);
+    if (((uintptr_t) p.kc | (uintptr_t) p.vc) & 15) launch_prompt<DH, 2, 128, MASK, true>(p, st);
+    else if (tile_q == 256) launch_prompt<DH, 8, 64, MASK>(p, st);
     else if (tile_q == 128) launch_prompt<DH, 4, 128, MASK>(p, st);
     else launch_prompt<DH, 2, 128, MASK>(p, st);
 }
@@ -464,7 +470,7 @@ int pm_launch_attn_prefill(const float * q, const void * kc, const void * vc, co
     if (mask && (n_kv < 1 || n_kv > n_ctx || n_kv % 4 || mask_stride % 4)) return -1;
     if ((v_rowmajor || mask_f16) && !mask) return -1;                 // the flash-attention form exists in ggml-graph mode only
     PfP p = {q, (const uint16_t *) kc, (const uint16_t *) vc, pos0, seq, seq_stride, out, n_tok, H, Hkv, n_ctx, scale, mask, mask_stride, n_kv, mask_f16 ? 1 : 0, (_Float16 *) out_f16, tiles, n_tiles};
-    if (tiles && (mask || n_tiles < 1)) return -1;
+    if (tiles && (mask || n_tiles < 1 || (((uintptr_t) kc | (uintptr_t) vc) & 15))) return -1;
     if (!tiles) tile_q = tile_of(n_tok, H);
     if (v_rowmajor) {
         if (out_f16 || seq) return -1;

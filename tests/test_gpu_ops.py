@@ -532,6 +532,29 @@ def test_attn_prefill_does_not_look_behind_the_attended_cells(P, H, Hkv, dh, T, 
     assert all(torch.equal(o, w) for o, w in zip(outs[len(outs) // 2:], outs))
 
 
+@pytest.mark.parametrize("off", [1, 4])
+@pytest.mark.parametrize("H,Hkv,dh,T,past,mask", [(8, 2, 128, 40, 60, False), (8, 4, 64, 70, 130, False), (8, 2, 64, 33, 0, True), (8, 2, 128, 130, 0, True)])
+def test_attn_prefill_of_caches_that_do_not_start_on_16_bytes(P, H, Hkv, dh, T, past, mask, off):
+    """views that begin 2 or 8 bytes into a buffer: the same bits as caches that start on 16"""
+    torch = P.torch
+    n = past + T
+    n_ctx = -(-n // 32) * 32
+    g = torch.Generator(device="cuda").manual_seed(n)
+    q = torch.randn((T, H * dh), generator=g, device="cuda")
+    K, V = (torch.randn(n_ctx * Hkv * dh, generator=g, device="cuda").half() for _ in range(2))
+    outs = []
+    for o in (0, off):
+        k, v = (torch.cat([torch.zeros(o, device="cuda").half(), x])[o:] for x in (K, V))
+        assert k.data_ptr() % 16 == 2 * o
+        if not mask:
+            outs.append(P.attn_prefill(q, k, v, past, H, Hkv, dh, n_ctx, dh ** -0.5))
+            continue
+        n_kv = -(-n // 4) * 4
+        hidden = torch.arange(n_kv, device="cuda")[None] > torch.arange(T, device="cuda")[:, None]
+        outs.append(_masked_attention(P, q, k, v, torch.zeros((T, n_kv), device="cuda").masked_fill_(hidden, -np.inf), n_kv, H, Hkv, dh, n_ctx, dh ** -0.5))
+    assert bool(outs[0].isfinite().all()) and torch.equal(*outs)
+
+
 @pytest.mark.parametrize("scale", [-0.09, 0.0])
 @pytest.mark.parametrize("H,Hkv,dh,T,past", [(8, 2, 128, 40, 60), (64, 8, 64, 300, 12)])
 def test_attn_prefill_scales_that_are_not_positive(P, H, Hkv, dh, T, past, scale):
