@@ -1,4 +1,4 @@
-// mmq_i8.hip — small-batch (up to 32 tokens per pass, 64 per call) quantized mat-mul on the INTEGER matrix cores
+// mmq_i8.hip — small-batch (9..32 tokens per pass, 64 per call; passes of fewer: mmq_rows.hip) quantized mat-mul on the INTEGER matrix cores
 // (v_mfma_i32_32x32x32_i8 / v_mfma_i32_32x32x16_i8). Q4_K, Q5_K, Q6_K weights x Q8_K activations.
 //
 // What it replaces: for 2..64 activation rows the reference runs ggml_compute_forward_mul_mat's vec_dot loop once per (row, token)
@@ -17,7 +17,7 @@
 //   B operand = weights    : lane (r = lane % 32, g)            holds the same k of weight row r
 //   result                 : lane (r, g) holds, for ITS OWN row r, tokens 8 (v / 4) + 4 g + v % 4, v = 0..15
 // so the per-row sub-block scale / min / d of a K-quant are lane-local scalars when the i32 tile is scaled (one v_mad_i32_i24 per result;
-// the instantiation keeps 4 / 8 / 16 result registers for <= 8 / 16 / 32 tokens). An MFMA never crosses a scale group. The min / -32
+// the instantiation keeps 8 / 16 result registers for <= 16 / 32 tokens). An MFMA never crosses a scale group. The min / -32
 // terms are one more MFMA per super-block in F16 (v_mfma_f32_32x32x16_f16: 6-bit mins or int8 scales x 16-value activation sums <= 2032,
 // all exact in F16, f32 accumulation of integers < 2^24 exact).
 //
@@ -36,9 +36,10 @@
 // interleaved pair by pair, so that those waves read adjacent 128-byte pieces of a row at the same time (ffn_down Q6_K: 76 -> 70 us) - and
 // their f32 partial tiles are added in a fixed order through LDS (bitwise reproducible). Multi-job form (MJ): up to 3 matrices of one
 // type and K that share the activations form one virtual row space (wq | wk | wv, ffn_gate | ffn_up): one launch, one fill / drain.
-// Measurements, ablation and what did not help: profiles/r02_small_batch_probe.txt, DESIGN.md section 3.
+// Measurements and what did not help: profiles/r02_small_batch_probe.txt, profiles/r04_small_batch.txt, profiles/r06_small_batch.txt.
 #include "pm355_device.h"
 #include "pm355_kernels.h"
+#include "pm355_mmq_rows.h"
 #include <mutex>
 
 namespace {
@@ -47,6 +48,7 @@ typedef int      i32x16 __attribute__((ext_vector_type(16)));
 typedef float    f32x16 __attribute__((ext_vector_type(16)));
 typedef _Float16 f16x8  __attribute__((ext_vector_type(8)));
 
+constexpr int ROWS_MAX = 8;             // passes of up to so many tokens: mmq_rows.hip
 constexpr int BLOCK = 512, NWAVE = 8;
 constexpr int PITCH = 144;            // LDS bytes per row of a 128-byte stream tile: 16 consecutive rows -> 16 distinct 16-byte bank slots
 constexpr int PITCH_H = 48;           // same for the 2 x 16-byte per-row header / scale tile
@@ -104,11 +106,10 @@ template <> struct Rows<true> {           // several matrices: a lane's rows may
 // the NEXT step's whole weight tile (ISA: vmcnt(14) where 31 loads were in flight), i.e. the prefetch overlapped half a step. Buffer loads
 // instead: unconditional instructions, the lanes without a token carry an out-of-range offset, return 0 and touch no memory.
 //
-// A 32 x 32 product has 32 token rows; up to 8 (16) tokens would leave three quarters (half) of the operand's lanes empty. They carry OTHER sub-blocks instead: operand lane
-// r = R q + t, R = 2 NV rows per sub-block, holds token t's bytes of sub-block P i + q (P = 16 / NV sub-blocks per register). The product with the weights of sub-block P i + q is
-// right in the rows R q .. R q + R - 1, i.e. in the result registers NV q .. NV q + NV - 1, and nobody reads the others. One load brings what P loads of half-empty lanes did: 2 (4)
-// loads per super-block instead of 8 and as many registers less. At 8 tokens these loads were 10 of the 60 us of a 57344 x 8192 Q4_K launch (the vector memory path is paid per
-// instruction): 57.4 -> 51.6 us on weights out of memory.
+// A 32 x 32 product has 32 token rows; up to 16 tokens would leave half of the operand's lanes empty. They carry OTHER sub-blocks instead: operand lane r = R q + t, R = 2 NV rows per
+// sub-block, holds token t's bytes of sub-block P i + q (P = 16 / NV sub-blocks per register). The product with the weights of sub-block P i + q is right in the rows R q .. R q + R - 1,
+// i.e. in the result registers NV q .. NV q + NV - 1, and nobody reads the others. One load brings what P loads of half-empty lanes did: 4 loads per super-block instead of 8 and as many
+// registers less (the vector memory path is paid per instruction).
 struct ActSrc {
     __amdgpu_buffer_rsrc_t rx, rb; uint32_t xo, bo;        // xo / bo: this lane's byte offset into the operand-ordered activations / the group-sum table (or out of range)
     // sub-block s of super-block sb: lane (t, g) gets the 16 bytes k = 32 s + 16 g .. + 15 of token t (one coalesced kilobyte per wave and 32 tokens)
@@ -409,11 +410,10 @@ template <> struct MT<PM_Q8_0> {
     }
 };
 
-// ABL (measurement only, PM355_MMQ_ABL): 1 = no activation loads in the loop, 2 = no weight loads in the loop, 4 = no MFMA / VALU work
 // the work of workgroup w of G on the launch p (its own grid, or one part of a two-part launch)
 // EPI: the wq | wk | wv epilogue (MmqP::e_*) is compiled in - instantiations of their own: carried by every kernel as a run-time switch it cost the launches
 // that never use it 2-6 us per layer (Qwen2.5-72B, NEOX rope: 236 -> 242 us at 8 tokens)
-template <int TYPE, int NV, int ABL, bool MJ, bool EPI = false>  // NV result registers per lane in use: 4 (<= 8 tokens), 8 (<= 16), 16 (<= 32)
+template <int TYPE, int NV, bool MJ, bool EPI = false>  // NV result registers per lane in use: 8 (<= 16 tokens), 16 (<= 32)
 __device__ __forceinline__ void mmq_i8_body(const MmqP & p, const int w, const int G, uint8_t * smem) {
     typedef MT<TYPE> M;
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;   // (a scalar: the K slice, the loop counters and the buffer loads' scalar offsets derive from it)
@@ -445,10 +445,9 @@ __device__ __forceinline__ void mmq_i8_body(const MmqP & p, const int w, const i
     xs.xo = act ? (uint32_t) (tq * 1024 + (32 * g + tt + p.t_off) * 16) : 0x80000000u;
     xs.bo = Q80 ? (uint32_t) (16 * lane) : act_b ? (uint32_t) ((lane + p.t_off) * 16) : 0x80000000u;   // (Q8_0: lane l carries 16 bytes of the step's [8 blocks][32 slots] activation scales)
     Rows<MJ> rw;
-    // (measured and rejected, again with the registers that the packed activations free: TWO weight tiles in flight per wave, the activations of the next step in front of them -
-    //  57344 x 8192 Q4_K at 8 tokens 53.0 -> 55.1 us, Q6_K 98.0 -> 102.4; and two workgroups that share a row group's K where 128 row groups leave half the chip idle - 4096 x 14336
-    //  Q6_K 24.7 -> 22.8 us, but Q4_K 14.3 -> 16.3 and 4096 x 8192 11.6 -> 13.1: the exchange costs what the second half of the chip saves. What Q6_K launches lose is memory traffic:
-    //  1.36 x the weights' bytes, the scale and d lines of a row tail are fetched again for every step)
+    // (measured and rejected at 8 tokens, when this kernel still took them: TWO weight tiles in flight per wave - 57344 x 8192 Q4_K 53.0 -> 55.1 us, Q6_K 98.0 -> 102.4; two workgroups that
+    //  share a row group's K where 128 row groups leave half the chip idle - 4096 x 14336 Q6_K 24.7 -> 22.8 us, but Q4_K 14.3 -> 16.3: the exchange costs what the second half of the chip
+    //  saves. What Q6_K launches lose is memory traffic: 1.36 x the weights' bytes, the scale and d lines of a row tail are fetched again for every step)
     typename M::B R;
     typename M::template A<NV> A0 = {}, A1 = {};                 // (inactive token lanes keep these zeros)
     // a step's weight tile goes out in FOUR parts. Issued in one burst (13 x 1 KiB per wave, 100 KB per CU) the wave sat in the issue itself until the
@@ -484,7 +483,6 @@ __device__ __forceinline__ void mmq_i8_body(const MmqP & p, const int w, const i
         rw.lm = ~0u;
         issue_b(R, pb);
         M::template issue_a<NV>(A0, xs, 2 * pb);
-        if constexpr (ABL & 1) M::template issue_a<NV>(A1, xs, 2 * pb);
     };
     if (rgi < nrg && pb < pe) first(rgi);                         // ... including the staging of the scale table:
     if constexpr (!Q80) {
@@ -517,23 +515,21 @@ __device__ __forceinline__ void mmq_i8_body(const MmqP & p, const int w, const i
                 // Issue order is the design (VMEM returns in order): the compiler's schedulers must not sink the prefetches towards
                 // their uses - no conditional code in the step (an odd tail super-block is computed on clamped data with the all-zero
                 // scale row) and scheduling barriers around the issue points.
-                if constexpr (!(ABL & 1)) M::template issue_a<NV>(A1, xs, sb1);
+                M::template issue_a<NV>(A1, xs, sb1);
                 const int prn = min(pr + pstep, pe - pstep);             // the tile these registers take next
                 rw.lm = pr + pstep < pe ? ~0u : 0u;                      // (past the wave's last step: a request for nothing)
                 __builtin_amdgcn_sched_barrier(0);
                 // (the 32-token Q6_K form has no registers for it - 404 B of spills, 88 -> 205 us: its tile still goes out in one burst)
-                constexpr bool SPREAD = !(TYPE == PM_Q6_K && NV == 16) && !(ABL & 4);
-                if constexpr (!SPREAD && !(ABL & 2)) { issue_b(Rc, prn); __builtin_amdgcn_sched_barrier(0); }
+                constexpr bool SPREAD = !(TYPE == PM_Q6_K && NV == 16);
+                if constexpr (!SPREAD) { issue_b(Rc, prn); __builtin_amdgcn_sched_barrier(0); }
                 auto part = [&](int n) __attribute__((always_inline)) {   // next tile, part n: unconditional, pinned between the quarters
-                    if constexpr (SPREAD && !(ABL & 2)) { __builtin_amdgcn_sched_barrier(0); issue_b_part(Rc, prn, n); __builtin_amdgcn_sched_barrier(0); }
+                    if constexpr (SPREAD) { __builtin_amdgcn_sched_barrier(0); issue_b_part(Rc, prn, n); __builtin_amdgcn_sched_barrier(0); }
                 };
-                if constexpr (!(ABL & 4)) M::template compute<NV>(A0, L, 0, r, g, dTl + sb0 * 32, p.t_off, out, part);
-                else { for (int s_ = 0; s_ < NV / 2; ++s_) asm volatile("" :: "v"(A0.q[s_])); asm volatile("" :: "v"(A0.bs)); asm volatile("" :: "v"(*(const u32x4 *) (L + 16 * lane))); }
+                M::template compute<NV>(A0, L, 0, r, g, dTl + sb0 * 32, p.t_off, out, part);
                 __builtin_amdgcn_sched_barrier(0);
-                if constexpr (!(ABL & 1)) M::template issue_a<NV>(A0, xs, min(2 * prn, nsb - 1));
+                M::template issue_a<NV>(A0, xs, min(2 * prn, nsb - 1));
                 __builtin_amdgcn_sched_barrier(0);
-                if constexpr (!(ABL & 4)) M::template compute<NV>(A1, L, 1, r, g, dTl + (2 * pr + 1 < nsb ? sb1 : nsb) * 32, p.t_off, out, [](int) {});
-                else { for (int s_ = 0; s_ < NV / 2; ++s_) asm volatile("" :: "v"(A1.q[s_])); asm volatile("" :: "v"(A1.bs)); asm volatile("" :: "v"(*(const u32x4 *) (L + 16 * lane + 1024))); }
+                M::template compute<NV>(A1, L, 1, r, g, dTl + (2 * pr + 1 < nsb ? sb1 : nsb) * 32, p.t_off, out, [](int) {});
                 __builtin_amdgcn_sched_barrier(0);
             };
             for (int pr = pb; pr < pe; pr += pstep) step(R, pr);
@@ -589,10 +585,10 @@ __device__ __forceinline__ void mmq_i8_body(const MmqP & p, const int w, const i
     }
 }
 
-template <int TYPE, int NV, int ABL = 0, bool MJ = false, bool EPI = false>
+template <int TYPE, int NV, bool MJ = false, bool EPI = false>
 __global__ __launch_bounds__(BLOCK, 2) void mmq_i8_kernel(MmqP p) {
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
-    mmq_i8_body<TYPE, NV, ABL, MJ, EPI>(p, (int) blockIdx.x, (int) gridDim.x, smem);
+    mmq_i8_body<TYPE, NV, MJ, EPI>(p, (int) blockIdx.x, (int) gridDim.x, smem);
 }
 
 // Two launches that share the activations as ONE grid: workgroups [0, ga) are the multi-job launch `a` (wq | wk, type TA), the rest the single matrix `b` of
@@ -602,8 +598,8 @@ struct MmqP2 { MmqP a, b; int ga; };
 template <int TA, int TB, int NV, bool EPI = false>
 __global__ __launch_bounds__(BLOCK, 2) void mmq_i8_dual_kernel(MmqP2 pp) {
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
-    if ((int) blockIdx.x < pp.ga) mmq_i8_body<TA, NV, 0, true, EPI>(pp.a, (int) blockIdx.x, pp.ga, smem);
-    else mmq_i8_body<TB, NV, 0, TB == PM_Q6_K, EPI>(pp.b, (int) blockIdx.x - pp.ga, (int) gridDim.x - pp.ga, smem);
+    if ((int) blockIdx.x < pp.ga) mmq_i8_body<TA, NV, true, EPI>(pp.a, (int) blockIdx.x, pp.ga, smem);
+    else mmq_i8_body<TB, NV, TB == PM_Q6_K, EPI>(pp.b, (int) blockIdx.x - pp.ga, (int) gridDim.x - pp.ga, smem);
 }
 
 // prologue: per super-block, the activation group sums as F16 in A-operand order and the transposed activation scales
@@ -756,6 +752,14 @@ int launch_q80(const void * W, const void * xq, const float * x_f32, float * Y, 
     for (int t0 = 0; t0 < T; t0 += tmax) {
         const int tn = T - t0 < tmax ? T - t0 : tmax;
         uint8_t * tab = base + (t0 / 32) * (qtab + dtab);
+        if (tn <= ROWS_MAX) {
+            RowsP q = {};
+            q.job[0] = {(const uint8_t *) W, Y + (size_t) t0 * N, bias, resid ? resid + (size_t) t0 * N : nullptr, N};
+            q.njobs = 1; q.K = K; q.T = tn; q.t_off = t0 % 32; q.qT = tab; q.dT = (const float *) (tab + qtab);
+            const int ty = PM_Q8_0;
+            if (pm_launch_mmq_rows(q, &ty, st)) return -3;
+            continue;
+        }
         MmqP p = {};
         p.t_off = t0 % 32;
         p.W = (const uint8_t *) W; p.row_stride = (long) pm_weight_row_stride(PM_Q8_0, K); p.N = N; p.K = K; p.T = tn;
@@ -766,7 +770,7 @@ int launch_q80(const void * W, const void * xq, const float * x_f32, float * Y, 
             pm_allow_big_lds((const void *) kern, 150 * 1024);
             hipLaunchKernelGGL(kern, dim3(grid), dim3(BLOCK), lds, st, p);
         };
-        if (tn <= 8) go(mmq_i8_kernel<PM_Q8_0, 4>); else go(mmq_i8_kernel<PM_Q8_0, 8>);
+        go(mmq_i8_kernel<PM_Q8_0, 8>);
     }
     return 0;
 }
@@ -835,6 +839,13 @@ int pm_launch_mmq_i8(int type, const void * W, const void * xq, const float * x_
     for (int t0 = 0, c = 0; t0 < T; t0 += tmax, ++c) {
         const int tn = T - t0 < tmax ? T - t0 : tmax;
         uint8_t * bsT = sc->p + (t0 / 32) * tab; float * dT = (float *) (bsT + (size_t) nsb * 1024);    // tables are per 32 tokens
+        if (tn <= ROWS_MAX) {
+            RowsP q = {};
+            q.job[0] = {(const uint8_t *) W, Y + (size_t) t0 * N, bias, resid ? resid + (size_t) t0 * N : nullptr, N};
+            q.njobs = 1; q.K = K; q.T = tn; q.t_off = t0 % 32; q.qT = sc->p + scr_q_off(K) + (size_t) (t0 / 32) * nsb * 8192; q.bsT = bsT; q.dT = dT;
+            if (pm_launch_mmq_rows(q, &type, st)) return -3;
+            continue;
+        }
         const uint8_t * xc = (const uint8_t *) xq + (size_t) t0 * xrow;
         MmqP p = {};
         p.t_off = t0 % 32;
@@ -846,26 +857,22 @@ int pm_launch_mmq_i8(int type, const void * W, const void * xq, const float * x_
             pm_allow_big_lds((const void *) kern, 150 * 1024);
             hipLaunchKernelGGL(kern, dim3(grid), dim3(BLOCK), lds, st, p);
         };
-#ifdef PM_MMQ_ABLATE      // measurement build (profiles/r02_small_batch_probe.txt): PM355_MMQ_ABL = 1 no activation loads | 2 no weight loads | 4 no compute
-        static const int abl = [] { const char * e = getenv("PM355_MMQ_ABL"); return e ? atoi(e) : 0; }();
-        if (abl && tn <= 8) {
-#define PM_ABL_CASE(T_) switch (abl) { case 1: go(mmq_i8_kernel<T_, 4, 1>); break; case 2: go(mmq_i8_kernel<T_, 4, 2>); break; case 3: go(mmq_i8_kernel<T_, 4, 3>); break; \
-                                       case 4: go(mmq_i8_kernel<T_, 4, 4>); break; case 5: go(mmq_i8_kernel<T_, 4, 5>); break; case 6: go(mmq_i8_kernel<T_, 4, 6>); break; \
-                                       default: go(mmq_i8_kernel<T_, 4, 7>); break; }
-            if (type == PM_Q4_K) PM_ABL_CASE(PM_Q4_K) else PM_ABL_CASE(PM_Q6_K)
-#undef PM_ABL_CASE
-        } else
-#endif
-        if (type == PM_Q4_K) { if (tn <= 8) go(mmq_i8_kernel<PM_Q4_K, 4>); else if (tn <= 16) go(mmq_i8_kernel<PM_Q4_K, 8>); else go(mmq_i8_kernel<PM_Q4_K, 16>); }
-        else if (type == PM_Q5_K) { if (tn <= 8) go(mmq_i8_kernel<PM_Q5_K, 4>); else go(mmq_i8_kernel<PM_Q5_K, 8>); }
-        else if (tn <= 8)    go(mmq_i8_kernel<PM_Q6_K, 4>);
-        else if (tn <= 16)   go(mmq_i8_kernel<PM_Q6_K, 8>);
-        else                 go(mmq_i8_kernel<PM_Q6_K, 16>);
+        if (type == PM_Q4_K) { if (tn <= 16) go(mmq_i8_kernel<PM_Q4_K, 8>); else go(mmq_i8_kernel<PM_Q4_K, 16>); }
+        else if (type == PM_Q5_K) go(mmq_i8_kernel<PM_Q5_K, 8>);
+        else if (tn <= 16) go(mmq_i8_kernel<PM_Q6_K, 8>);
+        else go(mmq_i8_kernel<PM_Q6_K, 16>);
     }
     return 0;
 }
 
 namespace {
+bool fill_epi(RowsP & p, const pm_qkv_epi * e) {
+    if (!e) return true;
+    if (e->neox || e->v_rowmajor || e->dyn || !e->tab || !e->pos || !e->kc || !e->vc || e->dh < 2 || (e->dh & 1) || (e->n_rot & 1)) return false;
+    p.e_on = 1; p.e_tab = e->tab; p.e_pos = e->pos; p.e_seq = e->seq; p.e_seq_stride = e->seq_stride; p.e_kc = (uint16_t *) e->kc; p.e_vc = (uint16_t *) e->vc;
+    p.e_dh = e->dh; p.e_nctx = e->n_ctx; p.e_nrot = e->n_rot; p.e_kvdim = e->Hkv * e->dh; p.e_rows = e->rows;
+    return true;
+}
 // wq | wk | wv epilogue of a launch (MmqP::e_*): NORM-mode rope, transposed F16 V cache, engine mode (cell = position). false: not served
 bool fill_epi(MmqP & p, const pm_qkv_epi * e, int r0, int r1, int r2) {
     if (!e) return true;
@@ -918,13 +925,22 @@ int pm_launch_mmq_i8_multi(int type, int njobs, const void * const * W, const in
     const size_t tab = (size_t) nsb * (1024 + 128);
     for (int t0 = 0, c = 0; t0 < T; t0 += 32, ++c) {                 // passes of 32 tokens, each with its own tables
         const int tn = T - t0 < 32 ? T - t0 : 32;
+        if (tn <= ROWS_MAX) {
+            RowsP q = {};
+            int ty[3];
+            q.njobs = njobs; q.K = K; q.T = tn; q.bsT = sc->p + c * tab; q.dT = (const float *) (q.bsT + (size_t) nsb * 1024); q.qT = sc->p + scr_q_off(K) + (size_t) c * nsb * 8192;
+            for (int j = 0; j < njobs; ++j) { q.job[j] = {(const uint8_t *) W[j], Y[j] + (size_t) t0 * N[j], bias ? bias[j] : nullptr, nullptr, N[j]}; ty[j] = type; }
+            if (!fill_epi(q, epi)) return -5;
+            if (pm_launch_mmq_rows(q, ty, st)) return -3;
+            continue;
+        }
         p.T = tn;
         p.bsT = sc->p + c * tab; p.dT = (const float *) (p.bsT + (size_t) nsb * 1024); p.qT = sc->p + scr_q_off(K) + (size_t) c * nsb * 8192;
         for (int j = 0; j < 3; ++j) { const int jj = j < njobs ? j : njobs - 1; p.yj[j] = Y[jj] + (size_t) t0 * N[jj]; }
-        if (p.e_on && type == PM_Q4_K) { if (tn <= 8) go(mmq_i8_kernel<PM_Q4_K, 4, 0, true, true>); else if (tn <= 16) go(mmq_i8_kernel<PM_Q4_K, 8, 0, true, true>); else go(mmq_i8_kernel<PM_Q4_K, 16, 0, true, true>); }
-        else if (p.e_on)         { if (tn <= 8) go(mmq_i8_kernel<PM_Q6_K, 4, 0, true, true>); else if (tn <= 16) go(mmq_i8_kernel<PM_Q6_K, 8, 0, true, true>); else go(mmq_i8_kernel<PM_Q6_K, 16, 0, true, true>); }
-        else if (type == PM_Q4_K) { if (tn <= 8) go(mmq_i8_kernel<PM_Q4_K, 4, 0, true>); else if (tn <= 16) go(mmq_i8_kernel<PM_Q4_K, 8, 0, true>); else go(mmq_i8_kernel<PM_Q4_K, 16, 0, true>); }
-        else                 { if (tn <= 8) go(mmq_i8_kernel<PM_Q6_K, 4, 0, true>); else if (tn <= 16) go(mmq_i8_kernel<PM_Q6_K, 8, 0, true>); else go(mmq_i8_kernel<PM_Q6_K, 16, 0, true>); }
+        if (p.e_on && type == PM_Q4_K) { if (tn <= 16) go(mmq_i8_kernel<PM_Q4_K, 8, true, true>); else go(mmq_i8_kernel<PM_Q4_K, 16, true, true>); }
+        else if (p.e_on)         { if (tn <= 16) go(mmq_i8_kernel<PM_Q6_K, 8, true, true>); else go(mmq_i8_kernel<PM_Q6_K, 16, true, true>); }
+        else if (type == PM_Q4_K) { if (tn <= 16) go(mmq_i8_kernel<PM_Q4_K, 8, true>); else go(mmq_i8_kernel<PM_Q4_K, 16, true>); }
+        else                 { if (tn <= 16) go(mmq_i8_kernel<PM_Q6_K, 8, true>); else go(mmq_i8_kernel<PM_Q6_K, 16, true>); }
     }
     return 0;
 }
@@ -948,6 +964,16 @@ int pm_launch_mmq_i8_dual(int ta, int na, const void * const * Wa, const int * N
     const Scr * sc = scratch(dev, st, K, reuse_prep != 0);
     if (!sc) return -3;
     if (!reuse_prep) launch_prep(sc, xq, K, T, st);
+    if (T <= ROWS_MAX) {
+        RowsP q = {};
+        int ty[4];
+        if (na > 2) return -5;
+        q.njobs = na + 1; q.K = K; q.T = T; q.bsT = sc->p; q.dT = (const float *) (sc->p + (size_t) nsb * 1024); q.qT = sc->p + scr_q_off(K);
+        for (int j = 0; j < na; ++j) { q.job[j] = {(const uint8_t *) Wa[j], Ya[j], ba ? ba[j] : nullptr, nullptr, Na[j]}; ty[j] = ta; }
+        q.job[na] = {(const uint8_t *) Wb, Yb, bb, nullptr, Nb}; ty[na] = tb;
+        if (!fill_epi(q, epi)) return -5;
+        return pm_launch_mmq_rows(q, ty, st);
+    }
     const int cus = pm_device_cus();
     const double bytes_a = (double) total * pm_weight_row_stride(ta, K), bytes_b = (double) Nb * pm_weight_row_stride(tb, K);
     int gb = (int) (cus * bytes_b / (bytes_a + bytes_b) + 0.5);
@@ -990,10 +1016,10 @@ int pm_launch_mmq_i8_dual(int ta, int na, const void * const * Wa, const int * N
         hipLaunchKernelGGL(kern, dim3(ga + gb), dim3(BLOCK), lds, st, pp);
     };
     if (epi) {
-        if (tb == PM_Q6_K) { if (T <= 8) go(mmq_i8_dual_kernel<PM_Q4_K, PM_Q6_K, 4, true>); else if (T <= 16) go(mmq_i8_dual_kernel<PM_Q4_K, PM_Q6_K, 8, true>); else go(mmq_i8_dual_kernel<PM_Q4_K, PM_Q6_K, 16, true>); }
-        else               { if (T <= 8) go(mmq_i8_dual_kernel<PM_Q4_K, PM_Q5_K, 4, true>); else go(mmq_i8_dual_kernel<PM_Q4_K, PM_Q5_K, 8, true>); }
+        if (tb == PM_Q6_K) { if (T <= 16) go(mmq_i8_dual_kernel<PM_Q4_K, PM_Q6_K, 8, true>); else go(mmq_i8_dual_kernel<PM_Q4_K, PM_Q6_K, 16, true>); }
+        else               { go(mmq_i8_dual_kernel<PM_Q4_K, PM_Q5_K, 8, true>); }
     }
-    else if (tb == PM_Q6_K) { if (T <= 8) go(mmq_i8_dual_kernel<PM_Q4_K, PM_Q6_K, 4>); else if (T <= 16) go(mmq_i8_dual_kernel<PM_Q4_K, PM_Q6_K, 8>); else go(mmq_i8_dual_kernel<PM_Q4_K, PM_Q6_K, 16>); }
-    else               { if (T <= 8) go(mmq_i8_dual_kernel<PM_Q4_K, PM_Q5_K, 4>); else go(mmq_i8_dual_kernel<PM_Q4_K, PM_Q5_K, 8>); }
+    else if (tb == PM_Q6_K) { if (T <= 16) go(mmq_i8_dual_kernel<PM_Q4_K, PM_Q6_K, 8>); else go(mmq_i8_dual_kernel<PM_Q4_K, PM_Q6_K, 16>); }
+    else               { go(mmq_i8_dual_kernel<PM_Q4_K, PM_Q5_K, 8>); }
     return 0;
 }

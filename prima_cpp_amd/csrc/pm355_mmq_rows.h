@@ -1,0 +1,18 @@
+// pm355_mmq_rows.h - launch of the 2..8-token quantized mat-mul (mmq_rows.hip) on activation tables that are already written
+#pragma once
+#include "pm355_device.h"
+#include "pm355_kernels.h"
+
+struct RowsJob { const uint8_t * W; float * y; const float * bias, * resid; int N, each, more; };      // each, more: rows of its workgroups (filled in by the launch)
+struct RowsP {
+    RowsJob job[3]; int njobs, K, T, t_off;                        // t_off: first slot of these tokens in the tables' 32
+    // K-quants: values in operand order [nsb][8][64][16], F16 group sums [nsb][64][8], scales [nsb][32]; Q8_0: values [nb][64][16], scales [nb][32] (pm_q8k_tables, mmq_i8.hip)
+    const uint8_t * qT, * bsT; const float * dT;
+    // the jobs are wq, wk, wv: NORM rope and the KV store in the epilogue (pm_qkv_epi)
+    int e_on; const float * e_tab; const int32_t * e_pos, * e_seq; long e_seq_stride; uint16_t * e_kc, * e_vc; int e_dh, e_nctx, e_nrot, e_kvdim, e_rows;
+};
+template <int TYPE> __device__ __forceinline__ size_t pm_rows_stride(int nb) {
+    return TYPE == PM_Q4_K ? (size_t) nb * 144 : TYPE == PM_Q5_K ? (size_t) nb * 176 : TYPE == PM_Q6_K ? pm_q6k_row_stride((size_t) nb) : (size_t) nb * 32 + (((size_t) nb * 2 + 15) & ~(size_t) 15);
+}
+// one or several matrices of one K (types[0]; only the last may be of another type) over 1..8 tokens; -5: types not served
+int pm_launch_mmq_rows(RowsP p, const int * types, hipStream_t st);

@@ -1440,3 +1440,31 @@ def test_small_batch_attention_fallback_is_indifferent_to_the_pre_rounded_query(
     raw = P.attn_decode(q, kc, vc, pos0, H, Hkv, dh, n_ctx, scale)
     rounded = P.attn_decode(q.half().float(), kc, vc, pos0, H, Hkv, dh, n_ctx, scale)
     assert torch.equal(raw, rounded)
+
+
+@pytest.mark.parametrize("t", [Q4_K, Q5_K, Q6_K, Q8_0])
+def test_small_batch_rows_kernel_at_its_edges(P, oracle, t):
+    """mmq_rows.hip (2..8 tokens): one and two super-blocks more than a step of eight pairs holds, odd and even counts, a single pair, blocks of 32 that end inside a pair; rows below, at and above
+    the 16 of a row group, one to three groups in one pass and several passes of 64 (activations in LDS where they fit, passes of 48 where they do not); every token count. Against the oracle:
+    the same integers, <= K / 256 (Q8_0: K / 32) f32 terms in another order - the bound of the other small-batch products."""
+    rng = np.random.default_rng(7100 + t)
+    tail = 32 if t == Q8_0 else 256
+    for K, N, T in ((512, 1, 8), (512, 15, 1), (768, 16, 2), (2048, 17, 3), (4096, 33, 4), (4096 + tail, 100, 5), (4352, 4096, 7), (4608, 4097, 8), (8192 + tail, 8192 + 31, 6), (1024, 12300, 8), (768, 28700, 3),
+                    (8192, 12290, 2), (12288, 16390, 8)):
+        b = rand_blocks(t, N, K, rng)
+        x = rng.normal(0, 1, (T, K)).astype(np.float32)
+        bias, resid = rng.normal(0, 1, N).astype(np.float32), rng.normal(0, 1, (T, N)).astype(np.float32)
+        w = P.upload_weight(t, b, K, N)
+        rows = np.unique(np.concatenate([np.arange(min(N, 70)), np.arange(max(N - 70, 0), N), rng.integers(0, N, 150)]))   # (the oracle is a scalar program)
+        bytes_per_row = b.size // N
+        want = oracle.mul_mat(t, b.reshape(N, bytes_per_row)[rows].copy(), K, len(rows), x)
+        tol = dict(rtol=2e-5, atol=2e-5 * np.sqrt(max(K, 4096) / 4096))
+        y = P.mul_mat_small(w, x=_dev(P, x)).cpu().numpy()
+        assert np.isfinite(y).all(), (K, N, T)
+        assert np.allclose(y[:, rows], want, **tol), (K, N, T, np.abs(y[:, rows] - want).max())
+        xq = P.quantize_act(_dev(P, x), P.vec_dot_act_type(t))
+        y2 = P.mul_mat_small(w, xq=xq, n_tokens=T, bias=_dev(P, bias), resid=_dev(P, resid)).cpu().numpy()
+        assert np.array_equal(y2, (y + bias[None]) + resid), (K, N, T)
+        # a token's sums do not depend on the tokens beside it
+        one = P.mul_mat_small(w, x=_dev(P, x[T - 1:])).cpu().numpy()
+        assert np.array_equal(one[0], y[T - 1]), (K, N, T)
