@@ -74,33 +74,36 @@ __device__ __forceinline__ void halves(u32x4 & x, u32x4 & y) {
 template <int TYPE> struct ASet { u32x4 q[8], bs; f32x4 yd; };
 template <> struct ASet<PM_Q8_0> { u32x4 q[4]; f32x4 yd[4]; };
 // from the tables that the quantizers (or mmq_i8.hip's prologue) write; lane offsets are out of range - zeros, no traffic - where the operand row is empty
-struct ASrc { __amdgpu_buffer_rsrc_t rq, rb, rd; uint32_t qo, bo, dd; int n; };
-template <int TYPE> __device__ __forceinline__ ASrc source_a(const RowsP & p, int nb, int lr, int kg) {
+// (g: the group of eight tokens; only the last one may have fewer)
+struct ASrc { __amdgpu_buffer_rsrc_t rq, rb, rd; uint32_t qo[2], bo[2], dd; int n; };
+template <int TYPE, int NG> __device__ __forceinline__ ASrc source_a(const RowsP & p, int nb, int lr, int kg) {
     constexpr bool Q80 = TYPE == PM_Q8_0;
     const int t = lr & 7, hk = kg >> 1;
-    const bool on = (lr >> 3) == hk && t < p.T;
+    const bool on = (lr >> 3) == hk, on_last = on && t + 8 * (NG - 1) < p.T;
     ASrc s;
     s.n = nb;
     s.rq = __builtin_amdgcn_make_buffer_rsrc((void *) p.qT, 0, nb * (Q80 ? 1024 : 8192), 0x00020000);
     s.rb = __builtin_amdgcn_make_buffer_rsrc((void *) p.bsT, 0, nb * 1024, 0x00020000);
     s.rd = __builtin_amdgcn_make_buffer_rsrc((void *) p.dT, 0, nb * 128, 0x00020000);
-    s.qo = on ? (uint32_t) (hk * (Q80 ? 4096 : 8192) + (32 * (kg & 1) + t + p.t_off) * 16) : 0x80000000u;
-    s.bo = on ? (uint32_t) (hk * 1024 + (32 * (kg & 1) + t + p.t_off) * 16) : 0x80000000u;
+    const uint32_t qo = (uint32_t) (hk * (Q80 ? 4096 : 8192) + (32 * (kg & 1) + t + p.t_off) * 16), bo = (uint32_t) (hk * 1024 + (32 * (kg & 1) + t + p.t_off) * 16);
+    s.qo[0] = on ? qo : 0x80000000u; s.qo[1] = on_last ? qo : 0x80000000u;
+    s.bo[0] = on ? bo : 0x80000000u; s.bo[1] = on_last ? bo : 0x80000000u;
     s.dd = (uint32_t) (hk * (Q80 ? 512 : 128) + 16 * (kg & 1) + 4 * p.t_off);
     return s;
 }
-template <int TYPE> __device__ __forceinline__ void load_q(ASet<TYPE> & a, const ASrc & s, int pair, int j) {
-    if constexpr (TYPE == PM_Q8_0) a.q[j] = ld_buf(s.rq, s.qo + (uint32_t) (pair * 8192 + j * 1024), 0);       // (zeros behind the last block of a row, where the tables end)
-    else a.q[j] = ld_buf(s.rq, s.qo + (uint32_t) ((j & 3) * 1024), first_of(pair, s.n) * 8192 + (j >> 2) * 4096);
+template <int TYPE> __device__ __forceinline__ void load_q(ASet<TYPE> & a, const ASrc & s, int g, bool last, int pair, int j) {
+    const uint32_t o = s.qo[last] + (uint32_t) (128 * g);
+    if constexpr (TYPE == PM_Q8_0) a.q[j] = ld_buf(s.rq, o + (uint32_t) (pair * 8192 + j * 1024), 0);       // (zeros behind the last block of a row, where the tables end)
+    else a.q[j] = ld_buf(s.rq, o + (uint32_t) ((j & 3) * 1024), first_of(pair, s.n) * 8192 + (j >> 2) * 4096);
 }
-template <int TYPE> __device__ __forceinline__ void load_yd(ASet<TYPE> & a, const ASrc & s, int pair, int hk) {
+template <int TYPE> __device__ __forceinline__ void load_yd(ASet<TYPE> & a, const ASrc & s, int g, bool last, int pair, int hk) {
     if constexpr (TYPE == PM_Q8_0) {
 #pragma unroll
-        for (int j = 0; j < 4; ++j) a.yd[j] = __builtin_bit_cast(f32x4, ld_buf(s.rd, s.dd + (uint32_t) (pair * 1024 + j * 128), 0));
+        for (int j = 0; j < 4; ++j) a.yd[j] = __builtin_bit_cast(f32x4, ld_buf(s.rd, s.dd + (uint32_t) (pair * 1024 + j * 128 + 32 * g), 0));
     } else {
         const int sb = first_of(pair, s.n);
-        a.bs = ld_buf(s.rb, s.bo, sb * 1024);
-        a.yd = __builtin_bit_cast(f32x4, ld_buf(s.rd, sb + hk >= 2 * pair ? s.dd : 0x80000000u, sb * 128));
+        a.bs = ld_buf(s.rb, s.bo[last] + (uint32_t) (128 * g), sb * 1024);
+        a.yd = __builtin_bit_cast(f32x4, ld_buf(s.rd, sb + hk >= 2 * pair ? s.dd + (uint32_t) (32 * g) : 0x80000000u, sb * 128));
     }
 }
 // All activations in LDS, 8 tokens of each super-block: where the waves go over them several times (more rows per workgroup than one pass takes)
@@ -198,30 +201,33 @@ template <> struct Scales<PM_Q5_K> {                               // (inside th
 template <int TYPE> struct Tile;
 
 // Q4_K / Q5_K: sum += scale_j * (w . a), scales and mins four to a dword (get_scale_min_k4, ggml-quants.c:1898-1906)
-struct K4 {
-    uint32_t sc[2], mn[2], dm; i32x4 sum;
-    __device__ __forceinline__ explicit K4(const u32x4 & hd) : dm(hd[0]), sum{0, 0, 0, 0} {
+template <int NG> struct K4 {
+    uint32_t sc[2], mn[2], dm; i32x4 sum[NG];
+    __device__ __forceinline__ explicit K4(const u32x4 & hd) : dm(hd[0]), sum{} {
         sc[0] = hd[1] & 0x3f3f3f3fu; sc[1] = (hd[3] & 0x0f0f0f0fu) | ((hd[1] >> 2) & 0x30303030u);
         mn[0] = hd[2] & 0x3f3f3f3fu; mn[1] = ((hd[3] >> 4) & 0x0f0f0f0fu) | ((hd[2] >> 2) & 0x30303030u);
     }
-    __device__ __forceinline__ void add(const i32x4 & acc, int j) {
+    __device__ __forceinline__ void add(const i32x4 & acc, int g, int j) {
         const int s = (int) ((sc[j >> 2] >> (8 * (j & 3))) & 0xFFu);
 #pragma unroll
-        for (int i = 0; i < 4; ++i) { sum[i] = __mul24(s, acc[i]) + sum[i]; asm("" : "+v"(sum[i])); }   // (keeps it ONE v_mad_i32_i24)
+        for (int i = 0; i < 4; ++i) { sum[g][i] = __mul24(s, acc[i]) + sum[g][i]; asm("" : "+v"(sum[g][i])); }   // (keeps it ONE v_mad_i32_i24)
     }
     // ... and the minima, exact: as F16 (0x6400 | m = 1024 + m), integer sums below 2^24 in f32
-    __device__ __forceinline__ void finish(const u32x4 & bs, const f32x4 & yd, f32x4 & out) const {
+    template <class A> __device__ __forceinline__ void finish(const A (&a)[NG], f32x4 (&out)[NG]) const {
         u32x4 m;
 #pragma unroll
         for (int i = 0; i < 4; ++i) m[i] = pk_fma(__builtin_amdgcn_perm(mn[i >> 1], 0x64646464u, i & 1 ? 0x00070006u : 0x00050004u), (_Float16) 1.0f, (_Float16) -1024.0f);
-        const f32x4 ms = mfma_h(bs, m);
         const float d = h2f((uint16_t) (dm & 0xFFFF)), dmin = h2f((uint16_t) (dm >> 16));
 #pragma unroll
-        for (int i = 0; i < 4; ++i) out[i] = fmaf(yd[i] * d, (float) sum[i], fmaf(-(yd[i] * dmin), ms[i], out[i]));
+        for (int g = 0; g < NG; ++g) {
+            const f32x4 ms = mfma_h(a[g].bs, m);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) out[g][i] = fmaf(a[g].yd[i] * d, (float) sum[g][i], fmaf(-(a[g].yd[i] * dmin), ms[i], out[g][i]));
+        }
     }
 };
 
-// mul: L - the lane's row in the step's scales, kw - the wave's pair in the step; used(j): operand j of the activations has been read
+// mul: L - the lane's row in the step's scales, kw - the wave's pair in the step; used(g, j): operand j of the activations of token group g has been read
 // ---- Q4_K: qa[U][16] | qb[U][16] | hdr[nb][16] (unit u: bytes of sub-blocks 2 u in the low, 2 u + 1 in the high nibbles)
 template <> struct Tile<PM_Q4_K> {
     u32x4 qa[2], qb[2];
@@ -230,17 +236,18 @@ template <> struct Tile<PM_Q4_K> {
         qa[0] = ld_nt16(pa + o.x); qb[0] = ld_nt16(pb + o.x);
         qa[1] = ld_nt16(pa + o.y); qb[1] = ld_nt16(pb + o.y);
     }
-    template <class F> __device__ __forceinline__ void mul(ASet<PM_Q4_K> & a, const uint8_t * L, int kw, int kg, f32x4 & out, F && used) {
-        K4 k(*(const u32x4 *) (L + (2 * kw + (kg >> 1)) * 16));
+    template <int NG, class F> __device__ __forceinline__ void mul(ASet<PM_Q4_K> (&a)[NG], const uint8_t * L, int kw, int kg, f32x4 (&out)[NG], F && used) {
+        K4<NG> k(*(const u32x4 *) (L + (2 * kw + (kg >> 1)) * 16));
         halves(qa[0], qa[1]); halves(qb[0], qb[1]);
         swap16(qa[0], qb[0]); swap16(qa[1], qb[1]);                // units 0, 1, 2, 3
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
             const u32x4 & w = (j >> 1) & 1 ? qb[j >> 2] : qa[j >> 2];
-            k.add(mfma_64(a.q[j], (j & 1 ? w >> 4 : w) & 0x0F0F0F0Fu), j);
-            used(j);
+            const u32x4 b = (j & 1 ? w >> 4 : w) & 0x0F0F0F0Fu;
+#pragma unroll
+            for (int g = 0; g < NG; ++g) { k.add(mfma_64(a[g].q[j], b), g, j); used(g, j); }
         }
-        k.finish(a.bs, a.yd, out);
+        k.finish(a, out);
     }
 };
 
@@ -255,15 +262,16 @@ template <> struct Tile<PM_Q5_K> {
 #pragma unroll
         for (int u = 0; u < 4; ++u) q[u] = ld_c16(p + 48 + 32 * u + (at + 16u * (kg & 1)));
     }
-    template <class F> __device__ __forceinline__ void mul(ASet<PM_Q5_K> & a, const uint8_t *, int, int, f32x4 & out, F && used) {
-        K4 k(hd);
+    template <int NG, class F> __device__ __forceinline__ void mul(ASet<PM_Q5_K> (&a)[NG], const uint8_t *, int, int, f32x4 (&out)[NG], F && used) {
+        K4<NG> k(hd);
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
             const u32x4 & w = q[j >> 1];
-            k.add(mfma_64(a.q[j], ((j & 1 ? w >> 4 : w) & 0x0F0F0F0Fu) | (((qh >> j) & 0x01010101u) << 4)), j);
-            used(j);
+            const u32x4 b = ((j & 1 ? w >> 4 : w) & 0x0F0F0F0Fu) | (((qh >> j) & 0x01010101u) << 4);
+#pragma unroll
+            for (int g = 0; g < NG; ++g) { k.add(mfma_64(a[g].q[j], b), g, j); used(g, j); }
         }
-        k.finish(a.bs, a.yd, out);
+        k.finish(a, out);
     }
 };
 
@@ -276,11 +284,11 @@ template <> struct Tile<PM_Q6_K> {
         la[0] = ld_nt16(pa + o.x); lb[0] = ld_nt16(pb + o.x); qh[0] = ld_nt16(ph + o.x);
         la[1] = ld_nt16(pa + o.y); lb[1] = ld_nt16(pb + o.y); qh[1] = ld_nt16(ph + o.y);
     }
-    template <class F> __device__ __forceinline__ void mul(ASet<PM_Q6_K> & a, const uint8_t * L, int kw, int kg, f32x4 & out, F && used) {
+    template <int NG, class F> __device__ __forceinline__ void mul(ASet<PM_Q6_K> (&a)[NG], const uint8_t * L, int kw, int kg, f32x4 (&out)[NG], F && used) {
         const u32x4 S = *(const u32x4 *) (L + (2 * kw + (kg >> 1)) * 16);
         const float d = h2f(*(const uint16_t *) (L + 256 + 2 * (2 * kw + (kg >> 1))));
         halves(la[0], la[1]); halves(lb[0], lb[1]); halves(qh[0], qh[1]);
-        i32x4 sum = {0, 0, 0, 0};
+        i32x4 sum[NG] = {};
 #pragma unroll
         for (int hh = 0; hh < 2; ++hh) {
             swap16h(la[hh]); swap16h(lb[hh]); swap16h(qh[hh]);
@@ -290,12 +298,15 @@ template <> struct Tile<PM_Q6_K> {
                 for (int v = 0; v < 2; ++v) {
                     const u32x2 l = c & 1 ? u32x2{lb[hh][2 * v], lb[hh][2 * v + 1]} : u32x2{la[hh][2 * v], la[hh][2 * v + 1]}, h = {qh[hh][2 * v], qh[hh][2 * v + 1]};
                     const u32x2 q = ((c >> 1 ? l >> 4 : l) & 0x0F0F0F0Fu) | ((c == 0 ? h << 4 : c == 1 ? h << 2 : c == 2 ? h : h >> 2) & 0x30303030u);
-                    const i32x4 acc = mfma_32(u32x2{a.q[4 * hh + c][2 * v], a.q[4 * hh + c][2 * v + 1]}, q);
                     const int G = 8 * hh + 2 * c + v, s = (int) (int8_t) (S[G >> 2] >> (8 * (G & 3)));
 #pragma unroll
-                    for (int i = 0; i < 4; ++i) { sum[i] = __mul24(s, acc[i]) + sum[i]; asm("" : "+v"(sum[i])); }   // |acc| <= 16 * 63 * 127
+                    for (int g = 0; g < NG; ++g) {
+                        const i32x4 acc = mfma_32(u32x2{a[g].q[4 * hh + c][2 * v], a[g].q[4 * hh + c][2 * v + 1]}, q);
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) { sum[g][i] = __mul24(s, acc[i]) + sum[g][i]; asm("" : "+v"(sum[g][i])); }   // |acc| <= 16 * 63 * 127
+                        if (v == 1) used(g, 4 * hh + c);
+                    }
                 }
-                used(4 * hh + c);
             }
         }
         // - 32 sum_G scale_G * bsum_G (the offset of every weight): operand slot s of lane kg = scale of group 2 s + kg % 2, times -32 (F16: 1024 + 128 + scale from the bytes)
@@ -303,9 +314,12 @@ template <> struct Tile<PM_Q6_K> {
         u32x4 m;
 #pragma unroll
         for (int i = 0; i < 4; ++i) m[i] = pk_fma(__builtin_amdgcn_perm(S[i] ^ 0x80808080u, 0x64646464u, sel), (_Float16) -32.0f, (_Float16) 36864.0f);
-        const f32x4 ms = mfma_h(a.bs, m);                              // (multiples of 32 below 2^29: exact)
 #pragma unroll
-        for (int i = 0; i < 4; ++i) out[i] = fmaf(a.yd[i] * d, (float) (sum[i] + (int) ms[i]), out[i]);
+        for (int g = 0; g < NG; ++g) {
+            const f32x4 ms = mfma_h(a[g].bs, m);                       // (multiples of 32 below 2^29: exact)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) out[g][i] = fmaf(a[g].yd[i] * d, (float) (sum[g][i] + (int) ms[i]), out[g][i]);
+        }
     }
 };
 
@@ -319,24 +333,27 @@ template <> struct Tile<PM_Q8_0> {
         qa[0] = ld_nt16(s.base + ox); qb[0] = ld_nt16(pb + ox);
         qa[1] = ld_nt16(s.base + oy); qb[1] = ld_nt16(pb + oy);
     }
-    template <class F> __device__ __forceinline__ void mul(ASet<PM_Q8_0> & a, const uint8_t * L, int kw, int kg, f32x4 & out, F && used) {
+    template <int NG, class F> __device__ __forceinline__ void mul(ASet<PM_Q8_0> (&a)[NG], const uint8_t * L, int kw, int kg, f32x4 (&out)[NG], F && used) {
         const u32x2 d4 = *(const u32x2 *) (L + kw * 16 + 8 * (kg >> 1));
         halves(qa[0], qa[1]); halves(qb[0], qb[1]);
         swap16(qa[0], qb[0]); swap16(qa[1], qb[1]);                // blocks 0 | 4, 1 | 5, 2 | 6, 3 | 7
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-            const i32x4 acc = mfma_64(a.q[j], j & 1 ? qb[j >> 1] : qa[j >> 1]);
-            used(j);
             const uint32_t hb = (d4[j >> 1] >> (16 * (j & 1))) & 0xFFFFu;
             const float dw = (hb & 0x7C00u) == 0x7C00u ? 0.0f : h2f((uint16_t) hb);      // (padding behind the row, times zero)
 #pragma unroll
-            for (int i = 0; i < 4; ++i) out[i] = fmaf((float) acc[i], dw * a.yd[j][i], out[i]);
+            for (int g = 0; g < NG; ++g) {
+                const i32x4 acc = mfma_64(a[g].q[j], j & 1 ? qb[j >> 1] : qa[j >> 1]);
+                used(g, j);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) out[g][i] = fmaf((float) acc[i], dw * a[g].yd[j][i], out[g][i]);
+            }
         }
     }
 };
 
-// A step: KW = 8 pairs, one per wave, of 16 R rows. D steps of weights are in flight; AL: activations from LDS
-template <int TYPE, int R, int D, bool AL, bool EPI>
+// A step: KW = 8 pairs, one per wave, of 16 R rows, times NG groups of eight tokens. D steps of weights are in flight; AL: activations from LDS
+template <int TYPE, int NG, int R, int D, bool AL, bool EPI>
 __device__ __forceinline__ void rows_body(const RowsP & p, const RowsJob & job, int w, int ji, uint8_t * smem) {
     constexpr int ROWS = 16 * R;
     typedef Scales<TYPE> SC;
@@ -351,16 +368,16 @@ __device__ __forceinline__ void rows_body(const RowsP & p, const RowsJob & job, 
     if (npass <= 0) return;
     // LDS: partial sums of two passes | scales of two steps | activations
     float * red = (float *) smem;
-    uint8_t * scl = smem + 2 * KW * R * 512;
+    uint8_t * scl = smem + 2 * KW * R * NG * 512;
     uint8_t * act = scl + 2 * ROWS * SC::PITCH;
-    const ASrc as = source_a<TYPE>(p, nb, lr, kg);
+    const ASrc as = source_a<TYPE, NG>(p, nb, lr, kg);
     WSrc ws;
     ws.nb = nb;
     const uint32_t stride = (uint32_t) pm_rows_stride<TYPE>(nb);
     ws.base = job.W + (long) r0 * stride;
     const int lim = r1 - r0 - 1;
     Tile<TYPE> W[D][R];
-    ASet<TYPE> A;
+    ASet<TYPE> A[NG];
     Off off[R];
     const uint32_t px = TYPE == PM_Q5_K ? 0 : 16u * (uint32_t) piece_of(kg, lr >> 3), py = 16u * (uint32_t) piece_of(kg, 1 - (lr >> 3));
     // the step whose weights are asked for next (behind the last one: the slice's first row, sixteen times)
@@ -398,17 +415,24 @@ __device__ __forceinline__ void rows_body(const RowsP & p, const RowsJob & job, 
     };
     // a thread's element of a pass' results: row 16 rg + rr, token t; what the end of the pass adds is asked for behind the first weights (at its use it was a round of latency on its own, in
     // the rotation's case three). No branches: rows and tokens past the end ask for the last one's, absent operands for some bytes of the matrix
-    const int rr = tid & 15, t = (tid >> 4) & 7, rg = tid >> 7;
-    struct { float add, resid, c, sn; int seq, pos; } e;
+    constexpr int NEL = (R * NG * 128 + NT - 1) / NT;
+    struct End { float add, resid, c, sn; int seq, pos; } end[NEL];
+    struct El { int rr, rg, g, t; };
+    auto el_of = [&](int i) __attribute__((always_inline)) { const int x = tid + i * NT; return El{x & 15, (x >> 7) % R, (x >> 7) / R, 8 * ((x >> 7) / R) + ((x >> 4) & 7)}; };
     auto load_end = [&](int pass) __attribute__((always_inline)) {
-        const int lrow = min(r0 + ROWS * pass + 16 * rg + rr, r1 - 1), tt = min(t, p.T - 1);
-        e.add = ld_g((job.bias ? job.bias : (const float *) job.W) + lrow);
-        if constexpr (EPI) {
-            const int dim = min(lrow % p.e_dh, p.e_nrot - 1);
-            e.seq = ld_g((p.e_seq ? p.e_seq : p.e_pos) + (p.e_rows ? tt : 0)); e.seq = p.e_seq ? e.seq : 0;
-            e.pos = ld_g(p.e_pos + tt * p.e_rows);
-            e.c = ld_g(p.e_tab + (long) tt * p.e_nrot + (dim & ~1)); e.sn = ld_g(p.e_tab + (long) tt * p.e_nrot + (dim & ~1) + 1);
-        } else e.resid = ld_g((job.resid ? job.resid : (const float *) job.W) + (long) tt * job.N + lrow);
+#pragma unroll
+        for (int i = 0; i < NEL; ++i) {
+            const El x = el_of(i);
+            End & e = end[i];
+            const int lrow = min(r0 + ROWS * pass + 16 * x.rg + x.rr, r1 - 1), tt = min(x.t, p.T - 1);
+            e.add = ld_g((job.bias ? job.bias : (const float *) job.W) + lrow);
+            if constexpr (EPI) {
+                const int dim = min(lrow % p.e_dh, p.e_nrot - 1);
+                e.seq = ld_g((p.e_seq ? p.e_seq : p.e_pos) + (p.e_rows ? tt : 0)); e.seq = p.e_seq ? e.seq : 0;
+                e.pos = ld_g(p.e_pos + tt * p.e_rows);
+                e.c = ld_g(p.e_tab + (long) tt * p.e_nrot + (dim & ~1)); e.sn = ld_g(p.e_tab + (long) tt * p.e_nrot + (dim & ~1) + 1);
+            } else e.resid = ld_g((job.resid ? job.resid : (const float *) job.W) + (long) tt * job.N + lrow);
+        }
     };
     constexpr int NQ = Q80 ? 4 : 8;
     rows_of(0);
@@ -421,8 +445,11 @@ __device__ __forceinline__ void rows_body(const RowsP & p, const RowsJob & job, 
         advance();
         if constexpr (!AL) if (d == 0) {
 #pragma unroll
-            for (int j = 0; j < NQ; ++j) load_q<TYPE>(A, as, wave, j);
-            load_yd<TYPE>(A, as, wave, hk);
+            for (int g = 0; g < NG; ++g) {
+#pragma unroll
+                for (int j = 0; j < NQ; ++j) load_q<TYPE>(A[g], as, g, g == NG - 1, wave, j);
+                load_yd<TYPE>(A[g], as, g, g == NG - 1, wave, hk);
+            }
         }
     }
     load_end(0);
@@ -432,9 +459,7 @@ __device__ __forceinline__ void rows_body(const RowsP & p, const RowsJob & job, 
     if constexpr (AL) al = lane_a<TYPE>(na, lr, kg);
     int e_pos0 = 0;
     if constexpr (EPI) if (!p.e_rows) e_pos0 = p.e_pos[p.e_seq ? p.e_seq[0] : 0];      // (scalar loads)
-    f32x4 out[R];
-#pragma unroll
-    for (int r = 0; r < R; ++r) out[r] = f32x4{0, 0, 0, 0};
+    f32x4 out[R][NG] = {};
     int pass = 0, it = 0;
     for (int step = 0; step < nstep; ) {
 #pragma unroll
@@ -442,62 +467,76 @@ __device__ __forceinline__ void rows_body(const RowsP & p, const RowsJob & job, 
             const bool wrap = it + 1 == nit;
             const int itn = wrap ? 0 : it + 1, next = wave + KW * itn;
             load_scales(wrap ? min(pass + 1, npass - 1) : pass, itn);
-            if constexpr (AL) read_a<TYPE>(A, act, al, wave + KW * it, na, hk);
+            if constexpr (AL) read_a<TYPE>(A[0], act, al, wave + KW * it, na, hk);
             __builtin_amdgcn_sched_barrier(0);
             const uint8_t * L = scl + (step & 1) * (ROWS * SC::PITCH) + lr * SC::PITCH;
             if constexpr (TYPE == PM_Q6_K) {
 #pragma unroll
-                for (int j = 0; j < NQ; ++j) swap16h(A.q[j]);
+                for (int g = 0; g < NG; ++g)
+#pragma unroll
+                    for (int j = 0; j < NQ; ++j) swap16h(A[g].q[j]);
             }
 #pragma unroll
             for (int r = 0; r < R; ++r) {
-                auto used = [&](int j) __attribute__((always_inline)) {
-                    if constexpr (!AL) if (r == R - 1) { __builtin_amdgcn_sched_barrier(0); load_q<TYPE>(A, as, next, j); __builtin_amdgcn_sched_barrier(0); }
+                auto used = [&](int g, int j) __attribute__((always_inline)) {
+                    if constexpr (!AL) if (r == R - 1) { __builtin_amdgcn_sched_barrier(0); load_q<TYPE>(A[g], as, g, g == NG - 1, next, j); __builtin_amdgcn_sched_barrier(0); }
                 };
                 if (r == 0 || ROWS * pass + 16 * r <= lim) W[d][r].mul(A, L + 16 * r * SC::PITCH, wave, kg, out[r], used);
                 else {                                                 // (the last pass: no such rows)
 #pragma unroll
-                    for (int j = 0; j < NQ; ++j) used(j);
+                    for (int j = 0; j < NQ; ++j)
+#pragma unroll
+                        for (int g = 0; g < NG; ++g) used(g, j);
                 }
                 __builtin_amdgcn_sched_barrier(0);
                 W[d][r].load(ws, off[r], kg, wave + KW * wn.it);
                 __builtin_amdgcn_sched_barrier(0);
             }
-            if constexpr (!AL) { load_yd<TYPE>(A, as, next, hk); __builtin_amdgcn_sched_barrier(0); }
+            if constexpr (!AL) {
+#pragma unroll
+                for (int g = 0; g < NG; ++g) load_yd<TYPE>(A[g], as, g, g == NG - 1, next, hk);
+                __builtin_amdgcn_sched_barrier(0);
+            }
             advance();
             if (wrap) {
                 // sums over the waves and the two super-blocks of a pair, in a fixed order: the latter here, 32 lanes of either
-                float * buf = red + (pass & 1) * (KW * R * 128);
+                float * buf = red + (pass & 1) * (KW * R * NG * 128);
 #pragma unroll
-                for (int r = 0; r < R; ++r) {
-                    f32x4 s;
+                for (int r = 0; r < R; ++r)
 #pragma unroll
-                    for (int i = 0; i < 4; ++i) {
-                        const float o = out[r][i];
-                        const u32x2 v = __builtin_bit_cast(u32x2, __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(uint32_t, o), __builtin_bit_cast(uint32_t, o), false, false));
-                        const uint32_t lo = v[0], hi = v[1];               // (a bit cast of a vector's element takes element 0 here)
-                        s[i] = __builtin_bit_cast(float, lo) + __builtin_bit_cast(float, hi);
+                    for (int g = 0; g < NG; ++g) {
+                        f32x4 s;
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) {
+                            const float o = out[r][g][i];
+                            const u32x2 v = __builtin_bit_cast(u32x2, __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(uint32_t, o), __builtin_bit_cast(uint32_t, o), false, false));
+                            const uint32_t lo = v[0], hi = v[1];               // (a bit cast of a vector's element takes element 0 here)
+                            s[i] = __builtin_bit_cast(float, lo) + __builtin_bit_cast(float, hi);
+                        }
+                        if (lane < 32) *(f32x4 *) (buf + (((wave * NG + g) * R + r) * 32 + lane) * 4) = s;
+                        out[r][g] = f32x4{0, 0, 0, 0};
                     }
-                    if (lane < 32) *(f32x4 *) (buf + ((wave * R + r) * 32 + lane) * 4) = s;
-                    out[r] = f32x4{0, 0, 0, 0};
-                }
             }
             store_scales((step + 1) & 1);
             __syncthreads();
             if (wrap) {
-                const float * buf = red + (pass & 1) * (KW * R * 128);
-                if (tid < ROWS * 8) {
+                const float * buf = red + (pass & 1) * (KW * R * NG * 128);
+#pragma unroll
+                for (int i = 0; i < NEL; ++i) {
+                    if (R * NG * 128 % NT != 0 && tid + i * NT >= R * NG * 128) continue;
+                    const El x = el_of(i);
+                    const End & e = end[i];
                     float s = 0.0f;
 #pragma unroll
-                    for (int k = 0; k < KW; ++k) s += buf[((k * R + rg) * 32 + 16 * (t >> 2) + rr) * 4 + (t & 3)];
-                    const int lrow = r0 + ROWS * pass + 16 * rg + rr;
-                    const bool live = t < p.T && lrow < r1;
+                    for (int k = 0; k < KW; ++k) s += buf[(((k * NG + x.g) * R + x.rg) * 32 + 16 * ((x.t >> 2) & 1) + x.rr) * 4 + (x.t & 3)];
+                    const int lrow = r0 + ROWS * pass + 16 * x.rg + x.rr;
+                    const bool live = x.t < p.T && lrow < r1;
                     if (job.bias) s += e.add;
                     if constexpr (EPI) {
                         const float sp = __shfl_xor(s, 1);                  // the pair's other row: the neighbouring lane, same token
                         if (live) {
                             const long kv = (long) e.seq * p.e_seq_stride;
-                            const int pos = p.e_rows ? e.pos : e_pos0 + t;
+                            const int pos = p.e_rows ? e.pos : e_pos0 + x.t;
                             if (ji == 2) p.e_vc[kv + (long) lrow * p.e_nctx + pos] = f2h(s);
                             else {
                                 const int dim = lrow % p.e_dh;
@@ -505,12 +544,12 @@ __device__ __forceinline__ void rows_body(const RowsP & p, const RowsJob & job, 
                                 if (dim < p.e_nrot) v = (dim & 1) ? sp * e.sn + s * e.c : s * e.c - sp * e.sn;
                                 const uint16_t hv = f2h(v);
                                 if (ji == 1) p.e_kc[kv + (long) pos * p.e_kvdim + lrow] = hv;
-                                else st_g(job.y + (long) t * job.N + lrow, h2f(hv));
+                                else st_g(job.y + (long) x.t * job.N + lrow, h2f(hv));
                             }
                         }
-                    } else if (live) st_g(job.y + (long) t * job.N + lrow, job.resid ? s + e.resid : s);
-                    if (pass + 1 < npass) load_end(pass + 1);
+                    } else if (live) st_g(job.y + (long) x.t * job.N + lrow, job.resid ? s + e.resid : s);
                 }
+                if (pass + 1 < npass) load_end(pass + 1);
                 ++pass;
             }
             it = itn;
@@ -520,24 +559,29 @@ __device__ __forceinline__ void rows_body(const RowsP & p, const RowsJob & job, 
 }
 
 // TA: the type of all jobs but the last, TB: of the last one. first1, first2: first workgroups of the second and third job (in registers when the kernel starts)
-template <int TA, int TB, int R, int D, bool AL, bool EPI>
+template <int TA, int TB, int NG, int R, int D, bool AL, bool EPI>
 __global__ __launch_bounds__(NT, 2) void mmq_rows_kernel(int first1, int first2, RowsP p) {
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
     const int b = (int) blockIdx.x, ji = (b >= first1) + (b >= first2);
     const RowsJob job = p.job[ji];
     const int w = b - (ji == 0 ? 0 : ji == 1 ? first1 : first2);
-    if (TA == TB || ji < p.njobs - 1) rows_body<TA, R, D, AL, EPI>(p, job, w, ji, smem);
-    else rows_body<TB, R, D, AL, EPI>(p, job, w, ji, smem);
+    if (TA == TB || ji < p.njobs - 1) rows_body<TA, NG, R, D, AL, EPI>(p, job, w, ji, smem);
+    else rows_body<TB, NG, R, D, AL, EPI>(p, job, w, ji, smem);
 }
-template <int TYPE> size_t lds_of(int R, bool AL, int K) {
+template <int TYPE> size_t lds_of(int NG, int R, bool AL, int K) {
     const int n = TYPE == PM_Q8_0 ? (K / 32 + 7) / 8 : K / 256;
-    return (size_t) 2 * KW * R * 512 + (size_t) 2 * 16 * R * Scales<TYPE>::PITCH + (AL ? ALds<TYPE>::bytes(n) : 0);
+    return (size_t) 2 * KW * R * NG * 512 + (size_t) 2 * 16 * R * Scales<TYPE>::PITCH + (AL ? ALds<TYPE>::bytes(n) : 0);
 }
-size_t lds_of(int type, int R, bool AL, int K) {
-    return type == PM_Q4_K ? lds_of<PM_Q4_K>(R, AL, K) : type == PM_Q5_K ? lds_of<PM_Q5_K>(R, AL, K) : type == PM_Q6_K ? lds_of<PM_Q6_K>(R, AL, K) : lds_of<PM_Q8_0>(R, AL, K);
+size_t lds_of(int type, int NG, int R, bool AL, int K) {
+    return type == PM_Q4_K ? lds_of<PM_Q4_K>(NG, R, AL, K) : type == PM_Q5_K ? lds_of<PM_Q5_K>(NG, R, AL, K) : type == PM_Q6_K ? lds_of<PM_Q6_K>(NG, R, AL, K) : lds_of<PM_Q8_0>(NG, R, AL, K);
 }
 
 }  // namespace
+
+// Several groups of eight tokens only where every workgroup has one group of rows: the activations of a K range are then asked for once per workgroup like the weights, and the chip is full (with
+// 32-row groups it is half empty). 16 / 23 tokens, us, mmq_i8.hip / here (4.5 of them the tables): 4096 x 4096 Q4_K 11.4 / 10.3, 13.3 / 11.9; 4096 x 14336 Q4_K 19.3 / 18.7, 23.0 / 21.5, Q6_K 31.8 /
+// 25.8, 39.1 / 29.4. With two groups of rows 8192 x 8192 16.5 / 18.2, 19.4 / 23.9; with four groups of tokens the registers do not hold the activations (29 tokens: 13.4 / 18.5).
+int pm_mmq_rows_max_tokens(int N) { return N <= 16 * pm_device_cus() ? 24 : 8; }
 
 int pm_launch_mmq_rows(RowsP p, const int * types, hipStream_t st) {
     const int cus = pm_device_cus(), n = p.njobs;
@@ -560,18 +604,27 @@ int pm_launch_mmq_rows(RowsP p, const int * types, hipStream_t st) {
     }
     // up to 48 rows a workgroup: one pass, activations by the wave that multiplies them; more: passes of 64 rows over activations in LDS where they fit (K up to 9 k: two thirds of it), else
     // again passes of 48
-    const auto lds = [&](int r, bool al) { return std::max(lds_of(ta, r, al, p.K), lds_of(tb, r, al, p.K)); };
-    const bool al = big > 3 && lds(4, true) <= 150 * 1024, deep = p.K > 4096;
+    const auto lds = [&](int g, int r, bool al) { return std::max(lds_of(ta, g, r, al, p.K), lds_of(tb, g, r, al, p.K)); };
+    const int ng = (p.T + 7) / 8;
+    const bool al = ng == 1 && big > 3 && lds(1, 4, true) <= 150 * 1024, deep = p.K > 4096;
     auto go = [&](auto kern, size_t bytes) {
         pm_allow_big_lds((const void *) kern, bytes);
         hipLaunchKernelGGL(kern, dim3(at), dim3(NT), bytes, st, first[1], first[2], p);
         return 0;
     };
-#define PM_ROWS_GO(TA_, TB_, R_, D_, AL_, E_) go(mmq_rows_kernel<TA_, TB_, R_, D_, AL_, E_>, lds(R_, AL_))
-#define PM_ROWS_R(TA_, TB_, E_) { if (al) return PM_ROWS_GO(TA_, TB_, 4, 1, true, E_); \
-                                  switch (big) { case 1: return deep ? PM_ROWS_GO(TA_, TB_, 1, 2, false, E_) : PM_ROWS_GO(TA_, TB_, 1, 1, false, E_); \
-                                                 case 2: return deep ? PM_ROWS_GO(TA_, TB_, 2, 2, false, E_) : PM_ROWS_GO(TA_, TB_, 2, 1, false, E_); \
-                                                 default: return PM_ROWS_GO(TA_, TB_, 3, 1, false, E_); } }
+#define PM_ROWS_GO(TA_, TB_, G_, R_, D_, AL_, E_) go(mmq_rows_kernel<TA_, TB_, G_, R_, D_, AL_, E_>, lds(G_, R_, AL_))
+#define PM_ROWS_R(TA_, TB_, E_) { if (al) return PM_ROWS_GO(TA_, TB_, 1, 4, 1, true, E_); \
+                                  switch (big) { case 1: return deep ? PM_ROWS_GO(TA_, TB_, 1, 1, 2, false, E_) : PM_ROWS_GO(TA_, TB_, 1, 1, 1, false, E_); \
+                                                 case 2: return deep ? PM_ROWS_GO(TA_, TB_, 1, 2, 2, false, E_) : PM_ROWS_GO(TA_, TB_, 1, 2, 1, false, E_); \
+                                                 default: return PM_ROWS_GO(TA_, TB_, 1, 3, 1, false, E_); } }
+    if (ng > 1) {
+        if (n > 1 || big > 1 || ng > 3) return -5;
+        const auto one = [&](auto two, auto three) { return go(ng == 2 ? two : three, lds(ng, 1, false)); };
+        return ta == PM_Q4_K ? one(mmq_rows_kernel<PM_Q4_K, PM_Q4_K, 2, 1, 1, false, false>, mmq_rows_kernel<PM_Q4_K, PM_Q4_K, 3, 1, 1, false, false>)
+             : ta == PM_Q5_K ? one(mmq_rows_kernel<PM_Q5_K, PM_Q5_K, 2, 1, 1, false, false>, mmq_rows_kernel<PM_Q5_K, PM_Q5_K, 3, 1, 1, false, false>)
+             : ta == PM_Q6_K ? one(mmq_rows_kernel<PM_Q6_K, PM_Q6_K, 2, 1, 1, false, false>, mmq_rows_kernel<PM_Q6_K, PM_Q6_K, 3, 1, 1, false, false>)
+             : ta == PM_Q8_0 ? one(mmq_rows_kernel<PM_Q8_0, PM_Q8_0, 2, 1, 1, false, false>, mmq_rows_kernel<PM_Q8_0, PM_Q8_0, 3, 1, 1, false, false>) : -5;
+    }
     if (p.e_on) {
         if (ta == PM_Q4_K && tb == PM_Q4_K) PM_ROWS_R(PM_Q4_K, PM_Q4_K, true)
         if (ta == PM_Q6_K && tb == PM_Q6_K) PM_ROWS_R(PM_Q6_K, PM_Q6_K, true)

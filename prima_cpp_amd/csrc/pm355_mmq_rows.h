@@ -1,4 +1,4 @@
-// pm355_mmq_rows.h - launch of the 2..8-token quantized mat-mul (mmq_rows.hip) on activation tables that are already written
+// pm355_mmq_rows.h - launch of the quantized mat-mul of few tokens (mmq_rows.hip) on activation tables that are already written
 #pragma once
 #include "pm355_device.h"
 #include "pm355_kernels.h"
@@ -14,5 +14,6 @@ struct RowsP {
 template <int TYPE> __device__ __forceinline__ size_t pm_rows_stride(int nb) {
     return TYPE == PM_Q4_K ? (size_t) nb * 144 : TYPE == PM_Q5_K ? (size_t) nb * 176 : TYPE == PM_Q6_K ? pm_q6k_row_stride((size_t) nb) : (size_t) nb * 32 + (((size_t) nb * 2 + 15) & ~(size_t) 15);
 }
-// one or several matrices of one K (types[0]; only the last may be of another type) over 1..8 tokens; -5: types not served
+// one or several matrices of one K (types[0]; only the last may be of another type) over 1..8 tokens, one matrix of N rows over 1..pm_mmq_rows_max_tokens(N); -5: not served
+int pm_mmq_rows_max_tokens(int N);
 int pm_launch_mmq_rows(RowsP p, const int * types, hipStream_t st);

@@ -1444,13 +1444,14 @@ def test_small_batch_attention_fallback_is_indifferent_to_the_pre_rounded_query(
 
 @pytest.mark.parametrize("t", [Q4_K, Q5_K, Q6_K, Q8_0])
 def test_small_batch_rows_kernel_at_its_edges(P, oracle, t):
-    """mmq_rows.hip (2..8 tokens): one and two super-blocks more than a step of eight pairs holds, odd and even counts, a single pair, blocks of 32 that end inside a pair; rows below, at and above
+    """mmq_rows.hip: one and two super-blocks more than a step of eight pairs holds, odd and even counts, a single pair, blocks of 32 that end inside a pair; rows below, at and above
     the 16 of a row group, one to three groups in one pass and several passes of 64 (activations in LDS where they fit, passes of 48 where they do not); every token count. Against the oracle:
     the same integers, <= K / 256 (Q8_0: K / 32) f32 terms in another order - the bound of the other small-batch products."""
     rng = np.random.default_rng(7100 + t)
     tail = 32 if t == Q8_0 else 256
     for K, N, T in ((512, 1, 8), (512, 15, 1), (768, 16, 2), (2048, 17, 3), (4096, 33, 4), (4096 + tail, 100, 5), (4352, 4096, 7), (4608, 4097, 8), (8192 + tail, 8192 + 31, 6), (1024, 12300, 8), (768, 28700, 3),
-                    (8192, 12290, 2), (12288, 16390, 8)):
+                    (8192, 12290, 2), (12288, 16390, 8),
+                    (512, 16, 17), (768, 4096, 16), (4096 + tail, 33, 9), (4608, 100, 24), (14336, 4095, 23)):     # (up to 24 tokens where a workgroup has one group of rows)
         b = rand_blocks(t, N, K, rng)
         x = rng.normal(0, 1, (T, K)).astype(np.float32)
         bias, resid = rng.normal(0, 1, N).astype(np.float32), rng.normal(0, 1, (T, N)).astype(np.float32)
