@@ -22,31 +22,6 @@ __device__ __forceinline__ u32x4 coh_ld16u(__amdgpu_buffer_rsrc_t r, uint32_t of
 __device__ __forceinline__ float coh_ld4(__amdgpu_buffer_rsrc_t r, uint32_t off) { return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, (int) off, 0, 17)); }
 
 
-// ---- reductions whose result every lane of a wave gets, without LDS: 16-lane rows by DPP, then the rows by lane swaps
-__device__ __forceinline__ uint32_t other_row(uint32_t v) { const u32x2 r = __builtin_bit_cast(u32x2, __builtin_amdgcn_permlane16_swap(v, v, false, false)); const uint32_t x = r[0], y = r[1]; return (threadIdx.x & 16) ? x : y; }
-__device__ __forceinline__ uint32_t other_half(uint32_t v) { const u32x2 r = __builtin_bit_cast(u32x2, __builtin_amdgcn_permlane32_swap(v, v, false, false)); const uint32_t x = r[0], y = r[1]; return (threadIdx.x & 32) ? x : y; }
-__device__ __forceinline__ float all_max(float v) {
-    v = fmaxf(v, __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0xB1, 0xF, 0xF, true)));
-    v = fmaxf(v, __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x4E, 0xF, 0xF, true)));
-    v = fmaxf(v, __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x141, 0xF, 0xF, true)));
-    v = fmaxf(v, __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x140, 0xF, 0xF, true)));
-    v = fmaxf(v, __builtin_bit_cast(float, other_row(__builtin_bit_cast(uint32_t, v))));
-    return fmaxf(v, __builtin_bit_cast(float, other_half(__builtin_bit_cast(uint32_t, v))));
-}
-template <class F> __device__ __forceinline__ double f64_moved(double v, F && f) {
-    const uint64_t u = __builtin_bit_cast(uint64_t, v);
-    const uint32_t lo = f((uint32_t) u), hi = f((uint32_t) (u >> 32));
-    return __builtin_bit_cast(double, ((uint64_t) hi << 32) | lo);
-}
-__device__ __forceinline__ double all_sum(double v) {
-    v += f64_moved(v, [](uint32_t x) __attribute__((always_inline)) { return (uint32_t) dpp_i<0xB1>((int) x); });
-    v += f64_moved(v, [](uint32_t x) __attribute__((always_inline)) { return (uint32_t) dpp_i<0x4E>((int) x); });
-    v += f64_moved(v, [](uint32_t x) __attribute__((always_inline)) { return (uint32_t) dpp_i<0x141>((int) x); });
-    v += f64_moved(v, [](uint32_t x) __attribute__((always_inline)) { return (uint32_t) dpp_i<0x140>((int) x); });
-    v += f64_moved(v, [](uint32_t x) __attribute__((always_inline)) { return other_row(x); });
-    return v + f64_moved(v, [](uint32_t x) __attribute__((always_inline)) { return other_half(x); });
-}
-
 // ---- up to 64 * KPL cells, four waves per head: every load is issued before anything is computed, ONE barrier. What bounds it is the number of cache lines a CU asks for, so an instruction
 // takes whole lines: K - DH / 8 lanes hold a key's row, a wave 4 keys of head_dim 128 at once; V^T - 8 KPL lanes hold a dimension's cells, eight each. (A key per lane, and a dimension per
 // lane for V - 64 lines an instruction, 8192 for a head of 128 over 256 cells instead of 1024: 7.9 us per launch of 32 heads x 204 cells, now 5.0; 4.3 at 36 cells, now 3.8.)

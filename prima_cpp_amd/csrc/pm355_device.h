@@ -106,6 +106,31 @@ __device__ __forceinline__ float wave_sum(float v) {
     return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), 63));
 }
 
+// ---- reductions whose result every lane of a wave gets, without LDS: 16-lane rows by DPP, then the rows by lane swaps
+__device__ __forceinline__ uint32_t other_row(uint32_t v) { const u32x2 r = __builtin_bit_cast(u32x2, __builtin_amdgcn_permlane16_swap(v, v, false, false)); const uint32_t x = r[0], y = r[1]; return (threadIdx.x & 16) ? x : y; }
+__device__ __forceinline__ uint32_t other_half(uint32_t v) { const u32x2 r = __builtin_bit_cast(u32x2, __builtin_amdgcn_permlane32_swap(v, v, false, false)); const uint32_t x = r[0], y = r[1]; return (threadIdx.x & 32) ? x : y; }
+__device__ __forceinline__ float all_max(float v) {
+    v = fmaxf(v, __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0xB1, 0xF, 0xF, true)));
+    v = fmaxf(v, __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x4E, 0xF, 0xF, true)));
+    v = fmaxf(v, __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x141, 0xF, 0xF, true)));
+    v = fmaxf(v, __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x140, 0xF, 0xF, true)));
+    v = fmaxf(v, __builtin_bit_cast(float, other_row(__builtin_bit_cast(uint32_t, v))));
+    return fmaxf(v, __builtin_bit_cast(float, other_half(__builtin_bit_cast(uint32_t, v))));
+}
+template <class F> __device__ __forceinline__ double f64_moved(double v, F && f) {
+    const uint64_t u = __builtin_bit_cast(uint64_t, v);
+    const uint32_t lo = f((uint32_t) u), hi = f((uint32_t) (u >> 32));
+    return __builtin_bit_cast(double, ((uint64_t) hi << 32) | lo);
+}
+__device__ __forceinline__ double all_sum(double v) {
+    v += f64_moved(v, [](uint32_t x) __attribute__((always_inline)) { return (uint32_t) dpp_i<0xB1>((int) x); });
+    v += f64_moved(v, [](uint32_t x) __attribute__((always_inline)) { return (uint32_t) dpp_i<0x4E>((int) x); });
+    v += f64_moved(v, [](uint32_t x) __attribute__((always_inline)) { return (uint32_t) dpp_i<0x141>((int) x); });
+    v += f64_moved(v, [](uint32_t x) __attribute__((always_inline)) { return (uint32_t) dpp_i<0x140>((int) x); });
+    v += f64_moved(v, [](uint32_t x) __attribute__((always_inline)) { return other_row(x); });
+    return v + f64_moved(v, [](uint32_t x) __attribute__((always_inline)) { return other_half(x); });
+}
+
 // max over aligned groups of 8 lanes, result in all 8 lanes
 __device__ __forceinline__ float group8_max(float v) {
     v = fmaxf(v, dpp_f<0xB1>(v));

@@ -167,8 +167,9 @@ __global__ __launch_bounds__(256) void silu_mul_q80_tab_kernel(const float * __r
 
 // rms_norm (+ weight) fused with Q8_K quantization. One 256-thread workgroup per row.
 // Optionally also writes the normalised f32 row (ynorm != nullptr).
-// NWV waves per row: 4 for many rows (prompts: one small workgroup per row fills the chip), 16 for a handful of rows (decode batches of 2..64
-// tokens are ONE latency chain per row - load, reduce, quantize block after block: with 4 waves a K = 8192 row took 11 us, a fifth of a 2-token layer)
+// NWV waves per row: 4 for many rows (prompts: small workgroups, several per CU), 16 while every row has a CU to itself - the launch is then ONE latency chain per row: load, reduce,
+// quantize block after block. us with 4 / 16 waves, K = 4096: 101 rows 5.1 / 3.9, 256 rows 5.3 / 4.2, 300 rows 5.4 / 6.0; K = 8192: 101 rows 7.9 / 4.9, 256 rows 8.2 / 5.4, 512 rows 9.3 / 8.5,
+// 700 rows 11.1 / 11.4. (8 rows 3.8 -> 3.6 with the sum by DPP and the weights asked for with the row.)
 template <int NWV>
 __global__ __launch_bounds__(64 * NWV) void rmsnorm_q8k_kernel(const float * __restrict__ x, const float * __restrict__ w,
                                                           float * __restrict__ ynorm, uint8_t * __restrict__ yq,
@@ -182,10 +183,15 @@ __global__ __launch_bounds__(64 * NWV) void rmsnorm_q8k_kernel(const float * __r
     // dependent load per block and pass - took 12 us for K = 8192.
     constexpr int HOLD = NWV == 4 ? 8 : 2;
     const bool held = nblk <= NWV * HOLD;
-    float4 f[HOLD];
+    float4 f[HOLD], wt[HOLD];                                          // (a handful of rows: the weights too, behind the sum they were a second round of latency)
+    constexpr bool WT = NWV > 4;
     if (held) {
 #pragma unroll
-        for (int i = 0; i < HOLD; ++i) { const int blk = min(wv + NWV * i, nblk - 1); f[i] = ((const float4 *) (xr + (size_t) blk * PM_QK_K))[lane]; }
+        for (int i = 0; i < HOLD; ++i) {
+            const int blk = min(wv + NWV * i, nblk - 1);
+            f[i] = ((const float4 *) (xr + (size_t) blk * PM_QK_K))[lane];
+            if constexpr (WT) wt[i] = w ? ((const float4 *) (w + (size_t) blk * PM_QK_K))[lane] : make_float4(1.0f, 1.0f, 1.0f, 1.0f);
+        }
     }
     // pass 1: sum of squares; products rounded to f32 like the reference, accumulated in f64 (same order as before: blocks ascending)
     double s = 0.0;
@@ -200,8 +206,7 @@ __global__ __launch_bounds__(64 * NWV) void rmsnorm_q8k_kernel(const float * __r
             s += (double) (g.x * g.x); s += (double) (g.y * g.y); s += (double) (g.z * g.z); s += (double) (g.w * g.w);
         }
     }
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off);
+    s = all_sum(s);
     if (lane == 0) red[wv] = s;
     __syncthreads();
     double tot = (red[0] + red[1]) + (red[2] + red[3]);
@@ -210,10 +215,10 @@ __global__ __launch_bounds__(64 * NWV) void rmsnorm_q8k_kernel(const float * __r
     const float mean  = (float) (tot / K);
     const float scale = 1.0f / sqrtf(mean + eps);
     // pass 2: normalise (+weight), write f32 and/or quantize
-    auto emit = [&](const float4 & fx, int blk) __attribute__((always_inline)) {
+    auto emit = [&](const float4 & fx, int blk, const float4 * held_w = nullptr) __attribute__((always_inline)) {
         float v[4] = {fx.x * scale, fx.y * scale, fx.z * scale, fx.w * scale};
         if (w) {
-            const float4 g = ((const float4 *) (w + (size_t) blk * PM_QK_K))[lane];
+            const float4 g = held_w ? *held_w : ((const float4 *) (w + (size_t) blk * PM_QK_K))[lane];
             v[0] *= g.x; v[1] *= g.y; v[2] *= g.z; v[3] *= g.w;
         }
         if (ynorm) ((float4 *) (ynorm + (size_t) row * K + (size_t) blk * PM_QK_K))[lane] = make_float4(v[0], v[1], v[2], v[3]);
@@ -225,7 +230,7 @@ __global__ __launch_bounds__(64 * NWV) void rmsnorm_q8k_kernel(const float * __r
     };
     if (held) {
 #pragma unroll
-        for (int i = 0; i < HOLD; ++i) if (wv + NWV * i < nblk) emit(f[i], wv + NWV * i);
+        for (int i = 0; i < HOLD; ++i) if (wv + NWV * i < nblk) emit(f[i], wv + NWV * i, WT ? &wt[i] : nullptr);
     } else {
         for (int blk = wv; blk < nblk; blk += NWV) emit(((const float4 *) (xr + (size_t) blk * PM_QK_K))[lane], blk);
     }
@@ -253,6 +258,6 @@ void pm_launch_quantize_q80(const float * x, void * y, int K, int rows, hipStrea
                        x, (uint8_t *) y, K, rows, pm_q80_row_bytes(K));
 }
 void pm_launch_rmsnorm_q8k(const float * x, const float * w, float * ynorm, void * yq, int K, int rows, float eps, hipStream_t st, void * ynorm_f16, pm_q8k_tables tab) {
-    if (rows <= 64) hipLaunchKernelGGL(rmsnorm_q8k_kernel<16>, dim3(rows), dim3(1024), 0, st, x, w, ynorm, (uint8_t *) yq, K, eps, pm_q8k_row_bytes(K), (_Float16 *) ynorm_f16, tab);
+    if (rows <= 256) hipLaunchKernelGGL(rmsnorm_q8k_kernel<16>, dim3(rows), dim3(1024), 0, st, x, w, ynorm, (uint8_t *) yq, K, eps, pm_q8k_row_bytes(K), (_Float16 *) ynorm_f16, tab);
     else            hipLaunchKernelGGL(rmsnorm_q8k_kernel<4>, dim3(rows), dim3(256), 0, st, x, w, ynorm, (uint8_t *) yq, K, eps, pm_q8k_row_bytes(K), (_Float16 *) ynorm_f16, tab);
 }

@@ -1469,3 +1469,17 @@ def test_small_batch_rows_kernel_at_its_edges(P, oracle, t):
         # a token's sums do not depend on the tokens beside it
         one = P.mul_mat_small(w, x=_dev(P, x[T - 1:])).cpu().numpy()
         assert np.array_equal(one[0], y[T - 1]), (K, N, T)
+
+
+@pytest.mark.parametrize("rows,K", [(65, 4096), (256, 8192), (257, 4096), (256, 12288), (2, 256)])
+def test_rms_norm_of_many_rows(P, oracle, rows, K):
+    """16 waves per row up to 256 rows, 4 beyond; rows that fit the registers of either form and rows that do not. The bound of the test of few rows: one unit in the last place (the f64 sum's
+    order), and the quantized rows are those of the values returned."""
+    rng = np.random.default_rng(rows + K)
+    x, w = rng.normal(0, 2, (rows, K)).astype(np.float32), (1 + rng.normal(0, 0.02, K)).astype(np.float32)
+    y, yq = P.rms_norm(_dev(P, x), _dev(P, w), 1e-5, want_f32=True, want_q8=True)
+    got = y.cpu().numpy()
+    at = [0, rows // 2, rows - 1]
+    want = oracle.rms_norm(x[at], w, 1e-5)
+    assert np.abs(got[at].view(np.int32).astype(np.int64) - want.view(np.int32).astype(np.int64)).max() <= 1
+    assert np.array_equal(P.act_to_ggml_blocks(yq, Q8_K, K, rows), P.act_to_ggml_blocks(P.quantize_act(y, Q8_K), Q8_K, K, rows))
