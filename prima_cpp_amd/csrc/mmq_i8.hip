@@ -748,11 +748,11 @@ int launch_q80(const void * W, const void * xq, const float * x_f32, float * Y, 
     const int grid = N / 32 >= cus ? cus : (N + 31) / 32;
     const int rows = (N + grid - 1) / grid, nrg = (rows + 31) / 32;
     const size_t lds = pm_mmq_i8_lds_bytes(PM_Q8_0, K);
-    const int rows_max = pm_mmq_rows_max_tokens(N), tmax = T <= rows_max ? rows_max : 16;   // (the 32-token form spills 236 B: 502 vs 422 us per Qwen2.5-72B layer at 32 tokens - two passes of 16 it is)
+    const int tmax = pm_mmq_rows_takes(PM_Q8_0, N, T) || pm_mmq_rows_takes(PM_Q8_0, N, 32) ? 32 : 16;      // (this file's 32-token form spills 236 B: 502 vs 422 us per Qwen2.5-72B layer at 32 tokens - two passes of 16 it is)
     for (int t0 = 0; t0 < T; t0 += tmax) {
         const int tn = T - t0 < tmax ? T - t0 : tmax;
         uint8_t * tab = base + (t0 / 32) * (qtab + dtab);
-        if (tn <= rows_max) {
+        if (pm_mmq_rows_takes(PM_Q8_0, N, tn)) {
             RowsP q = {};
             q.job[0] = {(const uint8_t *) W, Y + (size_t) t0 * N, bias, resid ? resid + (size_t) t0 * N : nullptr, N};
             q.njobs = 1; q.K = K; q.T = tn; q.t_off = t0 % 32; q.qT = tab; q.dT = (const float *) (tab + qtab);
@@ -835,11 +835,11 @@ int pm_launch_mmq_i8(int type, const void * W, const void * xq, const float * x_
     const int grid = N / 32 >= cus ? cus : (N + 31) / 32;
     const int rows = (N + grid - 1) / grid, nrg = (rows + 31) / 32;
     const size_t lds = pm_mmq_i8_lds_bytes(type, K);
-    const int rows_max = pm_mmq_rows_max_tokens(N), tmax = T <= rows_max ? rows_max : type == PM_Q5_K ? 16 : 32;                    // (Q5_K: 11 weight registers more per step - its 32-token form spills 388 B / lane)
+    const int tmax = type != PM_Q5_K || pm_mmq_rows_takes(type, N, T) || pm_mmq_rows_takes(type, N, 32) ? 32 : 16;                    // (Q5_K: 11 weight registers more per step - its 32-token form here spills 388 B / lane)
     for (int t0 = 0, c = 0; t0 < T; t0 += tmax, ++c) {
         const int tn = T - t0 < tmax ? T - t0 : tmax;
         uint8_t * bsT = sc->p + (t0 / 32) * tab; float * dT = (float *) (bsT + (size_t) nsb * 1024);    // tables are per 32 tokens
-        if (tn <= rows_max) {
+        if (pm_mmq_rows_takes(type, N, tn)) {
             RowsP q = {};
             q.job[0] = {(const uint8_t *) W, Y + (size_t) t0 * N, bias, resid ? resid + (size_t) t0 * N : nullptr, N};
             q.njobs = 1; q.K = K; q.T = tn; q.t_off = t0 % 32; q.qT = sc->p + scr_q_off(K) + (size_t) (t0 / 32) * nsb * 8192; q.bsT = bsT; q.dT = dT;

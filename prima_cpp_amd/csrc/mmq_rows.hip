@@ -1,4 +1,4 @@
-// mmq_rows.hip - quantized mat-mul for 2..8 tokens: weights from memory straight into the operands of v_mfma_i32_16x16x64_i8 / 16x16x32_i8, no LDS on their way.
+// mmq_rows.hip - quantized mat-mul for 2..8 tokens (some shapes and types: up to 32, pm_mmq_rows_takes): weights from memory straight into the operands of v_mfma_i32_16x16x64_i8 / 16x16x32_i8, no LDS on their way.
 //
 // The arithmetic is mmq_i8.hip's (activations in Q8_K / Q8_0 blocks, exact integer sums per super-block, one f32 multiply-add per super-block): what differs is where the bytes go. A workgroup
 // owns a slice of the rows of one matrix, its eight waves share K: a wave takes PAIRS of super-blocks, pair w, w + 8, ..., for all rows of the slice, 16 at a time. So
@@ -93,13 +93,15 @@ template <int TYPE, int NG> __device__ __forceinline__ ASrc source_a(const RowsP
 }
 template <int TYPE> __device__ __forceinline__ void load_q(ASet<TYPE> & a, const ASrc & s, int g, bool last, int pair, int j) {
     const uint32_t o = s.qo[last] + (uint32_t) (128 * g);
-    if constexpr (TYPE == PM_Q8_0) a.q[j] = ld_buf(s.rq, o + (uint32_t) (pair * 8192 + j * 1024), 0);       // (zeros behind the last block of a row, where the tables end)
+    if constexpr (TYPE == PM_Q8_0) a.q[j] = ld_buf(s.rq, o + (uint32_t) (j * 1024), min(pair, (s.n + 7) / 8 - 1) * 8192);
     else a.q[j] = ld_buf(s.rq, o + (uint32_t) ((j & 3) * 1024), first_of(pair, s.n) * 8192 + (j >> 2) * 4096);
 }
 template <int TYPE> __device__ __forceinline__ void load_yd(ASet<TYPE> & a, const ASrc & s, int g, bool last, int pair, int hk) {
     if constexpr (TYPE == PM_Q8_0) {
+        // blocks behind the last one of a row (and pairs behind the last one): scale 0
+        const int pc = min(pair, (s.n + 7) / 8 - 1);
 #pragma unroll
-        for (int j = 0; j < 4; ++j) a.yd[j] = __builtin_bit_cast(f32x4, ld_buf(s.rd, s.dd + (uint32_t) (pair * 1024 + j * 128 + 32 * g), 0));
+        for (int j = 0; j < 4; ++j) a.yd[j] = __builtin_bit_cast(f32x4, ld_buf(s.rd, 8 * pair + 4 * hk + j < s.n ? s.dd + (uint32_t) (j * 128 + 32 * g) : 0x80000000u, pc * 1024));
     } else {
         const int sb = first_of(pair, s.n);
         a.bs = ld_buf(s.rb, s.bo[last] + (uint32_t) (128 * g), sb * 1024);
@@ -488,6 +490,11 @@ __device__ __forceinline__ void rows_body(const RowsP & p, const RowsJob & job, 
 #pragma unroll
                         for (int g = 0; g < NG; ++g) used(g, j);
                 }
+                // (the sums now: sunk behind the requests below, they keep the old activations alive beside the new ones - copies at the end of the step that wait for every request)
+#pragma unroll
+                for (int g = 0; g < NG; ++g)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) { float v = out[r][g][i]; asm volatile("" : "+v"(v)); out[r][g][i] = v; }
                 __builtin_amdgcn_sched_barrier(0);
                 W[d][r].load(ws, off[r], kg, wave + KW * wn.it);
                 __builtin_amdgcn_sched_barrier(0);
@@ -578,10 +585,17 @@ size_t lds_of(int type, int NG, int R, bool AL, int K) {
 
 }  // namespace
 
-// Several groups of eight tokens only where every workgroup has one group of rows: the activations of a K range are then asked for once per workgroup like the weights, and the chip is full (with
-// 32-row groups it is half empty). 16 / 23 tokens, us, mmq_i8.hip / here (4.5 of them the tables): 4096 x 4096 Q4_K 11.4 / 10.3, 13.3 / 11.9; 4096 x 14336 Q4_K 19.3 / 18.7, 23.0 / 21.5, Q6_K 31.8 /
-// 25.8, 39.1 / 29.4. With two groups of rows 8192 x 8192 16.5 / 18.2, 19.4 / 23.9; with four groups of tokens the registers do not hold the activations (29 tokens: 13.4 / 18.5).
-int pm_mmq_rows_max_tokens(int N) { return N <= 16 * pm_device_cus() ? 24 : 8; }
+// Several groups of eight tokens, us, mmq_i8.hip / here (4.5 of them the tables). One group of rows per workgroup (N up to 16 per CU): the activations of a K range are asked for once per workgroup
+// like the weights, and the chip is full (with 32-row groups it is half empty). 16 / 23 tokens: 4096 x 4096 Q4_K 11.4 / 10.3, 13.3 / 11.5; 4096 x 14336 Q4_K 18.8 / 18.0, 22.9 / 20.9, Q6_K 31.6 /
+// 25.1, 39.1 / 28.9. Q4_K and Q6_K stop at 24: with four groups of tokens their registers spill (4096 x 4096 Q4_K 13.4 / 13.8, 4096 x 14336 Q6_K 39.0 / 38.5). With two groups of rows they lose
+// (8192 x 8192 Q4_K at 16 / 23 tokens 16.4 / 17.8, 19.3 / 20.1).
+// Q5_K and Q8_0, which mmq_i8.hip takes 16 tokens at a time, read the weights once here: 32 tokens with one group of rows (1024 x 8192 Q5_K 28.5 / 16.2, Q8_0 28.0 / 20.0; 4096 x 14336 Q5_K 41.9 /
+// 28.2), 17..24 with two (8192 x 29568 Q8_0 117 / 76, 59136 x 8192 192 / 155; 57344 x 8192 Q5_K 153 / 107, 8192 x 8192 35.3 / 23.2); 32 there spill (Q8_0 121 / 95 and 34.5 / 32.7, Q5_K 34 / 270),
+// and up to 16 tokens mmq_i8.hip is as fast or faster (59136 x 8192 Q8_0 105 / 133, 57344 x 8192 Q5_K 79 / 96).
+bool pm_mmq_rows_takes(int type, int N, int T) {
+    const bool one_group = N <= 16 * pm_device_cus(), by16 = type == PM_Q5_K || type == PM_Q8_0;
+    return T <= 8 || (one_group ? T <= (by16 ? 32 : 24) : by16 && T > 16 && T <= 24);
+}
 
 int pm_launch_mmq_rows(RowsP p, const int * types, hipStream_t st) {
     const int cus = pm_device_cus(), n = p.njobs;
@@ -617,13 +631,14 @@ int pm_launch_mmq_rows(RowsP p, const int * types, hipStream_t st) {
                                   switch (big) { case 1: return deep ? PM_ROWS_GO(TA_, TB_, 1, 1, 2, false, E_) : PM_ROWS_GO(TA_, TB_, 1, 1, 1, false, E_); \
                                                  case 2: return deep ? PM_ROWS_GO(TA_, TB_, 1, 2, 2, false, E_) : PM_ROWS_GO(TA_, TB_, 1, 2, 1, false, E_); \
                                                  default: return PM_ROWS_GO(TA_, TB_, 1, 3, 1, false, E_); } }
+#define PM_ROWS_G(T_, G_, R_) go(mmq_rows_kernel<T_, T_, G_, R_, 1, false, false>, lds(G_, R_, false))
     if (ng > 1) {
-        if (n > 1 || big > 1 || ng > 3) return -5;
-        const auto one = [&](auto two, auto three) { return go(ng == 2 ? two : three, lds(ng, 1, false)); };
-        return ta == PM_Q4_K ? one(mmq_rows_kernel<PM_Q4_K, PM_Q4_K, 2, 1, 1, false, false>, mmq_rows_kernel<PM_Q4_K, PM_Q4_K, 3, 1, 1, false, false>)
-             : ta == PM_Q5_K ? one(mmq_rows_kernel<PM_Q5_K, PM_Q5_K, 2, 1, 1, false, false>, mmq_rows_kernel<PM_Q5_K, PM_Q5_K, 3, 1, 1, false, false>)
-             : ta == PM_Q6_K ? one(mmq_rows_kernel<PM_Q6_K, PM_Q6_K, 2, 1, 1, false, false>, mmq_rows_kernel<PM_Q6_K, PM_Q6_K, 3, 1, 1, false, false>)
-             : ta == PM_Q8_0 ? one(mmq_rows_kernel<PM_Q8_0, PM_Q8_0, 2, 1, 1, false, false>, mmq_rows_kernel<PM_Q8_0, PM_Q8_0, 3, 1, 1, false, false>) : -5;
+        if (n > 1 || !pm_mmq_rows_takes(ta, p.job[0].N, p.T)) return -5;
+        if (big > 1) return ta == PM_Q5_K ? PM_ROWS_G(PM_Q5_K, 3, 2) : PM_ROWS_G(PM_Q8_0, 3, 2);
+        if (ta == PM_Q4_K) return ng == 2 ? PM_ROWS_G(PM_Q4_K, 2, 1) : PM_ROWS_G(PM_Q4_K, 3, 1);
+        if (ta == PM_Q6_K) return ng == 2 ? PM_ROWS_G(PM_Q6_K, 2, 1) : PM_ROWS_G(PM_Q6_K, 3, 1);
+        if (ta == PM_Q5_K) return ng == 2 ? PM_ROWS_G(PM_Q5_K, 2, 1) : ng == 3 ? PM_ROWS_G(PM_Q5_K, 3, 1) : PM_ROWS_G(PM_Q5_K, 4, 1);
+        return ng == 2 ? PM_ROWS_G(PM_Q8_0, 2, 1) : ng == 3 ? PM_ROWS_G(PM_Q8_0, 3, 1) : PM_ROWS_G(PM_Q8_0, 4, 1);
     }
     if (p.e_on) {
         if (ta == PM_Q4_K && tb == PM_Q4_K) PM_ROWS_R(PM_Q4_K, PM_Q4_K, true)
@@ -639,6 +654,7 @@ int pm_launch_mmq_rows(RowsP p, const int * types, hipStream_t st) {
     if (ta == PM_Q4_K && tb == PM_Q6_K) PM_ROWS_R(PM_Q4_K, PM_Q6_K, false)
     if (ta == PM_Q4_K && tb == PM_Q5_K) PM_ROWS_R(PM_Q4_K, PM_Q5_K, false)
 #undef PM_ROWS_R
+#undef PM_ROWS_G
 #undef PM_ROWS_GO
     return -5;
 }

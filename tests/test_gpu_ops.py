@@ -1451,7 +1451,8 @@ def test_small_batch_rows_kernel_at_its_edges(P, oracle, t):
     tail = 32 if t == Q8_0 else 256
     for K, N, T in ((512, 1, 8), (512, 15, 1), (768, 16, 2), (2048, 17, 3), (4096, 33, 4), (4096 + tail, 100, 5), (4352, 4096, 7), (4608, 4097, 8), (8192 + tail, 8192 + 31, 6), (1024, 12300, 8), (768, 28700, 3),
                     (8192, 12290, 2), (12288, 16390, 8),
-                    (512, 16, 17), (768, 4096, 16), (4096 + tail, 33, 9), (4608, 100, 24), (14336, 4095, 23)):     # (up to 24 tokens where a workgroup has one group of rows)
+                    (512, 16, 17), (768, 4096, 16), (4096 + tail, 33, 9), (4608, 100, 24), (14336, 4095, 23),      # (up to 24 tokens where a workgroup has one group of rows)
+                    (512, 40, 25), (4096 + tail, 4096, 32), (768, 17, 61), (4352, 8191, 17), (512, 4097, 24), (8192 + tail, 8230, 23)):     # (Q5_K, Q8_0: up to 32, and 17..24 with two and more)
         b = rand_blocks(t, N, K, rng)
         x = rng.normal(0, 1, (T, K)).astype(np.float32)
         bias, resid = rng.normal(0, 1, N).astype(np.float32), rng.normal(0, 1, (T, N)).astype(np.float32)
@@ -1466,9 +1467,10 @@ def test_small_batch_rows_kernel_at_its_edges(P, oracle, t):
         xq = P.quantize_act(_dev(P, x), P.vec_dot_act_type(t))
         y2 = P.mul_mat_small(w, xq=xq, n_tokens=T, bias=_dev(P, bias), resid=_dev(P, resid)).cpu().numpy()
         assert np.array_equal(y2, (y + bias[None]) + resid), (K, N, T)
-        # a token's sums do not depend on the tokens beside it
-        one = P.mul_mat_small(w, x=_dev(P, x[T - 1:])).cpu().numpy()
-        assert np.array_equal(one[0], y[T - 1]), (K, N, T)
+        # a token's sums do not depend on the tokens beside it (but for Q4_K and Q6_K of more tokens, which mmq_i8.hip takes)
+        if T <= 24 and N <= 4096 or T <= 8 or t in (Q5_K, Q8_0):
+            one = P.mul_mat_small(w, x=_dev(P, x[T - 1:])).cpu().numpy()
+            assert np.array_equal(one[0], y[T - 1]), (K, N, T)
 
 
 @pytest.mark.parametrize("rows,K", [(65, 4096), (256, 8192), (257, 4096), (256, 12288), (2, 256)])
