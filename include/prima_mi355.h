@@ -212,6 +212,12 @@ PM355_API int pm355_mul_mat_q_small_multi(int type, int njobs, const void * cons
  * (llama_tensor_get_type, src/llama.cpp:19447) - as ONE grid whose workgroups are divided by weight bytes. PM355_E_UNSUPPORTED: launch the jobs separately. */
 PM355_API int pm355_mul_mat_q_small_mixed(const int * types, int njobs, const void * const * W, const int64_t * N, float * const * y,
                                           const float * const * bias, const void * xq, int64_t K, int64_t n_tokens, pm355_stream_t stream);
+/* The same arithmetic for up to 512 tokens on the prompt GEMM's tiles (prima_cpp_amd/csrc/mmq_pf.hip), what batches of several sequences' short portions take: 1..3 Q4_K / Q5_K / Q6_K matrices
+ * of at most two types over f32 activations x [n_tokens][K], K % 256 == 0, N % 4 == 0. pair != 0: two matrices of one type and shape, y[1] = silu(W[0] x) * (W[1] x). scratch: device memory of
+ * pm355_mul_mat_q_wide_scratch(K) bytes, 16-byte aligned. */
+PM355_API int pm355_mul_mat_q_wide(const int * types, int njobs, const void * const * W, const int64_t * N, float * const * y, const float * const * bias, const float * const * resid,
+                                   const float * x, int64_t K, int64_t n_tokens, int pair, void * scratch, pm355_stream_t stream);
+PM355_API int64_t pm355_mul_mat_q_wide_scratch(int64_t K);
 /* test hook: additionally writes, per (row, unit), the exact int32 pair {sum scale*q_w*q_a, sum min*bsum} */
 PM355_API int pm355_mul_mat_vec_q_dbg(int type, const void * W, int64_t K, int64_t N, const void * xq, float * y,
                                       int32_t * int_partials, int64_t * units_per_row, pm355_stream_t stream);

@@ -251,6 +251,24 @@ int pm355_mul_mat_q_small_mixed(const int * types, int njobs, const void * const
     HIP_TRY(hipGetLastError());
     return 0;
 }
+int64_t pm355_mul_mat_q_wide_scratch(int64_t K) { return K < 256 || K % 256 ? 0 : (int64_t) pm_q8k_wide_bytes((int) K); }
+int pm355_mul_mat_q_wide(const int * types, int njobs, const void * const * W, const int64_t * N, float * const * y, const float * const * bias, const float * const * resid,
+                         const float * x, int64_t K, int64_t n_tokens, int pair, void * scratch, pm355_stream_t st) {
+    (void) hipGetLastError();
+    if (njobs < 1 || njobs > 3 || !types || !W || !N || !y || !x || !scratch || K < 512 || K % 256 || n_tokens < 1 || n_tokens > PM_WIDE_MAX_TOKENS)
+        return fail(PM355_E_RANGE, "mul_mat_q_wide: 1..3 jobs, 1..512 tokens, K a multiple of 256");
+    pm_gemm_pf_job j[3] = {};
+    for (int i = 0; i < njobs; ++i) {
+        j[i].type = types[i]; j[i].N = (int) N[i]; j[i].W = W[i]; j[i].Y = y[i]; j[i].bias = bias ? bias[i] : nullptr; j[i].resid = resid ? resid[i] : nullptr;
+        if (pm_gemm_wide_check(types[i], (int) K, (int) N[i], (int) n_tokens)) return fail(PM355_E_UNSUPPORTED, "mul_mat_q_wide: Q4_K / Q5_K / Q6_K, N a multiple of 4");
+    }
+    const pm_q8k_wide a = pm_q8k_wide_at(scratch, (int) K);
+    pm_launch_quantize_wide(x, a, (int) K, (int) n_tokens, S(st));
+    const int rc = pm_launch_gemm_wide(j, njobs, a, (int) K, (int) n_tokens, pair, S(st));
+    if (rc) return fail(rc == -3 ? PM355_E_HIP : PM355_E_UNSUPPORTED, "mul_mat_q_wide: more than two types, or jobs that are no pair");
+    HIP_TRY(hipGetLastError());
+    return 0;
+}
 int pm355_gemm_plan(int64_t n_row_tiles, int64_t K, int64_t n_tokens, int n_cus, int allow_tail_split, int32_t * out5) {
     if (n_row_tiles < 1 || K < 256 || n_tokens < 1 || n_cus < 8 || !out5) return fail(PM355_E_RANGE, "gemm_plan: n_row_tiles >= 1, K >= 256, n_tokens >= 1, n_cus >= 8");
     pm_gemm_pf_plan_t pl;

@@ -109,8 +109,9 @@ struct pm_window : pm355_model {
     // a pass over rows of several sequences (batch): every row's position and sequence in device memory; rag is set while one is launched. Attention: rows [0, n_rows) see at most max_cells
     // cells and have a workgroup per head and row, the last n_long rows (sequence and position on the host too) a key-split launch each, the rows between are the first n_tiles tiles of the
     // matrix-core kernel (all_tiles: those of all rows)
-    struct Ragged { const int32_t * pos, * seq, * tiles; int n_tiles, all_tiles, tile_q, n_rows, max_cells, n_long; const int32_t * h_pos, * h_seq; };
+    struct Ragged { const int32_t * pos, * seq, * tiles; int n_tiles, all_tiles, tile_q, n_rows, max_cells, n_long; const int32_t * h_pos, * h_seq; bool wide; };
     const Ragged * rag = nullptr; int32_t * d_rows = nullptr; float * head_lg = nullptr;
+    uint8_t * wide = nullptr;                     // activations of a wide pass (wide_path)
     uint64_t * am_part = nullptr;                 // argmax scratch of up to HEAD_ROWS rows: one user at a time, like the window's activations
     struct Advance { int by, rotate; };           // what the launch that ends a step still does to the position counters (step_body; the argmax does it on its way and clears this)
     int batch_rows(const pm355_batch_entry * e, int n, float * d_logits, int32_t * d_argmax, hipStream_t st, bool * served);
@@ -639,6 +640,18 @@ bool small_path(const pm_window * m, const Layer & L, int T) {
     return ok;
 }
 
+// passes of up to PM_WIDE_MAX_TOKENS rows with a small batch's arithmetic: every matrix is of a type that the wide product takes
+bool wide_path(const pm_window * m) {
+    if (m->no_fuse || m->no_mmq || MMQ_MAX_TOKENS >= PM_WIDE_MAX_TOKENS || !pm_gemm_pf_enabled()) return false;
+    for (const Layer & L : m->layers) {
+        for (int k : {PM355_T_WQ, PM355_T_WK, PM355_T_WV, PM355_T_WO, PM355_T_FFN_GATE, PM355_T_FFN_UP, PM355_T_FFN_DOWN})
+            if (pm_gemm_wide_check(L.t[k].type, (int) L.t[k].K, (int) L.t[k].N, 1)) return false;
+        const Tensor & q = L.t[PM355_T_WQ], & k = L.t[PM355_T_WK], & v = L.t[PM355_T_WV], & g = L.t[PM355_T_FFN_GATE], & u = L.t[PM355_T_FFN_UP];
+        if ((q.type != k.type && q.type != v.type && k.type != v.type) || g.type != u.type || g.N != u.N) return false;
+    }
+    return true;
+}
+
 // x_in -> x_out for layers [lo, hi); positions from device memory d_pos (pos of token 0)
 int run_window(pm_window * m, const int32_t * d_tokens, const float * d_x_in, int T, float * d_x_out,
                float * d_logits, int32_t * d_argmax, hipStream_t st, pm_window::Advance * adv = nullptr) {
@@ -755,6 +768,34 @@ int run_window(pm_window * m, const int32_t * d_tokens, const float * d_x_in, in
             pm_launch_silu_mul_q8k(m->h, m->h2, m->aq_k, F, T, st, TB(F));                   // silu(gate) * up straight into ffn_down's Q8_K rows
             float * x_next = (il == m->hi - 1 && d_x_out) ? d_x_out : ((x_mid == bufs[0]) ? bufs[1] : bufs[0]);
             if (GI(L.t[PM355_T_FFN_DOWN], x_next, nullptr, x_mid)) return seterr(m, PM355_E_UNSUPPORTED, "prefill: down mat-mul");
+            layer_release(m, il, st);
+            cur = x_next;
+            continue;
+        }
+        if (rg && rg->wide) {
+            // ---- rows of short portions, more than a small batch takes: 8-bit activations through the prompt GEMM's tiles
+            pm_gemm_pf_job j[3] = {};
+            auto job = [&](int i, int kind, float * y, int bias, const float * resid) {
+                const Tensor & w = L.t[kind];
+                j[i].type = w.type; j[i].N = (int) w.N; j[i].W = w.d; j[i].Y = y; j[i].bias = bias < 0 ? nullptr : (const float *) L.t[bias].d; j[i].resid = resid;
+            };
+            const pm_q8k_wide xe = pm_q8k_wide_at(m->wide, E), xa = pm_q8k_wide_at(m->wide, Eq), xf = pm_q8k_wide_at(m->wide, F);
+            float * x_mid = (cur == bufs[0]) ? bufs[1] : bufs[0];
+            float * x_next = (il == m->hi - 1 && d_x_out) ? d_x_out : ((x_mid == bufs[0]) ? bufs[1] : bufs[0]);
+            pm_launch_rmsnorm_wide(cur, (const float *) L.t[PM355_T_ATTN_NORM].d, xe, E, T, hp.rms_eps, st);
+            job(0, PM355_T_WQ, m->q, PM355_T_BQ, nullptr); job(1, PM355_T_WK, m->k, PM355_T_BK, nullptr); job(2, PM355_T_WV, m->v, PM355_T_BV, nullptr);
+            if (pm_launch_gemm_wide(j, 3, xe, E, T, 0, st)) return seterr(m, PM355_E_UNSUPPORTED, "batch: qkv mat-mul");
+            rope_store(L, 1);
+            if (attend_ragged(L)) return seterr(m, PM355_E_RANGE, "batch: n_ctx too large for the attention kernels");
+            pm_launch_quantize_wide(m->att, xa, Eq, T, st);
+            job(0, PM355_T_WO, x_mid, -1, cur);
+            if (pm_launch_gemm_wide(j, 1, xa, Eq, T, 0, st)) return seterr(m, PM355_E_UNSUPPORTED, "batch: wo mat-mul");
+            pm_launch_rmsnorm_wide(x_mid, (const float *) L.t[PM355_T_FFN_NORM].d, xe, E, T, hp.rms_eps, st);
+            job(0, PM355_T_FFN_GATE, nullptr, -1, nullptr); job(1, PM355_T_FFN_UP, m->h, -1, nullptr);
+            if (pm_launch_gemm_wide(j, 2, xe, E, T, 1, st)) return seterr(m, PM355_E_UNSUPPORTED, "batch: gate/up mat-mul");
+            pm_launch_quantize_wide(m->h, xf, F, T, st);
+            job(0, PM355_T_FFN_DOWN, x_next, -1, x_mid);
+            if (pm_launch_gemm_wide(j, 1, xf, F, T, 0, st)) return seterr(m, PM355_E_UNSUPPORTED, "batch: down mat-mul");
             layer_release(m, il, st);
             cur = x_next;
             continue;
@@ -977,7 +1018,7 @@ pm_window::~pm_window() {
     for (auto & L : m->layers) { for (auto & t : L.t) if (t.d) (void) hipFree(t.d); if (L.kc) (void) hipFree(L.kc); if (L.vc) (void) hipFree(L.vc); }
     Tensor * g[4] = {&m->tok_embd, &m->out_norm, &m->output, &m->rope_freqs};
     for (auto t : g) if (t->d) (void) hipFree(t->d);
-    void * s[] = {m->x, m->x1, m->q, m->k, m->v, m->att, m->h, m->h2, m->logits, m->xn, m->aq_k, m->aq_0, m->d_pos, m->d_tok, m->d_ctl, m->split_scratch, m->rope_tab, m->tab_big, m->ss, m->att_tk, m->d_last, m->rows, m->d_rows, m->head_lg, m->am_part};
+    void * s[] = {m->x, m->x1, m->q, m->k, m->v, m->att, m->h, m->h2, m->logits, m->xn, m->aq_k, m->aq_0, m->d_pos, m->d_tok, m->d_ctl, m->split_scratch, m->rope_tab, m->tab_big, m->ss, m->att_tk, m->d_last, m->rows, m->d_rows, m->head_lg, m->wide, m->am_part};
     for (auto p : s) if (p) (void) hipFree(p);
     pm355_uploader_free(m->up);
     if (m->cap_stream) (void) hipStreamDestroy(m->cap_stream);
@@ -1304,8 +1345,10 @@ int pm_window::finalize_pool(int max_tokens_, int n_seq_, int64_t pool_tokens) {
     const int rc = finalize(max_tokens_, n_seq_);
     if (rc) return rc;
     const size_t T = max_tokens;
-    for (void * p : {(void *) rows, (void *) d_rows, (void *) head_lg}) if (p) (void) hipFree(p);
-    rows = head_lg = nullptr; d_rows = nullptr;
+    for (void * p : {(void *) rows, (void *) d_rows, (void *) head_lg, (void *) wide}) if (p) (void) hipFree(p);
+    rows = head_lg = nullptr; d_rows = nullptr; wide = nullptr;
+    if (max_tokens > MMQ_MAX_TOKENS && wide_path(this) &&
+        hipMalloc((void **) &wide, pm_q8k_wide_bytes(std::max({hp.n_embd, hp.head_dim * hp.n_head, hp.n_ff}))) != hipSuccess) return seterr(this, PM355_E_NOMEM, "finalize_pool: activations");
     // (tables of a pass, pm_launch_batch_rows: 3 integers per row, 4 per tile, 2 per sequence, 1 per wanted row, 2 per kept token)
     return hipMalloc((void **) &rows, T * hp.n_embd * 4 + 256) == hipSuccess && hipMalloc((void **) &d_rows, 12 * T * 4 + 256) == hipSuccess &&
            hipMalloc((void **) &head_lg, (size_t) std::min(max_tokens, HEAD_ROWS) * hp.n_vocab * 4 + 256) == hipSuccess ? 0 : seterr(this, PM355_E_NOMEM, "finalize_pool: hidden rows");
@@ -1327,7 +1370,7 @@ int pm_window::pool_info(pm355_pool_info * o) {
     return 0;
 }
 // All entries as rows of common passes: the weights are read once per pass instead of once per sequence (eight sequences of the 8B shape, eight layers and
-// head: prompts of 12..24 tokens and twelve steps 47.0 ms one sequence after another, 14.0 ms as common passes). A portion keeps the arithmetic that it has alone - up to 32 tokens 8-bit
+// head: prompts of 12..24 tokens and twelve steps 47.0 ms one sequence after another, 9.8 ms as common passes). A portion keeps the arithmetic that it has alone - up to 32 tokens 8-bit
 // activations, beyond 16-bit ones; up to 15 where a layer has no 8-bit path, and between the two either, layer by layer - whatever shares the step with it: portions meet in passes of
 // their own tier, the longer ones (a sequence's first) first, and the attention of a portion is chosen by the cells that it attends itself. served = false and nothing done where a pass does
 // not take rows of several sequences.
@@ -1342,11 +1385,11 @@ int pm_window::batch_rows(const pm355_batch_entry * e, int n, float * d_logits, 
     for (int t : {every ? 0 : SMALL_PLAIN_MAX, any ? MMQ_MAX_TOKENS : 0, max_tokens}) if (t > (tier.empty() ? 0 : tier.back()) && (tier.empty() || tier.back() < max_tokens)) tier.push_back(std::min(t, max_tokens));
     enum { ROWS, TILES, LONG };                                                                            // attention, in the order of a pass's rows
     struct Piece { int entry, off, T, pos0, out0, att; };                                                  // tokens [off, off + T) of an entry, whose first wanted row is out0
-    struct Pass { std::vector<Piece> piece; int cap = 0, T = 0; };
+    struct Pass { std::vector<Piece> piece; int cap = 0, T = 0; bool wide = false; };
     // attention of a portion of T tokens: one pass over the keys on the matrix cores, or a workgroup per head and token (whose scores are in LDS: 4 bytes a cell). Alone, 16 tokens and more take
     // the matrix cores behind any history, and a single one behind 320 cells: they then round the probabilities in front of their division where a shared pass rounds behind it, or the other
     // way round, 2^-11 of each. Held to the same kernel here, short prompts pay for it (eight prompts of 12..24 tokens of the 8B shape: a tile launch of 8.5 us where the rows take 4; with twelve
-    // steps behind 13.41 instead of 13.22 ms)
+    // steps behind 13.41 instead of 13.22 ms; in a wide pass 9.73 instead of 9.77)
     auto in_tiles = [&](int T, int past) { return past + T > 32768 || (SMALL_ATTN_ENV ? small_attn_mfma(T, past) : past + T >= SMALL_ATTN_MFMA_CELLS); };
     std::vector<Pass> passes;
     for (int tr = (int) tier.size() - 1; tr >= 0; --tr) {
@@ -1355,14 +1398,18 @@ int pm_window::batch_rows(const pm355_batch_entry * e, int n, float * d_logits, 
         int64_t total = 0;
         for (int i = 0; i < n; ++i)
             for (int off = 0; off < e[i].n_tokens; off += max_tokens) { const int T = std::min(max_tokens, e[i].n_tokens - off); if (mine(T)) total += T; }
-        const int64_t k = (total + most - 1) / most;                                                       // passes of equal size: more than `above` rows, like every portion of the tier
+        // rows of short portions that need more than one small pass go out as wide ones. Prompts of two layers, us, small passes / wide: 8B shape, 40 rows in all 530 / 416, 80 904 / 553, 192 1808 / 795,
+        // Q6_K 679 / 451, 1120 / 590, 2211 / 878; 70B shape 1087 / 917, 1818 / 1247, 3578 / 1976, Q6_K 1394 / 1018, 2252 / 1380, 4407 / 2225 (192 rows as two passes of 96: 1069 on the 8B shape)
+        const bool wd = wide && every && most == MMQ_MAX_TOKENS && total > most;
+        const int cap = wd ? std::min(max_tokens, PM_WIDE_MAX_TOKENS) : most;
+        const int64_t k = (total + cap - 1) / cap;                                                         // passes of equal size: more than `above` rows, like every portion of the tier
         int64_t at = 0;
         for (int i = 0, out0 = 0; i < n; out0 += e[i].n_want, ++i)
             for (int p0 = 0; p0 < e[i].n_tokens; p0 += max_tokens) {
                 const int p1 = std::min(p0 + max_tokens, e[i].n_tokens), past = h_pos[e[i].seq];
                 if (!mine(p1 - p0)) continue;
                 for (int off = p0; off < p1;) {
-                    if (!at || passes.back().T == passes.back().cap) { passes.emplace_back(); passes.back().cap = (int) (total * (at + 1) / k - total * at / k); ++at; }
+                    if (!at || passes.back().T == passes.back().cap) { passes.emplace_back(); passes.back().cap = (int) (total * (at + 1) / k - total * at / k); passes.back().wide = wd; ++at; }
                     Pass & p = passes.back();
                     const int T = std::min(p.cap - p.T, p1 - off);
                     p.piece.push_back({i, off, T, past + off, out0, in_tiles(p1 - p0, past + p0) ? TILES : ROWS});
@@ -1446,7 +1493,7 @@ int pm_window::batch_rows(const pm355_batch_entry * e, int n, float * d_logits, 
         const int at_keep = put(keep.data(), keep.size());
         const pm_batch_layout lay = {T, at_seq, at_ent, (int) ent.size() / 2, (int) blk.size(), e[n - 1].seq};
         pm_launch_batch_rows(d_rows, blk.data(), lay, d_last, d_pos, d_ctl, st);
-        const Ragged r = {d_rows + at_pos, d_rows + at_seq, d_rows + at_tiles, n_tiles, (int) tl.size(), tile_q, n_rows, max_cells, n_long, pos.data(), seq.data()};
+        const Ragged r = {d_rows + at_pos, d_rows + at_seq, d_rows + at_tiles, n_tiles, (int) tl.size(), tile_q, n_rows, max_cells, n_long, pos.data(), seq.data(), p.wide};
         int rc;
         if (T == 1) {                                                                                      // (one row is a step of its own, and that sequence's)
             rc = decode(seq[0], d_rows, nullptr, 1, pos[0], W ? rows : nullptr, nullptr, nullptr, st);

@@ -43,7 +43,10 @@ struct PfJob {
     const uint8_t * W; float * Y; _Float16 * Yh; const float * bias; const float * resid; const float * silu_gate;
     long row_stride, ldy; int type, N, tile0;      // tile0: this job's first row tile in the launch's numbering of row tiles
 };
-struct PfP { PfJob job[PF_MAX_JOBS]; int njobs, nt_n, nt_t; const _Float16 * Xh; int K, T; int grp, pair; int splitk, full; float * ws; unsigned * cnt; unsigned long long * trace; };
+struct PfP {
+    PfJob job[PF_MAX_JOBS]; int njobs, nt_n, nt_t; const _Float16 * Xh; int K, T; int grp, pair; int splitk, full; float * ws; unsigned * cnt; unsigned long long * trace;
+    const uint8_t * Xd, * Xs; int ldt;               // 8-bit activations (pm_q8k_wide): scales, group sums
+};
 // Ablations (measurement builds only: -DPM_GEMM_ABLATE=1 adds instantiations of the Q4_K 256-token kernel, PM355_GEMM_EXP=<bits> picks one; results are WRONG when set):
 // 1 no activation DMA, 2 no weight DMA, 4 no vmcnt wait / barrier, 8 no B fragment reads, 16 no dequantization, 32 no MFMA, 64 no stores;
 // 128: s_memtime stamps of super-block 5's second k-step (waves 0 and 4 of workgroup 0), printed by the launcher: the phase timeline
@@ -76,7 +79,7 @@ template <int TYPE> constexpr int pf_wave_bytes() { return 2 * PfT<TYPE>::NSTREA
 
 // 8 weights -> one A operand: 16-k slice j of 64-k step ks (may be a run-time value) of 128-k piece mm of a super-block. Written stage by stage over the four independent half2
 // chains (and - perm - add - fma): a dependent vector instruction issues ~8-10 cycles after its producer, four chains side by side hide that
-template <int TYPE> __device__ __forceinline__ half8 pf_dequant(const u32x2 ql, const u32x2 qh, const int mm, const int ks, const int j, const half2v mul, const half2v add) {
+template <int TYPE> __device__ __forceinline__ half8 pf_dequant(const u32x2 ql, const u32x2 qh, const int mm, const int ks, const int j, const half2v mul, const half2v add, half8 * low = nullptr) {
     uint32_t v[2];
     half2v t[4];
     if (TYPE == PM_Q8_0) {
@@ -125,8 +128,14 @@ template <int TYPE> __device__ __forceinline__ half8 pf_dequant(const u32x2 ql, 
         for (int c = 0; c < 2; ++c) { t[2 * c] = h2(__builtin_amdgcn_perm(0x64646464u, v[c], 0x05010400u)); t[2 * c + 1] = h2(__builtin_amdgcn_perm(0x64646464u, v[c], 0x07030602u)); }
 #pragma unroll
         for (int c = 0; c < 4; ++c) t[c] = t[c] + bias;
+        half2v q[4];
 #pragma unroll
-        for (int c = 0; c < 4; ++c) t[c] = t[c] * mul;
+        for (int c = 0; c < 4; ++c) { q[c] = t[c]; t[c] = t[c] * mul; }
+        if (low) {                                             // what the rounded products are off by
+#pragma unroll
+            for (int c = 0; c < 4; ++c) q[c] = pk_fma(q[c], mul, -t[c]);
+            *low = __builtin_bit_cast(half8, u32x4{u2(q[0]), u2(q[1]), u2(q[2]), u2(q[3])});
+        }
     }
     return __builtin_bit_cast(half8, u32x4{u2(t[0]), u2(t[1]), u2(t[2]), u2(t[3])});
 }
@@ -484,14 +493,26 @@ __device__ __forceinline__ void pf_body(const PfP & p, const PfJob & jb, const i
 // Llama-3-8B's launches at 101 tokens, Q4_K, us before / now: wq | wk | wv 37 / 24, wo 34 / 23, ffn_gate | ffn_up 61 / 50, ffn_down 54 / 36.6. Taken back: 64 rows and a quarter of the
 // k per wave (half the LDS reads: no change, 1-2 us more for the longer merge); two activation buffers instead of three (2-10 % slower).
 template <int TYPE> constexpr int mid_slot() { return TYPE == PM_Q8_0 ? 4096 : PfT<TYPE>::NSTREAM * 1024; }           // 128 k of 32 rows
-template <int TYPE> constexpr int mid_ahead() { return TYPE == PM_Q8_0 ? 2 : TYPE == PM_Q6_K ? 3 : 4; }               // weights are requested this many steps ahead (what LDS has room for)
-template <int TYPE> constexpr int mid_group_bytes() { return (mid_ahead<TYPE>() + 1) * mid_slot<TYPE>() + 2048 + (TYPE == PM_Q5_K ? 4096 : TYPE == PM_Q6_K ? 1024 : 0); }   // + four headers, four qh, two groups of d
+// weights are requested this many steps ahead (what LDS has room for)
+template <int TYPE, bool EX> constexpr int mid_ahead() { return TYPE == PM_Q8_0 || (EX && TYPE == PM_Q5_K) ? 2 : TYPE == PM_Q6_K ? 3 : 4; }
+template <int TYPE, bool EX> constexpr int mid_group_bytes() { return (mid_ahead<TYPE, EX>() + 1) * mid_slot<TYPE>() + 2048 + (TYPE == PM_Q5_K ? 4096 : TYPE == PM_Q6_K ? 1024 : 0); }   // + four headers, four qh, two groups of d
+// EX, per super-block: 16 group sums (not for Q6_K: no minima) and a scale of every token, two buffers
+template <int TYPE, int NT> constexpr int mid_sum_bytes() { return TYPE == PM_Q6_K ? 0 : NT * 32 * 32; }
+template <int TYPE, int NT, bool EX> constexpr size_t mid_lds_bytes() { return (size_t) 6 * NT * 32 * 128 + (size_t) 4 * mid_group_bytes<TYPE, EX>() + (EX ? 2 * (mid_sum_bytes<TYPE, NT>() + NT * 32 * 4) : 0); }
 template <int N> __device__ __forceinline__ void mid_wait() { asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" : : "n"(N) : "memory"); }
 
-template <int TYPE, int NT>
+// EX - 8-bit activations (Q8_K blocks), the sums of mmq_i8.hip: what the matrix cores add up over a super-block are whole numbers. B = the 8-bit values as F16, A = quant x 6-bit sub-block scale
+// as F16 (Q4_K at most 945, Q5_K 1953: exact; Q6_K up to 4096: the rounded product and what it is off by, two products), and an f32 accumulator holds whole numbers up to 2^24 exactly - where
+// int32 sums are rounded too when they become f32. A super-block's sum is then multiplied by d of the row and d of the token and added in f32, the minima (one product: 16 group sums x
+// minima) by dmin. Against an integer GEMM: scales per 32 k applied to int32 results cost as much vector work as the products take, and scales inside 8-bit operands two products per
+// sub-block (mmq_big.hip); here scale and quant share the multiply that the F16 form needs anyway.
+// Bound by the LDS-DMA like the F16 form, by the vector work at a super-block's end (3 x 16 instructions per 32 tokens, registers 126 -> 240) and, Q6_K, by twice the products. 8B shape, 169 tokens,
+// us: ffn_gate | ffn_up 121 (six passes of 28 on mmq_i8.hip 26.6 each), wo and ffn_down Q4_K 41 on average (14.5 each), ffn_down Q6_K 72 (35 each), wq | wk | wv 37.
+template <int TYPE, int NT, bool EX>
 __device__ __forceinline__ void mid_body(const PfP & p, const PfJob & jb, const int n0, const int t0, uint8_t * smem, const int role, const int ks, const int S, const int tile_id) {
     constexpr int HB = NT * 32 * 128, BBUF = 2 * HB;           // activations: 32 NT tokens x 64 halfs, two of them per step
-    constexpr int SLOT = mid_slot<TYPE>(), AG = mid_group_bytes<TYPE>(), NH = NT / 2, AHEAD = mid_ahead<TYPE>(), HDR = (AHEAD + 1) * SLOT, XTRA = HDR + 2048;
+    constexpr int SLOT = mid_slot<TYPE>(), AG = mid_group_bytes<TYPE, EX>(), NH = NT / 2, AHEAD = mid_ahead<TYPE, EX>(), HDR = (AHEAD + 1) * SLOT, XTRA = HDR + 2048;
+    constexpr int XS = 3 * BBUF + 4 * AG, XSUM = mid_sum_bytes<TYPE, NT>(), XB = XSUM + NT * 32 * 4, XN = EX ? XSUM ? 2 : 1 : 0;      // EX: sums and scales; requests for them per super-block
     constexpr bool K45 = TYPE == PM_Q4_K || TYPE == PM_Q5_K, Q8 = TYPE == PM_Q8_0;
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), g = wave & 3, kk = wave >> 2;       // (waves w and w + 4 share a SIMD)
@@ -541,10 +562,16 @@ __device__ __forceinline__ void mid_body(const PfP & p, const PfJob & jb, const 
 #pragma unroll
         for (int v = 0; v < NH; ++v) { const int q = NH * u + v; dma16(Xg, xsrc[q] + sc * 256u, lds0 + bb + (q / NT) * HB + (g + 4 * (q % NT)) * 1024); }
     };
+    auto issue_X = [&](int b) __attribute__((always_inline)) {     // a quarter of a super-block's sums and scales per wave
+        const uint32_t at = (uint32_t) min(b, nb - 1) * (uint32_t) p.ldt + (uint32_t) t0, dst = lds0 + (uint32_t) (XS + (b & 1) * XB);
+        if (XSUM && lane < 16 * NT) dma16(p.Xs, at * 32u + (uint32_t) (g * 256 * NT + lane * 16), dst + (uint32_t) (g * 256 * NT));
+        if (lane < 2 * NT) dma16(p.Xd, at * 4u + (uint32_t) (g * 32 * NT + lane * 16), dst + (uint32_t) (XSUM + g * 32 * NT));
+    };
     // end of an even / odd step: the next one's weights (all but those of the AHEAD - 1 steps behind it) and activations are there, this wave's LDS reads are through
     auto settle = [&](bool even) __attribute__((always_inline)) {
         constexpr int W = SLOT / 1024, E = TYPE == PM_Q5_K || TYPE == PM_Q6_K ? 2 : 1;
-        if (kk) mid_wait<2 * NT>();
+        if (kk && even) mid_wait<2 * NT + XN>();
+        else if (kk) mid_wait<2 * NT>();
         else if (even) mid_wait<(AHEAD - 1) * W + AHEAD / 2 * E>();
         else mid_wait<(AHEAD - 1) * W + (AHEAD - 1) / 2 * E>();
         __builtin_amdgcn_s_barrier();
@@ -555,10 +582,16 @@ __device__ __forceinline__ void mid_body(const PfP & p, const PfJob & jb, const 
     for (int jt = 0; jt < NT; ++jt)
 #pragma unroll
         for (int e = 0; e < 16; ++e) acc[jt][e] = 0.0f;
+    float16v run[EX ? NT : 1];
+    if (EX)
+#pragma unroll
+        for (int jt = 0; jt < NT; ++jt)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) run[jt][e] = 0.0f;
     // the 4 slices of this wave's half of the step in buffer bb / slot sl: 128-k half mm of super-block b
     // a quarter of the step's requests behind each slice's MFMAs (an issue blocks the wave for 60-180 cycles: in front of the step they were 0.4 of its 1.25 us)
     auto multiply = [&](int b, int mm, uint32_t bb, uint32_t sl, auto && request) __attribute__((always_inline)) {
-        half8 bf[2][NT], af[2];
+        half8 bf[2][NT], af[2], al[2];
         auto read_B = [&](int j) __attribute__((always_inline)) {
 #pragma unroll
             for (int jt = 0; jt < NT; ++jt) bf[j & 1][jt] = *(const half8 *) (smem + bb + jt * 4096 + (boff0 ^ (uint32_t) (j << 5)));
@@ -589,16 +622,21 @@ __device__ __forceinline__ void mid_body(const PfP & p, const PfJob & jb, const 
                 const int sh = 8 * (2 * kk + (j >> 1));                                       // 32-weight sub-block 4 mm + 2 kk + j / 2
                 const uint32_t a = hd[1] >> sh, m = hd[2] >> sh, c = hd[3] >> sh;
                 const int sc = (int) (mm ? (c & 0x0Fu) | ((a & 0xC0u) >> 2) : a & 63u), mn = (int) (mm ? ((c >> 4) & 0x0Fu) | ((m & 0xC0u) >> 2) : m & 63u);
+                if (EX) mul = half2v{(_Float16) sc, (_Float16) sc};
+                else {
                 const _Float16 ds = (_Float16) (h2f((uint16_t) (hd[0] & 0xFFFF)) * (float) sc), ms = (_Float16) (h2f((uint16_t) (hd[0] >> 16)) * (float) mn);
                 mul = half2v{ds, ds}; add = half2v{(_Float16) -ms, (_Float16) -ms};
+                }
             } else if (TYPE == PM_Q6_K) {
-                const _Float16 dd = (_Float16) (h2f(d6) * (float) (int) (int8_t) (hd[0] >> (8 * j)));
+                const int sc = (int) (int8_t) (hd[0] >> (8 * j));
+                const _Float16 dd = EX ? (_Float16) sc : (_Float16) (h2f(d6) * (float) sc);
                 mul = half2v{dd, dd};
             } else if (Q8 && (j & 1) == 0) {
                 const _Float16 dd = __builtin_bit_cast(_Float16, (uint16_t) (hd[0] >> (16 * (j >> 1))));
                 mul = half2v{dd, dd};
             }
-            af[j & 1] = pf_dequant<TYPE>(ql[j], qh[j & 1], mm, kk, j, mul, add);
+            if constexpr (EX && TYPE == PM_Q6_K) af[j & 1] = pf_dequant<TYPE>(ql[j], qh[j & 1], mm, kk, j, mul, add, &al[j & 1]);
+            else af[j & 1] = pf_dequant<TYPE>(ql[j], qh[j & 1], mm, kk, j, mul, add);
         };
         read_B(0);
         operand(0);
@@ -607,17 +645,59 @@ __device__ __forceinline__ void mid_body(const PfP & p, const PfJob & jb, const 
             if (j < 3) { read_B(j + 1); operand(j + 1); }
 #pragma unroll
             for (int jt = 0; jt < NT; ++jt) acc[jt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[j & 1], bf[j & 1][jt], acc[jt], 0, 0, 0);
+            if (EX && TYPE == PM_Q6_K)
+#pragma unroll
+                for (int jt = 0; jt < NT; ++jt) acc[jt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(al[j & 1], bf[j & 1][jt], acc[jt], 0, 0, 0);
             request(j);
+        }
+    };
+    // EX: the whole numbers of super-block b (this wave's half of its k) onto the running sums; the minima by either half in turn
+    auto fold = [&](int b) __attribute__((always_inline)) {
+        const uint8_t * const xb = smem + XS + (b & 1) * XB;
+        float d[16], dm[16];
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+            const int row = (e & 3) + 8 * (e >> 2) + 4 * h;
+            if (K45) {
+                const uint32_t v = *(const uint32_t *) (ag + HDR + (b & 3) * 512 + row * 16);
+                d[e] = h2f((uint16_t) v); dm[e] = h2f((uint16_t) (v >> 16));
+            } else d[e] = h2f(*(const uint16_t *) (ag + XTRA + ((b >> 3) & 1) * 512 + row * 16 + (b & 7) * 2));
+        }
+        const bool mins = K45 && kk == (b & 1);
+        half8 mo = {0, 0, 0, 0, 0, 0, 0, 0};
+        if (mins) {                                             // minima of the row's sub-blocks 4 h .. 4 h + 3, each for two groups of 16
+            const u32x4 hd = *(const u32x4 *) (ag + HDR + (b & 3) * 512 + r * 16);
+            const uint32_t m = h ? ((hd[3] >> 4) & 0x0F0F0F0Fu) | ((hd[2] & 0xC0C0C0C0u) >> 2) : hd[2] & 0x3F3F3F3Fu;
+#pragma unroll
+            for (int i = 0; i < 8; ++i) mo[i] = (_Float16) (int) ((m >> (8 * (i >> 1))) & 63u);
+        }
+#pragma unroll
+        for (int jt = 0; jt < NT; ++jt) {
+            const float da = *(const float *) (xb + XSUM + (32 * jt + r) * 4);
+            if (mins) {
+                const float16v z = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
+                const float16v am = __builtin_amdgcn_mfma_f32_32x32x16_f16(mo, *(const half8 *) (xb + (32 * jt + r) * 32 + 16 * h), z, 0, 0, 0);
+#pragma unroll
+                for (int e = 0; e < 16; ++e) run[jt][e] = fmaf(da, fmaf(-dm[e], am[e], d[e] * acc[jt][e]), run[jt][e]);
+            } else {
+#pragma unroll
+                for (int e = 0; e < 16; ++e) run[jt][e] = fmaf(da, d[e] * acc[jt][e], run[jt][e]);
+            }
+#pragma unroll
+            for (int e = 0; e < 16; ++e) acc[jt][e] = 0.0f;
         }
     };
 
     // split K: slice ks of S takes the super-blocks [b0, b1)
     const int b0 = (int) ((long) ks * nb / S), b1 = (int) ((long) (ks + 1) * nb / S);
     uint32_t bb = 0, bn = BBUF, bw = 2 * BBUF, sl = 0, sw = AHEAD * SLOT;       // buffers of steps s, s + 1, s + 2, slots of steps s and s + AHEAD
-    auto request = [&](int s, bool even, int u) __attribute__((always_inline)) { if (kk) issue_B(s + 2, bw, u); else issue_A(s + AHEAD, sw, AHEAD & 1 ? !even : even, u); };
+    auto request = [&](int s, bool even, int u) __attribute__((always_inline)) { if (kk) { if (EX && even && u == 0) issue_X((s >> 1) + 1); issue_B(s + 2, bw, u); } else issue_A(s + AHEAD, sw, AHEAD & 1 ? !even : even, u); };
     auto turn = [&] __attribute__((always_inline)) { const uint32_t t = bb; bb = bn; bn = bw; bw = t; sw = sl; sl = sl == AHEAD * SLOT ? 0 : sl + SLOT; };
 #pragma unroll
-    for (int u = 0; u < 8; ++u) if (kk) issue_B(2 * b0 + (u >> 2), u & 4 ? bn : bb, u & 3);
+    for (int u = 0; u < 8; ++u) if (kk) {
+        if (EX && u == 0) issue_X(b0);
+        issue_B(2 * b0 + (u >> 2), u & 4 ? bn : bb, u & 3);
+    }
 #pragma unroll
     for (int w = 0; w < AHEAD; ++w)
 #pragma unroll
@@ -629,9 +709,13 @@ __device__ __forceinline__ void mid_body(const PfP & p, const PfJob & jb, const 
         turn();
         if (Q8 && 2 * b + 1 >= nsteps) break;
         multiply(b, 1, bb, sl, [&](int u) __attribute__((always_inline)) { request(2 * b + 1, false, u); });
+        if constexpr (EX) fold(b);
         settle(false);
         turn();
     }
+    if constexpr (EX)
+#pragma unroll
+        for (int jt = 0; jt < NT; ++jt) acc[jt] = run[jt];
     mid_wait<0>();                                             // (the last steps' look-ahead still lands in the buffers)
     __syncthreads();
     // ---- the two halves of K: every wave keeps its rows' tokens [32 NH kk, + 32 NH) and takes the partner's sums of them
@@ -737,7 +821,7 @@ __device__ __forceinline__ void mid_body(const PfP & p, const PfJob & jb, const 
 
 // block id -> (row tile, token tile): XCD x = id % 8 takes the row tiles x, x + 8, ..; its consecutive slots sweep the token tiles of one row tile, so the
 // workgroups that run together on an XCD share a few row tiles of weights and the activation k-slices in its L2 (mmq_big.hip's mapping)
-template <int TA, int TB, int NT, bool MID = false, int EXP = 0>
+template <int TA, int TB, int NT, bool MID = false, int EXP = 0, bool EX = false>
 __global__ __launch_bounds__(PF_NTHR) void gemm_pf_kernel(PfP p) {
     extern __shared__ __attribute__((aligned(1024))) uint8_t pf_smem[];
     const int id = (int) blockIdx.x, x = id & 7;
@@ -767,14 +851,14 @@ __global__ __launch_bounds__(PF_NTHR) void gemm_pf_kernel(PfP p) {
         if (TA == TB || jb.type == TA) pf_body<TA, NT, EXP>(p, jb, n0, t0, pf_smem, role, ks, S, tile_id);
         else pf_body<TB, NT, EXP>(p, jb, n0, t0, pf_smem, role, ks, S, tile_id);
     } else {
-        if (TA == TB || jb.type == TA) mid_body<TA, NT>(p, jb, n0, t0, pf_smem, role, ks, S, tile_id);
-        else mid_body<TB, NT>(p, jb, n0, t0, pf_smem, role, ks, S, tile_id);
+        if (TA == TB || jb.type == TA) mid_body<TA, NT, EX>(p, jb, n0, t0, pf_smem, role, ks, S, tile_id);
+        else mid_body<TB, NT, EX>(p, jb, n0, t0, pf_smem, role, ks, S, tile_id);
     }
 }
 
-template <int TA, int TB, int NT, bool MID = false> constexpr size_t pf_lds_bytes() {
+template <int TA, int TB, int NT, bool MID = false, bool EX = false> constexpr size_t pf_lds_bytes() {
     if (!MID) return (size_t) 3 * NT * 32 * 128 + (size_t) 8 * (pf_wave_bytes<TA>() > pf_wave_bytes<TB>() ? pf_wave_bytes<TA>() : pf_wave_bytes<TB>());
-    return (size_t) 6 * NT * 32 * 128 + (size_t) 4 * (mid_group_bytes<TA>() > mid_group_bytes<TB>() ? mid_group_bytes<TA>() : mid_group_bytes<TB>());
+    return mid_lds_bytes<TA, NT, EX>() > mid_lds_bytes<TB, NT, EX>() ? mid_lds_bytes<TA, NT, EX>() : mid_lds_bytes<TB, NT, EX>();
 }
 
 void pf_allow_lds(const void * kern, size_t lds) {
@@ -867,7 +951,7 @@ int pm_launch_gemm_pf(const pm_gemm_pf_job * jobs, int njobs, const void * xh, i
 
 // pair != 0: jobs[0] = ffn_gate, jobs[1] = ffn_up (same type, same N; jobs[0]'s outputs are ignored): jobs[1]'s output = silu(W0 . x) * (W1 . x) (+ its own bias / resid
 // before the product are NOT applied to the gate). One launch, the gate result stays on the chip.
-int pm_launch_gemm_pf_ex(const pm_gemm_pf_job * jobs, int njobs, const void * xh, int K, int T, int pair, hipStream_t st) {
+static int launch_pf(const pm_gemm_pf_job * jobs, int njobs, const void * xh, const pm_q8k_wide * wide, int K, int T, int pair, hipStream_t st) {
     if (njobs < 1 || njobs > PF_MAX_JOBS || !jobs || !xh) return -2;
     if (pair && (njobs != 2 || jobs[0].type != jobs[1].type || jobs[0].N != jobs[1].N || jobs[0].bias || jobs[0].resid || jobs[1].silu_gate)) return -2;
     static const int force_nt = [] { const char * e = getenv("PM355_GEMM_PF_NT"); return e ? atoi(e) : 0; }();
@@ -880,7 +964,8 @@ int pm_launch_gemm_pf_ex(const pm_gemm_pf_job * jobs, int njobs, const void * xh
     const int mid_nt = T <= 64 ? 2 : 4;
     long mid_wgs = 0;
     for (int j = 0; j < njobs && !(pair && j); ++j) mid_wgs += (jobs[j].N + (pair ? 63 : 127)) / (pair ? 64 : 128);
-    const bool mid = !force_nt && T <= 128 && mid_wgs <= cus;
+    // (8-bit activations: mid_body at any size - its tiles of 128 tokens side by side -, pf_body's registers are its accumulators')
+    const bool mid = wide || (!force_nt && T <= 128 && mid_wgs <= cus);
     const int rows = mid ? 128 : 256;
     PfP p = {};
     p.pair = pair ? 1 : 0;
@@ -899,6 +984,7 @@ int pm_launch_gemm_pf_ex(const pm_gemm_pf_job * jobs, int njobs, const void * xh
     static const int grp = [] { const char * e = getenv("PM355_GEMM_PF_GROUP"); return e ? atoi(e) : 0; }();
     p.grp = grp;
     p.njobs = njobs; p.nt_n = tiles; p.Xh = (const _Float16 *) xh; p.K = K; p.T = T;
+    if (wide) { p.Xd = (const uint8_t *) wide->d; p.Xs = (const uint8_t *) wide->s; p.ldt = wide->ldt; }
     static const int force_s = [] { const char * e = getenv("PM355_GEMM_PF_SPLITK"); return e ? atoi(e) : 0; }();
     static const bool no_mixed = [] { const char * e = getenv("PM355_GEMM_PF_MIXED"); return e && e[0] == '0'; }();
     // 256-token tiles (a dequantized operand serves 8 MFMAs; 128-token tiles only where the batch has no more tokens). Few tiles - wo / ffn_down / wq | wk | wv
@@ -947,7 +1033,7 @@ int pm_launch_gemm_pf_ex(const pm_gemm_pf_job * jobs, int njobs, const void * xh
         return 0;
     }
 #endif
-#define PF_GO(A, B) (mid ? nt == 4 ? go(gemm_pf_kernel<A, B, 4, true>, pf_lds_bytes<A, B, 4, true>()) : go(gemm_pf_kernel<A, B, 2, true>, pf_lds_bytes<A, B, 2, true>()) : nt == 8 ? go(gemm_pf_kernel<A, B, 8>, pf_lds_bytes<A, B, 8>()) : nt == 4 ? go(gemm_pf_kernel<A, B, 4>, pf_lds_bytes<A, B, 4>()) : go(gemm_pf_kernel<A, B, 2>, pf_lds_bytes<A, B, 2>()))
+#define PF_GO(A, B) (wide ? nt == 4 ? go(gemm_pf_kernel<A, B, 4, true, 0, A != PM_Q8_0>, pf_lds_bytes<A, B, 4, true, A != PM_Q8_0>()) : go(gemm_pf_kernel<A, B, 2, true, 0, A != PM_Q8_0>, pf_lds_bytes<A, B, 2, true, A != PM_Q8_0>()) : mid ? nt == 4 ? go(gemm_pf_kernel<A, B, 4, true>, pf_lds_bytes<A, B, 4, true>()) : go(gemm_pf_kernel<A, B, 2, true>, pf_lds_bytes<A, B, 2, true>()) : nt == 8 ? go(gemm_pf_kernel<A, B, 8>, pf_lds_bytes<A, B, 8>()) : nt == 4 ? go(gemm_pf_kernel<A, B, 4>, pf_lds_bytes<A, B, 4>()) : go(gemm_pf_kernel<A, B, 2>, pf_lds_bytes<A, B, 2>()))
     if (ta == tb) { if (ta == PM_Q4_K) PF_GO(PM_Q4_K, PM_Q4_K); else if (ta == PM_Q5_K) PF_GO(PM_Q5_K, PM_Q5_K); else if (ta == PM_Q8_0) PF_GO(PM_Q8_0, PM_Q8_0); else PF_GO(PM_Q6_K, PM_Q6_K); }
     else if (ta == PM_Q8_0 || tb == PM_Q8_0) return -1;      // (Q8_0 only as a launch of its own: ffn_down of the files whose n_ff is no multiple of 256)
     else if (ta == PM_Q4_K && tb == PM_Q5_K) PF_GO(PM_Q4_K, PM_Q5_K);
@@ -955,4 +1041,21 @@ int pm_launch_gemm_pf_ex(const pm_gemm_pf_job * jobs, int njobs, const void * xh
     else PF_GO(PM_Q5_K, PM_Q6_K);
 #undef PF_GO
     return 0;
+}
+int pm_launch_gemm_pf_ex(const pm_gemm_pf_job * jobs, int njobs, const void * xh, int K, int T, int pair, hipStream_t st) { return launch_pf(jobs, njobs, xh, nullptr, K, T, pair, st); }
+
+int pm_gemm_wide_check(int type, int K, int N, int T) {
+    if ((type != PM_Q4_K && type != PM_Q5_K && type != PM_Q6_K) || T < 1 || T > PM_WIDE_MAX_TOKENS) return -1;
+    return pm_gemm_pf_check(type, K, N, T);
+}
+int pm_launch_gemm_wide(const pm_gemm_pf_job * jobs, int njobs, const pm_q8k_wide & x, int K, int T, int pair, hipStream_t st) {
+    if (T > PM_WIDE_MAX_TOKENS || !x.q || x.ldt < (T <= 64 ? 64 : (T + 127) / 128 * 128) || x.ldt % 4 || (size_t) (K / 256) * x.ldt * 32 >= ((size_t) 1 << 32)) return -2;
+    for (int j = 0; j < njobs; ++j) if (pm_gemm_wide_check(jobs[j].type, K, jobs[j].N, T)) return -1;
+    return launch_pf(jobs, njobs, x.q, &x, K, T, pair, st);
+}
+size_t pm_q8k_wide_bytes(int K) { return (size_t) PM_WIDE_MAX_TOKENS * ((size_t) K * 2 + (size_t) (K / 256) * 36); }
+pm_q8k_wide pm_q8k_wide_at(void * buf, int K) {
+    pm_q8k_wide x;
+    x.q = (uint16_t *) buf; x.s = x.q + (size_t) PM_WIDE_MAX_TOKENS * K; x.d = (float *) (x.s + (size_t) PM_WIDE_MAX_TOKENS * (K / 256) * 16); x.ldt = PM_WIDE_MAX_TOKENS;
+    return x;
 }

@@ -49,6 +49,13 @@ static inline bool pm_type_is_repacked(int type) { return type == 12 || type == 
 // [super-block][32-value sub-block s][operand lane = 32 * (k / 16 % 2) + row % 32][16 bytes]: one coalesced load per sub-block instead of one
 // cache line per token
 struct pm_q8k_tables { uint8_t * base = nullptr; size_t tab_bytes = 0; int nsb = 0; uint8_t * qbase = nullptr; };
+// Q8_K activations of up to PM_WIDE_MAX_TOKENS rows for pm_launch_gemm_wide: the 8-bit values as F16 [row][K], sums of 16 as F16 [super-block][ldt][16], scales [super-block][ldt]
+constexpr int PM_WIDE_MAX_TOKENS = 512;
+struct pm_q8k_wide { uint16_t * q = nullptr, * s = nullptr; float * d = nullptr; int ldt = 0; };
+size_t pm_q8k_wide_bytes(int K);
+pm_q8k_wide pm_q8k_wide_at(void * buf, int K);                         // a buffer of pm_q8k_wide_bytes(K), 16-byte aligned
+void pm_launch_quantize_wide(const float * x, const pm_q8k_wide & y, int K, int rows, hipStream_t st);
+void pm_launch_rmsnorm_wide(const float * x, const float * w, const pm_q8k_wide & y, int K, int rows, float eps, hipStream_t st);
 void pm_launch_quantize_q8k(const float * x, void * y, int K, int rows, hipStream_t st, pm_q8k_tables tab = {});
 void pm_launch_quantize_q80(const float * x, void * y, int K, int rows, hipStream_t st);
 // silu(gate) * up -> Q8_0, written into the Q8_0 small-batch mat-mul's activation tables (pm_mmq_i8_q80_tables); then pm_launch_mmq_i8(PM_Q8_0, ..., reuse_prep = 1)
@@ -132,6 +139,9 @@ bool pm_gemm_pf_enabled();      // false under PM355_GEMM_KERNEL=1 / 2 (A/B agai
 int pm_launch_gemm_pf(const pm_gemm_pf_job * jobs, int njobs, const void * xh, int K, int T, hipStream_t st);
 // pair != 0: jobs = {ffn_gate, ffn_up} (same type and N): jobs[1]'s output = silu(W0 . x) * (W1 . x) in one launch, the gate result never leaves the chip
 int pm_launch_gemm_pf_ex(const pm_gemm_pf_job * jobs, int njobs, const void * xh, int K, int T, int pair, hipStream_t st);
+// the same for 8-bit activations (up to PM_WIDE_MAX_TOKENS rows; Q4_K, Q5_K, Q6_K): the whole-number sums of pm_launch_mmq_i8. Jobs of at most two types
+int pm_gemm_wide_check(int type, int K, int N, int T);
+int pm_launch_gemm_wide(const pm_gemm_pf_job * jobs, int njobs, const pm_q8k_wide & x, int K, int T, int pair, hipStream_t st);
 
 // up to 4 matrices over the same activations (f32 X converted once, or x_f16 given): ONE launch of mmq_pf.hip when it serves all of them, else one launch each
 int pm_launch_gemm_q_multi(const pm_gemm_pf_job * jobs, int njobs, const float * X, const void * x_f16, int K, int T, hipStream_t st);

@@ -44,7 +44,7 @@ __device__ __forceinline__ int wave_min_i(int v) {
 }
 
 // One wave quantizes one 256-value block held as 4 consecutive values per lane.
-__device__ __forceinline__ void q8k_block_from_regs(const float v[4], int lane, uint8_t * row_out, int K, int blk, const pm_q8k_tables & tb = pm_q8k_tables(), int row = 0) {
+__device__ __forceinline__ void q8k_block_from_regs(const float v[4], int lane, uint8_t * row_out, int K, int blk, const pm_q8k_tables & tb = pm_q8k_tables(), int row = 0, const pm_q8k_wide & wd = pm_q8k_wide()) {
     float a0 = fabsf(v[0]), a1 = fabsf(v[1]), a2 = fabsf(v[2]), a3 = fabsf(v[3]);
     const float amax = wave_max(fmaxf(fmaxf(a0, a1), fmaxf(a2, a3)));
     int8_t  * qs    = (int8_t *) row_out;
@@ -69,19 +69,27 @@ __device__ __forceinline__ void q8k_block_from_regs(const float v[4], int lane, 
             psum += q;
             packed |= (uint32_t) (q & 0xFF) << (8 * i);
         }
-        if (lane == 0) dd[blk] = 1 / iscale;
+        if (row_out && lane == 0) dd[blk] = 1 / iscale;
+        if (wd.q && lane == 0) wd.d[(size_t) blk * wd.ldt + row] = 1 / iscale;
         if (tb.base && lane == 0) ((float *) (tb.base + (size_t) (row >> 5) * tb.tab_bytes + (size_t) tb.nsb * 1024))[blk * 32 + (row & 31)] = 1 / iscale;
     } else if (lane == 0) {
-        dd[blk] = 0.0f;
+        if (row_out) dd[blk] = 0.0f;
+        if (wd.q) wd.d[(size_t) blk * wd.ldt + row] = 0.0f;
         if (tb.base) ((float *) (tb.base + (size_t) (row >> 5) * tb.tab_bytes + (size_t) tb.nsb * 1024))[blk * 32 + (row & 31)] = 0.0f;
     }
-    ((uint32_t *) (qs + (size_t) blk * PM_QK_K))[lane] = packed;
+    if (row_out) ((uint32_t *) (qs + (size_t) blk * PM_QK_K))[lane] = packed;
     // A-operand order (pm_q8k_tables::qbase): values 4 lane .. 4 lane + 3 = bytes 4 (lane % 4) of sub-block lane / 8, half (lane / 4) % 2
     if (tb.qbase) *(uint32_t *) (tb.qbase + (size_t) (row >> 5) * tb.nsb * 8192 + (size_t) blk * 8192 + (lane >> 3) * 1024 + ((((lane >> 2) & 1) * 32 + (row & 31)) * 16) + 4 * (lane & 3)) = packed;
     // bsums: 16 values = 4 lanes (one quad)
     psum += dpp_i<0xB1>(psum);
     psum += dpp_i<0x4E>(psum);
-    if ((lane & 3) == 0) bsums[blk * 16 + (lane >> 2)] = (int16_t) psum;
+    if (row_out && (lane & 3) == 0) bsums[blk * 16 + (lane >> 2)] = (int16_t) psum;
+    if (wd.q) {
+        typedef _Float16 h4 __attribute__((ext_vector_type(4)));
+        *(h4 *) (wd.q + (size_t) row * K + (size_t) blk * PM_QK_K + 4 * lane) =
+            h4{(_Float16) (int) (int8_t) packed, (_Float16) (int) (int8_t) (packed >> 8), (_Float16) (int) (int8_t) (packed >> 16), (_Float16) (int) (int8_t) (packed >> 24)};
+        if ((lane & 3) == 0) wd.s[((size_t) blk * wd.ldt + row) * 16 + (lane >> 2)] = __builtin_bit_cast(uint16_t, (_Float16) (float) psum);
+    }
     if (tb.base && (lane & 3) == 0) {              // group G = lane / 4 -> operand lane (row % 32) + 32 (G & 1), slot G / 2 (mmq_i8.hip mmq_prep_kernel)
         const int G = lane >> 2;
         ((_Float16 *) (tb.base + (size_t) (row >> 5) * tb.tab_bytes))[((size_t) blk * 64 + (row & 31) + 32 * (G & 1)) * 8 + (G >> 1)] = (_Float16) (float) psum;
@@ -89,7 +97,7 @@ __device__ __forceinline__ void q8k_block_from_regs(const float v[4], int lane, 
 }
 
 __global__ __launch_bounds__(256) void quantize_q8k_kernel(const float * __restrict__ x, uint8_t * __restrict__ y,
-                                                           int K, int rows, size_t y_row_bytes, pm_q8k_tables tb) {
+                                                           int K, int rows, size_t y_row_bytes, pm_q8k_tables tb, pm_q8k_wide wd) {
     const int lane = threadIdx.x & 63;
     const int nblk = K / PM_QK_K;
     const long wave = (long) blockIdx.x * 4 + (threadIdx.x >> 6);
@@ -97,7 +105,7 @@ __global__ __launch_bounds__(256) void quantize_q8k_kernel(const float * __restr
     const int row = (int) (wave / nblk), blk = (int) (wave % nblk);
     const float4 f = ((const float4 *) (x + (size_t) row * K + (size_t) blk * PM_QK_K))[lane];
     const float v[4] = {f.x, f.y, f.z, f.w};
-    q8k_block_from_regs(v, lane, y + (size_t) row * y_row_bytes, K, blk, tb, row);
+    q8k_block_from_regs(v, lane, y ? y + (size_t) row * y_row_bytes : nullptr, K, blk, tb, row, wd);
 }
 
 // silu(gate) * up (ggml_silu + ggml_mul of llm_build_ffn, src/llama.cpp:9804; same f32 expressions as layer_ops.hip's silu_mul_kernel) fused with
@@ -173,7 +181,7 @@ __global__ __launch_bounds__(256) void silu_mul_q80_tab_kernel(const float * __r
 template <int NWV>
 __global__ __launch_bounds__(64 * NWV) void rmsnorm_q8k_kernel(const float * __restrict__ x, const float * __restrict__ w,
                                                           float * __restrict__ ynorm, uint8_t * __restrict__ yq,
-                                                          int K, float eps, size_t yq_row_bytes, _Float16 * __restrict__ yh, pm_q8k_tables tb) {
+                                                          int K, float eps, size_t yq_row_bytes, _Float16 * __restrict__ yh, pm_q8k_tables tb, pm_q8k_wide wd) {
     __shared__ double red[NWV];
     const int row = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
     const int nblk = K / PM_QK_K;
@@ -226,7 +234,7 @@ __global__ __launch_bounds__(64 * NWV) void rmsnorm_q8k_kernel(const float * __r
             typedef _Float16 h4 __attribute__((ext_vector_type(4)));
             ((h4 *) (yh + (size_t) row * K + (size_t) blk * PM_QK_K))[lane] = h4{(_Float16) v[0], (_Float16) v[1], (_Float16) v[2], (_Float16) v[3]};
         }
-        if (yq) q8k_block_from_regs(v, lane, yq + (size_t) row * yq_row_bytes, K, blk, tb, row);
+        if (yq || wd.q) q8k_block_from_regs(v, lane, yq ? yq + (size_t) row * yq_row_bytes : nullptr, K, blk, tb, row, wd);
     };
     if (held) {
 #pragma unroll
@@ -240,7 +248,11 @@ __global__ __launch_bounds__(64 * NWV) void rmsnorm_q8k_kernel(const float * __r
 void pm_launch_quantize_q8k(const float * x, void * y, int K, int rows, hipStream_t st, pm_q8k_tables tab) {
     const long waves = (long) rows * (K / PM_QK_K);
     hipLaunchKernelGGL(quantize_q8k_kernel, dim3((unsigned) ((waves + 3) / 4)), dim3(256), 0, st,
-                       x, (uint8_t *) y, K, rows, pm_q8k_row_bytes(K), tab);
+                       x, (uint8_t *) y, K, rows, pm_q8k_row_bytes(K), tab, pm_q8k_wide());
+}
+void pm_launch_quantize_wide(const float * x, const pm_q8k_wide & y, int K, int rows, hipStream_t st) {
+    const long waves = (long) rows * (K / PM_QK_K);
+    hipLaunchKernelGGL(quantize_q8k_kernel, dim3((unsigned) ((waves + 3) / 4)), dim3(256), 0, st, x, (uint8_t *) nullptr, K, rows, 0, pm_q8k_tables(), y);
 }
 void pm_launch_silu_mul_q8k(const float * gate, const float * up, void * y, int K, int rows, hipStream_t st, pm_q8k_tables tab) {
     const long waves = (long) rows * (K / PM_QK_K);
@@ -258,6 +270,10 @@ void pm_launch_quantize_q80(const float * x, void * y, int K, int rows, hipStrea
                        x, (uint8_t *) y, K, rows, pm_q80_row_bytes(K));
 }
 void pm_launch_rmsnorm_q8k(const float * x, const float * w, float * ynorm, void * yq, int K, int rows, float eps, hipStream_t st, void * ynorm_f16, pm_q8k_tables tab) {
-    if (rows <= 256) hipLaunchKernelGGL(rmsnorm_q8k_kernel<16>, dim3(rows), dim3(1024), 0, st, x, w, ynorm, (uint8_t *) yq, K, eps, pm_q8k_row_bytes(K), (_Float16 *) ynorm_f16, tab);
-    else            hipLaunchKernelGGL(rmsnorm_q8k_kernel<4>, dim3(rows), dim3(256), 0, st, x, w, ynorm, (uint8_t *) yq, K, eps, pm_q8k_row_bytes(K), (_Float16 *) ynorm_f16, tab);
+    if (rows <= 256) hipLaunchKernelGGL(rmsnorm_q8k_kernel<16>, dim3(rows), dim3(1024), 0, st, x, w, ynorm, (uint8_t *) yq, K, eps, pm_q8k_row_bytes(K), (_Float16 *) ynorm_f16, tab, pm_q8k_wide());
+    else            hipLaunchKernelGGL(rmsnorm_q8k_kernel<4>, dim3(rows), dim3(256), 0, st, x, w, ynorm, (uint8_t *) yq, K, eps, pm_q8k_row_bytes(K), (_Float16 *) ynorm_f16, tab, pm_q8k_wide());
+}
+void pm_launch_rmsnorm_wide(const float * x, const float * w, const pm_q8k_wide & y, int K, int rows, float eps, hipStream_t st) {
+    if (rows <= 256) hipLaunchKernelGGL(rmsnorm_q8k_kernel<16>, dim3(rows), dim3(1024), 0, st, x, w, (float *) nullptr, (uint8_t *) nullptr, K, eps, 0, (_Float16 *) nullptr, pm_q8k_tables(), y);
+    else             hipLaunchKernelGGL(rmsnorm_q8k_kernel<4>, dim3(rows), dim3(256), 0, st, x, w, (float *) nullptr, (uint8_t *) nullptr, K, eps, 0, (_Float16 *) nullptr, pm_q8k_tables(), y);
 }

@@ -316,6 +316,22 @@ def mul_mat_small_mixed(ws, xq, n_tokens, biases=None):
     return ys
 
 
+def mul_mat_wide(ws, x, biases=None, resids=None, pair=False):
+    """1..3 matrices over up to 512 tokens of f32 activations x [T, K], quantized to Q8_K on the device (mmq_pf.hip, 8-bit form) -> list of f32 [T, N_j]; pair: silu(W0 x) * (W1 x)."""
+    import ctypes as C
+    lib = L.load()
+    n, x = len(ws), x.contiguous().view(-1, ws[0].K)
+    lib.pm355_mul_mat_q_wide.restype, lib.pm355_mul_mat_q_wide_scratch.restype = C.c_int, C.c_int64
+    lib.pm355_mul_mat_q_wide.argtypes = [C.c_void_p, C.c_int] + [C.c_void_p] * 6 + [C.c_int64, C.c_int64, C.c_int, C.c_void_p, C.c_void_p]
+    lib.pm355_mul_mat_q_wide_scratch.argtypes = [C.c_int64]
+    ys = [torch.empty((x.shape[0], w.N), dtype=torch.float32, device=w.data.device) for w in ws]
+    scratch = torch.empty(max(lib.pm355_mul_mat_q_wide_scratch(ws[0].K), 16), dtype=torch.uint8, device=ws[0].data.device)
+    arr = lambda v: (C.c_void_p * n)(*[ptr(e) for e in v]) if v else None
+    Tp, Np = (C.c_int * n)(*[w.type for w in ws]), (C.c_int64 * n)(*[w.N for w in ws])
+    check(lib.pm355_mul_mat_q_wide(Tp, n, arr([w.data for w in ws]), Np, arr(ys), arr(biases), arr(resids), ptr(x), ws[0].K, x.shape[0], int(pair), ptr(scratch), stream_ptr()), "mul_mat_q_wide")
+    return ys[1:] if pair else ys
+
+
 def mul_mat_i8(w, x, bias=None, resid=None):
     """Prompt-sized batches on the integer matrix cores (mmq_big.hip): x f32 [T, K] -> Q8_K on device -> f32 [T, N]."""
     import ctypes as C

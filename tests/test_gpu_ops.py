@@ -270,6 +270,44 @@ def test_prompt_matmul_on_integer_matrix_cores(P, oracle, t):
         assert np.allclose(y[:4], y1, rtol=1e-5, atol=1e-5)
 
 
+@pytest.mark.parametrize("t", [Q4_K, Q5_K, Q6_K])
+def test_wide_batch_matmul_with_8_bit_activations(P, oracle, t):
+    """The prompt GEMM's 8-bit form: whole-number sums of every super-block in the F16 matrix cores -> oracle.mul_mat (integers) within the tolerance of the integer kernels. Edges: rows and
+    tokens of partial tiles, either tile size (33 / 64, 65 / 128 tokens), an odd number of super-blocks, K split over workgroups (32 super-blocks), matrices of two types, pair tiles. Quants and
+    scales at their limits: weights of all-ones bytes (Q6_K: the largest quants with scales of -1, Q4_K / Q5_K the largest quants, scales and minima) and scales of -128 (Q6_K: products of 4096)."""
+    rng = np.random.default_rng(700 + t)
+    for K, N, T in ((768, 132, 33), (4096, 72, 64), (1024, 600, 65), (8192, 260, 128), (512, 4, 1), (1024, 132, 129), (512, 260, 512)):
+        b, b2 = rand_blocks(t, N, K, rng), rand_blocks(Q4_K if t == Q6_K else Q6_K, 64, K, rng)
+        x = rng.normal(0, 1, (T, K)).astype(np.float32)
+        x[0] = 0
+        bias, resid = rng.normal(0, 1, N).astype(np.float32), rng.normal(0, 1, (T, N)).astype(np.float32)
+        w, w2 = P.upload_weight(t, b, K, N), P.upload_weight(Q4_K if t == Q6_K else Q6_K, b2, K, 64)
+        want, want2 = oracle.mul_mat(t, b, K, N, x), oracle.mul_mat(w2.type, b2, K, 64, x)
+        tol = dict(rtol=2e-5, atol=2e-5 * np.sqrt(K / 4096))
+        y, y2 = P.mul_mat_wide([w, w2], _dev(P, x), biases=[_dev(P, bias), None], resids=[_dev(P, resid), None])
+        assert np.allclose(y.cpu().numpy(), want + bias[None] + resid, **tol), (K, N, T, np.abs(y.cpu().numpy() - want - bias[None] - resid).max())
+        assert np.allclose(y2.cpu().numpy(), want2, **tol)
+        g = P.mul_mat_wide([w, w], _dev(P, x / 8), pair=True)[0].cpu().numpy()
+        p = oracle.mul_mat(t, b, K, N, x / 8).astype(np.float64)
+        err = (2 + np.abs(p)) * 2e-5 * (np.abs(p) + np.sqrt(K / 4096))          # |d(silu(p) p) / dp| < 2 |p| + 0.2, times the error of p
+        assert (np.abs(g - p / (1 + np.exp(-p)) * p) <= err + 1e-6).all()
+    K, N, T = 1024, 64, 40
+    b = np.full(rand_blocks(t, N, K, rng).shape, 0xFF, np.uint8).reshape(N, K // 256, -1)
+    if t == Q6_K:
+        b[:, :, :192] = np.where(rng.random((N, K // 256, 192)) < 0.5, 0, 255)
+        b[:, :, 192:208] = np.where(rng.random((N, K // 256, 16)) < 0.5, 0x80, 0x7F)
+        b[:, :, 208:] = np.frombuffer(np.float16(0.01).tobytes(), np.uint8)
+    else:
+        b[:, :, :4] = np.frombuffer(np.float16([0.01, 0.02]).tobytes(), np.uint8)
+    b = b.reshape(-1)
+    for x in (np.ones((T, K), np.float32), rng.choice([-1.0, 1.0], (T, K)).astype(np.float32), rng.normal(0, 1, (T, K)).astype(np.float32)):
+        want = oracle.mul_mat(t, b, K, N, x)
+        y = P.mul_mat_wide([P.upload_weight(t, b, K, N)], _dev(P, x))[0].cpu().numpy()
+        # (a super-block's sums beyond 2^24 are rounded as they are added up: 16 instructions for each half of its k, 2^-24 of the largest partial sum each)
+        lim = (K // 256) * 2 * 16 * 2.0 ** -24 * (4096 * 127 * 128) * 0.01 * np.abs(x).max() / 127
+        assert np.allclose(y, want, rtol=2e-5, atol=2e-5 + lim), np.abs(y - want).max()
+
+
 @pytest.mark.parametrize("t", [Q4_K, Q6_K])
 def test_small_batch_matmul_multi_job_launch(P, oracle, t):
     """wq | wk | wv and ffn_gate | ffn_up as ONE launch over a virtual row space: every job equals its own single-job launch (same integers; the
