@@ -24,7 +24,6 @@
 // measured ~1e-6).
 #include "pm355_device.h"
 #include "pm355_kernels.h"
-#include "attn_tail_device.h"
 #include <stdlib.h>
 #include <stdio.h>
 #include <mutex>
@@ -44,7 +43,7 @@ struct PfJob {
     long row_stride, ldy; int type, N, tile0;      // tile0: this job's first row tile in the launch's numbering of row tiles
 };
 struct PfP {
-    PfJob job[PF_MAX_JOBS]; int njobs, nt_n, nt_t; const _Float16 * Xh; int K, T; int grp, pair; int splitk, full; float * ws; unsigned * cnt; unsigned long long * trace;
+    PfJob job[PF_MAX_JOBS]; int njobs, nt_n, nt_t; const _Float16 * Xh; int K, T; int grp, pair; int splitk, full; float * ws; unsigned long long * trace;
     const uint8_t * Xd, * Xs; int ldt;               // 8-bit activations (pm_q8k_wide): scales, group sums
 };
 // Ablations (measurement builds only: -DPM_GEMM_ABLATE=1 adds instantiations of the Q4_K 256-token kernel, PM355_GEMM_EXP=<bits> picks one; results are WRONG when set):
@@ -387,52 +386,14 @@ __device__ __forceinline__ void pf_body(const PfP & p, const PfJob & jb, const i
         if (!late && !(exp & 4)) __builtin_amdgcn_s_barrier();  // (the second group has passed one barrier more: level)
         __builtin_amdgcn_s_barrier();                           // every wave is out of the k loop: the tile memory is free
     }
-    // ---- split K: every slice leaves its partial tile in a slab (lane-linear, 1 KiB per store instruction); the LAST arriver of a tile adds the S partials in
-    //      slice order, so the sum does not depend on who arrives when, and runs the epilogue. Hand-off = plain stores, one agent-scope
-    //      release before the ticket, one acquire behind it (cdna_hip_programming.md, Guideline 16 counter form); the counter returns to 0 for the next launch.
+    // ---- split K: every slice leaves its partial tile in a slab (lane-linear, 1 KiB per store instruction) for pf_reduce_kernel
     if (S > 1) {
-        f32x4 * const slab0 = (f32x4 *) p.ws + (size_t) tile_id * S * (8 * NT * 4 * 64);
-        f32x4 * const mine = slab0 + (size_t) ks * (8 * NT * 4 * 64);
+        f32x4 * const mine = (f32x4 *) p.ws + (size_t) (tile_id * S + ks) * (8 * NT * 4 * 64);
 #pragma unroll
         for (int jt = 0; jt < NT; ++jt)
 #pragma unroll
             for (int g = 0; g < 4; ++g) *(PM_G f32x4 *) (mine + ((wave * NT + jt) * 4 + g) * 64 + lane) = f32x4{acc[jt][4 * g], acc[jt][4 * g + 1], acc[jt][4 * g + 2], acc[jt][4 * g + 3]};
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        __syncthreads();
-        if (tid == 0) {
-            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
-            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-            *(volatile unsigned *) smem = __hip_atomic_fetch_add(p.cnt + tile_id, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        }
-        __syncthreads();
-        const unsigned ticket = *(volatile unsigned *) smem;
-        if (ticket != (unsigned) (S - 1)) return;
-        if (tid == 0) {
-            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-            __hip_atomic_store(p.cnt + tile_id, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        }
-        __syncthreads();
-        // (all S slabs from memory, the reducer's own included - a second register copy of the tile would not fit; one token tile at a time, fenced:
-        //  left alone the scheduler puts every load of the tile in flight and spills the accumulators)
-#pragma unroll
-        for (int jt = 0; jt < NT; ++jt)
-#pragma unroll
-            for (int e = 0; e < 16; ++e) acc[jt][e] = 0.0f;
-        for (int q = 0; q < S; ++q) {
-            const f32x4 * sl = slab0 + (size_t) q * (8 * NT * 4 * 64) + lane;
-#pragma unroll
-            for (int jt = 0; jt < NT; ++jt) {
-                f32x4 v[4];
-#pragma unroll
-                for (int g = 0; g < 4; ++g) v[g] = *(const PM_G f32x4 *) (sl + ((wave * NT + jt) * 4 + g) * 64);
-#pragma unroll
-                for (int g = 0; g < 4; ++g)
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) acc[jt][4 * g + e] += v[g][e];
-                __builtin_amdgcn_sched_barrier(0);
-            }
-        }
-        __syncthreads();                                        // (the ticket word is tile memory: pair tiles write there next)
+        return;
     }
     // ---- pair tiles: the gate waves park their accumulators in LDS (same lane, same register index as the up wave that needs them)
     if (role) {
@@ -738,42 +699,14 @@ __device__ __forceinline__ void mid_body(const PfP & p, const PfJob & jb, const 
             for (int e = 0; e < 4; ++e) own[i][4 * q + e] += o[e];
         }
     __syncthreads();
-    // ---- split K: slabs, ticket, the last arriver adds them up in slice order (as above). The slabs are written through and read past the caches: a release of everything this
-    //      XCD's L2 holds cost more than the hand-over. Four slabs are on their way at a time (one by one: a trip to memory each, 10 us at S = 8)
+    // ---- split K: slabs, as above
     if (S > 1) {
-        constexpr int TILE = 8 * NH * 4 * 64, Q = NH * 4;
-        const __amdgpu_buffer_rsrc_t rs = coh_rsrc((f32x4 *) p.ws + (size_t) tile_id * S * TILE);
-        const uint32_t at = (uint32_t) ((wave * Q) * 64 + lane) * 16u;
-#pragma unroll
-        for (int q = 0; q < Q; ++q)
-            __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, f32x4{own[q / 4][4 * (q % 4)], own[q / 4][4 * (q % 4) + 1], own[q / 4][4 * (q % 4) + 2], own[q / 4][4 * (q % 4) + 3]}), rs,
-                                                   (int) (at + (uint32_t) ks * (TILE * 16u) + (uint32_t) q * 1024u), 0, 17);
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        __syncthreads();
-        if (tid == 0) *(volatile unsigned *) smem = __hip_atomic_fetch_add(p.cnt + tile_id, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        __syncthreads();
-        if (*(volatile unsigned *) smem != (unsigned) (S - 1)) return;
-        if (tid == 0) __hip_atomic_store(p.cnt + tile_id, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        f32x4 * const mine = (f32x4 *) p.ws + (size_t) (tile_id * S + ks) * (8 * NH * 4 * 64);
 #pragma unroll
         for (int i = 0; i < NH; ++i)
 #pragma unroll
-            for (int e = 0; e < 16; ++e) own[i][e] = 0.0f;
-        for (int u = 0; u < S; u += 4) {
-            u32x4 v[4][Q];
-#pragma unroll
-            for (int w = 0; w < 4; ++w)
-#pragma unroll
-                for (int q = 0; q < Q; ++q) v[w][q] = coh_ld16u(rs, at + (uint32_t) min(u + w, S - 1) * (TILE * 16u) + (uint32_t) q * 1024u);
-#pragma unroll
-            for (int w = 0; w < 4; ++w) {
-                if (u + w >= S) break;
-#pragma unroll
-                for (int q = 0; q < Q; ++q)
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) own[q / 4][4 * (q % 4) + e] += __builtin_bit_cast(f32x4, v[w][q])[e];
-            }
-        }
-        __syncthreads();                                        // (the ticket word is tile memory)
+            for (int q = 0; q < 4; ++q) *(PM_G f32x4 *) (mine + ((wave * NH + i) * 4 + q) * 64 + lane) = f32x4{own[i][4 * q], own[i][4 * q + 1], own[i][4 * q + 2], own[i][4 * q + 3]};
+        return;
     }
     // ---- pair tiles: the gate waves park their sums in LDS (same lane, same register index as the up wave that needs them)
     if (role) {
@@ -825,8 +758,8 @@ template <int TA, int TB, int NT, bool MID = false, int EXP = 0, bool EX = false
 __global__ __launch_bounds__(PF_NTHR) void gemm_pf_kernel(PfP p) {
     extern __shared__ __attribute__((aligned(1024))) uint8_t pf_smem[];
     const int id = (int) blockIdx.x, x = id & 7;
-    // slots [0, full) of an XCD run whole tiles; the slots behind them are split S ways along K, the slices of a tile neighbours on one XCD (the reducer reads
-    // their slabs out of its own L2). full = 0: every tile split (S = 1: none)
+    // slots [0, full) of an XCD run whole tiles; the slots behind them are split S ways along K, the slices of a tile neighbours on one XCD.
+    // full = 0: every tile split (S = 1: none)
     const int q = id >> 3;
     const int S = q < p.full ? 1 : p.splitk;
     const int ks = q < p.full ? 0 : (q - p.full) % p.splitk, slot = q < p.full ? q : p.full + (q - p.full) / p.splitk;
@@ -846,13 +779,81 @@ __global__ __launch_bounds__(PF_NTHR) void gemm_pf_kernel(PfP p) {
         n0 = (tile_n - jb.tile0) * ROWS;
     }
     const int t0 = tile_t * 32 * NT;
-    const int tile_id = (slot - p.full) * 8 + x;                 // (split tiles only: slab and counter index)
+    const int tile_id = (slot - p.full) * 8 + x;                 // (split tiles only: slab index)
     if constexpr (!MID) {
         if (TA == TB || jb.type == TA) pf_body<TA, NT, EXP>(p, jb, n0, t0, pf_smem, role, ks, S, tile_id);
         else pf_body<TB, NT, EXP>(p, jb, n0, t0, pf_smem, role, ks, S, tile_id);
     } else {
         if (TA == TB || jb.type == TA) mid_body<TA, NT, EX>(p, jb, n0, t0, pf_smem, role, ks, S, tile_id);
         else mid_body<TB, NT, EX>(p, jb, n0, t0, pf_smem, role, ks, S, tile_id);
+    }
+}
+
+// The slabs of a launch's split tiles, added in slice order, and the epilogue: a wave per 32 rows x 8 tokens, 8 lanes on a token's 32 rows, all S parts on their way at once. Bound by the slabs'
+// bytes. A launch of its own because all CUs then share them: the last arriver of a tile (64 of 256 workgroups for 8192 rows x 512 tokens, S = 4) read 1 MB of slabs and stored its tile by
+// itself, 48 us behind the last product. us, last arriver (as it was; its loads in fours and the slabs written through) / product + this launch: 512 tokens of 8192 x 8192 Q4_K 107 (102) / 66 + 17,
+// 8192 x 28672 264 (245) / 211 + 17, 10240 x 8192 131 (120) / 91 + 15; 101 tokens (mid_body) of 4096 x 4096 23.0 / 18.3 + 4.8, 4096 x 14336 35.9 / 27.7 + 5.9. KPW: 8-token groups of a wave, 1 (4: fewer
+// waves, 18.7 for 16.8 and 8.1 for 5.9)
+// nti: token sub-tiles of a wave; mid: mid_body's tiles (wave = row group + 4 x token half)
+template <int SMAX, int KPW> __global__ __launch_bounds__(256) void pf_reduce_kernel(PfP p, int mid, int nti, int units) {
+    const int u4 = (int) blockIdx.x * 4 + __builtin_amdgcn_readfirstlane((int) threadIdx.x >> 6), unit = u4 / (4 / KPW), k0 = u4 % (4 / KPW) * KPW, lane = threadIdx.x & 63;
+    if (unit >= units) return;
+    const int S = p.splitk, per_tile = (p.pair ? 4 : 8) * nti, tile_id = unit / per_tile, wv = unit % per_tile / nti, i = unit % nti;
+    const int x = tile_id & 7, slot = p.full + (tile_id >> 3), per_x = (p.nt_n + 7 - x) >> 3;
+    if (slot >= per_x * p.nt_t) return;
+    const int tile_n = x + 8 * (slot / p.nt_t), tile_t = slot % p.nt_t;
+    PfJob jb = p.job[0];
+    int n0 = tile_n * (mid ? 64 : 128), row = wv, half = 0, wave = wv, wave_g = 0;
+    if (p.pair) {
+        jb = p.job[1];
+        if (mid) { row = wv & 1; half = wv >> 1; wave_g = row + 4 * half; wave = wave_g + 2; } else { wave_g = wv; wave = wv + 4; }
+    } else {
+#pragma unroll
+        for (int q = 1; q < PF_MAX_JOBS; ++q) if (q < p.njobs && tile_n >= p.job[q].tile0) jb = p.job[q];
+        n0 = (tile_n - jb.tile0) * (mid ? 128 : 256);
+        if (mid) { row = wv & 3; half = wv >> 2; }
+    }
+    const int t0 = (tile_t * (mid ? 2 : 1) + half) * 32 * nti + 32 * i + 8 * k0, n = n0 + 32 * row + (lane & 7) * 4;
+    if (t0 >= p.T || n >= jb.N) return;                         // (N is a multiple of 4)
+    const size_t tile = (size_t) 8 * nti * 256;                 // of f32x4
+    const f32x4 * const slab = (const f32x4 *) p.ws + (size_t) tile_id * S * tile + (lane & 1) * 32 + ((lane & 7) >> 1) * 64 + 8 * k0 + (lane >> 3);
+    auto sums = [&](int w, f32x4 (&o)[KPW]) __attribute__((always_inline)) {
+        const f32x4 * const at = slab + (size_t) (w * nti + i) * 256;
+        f32x4 v[SMAX][KPW];
+#pragma unroll
+        for (int q = 0; q < SMAX; ++q)
+#pragma unroll
+            for (int k = 0; k < KPW; ++k) v[q][k] = *(const PM_G f32x4 *) (at + (size_t) (q < S ? q : S - 1) * tile + 8 * k);
+#pragma unroll
+        for (int k = 0; k < KPW; ++k) o[k] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int q = 0; q < SMAX; ++q) {
+            if (q >= S) break;
+#pragma unroll
+            for (int k = 0; k < KPW; ++k) o[k] += v[q][k];
+        }
+    };
+    f32x4 o[KPW], gate[KPW];
+    sums(wave, o);
+    if (p.pair) sums(wave_g, gate);
+#pragma unroll
+    for (int k = 0; k < KPW; ++k) {
+        const int t = t0 + 8 * k + (lane >> 3);
+        if (t >= p.T) continue;
+        const long at = (long) t * jb.ldy + n;
+        f32x4 v = o[k];
+        if (p.pair)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[e] *= gate[k][e] / (1.0f + expf(-gate[k][e]));
+        if (jb.bias) v += ld_g((const f32x4 *) (jb.bias + n));
+        if (jb.resid) v += ld_g((const f32x4 *) (jb.resid + at));
+        if (jb.silu_gate) {
+            const f32x4 gg = ld_g((const f32x4 *) (jb.silu_gate + at));
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[e] *= gg[e] / (1.0f + expf(-gg[e]));
+        }
+        if (jb.Yh) *(PM_G half4v *) (jb.Yh + at) = half4v{(_Float16) v[0], (_Float16) v[1], (_Float16) v[2], (_Float16) v[3]};
+        else *(PM_G f32x4 *) (jb.Y + at) = v;
     }
 }
 
@@ -870,7 +871,7 @@ void pf_allow_lds(const void * kern, size_t lds) {
     if (n_done < 64) { done[n_done].k = kern; done[n_done].dev = dev; ++n_done; }
 }
 
-// split-K workspace of a (device, stream): 64 KiB of tile counters (zero between launches: the reducer resets its own) + the partial-tile slabs
+// split-K workspace of a (device, stream): the partial-tile slabs
 struct PfWs { hipStream_t st; int dev; uint8_t * p; size_t bytes; uint64_t use; };
 PfWs g_pf_ws[16] = {};
 uint64_t g_pf_tick = 0;
@@ -888,7 +889,6 @@ uint8_t * pf_workspace(hipStream_t st, size_t need) {
     if (e->p) { (void) hipDeviceSynchronize(); (void) hipFree(e->p); e->p = nullptr; e->bytes = 0; }
     need = (need + ((size_t) 32 << 20)) & ~(((size_t) 16 << 20) - 1);     // (grow in steps: a later, larger batch does not reallocate at once)
     if (hipMalloc((void **) &e->p, need) != hipSuccess) { e->p = nullptr; return nullptr; }
-    (void) hipMemsetAsync(e->p, 0, 65536, st);
     e->st = st; e->dev = dev; e->bytes = need; e->use = ++g_pf_tick;
     return e->p;
 }
@@ -997,16 +997,18 @@ static int launch_pf(const pm_gemm_pf_job * jobs, int njobs, const void * xh, co
     p.splitk = S; p.full = full;
     const int split_slots = maxL - full;                       // per XCD
     if (S > 1) {
-        const size_t slab = (size_t) (mid ? 4 : 8) * nt * 4 * 64 * 16, need = 65536 + (size_t) 8 * split_slots * S * slab;
-        if ((size_t) 8 * split_slots > 16384) return -2;
-        uint8_t * w = pf_workspace(st, need);
-        if (!w) return -3;
-        p.cnt = (unsigned *) w; p.ws = (float *) (w + 65536);
+        const size_t slab = (size_t) (mid ? 4 : 8) * nt * 4 * 64 * 16, need = (size_t) 8 * split_slots * S * slab;
+        p.ws = (float *) pf_workspace(st, need);
+        if (!p.ws) return -3;
     }
     const int slots = full + split_slots * S;
     auto go = [&](auto kern, size_t lds) {
         pf_allow_lds((const void *) kern, lds);
         hipLaunchKernelGGL(kern, dim3(8 * slots), dim3(PF_NTHR), lds, st, p);
+        if (S == 1) return;
+        const int nti = mid ? nt / 2 : nt, units = 8 * split_slots * (p.pair ? 4 : 8) * nti;
+        if (S <= 4) hipLaunchKernelGGL((pf_reduce_kernel<4, 1>), dim3(units), dim3(256), 0, st, p, (int) mid, nti, units);
+        else        hipLaunchKernelGGL((pf_reduce_kernel<8, 1>), dim3(units), dim3(256), 0, st, p, (int) mid, nti, units);
     };
 #if PM_GEMM_ABLATE
     static const int exp_sw = [] { const char * e = getenv("PM355_GEMM_EXP"); return e ? atoi(e) : 0; }();

@@ -887,7 +887,7 @@ def test_prompt_gemm_tiles_of_128_rows(P, oracle, t, K, N, T):
 
 
 @pytest.mark.parametrize("t", [Q4_K, Q5_K, Q6_K])
-@pytest.mark.parametrize("K,N,T", [(1024, 384, 200), (2048, 132, 64), (512, 256, 257)])
+@pytest.mark.parametrize("K,N,T", [(1024, 384, 200), (2048, 132, 64), (512, 256, 257), (8192, 132, 200)])
 def test_prompt_gemm_pair_tiles_silu_gate_times_up(P, oracle, t, K, N, T):
     """ffn_gate | ffn_up as one launch of pair tiles: silu(gate) * up formed inside the workgroup == the two separate launches followed by the product
     (the reference's MUL_MAT, MUL_MAT, SILU, MUL: llm_build_ffn, src/llama.cpp:9804)."""
