@@ -700,6 +700,7 @@ int run_window(pm_window * m, const int32_t * d_tokens, const float * d_x_in, in
         return 0;
     };
     // the tokens' rows, and with them the cos / sin tables that the wq | wk | wv epilogues of all layers read
+    bool attn_normed = false;                                   // a layer's attn_norm came with the launch in front of it
     const bool one = T == 1 && !m->no_fuse, tab = (one ? m->qkv_epi && m->rope_tab : small_epi) && m->hi > m->lo;
     if (d_tokens) pm_launch_embed(m->tok_embd.type, m->tok_embd.d, E, d_tokens, T, m->x, st, &m->rope, d_pos, d_seq, (const float *) m->rope_freqs.d, tab ? m->rope_tab : nullptr, rg ? 1 : 0);
     else if (tab) pm_launch_rope_table(m->rope, d_pos, d_seq, (const float *) m->rope_freqs.d, m->rope_tab, st, T, rg ? 1 : 0);
@@ -808,7 +809,16 @@ int run_window(pm_window * m, const int32_t * d_tokens, const float * d_x_in, in
                          const float * silu_gate = nullptr, hipStream_t s2 = nullptr) {
                 return pm_launch_gemm_q_h(w.type, w.d, nullptr, xh, y, yh, (int) w.K, (int) w.N, T, bias, resid, silu_gate, 0, s2 ? s2 : st);
             };
-            pm_launch_rmsnorm_q8k(cur, (const float *) L.t[PM355_T_ATTN_NORM].d, nullptr, nullptr, E, T, hp.rms_eps, st, m->xn);
+            // a matrix whose result the next one takes through an RMS norm: with that norm in the launch that adds up its K slices, where it has one
+            auto GN = [&](const Tensor & w, const void * xh, float * y, const float * resid, const Tensor * norm_w, bool & normed) {
+                pm_gemm_norm nm = {norm_w ? (const float *) norm_w->d : nullptr, hp.rms_eps, m->xn, false};
+                const pm_gemm_pf_job j = {w.type, (int) w.N, w.d, y, nullptr, nullptr, resid, nullptr, 0};
+                const bool pf = nm.w && pm_gemm_pf_enabled() && pm_gemm_pf_check(w.type, (int) w.K, (int) w.N, T) == 0;
+                const int rc = pf ? pm_launch_gemm_pf_norm(j, xh, (int) w.K, T, &nm, st) : G(w, xh, y, nullptr, nullptr, resid);
+                normed = nm.done;
+                return rc;
+            };
+            if (!attn_normed) pm_launch_rmsnorm_q8k(cur, (const float *) L.t[PM355_T_ATTN_NORM].d, nullptr, nullptr, E, T, hp.rms_eps, st, m->xn);
             // wq | wk | wv: ONE launch over the shared activations, each matrix with its own quant type (mmq_pf.hip jobs; wk / wv alone - N = n_head_kv * head_dim -
             // filled a fraction of the chip: 212 TFLOP/s as their own launches)
             int rc;
@@ -829,10 +839,11 @@ int run_window(pm_window * m, const int32_t * d_tokens, const float * d_x_in, in
                     return seterr(m, PM355_E_RANGE, "prefill: n_ctx too large for the attention kernel");
             }
             float * x_mid = (cur == bufs[0]) ? bufs[1] : bufs[0];
-            if (att_h ? G(L.t[PM355_T_WO], m->att, x_mid, nullptr, nullptr, cur)
+            bool ffn_normed = false;
+            if (att_h ? GN(L.t[PM355_T_WO], m->att, x_mid, cur, &L.t[PM355_T_FFN_NORM], ffn_normed)
                       : pm_launch_gemm_q_ex(L.t[PM355_T_WO].type, L.t[PM355_T_WO].d, m->att, x_mid, (int) L.t[PM355_T_WO].K, (int) L.t[PM355_T_WO].N, T, nullptr, cur, nullptr, 0, st))
                 return seterr(m, PM355_E_UNSUPPORTED, "prefill: wo gemm");
-            pm_launch_rmsnorm_q8k(x_mid, (const float *) L.t[PM355_T_FFN_NORM].d, nullptr, nullptr, E, T, hp.rms_eps, st, m->xn);
+            if (!ffn_normed) pm_launch_rmsnorm_q8k(x_mid, (const float *) L.t[PM355_T_FFN_NORM].d, nullptr, nullptr, E, T, hp.rms_eps, st, m->xn);
             {
                 // ffn_gate | ffn_up as ONE launch of pair tiles: h2 = F16(silu(gate) * up) comes out of the up waves' epilogue, the gate result crosses over inside
                 // the workgroup and never reaches HBM (two launches: gate as f32, read back by ffn_up's epilogue - 2 x T x n_ff x 4 bytes per layer)
@@ -849,7 +860,9 @@ int run_window(pm_window * m, const int32_t * d_tokens, const float * d_x_in, in
             }
             if (rc) return seterr(m, PM355_E_UNSUPPORTED, "prefill: gate/up gemm");
             float * x_next = (il == m->hi - 1 && d_x_out) ? d_x_out : ((x_mid == bufs[0]) ? bufs[1] : bufs[0]);
-            if (G(L.t[PM355_T_FFN_DOWN], m->h2, x_next, nullptr, nullptr, x_mid)) return seterr(m, PM355_E_UNSUPPORTED, "prefill: down gemm");
+            // (the next layer's norm: its weights are there only if layers are not streamed, and it takes this path at more tokens than any small batch has)
+            const bool ahead = il + 1 < m->hi && !m->n_slots && T > MMQ_MAX_TOKENS && !m->tab_big;
+            if (GN(L.t[PM355_T_FFN_DOWN], m->h2, x_next, x_mid, ahead ? &m->layers[il + 1 - m->lo].t[PM355_T_ATTN_NORM] : nullptr, attn_normed)) return seterr(m, PM355_E_UNSUPPORTED, "prefill: down gemm");
             layer_release(m, il, st);
             cur = x_next;
             continue;

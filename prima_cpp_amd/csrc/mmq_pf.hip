@@ -139,6 +139,15 @@ template <int TYPE> __device__ __forceinline__ half8 pf_dequant(const u32x2 ql, 
     return __builtin_bit_cast(half8, u32x4{u2(t[0]), u2(t[1]), u2(t[2]), u2(t[3])});
 }
 
+// a wave's 32 x 32 results (matrix-core layout: token lane % 32, rows 8 g + 4 (lane / 32) .. + 3 in o[g]) -> slab [token][32 rows], through its LDS tile
+__device__ __forceinline__ void store_slab(const f32x4 (&o)[4], uint8_t * xe, f32x4 * slab, int lane) {
+    const int r = lane & 31, h = lane >> 5;
+#pragma unroll
+    for (int g = 0; g < 4; ++g) *(f32x4 *) (xe + r * 144 + (8 * g + 4 * h) * 4) = o[g];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) *(PM_G f32x4 *) (slab + q * 64 + lane) = *(const f32x4 *) (xe + (8 * q + (lane >> 3)) * 144 + (lane & 7) * 16);
+}
+
 // the k loop + epilogue of one workgroup tile: rows [n0, n0 + 256) of job jb, tokens [t0, t0 + 32 NT)
 // role: 0 plain; 1 / 2 = the gate / up half of a PAIR tile (waves 0-3 multiply ffn_gate's rows [n0, n0 + 128), waves 4-7 the same rows of ffn_up; the gate
 // accumulators cross over through LDS after the k loop and the up waves store silu(gate) * up: ffn_gate's result never travels to HBM)
@@ -386,13 +395,16 @@ __device__ __forceinline__ void pf_body(const PfP & p, const PfJob & jb, const i
         if (!late && !(exp & 4)) __builtin_amdgcn_s_barrier();  // (the second group has passed one barrier more: level)
         __builtin_amdgcn_s_barrier();                           // every wave is out of the k loop: the tile memory is free
     }
-    // ---- split K: every slice leaves its partial tile in a slab (lane-linear, 1 KiB per store instruction) for pf_reduce_kernel
+    // ---- split K: every slice leaves its partial tile in a slab for pf_reduce_kernel, 32 rows of a token as one line (turned in a wave-private LDS tile [token][32 rows + 4])
     if (S > 1) {
         f32x4 * const mine = (f32x4 *) p.ws + (size_t) (tile_id * S + ks) * (8 * NT * 4 * 64);
 #pragma unroll
-        for (int jt = 0; jt < NT; ++jt)
+        for (int jt = 0; jt < NT; ++jt) {
+            f32x4 o[4];
 #pragma unroll
-            for (int g = 0; g < 4; ++g) *(PM_G f32x4 *) (mine + ((wave * NT + jt) * 4 + g) * 64 + lane) = f32x4{acc[jt][4 * g], acc[jt][4 * g + 1], acc[jt][4 * g + 2], acc[jt][4 * g + 3]};
+            for (int g = 0; g < 4; ++g) o[g] = f32x4{acc[jt][4 * g], acc[jt][4 * g + 1], acc[jt][4 * g + 2], acc[jt][4 * g + 3]};
+            store_slab(o, smem + wave * (32 * 144), mine + (wave * NT + jt) * 256, lane);
+        }
         return;
     }
     // ---- pair tiles: the gate waves park their accumulators in LDS (same lane, same register index as the up wave that needs them)
@@ -703,9 +715,12 @@ __device__ __forceinline__ void mid_body(const PfP & p, const PfJob & jb, const 
     if (S > 1) {
         f32x4 * const mine = (f32x4 *) p.ws + (size_t) (tile_id * S + ks) * (8 * NH * 4 * 64);
 #pragma unroll
-        for (int i = 0; i < NH; ++i)
+        for (int i = 0; i < NH; ++i) {
+            f32x4 o[4];
 #pragma unroll
-            for (int q = 0; q < 4; ++q) *(PM_G f32x4 *) (mine + ((wave * NH + i) * 4 + q) * 64 + lane) = f32x4{own[i][4 * q], own[i][4 * q + 1], own[i][4 * q + 2], own[i][4 * q + 3]};
+            for (int q = 0; q < 4; ++q) o[q] = f32x4{own[i][4 * q], own[i][4 * q + 1], own[i][4 * q + 2], own[i][4 * q + 3]};
+            store_slab(o, smem + wave * (32 * 144), mine + (wave * NH + i) * 256, lane);
+        }
         return;
     }
     // ---- pair tiles: the gate waves park their sums in LDS (same lane, same register index as the up wave that needs them)
@@ -816,14 +831,14 @@ template <int SMAX, int KPW> __global__ __launch_bounds__(256) void pf_reduce_ke
     const int t0 = (tile_t * (mid ? 2 : 1) + half) * 32 * nti + 32 * i + 8 * k0, n = n0 + 32 * row + (lane & 7) * 4;
     if (t0 >= p.T || n >= jb.N) return;                         // (N is a multiple of 4)
     const size_t tile = (size_t) 8 * nti * 256;                 // of f32x4
-    const f32x4 * const slab = (const f32x4 *) p.ws + (size_t) tile_id * S * tile + (lane & 1) * 32 + ((lane & 7) >> 1) * 64 + 8 * k0 + (lane >> 3);
+    const f32x4 * const slab = (const f32x4 *) p.ws + (size_t) tile_id * S * tile + 64 * k0 + lane;
     auto sums = [&](int w, f32x4 (&o)[KPW]) __attribute__((always_inline)) {
         const f32x4 * const at = slab + (size_t) (w * nti + i) * 256;
         f32x4 v[SMAX][KPW];
 #pragma unroll
         for (int q = 0; q < SMAX; ++q)
 #pragma unroll
-            for (int k = 0; k < KPW; ++k) v[q][k] = *(const PM_G f32x4 *) (at + (size_t) (q < S ? q : S - 1) * tile + 8 * k);
+            for (int k = 0; k < KPW; ++k) v[q][k] = *(const PM_G f32x4 *) (at + (size_t) (q < S ? q : S - 1) * tile + 64 * k);
 #pragma unroll
         for (int k = 0; k < KPW; ++k) o[k] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
@@ -854,6 +869,60 @@ template <int SMAX, int KPW> __global__ __launch_bounds__(256) void pf_reduce_ke
         }
         if (jb.Yh) *(PM_G half4v *) (jb.Yh + at) = half4v{(_Float16) v[0], (_Float16) v[1], (_Float16) v[2], (_Float16) v[3]};
         else *(PM_G f32x4 *) (jb.Y + at) = v;
+    }
+}
+
+// The same for one matrix of which every tile is split, a workgroup per token, with the RMS norm of the token's new row (rmsnorm_q8k_kernel's expressions in its order, F16): the row does not
+// travel to memory and back, and a launch goes. Bound by the slabs. us, both launches / this one: 101 tokens x 4096, S = 4 4.8 + 4.6 / 5.3, S = 8 5.9 + 4.6 / 6.3; 512 x 8192, S = 4 16.8 + 9.9 / 20.8 (28.3
+// with 4 waves a token). For up to 512 tokens: beyond, few launches have every tile split
+template <int SMAX> __global__ __launch_bounds__(1024) void pf_reduce_norm_kernel(PfP p, int mid, int nti, const float * w, float eps, _Float16 * yh) {
+    constexpr int NWV = 16, HOLD = 2;
+    __shared__ double red[NWV];
+    const int t = blockIdx.x, lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane((int) threadIdx.x >> 6), S = p.splitk;
+    const PfJob & jb = p.job[0];
+    const int N = jb.N, rows = mid ? 128 : 256, tok = mid ? 64 * nti : 32 * nti;
+    const int tile_t = t / tok, tt = t % tok / 32, half = mid ? tt / nti : 0, i = mid ? tt % nti : tt;
+    const size_t tile = (size_t) 8 * nti * 256;                 // of f32x4
+    f32x4 f[HOLD], wt[HOLD];
+    double s = 0.0;
+#pragma unroll
+    for (int j = 0; j < HOLD; ++j) {
+        const int n = (wv + NWV * j) * 256 + 4 * lane;
+        if (n >= N) continue;
+        const int tile_n = n / rows, wave = n % rows / 32 + 4 * half;
+        const f32x4 * const at = (const f32x4 *) p.ws + (size_t) (((tile_n >> 3) * p.nt_t + tile_t) * 8 + (tile_n & 7)) * S * tile + (size_t) (wave * nti + i) * 256 + (t & 31) * 8 + (lane & 7);
+        f32x4 v[SMAX], o = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int q = 0; q < SMAX; ++q) v[q] = *(const PM_G f32x4 *) (at + (size_t) (q < S ? q : S - 1) * tile);
+        const f32x4 r = jb.resid ? ld_g((const f32x4 *) (jb.resid + (long) t * jb.ldy + n)) : f32x4{0.0f, 0.0f, 0.0f, 0.0f}, b = jb.bias ? ld_g((const f32x4 *) (jb.bias + n)) : f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+        wt[j] = ld_g((const f32x4 *) (w + n));
+#pragma unroll
+        for (int q = 0; q < SMAX; ++q) if (q < S) o += v[q];
+        if (jb.bias) o += b;
+        if (jb.resid) o += r;
+        f[j] = o;
+    }
+#pragma unroll
+    for (int j = 0; j < HOLD; ++j) {
+        const int n = (wv + NWV * j) * 256 + 4 * lane;
+        if (n >= N) continue;
+        *(PM_G f32x4 *) (jb.Y + (long) t * jb.ldy + n) = f[j];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) s += (double) (f[j][e] * f[j][e]);
+    }
+    s = all_sum(s);
+    if (lane == 0) red[wv] = s;
+    __syncthreads();
+    double tot = (red[0] + red[1]) + (red[2] + red[3]);
+#pragma unroll
+    for (int q = 4; q < NWV; q += 4) tot += (red[q] + red[q + 1]) + (red[q + 2] + red[q + 3]);
+    const float scale = 1.0f / sqrtf((float) (tot / N) + eps);
+#pragma unroll
+    for (int j = 0; j < HOLD; ++j) {
+        const int n = (wv + NWV * j) * 256 + 4 * lane;
+        if (n >= N) continue;
+        const f32x4 v = f[j] * scale * wt[j];
+        *(PM_G half4v *) (yh + (size_t) t * N + n) = half4v{(_Float16) v[0], (_Float16) v[1], (_Float16) v[2], (_Float16) v[3]};
     }
 }
 
@@ -951,7 +1020,7 @@ int pm_launch_gemm_pf(const pm_gemm_pf_job * jobs, int njobs, const void * xh, i
 
 // pair != 0: jobs[0] = ffn_gate, jobs[1] = ffn_up (same type, same N; jobs[0]'s outputs are ignored): jobs[1]'s output = silu(W0 . x) * (W1 . x) (+ its own bias / resid
 // before the product are NOT applied to the gate). One launch, the gate result stays on the chip.
-static int launch_pf(const pm_gemm_pf_job * jobs, int njobs, const void * xh, const pm_q8k_wide * wide, int K, int T, int pair, hipStream_t st) {
+static int launch_pf(const pm_gemm_pf_job * jobs, int njobs, const void * xh, const pm_q8k_wide * wide, int K, int T, int pair, hipStream_t st, pm_gemm_norm * norm = nullptr) {
     if (njobs < 1 || njobs > PF_MAX_JOBS || !jobs || !xh) return -2;
     if (pair && (njobs != 2 || jobs[0].type != jobs[1].type || jobs[0].N != jobs[1].N || jobs[0].bias || jobs[0].resid || jobs[1].silu_gate)) return -2;
     static const int force_nt = [] { const char * e = getenv("PM355_GEMM_PF_NT"); return e ? atoi(e) : 0; }();
@@ -1006,7 +1075,14 @@ static int launch_pf(const pm_gemm_pf_job * jobs, int njobs, const void * xh, co
         pf_allow_lds((const void *) kern, lds);
         hipLaunchKernelGGL(kern, dim3(8 * slots), dim3(PF_NTHR), lds, st, p);
         if (S == 1) return;
-        const int nti = mid ? nt / 2 : nt, units = 8 * split_slots * (p.pair ? 4 : 8) * nti;
+        const int nti = mid ? nt / 2 : nt;
+        if (norm && !full && T <= 512 && njobs == 1 && jobs[0].Y && !jobs[0].Yh && !jobs[0].silu_gate && p.job[0].ldy == p.job[0].N && jobs[0].N % 256 == 0 && jobs[0].N <= 8192) {
+            auto fused = [&](auto k) { hipLaunchKernelGGL(k, dim3(T), dim3(1024), 0, st, p, (int) mid, nti, norm->w, norm->eps, (_Float16 *) norm->yh); };
+            if (S <= 4) fused(pf_reduce_norm_kernel<4>); else fused(pf_reduce_norm_kernel<8>);
+            norm->done = true;
+            return;
+        }
+        const int units = 8 * split_slots * (p.pair ? 4 : 8) * nti;
         if (S <= 4) hipLaunchKernelGGL((pf_reduce_kernel<4, 1>), dim3(units), dim3(256), 0, st, p, (int) mid, nti, units);
         else        hipLaunchKernelGGL((pf_reduce_kernel<8, 1>), dim3(units), dim3(256), 0, st, p, (int) mid, nti, units);
     };
@@ -1045,6 +1121,8 @@ static int launch_pf(const pm_gemm_pf_job * jobs, int njobs, const void * xh, co
     return 0;
 }
 int pm_launch_gemm_pf_ex(const pm_gemm_pf_job * jobs, int njobs, const void * xh, int K, int T, int pair, hipStream_t st) { return launch_pf(jobs, njobs, xh, nullptr, K, T, pair, st); }
+
+int pm_launch_gemm_pf_norm(const pm_gemm_pf_job & job, const void * xh, int K, int T, pm_gemm_norm * norm, hipStream_t st) { norm->done = false; return launch_pf(&job, 1, xh, nullptr, K, T, 0, st, norm); }
 
 int pm_gemm_wide_check(int type, int K, int N, int T) {
     if ((type != PM_Q4_K && type != PM_Q5_K && type != PM_Q6_K) || T < 1 || T > PM_WIDE_MAX_TOKENS) return -1;

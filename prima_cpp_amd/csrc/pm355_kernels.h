@@ -139,6 +139,9 @@ bool pm_gemm_pf_enabled();      // false under PM355_GEMM_KERNEL=1 / 2 (A/B agai
 int pm_launch_gemm_pf(const pm_gemm_pf_job * jobs, int njobs, const void * xh, int K, int T, hipStream_t st);
 // pair != 0: jobs = {ffn_gate, ffn_up} (same type and N): jobs[1]'s output = silu(W0 . x) * (W1 . x) in one launch, the gate result never leaves the chip
 int pm_launch_gemm_pf_ex(const pm_gemm_pf_job * jobs, int njobs, const void * xh, int K, int T, int pair, hipStream_t st);
+// one matrix, and yh = F16 RMS norm of the rows of its f32 result (as pm_launch_rmsnorm_q8k) where that costs no launch (done; else the caller's own)
+struct pm_gemm_norm { const float * w; float eps; void * yh; bool done; };
+int pm_launch_gemm_pf_norm(const pm_gemm_pf_job & job, const void * xh, int K, int T, pm_gemm_norm * norm, hipStream_t st);
 // the same for 8-bit activations (up to PM_WIDE_MAX_TOKENS rows; Q4_K, Q5_K, Q6_K): the whole-number sums of pm_launch_mmq_i8. Jobs of at most two types
 int pm_gemm_wide_check(int type, int K, int N, int T);
 int pm_launch_gemm_wide(const pm_gemm_pf_job * jobs, int njobs, const pm_q8k_wide & x, int K, int T, int pair, hipStream_t st);

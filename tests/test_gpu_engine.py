@@ -193,6 +193,25 @@ def test_prefill_mfma_path_vs_oracle(E, oracle, arch):
     w.close()
 
 
+@pytest.mark.parametrize("T,n_embd", [(72, 2048), (130, 2048)])
+def test_prompt_with_norms_behind_split_products(E, oracle, T, n_embd):
+    """K slices of wo and ffn_down are added up by the launch that also forms the next RMS norm (128-row tiles up to 128 tokens, 256-row tiles beyond): hidden rows against the oracle."""
+    torch = E.torch
+    rng = np.random.default_rng(T)
+    d = tiny_model(rng, n_layer=2, n_embd=n_embd, n_head=n_embd // 128, n_head_kv=2, n_ff=4096, n_vocab=320, n_ctx=192, rope_freqs=True, quantize=_quantizer())
+    w = E.Window(_hp(d), n_ctx=192)
+    w.load_desc(d)
+    w.finalize(max_tokens=T)
+    ho = oracle.model_new(d)
+    toks = rng.integers(0, d.n_vocab, T).astype(np.int32)
+    hid, lg, _ = w.decode(tokens=torch.from_numpy(toks).cuda(), pos0=0)
+    h_ref, l_ref = oracle.model_eval(ho, d, tokens=toks, pos0=0)
+    assert _nmse(hid.cpu().numpy(), h_ref) < 2e-3
+    assert _nmse(lg.cpu().numpy(), l_ref) < 2e-3
+    oracle.model_free(ho)
+    w.close()
+
+
 @pytest.mark.parametrize("flash,n_head,n_embd,n_head_kv", [("1", 8, 512, 2), ("1", 4, 512, 2), ("0", 8, 512, 2), ("1", 8, 1024, 4), ("1", 16, 1024, 8)])
 def test_long_context_split_attention_path(E, monkeypatch, flash, n_head, n_embd, n_head_kv):
     """Beyond PM355_ATTN_SPLIT_MIN positions the engine switches from the one-workgroup-per-head attention kernel to the
@@ -509,6 +528,33 @@ def test_batches_of_several_sequences_equal_one_sequence_at_a_time(E, arch, max_
         m.step(token=tok, logits=o)
     a, b = out.double().cpu().numpy(), out1.double().cpu().numpy()
     assert ((a - b) ** 2).sum() < 1e-3 * (b ** 2).sum()
+    w.close()
+    w1.close()
+
+
+@pytest.mark.parametrize("arch,lens,max_tokens", [(0, [20, 17, 31, 3, 1], 64), (1, [30] * 5, 256), (0, [32, 31, 30, 9] * 2, 100), (0, [1] * 40, 64), (0, [13, 20], 33)])
+def test_batches_of_short_portions_in_wide_passes(E, arch, lens, max_tokens):
+    """More rows of short portions than one small pass takes go through the prompt GEMM with 8-bit activations, portions cut where passes end; then a token of every sequence. Against the same
+    portions one at a time: the same arithmetic with other summation orders (the bound of the comparisons above)."""
+    torch = E.torch
+    rng = np.random.default_rng(len(lens))
+    d = tiny_model(rng, arch=arch, n_layer=2, n_embd=512, n_head=4, n_head_kv=2, n_ff=1024, n_vocab=320, n_ctx=64, rope_freqs=arch == 0)
+    ws = []
+    for _ in range(2):
+        w = E.Window(_hp(d), n_ctx=64)
+        w.load_desc(d)
+        w.finalize_pool(max_tokens, len(lens), len(lens) * 64)
+        ws.append((w, [w.seq_new() for _ in lens]))
+    (w, seqs), (w1, seqs1) = ws
+    for k in range(2):
+        part = [rng.integers(0, 320, n if k == 0 else 1).astype(np.int32) for n in lens]
+        lg, lg1 = torch.full((len(lens), 320), float("nan"), device="cuda"), torch.empty((len(lens), 320), device="cuda")
+        w.batch([(q, t, [len(t) - 1]) for q, t in zip(seqs, part)], logits=lg)
+        for i, t in enumerate(part):
+            w1.batch([(seqs1[i], t, [len(t) - 1])], logits=lg1[i:i + 1])
+        a, b = lg.double().cpu().numpy(), lg1.double().cpu().numpy()
+        err = ((a - b) ** 2).sum(-1) / (b ** 2).sum(-1)
+        assert (err < 1e-3).all(), (k, err.max())
     w.close()
     w1.close()
 
