@@ -78,8 +78,28 @@ template <typename T> __global__ __launch_bounds__(256) void attn_prepare_kernel
     for (int d0 = 0; d0 < a.dv; d0 += 64) {
         __syncthreads();
         const int d = d0 + lane;
-        for (int i = wave; i < nt; i += 4)
-            if (d < a.dv) tile[i * 65 + lane] = mixed_value(a, t0 + i, g * a.dv + d, ld_any(a.raw, (size_t) (t0 + i) * a.ldraw + v_off(a, g) + d, a.raw_type));
+        // all sixteen tokens of the wave on their way at once (one by one, a trip to memory each: 835 tokens of 8 KV heads 31 us, now 23)
+        const int dc = d < a.dv ? d : a.dv - 1;
+        float v[16], vf[16];
+        auto at = [&](int j) __attribute__((always_inline)) -> size_t { const int i = wave + 4 * j; return t0 + (i < nt ? i : nt - 1); };
+        if (a.raw_type == PM_F32) {
+#pragma unroll
+            for (int j = 0; j < 16; ++j) v[j] = ld_g((const float *) a.raw + at(j) * a.ldraw + v_off(a, g) + dc);
+        } else {
+#pragma unroll
+            for (int j = 0; j < 16; ++j) v[j] = bf2f(ld_g((const uint16_t *) a.raw + at(j) * a.ldraw + v_off(a, g) + dc));
+        }
+        if (a.mixes == 1)
+#pragma unroll
+            for (int j = 0; j < 16; ++j) vf[j] = a.vfirst[at(j) * a.ld_vfirst + g * a.dv + dc];
+#pragma unroll
+        for (int j = 0; j < 16; ++j) {
+            const int i = wave + 4 * j;
+            if (i >= nt || d >= a.dv) continue;
+            if (a.mixes == 1) v[j] = (1.0f - a.lambda) * v[j] + a.lambda * vf[j];
+            if (a.mixes == 2) a.vfirst[(size_t) (t0 + i) * a.ld_vfirst + g * a.dv + d] = v[j];
+            tile[i * 65 + lane] = v[j];
+        }
         __syncthreads();
         for (int i = wave; i < 64; i += 4)
             if (d0 + i < a.dv && lane < nt) vrow[(size_t) (d0 + i) * PM_PAGE] = from_f<T>(tile[lane * 65 + i]);
