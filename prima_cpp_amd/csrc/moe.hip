@@ -52,7 +52,15 @@ __global__ __launch_bounds__(1024) void route_one_kernel(pm_route r, int T, int 
         for (int k = lane; k < r.top; k += 64) { r.id[t * r.top + k] = ids[t * r.top + k]; r.w[t * r.top + k] = ws[t * r.top + k]; }
     }
     __syncthreads();
-    for (int e = threadIdx.x; e < r.E; e += 1024) {
+    // few pairs: a wave per expert, a lane per pair (a thread per expert reads the pairs one after the other, a trip to LDS each: 5 tokens x 4 of 32 experts 8.2 us, now 7.3)
+    const bool few = pairs <= 256;
+    if (few) {
+        for (int e = wave; e < r.E; e += 16) {
+            int n = 0;
+            for (int i = lane; i - lane < pairs; i += 64) n += __popcll(__builtin_amdgcn_ballot_w64(i < pairs && ids[i < pairs ? i : 0] == e));
+            if (lane == 0) count[e] = n;
+        }
+    } else for (int e = threadIdx.x; e < r.E; e += 1024) {
         int n = 0;
         for (int i = 0; i < pairs; ++i) n += ids[i] == e;
         count[e] = n;
@@ -61,10 +69,21 @@ __global__ __launch_bounds__(1024) void route_one_kernel(pm_route r, int T, int 
     if (wave == 0) prefix(count, r.E, off);
     __syncthreads();
     if (wave == 0) lists(off, r, want_tiles);
+    if (few)
+        for (int e = wave; e < r.E; e += 16) {
+            int at = off[e];
+            if (!count[e]) continue;
+            for (int i = lane; i - lane < pairs; i += 64) {
+                const bool is = i < pairs && ids[i < pairs ? i : 0] == e;
+                const uint64_t on = __builtin_amdgcn_ballot_w64(is);
+                if (is) r.order[at + __popcll(on & ((1ull << lane) - 1))] = i;
+                at += __popcll(on);
+            }
+        }
     for (int e = threadIdx.x; e <= r.E; e += 1024) {
         int at = off[e];
         r.off[e] = at;
-        if (e < r.E && count[e]) for (int i = 0; i < pairs; ++i) if (ids[i] == e) r.order[at++] = i;
+        if (!few && e < r.E && count[e]) for (int i = 0; i < pairs; ++i) if (ids[i] == e) r.order[at++] = i;
     }
 }
 
