@@ -701,7 +701,10 @@ int run_window(pm_window * m, const int32_t * d_tokens, const float * d_x_in, in
     };
     // the tokens' rows, and with them the cos / sin tables that the wq | wk | wv epilogues of all layers read
     bool attn_normed = false;                                   // a layer's attn_norm came with the launch in front of it
-    const bool one = T == 1 && !m->no_fuse, tab = (one ? m->qkv_epi && m->rope_tab : small_epi) && m->hi > m->lo;
+    // prompts of up to 255 tokens: their wq | wk | wv may end with the rope (pm_gemm_rope); without tokens the table is a launch, which a single layer does not win back
+    const bool prompt_tab = T > MMQ_MAX_TOKENS && T < 256 && !m->no_fuse && m->rope_tab && m->rope.mode == 0 && m->hi - m->lo > (d_tokens ? 0 : 1);
+    const bool one = T == 1 && !m->no_fuse, tab = (one ? m->qkv_epi && m->rope_tab : small_epi || prompt_tab) && m->hi > m->lo;
+    auto qkv_rope = [&](const Layer & L, int round_q) { return pm_gemm_rope{m->rope_tab, d_pos, d_seq, kv_stride, L.kc, L.vc, Hkv, dh, hp.n_ctx, m->rope.n_dims, round_q, rg ? 1 : 0, false}; };
     if (d_tokens) pm_launch_embed(m->tok_embd.type, m->tok_embd.d, E, d_tokens, T, m->x, st, &m->rope, d_pos, d_seq, (const float *) m->rope_freqs.d, tab ? m->rope_tab : nullptr, rg ? 1 : 0);
     else if (tab) pm_launch_rope_table(m->rope, d_pos, d_seq, (const float *) m->rope_freqs.d, m->rope_tab, st, T, rg ? 1 : 0);
     if (T == 1 && !m->no_fuse) {
@@ -785,8 +788,9 @@ int run_window(pm_window * m, const int32_t * d_tokens, const float * d_x_in, in
             float * x_next = (il == m->hi - 1 && d_x_out) ? d_x_out : ((x_mid == bufs[0]) ? bufs[1] : bufs[0]);
             pm_launch_rmsnorm_wide(cur, (const float *) L.t[PM355_T_ATTN_NORM].d, xe, E, T, hp.rms_eps, st);
             job(0, PM355_T_WQ, m->q, PM355_T_BQ, nullptr); job(1, PM355_T_WK, m->k, PM355_T_BK, nullptr); job(2, PM355_T_WV, m->v, PM355_T_BV, nullptr);
-            if (pm_launch_gemm_wide(j, 3, xe, E, T, 0, st)) return seterr(m, PM355_E_UNSUPPORTED, "batch: qkv mat-mul");
-            rope_store(L, 1);
+            pm_gemm_rope qr = qkv_rope(L, 1);
+            if (pm_launch_gemm_wide(j, 3, xe, E, T, 0, st, prompt_tab ? &qr : nullptr)) return seterr(m, PM355_E_UNSUPPORTED, "batch: qkv mat-mul");
+            if (!qr.done) rope_store(L, 1);
             if (attend_ragged(L)) return seterr(m, PM355_E_RANGE, "batch: n_ctx too large for the attention kernels");
             pm_launch_quantize_wide(m->att, xa, Eq, T, st);
             job(0, PM355_T_WO, x_mid, -1, cur);
@@ -821,17 +825,18 @@ int run_window(pm_window * m, const int32_t * d_tokens, const float * d_x_in, in
             if (!attn_normed) pm_launch_rmsnorm_q8k(cur, (const float *) L.t[PM355_T_ATTN_NORM].d, nullptr, nullptr, E, T, hp.rms_eps, st, m->xn);
             // wq | wk | wv: ONE launch over the shared activations, each matrix with its own quant type (mmq_pf.hip jobs; wk / wv alone - N = n_head_kv * head_dim -
             // filled a fraction of the chip: 212 TFLOP/s as their own launches)
-            int rc;
+            int rc = 0;
+            pm_gemm_rope qr = qkv_rope(L, 0);
             {
                 const Tensor & wq = L.t[PM355_T_WQ], & wk = L.t[PM355_T_WK], & wv = L.t[PM355_T_WV];
                 const pm_gemm_pf_job qkvj[3] = {
                     {wq.type, (int) wq.N, wq.d, m->q, nullptr, (const float *) L.t[PM355_T_BQ].d, nullptr, nullptr, 0},
                     {wk.type, (int) wk.N, wk.d, m->k, nullptr, (const float *) L.t[PM355_T_BK].d, nullptr, nullptr, 0},
                     {wv.type, (int) wv.N, wv.d, m->v, nullptr, (const float *) L.t[PM355_T_BV].d, nullptr, nullptr, 0}};
-                rc = pm_launch_gemm_q_multi(qkvj, 3, nullptr, m->xn, E, T, st);
+                if (!(prompt_tab && pm_gemm_pf_enabled() && pm_launch_gemm_pf_rope(qkvj, m->xn, E, T, &qr, st) == 0)) rc = pm_launch_gemm_q_multi(qkvj, 3, nullptr, m->xn, E, T, st);
             }
             if (rc) return seterr(m, PM355_E_UNSUPPORTED, "prefill: qkv gemm");
-            rope_store(L, 0);
+            if (!qr.done) rope_store(L, 0);
             bool att_h = true;
             if (attend_mfma(L, nullptr, m->att)) {
                 att_h = false;
@@ -1134,7 +1139,7 @@ int pm_window::finalize(int max_tokens_, int n_seq_) {
               A((void **) &m->aq_k, T * pm_q8k_row_bytes((int) ((maxK + 255) / 256 * 256))) &&
               A((void **) &m->aq_0, T * pm_q80_row_bytes((int) ((maxK + 31) / 32 * 32))) &&
               A((void **) &m->d_pos, 64 * 4) && A((void **) &m->d_ctl, 64) && A((void **) &m->d_tok, 64 + T * 4) &&
-              A((void **) &m->rope_tab, (size_t) hp.head_dim * 4 * 32) &&      // cos / sin tables of up to 32 tokens (small-batch epilogue)
+              A((void **) &m->rope_tab, (size_t) hp.head_dim * 4 * std::max<size_t>(32, std::min<size_t>(T, 256))) &&      // cos / sin tables of the tokens (small-batch epilogue, prompts)
               A((void **) &m->ss, 2 * 256 * sizeof(double)) &&
               A((void **) &m->att_tk, 65 * 4) && A((void **) &m->d_last, 64 * 4);
     ok = ok && A((void **) &m->am_part, PM_ARGMAX_SCRATCH);

@@ -926,6 +926,45 @@ template <int SMAX> __global__ __launch_bounds__(1024) void pf_reduce_norm_kerne
     }
 }
 
+// The same for wq | wk | wv, with NORM rope (rope_kv_store_kernel's expressions, cos / sin from the pass's table) and the stores of K and V^T into the cache: the launch behind it and two trips of the
+// rows go. Bound by the chain of its loads. 101 tokens of 32 + 8 + 8 heads of 128, S = 4: 5.1 + 7.3 us as two launches, 6.4 as this one
+template <int SMAX> __global__ __launch_bounds__(1024) void pf_reduce_rope_kernel(PfP p, int mid, int nti, pm_gemm_rope a) {
+    constexpr int NWV = 16, HOLD = 3;                           // rows of 256: up to 48
+    const int t = blockIdx.x, lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane((int) threadIdx.x >> 6), S = p.splitk;
+    const int Nq = p.job[0].N, Nk = p.job[1].N, rows = mid ? 128 : 256, tok = mid ? 64 * nti : 32 * nti;
+    const int tile_t = t / tok, tt = t % tok / 32, half = mid ? tt / nti : 0, i = mid ? tt % nti : tt;
+    const size_t tile = (size_t) 8 * nti * 256;                 // of f32x4
+    const int seq = a.seq ? a.seq[a.rows ? t : 0] : 0, pos = a.rows ? a.pos[t] : a.pos[seq] + t;
+    uint16_t * const kc = (uint16_t *) a.kc + (long) seq * a.seq_stride + (long) pos * Nk, * const vc = (uint16_t *) a.vc + (long) seq * a.seq_stride + pos;
+#pragma unroll
+    for (int j = 0; j < HOLD; ++j) {
+        const int n0 = (wv + NWV * j) * 256;                    // (a wave's 256 rows are of one matrix)
+        if (n0 >= Nq + 2 * Nk) continue;
+        const int what = n0 < Nq ? 0 : n0 < Nq + Nk ? 1 : 2, n = n0 - (what == 0 ? 0 : what == 1 ? Nq : Nq + Nk) + 4 * lane;
+        const int tile0 = what == 0 ? 0 : what == 1 ? p.job[1].tile0 : p.job[2].tile0;
+        const float * const bias = what == 0 ? p.job[0].bias : what == 1 ? p.job[1].bias : p.job[2].bias;
+        const int tile_n = tile0 + n / rows, wave = n % rows / 32 + 4 * half, d = n % a.dh;
+        const f32x4 * const at = (const f32x4 *) p.ws + (size_t) (((tile_n >> 3) * p.nt_t + tile_t) * 8 + (tile_n & 7)) * S * tile + (size_t) (wave * nti + i) * 256 + (t & 31) * 8 + (lane & 7);
+        f32x4 v[SMAX], o = {0.0f, 0.0f, 0.0f, 0.0f}, cs = {1.0f, 0.0f, 1.0f, 0.0f};
+#pragma unroll
+        for (int q = 0; q < SMAX; ++q) v[q] = *(const PM_G f32x4 *) (at + (size_t) (q < S ? q : S - 1) * tile);
+        const f32x4 b = bias ? ld_g((const f32x4 *) (bias + n)) : o;
+        if (what < 2 && d < a.n_dims) cs = ld_g((const f32x4 *) (a.tab + (size_t) t * a.n_dims + d));
+#pragma unroll
+        for (int q = 0; q < SMAX; ++q) if (q < S) o += v[q];
+        if (bias) o += b;
+        if (what == 2) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) vc[(long) (n + e) * a.n_ctx] = f2h(o[e]);
+            continue;
+        }
+        if (d < a.n_dims) o = f32x4{o[0] * cs[0] - o[1] * cs[1], o[0] * cs[1] + o[1] * cs[0], o[2] * cs[2] - o[3] * cs[3], o[2] * cs[3] + o[3] * cs[2]};
+        const uint16_t h[4] = {f2h(o[0]), f2h(o[1]), f2h(o[2]), f2h(o[3])};
+        if (what == 1) *(PM_G u32x2 *) (kc + n) = u32x2{(uint32_t) h[0] | (uint32_t) h[1] << 16, (uint32_t) h[2] | (uint32_t) h[3] << 16};
+        else *(PM_G f32x4 *) (p.job[0].Y + (long) t * Nq + n) = a.round_q ? f32x4{h2f(h[0]), h2f(h[1]), h2f(h[2]), h2f(h[3])} : o;
+    }
+}
+
 template <int TA, int TB, int NT, bool MID = false, bool EX = false> constexpr size_t pf_lds_bytes() {
     if (!MID) return (size_t) 3 * NT * 32 * 128 + (size_t) 8 * (pf_wave_bytes<TA>() > pf_wave_bytes<TB>() ? pf_wave_bytes<TA>() : pf_wave_bytes<TB>());
     return mid_lds_bytes<TA, NT, EX>() > mid_lds_bytes<TB, NT, EX>() ? mid_lds_bytes<TA, NT, EX>() : mid_lds_bytes<TB, NT, EX>();
@@ -1020,7 +1059,7 @@ int pm_launch_gemm_pf(const pm_gemm_pf_job * jobs, int njobs, const void * xh, i
 
 // pair != 0: jobs[0] = ffn_gate, jobs[1] = ffn_up (same type, same N; jobs[0]'s outputs are ignored): jobs[1]'s output = silu(W0 . x) * (W1 . x) (+ its own bias / resid
 // before the product are NOT applied to the gate). One launch, the gate result stays on the chip.
-static int launch_pf(const pm_gemm_pf_job * jobs, int njobs, const void * xh, const pm_q8k_wide * wide, int K, int T, int pair, hipStream_t st, pm_gemm_norm * norm = nullptr) {
+static int launch_pf(const pm_gemm_pf_job * jobs, int njobs, const void * xh, const pm_q8k_wide * wide, int K, int T, int pair, hipStream_t st, pm_gemm_norm * norm = nullptr, pm_gemm_rope * rope = nullptr) {
     if (njobs < 1 || njobs > PF_MAX_JOBS || !jobs || !xh) return -2;
     if (pair && (njobs != 2 || jobs[0].type != jobs[1].type || jobs[0].N != jobs[1].N || jobs[0].bias || jobs[0].resid || jobs[1].silu_gate)) return -2;
     static const int force_nt = [] { const char * e = getenv("PM355_GEMM_PF_NT"); return e ? atoi(e) : 0; }();
@@ -1082,6 +1121,15 @@ static int launch_pf(const pm_gemm_pf_job * jobs, int njobs, const void * xh, co
             norm->done = true;
             return;
         }
+        // (a token's V^T is 2-byte pieces n_ctx apart: from 256 tokens on rope_kv_prompt_kernel turns them in tiles)
+        bool roped = rope && !full && T < 256 && njobs == 3 && !p.pair && jobs[1].N == jobs[2].N && jobs[1].N == rope->Hkv * rope->dh && jobs[0].N + 2 * jobs[1].N <= 48 * 256 && rope->dh % 4 == 0 && rope->n_dims % 4 == 0;
+        for (int j = 0; j < njobs && roped; ++j) roped = jobs[j].N % 256 == 0 && jobs[j].Y && !jobs[j].Yh && !jobs[j].resid && !jobs[j].silu_gate && p.job[j].ldy == p.job[j].N && jobs[j].N % rope->dh == 0;
+        if (roped) {
+            if (S <= 4) hipLaunchKernelGGL(pf_reduce_rope_kernel<4>, dim3(T), dim3(1024), 0, st, p, (int) mid, nti, *rope);
+            else        hipLaunchKernelGGL(pf_reduce_rope_kernel<8>, dim3(T), dim3(1024), 0, st, p, (int) mid, nti, *rope);
+            rope->done = true;
+            return;
+        }
         const int units = 8 * split_slots * (p.pair ? 4 : 8) * nti;
         if (S <= 4) hipLaunchKernelGGL((pf_reduce_kernel<4, 1>), dim3(units), dim3(256), 0, st, p, (int) mid, nti, units);
         else        hipLaunchKernelGGL((pf_reduce_kernel<8, 1>), dim3(units), dim3(256), 0, st, p, (int) mid, nti, units);
@@ -1122,16 +1170,18 @@ static int launch_pf(const pm_gemm_pf_job * jobs, int njobs, const void * xh, co
 }
 int pm_launch_gemm_pf_ex(const pm_gemm_pf_job * jobs, int njobs, const void * xh, int K, int T, int pair, hipStream_t st) { return launch_pf(jobs, njobs, xh, nullptr, K, T, pair, st); }
 
+int pm_launch_gemm_pf_rope(const pm_gemm_pf_job * jobs, const void * xh, int K, int T, pm_gemm_rope * rope, hipStream_t st) { rope->done = false; return launch_pf(jobs, 3, xh, nullptr, K, T, 0, st, nullptr, rope); }
 int pm_launch_gemm_pf_norm(const pm_gemm_pf_job & job, const void * xh, int K, int T, pm_gemm_norm * norm, hipStream_t st) { norm->done = false; return launch_pf(&job, 1, xh, nullptr, K, T, 0, st, norm); }
 
 int pm_gemm_wide_check(int type, int K, int N, int T) {
     if ((type != PM_Q4_K && type != PM_Q5_K && type != PM_Q6_K) || T < 1 || T > PM_WIDE_MAX_TOKENS) return -1;
     return pm_gemm_pf_check(type, K, N, T);
 }
-int pm_launch_gemm_wide(const pm_gemm_pf_job * jobs, int njobs, const pm_q8k_wide & x, int K, int T, int pair, hipStream_t st) {
+int pm_launch_gemm_wide(const pm_gemm_pf_job * jobs, int njobs, const pm_q8k_wide & x, int K, int T, int pair, hipStream_t st, pm_gemm_rope * rope) {
+    if (rope) rope->done = false;
     if (T > PM_WIDE_MAX_TOKENS || !x.q || x.ldt < (T <= 64 ? 64 : (T + 127) / 128 * 128) || x.ldt % 4 || (size_t) (K / 256) * x.ldt * 32 >= ((size_t) 1 << 32)) return -2;
     for (int j = 0; j < njobs; ++j) if (pm_gemm_wide_check(jobs[j].type, K, jobs[j].N, T)) return -1;
-    return launch_pf(jobs, njobs, x.q, &x, K, T, pair, st);
+    return launch_pf(jobs, njobs, x.q, &x, K, T, pair, st, nullptr, rope);
 }
 size_t pm_q8k_wide_bytes(int K) { return (size_t) PM_WIDE_MAX_TOKENS * ((size_t) K * 2 + (size_t) (K / 256) * 36); }
 pm_q8k_wide pm_q8k_wide_at(void * buf, int K) {

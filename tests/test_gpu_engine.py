@@ -195,7 +195,8 @@ def test_prefill_mfma_path_vs_oracle(E, oracle, arch):
 
 @pytest.mark.parametrize("T,n_embd", [(72, 2048), (130, 2048)])
 def test_prompt_with_norms_behind_split_products(E, oracle, T, n_embd):
-    """K slices of wo and ffn_down are added up by the launch that also forms the next RMS norm (128-row tiles up to 128 tokens, 256-row tiles beyond): hidden rows against the oracle."""
+    """K slices of wo and ffn_down are added up by the launch that also forms the next RMS norm, those of wq | wk | wv by one that rotates and stores (128-row tiles up to 128 tokens, 256-row
+    tiles beyond): hidden rows against the oracle."""
     torch = E.torch
     rng = np.random.default_rng(T)
     d = tiny_model(rng, n_layer=2, n_embd=n_embd, n_head=n_embd // 128, n_head_kv=2, n_ff=4096, n_vocab=320, n_ctx=192, rope_freqs=True, quantize=_quantizer())
