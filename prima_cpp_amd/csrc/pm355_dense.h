@@ -191,10 +191,7 @@ template <> __device__ __forceinline__ float from_f<float>(float v) { return v; 
 template <> __device__ __forceinline__ uint16_t from_f<uint16_t>(float v) { return f2bf(v); }
 __device__ __forceinline__ float ld_any(const void * p, size_t i, int type) { return type == PM_BF16 ? bf2f(((const uint16_t *) p)[i]) : ((const float *) p)[i]; }
 __device__ __forceinline__ void st_type(void * p, size_t i, int type, float v) { if (type == PM_BF16) ((uint16_t *) p)[i] = f2bf(v); else ((float *) p)[i] = v; }
-__device__ __forceinline__ float wave_max(float v) {
-    for (int o = 32; o; o >>= 1) v = fmaxf(v, __shfl_xor(v, o));
-    return v;
-}
+__device__ __forceinline__ float wave_max(float v) { return all_max(v); }
 // 1 KiB of LDS at byte address `dst` (wave-uniform) <- 64 x 16 bytes, lane l from base + voff (its own 32-bit offset). Inline asm for the reason given in mmq_pf.hip:
 // an LDS-DMA the compiler can see turns its counted lgkmcnt waits into full drains. The caller waits with pm_vm_drain().
 __device__ __forceinline__ void pm_dma16(const void * base, uint32_t voff, uint32_t dst) {
