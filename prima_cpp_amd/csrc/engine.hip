@@ -1418,8 +1418,9 @@ int pm_window::batch_rows(const pm355_batch_entry * e, int n, float * d_logits, 
             for (int off = 0; off < e[i].n_tokens; off += max_tokens) { const int T = std::min(max_tokens, e[i].n_tokens - off); if (mine(T)) total += T; }
         // rows of short portions that need more than one small pass go out as wide ones. Prompts of two layers, us, small passes / wide: 8B shape, 40 rows in all 530 / 416, 80 904 / 553, 192 1808 / 795,
         // Q6_K 679 / 451, 1120 / 590, 2211 / 878; 70B shape 1087 / 917, 1818 / 1247, 3578 / 1976, Q6_K 1394 / 1018, 2252 / 1380, 4407 / 2225 (192 rows as two passes of 96: 1069 on the 8B shape)
-        const bool wd = wide && every && most == MMQ_MAX_TOKENS && total > most;
-        const int cap = wd ? std::min(max_tokens, PM_WIDE_MAX_TOKENS) : most;
+        const int cap_w = std::min(max_tokens, PM_WIDE_MAX_TOKENS);
+        const bool wd = wide && every && most == MMQ_MAX_TOKENS && total > most && total / ((total + cap_w - 1) / cap_w) > most;
+        const int cap = wd ? cap_w : most;
         const int64_t k = (total + cap - 1) / cap;                                                         // passes of equal size: more than `above` rows, like every portion of the tier
         int64_t at = 0;
         for (int i = 0, out0 = 0; i < n; out0 += e[i].n_want, ++i)
