@@ -8,11 +8,12 @@
 //
 // Why a second kernel: at short contexts the fused kernel is a chain of dependent latencies (position -> rope -> LDS -> barrier ->
 // 128-term dot per THREAD -> two block reductions -> P.V -> reduction): 7.4 us per 70B layer for ~0 bytes. Here
-//   * up to 256 cells (head sizes up to 128; 64 cells for 256): attn_whole_lines (attn_tail_device.h), every load issued first, ONE workgroup barrier.
-//   * more cells (up to the long-context threshold): the per-head body of attn_device.h in its CACHED form.
+//   * up to 256 cells (head sizes up to 128; 64 cells for 256), where the cache has as many as the form takes: attn_short, every load issued first, ONE workgroup barrier.
+//   * the rest (up to the long-context threshold): the per-head body of attn_device.h in its CACHED form.
 #include "attn_device.h"
-#include "attn_tail_device.h"
+#include "pm355_kernels.h"
 #include "pm355_layer_ops.h"
+#include <algorithm>
 #include <type_traits>
 
 namespace {
@@ -29,6 +30,111 @@ __global__ __launch_bounds__(128) void rope_table_kernel(RopeP r, const int32_t 
     }
 }
 
+// What a wave of attn_short stages, bytes: rows of 16 KPL keys, then the same memory for its DH / 4 rows of V^T (16 bytes more than the data: consecutive rows start 4 banks on)
+template <int DH, int KPL> struct ShortLds {
+    static constexpr int K_PITCH = 2 * DH + 16, V_PITCH = 128 * KPL + 16, K = 16 * KPL * K_PITCH, V = DH / 4 * V_PITCH, STAGE = K > V ? K : V;
+    static constexpr int BYTES = 64 * KPL * (4 + 4 * 2) + 4 * (STAGE + DH * 4);   // scores | probabilities of each wave | q and stage of each wave
+};
+// Up to 64 * KPL cells, four waves per head. What bounds it is the number of cache lines a CU asks for, so an instruction takes whole lines: K - DH / 8 lanes hold a key's row, V^T - 8 KPL lanes a
+// dimension's cells - a wave a quarter of the keys and a quarter of the dimensions. They are multiplied out of LDS, which a wave fills for itself (no barrier): the sums of a decoded token stay
+// what a lane per key and a lane per dimension make them - the dimensions of a quarter in a row, the quarters as (0 + 1) + (2 + 3); the cells of a dimension in 64 / (DH / 4) rows, one lane each.
+// us per launch of 32 heads of 128 over 36 / 100 / 204 cells: a lane's own key and dimension straight from memory 3.3 / 4.4 / 7.0, this 2.8 / 3.7 / 5.7 (multiplied in the registers that the
+// lines arrive in, sums over lanes, 2.6 / 3.1 / 4.5: one other bit here turns 8-bit roundings behind it, 3 % of the logits of eight layers of the 8B shape).
+// Rounding points as everywhere: q, K, V F16, the normalised probabilities rounded to F16, f32 accumulation. n_kv <= 64 * KPL <= n_ctx; DH 64 / 128 (256: KPL = 1).
+template <int DH, int KPL>
+__device__ __forceinline__ void attn_short(const float * q_head, const uint16_t * kc, const uint16_t * vc, float * out_head, int hk, int Hkv, int n_ctx, int n_kv, float scale, const void * mask,
+                                           int mask_f16, char * smem, int lane, int wave) {
+    typedef ShortLds<DH, KPL> S;
+    constexpr int NKEY = 64 * KPL, NKW = NKEY / 4, LPK = DH / 8, KPI = 64 / LPK, NI = NKW / KPI, DPW = DH / 4, LV = 8 * KPL, DPI = 64 / LV, NV = DPW / DPI, KPP = NKEY * DPW / 64;
+    float * const part = (float *) smem, * const qs = (float *) (smem + 12 * NKEY) + DH * wave;
+    uint16_t * const pw = (uint16_t *) (part + NKEY) + NKEY * wave;
+    char * const st = smem + 12 * NKEY + 4 * DH * 4 + S::STAGE * wave;
+    const int kd = lane % LPK, ks = lane / LPK, c = lane % LV, ve = lane / LV;
+    const float * const qu = uniform_const_ptr(q_head);        // (every lane in the same quarter: q through the scalar cache)
+    f32x4 q4;
+    if constexpr (KPL < 4) q4 = *(const PM_G f32x4 *) (q_head + 4 * (lane % DPW));
+    u32x4 kreg[NI], vreg[NV];
+#pragma unroll
+    for (int i = 0; i < NI; ++i) kreg[i] = *(const PM_G u32x4 *) (kc + (long) max(min(KPI * (4 * i + wave) + ks, n_kv - 1), 0) * Hkv * DH + (long) hk * DH + 8 * kd);
+#pragma unroll
+    for (int i = 0; i < NV; ++i) vreg[i] = *(const PM_G u32x4 *) (vc + (long) (hk * DH + DPW * wave + DPI * i + ve) * n_ctx + (8 * c < n_kv ? 8 * c : 0));
+    float m_add[KPL];
+#pragma unroll
+    for (int k = 0; k < KPL; ++k) m_add[k] = lane + 64 * k < n_kv ? attn_mask_at(mask, mask_f16, lane + 64 * k) : 0.0f;
+    auto staged = []() __attribute__((always_inline)) {        // (a wave's LDS accesses execute in order: what it wrote is there for its other lanes, what it has read may be overwritten)
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+    };
+    if constexpr (KPL < 4) if (lane < DPW) *(f32x4 *) (qs + 4 * lane) = q4;
+#pragma unroll
+    for (int i = 0; i < NI; ++i) *(u32x4 *) (st + (KPI * i + ks) * S::K_PITCH + 16 * kd) = kreg[i];
+    staged();
+    // ---- scores: lane = (key l of the wave, quarters u0 .. u0 + KPL - 1 of the head)
+    const int l = lane % NKW, u0 = KPL * (lane / NKW);
+    float acc[KPL];
+#pragma unroll
+    for (int u = 0; u < KPL; ++u) acc[u] = 0.0f;
+#pragma unroll
+    for (int j = 0; j < DPW / 8; ++j)
+#pragma unroll
+        for (int u = 0; u < KPL; ++u) {
+            const int d = DPW * (u0 + u) + 8 * j;
+            const u32x4 w = *(const u32x4 *) (st + l * S::K_PITCH + 2 * d);
+            f32x4 q[2];
+            if constexpr (KPL < 4) { q[0] = *(const f32x4 *) (qs + d); q[1] = *(const f32x4 *) (qs + d + 4); }
+            else
+#pragma unroll
+                for (int t = 0; t < 8; ++t) q[t >> 2][t & 3] = qu[DPW * u + 8 * j + t];
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+                acc[u] = fmaf(h2f((uint16_t) (w[t] & 0xFFFF)), q[t >> 1][2 * (t & 1)], acc[u]);
+                acc[u] = fmaf(h2f((uint16_t) (w[t] >> 16)), q[t >> 1][2 * (t & 1) + 1], acc[u]);
+            }
+        }
+    float s = acc[0];
+    if constexpr (KPL == 1) s += __builtin_bit_cast(float, other_row(__builtin_bit_cast(uint32_t, s)));
+    else s += acc[1];
+    if constexpr (KPL == 4) s += acc[2] + acc[3];
+    else s += __builtin_bit_cast(float, other_half(__builtin_bit_cast(uint32_t, s)));
+    if (lane < NKW) part[KPI * (4 * (l / KPI) + wave) + l % KPI] = s;
+    staged();
+#pragma unroll
+    for (int i = 0; i < NV; ++i) *(u32x4 *) (st + (DPI * i + ve) * S::V_PITCH + 16 * c) = vreg[i];
+    __syncthreads();                                           // the only workgroup barrier of this path
+    float s_[KPL], mx = -INFINITY;
+#pragma unroll
+    for (int k = 0; k < KPL; ++k) {
+        const int key = lane + 64 * k;
+        s_[k] = key < n_kv ? part[key] * scale + m_add[k] : -INFINITY;
+        mx = fmaxf(mx, s_[k]);
+    }
+    mx = all_max(mx);
+    float ex[KPL];
+    double tot = 0.0;
+#pragma unroll
+    for (int k = 0; k < KPL; ++k) { ex[k] = lane + 64 * k < n_kv ? expf(s_[k] - mx) : 0.0f; tot += (double) ex[k]; }
+    const float inv = (float) (1.0 / all_sum(tot));
+#pragma unroll
+    for (int k = 0; k < KPL; ++k) pw[lane + 64 * k] = f2h(ex[k] * inv);            // p rounded to F16 (src1 of the V^T.p product)
+    staged();
+    // ---- P.V: lane = (dimension e, part kp of the cells). Pieces without an attended cell repeat the row's first one, against probabilities of zero
+    const int e = lane % DPW, kp = lane / DPW;
+    float o = 0.0f;
+#pragma unroll
+    for (int j = 0; j < KPP / 8; ++j) {
+        const u32x4 w = *(const u32x4 *) (st + e * S::V_PITCH + 2 * (KPP * kp + 8 * j));
+        const u32x4 p = *(const u32x4 *) (pw + KPP * kp + 8 * j);
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+            o = fmaf(h2f((uint16_t) (w[t] & 0xFFFF)), h2f((uint16_t) (p[t] & 0xFFFF)), o);
+            o = fmaf(h2f((uint16_t) (w[t] >> 16)), h2f((uint16_t) (p[t] >> 16)), o);
+        }
+    }
+    if constexpr (DPW <= 16) o += __builtin_bit_cast(float, other_row(__builtin_bit_cast(uint32_t, o)));
+    if constexpr (DPW <= 32) o += __builtin_bit_cast(float, other_half(__builtin_bit_cast(uint32_t, o)));
+    if (lane < DPW) st_g(out_head + DPW * wave + lane, o);
+}
+
 template <int DH, int VM>
 __global__ __launch_bounds__(256) void attn_cached_kernel(AttnP a_in) {
     // grid.y = tokens of a small batch (engine: 2..64-token steps after rope_kv_store has rotated / rounded q and stored every token's K / V):
@@ -39,7 +145,6 @@ __global__ __launch_bounds__(256) void attn_cached_kernel(AttnP a_in) {
     extern __shared__ __attribute__((aligned(16))) char smem[];
     __shared__ float redf[8];
     __shared__ double redd[4];
-    __shared__ __attribute__((aligned(16))) float part[256], pw[4][256];       // scores, probabilities by wave (attn_whole_lines)
     const int h = blockIdx.x;
     if constexpr (VM == 0) {
         const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -51,14 +156,14 @@ __global__ __launch_bounds__(256) void attn_cached_kernel(AttnP a_in) {
             n_kv = uniform_const_ptr(a.pos0_ptr)[a.rows ? a.tok : seq] + 1 + (a.rows ? 0 : a.tok);
         }
         const uint16_t * kc = a.kc + (long) seq * a.seq_stride, * vc = a.vc + (long) seq * a.seq_stride;
-        auto bar = [&]() __attribute__((always_inline)) { __syncthreads(); };
-        auto whole = [&](auto kpl) __attribute__((always_inline)) {
-            attn_whole_lines<DH, decltype(kpl)::value, false>(a.q + (long) h * DH, kc, vc, a.out + (long) h * DH, hk, Hkv, n_ctx, n_kv, a.scale, a.mask, a.mask_f16, part, &pw[0][0], lane, wave, bar);
+        auto go = [&](auto kpl) __attribute__((always_inline)) {
+            attn_short<DH, decltype(kpl)::value>(a.q + (long) h * DH, kc, vc, a.out + (long) h * DH, hk, Hkv, n_ctx, n_kv, a.scale, a.mask, a.mask_f16, smem, lane, wave);
         };
-        if (n_kv <= 64) return whole(std::integral_constant<int, 1>());
+        // (caches that hold fewer cells than the form takes: the general body, as it always was - its sums are in another order)
+        if (n_kv <= 64 && n_ctx >= 64) return go(std::integral_constant<int, 1>());
         if constexpr (DH <= 128) {
-            if (n_kv <= 128) return whole(std::integral_constant<int, 2>());
-            if (n_kv <= 256) return whole(std::integral_constant<int, 4>());
+            if (n_kv <= 128 && n_ctx >= 128) return go(std::integral_constant<int, 2>());
+            if (n_kv <= 256 && n_ctx >= 256) return go(std::integral_constant<int, 4>());
         }
     }
     attn_rope_body<DH, false, VM, true>(a, h, smem, redf, redd);
@@ -78,13 +183,17 @@ int pm_launch_attn_cached(const float * q, void * kc, void * vc, const int32_t *
                           int H, int Hkv, int dh, int n_ctx, float scale, hipStream_t st, const int32_t * dyn, const void * mask,
                           int max_keys, int v_rowmajor, int mask_f16, int n_tok, int rows) {
     if ((dh != 64 && dh != 128 && dh != 256) || n_ctx % 8 || n_tok < 1 || (n_tok > 1 && dyn) || (rows && (dyn || !seq || !pos0))) return -1;
-    const size_t lds = (size_t) (4 * dh + (v_rowmajor ? 2048 : 256) + (max_keys > 0 ? ((max_keys + 7) & ~7) : n_ctx) + 8) * 4;
+    size_t lds = (size_t) (4 * dh + (v_rowmajor ? 2048 : 256) + (max_keys > 0 ? ((max_keys + 7) & ~7) : n_ctx) + 8) * 4;
     if (lds > 150 * 1024) return -1;
+    // (two workgroups of the largest short form per CU, as many as their registers allow)
+    const int kpl = v_rowmajor || n_ctx < 64 ? 0 : n_ctx < 128 || dh > 128 ? 1 : n_ctx < 256 ? 2 : 4;
+    if (kpl) lds = std::max(lds, (size_t) (dh == 256 ? ShortLds<256, 1>::BYTES : dh == 128 ? kpl == 1 ? ShortLds<128, 1>::BYTES : kpl == 2 ? ShortLds<128, 2>::BYTES : ShortLds<128, 4>::BYTES :
+                                           kpl == 1 ? ShortLds<64, 1>::BYTES : kpl == 2 ? ShortLds<64, 2>::BYTES : ShortLds<64, 4>::BYTES));
     RopeP r = {};
     if (!pos0) pos0 = dyn;                       // ggml-graph mode: cells come from dyn; keep every pointer the kernel may touch valid
     if (!pos0) return -1;
     auto launch = [&](auto kern) {
-        if (lds > 48 * 1024) (void) hipFuncSetAttribute((const void *) kern, hipFuncAttributeMaxDynamicSharedMemorySize, 150 * 1024);
+        pm_allow_big_lds((const void *) kern, lds);
         AttnP a = {q, nullptr, nullptr, (uint16_t *) kc, (uint16_t *) vc, pos0, seq, seq_stride, nullptr, out, H, Hkv, n_ctx, scale, r, dyn,
                    (const float *) mask, mask_f16, pm_ts_next_slot(), 0, rows};
         hipLaunchKernelGGL(kern, dim3(H, n_tok), dim3(256), lds, st, a);

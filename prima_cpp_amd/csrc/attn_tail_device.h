@@ -1,7 +1,8 @@
 // attn_tail_device.h — single-token attention over cached cells for callers INSIDE a launch that also produced q and this token's cell
 // (the QKV launch's tail: mmvq.hip; the persistent engine's attention phase: decode_engine.hip). The arithmetic, its order and its rounding points are
 // attn_cached.hip's (ggml.c:12445-12473 K.q rows, :13783-13879 soft_max, F16-rounded probabilities against the F16 V rows: the reference's
-// ggml_compute_forward_mul_mat with an F16 src1 conversion) - the outputs are the same bits as attn_cached.hip's OF THE SAME ROUND (up to 256 cells both take attn_whole_lines below);
+// ggml_compute_forward_mul_mat with an F16 src1 conversion) - the outputs are the same bits as attn_cached.hip's (up to 256 cells both add four quarters of a head's
+// dimensions, each in a row, and the cells of a dimension in a row; the per-head body beyond adds in another order);
 // what differs is how memory is read: q and the newest
 // cell were written by OTHER compute units in this launch, so every load of q / K / V bypasses this XCD's caches (sc0 sc1).
 #pragma once
@@ -22,96 +23,75 @@ __device__ __forceinline__ u32x4 coh_ld16u(__amdgpu_buffer_rsrc_t r, uint32_t of
 __device__ __forceinline__ float coh_ld4(__amdgpu_buffer_rsrc_t r, uint32_t off) { return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, (int) off, 0, 17)); }
 
 
-// ---- up to 64 * KPL cells, four waves per head: every load is issued before anything is computed, ONE barrier. What bounds it is the number of cache lines a CU asks for, so an instruction
-// takes whole lines: K - DH / 8 lanes hold a key's row, a wave 4 keys of head_dim 128 at once; V^T - 8 KPL lanes hold a dimension's cells, eight each. (A key per lane, and a dimension per
-// lane for V - 64 lines an instruction, 8192 for a head of 128 over 256 cells instead of 1024: 7.9 us per launch of 32 heads x 204 cells, now 5.0; 4.3 at 36 cells, now 3.8.)
-// Rounding points as everywhere: q, K, V F16, the normalised probabilities rounded to F16, f32 accumulation. n_kv <= 64 * KPL, n_ctx a multiple of 8; DH 64 / 128 (256: KPL = 1).
-// COH: q / K / V through cache-bypassing loads, the output written through (callers inside a launch that produced them: attn_tail_head below).
-// part: LDS [64 * KPL] floats, pw: [4][64 * KPL]; bar(): barrier of exactly the four waves.
-template <int DH, int KPL, bool COH, class Bar>
-__device__ __forceinline__ void attn_whole_lines(const float * q_head, const uint16_t * kc, const uint16_t * vc, float * out_head, int hk, int Hkv, int n_ctx, int n_kv,
-                                                 float scale, const void * mask, int mask_f16, float * part, float * pw, int lane, int wave, Bar && bar) {
-    constexpr int NKEY = 64 * KPL, LPK = DH / 8, KPI = 64 / LPK, NI = NKEY / (4 * KPI), LV = 8 * KPL, DPI = 64 / LV, NV = DH / 4 / DPI, LR = LV < 16 ? LV : 16;
-    static_assert(NI <= LPK && NV <= LR, "a lane keeps one result of each kind");
-    u32x4 kreg[NI], vreg[NV];
+// ---- up to 64 * KPL cells with the KEYS IN THE LANES (attn_cached.hip's attn_short without its whole lines: the caller's LDS has no room for them): lane l owns keys l, l + 64, ...,
+// wave w the head dimensions [DPW w, DPW w + DPW); every load is issued before anything is computed, ONE barrier of the four waves. The general body
+// (thread per key, three reductions, a score buffer) costs 7.1 us per launch at 65 cells and 9.1 at 256 where this form costs ~4 (tools/r5/attn_short_probe.py).
+// Rounding points as everywhere: q, K, V F16, the normalised probabilities rounded to F16, f32 accumulation. n_kv <= 64 * KPL <= n_ctx, DH 64 / 128.
+// q / K / V through cache-bypassing loads, the output written through.
+// part / pw: LDS [4][64 * KPL] floats each; qstrip: LDS [DH] floats; bar(): barrier of exactly the four waves.
+template <int DH, int KPL, class Bar>
+__device__ __forceinline__ void attn_keys_in_lanes(const float * q_head, const uint16_t * kc, const uint16_t * vc, float * out_head, int hk, int Hkv, int n_ctx, int n_kv,
+                                                   float scale, float * part, float * pw, float * qstrip, int lane, int wave, Bar && bar) {
+    constexpr int NKEY = 64 * KPL, DPW = DH / 4, NK = DPW / 8, KP = 64 / DPW, KPP = NKEY / KP, NV = KPP / 8;
+    u32x4 kreg[KPL][NK], vreg[NV];
     const __amdgpu_buffer_rsrc_t rk = coh_rsrc(kc), rv = coh_rsrc(vc), rq = coh_rsrc(q_head);
-    const int kd = lane % LPK, ks = lane / LPK, c = lane % LV, ve = lane / LV;
-    f32x4 q[2];
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-        if constexpr (COH) q[j] = __builtin_bit_cast(f32x4, coh_ld16u(rq, (uint32_t) ((8 * kd + 4 * j) * 4)));
-        else q[j] = *(const PM_G f32x4 *) (q_head + 8 * kd + 4 * j);
-    }
-#pragma unroll
-    for (int i = 0; i < NI; ++i) {
-        const long off = (long) min(KPI * (4 * i + wave) + ks, n_kv - 1) * Hkv * DH + (long) hk * DH + 8 * kd;
-        if constexpr (COH) kreg[i] = coh_ld16u(rk, (uint32_t) (off * 2));
-        else kreg[i] = *(const PM_G u32x4 *) (kc + off);
-    }
-#pragma unroll
-    for (int i = 0; i < NV; ++i) {
-        const long off = (long) (hk * DH + DH / 4 * wave + DPI * i + ve) * n_ctx + (8 * c < n_kv ? 8 * c : 0);
-        if constexpr (COH) vreg[i] = coh_ld16u(rv, (uint32_t) (off * 2));
-        else vreg[i] = *(const PM_G u32x4 *) (vc + off);
-    }
-    float m_add[KPL];
 #pragma unroll
     for (int k = 0; k < KPL; ++k) {
-        const int key = lane + 64 * k;
-        m_add[k] = (mask && key < n_kv) ? (mask_f16 ? h2f(((const PM_G uint16_t *) mask)[key]) : ((const PM_G float *) mask)[key]) : 0.0f;
-    }
-    // scores: lane kd of a key's lanes keeps the one of instruction kd
-    float keep = 0.0f;
+        const long koff = (long) (lane + 64 * k) * Hkv * DH + (long) hk * DH + DPW * wave;
 #pragma unroll
-    for (int i = 0; i < NI; ++i) {
+        for (int j = 0; j < NK; ++j) kreg[k][j] = coh_ld16u(rk, (uint32_t) ((koff + 8 * j) * 2));
+    }
+    const int e = lane % DPW, kp = lane / DPW;
+    const long vrow = (long) (hk * DH + DPW * wave + e) * n_ctx + KPP * kp;
+#pragma unroll
+    for (int j = 0; j < NV; ++j) vreg[j] = coh_ld16u(rv, (uint32_t) ((vrow + 8 * j) * 2));
+    float * qw = qstrip + wave * DPW;
+    if (lane < DPW) qw[lane] = coh_ld4(rq, (uint32_t) ((DPW * wave + lane) * 4));
+    __builtin_amdgcn_s_waitcnt(0xc07f);
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int k = 0; k < KPL; ++k) {
         float acc = 0.0f;
 #pragma unroll
-        for (int t = 0; t < 4; ++t) {
-            const uint32_t w = kreg[i][t];
-            acc = fmaf(h2f((uint16_t) (w & 0xFFFF)), q[t >> 1][2 * (t & 1)], acc);
-            acc = fmaf(h2f((uint16_t) (w >> 16)), q[t >> 1][2 * (t & 1) + 1], acc);
-        }
-        acc += dpp_f<0xB1>(acc); acc += dpp_f<0x4E>(acc); acc += dpp_f<0x141>(acc);
-        if constexpr (LPK >= 16) acc += dpp_f<0x140>(acc);
-        if constexpr (LPK >= 32) acc += __builtin_bit_cast(float, other_row(__builtin_bit_cast(uint32_t, acc)));
-        keep = kd == i ? acc : keep;
+        for (int j = 0; j < NK; ++j)
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+                acc = fmaf(h2f((uint16_t) (kreg[k][j][t] & 0xFFFF)), qw[8 * j + 2 * t], acc);
+                acc = fmaf(h2f((uint16_t) (kreg[k][j][t] >> 16)), qw[8 * j + 2 * t + 1], acc);
+            }
+        part[wave * NKEY + lane + 64 * k] = acc;
     }
-    if (kd < NI) part[KPI * (4 * kd + wave) + ks] = keep;
     bar();
     float s_[KPL], mx = -INFINITY;
 #pragma unroll
     for (int k = 0; k < KPL; ++k) {
         const int key = lane + 64 * k;
-        s_[k] = key < n_kv ? part[key] * scale + m_add[k] : -INFINITY;
+        s_[k] = key < n_kv ? ((part[key] + part[NKEY + key]) + (part[2 * NKEY + key] + part[3 * NKEY + key])) * scale : -INFINITY;
         mx = fmaxf(mx, s_[k]);
     }
-    mx = all_max(mx);
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) mx = fmaxf(mx, __shfl_xor(mx, off));
     float ex[KPL];
     double tot = 0.0;
 #pragma unroll
     for (int k = 0; k < KPL; ++k) { ex[k] = lane + 64 * k < n_kv ? expf(s_[k] - mx) : 0.0f; tot += (double) ex[k]; }
-    const float inv = (float) (1.0 / all_sum(tot));
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) tot += __shfl_xor(tot, off);
+    const float inv = (float) (1.0 / tot);
 #pragma unroll
     for (int k = 0; k < KPL; ++k) pw[wave * NKEY + lane + 64 * k] = h2f(f2h(ex[k] * inv));        // p rounded to F16 (src1 of the V^T.p product)
     __builtin_amdgcn_wave_barrier();                       // (a wave's LDS accesses execute in order: its own copy needs no workgroup barrier)
-    const f32x4 p0 = *(const f32x4 *) (pw + wave * NKEY + 8 * c), p1 = *(const f32x4 *) (pw + wave * NKEY + 8 * c + 4);
-    keep = 0.0f;
+    float o = 0.0f;
 #pragma unroll
-    for (int i = 0; i < NV; ++i) {
-        float o = 0.0f;
+    for (int j = 0; j < NV; ++j)
 #pragma unroll
         for (int t = 0; t < 4; ++t) {
-            const uint32_t w = vreg[i][t];
-            const f32x4 & p = t < 2 ? p0 : p1;
-            o = fmaf(h2f((uint16_t) (w & 0xFFFF)), p[2 * (t & 1)], o);
-            o = fmaf(h2f((uint16_t) (w >> 16)), p[2 * (t & 1) + 1], o);
+            o = fmaf(h2f((uint16_t) (vreg[j][t] & 0xFFFF)), pw[wave * NKEY + KPP * kp + 8 * j + 2 * t], o);
+            o = fmaf(h2f((uint16_t) (vreg[j][t] >> 16)), pw[wave * NKEY + KPP * kp + 8 * j + 2 * t + 1], o);
         }
-        o += dpp_f<0xB1>(o); o += dpp_f<0x4E>(o); o += dpp_f<0x141>(o);
-        if constexpr (LV >= 16) o += dpp_f<0x140>(o);
-        keep = lane % LR == i ? o : keep;
-    }
-    if constexpr (LV == 32) keep += __builtin_bit_cast(float, other_row(__builtin_bit_cast(uint32_t, keep)));
-    if (lane % LR < NV && (LV < 32 || !(lane & 16))) st_act<COH>(out_head + DH / 4 * wave + DPI * (lane % LR) + ve, keep);
+#pragma unroll
+    for (int off = DPW; off < 64; off <<= 1) o += __shfl_xor(o, off);
+    if (lane < DPW) st_act<true>(out_head + DPW * wave + lane, o);
 }
 
 struct AttnTailP {
@@ -122,7 +102,7 @@ struct AttnTailP {
 static inline __host__ __device__ size_t attn_tail_lds(int dh, int max_keys) { return (size_t) (2048 + 8 + 8) * 4 + (size_t) (dh + 256 + ((max_keys + 15) & ~7)) * 4; }
 
 // head h by FOUR waves (threads 0 .. 255 of the caller's workgroup); bar() = a barrier of exactly those four waves that also orders their LDS traffic.
-// attn_cached.hip's short form (up to 256 cells, one barrier) and the cached form of attn_rope_body beyond.
+// attn_cached.hip's short path (<= 64 cells, one barrier) and the cached form of attn_rope_body beyond.
 template <int DH, class Bar>
 __device__ __forceinline__ void attn_tail_head(const AttnTailP & a, int h, char * smem, Bar && bar) {
     // (the thread id goes through an opaque asm: everything derived from it - dozens of LDS / cache offsets - is then recomputed here instead of being
@@ -142,13 +122,63 @@ __device__ __forceinline__ void attn_tail_head(const AttnTailP & a, int h, char 
     float * redf = pw + 1024;                              // [8]
     double * redd = (double *) (redf + 8);                 // [4]
     float * body = (float *) (redd + 4);                   // general path: qs[DH] | part[256] | sc[max_keys]
-    // ---- up to 256 cells (the same function attn_cached.hip calls: same bits)
-    const float * qh = a.q + (long) h * DH;
-    float * oh = a.out + (long) h * DH;
-    if (n_kv <= 64) { attn_whole_lines<DH, 1, true>(qh, a.kc + soff, a.vc + soff, oh, hk, Hkv, n_ctx, n_kv, scale, nullptr, 0, part, pw, lane, wave, bar); return; }
+    if (n_kv <= 64 && n_ctx >= 64) {
+        constexpr int DPW = DH / 4, NK = DPW / 8, KP = 64 / DPW, KPP = 64 / KP, NV = KPP / 8;
+        const int key = lane < n_ctx ? lane : 0;
+        u32x4 kreg[NK], vreg[NV];
+#pragma unroll
+        for (int j = 0; j < NK; ++j) kreg[j] = coh_ld16u(rk, (uint32_t) (((long) key * Hkv * DH + (long) hk * DH + DPW * wave + 8 * j) * 2));
+        const int e = lane % DPW, kp = lane / DPW;
+        const long vrow = (long) (hk * DH + DPW * wave + e) * n_ctx + (KPP * kp + KPP <= n_ctx ? KPP * kp : 0);
+#pragma unroll
+        for (int j = 0; j < NV; ++j) vreg[j] = coh_ld16u(rv, (uint32_t) ((vrow + 8 * j) * 2));
+        // this wave's q slice -> its own LDS strip, read back as broadcasts (a scalar load could hit a stale scalar-cache line: the rows were written by
+        // other CUs in this launch; DPW values in registers next to the K / V pieces spill)
+        float * qw = body + wave * DPW;
+        if (lane < DPW) qw[lane] = coh_ld4(rq, (uint32_t) (((long) h * DH + DPW * wave + lane) * 4));
+        __builtin_amdgcn_s_waitcnt(0xc07f);
+        __builtin_amdgcn_wave_barrier();
+        float acc = 0.0f;
+#pragma unroll
+        for (int j = 0; j < NK; ++j)
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+                acc = fmaf(h2f((uint16_t) (kreg[j][t] & 0xFFFF)), qw[8 * j + 2 * t], acc);
+                acc = fmaf(h2f((uint16_t) (kreg[j][t] >> 16)), qw[8 * j + 2 * t + 1], acc);
+            }
+        part[wave * 64 + lane] = acc;
+        bar();
+        const bool valid = lane < n_kv;
+        const float s_ = valid ? ((part[lane] + part[64 + lane]) + (part[128 + lane] + part[192 + lane])) * scale : -INFINITY;
+        float mx = s_;
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) mx = fmaxf(mx, __shfl_xor(mx, off));
+        const float ex = valid ? expf(s_ - mx) : 0.0f;
+        double tot = (double) ex;
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) tot += __shfl_xor(tot, off);
+        const float inv = (float) (1.0 / tot);
+        pw[wave * 64 + lane] = h2f(f2h(ex * inv));         // p rounded to F16 (src1 of the V^T.p product)
+        __builtin_amdgcn_wave_barrier();
+        float o = 0.0f;
+        const bool chunk_ok = KPP * kp + KPP <= n_ctx;
+#pragma unroll
+        for (int j = 0; j < NV; ++j)
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+                o = fmaf(h2f((uint16_t) (vreg[j][t] & 0xFFFF)), pw[wave * 64 + KPP * kp + 8 * j + 2 * t], o);
+                o = fmaf(h2f((uint16_t) (vreg[j][t] >> 16)), pw[wave * 64 + KPP * kp + 8 * j + 2 * t + 1], o);
+            }
+        if (!chunk_ok) o = 0.0f;
+#pragma unroll
+        for (int off = DPW; off < 64; off <<= 1) o += __shfl_xor(o, off);
+        if (lane < DPW) st_act<true>(a.out + (long) h * DH + DPW * wave + lane, o);
+        return;
+    }
+    // ---- up to 256 cells: keys in the lanes, two / four per lane (the same function attn_cached.hip calls: same bits)
     if constexpr (DH <= 128) {
-        if (n_kv <= 128) { attn_whole_lines<DH, 2, true>(qh, a.kc + soff, a.vc + soff, oh, hk, Hkv, n_ctx, n_kv, scale, nullptr, 0, part, pw, lane, wave, bar); return; }
-        if (n_kv <= 256) { attn_whole_lines<DH, 4, true>(qh, a.kc + soff, a.vc + soff, oh, hk, Hkv, n_ctx, n_kv, scale, nullptr, 0, part, pw, lane, wave, bar); return; }
+        if (n_kv <= 128 && n_ctx >= 128) { attn_keys_in_lanes<DH, 2>(a.q + (long) h * DH, a.kc + soff, a.vc + soff, a.out + (long) h * DH, hk, Hkv, n_ctx, n_kv, scale, part, pw, body, lane, wave, bar); return; }
+        if (n_kv <= 256 && n_ctx >= 256) { attn_keys_in_lanes<DH, 4>(a.q + (long) h * DH, a.kc + soff, a.vc + soff, a.out + (long) h * DH, hk, Hkv, n_ctx, n_kv, scale, part, pw, body, lane, wave, bar); return; }
     }
     // ---- general cached body (attn_rope_body<DH, COH, 0, true>): thread per key, three 4-wave reductions
     constexpr int PARTS = 256 / DH, KQ = DH / 8;

@@ -106,7 +106,7 @@ __device__ __forceinline__ float wave_sum(float v) {
     return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), 63));
 }
 
-// ---- reductions whose result every lane of a wave gets, without LDS: 16-lane rows by DPP, then the rows by lane swaps
+// ---- reductions whose result every lane of a wave gets, without LDS: 16-lane rows by DPP, rows and halves by lane swaps
 __device__ __forceinline__ uint32_t other_row(uint32_t v) { const u32x2 r = __builtin_bit_cast(u32x2, __builtin_amdgcn_permlane16_swap(v, v, false, false)); const uint32_t x = r[0], y = r[1]; return (threadIdx.x & 16) ? x : y; }
 __device__ __forceinline__ uint32_t other_half(uint32_t v) { const u32x2 r = __builtin_bit_cast(u32x2, __builtin_amdgcn_permlane32_swap(v, v, false, false)); const uint32_t x = r[0], y = r[1]; return (threadIdx.x & 32) ? x : y; }
 __device__ __forceinline__ float all_max(float v) {
@@ -122,13 +122,14 @@ template <class F> __device__ __forceinline__ double f64_moved(double v, F && f)
     const uint32_t lo = f((uint32_t) u), hi = f((uint32_t) (u >> 32));
     return __builtin_bit_cast(double, ((uint64_t) hi << 32) | lo);
 }
+// (halves, rows, then 8, 4, 2, 1 lanes apart: the order of a __shfl_xor loop from 32 down, bit for bit. A rotation by 8, then 4 lanes finds the partner: sums repeat every 16, then every 8 lanes)
 __device__ __forceinline__ double all_sum(double v) {
-    v += f64_moved(v, [](uint32_t x) __attribute__((always_inline)) { return (uint32_t) dpp_i<0xB1>((int) x); });
-    v += f64_moved(v, [](uint32_t x) __attribute__((always_inline)) { return (uint32_t) dpp_i<0x4E>((int) x); });
-    v += f64_moved(v, [](uint32_t x) __attribute__((always_inline)) { return (uint32_t) dpp_i<0x141>((int) x); });
-    v += f64_moved(v, [](uint32_t x) __attribute__((always_inline)) { return (uint32_t) dpp_i<0x140>((int) x); });
+    v += f64_moved(v, [](uint32_t x) __attribute__((always_inline)) { return other_half(x); });
     v += f64_moved(v, [](uint32_t x) __attribute__((always_inline)) { return other_row(x); });
-    return v + f64_moved(v, [](uint32_t x) __attribute__((always_inline)) { return other_half(x); });
+    v += f64_moved(v, [](uint32_t x) __attribute__((always_inline)) { return (uint32_t) dpp_i<0x128>((int) x); });
+    v += f64_moved(v, [](uint32_t x) __attribute__((always_inline)) { return (uint32_t) dpp_i<0x124>((int) x); });
+    v += f64_moved(v, [](uint32_t x) __attribute__((always_inline)) { return (uint32_t) dpp_i<0x4E>((int) x); });
+    return v + f64_moved(v, [](uint32_t x) __attribute__((always_inline)) { return (uint32_t) dpp_i<0xB1>((int) x); });
 }
 
 // max over aligned groups of 8 lanes, result in all 8 lanes

@@ -1,6 +1,8 @@
 """GPU parity tests (run with -m gpu on an MI355X): every op goes through the C ABI of
 libprima_mi355.so and is compared with the CPU oracle on the same seeded inputs.
 Integer / byte results: bit-exact. Float results: tolerance stated per test."""
+import os
+
 import numpy as np
 import pytest
 
@@ -1523,3 +1525,41 @@ def test_rms_norm_of_many_rows(P, oracle, rows, K):
     want = oracle.rms_norm(x[at], w, 1e-5)
     assert np.abs(got[at].view(np.int32).astype(np.int64) - want.view(np.int32).astype(np.int64)).max() <= 1
     assert np.array_equal(P.act_to_ggml_blocks(yq, Q8_K, K, rows), P.act_to_ggml_blocks(P.quantize_act(y, Q8_K), Q8_K, K, rows))
+
+
+SHORT_ATTENTION = [(dh, n_ctx, n_kv, mask) for dh, n_ctx, n_kvs in ((64, 256, (1, 36, 64, 65, 100, 128, 129, 204, 256)), (128, 320, (1, 36, 64, 65, 100, 128, 129, 204, 256)), (256, 64, (7, 64)),
+                                                                     (128, 32, (9, 32)), (64, 96, (64, 80)), (128, 200, (128, 199)), (256, 256, (65, 200)))
+                   for n_kv in n_kvs for mask in ([None] if n_kv not in (36, 204) else [None, "f32", "f16"])]
+
+
+def short_attention_inputs(dh, n_ctx, n_kv, mask):
+    """q (as the wq launch leaves it: F16 values), caches of two KV heads, three query heads each, random behind the attended cells too, a mask that hides every fifth cell"""
+    rng = np.random.default_rng(dh * 1000003 + n_ctx * 1009 + n_kv)
+    H, Hkv = 6, 2
+    q = rng.normal(0, 1, (H, dh)).astype(np.float16).astype(np.float32)
+    kc, vc = rng.normal(0, 1, (n_ctx, Hkv, dh)).astype(np.float16), rng.normal(0, 1, (Hkv, dh, n_ctx)).astype(np.float16)
+    m = None if mask is None else np.where(np.arange(n_ctx) % 5 == 3, -np.inf, rng.normal(0, 1, n_ctx).astype(np.float16)).astype(np.float32 if mask == "f32" else np.float16)
+    return q, kc, vc, m
+
+
+@pytest.mark.parametrize("dh,n_ctx,n_kv,mask", SHORT_ATTENTION)
+def test_single_token_attention_over_few_cells_keeps_its_sums(P, dh, n_ctx, n_kv, mask):
+    """Up to 256 cells: every rounding of a decoded token is what it is with a lane per key and a lane per dimension, whatever the loads look like - the 8-bit roundings behind it carry one other
+    bit to 3 % of an eight-layer model's logits. Bit for bit against outputs recorded with that form (golden/attn_short.npz: edges of the 64 / 128 / 256-cell forms, caches too small for a form,
+    masks), and against float64: probabilities rounded to F16 (2^-11 of each) and f32 sums of at most 256 terms."""
+    torch = P.torch
+    q, kc, vc, m = short_attention_inputs(dh, n_ctx, n_kv, mask)
+    H, Hkv = q.shape[0], kc.shape[1]
+    scale = dh ** -0.5
+    dyn = torch.tensor([n_kv - 1, n_kv], dtype=torch.int32, device="cuda")
+    run = lambda: P.attn_cached(_dev(P, q.reshape(1, -1)), _dev(P, kc.view(np.int16)), _dev(P, vc.view(np.int16)), None, H, Hkv, dh, n_ctx, scale, cell_nkv=dyn,  # noqa: E731
+                                mask=None if m is None else _dev(P, m.view(np.int16) if mask == "f16" else m), max_keys=n_ctx, flags=P.ATTN_MASK_F16 if mask == "f16" else 0).cpu().numpy().reshape(H, dh)
+    out = run()
+    k, v = kc[:n_kv].astype(np.float64), vc[:, :, :n_kv].astype(np.float64)
+    for h in range(H):
+        s = k[:, h // 3] @ q[h].astype(np.float64) * np.float32(scale) + (0 if m is None else m[:n_kv].astype(np.float64))
+        p = np.exp(s - s.max())
+        p /= p.sum()
+        assert np.abs(out[h] - v[h // 3] @ p).max() <= (2.0 ** -11 + 1e-5) * (np.abs(v[h // 3]) @ p).max() + 2.0 ** -25 * n_kv * np.abs(v).max()
+    want = np.load(os.path.join(os.path.dirname(os.path.abspath(__file__)), "golden", "attn_short.npz"))[f"{dh}_{n_ctx}_{n_kv}_{mask}"]
+    assert np.array_equal(out.view(np.uint32), want.view(np.uint32)), np.abs(out - want).max()
