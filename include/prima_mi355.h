@@ -17,6 +17,11 @@
  * (pass NULL for the default stream). Every call is asynchronous with respect to the host unless
  * stated otherwise. Return value: 0 on success, negative pm355 error code otherwise (no exceptions
  * cross this boundary; unsupported shapes return PM355_E_UNSUPPORTED and do nothing).
+ *
+ * Threads: an object (window, uploader, ring, ..) belongs to one host thread at a time. Several threads may each drive objects of their own on streams of their own. Work that meets on ONE stream
+ * is issued by one thread at a time, a whole call after the other: products of up to 64 rows of activations keep their tables, and (B)'s prompts their partial tiles, in scratch memory of the
+ * (device, stream). (A prompt's launches are issued together whoever else issues on the stream; the tables of small products are not guarded.) pm355_mul_mat_q_mfma* keep an F16 copy of their
+ * activations per DEVICE: one thread per device.
  */
 #ifndef PRIMA_MI355_H
 #define PRIMA_MI355_H

@@ -979,13 +979,13 @@ void pf_allow_lds(const void * kern, size_t lds) {
     if (n_done < 64) { done[n_done].k = kern; done[n_done].dev = dev; ++n_done; }
 }
 
-// split-K workspace of a (device, stream): the partial-tile slabs
+// split-K workspace of a (device, stream): the partial-tile slabs. A product leaves them for the launch behind it, so g_pf_mu is held from here until that one is issued: another host thread's
+// product on this stream, or its larger request, comes in front of both launches or behind both
 struct PfWs { hipStream_t st; int dev; uint8_t * p; size_t bytes; uint64_t use; };
 PfWs g_pf_ws[16] = {};
 uint64_t g_pf_tick = 0;
 std::mutex g_pf_mu;
 uint8_t * pf_workspace(hipStream_t st, size_t need) {
-    std::lock_guard<std::mutex> lk(g_pf_mu);
     const int dev = pm_cur_dev();
     PfWs * e = nullptr, * lru = &g_pf_ws[0];
     for (PfWs & c : g_pf_ws) {
@@ -1104,7 +1104,9 @@ static int launch_pf(const pm_gemm_pf_job * jobs, int njobs, const void * xh, co
     p.nt_t = pl.nt_t;
     p.splitk = S; p.full = full;
     const int split_slots = maxL - full;                       // per XCD
+    std::unique_lock<std::mutex> slabs(g_pf_mu, std::defer_lock);
     if (S > 1) {
+        slabs.lock();
         const size_t slab = (size_t) (mid ? 4 : 8) * nt * 4 * 64 * 16, need = (size_t) 8 * split_slots * S * slab;
         p.ws = (float *) pf_workspace(st, need);
         if (!p.ws) return -3;
