@@ -217,7 +217,8 @@ PM355_API int pm355_mul_mat_q_small_multi(int type, int njobs, const void * cons
  * (llama_tensor_get_type, src/llama.cpp:19447) - as ONE grid whose workgroups are divided by weight bytes. PM355_E_UNSUPPORTED: launch the jobs separately. */
 PM355_API int pm355_mul_mat_q_small_mixed(const int * types, int njobs, const void * const * W, const int64_t * N, float * const * y,
                                           const float * const * bias, const void * xq, int64_t K, int64_t n_tokens, pm355_stream_t stream);
-/* The same arithmetic for up to 512 tokens on the prompt GEMM's tiles (prima_cpp_amd/csrc/mmq_pf.hip), what batches of several sequences' short portions take: 1..3 Q4_K / Q5_K / Q6_K matrices
+/* Up to 512 tokens on the prompt GEMM's tiles (prima_cpp_amd/csrc/mmq_pf.hip), what batches of several sequences' short portions take: the same 8-bit activations and whole-number sums, exact,
+ * per half of a super-block (above: per super-block), added up in f32 in another order; no farther from 64 bits. 1..3 Q4_K / Q5_K / Q6_K matrices
  * of at most two types over f32 activations x [n_tokens][K], K % 256 == 0, N % 4 == 0. pair != 0: two matrices of one type and shape, y[1] = silu(W[0] x) * (W[1] x). scratch: device memory of
  * pm355_mul_mat_q_wide_scratch(K) bytes, 16-byte aligned. */
 PM355_API int pm355_mul_mat_q_wide(const int * types, int njobs, const void * const * W, const int64_t * N, float * const * y, const float * const * bias, const float * const * resid,

@@ -1390,7 +1390,8 @@ int pm_window::pool_info(pm355_pool_info * o) {
 // All entries as rows of common passes: the weights are read once per pass instead of once per sequence (eight sequences of the 8B shape, eight layers and
 // head: prompts of 12..24 tokens and twelve steps 47.0 ms one sequence after another, 9.8 ms as common passes). A portion keeps the arithmetic that it has alone - up to 32 tokens 8-bit
 // activations, beyond 16-bit ones; up to 15 where a layer has no 8-bit path, and between the two either, layer by layer - whatever shares the step with it: portions meet in passes of
-// their own tier, the longer ones (a sequence's first) first, and the attention of a portion is chosen by the cells that it attends itself. served = false and nothing done where a pass does
+// their own tier (how many rows share one decides which kernel forms the 8-bit products: exact whole-number sums in all of them, added up in f32 in another order), the longer ones (a sequence's
+// first) first, and the attention of a portion is chosen by the cells that it attends itself. served = false and nothing done where a pass does
 // not take rows of several sequences.
 int pm_window::batch_rows(const pm355_batch_entry * e, int n, float * d_logits, int32_t * d_argmax, hipStream_t st, bool * served) {
     pm_window * m = this;
@@ -1416,8 +1417,8 @@ int pm_window::batch_rows(const pm355_batch_entry * e, int n, float * d_logits, 
         int64_t total = 0;
         for (int i = 0; i < n; ++i)
             for (int off = 0; off < e[i].n_tokens; off += max_tokens) { const int T = std::min(max_tokens, e[i].n_tokens - off); if (mine(T)) total += T; }
-        // rows of short portions that need more than one small pass go out as wide ones. Prompts of two layers, us, small passes / wide: 8B shape, 40 rows in all 530 / 416, 80 904 / 553, 192 1808 / 795,
-        // Q6_K 679 / 451, 1120 / 590, 2211 / 878; 70B shape 1087 / 917, 1818 / 1247, 3578 / 1976, Q6_K 1394 / 1018, 2252 / 1380, 4407 / 2225 (192 rows as two passes of 96: 1069 on the 8B shape)
+        // rows of short portions that need more than one small pass go out as wide ones. Prompts of 8 tokens through two layers and the head, us, small passes / wide, 40, 80 and 192 rows in all: 8B shape
+        // Q4_K_M 531 / 413, 752 / 516, 1421 / 772, Q6_K 658 / 462, 957 / 628, 1859 / 936; 70B shape 1031 / 895, 1499 / 1195, 2897 / 1901, Q6_K 1325 / 1075, 1913 / 1650, 3735 / 2416
         const int cap_w = std::min(max_tokens, PM_WIDE_MAX_TOKENS);
         const bool wd = wide && every && most == MMQ_MAX_TOKENS && total > most && total / ((total + cap_w - 1) / cap_w) > most;
         const int cap = wd ? cap_w : most;

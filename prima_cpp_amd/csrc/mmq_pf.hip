@@ -127,14 +127,19 @@ template <int TYPE> __device__ __forceinline__ half8 pf_dequant(const u32x2 ql, 
         for (int c = 0; c < 2; ++c) { t[2 * c] = h2(__builtin_amdgcn_perm(0x64646464u, v[c], 0x05010400u)); t[2 * c + 1] = h2(__builtin_amdgcn_perm(0x64646464u, v[c], 0x07030602u)); }
 #pragma unroll
         for (int c = 0; c < 4; ++c) t[c] = t[c] + bias;
-        half2v q[4];
+        if (low) {                                             // products (whole numbers up to 4096) as 64 x (-64 .. 64) + (-32 .. 32): 1536 + x rounds x to a whole number
+            const half2v m64 = mul * half2v{(_Float16) 0.015625f, (_Float16) 0.015625f}, up = {(_Float16) 1536.0f, (_Float16) 1536.0f}, by = {(_Float16) -64.0f, (_Float16) -64.0f};
+            half2v q[4];
 #pragma unroll
-        for (int c = 0; c < 4; ++c) { q[c] = t[c]; t[c] = t[c] * mul; }
-        if (low) {                                             // what the rounded products are off by
+            for (int c = 0; c < 4; ++c) { q[c] = t[c]; t[c] = pk_fma(t[c], m64, up); }
 #pragma unroll
-            for (int c = 0; c < 4; ++c) q[c] = pk_fma(q[c], mul, -t[c]);
+            for (int c = 0; c < 4; ++c) t[c] = t[c] - up;
+#pragma unroll
+            for (int c = 0; c < 4; ++c) q[c] = pk_fma(q[c], mul, t[c] * by);
             *low = __builtin_bit_cast(half8, u32x4{u2(q[0]), u2(q[1]), u2(q[2]), u2(q[3])});
-        }
+        } else
+#pragma unroll
+            for (int c = 0; c < 4; ++c) t[c] = t[c] * mul;
     }
     return __builtin_bit_cast(half8, u32x4{u2(t[0]), u2(t[1]), u2(t[2]), u2(t[3])});
 }
@@ -474,13 +479,17 @@ template <int TYPE, int NT> constexpr int mid_sum_bytes() { return TYPE == PM_Q6
 template <int TYPE, int NT, bool EX> constexpr size_t mid_lds_bytes() { return (size_t) 6 * NT * 32 * 128 + (size_t) 4 * mid_group_bytes<TYPE, EX>() + (EX ? 2 * (mid_sum_bytes<TYPE, NT>() + NT * 32 * 4) : 0); }
 template <int N> __device__ __forceinline__ void mid_wait() { asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" : : "n"(N) : "memory"); }
 
-// EX - 8-bit activations (Q8_K blocks), the sums of mmq_i8.hip: what the matrix cores add up over a super-block are whole numbers. B = the 8-bit values as F16, A = quant x 6-bit sub-block scale
-// as F16 (Q4_K at most 945, Q5_K 1953: exact; Q6_K up to 4096: the rounded product and what it is off by, two products), and an f32 accumulator holds whole numbers up to 2^24 exactly - where
-// int32 sums are rounded too when they become f32. A super-block's sum is then multiplied by d of the row and d of the token and added in f32, the minima (one product: 16 group sums x
-// minima) by dmin. Against an integer GEMM: scales per 32 k applied to int32 results cost as much vector work as the products take, and scales inside 8-bit operands two products per
-// sub-block (mmq_big.hip); here scale and quant share the multiply that the F16 form needs anyway.
-// Bound by the LDS-DMA like the F16 form, by the vector work at a super-block's end (3 x 16 instructions per 32 tokens, registers 126 -> 240) and, Q6_K, by twice the products. 8B shape, 169 tokens,
-// us: ffn_gate | ffn_up 121 (six passes of 28 on mmq_i8.hip 26.6 each), wo and ffn_down Q4_K 41 on average (14.5 each), ffn_down Q6_K 72 (35 each), wq | wk | wv 37.
+// EX - 8-bit activations (Q8_K blocks): what the matrix cores add up over a wave's 128 k of a super-block are whole numbers, and exact. B = the 8-bit values as F16, A = quant x 6-bit sub-block
+// scale as F16; an f32 accumulator holds whole numbers up to 2^24. Q4_K: at most 945 x 127 x 128, one accumulator. Q5_K: 1953 x 127 x 64 fits, so one accumulator per 64 k, added at the end;
+// Q6_K: products of up to 4096 as 64 x hi + lo, two products with an accumulator each (64 x 127 x 128 at most). Their sum is rounded once on its way to f32, as an int32 sum is when it becomes
+// one. It is then multiplied by d of the row and d of the token and added in f32, the minima (one product: 16 group sums x minima, exact) by dmin. mmq_i8.hip and mmq_rows.hip do this for all
+// 256 k of a super-block at once: here the halves of a super-block meet as f32. Against an integer GEMM: scales per 32 k applied to int32 results cost as much vector work as the products
+// take, and scales inside 8-bit operands two products per sub-block (mmq_big.hip); here scale and quant share the multiply that the F16 form needs anyway.
+// Bound by the LDS-DMA like the F16 form, by the vector work at a super-block's end (3 x 16 instructions per 32 tokens) and, Q6_K, by twice the products; two sets of accumulators beside the
+// running sums leave room for 64 tokens per workgroup. 8B shape, 169 tokens, us with the quantizer's launch: ffn_gate | ffn_up 115 (Q6_K 162; six passes of 28 on mmq_i8.hip 26.6 each), wo 32,
+// ffn_down Q4_K 66, Q6_K 101 (35 each), wq | wk | wv with a Q6_K wv 58. (Q6_K's product and its remainder in ONE accumulator, 128 tokens: 148 and 84, and sums beyond 2^24 rounded 16 times.)
+// Distance from 64 bits (2-norm, normal weights) of mmq_i8.hip / this form: Q4_K 4096 x 4096 1.20e-7 / 0.89e-7, x 14336 1.33e-7 / 1.06e-7, Q5_K 1.20e-7 / 0.88e-7, Q6_K 4096 x 14336 0.81e-7 / 0.79e-7,
+// 8192 x 28672 0.92e-7 / 0.86e-7 (running sums over all of a slice's super-blocks: 1.43e-7; minima of a whole super-block by either half in turn: Q4_K x 14336 1.84e-7).
 template <int TYPE, int NT, bool EX>
 __device__ __forceinline__ void mid_body(const PfP & p, const PfJob & jb, const int n0, const int t0, uint8_t * smem, const int role, const int ks, const int S, const int tile_id) {
     constexpr int HB = NT * 32 * 128, BBUF = 2 * HB;           // activations: 32 NT tokens x 64 halfs, two of them per step
@@ -555,12 +564,16 @@ __device__ __forceinline__ void mid_body(const PfP & p, const PfJob & jb, const 
     for (int jt = 0; jt < NT; ++jt)
 #pragma unroll
         for (int e = 0; e < 16; ++e) acc[jt][e] = 0.0f;
-    float16v run[EX ? NT : 1];
+    constexpr bool TWO = EX && (TYPE == PM_Q5_K || TYPE == PM_Q6_K);
+    static_assert(!TWO || NT == 2, "three sets of accumulators: 64 tokens, or registers spill");
+    constexpr bool SUMS = EX && NT == 2;                         // (registers left: running sums of four super-blocks, and those of them)
+    float16v run[EX ? NT : 1], ac2[TWO ? NT : 1], tot[SUMS ? NT : 1];
+    const float16v zero = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
     if (EX)
 #pragma unroll
         for (int jt = 0; jt < NT; ++jt)
 #pragma unroll
-            for (int e = 0; e < 16; ++e) run[jt][e] = 0.0f;
+            for (int e = 0; e < 16; ++e) { run[jt][e] = 0.0f; if (SUMS) tot[jt][e] = 0.0f; }
     // the 4 slices of this wave's half of the step in buffer bb / slot sl: 128-k half mm of super-block b
     // a quarter of the step's requests behind each slice's MFMAs (an issue blocks the wave for 60-180 cycles: in front of the step they were 0.4 of its 1.25 us)
     auto multiply = [&](int b, int mm, uint32_t bb, uint32_t sl, auto && request) __attribute__((always_inline)) {
@@ -617,47 +630,55 @@ __device__ __forceinline__ void mid_body(const PfP & p, const PfJob & jb, const 
         for (int j = 0; j < 4; ++j) {
             if (j < 3) { read_B(j + 1); operand(j + 1); }
 #pragma unroll
-            for (int jt = 0; jt < NT; ++jt) acc[jt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[j & 1], bf[j & 1][jt], acc[jt], 0, 0, 0);
-            if (EX && TYPE == PM_Q6_K)
+            for (int jt = 0; jt < NT; ++jt) {
+                if constexpr (TWO && TYPE == PM_Q5_K) {
+                    if (mm) ac2[jt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[j & 1], bf[j & 1][jt], j ? ac2[jt] : zero, 0, 0, 0);
+                    else    acc[jt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[j & 1], bf[j & 1][jt], j ? acc[jt] : zero, 0, 0, 0);
+                } else acc[jt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[j & 1], bf[j & 1][jt], EX && mm + j == 0 ? zero : acc[jt], 0, 0, 0);
+            }
+            if constexpr (TWO && TYPE == PM_Q6_K)
 #pragma unroll
-                for (int jt = 0; jt < NT; ++jt) acc[jt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(al[j & 1], bf[j & 1][jt], acc[jt], 0, 0, 0);
+                for (int jt = 0; jt < NT; ++jt) ac2[jt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(al[j & 1], bf[j & 1][jt], mm + j == 0 ? zero : ac2[jt], 0, 0, 0);
             request(j);
         }
     };
-    // EX: the whole numbers of super-block b (this wave's half of its k) onto the running sums; the minima by either half in turn
+    // EX: the whole numbers of super-block b (this wave's half of its k, and the minima of that half: without them the halves' sums are twice as large, and their roundings) onto the running sums
     auto fold = [&](int b) __attribute__((always_inline)) {
         const uint8_t * const xb = smem + XS + (b & 1) * XB;
-        float d[16], dm[16];
+        uint32_t dd[16];                                        // d, dmin of the rows (F16)
 #pragma unroll
         for (int e = 0; e < 16; ++e) {
             const int row = (e & 3) + 8 * (e >> 2) + 4 * h;
-            if (K45) {
-                const uint32_t v = *(const uint32_t *) (ag + HDR + (b & 3) * 512 + row * 16);
-                d[e] = h2f((uint16_t) v); dm[e] = h2f((uint16_t) (v >> 16));
-            } else d[e] = h2f(*(const uint16_t *) (ag + XTRA + ((b >> 3) & 1) * 512 + row * 16 + (b & 7) * 2));
+            if (K45) dd[e] = *(const uint32_t *) (ag + HDR + (b & 3) * 512 + row * 16);
+            else dd[e] = *(const uint16_t *) (ag + XTRA + ((b >> 3) & 1) * 512 + row * 16 + (b & 7) * 2);
         }
-        const bool mins = K45 && kk == (b & 1);
+        auto d = [&](int e) __attribute__((always_inline)) { return h2f((uint16_t) dd[e]); };
+        auto dm = [&](int e) __attribute__((always_inline)) { return h2f((uint16_t) (dd[e] >> 16)); };
         half8 mo = {0, 0, 0, 0, 0, 0, 0, 0};
-        if (mins) {                                             // minima of the row's sub-blocks 4 h .. 4 h + 3, each for two groups of 16
+        if (K45) {                                              // minima of the row's sub-blocks 4 h .. 4 h + 3, each for two groups of 16: 4 h + 2 kk, + 1 are this half's
             const u32x4 hd = *(const u32x4 *) (ag + HDR + (b & 3) * 512 + r * 16);
             const uint32_t m = h ? ((hd[3] >> 4) & 0x0F0F0F0Fu) | ((hd[2] & 0xC0C0C0C0u) >> 2) : hd[2] & 0x3F3F3F3Fu;
 #pragma unroll
-            for (int i = 0; i < 8; ++i) mo[i] = (_Float16) (int) ((m >> (8 * (i >> 1))) & 63u);
+            for (int i = 0; i < 4; ++i) {
+                const _Float16 v = (_Float16) (int) ((m >> (16 * kk + 8 * (i >> 1))) & 63u);
+                mo[i] = kk ? (_Float16) 0.0f : v; mo[4 + i] = kk ? v : (_Float16) 0.0f;
+            }
         }
 #pragma unroll
         for (int jt = 0; jt < NT; ++jt) {
+            if (NT == 4) __builtin_amdgcn_sched_barrier(0);     // (the minima of all four token tiles at once: registers spill)
             const float da = *(const float *) (xb + XSUM + (32 * jt + r) * 4);
-            if (mins) {
-                const float16v z = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
-                const float16v am = __builtin_amdgcn_mfma_f32_32x32x16_f16(mo, *(const half8 *) (xb + (32 * jt + r) * 32 + 16 * h), z, 0, 0, 0);
+            if constexpr (TWO)
 #pragma unroll
-                for (int e = 0; e < 16; ++e) run[jt][e] = fmaf(da, fmaf(-dm[e], am[e], d[e] * acc[jt][e]), run[jt][e]);
+                for (int e = 0; e < 16; ++e) acc[jt][e] = TYPE == PM_Q6_K ? fmaf(64.0f, acc[jt][e], ac2[jt][e]) : acc[jt][e] + ac2[jt][e];
+            if (K45) {
+                const float16v am = __builtin_amdgcn_mfma_f32_32x32x16_f16(mo, *(const half8 *) (xb + (32 * jt + r) * 32 + 16 * h), zero, 0, 0, 0);
+#pragma unroll
+                for (int e = 0; e < 16; ++e) run[jt][e] = fmaf(da, fmaf(-dm(e), am[e], d(e) * acc[jt][e]), run[jt][e]);
             } else {
 #pragma unroll
-                for (int e = 0; e < 16; ++e) run[jt][e] = fmaf(da, d[e] * acc[jt][e], run[jt][e]);
+                for (int e = 0; e < 16; ++e) run[jt][e] = fmaf(da, d(e) * acc[jt][e], run[jt][e]);
             }
-#pragma unroll
-            for (int e = 0; e < 16; ++e) acc[jt][e] = 0.0f;
         }
     };
 
@@ -683,12 +704,21 @@ __device__ __forceinline__ void mid_body(const PfP & p, const PfJob & jb, const 
         if (Q8 && 2 * b + 1 >= nsteps) break;
         multiply(b, 1, bb, sl, [&](int u) __attribute__((always_inline)) { request(2 * b + 1, false, u); });
         if constexpr (EX) fold(b);
+        if constexpr (SUMS)
+            if (((b - b0) & 3) == 3)
+#pragma unroll
+                for (int jt = 0; jt < NT; ++jt) {
+                    tot[jt] += run[jt]; run[jt] = zero;
+                }
         settle(false);
         turn();
     }
     if constexpr (EX)
 #pragma unroll
-        for (int jt = 0; jt < NT; ++jt) acc[jt] = run[jt];
+        for (int jt = 0; jt < NT; ++jt) {
+            acc[jt] = run[jt];
+            if constexpr (SUMS) acc[jt] += tot[jt];
+        }
     mid_wait<0>();                                             // (the last steps' look-ahead still lands in the buffers)
     __syncthreads();
     // ---- the two halves of K: every wave keeps its rows' tokens [32 NH kk, + 32 NH) and takes the partner's sums of them
@@ -1069,7 +1099,9 @@ static int launch_pf(const pm_gemm_pf_job * jobs, int njobs, const void * xh, co
     // 101 tokens 65.8 / 70, 128256 x 4096 (Q6_K) 209 / 235. Beyond 128 tokens mid_body is still the faster one (4096 x 4096: 256 tokens 55.8 / 26.6, 512 60 / 36) and not taken for its
     // results: it adds the halves of every 128 k in another order, and tokens decoded behind such a prompt then differ from those behind pf_body's by up to 3 % of their logits (eight layers of
     // the 8B shape; their 8-bit roundings turn), although neither is nearer to 64 bits
-    const int mid_nt = T <= 64 ? 2 : 4;
+    bool two = false;                                           // 8-bit activations: tiles of 64 tokens for what needs a second set of accumulators
+    for (int j = 0; j < njobs; ++j) two |= wide && jobs[j].type != PM_Q4_K;
+    const int mid_nt = T <= 64 || two ? 2 : 4;
     long mid_wgs = 0;
     for (int j = 0; j < njobs && !(pair && j); ++j) mid_wgs += (jobs[j].N + (pair ? 63 : 127)) / (pair ? 64 : 128);
     // (8-bit activations: mid_body at any size - its tiles of 128 tokens side by side -, pf_body's registers are its accumulators')
@@ -1161,7 +1193,7 @@ static int launch_pf(const pm_gemm_pf_job * jobs, int njobs, const void * xh, co
         return 0;
     }
 #endif
-#define PF_GO(A, B) (wide ? nt == 4 ? go(gemm_pf_kernel<A, B, 4, true, 0, A != PM_Q8_0>, pf_lds_bytes<A, B, 4, true, A != PM_Q8_0>()) : go(gemm_pf_kernel<A, B, 2, true, 0, A != PM_Q8_0>, pf_lds_bytes<A, B, 2, true, A != PM_Q8_0>()) : mid ? nt == 4 ? go(gemm_pf_kernel<A, B, 4, true>, pf_lds_bytes<A, B, 4, true>()) : go(gemm_pf_kernel<A, B, 2, true>, pf_lds_bytes<A, B, 2, true>()) : nt == 8 ? go(gemm_pf_kernel<A, B, 8>, pf_lds_bytes<A, B, 8>()) : nt == 4 ? go(gemm_pf_kernel<A, B, 4>, pf_lds_bytes<A, B, 4>()) : go(gemm_pf_kernel<A, B, 2>, pf_lds_bytes<A, B, 2>()))
+#define PF_GO(A, B) (wide ? nt == 4 ? go(gemm_pf_kernel<PM_Q4_K, PM_Q4_K, 4, true, 0, true>, pf_lds_bytes<PM_Q4_K, PM_Q4_K, 4, true, true>()) : go(gemm_pf_kernel<A, B, 2, true, 0, A != PM_Q8_0>, pf_lds_bytes<A, B, 2, true, A != PM_Q8_0>()) : mid ? nt == 4 ? go(gemm_pf_kernel<A, B, 4, true>, pf_lds_bytes<A, B, 4, true>()) : go(gemm_pf_kernel<A, B, 2, true>, pf_lds_bytes<A, B, 2, true>()) : nt == 8 ? go(gemm_pf_kernel<A, B, 8>, pf_lds_bytes<A, B, 8>()) : nt == 4 ? go(gemm_pf_kernel<A, B, 4>, pf_lds_bytes<A, B, 4>()) : go(gemm_pf_kernel<A, B, 2>, pf_lds_bytes<A, B, 2>()))
     if (ta == tb) { if (ta == PM_Q4_K) PF_GO(PM_Q4_K, PM_Q4_K); else if (ta == PM_Q5_K) PF_GO(PM_Q5_K, PM_Q5_K); else if (ta == PM_Q8_0) PF_GO(PM_Q8_0, PM_Q8_0); else PF_GO(PM_Q6_K, PM_Q6_K); }
     else if (ta == PM_Q8_0 || tb == PM_Q8_0) return -1;      // (Q8_0 only as a launch of its own: ffn_down of the files whose n_ff is no multiple of 256)
     else if (ta == PM_Q4_K && tb == PM_Q5_K) PF_GO(PM_Q4_K, PM_Q5_K);

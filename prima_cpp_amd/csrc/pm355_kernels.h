@@ -145,7 +145,7 @@ int pm_launch_gemm_pf_norm(const pm_gemm_pf_job & job, const void * xh, int K, i
 // wq, wk, wv (jobs 0..2), then NORM rope and the stores into the cache (as pm_launch_rope_kv_store; tab: pm_launch_rope_table's) where that costs no launch (done; else the caller's own)
 struct pm_gemm_rope { const float * tab; const int32_t * pos, * seq; long seq_stride; void * kc, * vc; int Hkv, dh, n_ctx, n_dims, round_q, rows; bool done; };
 int pm_launch_gemm_pf_rope(const pm_gemm_pf_job * jobs, const void * xh, int K, int T, pm_gemm_rope * rope, hipStream_t st);
-// the same for 8-bit activations (up to PM_WIDE_MAX_TOKENS rows; Q4_K, Q5_K, Q6_K): the whole-number sums of pm_launch_mmq_i8. Jobs of at most two types
+// the same for 8-bit activations (up to PM_WIDE_MAX_TOKENS rows; Q4_K, Q5_K, Q6_K): whole-number sums as exact as pm_launch_mmq_i8's, of half a super-block each. Jobs of at most two types
 int pm_gemm_wide_check(int type, int K, int N, int T);
 int pm_launch_gemm_wide(const pm_gemm_pf_job * jobs, int njobs, const pm_q8k_wide & x, int K, int T, int pair, hipStream_t st, pm_gemm_rope * rope = nullptr);
 

@@ -274,7 +274,7 @@ def test_prompt_matmul_on_integer_matrix_cores(P, oracle, t):
 
 @pytest.mark.parametrize("t", [Q4_K, Q5_K, Q6_K])
 def test_wide_batch_matmul_with_8_bit_activations(P, oracle, t):
-    """The prompt GEMM's 8-bit form: whole-number sums of every super-block in the F16 matrix cores -> oracle.mul_mat (integers) within the tolerance of the integer kernels. Edges: rows and
+    """The prompt GEMM's 8-bit form: whole-number sums of every half super-block in the F16 matrix cores -> oracle.mul_mat (integers) within the tolerance of the integer kernels. Edges: rows and
     tokens of partial tiles, either tile size (33 / 64, 65 / 128 tokens), an odd number of super-blocks, K split over workgroups (32 super-blocks), matrices of two types, pair tiles. Quants and
     scales at their limits: weights of all-ones bytes (Q6_K: the largest quants with scales of -1, Q4_K / Q5_K the largest quants, scales and minima) and scales of -128 (Q6_K: products of 4096)."""
     rng = np.random.default_rng(700 + t)
@@ -305,9 +305,35 @@ def test_wide_batch_matmul_with_8_bit_activations(P, oracle, t):
     for x in (np.ones((T, K), np.float32), rng.choice([-1.0, 1.0], (T, K)).astype(np.float32), rng.normal(0, 1, (T, K)).astype(np.float32)):
         want = oracle.mul_mat(t, b, K, N, x)
         y = P.mul_mat_wide([P.upload_weight(t, b, K, N)], _dev(P, x))[0].cpu().numpy()
-        # (a super-block's sums beyond 2^24 are rounded as they are added up: 16 instructions for each half of its k, 2^-24 of the largest partial sum each)
-        lim = (K // 256) * 2 * 16 * 2.0 ** -24 * (4096 * 127 * 128) * 0.01 * np.abs(x).max() / 127
+        # (the sums cancel: three f32 roundings of each half super-block's sum and one of every sum so far, 2^-24 of at most sum |w x| each, here and in the oracle)
+        lim = (3 + 2 * (K // 256)) * 2 * 2.0 ** -24 * K * {Q4_K: 945, Q5_K: 1953, Q6_K: 4096}[t] * 0.01 * np.abs(x).max()
         assert np.allclose(y, want, rtol=2e-5, atol=2e-5 + lim), np.abs(y - want).max()
+
+
+@pytest.mark.parametrize("T", [40, 130])
+@pytest.mark.parametrize("t", [Q4_K, Q5_K, Q6_K])
+def test_wide_batch_matmul_adds_whole_numbers_exactly(P, oracle, t, T):
+    """Quants and scales at their largest (Q6_K: 31 x 127, odd), values of 126 and 127 that change sign between the 128-k halves of a super-block: partial sums of up to 64 x 3937 x 127 = 2^24.9 on
+    the way to a few ten thousand. Whole numbers of that size are not all in f32's 24 bits: the sums of a super-block have to be exact, as in the integer kernels. Bound: three roundings of each
+    half super-block's sum and one of every sum so far, 2^-24 of what they round, here and in the oracle."""
+    rng = np.random.default_rng(900 + t + T)
+    K, N = 1024, 64
+    nb = K // 256
+    b = np.full(rand_blocks(t, N, K, rng).shape, 0xFF, np.uint8).reshape(N, nb, -1)
+    if t == Q6_K:
+        b[:, :, 192:208], b[:, :, 208:] = 0x7F, np.frombuffer(np.float16(0.01).tobytes(), np.uint8)
+    else:
+        b[:, :, :4] = np.frombuffer(np.float16([0.01, 0.0]).tobytes(), np.uint8)
+    b = b.reshape(-1)
+    v = rng.integers(126, 128, (T, nb, 2, 128))
+    v[:, :, 0, 0] = 127
+    v[:, :, 1] *= -1
+    x = (v / 127.0).astype(np.float32).reshape(T, K)
+    half = np.abs(v.reshape(T, nb, 2, 2, 64).sum((2, 4))).sum((1, 2)) * {Q4_K: 15 * 63, Q5_K: 31 * 63, Q6_K: 31 * 127}[t] * float(np.float16(0.01)) / 127
+    want = oracle.mul_mat(t, b, K, N, x)
+    y = P.mul_mat_wide([P.upload_weight(t, b, K, N)], _dev(P, x))[0].cpu().numpy()
+    err = np.abs(y.astype(np.float64) - want)
+    assert (err <= (half * (3 + 2 * nb) * 2 * 2.0 ** -24)[:, None]).all(), (err.max(), half.max())
 
 
 @pytest.mark.parametrize("t", [Q4_K, Q6_K])
