@@ -783,7 +783,8 @@ int run_window(pm_window * m, const int32_t * d_tokens, const float * d_x_in, in
                 const Tensor & w = L.t[kind];
                 j[i].type = w.type; j[i].N = (int) w.N; j[i].W = w.d; j[i].Y = y; j[i].bias = bias < 0 ? nullptr : (const float *) L.t[bias].d; j[i].resid = resid;
             };
-            const pm_q8k_wide xe = pm_q8k_wide_at(m->wide, E), xa = pm_q8k_wide_at(m->wide, Eq), xf = pm_q8k_wide_at(m->wide, F);
+            const int wr = std::min(m->max_tokens, PM_WIDE_MAX_TOKENS);
+            const pm_q8k_wide xe = pm_q8k_wide_at(m->wide, E, wr), xa = pm_q8k_wide_at(m->wide, Eq, wr), xf = pm_q8k_wide_at(m->wide, F, wr);
             float * x_mid = (cur == bufs[0]) ? bufs[1] : bufs[0];
             float * x_next = (il == m->hi - 1 && d_x_out) ? d_x_out : ((x_mid == bufs[0]) ? bufs[1] : bufs[0]);
             pm_launch_rmsnorm_wide(cur, (const float *) L.t[PM355_T_ATTN_NORM].d, xe, E, T, hp.rms_eps, st);
@@ -1365,11 +1366,16 @@ int pm_window::finalize_pool(int max_tokens_, int n_seq_, int64_t pool_tokens) {
     const size_t T = max_tokens;
     for (void * p : {(void *) rows, (void *) d_rows, (void *) head_lg, (void *) wide}) if (p) (void) hipFree(p);
     rows = head_lg = nullptr; d_rows = nullptr; wide = nullptr;
-    if (max_tokens > MMQ_MAX_TOKENS && wide_path(this) &&
-        hipMalloc((void **) &wide, pm_q8k_wide_bytes(std::max({hp.n_embd, hp.head_dim * hp.n_head, hp.n_ff}))) != hipSuccess) return seterr(this, PM355_E_NOMEM, "finalize_pool: activations");
     // (tables of a pass, pm_launch_batch_rows: 3 integers per row, 4 per tile, 2 per sequence, 1 per wanted row, 2 per kept token)
-    return hipMalloc((void **) &rows, T * hp.n_embd * 4 + 256) == hipSuccess && hipMalloc((void **) &d_rows, 12 * T * 4 + 256) == hipSuccess &&
-           hipMalloc((void **) &head_lg, (size_t) std::min(max_tokens, HEAD_ROWS) * hp.n_vocab * 4 + 256) == hipSuccess ? 0 : seterr(this, PM355_E_NOMEM, "finalize_pool: hidden rows");
+    if (hipMalloc((void **) &rows, T * hp.n_embd * 4 + 256) != hipSuccess || hipMalloc((void **) &d_rows, 12 * T * 4 + 256) != hipSuccess ||
+        hipMalloc((void **) &head_lg, (size_t) std::min(max_tokens, HEAD_ROWS) * hp.n_vocab * 4 + 256) != hipSuccess) return seterr(this, PM355_E_NOMEM, "finalize_pool: hidden rows");
+    // (wide passes only make batches shorter: without the memory for them the rows go through small ones)
+    if (max_tokens > MMQ_MAX_TOKENS && wide_path(this) &&
+        hipMalloc((void **) &wide, pm_q8k_wide_bytes(std::max({hp.n_embd, hp.head_dim * hp.n_head, hp.n_ff}), std::min(max_tokens, PM_WIDE_MAX_TOKENS))) != hipSuccess) {
+        wide = nullptr;
+        (void) hipGetLastError();
+    }
+    return 0;
 }
 int pm_window::seq_new() {
     if (!finalized) return seterr(this, PM355_E_SHAPE, "seq_new: model not finalized");

@@ -1217,9 +1217,11 @@ int pm_launch_gemm_wide(const pm_gemm_pf_job * jobs, int njobs, const pm_q8k_wid
     for (int j = 0; j < njobs; ++j) if (pm_gemm_wide_check(jobs[j].type, K, jobs[j].N, T)) return -1;
     return launch_pf(jobs, njobs, x.q, &x, K, T, pair, st, nullptr, rope);
 }
-size_t pm_q8k_wide_bytes(int K) { return (size_t) PM_WIDE_MAX_TOKENS * ((size_t) K * 2 + (size_t) (K / 256) * 36); }
-pm_q8k_wide pm_q8k_wide_at(void * buf, int K) {
+static size_t wide_rows(int rows) { return rows <= 64 ? 64 : (size_t) (rows + 127) / 128 * 128; }
+size_t pm_q8k_wide_bytes(int K, int rows) { return wide_rows(rows) * ((size_t) K * 2 + (size_t) (K / 256) * 36); }
+pm_q8k_wide pm_q8k_wide_at(void * buf, int K, int rows) {
+    const size_t n = wide_rows(rows);
     pm_q8k_wide x;
-    x.q = (uint16_t *) buf; x.s = x.q + (size_t) PM_WIDE_MAX_TOKENS * K; x.d = (float *) (x.s + (size_t) PM_WIDE_MAX_TOKENS * (K / 256) * 16); x.ldt = PM_WIDE_MAX_TOKENS;
+    x.q = (uint16_t *) buf; x.s = x.q + n * K; x.d = (float *) (x.s + n * (K / 256) * 16); x.ldt = (int) n;
     return x;
 }

@@ -52,8 +52,8 @@ struct pm_q8k_tables { uint8_t * base = nullptr; size_t tab_bytes = 0; int nsb =
 // Q8_K activations of up to PM_WIDE_MAX_TOKENS rows for pm_launch_gemm_wide: the 8-bit values as F16 [row][K], sums of 16 as F16 [super-block][ldt][16], scales [super-block][ldt]
 constexpr int PM_WIDE_MAX_TOKENS = 512;
 struct pm_q8k_wide { uint16_t * q = nullptr, * s = nullptr; float * d = nullptr; int ldt = 0; };
-size_t pm_q8k_wide_bytes(int K);
-pm_q8k_wide pm_q8k_wide_at(void * buf, int K);                         // a buffer of pm_q8k_wide_bytes(K), 16-byte aligned
+size_t pm_q8k_wide_bytes(int K, int rows = PM_WIDE_MAX_TOKENS);       // rows that a pass of `rows` tokens reads, whole tiles
+pm_q8k_wide pm_q8k_wide_at(void * buf, int K, int rows = PM_WIDE_MAX_TOKENS);      // a buffer of pm_q8k_wide_bytes(K, rows), 16-byte aligned
 void pm_launch_quantize_wide(const float * x, const pm_q8k_wide & y, int K, int rows, hipStream_t st);
 void pm_launch_rmsnorm_wide(const float * x, const float * w, const pm_q8k_wide & y, int K, int rows, float eps, hipStream_t st);
 void pm_launch_quantize_q8k(const float * x, void * y, int K, int rows, hipStream_t st, pm_q8k_tables tab = {});

@@ -1,0 +1,129 @@
+"""What the library's host code launches, and in what order, on the CPU: in a process of its own, in front of a HIP runtime that runs nothing (hip_shim.cpp)."""
+import os
+import subprocess
+import sys
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+ROOT = os.path.dirname(HERE)
+LIB = os.path.join(ROOT, "prima_cpp_amd", "libprima_mi355.so")
+
+COMMON = r"""
+import ctypes as C, sys, threading
+shim = C.CDLL(sys.argv[1])
+shim.shim_launches.restype, shim.shim_held.restype = C.c_long, C.c_size_t
+shim.shim_refuse.argtypes = [C.c_size_t]
+def launches():
+    out, name, r = (C.c_int * 4)(), C.create_string_buffer(500), []
+    for i in range(shim.shim_launches()):
+        shim.shim_launch(C.c_long(i), out, name, C.c_long(500))
+        r.append((out[0], name.value.decode().replace("(anonymous namespace)::", ""), tuple(out[1:])))
+    return r
+"""
+WINDOW = COMMON + r"""
+import numpy as np, torch
+torch.cuda.current_device = lambda: 0
+import prima_cpp_amd.engine as E
+E.stream_ptr = lambda: 1
+Q4_K, Q6_K = 12, 14
+def window(n_ctx=64, down=Q4_K, max_tokens=64, seqs=8, **hp):
+    hp = dict(dict(arch=0, n_layer=1, n_embd=2048, n_head=16, n_head_kv=4, head_dim=128, n_ff=4096, n_vocab=320, rms_eps=1e-5, rope_freq_base=10000.0), **hp)
+    w = E.Window(hp, n_ctx=n_ctx)
+    for il in range(hp["n_layer"]):
+        for k in (E.T_ATTN_NORM, E.T_FFN_NORM):
+            w.fill_tensor(k, il, 0, 1, 1.0)
+        for k in (E.T_WQ, E.T_WK, E.T_WV, E.T_WO, E.T_FFN_GATE, E.T_FFN_UP, E.T_FFN_DOWN):
+            w.fill_tensor(k, il, down if k == E.T_FFN_DOWN else Q4_K, 1, 1.0)
+    w.fill_tensor(E.T_OUT_NORM, -1, 0, 1, 1.0); w.fill_tensor(E.T_OUTPUT, -1, Q6_K, 1, 1.0); w.fill_tensor(E.T_TOK_EMBD, -1, Q4_K, 1, 1.0)
+    w.finalize_pool(max_tokens, seqs, seqs * n_ctx)
+    return w
+def batch(w, lens):
+    qs = [w.seq_new() for _ in lens]
+    shim.shim_forget()
+    w.batch([(q, np.zeros(n, np.int32), (n - 1,)) for q, n in zip(qs, lens)], logits=torch.zeros(len(lens), 320))
+    return [name for _, name, _ in launches()]
+def wide(names):
+    return sum("gemm_pf_kernel" in n and "true, 0, true>" in n for n in names)
+"""
+
+
+@pytest.fixture(scope="module")
+def run(tmp_path_factory):
+    if not os.path.exists(LIB):
+        pytest.skip("library not built")
+    shim = str(tmp_path_factory.mktemp("shim") / "hip_shim.so")
+    subprocess.run(["g++", "-O1", "-shared", "-fPIC", "-std=c++17", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include", os.path.join(HERE, "hip_shim.cpp"), "-o", shim, "-lpthread"], check=True)
+
+    def go(program):
+        env = dict(os.environ, LD_PRELOAD=shim, PYTHONPATH=ROOT)
+        r = subprocess.run([sys.executable, "-c", program, shim, LIB], env=env, capture_output=True, text=True, timeout=300)
+        assert r.returncode == 0 and r.stdout.strip().endswith("ok"), r.stdout + r.stderr
+    return go
+
+
+def test_slices_of_a_product_are_added_up_before_another_product_of_the_stream(run):
+    """The slices of a product that is split along K wait in scratch memory of the (device, stream) for the launch that adds them up: no other thread's launch of the same kind comes between."""
+    run(COMMON + r"""
+lib = C.CDLL(sys.argv[2])
+f = lib.pm355_mul_mat_q_wide
+f.argtypes = [C.c_void_p, C.c_int] + [C.c_void_p] * 6 + [C.c_int64, C.c_int64, C.c_int, C.c_void_p, C.c_void_p]
+K, N, T, CALLS = 8192, 256, 40, 20                     # 32 super-blocks over two row tiles: split along K
+at = C.addressof(C.create_string_buffer(256))
+shim.shim_pause(300)
+bad = []
+def work(i):
+    shim.shim_thread(i)
+    ty, W, y, n = (C.c_int * 1)(12), (C.c_void_p * 1)(at), (C.c_void_p * 1)(at), (C.c_int64 * 1)(N)
+    for _ in range(CALLS):
+        rc = f(ty, 1, W, n, y, None, None, at, K, T, 0, at, 1)
+        if rc: bad.append(rc)
+ts = [threading.Thread(target=work, args=(i,)) for i in range(2)]
+[t.start() for t in ts]; [t.join() for t in ts]
+assert not bad, bad
+log = launches()
+assert len(log) == 2 * CALLS * 3, len(log)              # quantizer, product, its slices added up
+both = [e for e in log if "quantize" not in e[1]]       # (the quantizer writes memory of the call's own)
+for i in range(0, len(both), 2):
+    a, b = both[i:i + 2]
+    assert a[0] == b[0] and "gemm_pf_kernel" in a[1] and "pf_reduce" in b[1], (i, both[max(i - 2, 0):i + 4])
+assert sum(log[i][0] != log[i + 1][0] for i in range(len(log) - 1)) > 4     # (the threads did meet)
+print("ok")
+""")
+
+
+def test_a_pool_without_memory_for_wide_passes_serves_small_ones(run):
+    """Activations of wide passes: as many rows as a pass may have, and where the device does not have them the pool is there all the same."""
+    run(WINDOW + r"""
+rows = lambda n, K: n * (2 * K + K // 256 * 36)         # values as F16, 16 sums as F16 and a scale per super-block
+for n, m in ((33, 64), (64, 64), (100, 128), (300, 384), (512, 512)):
+    h = shim.shim_held(); w = window(max_tokens=n); full = shim.shim_held() - h
+    assert wide(batch(w, [7] * 8)) == (4 if n > 33 else 0)
+    w.close()
+    shim.shim_refuse(rows(m, 4096))                     # (n_ff is the longest row)
+    h = shim.shim_held(); w = window(max_tokens=n); less = shim.shim_held() - h
+    assert full - less == rows(m, 4096), (n, full - less)
+    assert wide(batch(w, [7] * 8)) == 0 and shim.shim_last() == 0
+    w.close()
+    shim.shim_refuse(0)
+print("ok")
+""")
+
+
+def test_which_portions_meet_in_wide_passes(run):
+    """More rows of short portions than one small pass takes: wide passes, whose wq | wk | wv ends with the rope and the cache stores at up to 255 rows, plain beyond."""
+    run(WINDOW + r"""
+w = window(max_tokens=512, seqs=24)
+names = batch(w, [7] * 8)
+assert wide(names) == 4 and sum("pf_reduce_rope_kernel" in n for n in names) == 1 and not any("rope_kv" in n for n in names), names
+w = window(max_tokens=512, seqs=24)
+names = batch(w, [30] * 10)                             # 300 rows
+assert wide(names) == 4 and not any("pf_reduce_rope_kernel" in n for n in names) and any("rope_kv" in n for n in names), names
+w = window(max_tokens=512, seqs=24)
+assert wide(batch(w, [4] * 8)) == 0                     # 32 rows: one small pass
+w = window(max_tokens=33, seqs=24)
+assert wide(batch(w, [4] * 9)) == 0                     # two passes of 18: small ones
+w = window(max_tokens=512, seqs=24)
+assert wide(batch(w, [40, 50])) == 0                    # longer portions: 16-bit activations
+print("ok")
+""")
