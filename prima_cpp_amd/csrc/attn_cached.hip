@@ -43,7 +43,8 @@ template <int DH, int KPL> struct ShortLds {
 // Rounding points as everywhere: q, K, V F16, the normalised probabilities rounded to F16, f32 accumulation. n_kv <= 64 * KPL <= n_ctx; DH 64 / 128 (256: KPL = 1).
 template <int DH, int KPL>
 __device__ __forceinline__ void attn_short(const float * q_head, const uint16_t * kc, const uint16_t * vc, float * out_head, int hk, int Hkv, int n_ctx, int n_kv, float scale, const void * mask,
-                                           int mask_f16, char * smem, int lane, int wave) {
+                                           int mask_f16, char * smem, int lane, int wave, unsigned long long * ts) {
+    unsigned long long tsv[6] = {PM_TS_NOW(), 0, 0, 0, 0, 0};
     typedef ShortLds<DH, KPL> S;
     constexpr int NKEY = 64 * KPL, NKW = NKEY / 4, LPK = DH / 8, KPI = 64 / LPK, NI = NKW / KPI, DPW = DH / 4, LV = 8 * KPL, DPI = 64 / LV, NV = DPW / DPI, KPP = NKEY * DPW / 64;
     float * const part = (float *) smem, * const qs = (float *) (smem + 12 * NKEY) + DH * wave;
@@ -69,6 +70,7 @@ __device__ __forceinline__ void attn_short(const float * q_head, const uint16_t 
 #pragma unroll
     for (int i = 0; i < NI; ++i) *(u32x4 *) (st + (KPI * i + ks) * S::K_PITCH + 16 * kd) = kreg[i];
     staged();
+    tsv[1] = PM_TS_NOW();                                      // loads back
     // ---- scores: lane = (key l of the wave, quarters u0 .. u0 + KPL - 1 of the head)
     const int l = lane % NKW, u0 = KPL * (lane / NKW);
     float acc[KPL];
@@ -101,6 +103,7 @@ __device__ __forceinline__ void attn_short(const float * q_head, const uint16_t 
 #pragma unroll
     for (int i = 0; i < NV; ++i) *(u32x4 *) (st + (DPI * i + ve) * S::V_PITCH + 16 * c) = vreg[i];
     __syncthreads();                                           // the only workgroup barrier of this path
+    tsv[2] = PM_TS_NOW();                                      // scores
     float s_[KPL], mx = -INFINITY;
 #pragma unroll
     for (int k = 0; k < KPL; ++k) {
@@ -117,6 +120,7 @@ __device__ __forceinline__ void attn_short(const float * q_head, const uint16_t 
 #pragma unroll
     for (int k = 0; k < KPL; ++k) pw[lane + 64 * k] = f2h(ex[k] * inv);            // p rounded to F16 (src1 of the V^T.p product)
     staged();
+    tsv[3] = PM_TS_NOW();                                      // softmax
     // ---- P.V: lane = (dimension e, part kp of the cells). Pieces without an attended cell repeat the row's first one, against probabilities of zero
     const int e = lane % DPW, kp = lane / DPW;
     float o = 0.0f;
@@ -130,9 +134,12 @@ __device__ __forceinline__ void attn_short(const float * q_head, const uint16_t 
             o = fmaf(h2f((uint16_t) (w[t] >> 16)), h2f((uint16_t) (p[t] >> 16)), o);
         }
     }
+    tsv[4] = PM_TS_NOW();                                      // P.V
     if constexpr (DPW <= 16) o += __builtin_bit_cast(float, other_row(__builtin_bit_cast(uint32_t, o)));
     if constexpr (DPW <= 32) o += __builtin_bit_cast(float, other_half(__builtin_bit_cast(uint32_t, o)));
     if (lane < DPW) st_g(out_head + DPW * wave + lane, o);
+    tsv[5] = PM_TS_NOW();
+    pm_ts_store(ts, 2, tsv);
 }
 
 template <int DH, int VM>
@@ -157,7 +164,7 @@ __global__ __launch_bounds__(256) void attn_cached_kernel(AttnP a_in) {
         }
         const uint16_t * kc = a.kc + (long) seq * a.seq_stride, * vc = a.vc + (long) seq * a.seq_stride;
         auto go = [&](auto kpl) __attribute__((always_inline)) {
-            attn_short<DH, decltype(kpl)::value>(a.q + (long) h * DH, kc, vc, a.out + (long) h * DH, hk, Hkv, n_ctx, n_kv, a.scale, a.mask, a.mask_f16, smem, lane, wave);
+            attn_short<DH, decltype(kpl)::value>(a.q + (long) h * DH, kc, vc, a.out + (long) h * DH, hk, Hkv, n_ctx, n_kv, a.scale, a.mask, a.mask_f16, smem, lane, wave, a.ts);
         };
         // (caches that hold fewer cells than the form takes: the general body, as it always was - its sums are in another order)
         if (n_kv <= 64 && n_ctx >= 64) return go(std::integral_constant<int, 1>());
