@@ -837,11 +837,11 @@ __global__ __launch_bounds__(PF_NTHR) void gemm_pf_kernel(PfP p) {
 // The slabs of a launch's split tiles, added in slice order, and the epilogue: a wave per 32 rows x 8 tokens, 8 lanes on a token's 32 rows, all S parts on their way at once. Bound by the slabs'
 // bytes. A launch of its own because all CUs then share them: the last arriver of a tile (64 of 256 workgroups for 8192 rows x 512 tokens, S = 4) read 1 MB of slabs and stored its tile by
 // itself, 48 us behind the last product. us, last arriver (as it was; its loads in fours and the slabs written through) / product + this launch: 512 tokens of 8192 x 8192 Q4_K 107 (102) / 66 + 17,
-// 8192 x 28672 264 (245) / 211 + 17, 10240 x 8192 131 (120) / 91 + 15; 101 tokens (mid_body) of 4096 x 4096 23.0 / 18.3 + 4.8, 4096 x 14336 35.9 / 27.7 + 5.9. KPW: 8-token groups of a wave, 1 (4: fewer
-// waves, 18.7 for 16.8 and 8.1 for 5.9)
+// 8192 x 28672 264 (245) / 211 + 17, 10240 x 8192 131 (120) / 91 + 15; 101 tokens (mid_body) of 4096 x 4096 23.0 / 18.3 + 4.8, 4096 x 14336 35.9 / 27.7 + 5.9. (A wave per 32 tokens: 18.7 for 16.8 and
+// 8.1 for 5.9)
 // nti: token sub-tiles of a wave; mid: mid_body's tiles (wave = row group + 4 x token half)
-template <int SMAX, int KPW> __global__ __launch_bounds__(256) void pf_reduce_kernel(PfP p, int mid, int nti, int units) {
-    const int u4 = (int) blockIdx.x * 4 + __builtin_amdgcn_readfirstlane((int) threadIdx.x >> 6), unit = u4 / (4 / KPW), k0 = u4 % (4 / KPW) * KPW, lane = threadIdx.x & 63;
+template <int SMAX> __global__ __launch_bounds__(256) void pf_reduce_kernel(PfP p, int mid, int nti, int units) {
+    const int u4 = (int) blockIdx.x * 4 + __builtin_amdgcn_readfirstlane((int) threadIdx.x >> 6), unit = u4 >> 2, k0 = u4 & 3, lane = threadIdx.x & 63;
     if (unit >= units) return;
     const int S = p.splitk, per_tile = (p.pair ? 4 : 8) * nti, tile_id = unit / per_tile, wv = unit % per_tile / nti, i = unit % nti;
     const int x = tile_id & 7, slot = p.full + (tile_id >> 3), per_x = (p.nt_n + 7 - x) >> 3;
@@ -858,48 +858,35 @@ template <int SMAX, int KPW> __global__ __launch_bounds__(256) void pf_reduce_ke
         n0 = (tile_n - jb.tile0) * (mid ? 128 : 256);
         if (mid) { row = wv & 3; half = wv >> 2; }
     }
-    const int t0 = (tile_t * (mid ? 2 : 1) + half) * 32 * nti + 32 * i + 8 * k0, n = n0 + 32 * row + (lane & 7) * 4;
+    const int t0 = (tile_t * (mid ? 2 : 1) + half) * 32 * nti + 32 * i + 8 * k0, t = t0 + (lane >> 3), n = n0 + 32 * row + (lane & 7) * 4;
     if (t0 >= p.T || n >= jb.N) return;                         // (N is a multiple of 4)
     const size_t tile = (size_t) 8 * nti * 256;                 // of f32x4
     const f32x4 * const slab = (const f32x4 *) p.ws + (size_t) tile_id * S * tile + 64 * k0 + lane;
-    auto sums = [&](int w, f32x4 (&o)[KPW]) __attribute__((always_inline)) {
+    auto sum = [&](int w) __attribute__((always_inline)) {
         const f32x4 * const at = slab + (size_t) (w * nti + i) * 256;
-        f32x4 v[SMAX][KPW];
+        f32x4 v[SMAX], o = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-        for (int q = 0; q < SMAX; ++q)
+        for (int q = 0; q < SMAX; ++q) v[q] = *(const PM_G f32x4 *) (at + (size_t) (q < S ? q : S - 1) * tile);
 #pragma unroll
-            for (int k = 0; k < KPW; ++k) v[q][k] = *(const PM_G f32x4 *) (at + (size_t) (q < S ? q : S - 1) * tile + 64 * k);
-#pragma unroll
-        for (int k = 0; k < KPW; ++k) o[k] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-        for (int q = 0; q < SMAX; ++q) {
-            if (q >= S) break;
-#pragma unroll
-            for (int k = 0; k < KPW; ++k) o[k] += v[q][k];
-        }
+        for (int q = 0; q < SMAX; ++q) if (q < S) o += v[q];
+        return o;
     };
-    f32x4 o[KPW], gate[KPW];
-    sums(wave, o);
-    if (p.pair) sums(wave_g, gate);
+    f32x4 v = sum(wave), gate;
+    if (p.pair) gate = sum(wave_g);
+    if (t >= p.T) return;
+    const long at = (long) t * jb.ldy + n;
+    if (p.pair)
 #pragma unroll
-    for (int k = 0; k < KPW; ++k) {
-        const int t = t0 + 8 * k + (lane >> 3);
-        if (t >= p.T) continue;
-        const long at = (long) t * jb.ldy + n;
-        f32x4 v = o[k];
-        if (p.pair)
+        for (int e = 0; e < 4; ++e) v[e] *= gate[e] / (1.0f + expf(-gate[e]));
+    if (jb.bias) v += ld_g((const f32x4 *) (jb.bias + n));
+    if (jb.resid) v += ld_g((const f32x4 *) (jb.resid + at));
+    if (jb.silu_gate) {
+        const f32x4 gg = ld_g((const f32x4 *) (jb.silu_gate + at));
 #pragma unroll
-            for (int e = 0; e < 4; ++e) v[e] *= gate[k][e] / (1.0f + expf(-gate[k][e]));
-        if (jb.bias) v += ld_g((const f32x4 *) (jb.bias + n));
-        if (jb.resid) v += ld_g((const f32x4 *) (jb.resid + at));
-        if (jb.silu_gate) {
-            const f32x4 gg = ld_g((const f32x4 *) (jb.silu_gate + at));
-#pragma unroll
-            for (int e = 0; e < 4; ++e) v[e] *= gg[e] / (1.0f + expf(-gg[e]));
-        }
-        if (jb.Yh) *(PM_G half4v *) (jb.Yh + at) = half4v{(_Float16) v[0], (_Float16) v[1], (_Float16) v[2], (_Float16) v[3]};
-        else *(PM_G f32x4 *) (jb.Y + at) = v;
+        for (int e = 0; e < 4; ++e) v[e] *= gg[e] / (1.0f + expf(-gg[e]));
     }
+    if (jb.Yh) *(PM_G half4v *) (jb.Yh + at) = half4v{(_Float16) v[0], (_Float16) v[1], (_Float16) v[2], (_Float16) v[3]};
+    else *(PM_G f32x4 *) (jb.Y + at) = v;
 }
 
 // The same for one matrix of which every tile is split, a workgroup per token, with the RMS norm of the token's new row (rmsnorm_q8k_kernel's expressions in its order, F16): the row does not
@@ -1051,7 +1038,7 @@ int pm_gemm_pf_check(int type, int K, int N, int T) {
 // arithmetic only (tests/test_gemm_plan.py plans the layer shapes without a device). nt: 32-token sub-tiles per workgroup tile (2 / 4 / 8 = 64 / 128 / 256
 // tokens: a dequantized operand serves nt MFMAs; smaller tiles only where the batch has no more tokens). Few tiles - wo / ffn_down / wq | wk | wv at the
 // reference's default n_ubatch 512 (common/common.h:178) are 64-80 tiles for 256 CUs - are split along K: S slices per tile, the slice count that minimises
-// rounds of workgroups x (super-blocks per slice + ~3 for prologue, slab traffic and the reducer's pass). A launch of R full rounds + a short tail (wq | wk | wv
+// rounds of workgroups x (super-blocks per slice + ~3 for prologue, slab traffic and the launch that adds the slices up). A launch of R full rounds + a short tail (wq | wk | wv
 // at 2048 tokens: 320 tiles = 256 + 64; Qwen2.5-72B's ffn_gate | ffn_up: 1848 = 7 x 256 + 56) runs whole tiles in the full rounds and splits ONLY the tail's
 // tiles - as many slices as fill the idle CUs of the last round (`full` whole-tile slots per XCD come first in the grid). Splitting every tile instead sends
 // every partial tile through memory: 3 x 320 slabs of 256 KB for the qkv launch, 501 us = 685 TFLOP/s against 406 us = 846.
@@ -1066,7 +1053,7 @@ void pm_gemm_pf_plan(int tiles, int K, int T, int cus, int force_nt, int force_s
     const int minL = (tiles / 8) * nt_t, maxL = ((tiles + 7) / 8) * nt_t, cpx = cus / 8;      // per-XCD slot counts (XCD x owns the row tiles x, x + 8, ..)
     double best = (double) ((wgs + cus - 1) / cus) * nb;
     for (int q = 2; q <= 8; ++q) {
-        if (nb / q < 4 || wgs * q > 16384) break;
+        if (nb / q < 4 || wgs * q > 16384) break;               // (slabs of 256 KB: 4 GB at most)
         const double c = (double) ((wgs * q + cus - 1) / cus) * ((double) nb / q + 3.0);
         if (c < best * 0.97) { best = c; S = q; }
     }
@@ -1129,7 +1116,7 @@ static int launch_pf(const pm_gemm_pf_job * jobs, int njobs, const void * xh, co
     static const bool no_mixed = [] { const char * e = getenv("PM355_GEMM_PF_MIXED"); return e && e[0] == '0'; }();
     // 256-token tiles (a dequantized operand serves 8 MFMAs; 128-token tiles only where the batch has no more tokens). Few tiles - wo / ffn_down / wq | wk | wv
     // at the reference's default n_ubatch 512 (common/common.h:178) are 64-80 tiles for 256 CUs - are split along K: S slices per tile, the slice count that
-    // minimises  rounds of workgroups x (super-blocks per slice + ~3 for prologue, slab traffic and the reducer's pass)
+    // minimises  rounds of workgroups x (super-blocks per slice + ~3 for prologue, slab traffic and the launch that adds the slices up)
     pm_gemm_pf_plan_t pl;
     pm_gemm_pf_plan(tiles, K, T, cus, mid ? mid_nt : force_nt, force_s, no_mixed ? 0 : 1, &pl);
     const int nt = pl.nt, S = pl.splitk, full = pl.full, maxL = ((tiles + 7) / 8) * pl.nt_t;
@@ -1165,8 +1152,8 @@ static int launch_pf(const pm_gemm_pf_job * jobs, int njobs, const void * xh, co
             return;
         }
         const int units = 8 * split_slots * (p.pair ? 4 : 8) * nti;
-        if (S <= 4) hipLaunchKernelGGL((pf_reduce_kernel<4, 1>), dim3(units), dim3(256), 0, st, p, (int) mid, nti, units);
-        else        hipLaunchKernelGGL((pf_reduce_kernel<8, 1>), dim3(units), dim3(256), 0, st, p, (int) mid, nti, units);
+        if (S <= 4) hipLaunchKernelGGL(pf_reduce_kernel<4>, dim3(units), dim3(256), 0, st, p, (int) mid, nti, units);
+        else        hipLaunchKernelGGL(pf_reduce_kernel<8>, dim3(units), dim3(256), 0, st, p, (int) mid, nti, units);
     };
 #if PM_GEMM_ABLATE
     static const int exp_sw = [] { const char * e = getenv("PM355_GEMM_EXP"); return e ? atoi(e) : 0; }();

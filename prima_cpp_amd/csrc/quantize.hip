@@ -270,10 +270,10 @@ void pm_launch_quantize_q80(const float * x, void * y, int K, int rows, hipStrea
                        x, (uint8_t *) y, K, rows, pm_q80_row_bytes(K));
 }
 void pm_launch_rmsnorm_q8k(const float * x, const float * w, float * ynorm, void * yq, int K, int rows, float eps, hipStream_t st, void * ynorm_f16, pm_q8k_tables tab) {
-    if (rows <= 256) hipLaunchKernelGGL(rmsnorm_q8k_kernel<16>, dim3(rows), dim3(1024), 0, st, x, w, ynorm, (uint8_t *) yq, K, eps, pm_q8k_row_bytes(K), (_Float16 *) ynorm_f16, tab, pm_q8k_wide());
+    if (rows <= pm_device_cus()) hipLaunchKernelGGL(rmsnorm_q8k_kernel<16>, dim3(rows), dim3(1024), 0, st, x, w, ynorm, (uint8_t *) yq, K, eps, pm_q8k_row_bytes(K), (_Float16 *) ynorm_f16, tab, pm_q8k_wide());
     else            hipLaunchKernelGGL(rmsnorm_q8k_kernel<4>, dim3(rows), dim3(256), 0, st, x, w, ynorm, (uint8_t *) yq, K, eps, pm_q8k_row_bytes(K), (_Float16 *) ynorm_f16, tab, pm_q8k_wide());
 }
 void pm_launch_rmsnorm_wide(const float * x, const float * w, const pm_q8k_wide & y, int K, int rows, float eps, hipStream_t st) {
-    if (rows <= 256) hipLaunchKernelGGL(rmsnorm_q8k_kernel<16>, dim3(rows), dim3(1024), 0, st, x, w, (float *) nullptr, (uint8_t *) nullptr, K, eps, 0, (_Float16 *) nullptr, pm_q8k_tables(), y);
+    if (rows <= pm_device_cus()) hipLaunchKernelGGL(rmsnorm_q8k_kernel<16>, dim3(rows), dim3(1024), 0, st, x, w, (float *) nullptr, (uint8_t *) nullptr, K, eps, 0, (_Float16 *) nullptr, pm_q8k_tables(), y);
     else             hipLaunchKernelGGL(rmsnorm_q8k_kernel<4>, dim3(rows), dim3(256), 0, st, x, w, (float *) nullptr, (uint8_t *) nullptr, K, eps, 0, (_Float16 *) nullptr, pm_q8k_tables(), y);
 }
