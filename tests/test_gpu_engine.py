@@ -213,6 +213,82 @@ def test_prompt_with_norms_behind_split_products(E, oracle, T, n_embd):
     w.close()
 
 
+def _filled_window(E, n_embd, n_head, n_head_kv, n_ff, n_ctx, bias, flags=0, down=Q6_K):
+    """two layers of random weights made on the device (n_vocab 320 where the window has its ends)"""
+    w = E.Window(dict(arch=0, n_layer=2, n_embd=n_embd, n_head=n_head, n_head_kv=n_head_kv, head_dim=128, n_ff=n_ff, n_vocab=320, rms_eps=1e-5, rope_freq_base=10000.0), flags=flags, n_ctx=n_ctx)
+    for il in range(2):
+        for i, kind in enumerate((E.T_ATTN_NORM, E.T_FFN_NORM)):
+            w.fill_tensor(kind, il, E.F32, 100 * il + 1 + i, 0.0)
+        for i, kind in enumerate((E.T_WQ, E.T_WK, E.T_WV, E.T_WO, E.T_FFN_GATE, E.T_FFN_UP, E.T_FFN_DOWN)):
+            w.fill_tensor(kind, il, down if kind == E.T_FFN_DOWN else Q4_K, 100 * il + 10 + i, 2.0 / np.sqrt(n_ff if kind == E.T_FFN_DOWN else n_embd))
+        for i, kind in enumerate((E.T_BQ, E.T_BK, E.T_BV) if bias else ()):
+            w.fill_tensor(kind, il, E.F32, 100 * il + 20 + i, 0.5)
+    if flags:
+        w.fill_tensor(E.T_OUT_NORM, -1, E.F32, 300, 0.0)
+        w.fill_tensor(E.T_OUTPUT, -1, Q6_K, 301, 2.0 / np.sqrt(n_embd))
+        w.fill_tensor(E.T_TOK_EMBD, -1, Q4_K, 302, 1.0)
+    return w
+
+
+# rows of a norm beyond 4096 and of wq | wk | wv beyond 4096 and 8192 (a wave's second and third column), K in five to eight slices and in fewer, tiles of 128 and of 256 rows
+# (test_host_launches.py holds which shape reaches which form)
+SLICED = [(4352, 32, 8, 14336), (8192, 64, 8, 28672), (8192, 16, 4, 4096)]
+
+
+@pytest.mark.parametrize("bias", [False, True])
+@pytest.mark.parametrize("n_embd,n_head,n_head_kv,n_ff", SLICED)
+def test_prompts_with_slices_added_up_in_the_norm_and_the_rope(E, n_embd, n_head, n_head_kv, n_ff, bias):
+    """560 tokens in one pass - slices, norms, rope and cache stores are launches of their own at that size - against passes of 72 (128-row tiles), 130, 200 and 158 tokens, whose slices are added
+    up by the launches that form the norm and that rotate and store, and of 512 and 48 (norm only). The same sums in slices of other lengths: f32 rounding, which turns F16 roundings of the
+    activations (2^-11 of one) here and there; a wrong row, column, position or slice is another value altogether."""
+    torch = E.torch
+    T = 560
+    w = _filled_window(E, n_embd, n_head, n_head_kv, n_ff, 576, bias)
+    w.finalize(max_tokens=T)
+    x = torch.randn((T, n_embd), generator=torch.Generator(device="cuda").manual_seed(n_embd + n_head), device="cuda")
+    one = torch.randn((3, n_embd), generator=torch.Generator(device="cuda").manual_seed(1), device="cuda")
+    want = w.decode(x_in=x, pos0=0)[0].double()
+    behind = [w.decode(x_in=one[i:i + 1], pos0=T + i)[0].double() for i in range(3)]
+    for lens in ((72, 130, 200, 158), (512, 48)):
+        w.kv_clear()
+        at = 0
+        for n in lens:
+            got = w.decode(x_in=x[at:at + n].contiguous(), pos0=at)[0].double()
+            err = (got - want[at:at + n]).norm(dim=1) / want[at:at + n].norm(dim=1)
+            assert err.max() < 2e-3, (lens, at, err.max().item(), err.argmax().item())
+            at += n
+        for i in range(3):                                      # single tokens read the cache that the passes left
+            got = w.decode(x_in=one[i:i + 1], pos0=T + i)[0].double()
+            assert (got - behind[i]).norm() < 2e-2 * behind[i].norm(), ((got - behind[i]).norm() / behind[i].norm()).item()
+    w.close()
+
+
+@pytest.mark.parametrize("n_embd,n_head,n_head_kv,n_ff,lens", [(2048, 16, 4, 4096, [7, 31, 2, 19, 1, 12]), (2048, 16, 4, 4096, [30] * 9), (8192, 16, 4, 4096, [5, 27, 14, 1])])
+@pytest.mark.parametrize("bias", [False, True])
+def test_wide_passes_with_split_products_equal_the_portions_alone(E, n_embd, n_head, n_head_kv, n_ff, lens, bias):
+    """Wide passes whose K is split: wq | wk | wv ends with the rope and the cache stores of every row's own sequence and position (up to 255 rows; 270 in a launch of its own), q rounded as the
+    small passes round it. Three rounds, so that positions differ and the stored cells are read back. Against the same portions alone, which small passes take."""
+    torch = E.torch
+    rng = np.random.default_rng(len(lens) + n_embd)
+    ws = []
+    for _ in range(2):
+        w = _filled_window(E, n_embd, n_head, n_head_kv, n_ff, 96, bias, flags=E.HAS_EMBD | E.HAS_HEAD)
+        w.finalize_pool(512, len(lens), len(lens) * 96)
+        ws.append((w, [w.seq_new() for _ in lens]))
+    (w, seqs), (w1, seqs1) = ws
+    for k in range(3):
+        part = [rng.integers(0, 320, 1 if k == 2 else n if k == 0 else max(1, n // 2) + 9).astype(np.int32) for n in lens]
+        lg, lg1 = torch.full((len(lens), 320), float("nan"), device="cuda"), torch.empty((len(lens), 320), device="cuda")
+        w.batch([(q, t, [len(t) - 1]) for q, t in zip(seqs, part)], logits=lg)
+        for i, t in enumerate(part):
+            w1.batch([(seqs1[i], t, [len(t) - 1])], logits=lg1[i:i + 1])
+        a, b = lg.double(), lg1.double()
+        err = ((a - b) ** 2).sum(-1) / (b ** 2).sum(-1)
+        assert (err < 1e-3).all(), (k, err.max().item())
+    w.close()
+    w1.close()
+
+
 @pytest.mark.parametrize("flash,n_head,n_embd,n_head_kv", [("1", 8, 512, 2), ("1", 4, 512, 2), ("0", 8, 512, 2), ("1", 8, 1024, 4), ("1", 16, 1024, 8)])
 def test_long_context_split_attention_path(E, monkeypatch, flash, n_head, n_embd, n_head_kv):
     """Beyond PM355_ATTN_SPLIT_MIN positions the engine switches from the one-workgroup-per-head attention kernel to the

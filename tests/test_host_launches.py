@@ -10,7 +10,7 @@ ROOT = os.path.dirname(HERE)
 LIB = os.path.join(ROOT, "prima_cpp_amd", "libprima_mi355.so")
 
 COMMON = r"""
-import ctypes as C, sys, threading
+import ctypes as C, re, sys, threading
 shim = C.CDLL(sys.argv[1])
 shim.shim_launches.restype, shim.shim_held.restype = C.c_long, C.c_size_t
 shim.shim_refuse.argtypes = [C.c_size_t]
@@ -18,7 +18,8 @@ def launches():
     out, name, r = (C.c_int * 4)(), C.create_string_buffer(500), []
     for i in range(shim.shim_launches()):
         shim.shim_launch(C.c_long(i), out, name, C.c_long(500))
-        r.append((out[0], name.value.decode().replace("(anonymous namespace)::", ""), tuple(out[1:])))
+        n = name.value.decode().replace("(anonymous namespace)::", "")
+        r.append((out[0], re.sub(r"^_Z.*?([a-z]\w*_kernel)ILi(\d+)EE.*", r"\1<\2>", n), tuple(out[1:])))     # (names with _Float16 in them stay mangled)
     return r
 """
 WINDOW = COMMON + r"""
@@ -38,6 +39,11 @@ def window(n_ctx=64, down=Q4_K, max_tokens=64, seqs=8, **hp):
     w.fill_tensor(E.T_OUT_NORM, -1, 0, 1, 1.0); w.fill_tensor(E.T_OUTPUT, -1, Q6_K, 1, 1.0); w.fill_tensor(E.T_TOK_EMBD, -1, Q4_K, 1, 1.0)
     w.finalize_pool(max_tokens, seqs, seqs * n_ctx)
     return w
+def decode(w, n):
+    x = torch.zeros(n, w.hp.n_embd)
+    shim.shim_forget()
+    assert w.lib.pm355_model_decode(w.h, None, x.data_ptr(), n, 0, x.data_ptr(), None, None, 1) == 0
+    return [name for _, name, _ in launches()]
 def batch(w, lens):
     qs = [w.seq_new() for _ in lens]
     shim.shim_forget()
@@ -125,5 +131,33 @@ w = window(max_tokens=33, seqs=24)
 assert wide(batch(w, [4] * 9)) == 0                     # two passes of 18: small ones
 w = window(max_tokens=512, seqs=24)
 assert wide(batch(w, [40, 50])) == 0                    # longer portions: 16-bit activations
+print("ok")
+""")
+
+
+def test_which_forms_add_up_the_slices_of_a_prompt(run):
+    """The shapes of test_gpu_engine.py's SLICED: norms with up to four slices and with more, rows beyond one and two columns of a wave, 128-row tiles up to 128 tokens; nothing rides along from 256
+    (rope) and 513 tokens (norm) on."""
+    run(WINDOW + r"""
+def forms(n_embd, n_head, n_head_kv, n_ff, tokens):
+    w = window(n_ctx=576, down=Q6_K, max_tokens=560, seqs=1, n_layer=2, n_embd=n_embd, n_head=n_head, n_head_kv=n_head_kv, n_ff=n_ff)
+    out = []
+    for n in tokens:
+        names = decode(w, n)
+        mid = any(re.search(r"gemm_pf_kernel<1., 1., ., true", x) for x in names)
+        out.append((mid, sorted(m.group(1) for x in names for m in [re.search(r"pf_reduce_((?:norm|rope)_kernel<.>)", x)] if m), any("rope_kv" in x for x in names)))
+    w.close()
+    return out
+N4, N8, R4, R8 = "norm_kernel<4>", "norm_kernel<8>", "rope_kernel<4>", "rope_kernel<8>"
+# (the second layer's ffn_down has no norm behind it)
+got = forms(4352, 32, 8, 14336, (72, 130, 512, 560))
+assert got[0] == (True, [N4, N4, N8, R4, R4], False), got[0]
+assert got[1][1].count(N4) + got[1][1].count(N8) == 3 and not got[1][2], got[1]
+assert got[2][2] and len(got[2][1]) == 3 and all("norm" in x for x in got[2][1]), got[2]
+assert got[3] == (False, [], True), got[3]
+got = forms(8192, 64, 8, 28672, (72, 130, 200))
+assert got[0][0] and got[1] == got[2] == (False, [N8, N8, N8, R8, R8], False), got
+got = forms(8192, 16, 4, 4096, (72,))
+assert got[0][0] and got[0][1].count(R8) == 2, got
 print("ok")
 """)
