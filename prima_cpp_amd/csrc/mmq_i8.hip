@@ -1,4 +1,4 @@
-// mmq_i8.hip — small-batch (9..32 tokens per pass, 64 per call; passes of fewer: mmq_rows.hip) quantized mat-mul on the INTEGER matrix cores
+// mmq_i8.hip — small-batch (up to 32 tokens per pass, 64 per call; where it is the faster one, pm_mmq_rows_takes, mmq_rows.hip) quantized mat-mul on the INTEGER matrix cores
 // (v_mfma_i32_32x32x32_i8 / v_mfma_i32_32x32x16_i8). Q4_K, Q5_K, Q6_K weights x Q8_K activations.
 //
 // What it replaces: for 2..64 activation rows the reference runs ggml_compute_forward_mul_mat's vec_dot loop once per (row, token)
@@ -17,7 +17,7 @@
 //   B operand = weights    : lane (r = lane % 32, g)            holds the same k of weight row r
 //   result                 : lane (r, g) holds, for ITS OWN row r, tokens 8 (v / 4) + 4 g + v % 4, v = 0..15
 // so the per-row sub-block scale / min / d of a K-quant are lane-local scalars when the i32 tile is scaled (one v_mad_i32_i24 per result;
-// the instantiation keeps 8 / 16 result registers for <= 16 / 32 tokens). An MFMA never crosses a scale group. The min / -32
+// the instantiation keeps 4 / 8 / 16 result registers for <= 8 / 16 / 32 tokens). An MFMA never crosses a scale group. The min / -32
 // terms are one more MFMA per super-block in F16 (v_mfma_f32_32x32x16_f16: 6-bit mins or int8 scales x 16-value activation sums <= 2032,
 // all exact in F16, f32 accumulation of integers < 2^24 exact).
 //
@@ -48,7 +48,6 @@ typedef int      i32x16 __attribute__((ext_vector_type(16)));
 typedef float    f32x16 __attribute__((ext_vector_type(16)));
 typedef _Float16 f16x8  __attribute__((ext_vector_type(8)));
 
-constexpr int ROWS_MAX = 8;             // passes of up to so many tokens: mmq_rows.hip
 constexpr int BLOCK = 512, NWAVE = 8;
 constexpr int PITCH = 144;            // LDS bytes per row of a 128-byte stream tile: 16 consecutive rows -> 16 distinct 16-byte bank slots
 constexpr int PITCH_H = 48;           // same for the 2 x 16-byte per-row header / scale tile
@@ -106,10 +105,11 @@ template <> struct Rows<true> {           // several matrices: a lane's rows may
 // the NEXT step's whole weight tile (ISA: vmcnt(14) where 31 loads were in flight), i.e. the prefetch overlapped half a step. Buffer loads
 // instead: unconditional instructions, the lanes without a token carry an out-of-range offset, return 0 and touch no memory.
 //
-// A 32 x 32 product has 32 token rows; up to 16 tokens would leave half of the operand's lanes empty. They carry OTHER sub-blocks instead: operand lane r = R q + t, R = 2 NV rows per
-// sub-block, holds token t's bytes of sub-block P i + q (P = 16 / NV sub-blocks per register). The product with the weights of sub-block P i + q is right in the rows R q .. R q + R - 1,
-// i.e. in the result registers NV q .. NV q + NV - 1, and nobody reads the others. One load brings what P loads of half-empty lanes did: 4 loads per super-block instead of 8 and as many
-// registers less (the vector memory path is paid per instruction).
+// A 32 x 32 product has 32 token rows; up to 8 (16) tokens would leave three quarters (half) of the operand's lanes empty. They carry OTHER sub-blocks instead: operand lane
+// r = R q + t, R = 2 NV rows per sub-block, holds token t's bytes of sub-block P i + q (P = 16 / NV sub-blocks per register). The product with the weights of sub-block P i + q is
+// right in the rows R q .. R q + R - 1, i.e. in the result registers NV q .. NV q + NV - 1, and nobody reads the others. One load brings what P loads of half-empty lanes did: 2 (4)
+// loads per super-block instead of 8 and as many registers less. At 8 tokens these loads were 10 of the 60 us of a 57344 x 8192 Q4_K launch (the vector memory path is paid per
+// instruction): 57.4 -> 51.6 us on weights out of memory.
 struct ActSrc {
     __amdgpu_buffer_rsrc_t rx, rb; uint32_t xo, bo;        // xo / bo: this lane's byte offset into the operand-ordered activations / the group-sum table (or out of range)
     // sub-block s of super-block sb: lane (t, g) gets the 16 bytes k = 32 s + 16 g .. + 15 of token t (one coalesced kilobyte per wave and 32 tokens)
@@ -413,7 +413,7 @@ template <> struct MT<PM_Q8_0> {
 // the work of workgroup w of G on the launch p (its own grid, or one part of a two-part launch)
 // EPI: the wq | wk | wv epilogue (MmqP::e_*) is compiled in - instantiations of their own: carried by every kernel as a run-time switch it cost the launches
 // that never use it 2-6 us per layer (Qwen2.5-72B, NEOX rope: 236 -> 242 us at 8 tokens)
-template <int TYPE, int NV, bool MJ, bool EPI = false>  // NV result registers per lane in use: 8 (<= 16 tokens), 16 (<= 32)
+template <int TYPE, int NV, bool MJ, bool EPI = false>  // NV result registers per lane in use: 4 (<= 8 tokens), 8 (<= 16), 16 (<= 32)
 __device__ __forceinline__ void mmq_i8_body(const MmqP & p, const int w, const int G, uint8_t * smem) {
     typedef MT<TYPE> M;
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;   // (a scalar: the K slice, the loop counters and the buffer loads' scalar offsets derive from it)
@@ -445,7 +445,7 @@ __device__ __forceinline__ void mmq_i8_body(const MmqP & p, const int w, const i
     xs.xo = act ? (uint32_t) (tq * 1024 + (32 * g + tt + p.t_off) * 16) : 0x80000000u;
     xs.bo = Q80 ? (uint32_t) (16 * lane) : act_b ? (uint32_t) ((lane + p.t_off) * 16) : 0x80000000u;   // (Q8_0: lane l carries 16 bytes of the step's [8 blocks][32 slots] activation scales)
     Rows<MJ> rw;
-    // (measured and rejected at 8 tokens, when this kernel still took them: TWO weight tiles in flight per wave - 57344 x 8192 Q4_K 53.0 -> 55.1 us, Q6_K 98.0 -> 102.4; two workgroups that
+    // (measured and rejected at 8 tokens: TWO weight tiles in flight per wave - 57344 x 8192 Q4_K 53.0 -> 55.1 us, Q6_K 98.0 -> 102.4; two workgroups that
     //  share a row group's K where 128 row groups leave half the chip idle - 4096 x 14336 Q6_K 24.7 -> 22.8 us, but Q4_K 14.3 -> 16.3: the exchange costs what the second half of the chip
     //  saves. What Q6_K launches lose is memory traffic: 1.36 x the weights' bytes, the scale and d lines of a row tail are fetched again for every step)
     typename M::B R;
@@ -748,11 +748,11 @@ int launch_q80(const void * W, const void * xq, const float * x_f32, float * Y, 
     const int grid = N / 32 >= cus ? cus : (N + 31) / 32;
     const int rows = (N + grid - 1) / grid, nrg = (rows + 31) / 32;
     const size_t lds = pm_mmq_i8_lds_bytes(PM_Q8_0, K);
-    const int tmax = pm_mmq_rows_takes(PM_Q8_0, N, T) || pm_mmq_rows_takes(PM_Q8_0, N, 32) ? 32 : 16;      // (this file's 32-token form spills 236 B: 502 vs 422 us per Qwen2.5-72B layer at 32 tokens - two passes of 16 it is)
+    const int tmax = pm_mmq_rows_takes(PM_Q8_0, N, K, T) || pm_mmq_rows_takes(PM_Q8_0, N, K, 32) ? 32 : 16;      // (this file's 32-token form spills 236 B: 502 vs 422 us per Qwen2.5-72B layer at 32 tokens - two passes of 16 it is)
     for (int t0 = 0; t0 < T; t0 += tmax) {
         const int tn = T - t0 < tmax ? T - t0 : tmax;
         uint8_t * tab = base + (t0 / 32) * (qtab + dtab);
-        if (pm_mmq_rows_takes(PM_Q8_0, N, tn)) {
+        if (pm_mmq_rows_takes(PM_Q8_0, N, K, tn)) {
             RowsP q = {};
             q.job[0] = {(const uint8_t *) W, Y + (size_t) t0 * N, bias, resid ? resid + (size_t) t0 * N : nullptr, N};
             q.njobs = 1; q.K = K; q.T = tn; q.t_off = t0 % 32; q.qT = tab; q.dT = (const float *) (tab + qtab);
@@ -770,7 +770,7 @@ int launch_q80(const void * W, const void * xq, const float * x_f32, float * Y, 
             pm_allow_big_lds((const void *) kern, 150 * 1024);
             hipLaunchKernelGGL(kern, dim3(grid), dim3(BLOCK), lds, st, p);
         };
-        go(mmq_i8_kernel<PM_Q8_0, 8>);
+        if (tn <= 8) go(mmq_i8_kernel<PM_Q8_0, 4>); else go(mmq_i8_kernel<PM_Q8_0, 8>);
     }
     return 0;
 }
@@ -835,11 +835,11 @@ int pm_launch_mmq_i8(int type, const void * W, const void * xq, const float * x_
     const int grid = N / 32 >= cus ? cus : (N + 31) / 32;
     const int rows = (N + grid - 1) / grid, nrg = (rows + 31) / 32;
     const size_t lds = pm_mmq_i8_lds_bytes(type, K);
-    const int tmax = type != PM_Q5_K || pm_mmq_rows_takes(type, N, T) || pm_mmq_rows_takes(type, N, 32) ? 32 : 16;                    // (Q5_K: 11 weight registers more per step - its 32-token form here spills 388 B / lane)
+    const int tmax = type != PM_Q5_K || pm_mmq_rows_takes(type, N, K, T) || pm_mmq_rows_takes(type, N, K, 32) ? 32 : 16;                    // (Q5_K: 11 weight registers more per step - its 32-token form here spills 388 B / lane)
     for (int t0 = 0, c = 0; t0 < T; t0 += tmax, ++c) {
         const int tn = T - t0 < tmax ? T - t0 : tmax;
         uint8_t * bsT = sc->p + (t0 / 32) * tab; float * dT = (float *) (bsT + (size_t) nsb * 1024);    // tables are per 32 tokens
-        if (pm_mmq_rows_takes(type, N, tn)) {
+        if (pm_mmq_rows_takes(type, N, K, tn)) {
             RowsP q = {};
             q.job[0] = {(const uint8_t *) W, Y + (size_t) t0 * N, bias, resid ? resid + (size_t) t0 * N : nullptr, N};
             q.njobs = 1; q.K = K; q.T = tn; q.t_off = t0 % 32; q.qT = sc->p + scr_q_off(K) + (size_t) (t0 / 32) * nsb * 8192; q.bsT = bsT; q.dT = dT;
@@ -857,10 +857,11 @@ int pm_launch_mmq_i8(int type, const void * W, const void * xq, const float * x_
             pm_allow_big_lds((const void *) kern, 150 * 1024);
             hipLaunchKernelGGL(kern, dim3(grid), dim3(BLOCK), lds, st, p);
         };
-        if (type == PM_Q4_K) { if (tn <= 16) go(mmq_i8_kernel<PM_Q4_K, 8>); else go(mmq_i8_kernel<PM_Q4_K, 16>); }
-        else if (type == PM_Q5_K) go(mmq_i8_kernel<PM_Q5_K, 8>);
+        if (type == PM_Q4_K) { if (tn <= 8) go(mmq_i8_kernel<PM_Q4_K, 4>); else if (tn <= 16) go(mmq_i8_kernel<PM_Q4_K, 8>); else go(mmq_i8_kernel<PM_Q4_K, 16>); }
+        else if (type == PM_Q5_K) { if (tn <= 8) go(mmq_i8_kernel<PM_Q5_K, 4>); else go(mmq_i8_kernel<PM_Q5_K, 8>); }
+        else if (tn <= 8)  go(mmq_i8_kernel<PM_Q6_K, 4>);
         else if (tn <= 16) go(mmq_i8_kernel<PM_Q6_K, 8>);
-        else go(mmq_i8_kernel<PM_Q6_K, 16>);
+        else               go(mmq_i8_kernel<PM_Q6_K, 16>);
     }
     return 0;
 }
@@ -925,7 +926,7 @@ int pm_launch_mmq_i8_multi(int type, int njobs, const void * const * W, const in
     const size_t tab = (size_t) nsb * (1024 + 128);
     for (int t0 = 0, c = 0; t0 < T; t0 += 32, ++c) {                 // passes of 32 tokens, each with its own tables
         const int tn = T - t0 < 32 ? T - t0 : 32;
-        if (tn <= ROWS_MAX) {
+        if (tn <= 8 && pm_mmq_rows_takes(type, total, K, tn, PM_ROWS_SEVERAL)) {
             RowsP q = {};
             int ty[3];
             q.njobs = njobs; q.K = K; q.T = tn; q.bsT = sc->p + c * tab; q.dT = (const float *) (q.bsT + (size_t) nsb * 1024); q.qT = sc->p + scr_q_off(K) + (size_t) c * nsb * 8192;
@@ -937,10 +938,12 @@ int pm_launch_mmq_i8_multi(int type, int njobs, const void * const * W, const in
         p.T = tn;
         p.bsT = sc->p + c * tab; p.dT = (const float *) (p.bsT + (size_t) nsb * 1024); p.qT = sc->p + scr_q_off(K) + (size_t) c * nsb * 8192;
         for (int j = 0; j < 3; ++j) { const int jj = j < njobs ? j : njobs - 1; p.yj[j] = Y[jj] + (size_t) t0 * N[jj]; }
-        if (p.e_on && type == PM_Q4_K) { if (tn <= 16) go(mmq_i8_kernel<PM_Q4_K, 8, true, true>); else go(mmq_i8_kernel<PM_Q4_K, 16, true, true>); }
-        else if (p.e_on)         { if (tn <= 16) go(mmq_i8_kernel<PM_Q6_K, 8, true, true>); else go(mmq_i8_kernel<PM_Q6_K, 16, true, true>); }
-        else if (type == PM_Q4_K) { if (tn <= 16) go(mmq_i8_kernel<PM_Q4_K, 8, true>); else go(mmq_i8_kernel<PM_Q4_K, 16, true>); }
-        else                 { if (tn <= 16) go(mmq_i8_kernel<PM_Q6_K, 8, true>); else go(mmq_i8_kernel<PM_Q6_K, 16, true>); }
+#define PM_I8_GO(T_, E_) { if (tn <= 8) go(mmq_i8_kernel<T_, 4, true, E_>); else if (tn <= 16) go(mmq_i8_kernel<T_, 8, true, E_>); else go(mmq_i8_kernel<T_, 16, true, E_>); }
+        if (p.e_on && type == PM_Q4_K) PM_I8_GO(PM_Q4_K, true)
+        else if (p.e_on)               PM_I8_GO(PM_Q6_K, true)
+        else if (type == PM_Q4_K)      PM_I8_GO(PM_Q4_K, false)
+        else                           PM_I8_GO(PM_Q6_K, false)
+#undef PM_I8_GO
     }
     return 0;
 }
@@ -964,10 +967,9 @@ int pm_launch_mmq_i8_dual(int ta, int na, const void * const * Wa, const int * N
     const Scr * sc = scratch(dev, st, K, reuse_prep != 0);
     if (!sc) return -3;
     if (!reuse_prep) launch_prep(sc, xq, K, T, st);
-    if (T <= ROWS_MAX) {
+    if (T <= 8 && na <= 2 && pm_mmq_rows_takes(ta, total + Nb, K, T, PM_ROWS_MIXED)) {
         RowsP q = {};
-        int ty[4];
-        if (na > 2) return -5;
+        int ty[3];
         q.njobs = na + 1; q.K = K; q.T = T; q.bsT = sc->p; q.dT = (const float *) (sc->p + (size_t) nsb * 1024); q.qT = sc->p + scr_q_off(K);
         for (int j = 0; j < na; ++j) { q.job[j] = {(const uint8_t *) Wa[j], Ya[j], ba ? ba[j] : nullptr, nullptr, Na[j]}; ty[j] = ta; }
         q.job[na] = {(const uint8_t *) Wb, Yb, bb, nullptr, Nb}; ty[na] = tb;
@@ -1016,10 +1018,10 @@ int pm_launch_mmq_i8_dual(int ta, int na, const void * const * Wa, const int * N
         hipLaunchKernelGGL(kern, dim3(ga + gb), dim3(BLOCK), lds, st, pp);
     };
     if (epi) {
-        if (tb == PM_Q6_K) { if (T <= 16) go(mmq_i8_dual_kernel<PM_Q4_K, PM_Q6_K, 8, true>); else go(mmq_i8_dual_kernel<PM_Q4_K, PM_Q6_K, 16, true>); }
-        else               { go(mmq_i8_dual_kernel<PM_Q4_K, PM_Q5_K, 8, true>); }
+        if (tb == PM_Q6_K) { if (T <= 8) go(mmq_i8_dual_kernel<PM_Q4_K, PM_Q6_K, 4, true>); else if (T <= 16) go(mmq_i8_dual_kernel<PM_Q4_K, PM_Q6_K, 8, true>); else go(mmq_i8_dual_kernel<PM_Q4_K, PM_Q6_K, 16, true>); }
+        else               { if (T <= 8) go(mmq_i8_dual_kernel<PM_Q4_K, PM_Q5_K, 4, true>); else go(mmq_i8_dual_kernel<PM_Q4_K, PM_Q5_K, 8, true>); }
     }
-    else if (tb == PM_Q6_K) { if (T <= 16) go(mmq_i8_dual_kernel<PM_Q4_K, PM_Q6_K, 8>); else go(mmq_i8_dual_kernel<PM_Q4_K, PM_Q6_K, 16>); }
-    else               { go(mmq_i8_dual_kernel<PM_Q4_K, PM_Q5_K, 8>); }
+    else if (tb == PM_Q6_K) { if (T <= 8) go(mmq_i8_dual_kernel<PM_Q4_K, PM_Q6_K, 4>); else if (T <= 16) go(mmq_i8_dual_kernel<PM_Q4_K, PM_Q6_K, 8>); else go(mmq_i8_dual_kernel<PM_Q4_K, PM_Q6_K, 16>); }
+    else               { if (T <= 8) go(mmq_i8_dual_kernel<PM_Q4_K, PM_Q5_K, 4>); else go(mmq_i8_dual_kernel<PM_Q4_K, PM_Q5_K, 8>); }
     return 0;
 }

@@ -1,4 +1,4 @@
-// mmq_rows.hip - quantized mat-mul for 2..8 tokens (some shapes and types: up to 32, pm_mmq_rows_takes): weights from memory straight into the operands of v_mfma_i32_16x16x64_i8 / 16x16x32_i8, no LDS on their way.
+// mmq_rows.hip - quantized mat-mul for 1..8 tokens, some shapes and types up to 32 (pm_mmq_rows_takes: the rest is mmq_i8.hip's): weights from memory straight into the operands of v_mfma_i32_16x16x64_i8 / 16x16x32_i8, no LDS on their way.
 //
 // The arithmetic is mmq_i8.hip's (activations in Q8_K / Q8_0 blocks, exact integer sums per super-block, one f32 multiply-add per super-block): what differs is where the bytes go. A workgroup
 // owns a slice of the rows of one matrix, its eight waves share K: a wave takes PAIRS of super-blocks, pair w, w + 8, ..., for all rows of the slice, 16 at a time. So
@@ -579,22 +579,49 @@ template <int TYPE> size_t lds_of(int NG, int R, bool AL, int K) {
     const int n = TYPE == PM_Q8_0 ? (K / 32 + 7) / 8 : K / 256;
     return (size_t) 2 * KW * R * NG * 512 + (size_t) 2 * 16 * R * Scales<TYPE>::PITCH + (AL ? ALds<TYPE>::bytes(n) : 0);
 }
+constexpr size_t LDS_MOST = 150 * 1024;
 size_t lds_of(int type, int NG, int R, bool AL, int K) {
     return type == PM_Q4_K ? lds_of<PM_Q4_K>(NG, R, AL, K) : type == PM_Q5_K ? lds_of<PM_Q5_K>(NG, R, AL, K) : type == PM_Q6_K ? lds_of<PM_Q6_K>(NG, R, AL, K) : lds_of<PM_Q8_0>(NG, R, AL, K);
 }
 
 }  // namespace
 
-// Several groups of eight tokens, us, mmq_i8.hip / here (4.5 of them the tables). One group of rows per workgroup (N up to 16 per CU): the activations of a K range are asked for once per workgroup
-// like the weights, and the chip is full (with 32-row groups it is half empty). 16 / 23 tokens: 4096 x 4096 Q4_K 11.4 / 10.3, 13.3 / 11.5; 4096 x 14336 Q4_K 18.8 / 18.0, 22.9 / 20.9, Q6_K 31.6 /
-// 25.1, 39.1 / 28.9. Q4_K and Q6_K stop at 24: with four groups of tokens their registers spill (4096 x 4096 Q4_K 13.4 / 13.8, 4096 x 14336 Q6_K 39.0 / 38.5). With two groups of rows they lose
-// (8192 x 8192 Q4_K at 16 / 23 tokens 16.4 / 17.8, 19.3 / 20.1).
-// Q5_K and Q8_0, which mmq_i8.hip takes 16 tokens at a time, read the weights once here: 32 tokens with one group of rows (1024 x 8192 Q5_K 28.5 / 16.2, Q8_0 28.0 / 20.0; 4096 x 14336 Q5_K 41.9 /
-// 28.2), 17..24 with two (8192 x 29568 Q8_0 117 / 76, 59136 x 8192 192 / 155; 57344 x 8192 Q5_K 153 / 107, 8192 x 8192 35.3 / 23.2); 32 there spill (Q8_0 121 / 95 and 34.5 / 32.7, Q5_K 34 / 270),
-// and up to 16 tokens mmq_i8.hip is as fast or faster (59136 x 8192 Q8_0 105 / 133, 57344 x 8192 Q5_K 79 / 96).
-bool pm_mmq_rows_takes(int type, int N, int T) {
-    const bool one_group = N <= 16 * pm_device_cus(), by16 = type == PM_Q5_K || type == PM_Q8_0;
-    return T <= 8 || (one_group ? T <= (by16 ? 32 : 24) : by16 && T > 16 && T <= 24);
+// Where this form is the faster one, by rows per CU (groups of 16) and K. Its workgroup takes all of K at once, eight pairs of super-blocks a step: with one row group the chip is full where
+// 32-row groups fill half of it, with more it pays for the steps' empty pairs (K = 2048: four of eight), for a round of sums over the waves per pass, and for a last pass of few rows (passes of 48
+// rows, of 64 where the activations fit LDS). Weights out of memory, time here / time of mmq_i8.hip:
+//   8 tokens, one matrix, N = 4096 / 8192 / 12288 / 16384 / 36864 / 128256: Q4_K K = 1024 0.96 1.15 1.23 1.37 1.37 1.51, 2048 0.91 1.07 1.16 1.25 1.14 1.22, 3072 0.84 0.99 1.00 1.11 0.97 0.92,
+//   4096 0.82 0.94 0.94 1.03 0.89 0.87, 5120 0.87 1.13 1.09 1.21 1.07 1.05, 8192 0.86 1.02 0.93 0.98 0.88, 14336 0.92 1.12 0.99 1.24 0.95; Q6_K 1024 0.96 1.24 1.40 1.65 1.60 1.65, 4096 0.74 0.95
+//   0.94 1.07 0.86 0.82, 5120 0.86 1.20 1.13 1.30 1.07, 8192 0.76 1.04 0.90 0.98 0.80, 14336 0.76 1.08 0.93 1.09 0.82; Q5_K 2048 0.89 1.07 1.19 1.36 1.29 1.32, 4096 0.75 1.01 1.03 1.07 1.00,
+//   8192 0.84 1.17 1.04 1.10 0.98; Q8_0 1024 1.00 1.19 1.20 1.27 1.17, 2048 0.92 1.05 1.06 1.09 0.97 0.89, 4096 0.92 1.07 1.04 1.02 0.95, 8192 0.89 1.09 0.97 0.98 0.98
+//   several matrices of one type (mmq_i8.hip looks their rows up one by one), N in all 6144 / 8192 / 16384 / 28672: Q4_K 2048 0.99 0.98 1.12 1.12, 3072 0.89 0.90 1.02 0.94, 4096 0.87 0.87 0.94
+//   0.88, 5120 1.01 1.02 1.13 1.04, 8192 0.96 0.96 0.94 0.88; Q6_K 4096 0.84 0.88 1.00 0.89; two types, 6144 / 10240 / 16384: 2048 0.95 1.11 1.16, 3072 0.84 0.98 1.00, 5120 0.99 1.06 1.14, 8192
+//   0.91 0.93 0.88
+//   12 / 20 tokens, one row group: Q4_K K = 1024 1.05 1.07, 2048 1.02 1.02, 3072 0.89 0.88, 8192 0.90 0.88; Q6_K 1024 1.05 1.06, 2048 0.98 0.96, 4096 0.79 0.75; Q5_K 1024 0.96 0.69, 4096 0.83 0.55
+//   (32 tokens 0.62); Q8_0 1024 1.09 0.76, 4096 1.01 0.67 (32: 0.71), 8192 0.98 0.64. Q4_K and Q6_K stop at 24 tokens: with four groups of them registers spill
+//   20 tokens, more rows (Q5_K and Q8_0, which mmq_i8.hip takes 16 tokens at a time): N = 8192 / 16384 / 49152 Q5_K 1024 0.84 1.02 1.31, 2048 0.84 1.04 1.07, 3072 0.71 0.84 0.79, 8192 0.73 0.78 0.74; Q8_0
+//   512 0.95 1.11 1.27, 1024 0.90 0.94 0.93, 4096 0.81 0.80 0.78. (32 tokens there spill)
+bool pm_mmq_rows_takes(int type, long N, int K, int T, int form) {
+    const int cus = pm_device_cus();
+    const long rows = (N + cus - 1) / cus, groups = (rows + 15) / 16;
+    const bool q5 = type == PM_Q5_K, q8 = type == PM_Q8_0;
+    if (T > 8) {
+        if (form != PM_ROWS_ONE || T > (q5 || q8 ? 32 : 24)) return false;
+        if (groups == 1) return q5 || (q8 && T > 16) || K >= (q8 ? 7168 : type == PM_Q6_K ? 2048 : 3072);
+        return (q5 || q8) && T > 16 && T <= 24 && (groups == 2 || K >= (q5 ? 3072 : 1024));
+    }
+    if (groups == 1) return !q8 || K >= 1024;
+    if (q5) return groups == 2 && K >= 3072 && K <= 4096;
+    const int pairs = (K + (q8 ? 255 : 511)) / (q8 ? 256 : 512), steps = (pairs + 7) / 8;
+    const bool lds = groups > 3 && lds_of(type, 1, 4, true, K) <= LDS_MOST;         // passes of 64 rows
+    // rows of the passes that are there, per cent
+    const long filled = groups <= 3 ? 100 : lds ? 100 * rows / (64 * ((rows + 63) / 64)) : 100 * rows / (48 * ((rows + 47) / 48));
+    if (q8) return filled >= (lds ? 70 : 80) && ((groups >= 3 && K >= 5120) || (groups >= 9 && K >= 1536));
+    if (pairs == 6) return groups <= (form == PM_ROWS_ONE && type == PM_Q6_K ? 2 : 3) || (form == PM_ROWS_ONE ? groups >= 9 : form == PM_ROWS_SEVERAL && groups >= 7);
+    if (form == PM_ROWS_MIXED) return pairs == 8 * steps || (pairs >= 7 * steps && K <= 9216) || (rows <= 24 && pairs >= 4);
+    // (at least 7 of 8 pairs; Q4_K whose activations do not fit LDS 9 of 10)
+    if ((!lds && filled < (type == PM_Q6_K ? 75 : 80)) || 10 * pairs < (type == PM_Q4_K && K > 9216 ? 72 : 70) * steps) return false;
+    if (form == PM_ROWS_ONE && groups == 2) return K <= 4096 || (type == PM_Q6_K && K > 16384);
+    return form != PM_ROWS_ONE || groups != 4 || K >= 8192;
 }
 
 int pm_launch_mmq_rows(RowsP p, const int * types, hipStream_t st) {
@@ -620,7 +647,7 @@ int pm_launch_mmq_rows(RowsP p, const int * types, hipStream_t st) {
     // again passes of 48
     const auto lds = [&](int g, int r, bool al) { return std::max(lds_of(ta, g, r, al, p.K), lds_of(tb, g, r, al, p.K)); };
     const int ng = (p.T + 7) / 8;
-    const bool al = ng == 1 && big > 3 && lds(1, 4, true) <= 150 * 1024, deep = p.K > 4096;
+    const bool al = ng == 1 && big > 3 && lds(1, 4, true) <= LDS_MOST, deep = p.K > 4096;
     auto go = [&](auto kern, size_t bytes) {
         pm_allow_big_lds((const void *) kern, bytes);
         hipLaunchKernelGGL(kern, dim3(at), dim3(NT), bytes, st, first[1], first[2], p);
@@ -633,7 +660,7 @@ int pm_launch_mmq_rows(RowsP p, const int * types, hipStream_t st) {
                                                  default: return PM_ROWS_GO(TA_, TB_, 1, 3, 1, false, E_); } }
 #define PM_ROWS_G(T_, G_, R_) go(mmq_rows_kernel<T_, T_, G_, R_, 1, false, false>, lds(G_, R_, false))
     if (ng > 1) {
-        if (n > 1 || !pm_mmq_rows_takes(ta, p.job[0].N, p.T)) return -5;
+        if (n > 1 || !pm_mmq_rows_takes(ta, p.job[0].N, p.K, p.T)) return -5;
         if (big > 1) return ta == PM_Q5_K ? PM_ROWS_G(PM_Q5_K, 3, 2) : PM_ROWS_G(PM_Q8_0, 3, 2);
         if (ta == PM_Q4_K) return ng == 2 ? PM_ROWS_G(PM_Q4_K, 2, 1) : PM_ROWS_G(PM_Q4_K, 3, 1);
         if (ta == PM_Q6_K) return ng == 2 ? PM_ROWS_G(PM_Q6_K, 2, 1) : PM_ROWS_G(PM_Q6_K, 3, 1);
@@ -649,7 +676,10 @@ int pm_launch_mmq_rows(RowsP p, const int * types, hipStream_t st) {
     }
     if (ta == PM_Q4_K && tb == PM_Q4_K) PM_ROWS_R(PM_Q4_K, PM_Q4_K, false)
     if (ta == PM_Q6_K && tb == PM_Q6_K) PM_ROWS_R(PM_Q6_K, PM_Q6_K, false)
-    if (ta == PM_Q5_K && tb == PM_Q5_K) PM_ROWS_R(PM_Q5_K, PM_Q5_K, false)
+    if (ta == PM_Q5_K && tb == PM_Q5_K) {                             // (up to two groups)
+        if (big > 2) return -5;
+        return big == 2 ? PM_ROWS_GO(PM_Q5_K, PM_Q5_K, 1, 2, 1, false, false) : deep ? PM_ROWS_GO(PM_Q5_K, PM_Q5_K, 1, 1, 2, false, false) : PM_ROWS_GO(PM_Q5_K, PM_Q5_K, 1, 1, 1, false, false);
+    }
     if (ta == PM_Q8_0 && tb == PM_Q8_0) PM_ROWS_R(PM_Q8_0, PM_Q8_0, false)
     if (ta == PM_Q4_K && tb == PM_Q6_K) PM_ROWS_R(PM_Q4_K, PM_Q6_K, false)
     if (ta == PM_Q4_K && tb == PM_Q5_K) PM_ROWS_R(PM_Q4_K, PM_Q5_K, false)

@@ -14,6 +14,8 @@ struct RowsP {
 template <int TYPE> __device__ __forceinline__ size_t pm_rows_stride(int nb) {
     return TYPE == PM_Q4_K ? (size_t) nb * 144 : TYPE == PM_Q5_K ? (size_t) nb * 176 : TYPE == PM_Q6_K ? pm_q6k_row_stride((size_t) nb) : (size_t) nb * 32 + (((size_t) nb * 2 + 15) & ~(size_t) 15);
 }
-// one or several matrices of one K (types[0]; only the last may be of another type) over 1..8 tokens, one matrix of N rows over the T that pm_mmq_rows_takes; -5: not served
-bool pm_mmq_rows_takes(int type, int N, int T);                     // one of the passes of up to 32 tokens
+// one or several matrices of one K (types[0]; only the last may be of another type) over 1..8 tokens, one matrix over more; -5: not served
+enum { PM_ROWS_ONE, PM_ROWS_SEVERAL, PM_ROWS_MIXED };               // one matrix; several of one type; two types
+// whether a pass over T tokens of N rows in all is one for it (else mmq_i8.hip's kernels); type: of the first matrix
+bool pm_mmq_rows_takes(int type, long N, int K, int T, int form = PM_ROWS_ONE);
 int pm_launch_mmq_rows(RowsP p, const int * types, hipStream_t st);

@@ -1518,7 +1518,9 @@ def test_small_batch_rows_kernel_at_its_edges(P, oracle, t):
     for K, N, T in ((512, 1, 8), (512, 15, 1), (768, 16, 2), (2048, 17, 3), (4096, 33, 4), (4096 + tail, 100, 5), (4352, 4096, 7), (4608, 4097, 8), (8192 + tail, 8192 + 31, 6), (1024, 12300, 8), (768, 28700, 3),
                     (8192, 12290, 2), (12288, 16390, 8),
                     (512, 16, 17), (768, 4096, 16), (4096 + tail, 33, 9), (4608, 100, 24), (14336, 4095, 23),      # (up to 24 tokens where a workgroup has one group of rows)
-                    (512, 40, 25), (4096 + tail, 4096, 32), (768, 17, 61), (4352, 8191, 17), (512, 4097, 24), (8192 + tail, 8230, 23)):     # (Q5_K, Q8_0: up to 32, and 17..24 with two and more)
+                    (512, 40, 25), (4096 + tail, 4096, 32), (768, 17, 61), (4352, 8191, 17), (512, 4097, 24), (8192 + tail, 8230, 23),      # (Q5_K, Q8_0: up to 32, and 17..24 with two and more)
+                    (4096, 4999, 7), (4096, 10243, 8), (8192 + tail, 10243, 3), (8192, 20491, 5), (12288, 20487, 8), (3072, 9001, 2)):      # (two and three groups, 64-row and 48-row passes of the
+                                                                                                                                            # types that have them: test_host_launches.py)
         b = rand_blocks(t, N, K, rng)
         x = rng.normal(0, 1, (T, K)).astype(np.float32)
         bias, resid = rng.normal(0, 1, N).astype(np.float32), rng.normal(0, 1, (T, N)).astype(np.float32)
@@ -1533,8 +1535,8 @@ def test_small_batch_rows_kernel_at_its_edges(P, oracle, t):
         xq = P.quantize_act(_dev(P, x), P.vec_dot_act_type(t))
         y2 = P.mul_mat_small(w, xq=xq, n_tokens=T, bias=_dev(P, bias), resid=_dev(P, resid)).cpu().numpy()
         assert np.array_equal(y2, (y + bias[None]) + resid), (K, N, T)
-        # a token's sums do not depend on the tokens beside it (but for Q4_K and Q6_K of more tokens, which mmq_i8.hip takes)
-        if T <= 24 and N <= 4096 or T <= 8 or t in (Q5_K, Q8_0):
+        # a token's sums do not depend on the tokens beside it, where those do not turn the pass over to the other kernel (pm_mmq_rows_takes)
+        if T <= 8 or N <= 4096 and (t == Q5_K or t == Q8_0 and T > 16 and K >= 1024 or t in (Q4_K, Q6_K) and T <= 24 and K >= 3072):
             one = P.mul_mat_small(w, x=_dev(P, x[T - 1:])).cpu().numpy()
             assert np.array_equal(one[0], y[T - 1]), (K, N, T)
 
