@@ -51,9 +51,7 @@ __device__ __forceinline__ void attn_short(const float * q_head, const uint16_t 
     uint16_t * const pw = (uint16_t *) (part + NKEY) + NKEY * wave;
     char * const st = smem + 12 * NKEY + 4 * DH * 4 + S::STAGE * wave;
     const int kd = lane % LPK, ks = lane / LPK, c = lane % LV, ve = lane / LV;
-    const float * const qu = uniform_const_ptr(q_head);        // (every lane in the same quarter: q through the scalar cache)
-    f32x4 q4;
-    if constexpr (KPL < 4) q4 = *(const PM_G f32x4 *) (q_head + 4 * (lane % DPW));
+    const f32x4 q4 = *(const PM_G f32x4 *) (q_head + 4 * (lane % DPW));
     u32x4 kreg[NI], vreg[NV];
 #pragma unroll
     for (int i = 0; i < NI; ++i) kreg[i] = *(const PM_G u32x4 *) (kc + (long) max(min(KPI * (4 * i + wave) + ks, n_kv - 1), 0) * Hkv * DH + (long) hk * DH + 8 * kd);
@@ -66,7 +64,7 @@ __device__ __forceinline__ void attn_short(const float * q_head, const uint16_t 
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
         __builtin_amdgcn_wave_barrier();
     };
-    if constexpr (KPL < 4) if (lane < DPW) *(f32x4 *) (qs + 4 * lane) = q4;
+    if (lane < DPW) *(f32x4 *) (qs + 4 * lane) = q4;
 #pragma unroll
     for (int i = 0; i < NI; ++i) *(u32x4 *) (st + (KPI * i + ks) * S::K_PITCH + 16 * kd) = kreg[i];
     staged();
@@ -82,11 +80,7 @@ __device__ __forceinline__ void attn_short(const float * q_head, const uint16_t 
         for (int u = 0; u < KPL; ++u) {
             const int d = DPW * (u0 + u) + 8 * j;
             const u32x4 w = *(const u32x4 *) (st + l * S::K_PITCH + 2 * d);
-            f32x4 q[2];
-            if constexpr (KPL < 4) { q[0] = *(const f32x4 *) (qs + d); q[1] = *(const f32x4 *) (qs + d + 4); }
-            else
-#pragma unroll
-                for (int t = 0; t < 8; ++t) q[t >> 2][t & 3] = qu[DPW * u + 8 * j + t];
+            const f32x4 q[2] = {*(const f32x4 *) (qs + d), *(const f32x4 *) (qs + d + 4)};
 #pragma unroll
             for (int t = 0; t < 4; ++t) {
                 acc[u] = fmaf(h2f((uint16_t) (w[t] & 0xFFFF)), q[t >> 1][2 * (t & 1)], acc[u]);
