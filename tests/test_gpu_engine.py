@@ -213,14 +213,14 @@ def test_prompt_with_norms_behind_split_products(E, oracle, T, n_embd):
     w.close()
 
 
-def _filled_window(E, n_embd, n_head, n_head_kv, n_ff, n_ctx, bias, flags=0, down=Q6_K):
-    """two layers of random weights made on the device (n_vocab 320 where the window has its ends)"""
+def _filled_window(E, n_embd, n_head, n_head_kv, n_ff, n_ctx, bias, flags=0):
+    """two layers of random weights made on the device (n_vocab 320 where the window has its ends); ffn_down is Q6_K, with biases wv too (a launch of two types, tiles of 64 tokens in a wide pass)"""
     w = E.Window(dict(arch=0, n_layer=2, n_embd=n_embd, n_head=n_head, n_head_kv=n_head_kv, head_dim=128, n_ff=n_ff, n_vocab=320, rms_eps=1e-5, rope_freq_base=10000.0), flags=flags, n_ctx=n_ctx)
     for il in range(2):
         for i, kind in enumerate((E.T_ATTN_NORM, E.T_FFN_NORM)):
             w.fill_tensor(kind, il, E.F32, 100 * il + 1 + i, 0.0)
         for i, kind in enumerate((E.T_WQ, E.T_WK, E.T_WV, E.T_WO, E.T_FFN_GATE, E.T_FFN_UP, E.T_FFN_DOWN)):
-            w.fill_tensor(kind, il, down if kind == E.T_FFN_DOWN else Q4_K, 100 * il + 10 + i, 2.0 / np.sqrt(n_ff if kind == E.T_FFN_DOWN else n_embd))
+            w.fill_tensor(kind, il, Q6_K if kind == E.T_FFN_DOWN or bias and kind == E.T_WV else Q4_K, 100 * il + 10 + i, 2.0 / np.sqrt(n_ff if kind == E.T_FFN_DOWN else n_embd))
         for i, kind in enumerate((E.T_BQ, E.T_BK, E.T_BV) if bias else ()):
             w.fill_tensor(kind, il, E.F32, 100 * il + 20 + i, 0.5)
     if flags:
@@ -263,7 +263,7 @@ def test_prompts_with_slices_added_up_in_the_norm_and_the_rope(E, n_embd, n_head
     w.close()
 
 
-@pytest.mark.parametrize("n_embd,n_head,n_head_kv,n_ff,lens", [(2048, 16, 4, 4096, [7, 31, 2, 19, 1, 12]), (2048, 16, 4, 4096, [30] * 9), (8192, 16, 4, 4096, [5, 27, 14, 1])])
+@pytest.mark.parametrize("n_embd,n_head,n_head_kv,n_ff,lens", [(2048, 16, 4, 4096, [7, 31, 2, 19, 1, 12]), (2048, 16, 4, 4096, [30] * 9), (2048, 16, 4, 4096, [30, 29] * 3 + [23]), (8192, 16, 4, 4096, [5, 27, 14, 1])])
 @pytest.mark.parametrize("bias", [False, True])
 def test_wide_passes_with_split_products_equal_the_portions_alone(E, n_embd, n_head, n_head_kv, n_ff, lens, bias):
     """Wide passes whose K is split: wq | wk | wv ends with the rope and the cache stores of every row's own sequence and position (up to 255 rows; 270 in a launch of its own), q rounded as the
