@@ -1,5 +1,5 @@
-// mmq_i8.hip — small-batch (up to 32 tokens per pass, 64 per call; where it is the faster one, pm_mmq_rows_takes, mmq_rows.hip) quantized mat-mul on the INTEGER matrix cores
-// (v_mfma_i32_32x32x32_i8 / v_mfma_i32_32x32x16_i8). Q4_K, Q5_K, Q6_K weights x Q8_K activations.
+// mmq_i8.hip - small-batch (up to 32 tokens per pass, 64 per call) quantized mat-mul on the INTEGER matrix cores: what is launched for a call, the activations' tables, and the kernel for
+// one matrix of Q5_K or Q8_0 over up to 16 tokens. Beside it: mmq_rows.hip (1..8 tokens and some shapes beyond, pm_mmq_rows_takes) and mmq_mid.hip (the rest).
 //
 // What it replaces: for 2..64 activation rows the reference runs ggml_compute_forward_mul_mat's vec_dot loop once per (row, token)
 // (ggml/src/ggml.c:12377 -> ggml_vec_dot_q4_K_q8_K / ggml_vec_dot_q5_K_q8_K / ggml_vec_dot_q6_K_q8_K, ggml-quants.c:7713 / :8281 / :8918), its
@@ -7,39 +7,36 @@
 // exact int32 sums  sum_s scale_s * (q_w . q_a)  and  sum_s min_s * bsum_s  per 256-weight super-block, then ONE f32 multiply-add per
 // super-block with d_w * d_a - only the order in which the super-block terms are added in f32 differs (K split over waves).
 //
-// Why a third mat-mul kernel: between the mat-vec (1 token: weight-stream bound) and the F16 MFMA GEMM (256-token tiles: a 16-token
-// batch pays for 256) sits the regime of speculative decoding, parallel sequences and short prompts. The multi-column mat-vec
+// Why a third mat-mul kernel: between the mat-vec (1 token: weight-stream bound) and the F16 MFMA GEMM (a 16-token
+// batch pays for its whole tile) sits the regime of speculative decoding, parallel sequences and short prompts. The multi-column mat-vec
 // (mmvq_cols.hip) re-reads its activations from LDS for every decoded weight and costs ~10 us per extra column on the ffn_gate shape
-// (profiles/r02_small_batch_probe.txt); this kernel streams the weights ONCE per 32 tokens and does the products on the matrix cores.
+// (profiles/r02_small_batch_probe.txt); these kernels stream the weights ONCE per 32 tokens and do the products on the matrix cores.
 //
-// Mapping (one MFMA = 32 tokens x 32 weight rows x 32 k for Q4_K / Q5_K = one 32-weight sub-block; x 16 k for Q6_K = one 16-weight group):
-//   A operand = activations: lane (t = lane % 32, g = lane / 32) holds 16 (8) consecutive int8 of token t (up to 16 tokens: several sub-blocks share a register, ActSrc)
+// The kernel here (mmq_mid.hip for 17..32 tokens, 7-17 % faster than it would be for up to 16: Q5_K 57344 x 8192 at 8 tokens 69 us / 77 with mmq_mid.hip's, Q8_0 28672 x 2048 15.6 / 18.4).
+// Mapping (one MFMA = 32 tokens x 32 weight rows x 32 k = one 32-weight sub-block or block):
+//   A operand = activations: lane (t = lane % 32, g = lane / 32) holds 16 consecutive int8 of token t (several sub-blocks share a register, ActSrc)
 //   B operand = weights    : lane (r = lane % 32, g)            holds the same k of weight row r
 //   result                 : lane (r, g) holds, for ITS OWN row r, tokens 8 (v / 4) + 4 g + v % 4, v = 0..15
 // so the per-row sub-block scale / min / d of a K-quant are lane-local scalars when the i32 tile is scaled (one v_mad_i32_i24 per result;
-// the instantiation keeps 4 / 8 / 16 result registers for <= 8 / 16 / 32 tokens). An MFMA never crosses a scale group. The min / -32
-// terms are one more MFMA per super-block in F16 (v_mfma_f32_32x32x16_f16: 6-bit mins or int8 scales x 16-value activation sums <= 2032,
+// the instantiation keeps 4 / 8 result registers for <= 8 / 16 tokens). An MFMA never crosses a scale group. The min
+// terms are one more MFMA per super-block in F16 (v_mfma_f32_32x32x16_f16: 6-bit mins x 16-value activation sums <= 2032,
 // all exact in F16, f32 accumulation of integers < 2^24 exact).
 //
-// Data movement: weights keep the mat-vec's HBM layout (repack.hip; Q5_K native). A wave owns 32 rows x 512 k per step: it loads them
-// with FULL 128-byte lines per row and stream (8 lanes per line, non-temporal; the per-row headers / scales cached), parks them in its
+// Data movement: weights keep the mat-vec's HBM layout (repack.hip; Q5_K native). A wave owns 32 rows x 512 k (Q8_0: 256) per step: it loads them
+// with FULL 128-byte lines per row and stream (8 lanes per line, non-temporal; the per-row scales cached), parks them in its
 // private LDS tile and reads them back in MFMA operand order - no barrier, a wave's LDS accesses execute in order. The next step's loads
 // are in flight while the current one is computed (VMEM returns in order: the activation loads a step waits for are always issued BEFORE
 // the weight prefetch that overlaps it; scheduling barriers keep the compiler from sinking them). Activations come from L2 as ONE coalesced
 // kilobyte per 32-value sub-block out of a table in A-operand order; two more small tables hold the activation scales (transposed, -> LDS) and the
 // F16 group sums in A-operand order - all three written by the Q8_K quantizers as a second output (pm_q8k_tables) or by a prologue launch.
-// [Round 4: the operand-ordered table replaced per-token loads (one cache line per token and instruction, 16 B of it used: at 8 tokens the
-//  activation loads cost 11 of the 67 us of an ffn_down launch, at 32 tokens more); Q6_K's 16-k products take their halves from the 16-byte
-//  loads through v_permlane32_swap. The loads are buffer loads whose token slots >= T carry an out-of-range offset - unconditional instructions
-//  (a branch around them made the compiler's vmcnt bookkeeping wait for the NEXT weight tile before THIS step's products).]
 // Work split: workgroup = 8 waves, a balanced slice of rows = up to 8 groups of 32; K is split over the waves that share a row group -
-// interleaved pair by pair, so that those waves read adjacent 128-byte pieces of a row at the same time (ffn_down Q6_K: 76 -> 70 us) - and
-// their f32 partial tiles are added in a fixed order through LDS (bitwise reproducible). Multi-job form (MJ): up to 3 matrices of one
-// type and K that share the activations form one virtual row space (wq | wk | wv, ffn_gate | ffn_up): one launch, one fill / drain.
+// interleaved pair by pair, so that those waves read adjacent 128-byte pieces of a row at the same time (ffn_down: 76 -> 70 us) - and
+// their f32 partial tiles are added in a fixed order through LDS (bitwise reproducible).
 // Measurements and what did not help: profiles/r02_small_batch_probe.txt, profiles/r04_small_batch.txt, profiles/r06_small_batch.txt.
 #include "pm355_device.h"
 #include "pm355_kernels.h"
 #include "pm355_mmq_rows.h"
+#include <algorithm>
 #include <mutex>
 
 namespace {
@@ -55,48 +52,27 @@ constexpr int PITCH_H = 48;           // same for the 2 x 16-byte per-row header
 struct MmqP {
     const uint8_t * W; long row_stride; int N, K, T, rgb_log2;     // 1 << rgb_log2 row groups per batch (1, 2, 4, 8)
     int t_off;                                                     // first table slot of this pass (16-token passes of a 32-slot table)
-    const uint8_t * xq; long xq_stride;                            // row-SoA Q8_K activations [T]
     const uint8_t * bsT; const float * dT;                         // prologue tables: [nsb][64 lanes][8 f16], [nsb][32]
     const uint8_t * qT;                                            // the activations in A-operand order: [nsb][8 sub-blocks][64 lanes][16 B]
-    float * y; long y_stride; const float * bias; const float * resid;
-    // multi-job launches (MJ kernels): up to 3 matrices of one type and K that share the activations (wq | wk | wv, ffn_gate | ffn_up) form
-    // ONE virtual row space [0, N): job j owns rows [start[j], start[j] + nj[j]); y / bias per job, output token stride nj[j]
-    const uint8_t * Wj[3]; float * yj[3]; const float * bj[3]; int start[3], nj[3], njobs;
-    // wq | wk | wv epilogue (e_on; round 6): RoPE (NORM pairing: rows 2 i, 2 i + 1 of a head) with the per-token cos / sin tables of pm_launch_rope_table, q ->
-    // F16-rounded f32 into its y, k -> the F16 K-cache row of cell pos + t, v -> the transposed F16 V cache - what rope_kv_store_kernel (layer_ops.hip) does in a
-    // launch of its own, the same expressions (ggml_compute_forward_rope_f32 ggml.c:14224-14237; llm_build_kv_store src/llama.cpp:9688-9716).
-    // e_role[j]: 1 q, 2 k, 3 v (single-job launches: e_role[0]). Workgroup row slices start on even rows then.
-    int e_on, e_role[3]; const float * e_tab; const int32_t * e_pos, * e_seq; long e_seq_stride; uint16_t * e_kc, * e_vc; int e_dh, e_nctx, e_nrot, e_kvdim, e_rows;   // e_rows: e_pos[t], e_seq[t] per token
+    float * y; const float * bias, * resid;                        // [T][N]
 };
 
-__device__ __forceinline__ long pk(uint32_t a, uint32_t b) { return (long) (((uint64_t) b << 32) | a); }
 __device__ __forceinline__ u32x4 ld_c16(const void * p) { return *(const PM_G u32x4 *) p; }
-__device__ __forceinline__ u32x2 ld_c8(const void * p)  { return *(const PM_G u32x2 *) p; }
-__device__ __forceinline__ i32x16 mfma_i8(long a, long b, i32x16 c) { return __builtin_amdgcn_mfma_i32_32x32x16_i8(a, b, c, 0, 0, 0); }
 typedef int i32x4 __attribute__((ext_vector_type(4)));
 // gfx950's 2 x K form: lane (i, g) holds 16 consecutive int8 (k = 16 g .. 16 g + 15)
 __device__ __forceinline__ i32x16 mfma_i8x32(u32x4 a, u32x4 b, i32x16 c) {
     return __builtin_amdgcn_mfma_i32_32x32x32_i8(__builtin_bit_cast(i32x4, a), __builtin_bit_cast(i32x4, b), c, 0, 0, 0);
 }
 
-// where the loader lanes of a wave point: lane (rr = lane / 8, c = lane % 8) fetches 16-byte chunk c of rows rr, rr + 8, rr + 16, rr + 24
-template <bool MJ> struct Rows;
+// where the loader lanes of a wave point: lane (rr = lane / 8, c = lane % 8) fetches 16-byte chunk c of rows rr, rr + 8, rr + 16, rr + 24: wave-uniform base + 32-bit lane offsets
 // lm: all ones, or 0 for a look-ahead request past the wave's last step (the step code has no branches - the compiler's vmcnt bookkeeping stays exact - so
-// the request is issued anyway): every lane then asks for the same few addresses at the start of a row instead of re-loading the last tile (round 6: that
+// the request is issued anyway): every lane then asks for the same few addresses at the start of a row instead of re-loading the last tile (that
 // re-load was a third of wo's L2 -> CU traffic - two real tiles per wave and one for nothing)
-template <> struct Rows<false> {          // one matrix: wave-uniform base + 32-bit lane offsets
-    const uint8_t * base; uint32_t stride, off_d, lm; int lim /*last valid row of the group, relative*/, rr, rh;
+struct Rows {
+    const uint8_t * base; uint32_t stride, lm; int lim /*last valid row of the group, relative*/, rr, rh;
     __device__ __forceinline__ const uint8_t * at(int n, uint32_t x) const { return base + (((uint32_t) min(rr + 8 * n, lim) * stride + x) & lm); }
     __device__ __forceinline__ const uint8_t * at_h(uint32_t x) const { return base + (((uint32_t) min(rh, lim) * stride + x) & lm); }
-    __device__ __forceinline__ const uint8_t * at_d(uint32_t x) const { return base + ((off_d + x) & lm); }
     __device__ __forceinline__ const uint8_t * at_row(int row, uint32_t x) const { return base + (((uint32_t) min(row, lim) * stride + x) & lm); }   // any row of the group
-};
-template <> struct Rows<true> {           // several matrices: a lane's rows may sit in different allocations -> 64-bit row pointers per lane
-    const uint8_t * rp[4], * rph, * rpd; uint32_t lm;
-    __device__ __forceinline__ const uint8_t * at(int n, uint32_t x) const { return rp[n] + (x & lm); }
-    __device__ __forceinline__ const uint8_t * at_h(uint32_t x) const { return rph + (x & lm); }
-    __device__ __forceinline__ const uint8_t * at_d(uint32_t x) const { return rpd + (x & lm); }
-    __device__ __forceinline__ const uint8_t * at_row(int, uint32_t) const { return nullptr; }     // (native-layout types are single-job only)
 };
 
 // Where a lane's activation operand comes from. Token slots >= T must not cost memory traffic (the texture path is paid per ACTIVE lane,
@@ -122,77 +98,6 @@ struct ActSrc {
 
 template <int TYPE> struct MT;
 
-// ---------------------------------------------------------------- Q4_K: row = qa[U][16] | qb[U][16] | hdr[nb][16] ------------
-template <> struct MT<PM_Q4_K> {
-    static constexpr int QA = 0, QB = 32 * PITCH, HD = 64 * PITCH, WAVE_LDS = 64 * PITCH + 32 * PITCH_H;
-    struct B { u32x4 qa[4], qb[4], h; };
-    template <int NV> struct A { u32x4 q[NV / 2]; f16x8 bs; };
-    // part n of a step's tile (4 parts: rows rr + 8 n of both nibble streams; part 0 also the headers)
-    template <class RW>
-    static __device__ __forceinline__ void issue_b_part(B & b, const RW & rw, int nb, int pr, int lane, int n) {
-        const uint32_t u = (uint32_t) min(8 * pr + (lane & 7), 4 * nb - 1), sb = (uint32_t) min(2 * pr + (lane & 1), nb - 1);
-        b.qa[n] = ld_nt16(rw.at(n, u * 16u));
-        b.qb[n] = ld_nt16(rw.at(n, (uint32_t) nb * 64u + u * 16u));
-        if (n == 0) b.h = ld_c16(rw.at_h((uint32_t) nb * 128u + sb * 16u));   // cached: 4 steps share the line (as nt loads they re-fetched it from HBM: +29 % traffic)
-    }
-    static __device__ __forceinline__ void stash(const B & b, uint8_t * L, int lane) {
-        const int rr = lane >> 3, c = lane & 7;
-#pragma unroll
-        for (int n = 0; n < 4; ++n) {
-            *(u32x4 *) (L + QA + (rr + 8 * n) * PITCH + c * 16) = b.qa[n];
-            *(u32x4 *) (L + QB + (rr + 8 * n) * PITCH + c * 16) = b.qb[n];
-        }
-        *(u32x4 *) (L + HD + (lane >> 1) * PITCH_H + (lane & 1) * 16) = b.h;
-    }
-    // sub-block s (32 weights) = the 16 bytes at 32 s + 16 g of the super-block
-    template <int NV>
-    static __device__ __forceinline__ void issue_a(A<NV> & a, const ActSrc & x, int sb) {
-#pragma unroll
-        for (int i = 0; i < NV / 2; ++i) a.q[i] = x.ld_sub(sb, i * (16 / NV));
-        a.bs = x.ld_bs(sb);
-    }
-    template <int NV, class F>
-    static __device__ __forceinline__ void compute(const A<NV> & a, const uint8_t * L, int sbi, int r, int g, const float * yd_lds, int /*t_off*/, f32x16 & out, F && between) {
-        const u32x4 hd = *(const u32x4 *) (L + HD + r * PITCH_H + sbi * 16);
-        const i32x16 zero = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
-        i32x16 isum = zero;
-        // the 8 six-bit scales / mins of the super-block, four per dword (get_scale_min_k4, ggml-quants.c:1898-1906, on whole dwords)
-        const uint32_t sc4[2] = {hd[1] & 0x3f3f3f3fu, (hd[3] & 0x0f0f0f0fu) | ((hd[1] >> 2) & 0x30303030u)};
-        const uint32_t mn4[2] = {hd[2] & 0x3f3f3f3fu, ((hd[3] >> 4) & 0x0f0f0f0fu) | ((hd[2] >> 2) & 0x30303030u)};
-        f16x8 bm;
-#pragma unroll
-        for (int sb = 0; sb < 8; ++sb) bm[sb] = (_Float16) (float) ((mn4[sb >> 2] >> (8 * (sb & 3))) & 0xFFu);
-        // (round 6, measured and rejected for 17..32 tokens, where the 16 v_mad_i32_i24 per sub-block are what the wave does: the scale INSIDE the weight operand -
-        //  sc = 8 hi + lo, q * lo and q * hi are bytes <= 105, four v_pk_mul_lo_u16 per operand, two MFMA chains that accumulate across the sub-blocks,
-        //  sum = lo-chain + 8 * hi-chain: the same integers, 8 instead of 16 vector instructions and 2 instead of 1 MFMA per sub-block. 52-100 B of spills,
-        //  ffn_gate 43.6 -> 49.8 us, 202.5 -> 229.8 us per 70B layer at 32 tokens: profiles/r06_small_batch.txt)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            between(j);
-            const u32x4 w = *(const u32x4 *) (L + (g ? QB : QA) + r * PITCH + (4 * sbi + j) * 16);
-            const int sc0 = (int) ((sc4[(2 * j) >> 2] >> (8 * ((2 * j) & 3))) & 0xFFu), sc1 = (int) ((sc4[(2 * j + 1) >> 2] >> (8 * ((2 * j + 1) & 3))) & 0xFFu);
-            i32x16 acc = mfma_i8x32(a.q[2 * j / (16 / NV)], w & 0x0F0F0F0Fu, zero);                    // one 32-k MFMA = one 32-weight sub-block
-#pragma unroll
-            for (int v = 0; v < NV; ++v) { isum[v] = __mul24(sc0, acc[NV * (2 * j % (16 / NV)) + v]) + isum[v]; asm volatile("" : "+v"(isum[v])); }   // (keeps it ONE v_mad_i32_i24:
-            acc = mfma_i8x32(a.q[(2 * j + 1) / (16 / NV)], (w >> 4) & 0x0F0F0F0Fu, zero);                //  the re-associated mul, mul, add3 form is 1.5 instructions per term)
-#pragma unroll
-            for (int v = 0; v < NV; ++v) { isum[v] = __mul24(sc1, acc[NV * ((2 * j + 1) % (16 / NV)) + v]) + isum[v]; asm volatile("" : "+v"(isum[v])); }
-        }
-        const f32x16 fz = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
-        const f32x16 ms = __builtin_amdgcn_mfma_f32_32x32x16_f16(a.bs, bm, fz, 0, 0, 0);   // sum_s min_s * (bsum[2s] + bsum[2s+1]), exact
-        const float d = h2f((uint16_t) (hd[0] & 0xFFFF)), dmin = h2f((uint16_t) (hd[0] >> 16));
-#pragma unroll
-        for (int q = 0; q < NV / 4; ++q) {
-            const f32x4 yd = *(const f32x4 *) (yd_lds + 8 * q + 4 * g);
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const int v = 4 * q + i;
-                out[v] = fmaf(yd[i] * d, (float) isum[v], fmaf(-(yd[i] * dmin), ms[v], out[v]));
-            }
-        }
-    }
-};
-
 // ---------------------------------------------------------------- Q5_K: native 176-byte blocks (d, dmin | scales[12] | qh[32] | qs[128]) ------
 // A step's 2 super-blocks are 352 contiguous bytes per row = 22 chunks of 16: lane l fetches chunks l, l + 64, ... (11 loads) of the 32 x 22
 // chunk tile; LDS row pitch 368 B (23 x 16: 16 consecutive rows -> 16 distinct bank slots).
@@ -200,8 +105,7 @@ template <> struct MT<PM_Q5_K> {
     static constexpr int RP = 368, WAVE_LDS = 32 * RP;
     struct B { u32x4 c[11]; };
     template <int NV> struct A { u32x4 q[NV / 2]; f16x8 bs; };
-    template <class RW>
-    static __device__ __forceinline__ void issue_b_part(B & b, const RW & rw, int nb, int pr, int lane, int n) {
+    static __device__ __forceinline__ void issue_b_part(B & b, const Rows & rw, int nb, int pr, int lane, int n) {
 #pragma unroll
         for (int i = 3 * n; i < (n == 3 ? 11 : 3 * n + 3); ++i) {
             const int ci = lane + 64 * i, row = ci / 22, c = ci - row * 22;
@@ -261,98 +165,6 @@ template <> struct MT<PM_Q5_K> {
     }
 };
 
-// ---------------------------------------------------------------- Q6_K: row = la[U][16] | lb[U][16] | qh[U][16] | scales[nb][16] | d[nb] ------
-template <> struct MT<PM_Q6_K> {
-    static constexpr int LA = 0, LB = 32 * PITCH, QH = 64 * PITCH, SC = 96 * PITCH, DD = SC + 32 * PITCH_H, WAVE_LDS = DD + 128;
-    struct B { u32x4 la[4], lb[4], qh[4], s; uint16_t d; };
-    template <int NV> struct A { u32x4 q[NV / 2]; f16x8 bs; };       // as loaded: lane (t, g) holds the WHOLE 16-weight group 2 s + g of sub-block s (operand(): the halves the 16-k products need)
-    template <class RW>
-    static __device__ __forceinline__ void issue_b_part(B & b, const RW & rw, int nb, int pr, int lane, int n) {
-        const uint32_t u = (uint32_t) min(8 * pr + (lane & 7), 4 * nb - 1), sb = (uint32_t) min(2 * pr + (lane & 1), nb - 1);
-        b.la[n] = ld_nt16(rw.at(n, u * 16u));
-        b.lb[n] = ld_nt16(rw.at(n, (uint32_t) nb * 64u + u * 16u));
-        b.qh[n] = ld_nt16(rw.at(n, (uint32_t) nb * 128u + u * 16u));
-        if (n == 0) b.s = ld_c16(rw.at_h(pm_q6k_sc_off((uint32_t) nb, sb)));   // cached, like Q4_K's header
-        // (d: one 2-byte load per lane (row lane % 32, super-block 2 pr + lane / 32), issued by the kernel with its own row offset)
-    }
-    static __device__ __forceinline__ void stash(const B & b, uint8_t * L, int lane) {
-        const int rr = lane >> 3, c = lane & 7;
-#pragma unroll
-        for (int n = 0; n < 4; ++n) {
-            *(u32x4 *) (L + LA + (rr + 8 * n) * PITCH + c * 16) = b.la[n];
-            *(u32x4 *) (L + LB + (rr + 8 * n) * PITCH + c * 16) = b.lb[n];
-            *(u32x4 *) (L + QH + (rr + 8 * n) * PITCH + c * 16) = b.qh[n];
-        }
-        *(u32x4 *) (L + SC + (lane >> 1) * PITCH_H + (lane & 1) * 16) = b.s;
-        *(uint16_t *) (L + DD + lane * 2) = b.d;                     // [c = lane / 32][r = lane % 32]
-    }
-    // 16-weight group G = the 8 bytes at 16 G + 8 g of the super-block
-    template <int NV>
-    static __device__ __forceinline__ void issue_a(A<NV> & a, const ActSrc & x, int sb) {
-#pragma unroll
-        for (int i = 0; i < NV / 2; ++i) a.q[i] = x.ld_sub(sb, i * (16 / NV));
-        a.bs = x.ld_bs(sb);
-    }
-    // A operand of the 16-k product over group G: lane (t, g) needs bytes 8 g .. 8 g + 7 of group G. The lane pair (t, 0) / (t, 1) holds groups
-    // 2 s / 2 s + 1 whole: v_permlane32_swap hands the upper half of the even group to lane (t, 1) and the lower half of the odd group to (t, 0)
-    static __device__ __forceinline__ void operands(const u32x4 & v, u32x2 & even, u32x2 & odd) {
-#pragma unroll
-        for (int i = 0; i < 2; ++i) {
-            const u32x2 r = __builtin_bit_cast(u32x2, __builtin_amdgcn_permlane32_swap(v[i], v[2 + i], false, false));
-            even[i] = r[0]; odd[i] = r[1];
-        }
-    }
-    template <int NV, class F>
-    static __device__ __forceinline__ void compute(const A<NV> & a, const uint8_t * L, int sbi, int r, int g, const float * yd_lds, int /*t_off*/, f32x16 & out, F && between) {
-        const u32x4 s16 = *(const u32x4 *) (L + SC + r * PITCH_H + sbi * 16);
-        const float d = h2f(*(const uint16_t *) (L + DD + (sbi * 32 + r) * 2));
-        const i32x16 zero = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
-        i32x16 isum = zero;
-        u32x2 aop[NV];                                   // (the swaps work in place on the registers of a.q)
-#pragma unroll
-        for (int i = 0; i < NV / 2; ++i) operands(a.q[i], aop[2 * i], aop[2 * i + 1]);
-#pragma unroll
-        for (int hh = 0; hh < 2; ++hh)
-#pragma unroll
-            for (int v2 = 0; v2 < 2; ++v2) {
-                between(2 * hh + v2);
-                const int uo = (4 * sbi + 2 * hh + v2) * 16 + 8 * g;
-                const u32x2 la = *(const u32x2 *) (L + LA + r * PITCH + uo), lb = *(const u32x2 *) (L + LB + r * PITCH + uo),
-                            qh = *(const u32x2 *) (L + QH + r * PITCH + uo);
-                u32x2 qv[4];
-                qv[0] = (la & 0x0F0F0F0Fu)        | ((qh << 4) & 0x30303030u);
-                qv[1] = (lb & 0x0F0F0F0Fu)        | ((qh << 2) & 0x30303030u);
-                qv[2] = ((la >> 4) & 0x0F0F0F0Fu) | (qh & 0x30303030u);
-                qv[3] = ((lb >> 4) & 0x0F0F0F0Fu) | ((qh >> 2) & 0x30303030u);
-#pragma unroll
-                for (int c = 0; c < 4; ++c) {
-                    const int G = 8 * hh + 2 * c + v2;                                   // group index inside the super-block = scale index
-                    const int sc = (int) (int8_t) (s16[G >> 2] >> (8 * (G & 3)));
-                    constexpr int P = 16 / NV;                                           // sub-blocks G / 2 per operand register
-                    const u32x2 op = aop[2 * ((G >> 1) / P) + (G & 1)];
-                    const i32x16 acc = mfma_i8(pk(op[0], op[1]), pk(qv[c][0], qv[c][1]), zero);
-#pragma unroll
-                    for (int v = 0; v < NV; ++v) { isum[v] = __mul24(sc, acc[NV * ((G >> 1) % P) + v]) + isum[v]; if constexpr (NV < 16) asm volatile("" : "+v"(isum[v])); }   // |acc| <= 16*63*127 (NV = 16: the barrier costs 100 B of spills)
-                }
-            }
-        // sum_G scale_G * bsum_G (the -32 offset of every weight): B slot s of lane group g = scale[2 s + g]
-        f16x8 bm;
-#pragma unroll
-        for (int s = 0; s < 8; ++s) { const int G = 2 * s + g; bm[s] = (_Float16) (float) (int) (int8_t) (s16[G >> 2] >> (8 * (G & 3))); }
-        const f32x16 fz = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
-        const f32x16 ms = __builtin_amdgcn_mfma_f32_32x32x16_f16(a.bs, bm, fz, 0, 0, 0);
-#pragma unroll
-        for (int q = 0; q < NV / 4; ++q) {
-            const f32x4 yd = *(const f32x4 *) (yd_lds + 8 * q + 4 * g);
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const int v = 4 * q + i;
-                out[v] = fmaf(yd[i] * d, (float) (isum[v] - 32 * (int) ms[v]), out[v]);   // the reference's integer sum, then one rounding
-            }
-        }
-    }
-};
-
 // ---------------------------------------------------------------- Q8_0: row = qa[nb][16] | qb[nb][16] | d[nb] (f16), nb = K / 32 ------------
 // Weights and activations in 32-value blocks (ggml_vec_dot_q8_0_q8_0, ggml-quants.c:5518: sumf += sumi * d_w * d_a per block): one 32-k MFMA is one
 // block, its 32 x 32 integer tile is scaled by d_w (lane-local: the lane's own row) x d_a (the token of the result register). In this kernel's
@@ -365,8 +177,7 @@ template <> struct MT<PM_Q8_0> {
     template <int NV> struct A { u32x4 q[NV / 4]; };
     // (ds: the ACTIVATION scales of the step's 8 blocks, [block][32 token slots] f32 = 1 KiB per wave and step, travel with the weight tile into the wave's
     //  LDS image - held in registers per result token they cost 32 VGPRs per operand set and the 16-token form spilled)
-    template <class RW>
-    static __device__ __forceinline__ void issue_b_part(B & b, const RW & rw, int nb /*blocks per row*/, int pr, int lane, int n) {
+    static __device__ __forceinline__ void issue_b_part(B & b, const Rows & rw, int nb /*blocks per row*/, int pr, int lane, int n) {
         const uint32_t u = (uint32_t) min(8 * pr + (lane & 7), nb - 1);
         b.qa[n] = ld_nt16(rw.at(n, u * 16u));
         b.qb[n] = ld_nt16(rw.at(n, (uint32_t) nb * 16u + u * 16u));
@@ -410,11 +221,10 @@ template <> struct MT<PM_Q8_0> {
     }
 };
 
-// the work of workgroup w of G on the launch p (its own grid, or one part of a two-part launch)
-// EPI: the wq | wk | wv epilogue (MmqP::e_*) is compiled in - instantiations of their own: carried by every kernel as a run-time switch it cost the launches
-// that never use it 2-6 us per layer (Qwen2.5-72B, NEOX rope: 236 -> 242 us at 8 tokens)
-template <int TYPE, int NV, bool MJ, bool EPI = false>  // NV result registers per lane in use: 4 (<= 8 tokens), 8 (<= 16), 16 (<= 32)
-__device__ __forceinline__ void mmq_i8_body(const MmqP & p, const int w, const int G, uint8_t * smem) {
+template <int TYPE, int NV>                                        // NV result registers per lane in use: 4 (<= 8 tokens), 8 (<= 16)
+__global__ __launch_bounds__(BLOCK, 2) void mmq_i8_kernel(MmqP p) {
+    extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
+    const int w = (int) blockIdx.x, G = (int) gridDim.x;
     typedef MT<TYPE> M;
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;   // (a scalar: the K slice, the loop counters and the buffer loads' scalar offsets derive from it)
     constexpr bool Q80 = TYPE == PM_Q8_0;                         // 32-value blocks: "super-block" = 4 blocks, no scale table in LDS (scales travel with the operands)
@@ -422,32 +232,24 @@ __device__ __forceinline__ void mmq_i8_body(const MmqP & p, const int w, const i
     const int nbw = Q80 ? p.K / 32 : nsb;                         // what the tile loader counts in: blocks of the row
     float * dTl = (float *) smem;                                 // activation scales [nsb + 1][32] (0 for token slots >= T; last row all 0)
     uint8_t * stage = smem + (Q80 ? 0 : (size_t) (nsb + 1) * 128);   // NWAVE x WAVE_LDS; afterwards the 32 KB reduction buffer
-    int r0 = (int) ((long) p.N * w / G), r1 = (int) ((long) p.N * (w + 1) / G);            // (MJ: virtual rows over all jobs)
-    if constexpr (EPI) { r0 &= ~1; r1 &= ~1; }                    // rotation pairs stay inside a workgroup (N and the job boundaries are even)
+    const int r0 = (int) ((long) p.N * w / G), r1 = (int) ((long) p.N * (w + 1) / G);
     const int nrg = (r1 - r0 + 31) >> 5;
     const int RGB = 1 << p.rgb_log2, KS = NWAVE >> p.rgb_log2;
     const int rgi = wave & (RGB - 1), ks = wave >> p.rgb_log2;
-#ifdef PM_MMQ_KCONTIG
-    const int pb = npairs * ks / KS, pe = npairs * (ks + 1) / KS, pstep = 1;
-#else
     // K slices INTERLEAVED over the waves that share a row group: at any time those waves read ADJACENT 128-byte pieces of a row (KS x 128 B
     // contiguous per row and stream) instead of pieces a whole slice apart - HBM sees longer bursts per open page
     const int pstep = KS, pb = ks, pe = npairs <= ks ? ks : ks + ((npairs - ks + KS - 1) / KS) * KS;      // pairs pb, pb + KS, ... < pe
-#endif
     uint8_t * L = stage + wave * M::WAVE_LDS;
     const int r = lane & 31, g = lane >> 5;
     constexpr int RT = 2 * NV;                                                      // operand rows per sub-block
     const int tq = r / RT, tt = r % RT;                                              // this lane's sub-block of a register, and its token
-    const bool act = NV == 16 ? true : tt < p.T, act_b = NV == 16 ? true : r < p.T; // token slots >= T: operand bytes are don't-care (scale row 0, never stored)
+    const bool act = tt < p.T, act_b = r < p.T; // token slots >= T: operand bytes are don't-care (scale row 0, never stored)
     ActSrc xs;
     xs.rx = __builtin_amdgcn_make_buffer_rsrc((void *) p.qT, 0, Q80 ? nbw * 1024 : nsb * 8192, 0x00020000);
     xs.rb = __builtin_amdgcn_make_buffer_rsrc((void *) p.bsT, 0, Q80 ? nbw * 128 : nsb * 1024 + 512, 0x00020000);   // (+ t_off slots of the last super-block: inside the table allocation)
     xs.xo = act ? (uint32_t) (tq * 1024 + (32 * g + tt + p.t_off) * 16) : 0x80000000u;
     xs.bo = Q80 ? (uint32_t) (16 * lane) : act_b ? (uint32_t) ((lane + p.t_off) * 16) : 0x80000000u;   // (Q8_0: lane l carries 16 bytes of the step's [8 blocks][32 slots] activation scales)
-    Rows<MJ> rw;
-    // (measured and rejected at 8 tokens: TWO weight tiles in flight per wave - 57344 x 8192 Q4_K 53.0 -> 55.1 us, Q6_K 98.0 -> 102.4; two workgroups that
-    //  share a row group's K where 128 row groups leave half the chip idle - 4096 x 14336 Q6_K 24.7 -> 22.8 us, but Q4_K 14.3 -> 16.3: the exchange costs what the second half of the chip
-    //  saves. What Q6_K launches lose is memory traffic: 1.36 x the weights' bytes, the scale and d lines of a row tail are fetched again for every step)
+    Rows rw;
     typename M::B R;
     typename M::template A<NV> A0 = {}, A1 = {};                 // (inactive token lanes keep these zeros)
     // a step's weight tile goes out in FOUR parts. Issued in one burst (13 x 1 KiB per wave, 100 KB per CU) the wave sat in the issue itself until the
@@ -456,7 +258,6 @@ __device__ __forceinline__ void mmq_i8_body(const MmqP & p, const int w, const i
     // products keeps both busy.
     auto issue_b_part = [&](typename M::B & R, int pr, int n) __attribute__((always_inline)) {
         M::issue_b_part(R, rw, nbw, pr, lane, n);
-        if constexpr (TYPE == PM_Q6_K) if (n == 0) R.d = *(const PM_G uint16_t *) rw.at_d(pm_q6k_d_off((uint32_t) nsb, (uint32_t) min(2 * pr + g, nsb - 1)));   // cached: 32 steps share the line
         if constexpr (Q80) if (n == 0) M::issue_ds(R, xs, pr);
     };
     auto issue_b = [&](typename M::B & R, int pr) __attribute__((always_inline)) {
@@ -466,20 +267,8 @@ __device__ __forceinline__ void mmq_i8_body(const MmqP & p, const int w, const i
     // the first weight tile and activation slice of a row group (in flight before anything waits)
     auto first = [&](int rg) __attribute__((always_inline)) {
         const int rbase = r0 + 32 * rg;
-        if constexpr (!MJ) {
-            rw.base = p.W + (long) rbase * p.row_stride;
-            rw.stride = (uint32_t) p.row_stride; rw.lim = r1 - 1 - rbase; rw.rr = lane >> 3; rw.rh = lane >> 1;
-            rw.off_d = (uint32_t) min(r, rw.lim) * rw.stride;
-        } else {
-            auto rowptr = [&](int v) __attribute__((always_inline)) {                     // virtual row -> its matrix row
-                v = min(v, r1 - 1);
-                const int j = (v >= p.start[1] && p.njobs > 1) + (v >= p.start[2] && p.njobs > 2);
-                return (j == 0 ? p.Wj[0] : j == 1 ? p.Wj[1] : p.Wj[2]) + (long) (v - (j == 0 ? 0 : j == 1 ? p.start[1] : p.start[2])) * p.row_stride;
-            };
-#pragma unroll
-            for (int n = 0; n < 4; ++n) rw.rp[n] = rowptr(rbase + (lane >> 3) + 8 * n);
-            rw.rph = rowptr(rbase + (lane >> 1)); rw.rpd = rowptr(rbase + r);
-        }
+        rw.base = p.W + (long) rbase * p.row_stride;
+        rw.stride = (uint32_t) p.row_stride; rw.lim = r1 - 1 - rbase; rw.rr = lane >> 3; rw.rh = lane >> 1;
         rw.lm = ~0u;
         issue_b(R, pb);
         M::template issue_a<NV>(A0, xs, 2 * pb);
@@ -519,11 +308,8 @@ __device__ __forceinline__ void mmq_i8_body(const MmqP & p, const int w, const i
                 const int prn = min(pr + pstep, pe - pstep);             // the tile these registers take next
                 rw.lm = pr + pstep < pe ? ~0u : 0u;                      // (past the wave's last step: a request for nothing)
                 __builtin_amdgcn_sched_barrier(0);
-                // (the 32-token Q6_K form has no registers for it - 404 B of spills, 88 -> 205 us: its tile still goes out in one burst)
-                constexpr bool SPREAD = !(TYPE == PM_Q6_K && NV == 16);
-                if constexpr (!SPREAD) { issue_b(Rc, prn); __builtin_amdgcn_sched_barrier(0); }
                 auto part = [&](int n) __attribute__((always_inline)) {   // next tile, part n: unconditional, pinned between the quarters
-                    if constexpr (SPREAD) { __builtin_amdgcn_sched_barrier(0); issue_b_part(Rc, prn, n); __builtin_amdgcn_sched_barrier(0); }
+                    __builtin_amdgcn_sched_barrier(0); issue_b_part(Rc, prn, n); __builtin_amdgcn_sched_barrier(0);
                 };
                 M::template compute<NV>(A0, L, 0, r, g, dTl + sb0 * 32, p.t_off, out, part);
                 __builtin_amdgcn_sched_barrier(0);
@@ -546,60 +332,13 @@ __device__ __forceinline__ void mmq_i8_body(const MmqP & p, const int w, const i
             float s = 0.0f;
             for (int k = 0; k < KS; ++k) s += red[(((k << p.rgb_log2) + gi) * 16 + v) * 64 + l];
             const int t = 8 * (v >> 2) + 4 * (l >> 5) + (v & 3), row = r0 + 32 * (rg0 + gi) + (l & 31);
-            const bool live = t < p.T && row < r1;
-            // the element's job: local row, output, bias
-            int j = 0, lr = row, nj = p.N; const float * bj = p.bias; float * yj = p.y;
-            if constexpr (MJ) {
-                j = (row >= p.start[1] && p.njobs > 1) + (row >= p.start[2] && p.njobs > 2);
-                lr = row - (j == 0 ? 0 : j == 1 ? p.start[1] : p.start[2]); nj = j == 0 ? p.nj[0] : j == 1 ? p.nj[1] : p.nj[2];
-                bj = j == 0 ? p.bj[0] : j == 1 ? p.bj[1] : p.bj[2];
-                yj = j == 0 ? p.yj[0] : j == 1 ? p.yj[1] : p.yj[2];
-            }
-            if (live && bj) s += ld_g(bj + lr);
-            if constexpr (EPI) {
-                const float sp = __shfl_xor(s, 1);                      // the pair's other row: the neighbouring lane (r0 even), same token
-                if (live) {
-                    const int role = j == 0 ? p.e_role[0] : j == 1 ? p.e_role[1] : p.e_role[2];
-                    const int seq = p.e_seq ? p.e_seq[p.e_rows ? t : 0] : 0;
-                    const int pos = p.e_rows ? p.e_pos[t] : p.e_pos[seq] + t;
-                    const long kv_off = (long) seq * p.e_seq_stride;
-                    if (role == 3) p.e_vc[kv_off + (long) lr * p.e_nctx + pos] = f2h(s);
-                    else {
-                        const int d = lr % p.e_dh;
-                        float o = s;
-                        if (d < p.e_nrot) {
-                            const float c = ld_g(p.e_tab + (long) t * p.e_nrot + (d & ~1)), sn = ld_g(p.e_tab + (long) t * p.e_nrot + (d & ~1) + 1);
-                            o = (d & 1) ? sp * sn + s * c : s * c - sp * sn;          // o1 = x0 sin + x1 cos | o0 = x0 cos - x1 sin
-                        }
-                        const uint16_t hv = f2h(o);
-                        if (role == 2) p.e_kc[kv_off + (long) pos * p.e_kvdim + lr] = hv;
-                        else st_g(yj + (long) t * nj + lr, role == 1 ? h2f(hv) : o);
-                    }
-                }
-            } else if (live) {
-                if (p.resid) s += ld_g(p.resid + (long) t * (MJ ? nj : (int) p.y_stride) + lr);
-                st_g(yj + (long) t * (MJ ? nj : (int) p.y_stride) + lr, s);
-            }
+            if (t >= p.T || row >= r1) continue;
+            if (p.bias) s += ld_g(p.bias + row);
+            if (p.resid) s += ld_g(p.resid + (long) t * p.N + row);
+            st_g(p.y + (long) t * p.N + row, s);
         }
         __syncthreads();
     }
-}
-
-template <int TYPE, int NV, bool MJ = false, bool EPI = false>
-__global__ __launch_bounds__(BLOCK, 2) void mmq_i8_kernel(MmqP p) {
-    extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
-    mmq_i8_body<TYPE, NV, MJ, EPI>(p, (int) blockIdx.x, (int) gridDim.x, smem);
-}
-
-// Two launches that share the activations as ONE grid: workgroups [0, ga) are the multi-job launch `a` (wq | wk, type TA), the rest the single matrix `b` of
-// another type (wv: Q6_K or Q5_K in the Q4_K_M files, src/llama.cpp:19447 use_more_bits) - by itself a 7 MB matrix is a launch of ~14 us that 32 workgroups
-// spend mostly on their fixed costs (profiles/r06_small_batch.txt); here it rides in the shadow of the large part.
-struct MmqP2 { MmqP a, b; int ga; };
-template <int TA, int TB, int NV, bool EPI = false>
-__global__ __launch_bounds__(BLOCK, 2) void mmq_i8_dual_kernel(MmqP2 pp) {
-    extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
-    if ((int) blockIdx.x < pp.ga) mmq_i8_body<TA, NV, true, EPI>(pp.a, (int) blockIdx.x, pp.ga, smem);
-    else mmq_i8_body<TB, NV, TB == PM_Q6_K, EPI>(pp.b, (int) blockIdx.x - pp.ga, (int) gridDim.x - pp.ga, smem);
 }
 
 // prologue: per super-block, the activation group sums as F16 in A-operand order and the transposed activation scales
@@ -628,10 +367,22 @@ __global__ __launch_bounds__(64) void mmq_prep_q80_kernel(const uint8_t * xq, lo
 }
 
 // row groups a workgroup works on side by side (the other waves split K): 5..7 groups take all 8 wave slots in ONE round (one fill / drain of the step
-// pipeline, no K split) instead of two rounds of 4 (ffn_gate | ffn_up of the 70B shape: 7 groups per workgroup); PM355_MMQ_RGB8_MIN=8: the round-5 rule
-int rgb_log2_for(int nrg) {
-    static const int rgb8_min = [] { const char * e = getenv("PM355_MMQ_RGB8_MIN"); const int v = e ? atoi(e) : 0; return v >= 3 && v <= 8 ? v : 5; }();
-    return nrg >= rgb8_min ? 3 : nrg >= 3 ? 2 : nrg == 2 ? 1 : 0;
+// pipeline, no K split) instead of two rounds of 4
+int rgb_log2_for(int nrg) { return nrg >= 5 ? 3 : nrg >= 3 ? 2 : nrg == 2 ? 1 : 0; }
+size_t lds_of(int type, int K) { return type == PM_Q8_0 ? (size_t) NWAVE * MT<PM_Q8_0>::WAVE_LDS : (size_t) (K / 256 + 1) * 128 + NWAVE * MT<PM_Q5_K>::WAVE_LDS; }
+// one matrix of Q5_K or Q8_0 over up to 16 tokens (q: one job)
+int launch_16(const RowsP & q, int type, hipStream_t st) {
+    const int cus = pm_device_cus(), N = q.job[0].N, grid = N / 32 >= cus ? cus : (N + 31) / 32;
+    MmqP p = {q.job[0].W, (long) pm_weight_row_stride(type, q.K), N, q.K, q.T, rgb_log2_for(((N + grid - 1) / grid + 31) / 32), q.t_off, type == PM_Q8_0 ? (const uint8_t *) q.dT : q.bsT, q.dT, q.qT,
+              q.job[0].y, q.job[0].bias, q.job[0].resid};           // (Q8_0: bsT are the f32 activation scales [blk][32])
+    const size_t lds = lds_of(type, q.K);
+    auto go = [&](auto kern) {
+        pm_allow_big_lds((const void *) kern, 150 * 1024);
+        hipLaunchKernelGGL(kern, dim3(grid), dim3(BLOCK), lds, st, p);
+        return 0;
+    };
+    if (type == PM_Q5_K) return q.T <= 8 ? go(mmq_i8_kernel<PM_Q5_K, 4>) : go(mmq_i8_kernel<PM_Q5_K, 8>);
+    return q.T <= 8 ? go(mmq_i8_kernel<PM_Q8_0, 4>) : go(mmq_i8_kernel<PM_Q8_0, 8>);
 }
 
 // per-device scratch (grown on demand, like mmq.hip's f16 activation copy): quantized activations of an f32 call + the two tables
@@ -644,20 +395,15 @@ Scr g_scr80[16][NSCR] = {};             // Q8_0 launches: their own tables (neve
 uint64_t g_tick = 0;
 std::mutex g_scr_mu;
 
-}  // namespace
 
-size_t pm_mmq_i8_lds_bytes(int type, int K) {
-    if (type == PM_Q8_0) return (size_t) NWAVE * MT<PM_Q8_0>::WAVE_LDS;
-    const size_t w = type == PM_Q4_K ? MT<PM_Q4_K>::WAVE_LDS : type == PM_Q5_K ? MT<PM_Q5_K>::WAVE_LDS : MT<PM_Q6_K>::WAVE_LDS;
-    return (size_t) (K / 256 + 1) * 128 + NWAVE * w;
-}
+}  // namespace
 
 // 0 when pm_launch_mmq_i8 serves this shape
 int pm_mmq_i8_check(int type, int K, int N, int T) {
     if (type != PM_Q4_K && type != PM_Q5_K && type != PM_Q6_K && type != PM_Q8_0) return -1;
     if (type == PM_Q8_0) return (T < 1 || T > 64 || K % 32 || K < 512 || N < 1) ? -2 : 0;
     if (T < 1 || T > 64 || K % 256 || K < 512 || N < 1) return -2;
-    if (pm_mmq_i8_lds_bytes(type, K) > 150 * 1024) return -4;
+    if (K > (type == PM_Q4_K ? 134912 : type == PM_Q5_K ? 113920 : 59136)) return -4;
     return 0;
 }
 
@@ -705,7 +451,18 @@ void launch_prep(const Scr * sc, const void * xq, int K, int T, hipStream_t st) 
 }  // namespace
 
 namespace {
-// Q8_0 weights x Q8_0 activations, passes of up to 16 tokens. xq: row-SoA Q8_0 rows (quantize.hip) or null and x_f32 is quantized first. Its tables
+// Q5_K and Q8_0: whether 17..32 tokens go in one pass (else two of up to 16, or mmq_rows.hip). Us, as it was / one pass: Q8_0 20 tokens 8192 x 2048 10.6 / 8.3, 14336 x 4096 24.6 / 17.2,
+// 8192 x 8192 24.9 / 18.3, 8192 x 29568 75 / 55; 28 tokens 16384 x 1024 16.7 / 9.1, 14336 x 4096 33.1 / 18.3, 8192 x 8192 34.3 / 19.2; Q5_K 8192 x 8192 20 tokens 21.0 / 16.8, 28 31.7 / 17.8. On the
+// other side of the lines one pass would be the faster one too (8192 x 4096 at 32 tokens 20.6 / 12.0, Q5_K 14336 x 4096 20.3 / 16.0): there the forms are those that test_host_launches.py has
+bool one_pass(int type, long N, int K, int T) {
+    const int cus = pm_device_cus();
+    const long groups = ((N + cus - 1) / cus + 15) / 16;
+    if (T <= 16 || groups == 1) return false;
+    if (type == PM_Q5_K) return K > 4096;
+    return T <= 24 ? K >= 2048 : K > 4096 || groups > 2;
+}
+
+// Q8_0 weights x Q8_0 activations. xq: row-SoA Q8_0 rows (quantize.hip) or null and x_f32 is quantized first. Its tables
 // (operand-ordered values + f32 scales of both 32-slot halves, then a quantized copy of 64 f32 rows) are written by a prologue launch per call.
 Scr * scratch80(int dev, hipStream_t st, size_t need) {
     std::lock_guard<std::mutex> lk(g_scr_mu);
@@ -744,33 +501,16 @@ int launch_q80(const void * W, const void * xq, const float * x_f32, float * Y, 
         hipLaunchKernelGGL(mmq_prep_q80_kernel, dim3(nb), dim3(64), 0, st, (const uint8_t *) xq + (size_t) t0 * xrow, (long) xrow, K, T - t0 < 32 ? T - t0 : 32,
                            base + c * (qtab + dtab), (float *) (base + c * (qtab + dtab) + qtab));
     }
-    const int cus = pm_device_cus();
-    const int grid = N / 32 >= cus ? cus : (N + 31) / 32;
-    const int rows = (N + grid - 1) / grid, nrg = (rows + 31) / 32;
-    const size_t lds = pm_mmq_i8_lds_bytes(PM_Q8_0, K);
-    const int tmax = pm_mmq_rows_takes(PM_Q8_0, N, K, T) || pm_mmq_rows_takes(PM_Q8_0, N, K, 32) ? 32 : 16;      // (this file's 32-token form spills 236 B: 502 vs 422 us per Qwen2.5-72B layer at 32 tokens - two passes of 16 it is)
+    const int tmax = one_pass(PM_Q8_0, N, K, std::min(T, 32)) || pm_mmq_rows_takes(PM_Q8_0, N, K, T) || pm_mmq_rows_takes(PM_Q8_0, N, K, 32) ? 32 : 16;
     for (int t0 = 0; t0 < T; t0 += tmax) {
         const int tn = T - t0 < tmax ? T - t0 : tmax;
         uint8_t * tab = base + (t0 / 32) * (qtab + dtab);
-        if (pm_mmq_rows_takes(PM_Q8_0, N, K, tn)) {
-            RowsP q = {};
-            q.job[0] = {(const uint8_t *) W, Y + (size_t) t0 * N, bias, resid ? resid + (size_t) t0 * N : nullptr, N};
-            q.njobs = 1; q.K = K; q.T = tn; q.t_off = t0 % 32; q.qT = tab; q.dT = (const float *) (tab + qtab);
-            const int ty = PM_Q8_0;
-            if (pm_launch_mmq_rows(q, &ty, st)) return -3;
-            continue;
-        }
-        MmqP p = {};
-        p.t_off = t0 % 32;
-        p.W = (const uint8_t *) W; p.row_stride = (long) pm_weight_row_stride(PM_Q8_0, K); p.N = N; p.K = K; p.T = tn;
-        p.qT = tab; p.bsT = tab + qtab;                            // (bsT: here the f32 activation scales [blk][32])
-        p.y = Y + (size_t) t0 * N; p.y_stride = N; p.bias = bias; p.resid = resid ? resid + (size_t) t0 * N : nullptr;
-        p.rgb_log2 = rgb_log2_for(nrg);
-        auto go = [&](auto kern) {
-            pm_allow_big_lds((const void *) kern, 150 * 1024);
-            hipLaunchKernelGGL(kern, dim3(grid), dim3(BLOCK), lds, st, p);
-        };
-        if (tn <= 8) go(mmq_i8_kernel<PM_Q8_0, 4>); else go(mmq_i8_kernel<PM_Q8_0, 8>);
+        RowsP q = {};
+        q.job[0] = {(const uint8_t *) W, Y + (size_t) t0 * N, bias, resid ? resid + (size_t) t0 * N : nullptr, N};
+        q.njobs = 1; q.K = K; q.T = tn; q.t_off = t0 % 32; q.qT = tab; q.dT = (const float *) (tab + qtab);
+        const int ty = PM_Q8_0;
+        const bool once = one_pass(PM_Q8_0, N, K, tn);
+        if (!once && pm_mmq_rows_takes(PM_Q8_0, N, K, tn) ? pm_launch_mmq_rows(q, &ty, st) : once ? pm_launch_mmq_mid(q, &ty, st) : launch_16(q, ty, st)) return -3;
     }
     return 0;
 }
@@ -822,7 +562,7 @@ int pm_launch_mmq_i8(int type, const void * W, const void * xq, const float * x_
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 16) return -3;
     const int nsb = K / 256;
-    const size_t xrow = pm_q8k_row_bytes(K), tab = (size_t) nsb * (1024 + 128);
+    const size_t tab = (size_t) nsb * (1024 + 128);
     const Scr * sc = scratch(dev, st, K, reuse_prep != 0);
     if (!sc) return -3;
     if (!xq) {
@@ -831,37 +571,15 @@ int pm_launch_mmq_i8(int type, const void * W, const void * xq, const float * x_
         xq = q;
     }
     if (!reuse_prep) launch_prep(sc, xq, K, T, st);
-    const int cus = pm_device_cus();
-    const int grid = N / 32 >= cus ? cus : (N + 31) / 32;
-    const int rows = (N + grid - 1) / grid, nrg = (rows + 31) / 32;
-    const size_t lds = pm_mmq_i8_lds_bytes(type, K);
-    const int tmax = type != PM_Q5_K || pm_mmq_rows_takes(type, N, K, T) || pm_mmq_rows_takes(type, N, K, 32) ? 32 : 16;                    // (Q5_K: 11 weight registers more per step - its 32-token form here spills 388 B / lane)
+    const int tmax = type != PM_Q5_K || one_pass(type, N, K, std::min(T, 32)) || pm_mmq_rows_takes(type, N, K, T) || pm_mmq_rows_takes(type, N, K, 32) ? 32 : 16;
     for (int t0 = 0, c = 0; t0 < T; t0 += tmax, ++c) {
         const int tn = T - t0 < tmax ? T - t0 : tmax;
         uint8_t * bsT = sc->p + (t0 / 32) * tab; float * dT = (float *) (bsT + (size_t) nsb * 1024);    // tables are per 32 tokens
-        if (pm_mmq_rows_takes(type, N, K, tn)) {
-            RowsP q = {};
-            q.job[0] = {(const uint8_t *) W, Y + (size_t) t0 * N, bias, resid ? resid + (size_t) t0 * N : nullptr, N};
-            q.njobs = 1; q.K = K; q.T = tn; q.t_off = t0 % 32; q.qT = sc->p + scr_q_off(K) + (size_t) (t0 / 32) * nsb * 8192; q.bsT = bsT; q.dT = dT;
-            if (pm_launch_mmq_rows(q, &type, st)) return -3;
-            continue;
-        }
-        const uint8_t * xc = (const uint8_t *) xq + (size_t) t0 * xrow;
-        MmqP p = {};
-        p.t_off = t0 % 32;
-        p.W = (const uint8_t *) W; p.row_stride = (long) pm_weight_row_stride(type, K); p.N = N; p.K = K; p.T = tn;
-        p.xq = xc; p.xq_stride = (long) xrow; p.bsT = bsT; p.dT = dT; p.qT = sc->p + scr_q_off(K) + (size_t) (t0 / 32) * nsb * 8192;
-        p.y = Y + (size_t) t0 * N; p.y_stride = N; p.bias = bias; p.resid = resid ? resid + (size_t) t0 * N : nullptr;
-        p.rgb_log2 = rgb_log2_for(nrg);
-        auto go = [&](auto kern) {
-            pm_allow_big_lds((const void *) kern, 150 * 1024);
-            hipLaunchKernelGGL(kern, dim3(grid), dim3(BLOCK), lds, st, p);
-        };
-        if (type == PM_Q4_K) { if (tn <= 8) go(mmq_i8_kernel<PM_Q4_K, 4>); else if (tn <= 16) go(mmq_i8_kernel<PM_Q4_K, 8>); else go(mmq_i8_kernel<PM_Q4_K, 16>); }
-        else if (type == PM_Q5_K) { if (tn <= 8) go(mmq_i8_kernel<PM_Q5_K, 4>); else go(mmq_i8_kernel<PM_Q5_K, 8>); }
-        else if (tn <= 8)  go(mmq_i8_kernel<PM_Q6_K, 4>);
-        else if (tn <= 16) go(mmq_i8_kernel<PM_Q6_K, 8>);
-        else               go(mmq_i8_kernel<PM_Q6_K, 16>);
+        RowsP q = {};
+        q.job[0] = {(const uint8_t *) W, Y + (size_t) t0 * N, bias, resid ? resid + (size_t) t0 * N : nullptr, N};
+        q.njobs = 1; q.K = K; q.T = tn; q.t_off = t0 % 32; q.qT = sc->p + scr_q_off(K) + (size_t) (t0 / 32) * nsb * 8192; q.bsT = bsT; q.dT = dT;
+        const bool once = type != PM_Q5_K || one_pass(type, N, K, tn);
+        if (!(type == PM_Q5_K && once) && pm_mmq_rows_takes(type, N, K, tn) ? pm_launch_mmq_rows(q, &type, st) : once ? pm_launch_mmq_mid(q, &type, st) : launch_16(q, type, st)) return -3;
     }
     return 0;
 }
@@ -871,15 +589,6 @@ bool fill_epi(RowsP & p, const pm_qkv_epi * e) {
     if (!e) return true;
     if (e->neox || e->v_rowmajor || e->dyn || !e->tab || !e->pos || !e->kc || !e->vc || e->dh < 2 || (e->dh & 1) || (e->n_rot & 1)) return false;
     p.e_on = 1; p.e_tab = e->tab; p.e_pos = e->pos; p.e_seq = e->seq; p.e_seq_stride = e->seq_stride; p.e_kc = (uint16_t *) e->kc; p.e_vc = (uint16_t *) e->vc;
-    p.e_dh = e->dh; p.e_nctx = e->n_ctx; p.e_nrot = e->n_rot; p.e_kvdim = e->Hkv * e->dh; p.e_rows = e->rows;
-    return true;
-}
-// wq | wk | wv epilogue of a launch (MmqP::e_*): NORM-mode rope, transposed F16 V cache, engine mode (cell = position). false: not served
-bool fill_epi(MmqP & p, const pm_qkv_epi * e, int r0, int r1, int r2) {
-    if (!e) return true;
-    if (e->neox || e->v_rowmajor || e->dyn || !e->tab || !e->pos || !e->kc || !e->vc || e->dh < 2 || (e->dh & 1) || (e->n_rot & 1)) return false;
-    p.e_on = 1; p.e_role[0] = r0; p.e_role[1] = r1; p.e_role[2] = r2;
-    p.e_tab = e->tab; p.e_pos = e->pos; p.e_seq = e->seq; p.e_seq_stride = e->seq_stride; p.e_kc = (uint16_t *) e->kc; p.e_vc = (uint16_t *) e->vc;
     p.e_dh = e->dh; p.e_nctx = e->n_ctx; p.e_nrot = e->n_rot; p.e_kvdim = e->Hkv * e->dh; p.e_rows = e->rows;
     return true;
 }
@@ -898,52 +607,18 @@ int pm_launch_mmq_i8_multi(int type, int njobs, const void * const * W, const in
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 16) return -3;
     const int nsb = K / 256;
-    const size_t xrow = pm_q8k_row_bytes(K);
     const Scr * sc = scratch(dev, st, K, reuse_prep != 0);
     if (!sc) return -3;
     if (!reuse_prep) launch_prep(sc, xq, K, T, st);
-    const int cus = pm_device_cus();
-    const int grid = total / 32 >= cus ? cus : (int) ((total + 31) / 32);
-    const int rows = (int) ((total + grid - 1) / grid), nrg = (rows + 31) / 32;
-    MmqP p = {};
-    p.row_stride = (long) pm_weight_row_stride(type, K); p.N = (int) total; p.K = K; p.T = T;
-    p.xq = (const uint8_t *) xq; p.xq_stride = (long) xrow; p.bsT = sc->p; p.dT = (const float *) (sc->p + (size_t) nsb * 1024); p.qT = sc->p + scr_q_off(K);
-    p.njobs = njobs;
-    int at = 0;
-    for (int j = 0; j < 3; ++j) {
-        const int jj = j < njobs ? j : njobs - 1;
-        p.Wj[j] = (const uint8_t *) W[jj]; p.yj[j] = Y[jj]; p.bj[j] = bias ? bias[jj] : nullptr; p.nj[j] = N[jj];
-        p.start[j] = j < njobs ? at : (int) total;
-        if (j < njobs) at += N[j];
-    }
-    p.rgb_log2 = rgb_log2_for(nrg);
-    if (!fill_epi(p, epi, 1, 2, 3)) return -5;
-    const size_t lds = pm_mmq_i8_lds_bytes(type, K);
-    auto go = [&](auto kern) {
-        pm_allow_big_lds((const void *) kern, 150 * 1024);
-        hipLaunchKernelGGL(kern, dim3(grid), dim3(BLOCK), lds, st, p);
-    };
     const size_t tab = (size_t) nsb * (1024 + 128);
     for (int t0 = 0, c = 0; t0 < T; t0 += 32, ++c) {                 // passes of 32 tokens, each with its own tables
         const int tn = T - t0 < 32 ? T - t0 : 32;
-        if (tn <= 8 && pm_mmq_rows_takes(type, total, K, tn, PM_ROWS_SEVERAL)) {
-            RowsP q = {};
-            int ty[3];
-            q.njobs = njobs; q.K = K; q.T = tn; q.bsT = sc->p + c * tab; q.dT = (const float *) (q.bsT + (size_t) nsb * 1024); q.qT = sc->p + scr_q_off(K) + (size_t) c * nsb * 8192;
-            for (int j = 0; j < njobs; ++j) { q.job[j] = {(const uint8_t *) W[j], Y[j] + (size_t) t0 * N[j], bias ? bias[j] : nullptr, nullptr, N[j]}; ty[j] = type; }
-            if (!fill_epi(q, epi)) return -5;
-            if (pm_launch_mmq_rows(q, ty, st)) return -3;
-            continue;
-        }
-        p.T = tn;
-        p.bsT = sc->p + c * tab; p.dT = (const float *) (p.bsT + (size_t) nsb * 1024); p.qT = sc->p + scr_q_off(K) + (size_t) c * nsb * 8192;
-        for (int j = 0; j < 3; ++j) { const int jj = j < njobs ? j : njobs - 1; p.yj[j] = Y[jj] + (size_t) t0 * N[jj]; }
-#define PM_I8_GO(T_, E_) { if (tn <= 8) go(mmq_i8_kernel<T_, 4, true, E_>); else if (tn <= 16) go(mmq_i8_kernel<T_, 8, true, E_>); else go(mmq_i8_kernel<T_, 16, true, E_>); }
-        if (p.e_on && type == PM_Q4_K) PM_I8_GO(PM_Q4_K, true)
-        else if (p.e_on)               PM_I8_GO(PM_Q6_K, true)
-        else if (type == PM_Q4_K)      PM_I8_GO(PM_Q4_K, false)
-        else                           PM_I8_GO(PM_Q6_K, false)
-#undef PM_I8_GO
+        RowsP q = {};
+        int ty[3];
+        q.njobs = njobs; q.K = K; q.T = tn; q.bsT = sc->p + c * tab; q.dT = (const float *) (q.bsT + (size_t) nsb * 1024); q.qT = sc->p + scr_q_off(K) + (size_t) c * nsb * 8192;
+        for (int j = 0; j < njobs; ++j) { q.job[j] = {(const uint8_t *) W[j], Y[j] + (size_t) t0 * N[j], bias ? bias[j] : nullptr, nullptr, N[j]}; ty[j] = type; }
+        if (!fill_epi(q, epi)) return -5;
+        if (tn <= 8 && pm_mmq_rows_takes(type, total, K, tn, PM_ROWS_SEVERAL) ? pm_launch_mmq_rows(q, ty, st) : pm_launch_mmq_mid(q, ty, st)) return -3;
     }
     return 0;
 }
@@ -954,7 +629,7 @@ int pm_launch_mmq_i8_dual(int ta, int na, const void * const * Wa, const int * N
                           int tb, const void * Wb, int Nb, float * Yb, const float * bb, const void * xq, int K, int T, int reuse_prep, hipStream_t st,
                           const pm_qkv_epi * epi) {
     static const bool off = [] { const char * e = getenv("PM355_MMQ_DUAL"); return e && e[0] == '0'; }();
-    if (off || ta != PM_Q4_K || (tb != PM_Q6_K && tb != PM_Q5_K) || na < 1 || na > 3 || T < 1 || T > (tb == PM_Q5_K ? 16 : 32)) return -5;
+    if (off || ta != PM_Q4_K || (tb != PM_Q6_K && tb != PM_Q5_K) || na < 1 || na > 2 || T < 1 || T > (tb == PM_Q5_K ? 16 : 32)) return -5;
     long total = 0;
     for (int j = 0; j < na; ++j) { if (pm_mmq_i8_check(ta, K, Na[j], T)) return -5; total += Na[j]; }
     if (pm_mmq_i8_check(tb, K, Nb, T)) return -5;
@@ -963,65 +638,14 @@ int pm_launch_mmq_i8_dual(int ta, int na, const void * const * Wa, const int * N
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 16) return -3;
     const int nsb = K / 256;
-    const size_t xrow = pm_q8k_row_bytes(K);
     const Scr * sc = scratch(dev, st, K, reuse_prep != 0);
     if (!sc) return -3;
     if (!reuse_prep) launch_prep(sc, xq, K, T, st);
-    if (T <= 8 && na <= 2 && pm_mmq_rows_takes(ta, total + Nb, K, T, PM_ROWS_MIXED)) {
-        RowsP q = {};
-        int ty[3];
-        q.njobs = na + 1; q.K = K; q.T = T; q.bsT = sc->p; q.dT = (const float *) (sc->p + (size_t) nsb * 1024); q.qT = sc->p + scr_q_off(K);
-        for (int j = 0; j < na; ++j) { q.job[j] = {(const uint8_t *) Wa[j], Ya[j], ba ? ba[j] : nullptr, nullptr, Na[j]}; ty[j] = ta; }
-        q.job[na] = {(const uint8_t *) Wb, Yb, bb, nullptr, Nb}; ty[na] = tb;
-        if (!fill_epi(q, epi)) return -5;
-        return pm_launch_mmq_rows(q, ty, st);
-    }
-    const int cus = pm_device_cus();
-    const double bytes_a = (double) total * pm_weight_row_stride(ta, K), bytes_b = (double) Nb * pm_weight_row_stride(tb, K);
-    int gb = (int) (cus * bytes_b / (bytes_a + bytes_b) + 0.5);
-    gb = gb < 1 ? 1 : gb;
-    if (gb > (Nb + 31) / 32) gb = (Nb + 31) / 32;
-    int ga = cus - gb;
-    if (ga > (int) ((total + 31) / 32)) ga = (int) ((total + 31) / 32);
-    if (ga < 1) return -5;
-    MmqP2 pp = {};
-    {
-        MmqP & p = pp.a;
-        p.row_stride = (long) pm_weight_row_stride(ta, K); p.N = (int) total; p.K = K; p.T = T;
-        p.xq = (const uint8_t *) xq; p.xq_stride = (long) xrow; p.bsT = sc->p; p.dT = (const float *) (sc->p + (size_t) nsb * 1024); p.qT = sc->p + scr_q_off(K);
-        p.njobs = na;
-        int at = 0;
-        for (int j = 0; j < 3; ++j) {
-            const int jj = j < na ? j : na - 1;
-            p.Wj[j] = (const uint8_t *) Wa[jj]; p.yj[j] = Ya[jj]; p.bj[j] = ba ? ba[jj] : nullptr; p.nj[j] = Na[jj];
-            p.start[j] = j < na ? at : (int) total;
-            if (j < na) at += Na[j];
-        }
-        const int rows = (int) ((total + ga - 1) / ga);
-        p.rgb_log2 = rgb_log2_for((rows + 31) / 32);
-    }
-    {
-        MmqP & p = pp.b;
-        p.W = (const uint8_t *) Wb; p.row_stride = (long) pm_weight_row_stride(tb, K); p.N = Nb; p.K = K; p.T = T;
-        p.xq = (const uint8_t *) xq; p.xq_stride = (long) xrow; p.bsT = pp.a.bsT; p.dT = pp.a.dT; p.qT = pp.a.qT;
-        p.y = Yb; p.y_stride = Nb; p.bias = bb;
-        p.njobs = 1;
-        for (int j = 0; j < 3; ++j) { p.Wj[j] = p.W; p.yj[j] = Yb; p.bj[j] = bb; p.nj[j] = Nb; p.start[j] = j == 0 ? 0 : Nb; }
-        const int rows = (Nb + gb - 1) / gb;
-        p.rgb_log2 = rgb_log2_for((rows + 31) / 32);
-    }
-    pp.ga = ga;
-    if (!fill_epi(pp.a, epi, 1, 2, 0) || !fill_epi(pp.b, epi, 3, 0, 0)) return -5;
-    const size_t la = pm_mmq_i8_lds_bytes(ta, K), lb = pm_mmq_i8_lds_bytes(tb, K), lds = la > lb ? la : lb;
-    auto go = [&](auto kern) {
-        pm_allow_big_lds((const void *) kern, 150 * 1024);
-        hipLaunchKernelGGL(kern, dim3(ga + gb), dim3(BLOCK), lds, st, pp);
-    };
-    if (epi) {
-        if (tb == PM_Q6_K) { if (T <= 8) go(mmq_i8_dual_kernel<PM_Q4_K, PM_Q6_K, 4, true>); else if (T <= 16) go(mmq_i8_dual_kernel<PM_Q4_K, PM_Q6_K, 8, true>); else go(mmq_i8_dual_kernel<PM_Q4_K, PM_Q6_K, 16, true>); }
-        else               { if (T <= 8) go(mmq_i8_dual_kernel<PM_Q4_K, PM_Q5_K, 4, true>); else go(mmq_i8_dual_kernel<PM_Q4_K, PM_Q5_K, 8, true>); }
-    }
-    else if (tb == PM_Q6_K) { if (T <= 8) go(mmq_i8_dual_kernel<PM_Q4_K, PM_Q6_K, 4>); else if (T <= 16) go(mmq_i8_dual_kernel<PM_Q4_K, PM_Q6_K, 8>); else go(mmq_i8_dual_kernel<PM_Q4_K, PM_Q6_K, 16>); }
-    else               { if (T <= 8) go(mmq_i8_dual_kernel<PM_Q4_K, PM_Q5_K, 4>); else go(mmq_i8_dual_kernel<PM_Q4_K, PM_Q5_K, 8>); }
-    return 0;
+    RowsP q = {};
+    int ty[3];
+    q.njobs = na + 1; q.K = K; q.T = T; q.bsT = sc->p; q.dT = (const float *) (sc->p + (size_t) nsb * 1024); q.qT = sc->p + scr_q_off(K);
+    for (int j = 0; j < na; ++j) { q.job[j] = {(const uint8_t *) Wa[j], Ya[j], ba ? ba[j] : nullptr, nullptr, Na[j]}; ty[j] = ta; }
+    q.job[na] = {(const uint8_t *) Wb, Yb, bb, nullptr, Nb}; ty[na] = tb;
+    if (!fill_epi(q, epi)) return -5;
+    return T <= 8 && pm_mmq_rows_takes(ta, total + Nb, K, T, PM_ROWS_MIXED) ? pm_launch_mmq_rows(q, ty, st) : pm_launch_mmq_mid(q, ty, st);
 }

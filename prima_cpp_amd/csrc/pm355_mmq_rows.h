@@ -1,4 +1,4 @@
-// pm355_mmq_rows.h - launch of the quantized mat-mul of few tokens (mmq_rows.hip) on activation tables that are already written
+// pm355_mmq_rows.h - launches of the quantized mat-mul of few tokens (mmq_rows.hip, mmq_mid.hip) on activation tables that are already written
 #pragma once
 #include "pm355_device.h"
 #include "pm355_kernels.h"
@@ -19,3 +19,5 @@ enum { PM_ROWS_ONE, PM_ROWS_SEVERAL, PM_ROWS_MIXED };               // one matri
 // whether a pass over T tokens of N rows in all is one for it (else mmq_i8.hip's kernels); type: of the first matrix
 bool pm_mmq_rows_takes(int type, long N, int K, int T, int form = PM_ROWS_ONE);
 int pm_launch_mmq_rows(RowsP p, const int * types, hipStream_t st);
+// mmq_mid.hip: one or several matrices of one K (types[0]; only the last may be of another type) over 1..32 tokens; -5: not served
+int pm_launch_mmq_mid(RowsP p, const int * types, hipStream_t st);

@@ -1591,3 +1591,33 @@ def test_single_token_attention_over_few_cells_keeps_its_sums(P, dh, n_ctx, n_kv
         assert np.abs(out[h] - v[h // 3] @ p).max() <= (2.0 ** -11 + 1e-5) * (np.abs(v[h // 3]) @ p).max() + 2.0 ** -25 * n_kv * np.abs(v).max()
     want = np.load(os.path.join(os.path.dirname(os.path.abspath(__file__)), "golden", "attn_short.npz"))[f"{dh}_{n_ctx}_{n_kv}_{mask}"]
     assert np.array_equal(out.view(np.uint32), want.view(np.uint32)), np.abs(out - want).max()
+
+
+@pytest.mark.parametrize("t", [Q4_K, Q5_K, Q6_K, Q8_0])
+def test_small_batch_cells_at_their_edges(P, oracle, t):
+    """mmq_mid.hip: one step per round and several, pairs that do not divide among the cells, odd super-blocks, blocks of 32 that end inside a pair; up to 32, 33..64 and more rows per workgroup
+    (one, two and four row groups at a time), a group of one row, a cell without rows, several rounds, blocks of scales that reach into the next round; 8, 16, 24 and 32 tokens and one more.
+    Against the oracle: the same integers, <= K / 256 (Q8_0: K / 32) f32 terms in another order - the bound of the other small-batch products."""
+    rng = np.random.default_rng(8100 + t)
+    tail = 32 if t == Q8_0 else 256
+    for K, N, T in ((4352, 4097, 17), (4608, 8193, 20), (8192 + tail, 8230, 25), (5120, 16385, 24), (4096 + tail, 16500, 32), (5120 + tail, 20000, 17), (512, 33000, 9), (1024, 40000, 25), (2560, 41000, 20), (4608, 33100, 28),
+                    (2048, 70, 25), (768, 5000, 12), (12288 + tail, 4200, 18), (5120, 50000, 16), (4864, 33000, 8)):
+        b = rand_blocks(t, N, K, rng)
+        x = rng.normal(0, 1, (T, K)).astype(np.float32)
+        bias, resid = rng.normal(0, 1, N).astype(np.float32), rng.normal(0, 1, (T, N)).astype(np.float32)
+        w = P.upload_weight(t, b, K, N)
+        rows = np.unique(np.concatenate([np.arange(min(N, 40)), np.arange(max(N - 40, 0), N), rng.integers(0, N, 120)]))   # (the oracle is a scalar program)
+        want = oracle.mul_mat(t, b.reshape(N, b.size // N)[rows].copy(), K, len(rows), x)
+        tol = dict(rtol=2e-5, atol=2e-5 * np.sqrt(max(K, 4096) / 4096))
+        y = P.mul_mat_small(w, x=_dev(P, x)).cpu().numpy()
+        assert np.isfinite(y).all(), (K, N, T)
+        assert np.allclose(y[:, rows], want, **tol), (K, N, T, np.abs(y[:, rows] - want).max())
+        xq = P.quantize_act(_dev(P, x), P.vec_dot_act_type(t))
+        y2 = P.mul_mat_small(w, xq=xq, n_tokens=T, bias=_dev(P, bias), resid=_dev(P, resid)).cpu().numpy()
+        assert np.array_equal(y2, (y + bias[None]) + resid), (K, N, T)
+        if t in (Q4_K, Q6_K) and N > 5000:                         # two matrices share the workgroups
+            n0 = N // 2 + 13
+            rb = b.size // N
+            ws = [P.upload_weight(t, b.reshape(N, rb)[:n0], K, n0), P.upload_weight(t, b.reshape(N, rb)[n0:], K, N - n0)]
+            y3 = np.concatenate([v.cpu().numpy() for v in P.mul_mat_small_multi(ws, xq, T)], axis=1)
+            assert np.allclose(y3[:, rows], want, **tol), (K, N, T, np.abs(y3[:, rows] - want).max())
