@@ -41,6 +41,12 @@ template <> struct Frag<float> {
     }
 };
 
+__device__ __forceinline__ uint32_t wave_or(uint32_t v) {
+    v |= (uint32_t) dpp_i<0xB1>((int) v); v |= (uint32_t) dpp_i<0x4E>((int) v); v |= (uint32_t) dpp_i<0x141>((int) v); v |= (uint32_t) dpp_i<0x140>((int) v);
+    v |= other_row(v);
+    return (uint32_t) __builtin_amdgcn_readfirstlane((int) (v | other_half(v)));
+}
+
 // x + norm(y) of token wave / (8 / TP) in VP values per lane: everything the rows need is requested before the first weights (loads return in order), the sums run
 // while those are on their way. Result -> LDS (T, stride ldl) and, from workgroup 0, the residual stream.
 template <typename T, int TP> struct AddNorm {
@@ -127,25 +133,48 @@ template <typename T, int NT, int RM, int SRC, int EXP> __global__ __launch_boun
         __shared__ int ids[64]; __shared__ float w[64];
         const int top = p.r.top, t = blockIdx.y / top, k = blockIdx.y % top;
         if (wave == 0) {
-            route_token(p.r.logits + (size_t) t * p.r.ldl, p.r.E, top, p.r.groups, p.r.keep, (float *) smem, (float *) smem + 1024, ids, w);
-            if (blockIdx.x == 0 && k == 0 && lane < top) { p.r.id[t * top + lane] = ids[lane]; p.r.w[t * top + lane] = w[lane]; }
+            if (p.r.logits) {
+                route_token([&](int e) { return ld_g(p.r.logits + (size_t) t * p.r.ldl + e); }, p.r.E, top, p.r.groups, p.r.keep, (float *) smem, (float *) smem + 1024, ids, w);
+                if (blockIdx.x == 0 && k == 0 && lane < top) { p.r.id[t * top + lane] = ids[lane]; p.r.w[t * top + lane] = w[lane]; }
+            } else if (lane == k) { ids[k] = ld_g(p.r.id + blockIdx.y); w[k] = ld_g(p.r.w + blockIdx.y); }
         }
         __syncthreads();
         W += (size_t) __builtin_amdgcn_readfirstlane(ids[k]) * p.e_stride;
         weight = w[k]; base = blockIdx.y; act += (size_t) t * p.lda; t0 = 0; n_tok = 1;
     }
     if constexpr (EXP == CONCAT) { const int t = blockIdx.y; cat = uniform_const_ptr(p.r.id + t * p.r.top); base = t; act += (size_t) t * p.lda; t0 = 0; n_tok = 1; }
+    __shared__ int local[EXP == SORTED ? 64 : 1];          // SORTED without tables: the expert's pairs
     if constexpr (EXP == SORTED) {
-        if ((int) blockIdx.y >= ld_g(p.r.active)) return;
-        const int e = __builtin_amdgcn_readfirstlane(ld_g(p.r.active + 1 + blockIdx.y));
-        base = __builtin_amdgcn_readfirstlane(ld_g(p.r.off + e)); n_tok = __builtin_amdgcn_readfirstlane(ld_g(p.r.off + e + 1)) - base;
+        int e;
+        if (p.r.logits) {
+            if ((int) blockIdx.y >= ld_g(p.r.active)) return;
+            e = __builtin_amdgcn_readfirstlane(ld_g(p.r.active + 1 + blockIdx.y));
+            base = __builtin_amdgcn_readfirstlane(ld_g(p.r.off + e)); n_tok = __builtin_amdgcn_readfirstlane(ld_g(p.r.off + e + 1)) - base;
+        } else {
+            // up to 64 pairs of up to 64 experts: a lane per pair, this workgroup's expert is the blockIdx.y-th that has one. (One load in front of the weights instead of three, one behind the
+            // other, and no launch that sorts; every wave finds the same)
+            const bool pair = lane < p.T * p.r.top;
+            const int mine = pair ? ld_g(p.r.id + lane) : p.r.E;
+            uint32_t has[2] = {pair && mine < 32 ? 1u << mine : 0u, pair && mine >= 32 ? 1u << (mine - 32) : 0u};
+#pragma unroll
+            for (int i = 0; i < 2; ++i) has[i] = wave_or(has[i]);
+            const uint64_t on = (uint64_t) has[1] << 32 | has[0];
+            if ((int) blockIdx.y >= __popcll(on)) return;
+            e = __builtin_ctzll(__builtin_amdgcn_ballot_w64((on >> lane & 1) && __popcll(on & ((1ull << lane) - 1)) == (int) blockIdx.y));
+            const uint64_t its = __builtin_amdgcn_ballot_w64(mine == e);
+            base = __popcll(__builtin_amdgcn_ballot_w64(mine < e)); n_tok = __popcll(its);
+            if (its >> lane & 1) local[__popcll(its & ((1ull << lane) - 1))] = lane;
+            wave_fence();
+        }
         W += (size_t) e * p.e_stride; t0 = 0;
     }
+    // sorted pair base + t
+    auto pair_at = [&](int t) __attribute__((always_inline)) -> int { return EXP == SORTED && !p.r.logits ? local[t] : ld_g(p.r.order + base + t); };
     if (EXP == DENSE && p.group) act += (size_t) (r0 / p.group) * p.g_act;
     // activation row of the tile's token t (< n_tok)
     auto row_in = [&](int t) __attribute__((always_inline)) -> const T * {
         if constexpr (EXP == PAIR || EXP == CONCAT) return act;
-        if constexpr (EXP == SORTED) return act + (size_t) (p.in_sorted ? base + t : ld_g(p.r.order + base + t) / p.r.top) * p.lda;
+        if constexpr (EXP == SORTED) return act + (size_t) (p.in_sorted ? base + t : pair_at(t) / p.r.top) * p.lda;
         return act + (size_t) t * p.lda;
     };
     const int nb1 = p.K >> 6, nblk = EXP == CONCAT ? nb1 * p.r.top : nb1, mine = (nblk - wave + 7) >> 3;      // 64-k blocks wave, wave + 8, ..
@@ -294,7 +323,7 @@ template <typename T, int NT, int RM, int SRC, int EXP> __global__ __launch_boun
         if constexpr (EXP == PAIR) { v *= weight; tok = base; }
         if constexpr (EXP == CONCAT) tok = base;
         if constexpr (EXP == SORTED) {
-            const int pair = ld_g(p.r.order + base + tok);
+            const int pair = pair_at(tok);
             if (p.weigh) v *= ld_g(p.r.w + pair);
             tok = p.out_sorted ? base + tok : pair;
         }

@@ -133,7 +133,8 @@ void pm_launch_latent_spread(const pm_latent_expand & e, hipStream_t st);       
 // experts (moe.hip, dense_*.hip). Routing of T tokens: softmax over E logits, the `keep` best of `groups` groups of neighbours (by their largest score), the `top` largest
 // scores among these, not renormalized
 struct pm_route {
-    const float * logits; int ldl, E, top, groups, keep;
+    const float * logits;                   // (null: id and w are there, nothing else is: pm_launch_route_stream)
+    int ldl, E, top, groups, keep;
     int32_t * id; float * w;                // [T * top] expert and weight per (token, slot)
     int32_t * pos;                          // [T * top] place among the expert's pairs
     int32_t * count;                        // [E] cleared by the embedding launch
@@ -147,6 +148,10 @@ struct pm_route {
 static inline int pm_expert_tile(int64_t pairs, int E) { return pairs >= 384 * (int64_t) E ? 256 : 128; }
 constexpr int PM_ROUTE_PAIR_MAX = 4, PM_ROUTE_ONE_MAX = 64;      // tokens up to which the pairs go one by one / one workgroup routes and sorts
 void pm_launch_route(const pm_route & r, int T, int want_tiles, hipStream_t st);
+// few tokens, bf16, RMS: x += norm(y), xb = norm(x) (pm_launch_add_norm), the router product W . xb (rows of K values) and r.id, r.w in one; rows of x, y, xb: ld values. The expert products
+// are then called without logits
+bool pm_route_stream_ok(const pm_route & r, const pm_norm_args & q, int K, int T);
+void pm_launch_route_stream(const pm_route & r, const pm_norm_args & q, float * x, const float * y, const void * W, int K, void * xb, int ld, int T, hipStream_t st);
 struct pm_expert_args {
     int type; pm_route r; int T, width_p, ffp, width;             // width_p, ffp: padded row lengths of up and down
     const void * up, * down; int64_t up_stride, down_stride;      // values between experts: [E][ffp][width_p], [E][width_p][ffp]

@@ -770,8 +770,6 @@ int pm_stack::launch(const Step & p, hipStream_t st) {
     auto experts = [&](LayerState & L, int & parts, int & y_type) -> int {
         const pm355_layer_spec & s = L.s;
         const int Ep = L.router.Np, small = ty == PM_F32 || T <= PM_ROUTE_ONE_MAX;
-        int rc = from_stream(L.router, L.pre2, true, rlog, Ep, PM_F32, s.n_expert, nullptr, PM355_ACT_NONE);
-        if (rc) return rc;
         pm_expert_args a{};
         a.type = ty; a.T = T; a.width_p = Wp; a.ffp = L.ffp; a.width = d.n_embd; a.up = L.e_up.d; a.down = L.e_down.d; a.up_stride = (int64_t) L.ffp * Wp; a.down_stride = (int64_t) Wp * L.ffp;
         a.act_fn = s.act; a.x = xb; a.ldx = Wp; a.hid = hid;
@@ -779,7 +777,15 @@ int pm_stack::launch(const Step & p, hipStream_t st) {
         const bool pairs = T <= PM_ROUTE_PAIR_MAX;
         parts = pairs ? 0 : s.n_expert_used; y_type = small ? PM_F32 : PM_BF16;
         a.y = pairs ? (void *) y : yrows; a.ldy = Wp; a.y_type = y_type;
-        if (!pairs) pm_launch_route(a.r, T, !small, st);
+        const pm_norm_args nq{rms, pend.w, pend.b, L.pre2, d.norm_eps, d.n_embd, pend.type, pend.parts, true};
+        if (!plain && ty == PM_BF16 && pend.on && pm_route_stream_ok(a.r, nq, L.router.Kp, T)) {
+            pm_launch_route_stream(a.r, nq, x[cur], y, L.router.d, L.router.Kp, xb, Wp, T, st);
+            pend.on = false; a.r.logits = nullptr;
+        } else {
+            const int rc = from_stream(L.router, L.pre2, true, rlog, Ep, PM_F32, s.n_expert, nullptr, PM355_ACT_NONE);
+            if (rc) return rc;
+            if (!pairs) pm_launch_route(a.r, T, !small, st);
+        }
         return small ? pm_launch_experts_small(a, st) : pm_launch_experts_gemm(a, st);
     };
 
