@@ -1,9 +1,9 @@
-// dense_gemm.hip — y[t][n] = act(W[n] . x[t] + bias) for prompt-sized batches, bf16 x bf16 with f32 accumulation on v_mfma_f32_32x32x16_bf16.
+// dense_gemm.hip — y[t][n] = act(W[n] . x[t] + bias) for prompt-sized batches, bf16 x bf16 with f32 accumulation on the matrix cores.
 // Both operands travel by LDS-DMA as whole 128-byte lines (64 k per stage) into two stages; 16-byte chunks are XOR-swizzled on the source side (chunk c of row r at
 // c ^ ((r >> 1) & 7): the sixteen lanes a ds_read_b128 serves hit sixteen bank groups). One barrier per stage: behind it the stage of the previous step is free and takes
-// the next k-step's DMA, which has this step's MFMAs to land. Tiles 256 x 256 (eight waves, 128 tokens x 64 rows each) or 128 x 128 (four waves, 64 x 64), chosen by how
-// many rounds the grid takes; tiles of one XCD form compact blocks of the output so that its L2 serves both operands.
-// The same loop multiplies experts (token tiles from the routing tables, rows gathered and scattered by pair) and expands latent cache pages into keys and transposed values.
+// the next k-step's DMA, which has this step's MFMAs to land. Tiles of one XCD form compact blocks of the output so that its L2 serves both operands.
+// dense_tile_kernel: one matrix, tiles of 128 .. 256 tokens x 128 or 256 rows, chosen by the time their rounds take. dense_gemm_kernel: two 128 x 128 tiles per CU where that is the quickest; experts
+// (token tiles of 128 or 256 from the routing tables, rows gathered and scattered by pair); latent cache pages into keys and transposed values.
 #include "pm355_dense.h"
 #include "pm355_kernels.h"
 #include "../../include/prima_mi355.h"
@@ -19,7 +19,7 @@ struct GemmP {
     const int32_t * tiles, * order; const float * weight; int64_t e_stride; int top, gather, scatter;
     // KEYS: X rows are those of cache pages; VALUES: the rows of W are (tokens become the columns of the output)
     const int32_t * pages; int H, per, rows_h, pad;              // heads, values per head, rows of W per head, padded head size of the output
-    int splits, split_steps;                                     // DENSE: k ranges of so many 64-k steps; with more than one, y = f32 sums [splits][T][ldy] (reduce_kernel)
+    int splits, split_steps, rows;                               // dense_tile_kernel: k ranges of so many 64-k steps; with more than one, y = f32 sums [splits][T][ldy] (reduce_kernel), or [T][splits][ldy] (rows)
 };
 
 template <int N> __device__ __forceinline__ void vm_wait() { asm volatile("s_waitcnt vmcnt(%0)" :: "n"(N) : "memory"); }
@@ -31,11 +31,9 @@ template <int BM, int BN, int WM, int WN, int STAGES, int KIND> __global__ __lau
     const int wm = wave / (BN / WN), wn = wave % (BN / WN);
     // tile order: XCD x = blockIdx % 8 takes a contiguous run of tiles; runs walk blocks of 8 token tiles column by column
     const int nt = KIND == EXPERTS ? __builtin_amdgcn_readfirstlane(ld_g(p.tiles)) : p.nt;      // (the grid has room for the most tiles there can be)
-    const int tiles = nt * p.nn, total = KIND == DENSE ? tiles * p.splits : tiles, per = (total + 7) / 8;
-    int slot = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
+    const int total = nt * p.nn, per = (total + 7) / 8;
+    const int slot = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
     if (slot >= total || (int) (blockIdx.x >> 3) >= per) return;
-    const int split = KIND == DENSE ? slot / tiles : 0;
-    slot -= split * tiles;
     const int band = slot / (8 * p.nn), left = nt - band * 8, bh = left < 8 ? left : 8, in = slot - band * 8 * p.nn;
     int t0 = (band * 8 + in % bh) * BM, n_tok = p.T;
     const int n0 = (in / bh) * BN;
@@ -70,10 +68,9 @@ template <int BM, int BN, int WM, int WN, int STAGES, int KIND> __global__ __lau
             off[i] = (uint32_t) (lane >> 3) * (uint32_t) p.lda * 2u + swz;
         } else off[i] = (uint32_t) row * pitch + swz;
     }
-    const int k0 = KIND == DENSE ? split * p.split_steps : 0;
     auto request = [&](int k, int stage) __attribute__((always_inline)) {
 #pragma unroll
-        for (int i = 0; i < PIECES; ++i) pm_dma16((KIND >= KEYS && paged ? pbase[i] : base) + (size_t) (k0 + k) * 128, off[i], lds0 + (uint32_t) stage * STAGE + (uint32_t) i * 1024u);
+        for (int i = 0; i < PIECES; ++i) pm_dma16((KIND >= KEYS && paged ? pbase[i] : base) + (size_t) k * 128, off[i], lds0 + (uint32_t) stage * STAGE + (uint32_t) i * 1024u);
     };
     f32x16 acc[MI][NI];
 #pragma unroll
@@ -91,7 +88,7 @@ template <int BM, int BN, int WM, int WN, int STAGES, int KIND> __global__ __lau
     float bias[NI];
 #pragma unroll
     for (int n = 0; n < NI; ++n) { const int col = n0 + wn * WN + n * 32 + lr; bias[n] = KIND == DENSE && p.bias && col < p.n_store ? ld_g(p.bias + col) : 0.0f; }
-    const int steps = KIND == DENSE && p.split_steps < (p.K >> 6) - k0 ? p.split_steps : (p.K >> 6) - k0;
+    const int steps = p.K >> 6;
 #pragma unroll
     for (int i = 0; i < STAGES - 1; ++i) if (i < steps) request(i, i);
     for (int k = 0; k < steps; ++k) {
@@ -195,7 +192,7 @@ template <int BM, int BN, int WM, int WN, int STAGES, int KIND> __global__ __lau
                     float w = 1.0f;
                     int tok = t0 + in;
                     if constexpr (KIND == EXPERTS) { w = s_weight[in]; tok = s_pair[in]; }
-                    auto * row = y + (size_t) (KIND == DENSE ? split * p.T + tok : tok) * p.ldy + n0 + wn * WN + lr;
+                    auto * row = y + (size_t) tok * p.ldy + n0 + wn * WN + lr;
 #pragma unroll
                     for (int n = 0; n < NI; ++n)
                         if (whole || n0 + wn * WN + n * 32 + lr < p.n_store) st_g(row + n * 32, from_f<std::remove_reference_t<decltype(*y)>>(KIND == EXPERTS ? acc[m][n][e] * w : acc[m][n][e]));
@@ -205,6 +202,130 @@ template <int BM, int BN, int WM, int WN, int STAGES, int KIND> __global__ __lau
         if (p.y_type == PM_BF16) { if (whole) put((uint16_t *) p.y, true); else put((uint16_t *) p.y, false); }
         else { if (whole) put((float *) p.y, true); else put((float *) p.y, false); }
     }
+}
+
+// One matrix over many tokens: tiles of 32 MI tokens x 64 NI rows, eight waves of 16 MI x 16 NI, so that tiles can be cut to what a batch has (835 tokens are 3.3 tiles of 256 and 3.7 of 224, and
+// 10240 rows 40 tiles of 256 - 160 workgroups - and 54 of 192). v_mfma_f32_16x16x32_bf16 (the rate of 32 x 32 x 16 per bit of operand): rows of W are the tile's rows, so that a lane holds
+// four neighbouring outputs of a token and stores them together. Both operands by LDS-DMA as in the kernel above, as many stages as fit, up to four.
+// What bounds it: a step of 64 k of a 256 x 256 tile takes 1.65 us - its products and the LDS reads for them 1.4, its lines from the L2s 1.45 beside that -, in proportion to the tile's area.
+template <int MI, int NI> struct Tile { static constexpr int BM = 32 * MI, BN = 64 * NI, STAGE = (BM + BN) * 128, STAGES = 4 * STAGE <= 160 * 1024 ? 4 : 3 * STAGE <= 160 * 1024 ? 3 : 2; };
+template <int MI, int NI> __global__ __launch_bounds__(512) void dense_tile_kernel(GemmP p) {
+    typedef Tile<MI, NI> S;
+    constexpr int BM = S::BM, BN = S::BN, STAGE = S::STAGE, STAGES = S::STAGES, ALL = (BM + BN) / 8, PIECES = (ALL + 7) / 8;
+    extern __shared__ __attribute__((aligned(1024))) char smem[];
+    const int wave = __builtin_amdgcn_readfirstlane((int) threadIdx.x >> 6), lane = threadIdx.x & 63, lr = lane & 15, g = lane >> 4;
+    const int wm = wave >> 2, wn = wave & 3;
+    const int tiles = p.nt * p.nn, total = tiles * p.splits, per = (total + 7) / 8;         // (order of the tiles: as above)
+    int slot = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
+    if (slot >= total || (int) (blockIdx.x >> 3) >= per) return;
+    const int split = slot / tiles;
+    slot -= split * tiles;
+    const int band = slot / (8 * p.nn), left = p.nt - band * 8, bh = left < 8 ? left : 8, in = slot - band * 8 * p.nn;
+    const int t0 = (band * 8 + in % bh) * BM, n0 = (in / bh) * BN, k0 = split * p.split_steps;
+    const int steps = p.split_steps < (p.K >> 6) - k0 ? p.split_steps : (p.K >> 6) - k0;
+    // pieces of 8 rows x 128 bytes, wave, wave + 8, .. (a wave without a last one brings the last one again: the same bytes to the same place)
+    const char * xb = (const char *) (p.X + (size_t) t0 * p.lda), * wb = (const char *) (p.W + (size_t) n0 * p.K);
+    const int x_last = p.T - 1 - t0, w_last = p.N - 1 - n0;
+    const uint32_t lds0 = (uint32_t) (uintptr_t) (__attribute__((address_space(3))) char *) smem;
+    uint32_t off[PIECES];
+#pragma unroll
+    for (int i = 0; i < PIECES; ++i) {
+        const int q = min(wave + 8 * i, ALL - 1), r = q * 8 + (lane >> 3);
+        const bool tok = q < BM / 8;
+        const int row = tok ? min(r, x_last) : min(r - BM, w_last);
+        off[i] = (uint32_t) row * (uint32_t) (tok ? p.lda : p.K) * 2u + (uint32_t) ((lane & 7) ^ ((r >> 1) & 7)) * 16u;
+    }
+    auto request = [&](int k, int stage) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < PIECES; ++i) {
+            const int q = min(wave + 8 * i, ALL - 1);
+            pm_dma16((q < BM / 8 ? xb : wb) + (size_t) (k0 + k) * 128, off[i], lds0 + (uint32_t) (stage * STAGE) + (uint32_t) q * 1024u);
+        }
+    };
+    f32x4 acc[NI][MI];
+#pragma unroll
+    for (int n = 0; n < NI; ++n)
+#pragma unroll
+        for (int m = 0; m < MI; ++m) acc[n][m] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    // (rows of one operand's blocks are 16 apart: the swizzle is the lane's own)
+    const uint32_t x_at = (uint32_t) (wm * 16 * MI + lr) * 128u, w_at = (uint32_t) (BM + wn * 16 * NI + lr) * 128u, sw = (uint32_t) (lr >> 1) & 7u;
+#pragma unroll
+    for (int i = 0; i < STAGES - 1; ++i) if (i < steps) request(i, i);
+    int stage = 0, next = STAGES - 1;
+    for (int k = 0; k < steps; ++k) {
+        const int ahead = steps - 1 - k;                   // (as in the kernel above)
+        if (STAGES > 2 && ahead >= STAGES - 2) vm_wait<PIECES * (STAGES - 2)>();
+        else if (STAGES > 3 && ahead == 1) vm_wait<PIECES>();
+        else vm_wait<0>();
+        __syncthreads();
+        if (k + STAGES - 1 < steps) request(k + STAGES - 1, next);
+        const char * s = smem + stage * STAGE;
+        bf16x8 x[2][MI], w[2][NI];
+        auto read = [&](int j) __attribute__((always_inline)) {                  // 32 k of the stage
+            const uint32_t c = ((uint32_t) (j * 4 + g) ^ sw) * 16u;
+#pragma unroll
+            for (int n = 0; n < NI; ++n) w[j][n] = *(const bf16x8 *) (s + w_at + n * 2048 + c);
+#pragma unroll
+            for (int m = 0; m < MI; ++m) x[j][m] = *(const bf16x8 *) (s + x_at + m * 2048 + c);
+        };
+        read(0);
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            if (j == 0) read(1);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int m = 0; m < MI; ++m)
+#pragma unroll
+                for (int n = 0; n < NI; ++n) acc[n][m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[j][n], x[j][m], acc[n][m], 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        stage = stage == STAGES - 1 ? 0 : stage + 1;
+        next = next == STAGES - 1 ? 0 : next + 1;
+    }
+    f32x4 bias[NI];
+#pragma unroll
+    for (int n = 0; n < NI; ++n)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) { const int col = n0 + (wn * NI + n) * 16 + g * 4 + e; bias[n][e] = p.bias && split == 0 && col < p.n_store ? ld_g(p.bias + col) : 0.0f; }
+#pragma unroll
+    for (int n = 0; n < NI; ++n) asm volatile("" : "+v"(bias[n]));
+    auto put = [&](auto * y, bool whole) __attribute__((always_inline)) {
+        typedef std::remove_reference_t<decltype(*y)> Y;
+#pragma unroll
+        for (int m = 0; m < MI; ++m) {
+            const int tok = t0 + (wm * MI + m) * 16 + lr;
+            if (tok >= p.T) continue;
+            Y * row = y + (p.rows ? (size_t) tok * p.splits + split : (size_t) split * p.T + tok) * p.ldy + n0 + wn * 16 * NI + g * 4;
+#pragma unroll
+            for (int n = 0; n < NI; ++n) {
+                f32x4 v = acc[n][m] + bias[n];
+                if (p.act_fn) {
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) v[e] = act_apply(p.act_fn, v[e]);
+                }
+                if (whole) {
+                    if constexpr (sizeof(Y) == 4) *(PM_G f32x4 *) (row + n * 16) = v;
+                    else *(PM_G u32x2 *) (row + n * 16) = u32x2{(uint32_t) f2bf(v[0]) | (uint32_t) f2bf(v[1]) << 16, (uint32_t) f2bf(v[2]) | (uint32_t) f2bf(v[3]) << 16};
+                } else {
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) if (n0 + (wn * NI + n) * 16 + g * 4 + e < p.n_store) st_g(row + n * 16 + e, from_f<Y>(v[e]));
+                }
+            }
+        }
+    };
+    // (four outputs together where rows and their start allow it)
+    const bool whole = n0 + BN <= p.n_store && p.ldy % 4 == 0 && ((uintptr_t) p.y & 15) == 0;
+    if (p.y_type == PM_BF16) { if (whole) put((uint16_t *) p.y, true); else put((uint16_t *) p.y, false); }
+    else { if (whole) put((float *) p.y, true); else put((float *) p.y, false); }
+}
+template <int MI, int NI> int launch_tile(GemmP p, hipStream_t st) {
+    typedef Tile<MI, NI> S;
+    if (p.splits < 1) { p.splits = 1; p.split_steps = p.K >> 6; }
+    p.nt = (p.T + S::BM - 1) / S::BM; p.nn = (p.n_store + S::BN - 1) / S::BN;
+    const size_t lds = (size_t) S::STAGES * S::STAGE;
+    pm_allow_big_lds((const void *) dense_tile_kernel<MI, NI>, lds);
+    hipLaunchKernelGGL((dense_tile_kernel<MI, NI>), dim3((p.nt * p.nn * p.splits + 7) / 8 * 8), dim3(512), lds, st, p);
+    return 0;
 }
 
 // sums of k ranges -> act(sum + bias)
@@ -228,18 +349,17 @@ __global__ __launch_bounds__(256) void reduce_kernel(const float * part, int spl
 
 template <int BM, int BN, int WM, int WN, int STAGES, int KIND> int launch_stages(GemmP p, hipStream_t st) {
     constexpr int threads = BM / WM * (BN / WN) * 64;
-    if (p.splits < 1) { p.splits = 1; p.split_steps = p.K >> 6; }
     if (KIND != EXPERTS) p.nt = (p.T + BM - 1) / BM;
     p.nn = (p.n_store + BN - 1) / BN;
     const size_t lds = (size_t) STAGES * (BM + BN) * 128;
     pm_allow_big_lds((const void *) dense_gemm_kernel<BM, BN, WM, WN, STAGES, KIND>, lds);
-    const int per = (p.nt * p.nn * p.splits + 7) / 8;
+    const int per = (p.nt * p.nn + 7) / 8;
     hipLaunchKernelGGL((dense_gemm_kernel<BM, BN, WM, WN, STAGES, KIND>), dim3(per * 8), dim3(threads), lds, st, p);
     return 0;
 }
 // up to one tile per CU: twice the stages hide the memory's latency; more: two tiles share a CU
 template <int KIND> int launch_128(const GemmP & p, hipStream_t st) {
-    if constexpr (KIND != EXPERTS) if ((long) ((p.T + 127) / 128) * ((p.n_store + 127) / 128) * (p.splits > 1 ? p.splits : 1) <= 256) return launch_stages<128, 128, 64, 64, 4, KIND>(p, st);
+    if constexpr (KIND != EXPERTS) if ((long) ((p.T + 127) / 128) * ((p.n_store + 127) / 128) <= 256) return launch_stages<128, 128, 64, 64, 4, KIND>(p, st);
     return launch_stages<128, 128, 64, 64, 2, KIND>(p, st);
 }
 
@@ -252,20 +372,37 @@ int pm_launch_dense_gemm(const pm_dense_args & a, hipStream_t st) {
     GemmP p = {};
     p.W = (const uint16_t *) a.W; p.X = (const uint16_t *) a.act; p.y = a.y; p.bias = a.bias; p.K = a.K; p.N = a.N; p.T = a.T; p.lda = a.lda; p.ldy = a.ldy; p.y_type = a.y_type;
     p.n_store = a.n_store; p.act_fn = a.act_fn;
-    // rounds of the grid x time of a tile: a 256-tile does four times a 128-tile's work on a whole CU in ~3.4x its time (two 128-tiles share a CU)
-    const long big = (long) ((a.T + 255) / 256) * ((a.n_store + 255) / 256), small = (long) ((a.T + 127) / 128) * ((a.n_store + 127) / 128);
-    // too few tiles for the chip: ranges of k to different workgroups, their sums to scratch
-    const int steps = a.K >> 6, ldp = (a.n_store + 3) / 4 * 4;
-    const int most = steps / 4 < (int) (256 / small) ? steps / 4 : (int) (256 / small);
-    if (a.split && small <= 128 && most > 1 && (size_t) most * a.T * ldp <= a.split_floats) {
-        p.split_steps = (steps + most - 1) / most; p.splits = (steps + p.split_steps - 1) / p.split_steps;
-        p.y = a.split; p.ldy = ldp; p.y_type = PM_F32; p.bias = nullptr; p.act_fn = PM355_ACT_NONE;
-        launch_128<DENSE>(p, st);
+    // The tile whose rounds take the least time: us per 64-k step of a workgroup on a full chip, a CU to itself (two 128 x 128 tiles of the kernel with two stages share one), and what a round
+    // takes besides; half a chip of workgroups runs its steps in 0.77 of that. With too few tiles for the chip ranges of k go to different workgroups; their f32 sums are written and read again.
+    // Measured on 835 tokens, in a pass between other launches: 10240 x 4096 98 us in 160 tiles of 256 x 256, 79 in 240 of 160 x 256; 14336 x 4096 107 (224 of 256 x 256) / 100 (224 of 224 x
+    // 256); 4096 x 14336 135 (224 of 128 x 128, four waves) / 90 and 6 more in the norm behind it (64 of 224 x 256 in four ranges); 4096 x 4096 44 / 41 (128 x 128 tiles by eight waves)
+    const int steps = a.K >> 6, ldp = a.parts ? a.ldy : (a.n_store + 3) / 4 * 4;
+    const bool may_split = a.split && (!a.parts || a.act_fn == PM355_ACT_NONE);
+    static const struct { int bm, bn, per_cu; float step; } forms[] = {{128, 128, 1, 0.63f}, {160, 256, 1, 1.28f}, {224, 256, 1, 1.62f}, {256, 256, 1, 1.77f}, {128, 128, 2, 1.04f}};
+    int form = 0, splits = 1;
+    float best = INFINITY;
+    for (int f = 0; f < 5; ++f) {
+        const int64_t tiles = (int64_t) ((a.T + forms[f].bm - 1) / forms[f].bm) * ((a.n_store + forms[f].bn - 1) / forms[f].bn), room = (int64_t) pm_device_cus() * forms[f].per_cu;
+        for (int s = 1; s == 1 || (f < 4 && may_split && s * tiles <= room && s * 4 <= steps && (size_t) s * a.T * ldp <= a.split_floats); ++s) {
+            const int64_t all = tiles * s, last = all % room;
+            const float rounds = (float) (all / room) + (last ? 0.55f + 0.45f * (float) last / (float) room : 0.0f);      // (in time of a full one's steps)
+            const float t = rounds * (float) ((steps + s - 1) / s) * forms[f].step + (float) ((all + room - 1) / room) * 5.0f + (s > 1 ? (float) s * a.T * ldp * 8 / 4.5e6f + (a.parts ? 0.0f : 5.0f) : 0.0f);
+            if (t < best) { best = t; form = f; splits = s; }
+        }
+    }
+    auto go = [&]() { return form == 0 ? launch_tile<4, 2>(p, st) : form == 1 ? launch_tile<5, 4>(p, st) : form == 2 ? launch_tile<7, 4>(p, st) : form == 3 ? launch_tile<8, 4>(p, st) :
+                             launch_stages<128, 128, 64, 64, 2, DENSE>(p, st); };
+    if (a.parts) *a.parts = 0;
+    if (splits > 1) {
+        p.split_steps = (steps + splits - 1) / splits; p.splits = (steps + p.split_steps - 1) / p.split_steps;
+        p.y = a.split; p.ldy = ldp; p.y_type = PM_F32; p.act_fn = PM355_ACT_NONE;
+        if (a.parts) { *a.parts = p.splits; p.rows = 1; return go(); }
+        p.bias = nullptr;
+        go();
         hipLaunchKernelGGL(reduce_kernel, dim3((unsigned) (((long) a.T * (ldp / 4) + 255) / 256)), dim3(256), 0, st, a.split, p.splits, a.T, ldp, a.bias, a.act_fn, a.y, a.ldy, a.y_type, a.n_store);
         return 0;
     }
-    const double cb = (double) ((big + 255) / 256) * 1.7, cs = (double) ((small + 511) / 512);
-    return cb <= cs ? launch_stages<256, 256, 128, 64, 2, DENSE>(p, st) : launch_128<DENSE>(p, st);
+    return go();
 }
 
 int pm_launch_dense(const pm_dense_args & a, hipStream_t st) {

@@ -636,12 +636,12 @@ int pm_stack::launch(const Step & p, hipStream_t st) {
     const bool fuse = !plain && pm_dense_pro_ok(T, d.n_embd), raw32 = ty == PM_F32 || T <= RAW_F32_MAX, single = !p.n_multi;
     const int raw_type = raw32 ? PM_F32 : PM_BF16;
     int cur = 0;
-    // a sublayer's output whose norm has not joined the residual stream yet: y, or the sum of `parts` rows of yrows per token
-    struct { const float * w, * b; int parts, type; bool on; } pend = {nullptr, nullptr, 0, PM_F32, false};
+    // a sublayer's output whose norm has not joined the residual stream yet: y, or the sum of `parts` rows of src per token (experts, k ranges of a product)
+    struct { const float * w, * b; int parts, type; bool on; const void * src; } pend = {nullptr, nullptr, 0, PM_F32, false, nullptr};
     const int rms = d.norm == PM355_NORM_RMS;
     auto norm_b = [&](float * b) -> const float * { return rms ? nullptr : b; };
     auto settle = [&](const float * pre) {
-        if (pend.on) pm_launch_add_norm(ty, pm_norm_args{rms, pend.w, pend.b, pre, d.norm_eps, d.n_embd, pend.type, pend.parts, true}, x[cur], pend.parts ? yrows : (void *) y, Wp, Wp, T, xb, Wp, st);
+        if (pend.on) pm_launch_add_norm(ty, pm_norm_args{rms, pend.w, pend.b, pre, d.norm_eps, d.n_embd, pend.type, pend.parts, true}, x[cur], pend.parts ? pend.src : y, Wp, Wp, T, xb, Wp, st);
         pend.on = false;
     };
     // W . (residual stream, normed by `pre` where the design norms in front of a sublayer); keep: the activations are read again from xb
@@ -659,13 +659,16 @@ int pm_stack::launch(const Step & p, hipStream_t st) {
         a.act = xb; a.lda = Wp;
         return pm_launch_dense(a, st);
     };
-    auto product = [&](const Mat & m, const void * act, int lda, void * out, int ldo, int otype, int n_store, const float * bias, int rows) {
+    auto product = [&](const Mat & m, const void * act, int lda, void * out, int ldo, int otype, int n_store, const float * bias, int rows, int * parts = nullptr) {
         pm_dense_args a{};
         a.type = ty; a.W = m.d; a.K = m.Kp; a.N = m.Np; a.act = act; a.lda = lda; a.T = rows; a.y = out; a.ldy = ldo; a.y_type = otype; a.n_store = n_store; a.bias = bias;
         a.split = ksplit; a.split_floats = PM_SPLIT_FLOATS;
+        a.parts = ksplit ? parts : nullptr;
         return pm_launch_dense(a, st);
     };
     auto dense = [&](const Mat & m, const void * act, void * out, int ldo, int otype, int n_store, const float * bias, int rows) { return product(m, act, m.Kp, out, ldo, otype, n_store, bias, rows); };
+    int kept = 0;                                           // rows per token of the last sublayer's output where its product left k ranges in ksplit
+    auto to_norm = [&](const Mat & m, const void * act, const float * bias) { kept = 0; return product(m, act, m.Kp, y, Wp, PM_F32, d.n_embd, bias, T, &kept); };
     auto seen_keys = [&](const pm355_layer_spec & s) { return s.mask == PM355_MASK_CAUSAL ? p.keys : std::min(p.keys, s.mask_size + 2 * PM_PAGE); };
 
     auto attention = [&](LayerState & L) -> int {
@@ -687,7 +690,7 @@ int pm_stack::launch(const Step & p, hipStream_t st) {
                 if (!rc && p.n_rows) rc = pm_launch_attn_decode_paged(a, p.b, nullptr, p.n_rows, 0, seen_keys(s), st);
             }
         }
-        return rc ? rc : dense(L.out, a.out, y, Wp, PM_F32, d.n_embd, nullptr, T);
+        return rc ? rc : to_norm(L.out, a.out, nullptr);
     };
 
     auto latent = [&](LayerState & L) -> int {
@@ -744,7 +747,7 @@ int pm_stack::launch(const Step & p, hipStream_t st) {
             rc = pm_launch_attn_tiles(t, p.b, r.tiles, r.n_tiles, st);
             if (rc) return rc;
         }
-        return dense(L.out, out, y, Wp, PM_F32, d.n_embd, nullptr, T);
+        return to_norm(L.out, out, nullptr);
     };
 
     auto ssm = [&](LayerState & L) -> int {
@@ -764,7 +767,7 @@ int pm_stack::launch(const Step & p, hipStream_t st) {
             if (rc) return rc;
             pm_launch_ssm_scan(a, p.b, p.chunks, p.n_chunks, p.multi_chunk, st);
         }
-        return dense(L.out, a.y, y, Wp, PM_F32, d.n_embd, nullptr, T);
+        return to_norm(L.out, a.y, nullptr);
     };
 
     auto experts = [&](LayerState & L, int & parts, int & y_type) -> int {
@@ -798,15 +801,17 @@ int pm_stack::launch(const Step & p, hipStream_t st) {
         const pm355_layer_spec & s = L.s;
         int rc = s.mixer == PM355_MIXER_LATENT ? latent(L) : s.mixer == PM355_MIXER_SSM ? ssm(L) : attention(L);
         if (rc) return fail(rc, "batch: mixer");
-        pend = {L.norm1, norm_b(L.norm1_b), 0, PM_F32, true};
+        pend = {L.norm1, norm_b(L.norm1_b), kept, PM_F32, true, ksplit};
         int parts = 0, y_type = PM_F32;
+        const void * src = yrows;
         if (s.ff == PM355_FF_NONE) continue;
         if (s.ff == PM355_FF_DENSE) {
             rc = from_stream(L.up, L.pre2, false, hb, L.up.Np, ty, L.up.Np, L.up_b, s.act);       // (padding columns: zero weights and bias)
-            if (!rc) rc = dense(L.down, hb, y, Wp, PM_F32, d.n_embd, L.down_b, T);
+            if (!rc) rc = to_norm(L.down, hb, L.down_b);
+            parts = kept; src = ksplit;
         } else rc = experts(L, parts, y_type);
         if (rc) return fail(rc, "batch: feed-forward");
-        pend = {L.norm2, norm_b(L.norm2_b), parts, y_type, true};
+        pend = {L.norm2, norm_b(L.norm2_b), parts, y_type, true, src};
     }
     if (p.n_want) {
         settle(nullptr);

@@ -139,6 +139,27 @@ def test_dense_mul_mat_few_tokens_over_many_rows(T, K, n_store):
         assert (y[:, n_store:] == 7.0).all()
 
 
+# prompts: every tile size (128 x 128 by eight and by four waves, 160, 224 and 256 x 256), a last token tile of one token, rows that end inside a tile and inside four neighbouring outputs, rows
+# of y that do not start on 16 bytes, one k step and fewer than there are stages
+@pytest.mark.parametrize("T,K,n_store,pad", [(65, 64, 100, 0), (129, 192, 33, 3), (300, 1024, 2050, 0), (835, 1024, 10200, 0), (640, 1024, 10239, 1), (835, 1024, 14280, 4), (673, 576, 14334, 0), (1000, 1024, 16001, 0),
+                                             (1025, 1024, 12288, 2), (640, 128, 8190, 0), (897, 1024, 7168, 0)])
+def test_dense_mul_mat_prompt_tiles(T, K, n_store, pad):
+    import prima_cpp_amd.ops as O
+    N = (n_store + 63) // 64 * 64
+    g = torch.Generator(device="cuda").manual_seed(T + K)
+    w = (torch.randn(N, K, generator=g, device="cuda") / K ** 0.5).bfloat16()
+    x = torch.randn(T, K + 64, generator=g, device="cuda").bfloat16()[:, :K]
+    b = torch.randn(N, generator=g, device="cuda")
+    ref = x.double() @ w.double().T
+    for bias, act, ydt in ((None, 0, torch.float32), (b, 1, torch.bfloat16)):
+        y = torch.full((T, N + pad), 7.0, dtype=ydt, device="cuda")
+        O.dense_mul_mat(w, x, y, n_store=n_store, bias=bias, act=act)
+        want = ref if bias is None else (ref + b.double()).clamp(min=0) ** 2
+        tol = 2e-6 * K ** 0.5 if ydt == torch.float32 else 1e-2
+        assert ((y.double()[:, :N] - want)[:, :n_store].abs() <= tol * (1 + want[:, :n_store].abs())).all()
+        assert (y[:, n_store:] == 7.0).all()
+
+
 @pytest.mark.parametrize("T,K,off_x,off_w", [(3, 1024, 4, 0), (8, 4096, 1, 0), (1, 8192, 0, 4), (5, 9216, 2, 2)])
 def test_dense_mul_mat_of_operands_that_do_not_start_on_16_bytes(T, K, off_x, off_w):
     import prima_cpp_amd.ops as O
