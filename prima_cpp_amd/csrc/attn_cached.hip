@@ -13,6 +13,7 @@
 #include "attn_device.h"
 #include "pm355_kernels.h"
 #include "pm355_layer_ops.h"
+#include "pm355_q8k.h"
 #include <algorithm>
 #include <type_traits>
 
@@ -41,8 +42,9 @@ template <int DH, int KPL> struct ShortLds {
 // us per launch of 32 heads of 128 over 36 / 100 / 204 cells: a lane's own key and dimension straight from memory 3.3 / 4.4 / 7.0, this 2.8 / 3.7 / 5.7 (multiplied in the registers that the
 // lines arrive in, sums over lanes, 2.6 / 3.1 / 4.5: one other bit here turns 8-bit roundings behind it, 3 % of the logits of eight layers of the 8B shape).
 // Rounding points as everywhere: q, K, V F16, the normalised probabilities rounded to F16, f32 accumulation. n_kv <= 64 * KPL <= n_ctx; DH 64 / 128 (256: KPL = 1).
-template <int DH, int KPL>
-__device__ __forceinline__ void attn_short(const float * q_head, const uint16_t * kc, const uint16_t * vc, float * out_head, int hk, int Hkv, int n_ctx, int n_kv, float scale, const void * mask,
+// put(d, value): the head's result.
+template <int DH, int KPL, class Put>
+__device__ __forceinline__ void attn_short(const float * q_head, const uint16_t * kc, const uint16_t * vc, Put put, int hk, int Hkv, int n_ctx, int n_kv, float scale, const void * mask,
                                            int mask_f16, char * smem, int lane, int wave, unsigned long long * ts) {
     unsigned long long tsv[6] = {PM_TS_NOW(), 0, 0, 0, 0, 0};
     typedef ShortLds<DH, KPL> S;
@@ -131,7 +133,7 @@ __device__ __forceinline__ void attn_short(const float * q_head, const uint16_t 
     tsv[4] = PM_TS_NOW();                                      // P.V
     if constexpr (DPW <= 16) o += __builtin_bit_cast(float, other_row(__builtin_bit_cast(uint32_t, o)));
     if constexpr (DPW <= 32) o += __builtin_bit_cast(float, other_half(__builtin_bit_cast(uint32_t, o)));
-    if (lane < DPW) st_g(out_head + DPW * wave + lane, o);
+    if (lane < DPW) put(DPW * wave + lane, o);
     tsv[5] = PM_TS_NOW();
     pm_ts_store(ts, 2, tsv);
 }
@@ -158,7 +160,8 @@ __global__ __launch_bounds__(256) void attn_cached_kernel(AttnP a_in) {
         }
         const uint16_t * kc = a.kc + (long) seq * a.seq_stride, * vc = a.vc + (long) seq * a.seq_stride;
         auto go = [&](auto kpl) __attribute__((always_inline)) {
-            attn_short<DH, decltype(kpl)::value>(a.q + (long) h * DH, kc, vc, a.out + (long) h * DH, hk, Hkv, n_ctx, n_kv, a.scale, a.mask, a.mask_f16, smem, lane, wave, a.ts);
+            float * out = a.out + (long) h * DH;
+            attn_short<DH, decltype(kpl)::value>(a.q + (long) h * DH, kc, vc, [&](int d, float v) __attribute__((always_inline)) { st_g(out + d, v); }, hk, Hkv, n_ctx, n_kv, a.scale, a.mask, a.mask_f16, smem, lane, wave, a.ts);
         };
         // (caches that hold fewer cells than the form takes: the general body, as it always was - its sums are in another order)
         if (n_kv <= 64 && n_ctx >= 64) return go(std::integral_constant<int, 1>());
@@ -170,7 +173,41 @@ __global__ __launch_bounds__(256) void attn_cached_kernel(AttnP a_in) {
     attn_rope_body<DH, false, VM, true>(a, h, smem, redf, redd);
 }
 
+// The same for rows of up to 256 cells and two heads of 128 per workgroup, whose results meet in LDS and leave as a Q8_K block (the wo product's activations) - no f32 rows and no launch that
+// quantizes them: 8 sequences of the 8B shape, 4.0 + 3.2 us and the gap between them, now 6.4
+__global__ __launch_bounds__(512) void attn_cached_q8k_kernel(AttnP a, pm_q8k_out y) {
+    extern __shared__ __attribute__((aligned(16))) char smem[];
+    __shared__ __attribute__((aligned(16))) float row[256];
+    const int tid = threadIdx.x, lane = tid & 63, w8 = __builtin_amdgcn_readfirstlane(tid >> 6), half = w8 >> 2, wave = w8 & 3;
+    const int t = blockIdx.y, blk = blockIdx.x, h = 2 * blk + half, hk = h / (a.H / a.Hkv), seq = uniform_const_ptr(a.seq_ptr)[t], n_kv = uniform_const_ptr(a.pos0_ptr)[t] + 1;
+    auto go = [&](auto kpl) __attribute__((always_inline)) {     // (chosen by the row's own cells, as above: the sums do not depend on what else is in the batch)
+        constexpr int KPL = decltype(kpl)::value;
+        attn_short<128, KPL>(a.q + ((long) t * a.H + h) * 128, a.kc + (long) seq * a.seq_stride, a.vc + (long) seq * a.seq_stride, [&](int d, float v) __attribute__((always_inline)) { row[128 * half + d] = v; },
+                             hk, a.Hkv, a.n_ctx, n_kv, a.scale, nullptr, 0, smem + ShortLds<128, KPL>::BYTES * half, lane, wave, nullptr);
+    };
+    if (n_kv <= 64) go(std::integral_constant<int, 1>());
+    else if (n_kv <= 128) go(std::integral_constant<int, 2>());
+    else go(std::integral_constant<int, 4>());
+    __syncthreads();
+    if (w8) return;
+    const f32x4 f = *(const f32x4 *) (row + 4 * lane);
+    const float v[4] = {f[0], f[1], f[2], f[3]};
+    const int K = a.H * 128;
+    q8k_block_from_regs(v, lane, y.y + (size_t) t * y.row_bytes, K, blk, y.tab, t);
+}
+
 } // namespace
+
+int pm_launch_attn_cached_q8k(const float * q, void * kc, void * vc, const int32_t * pos, const int32_t * seq, long seq_stride, int H, int Hkv, int dh, int n_ctx, float scale, hipStream_t st,
+                              int max_cells, int n_tok, const pm_q8k_out & out) {
+    const int kpl = max_cells <= 64 ? 1 : max_cells <= 128 ? 2 : 4;
+    if (dh != 128 || H % 2 || n_ctx % 8 || n_tok < 1 || max_cells < 1 || max_cells > 256 || n_ctx < 64 * kpl || !pos || !seq) return -1;
+    AttnP a = {q, nullptr, nullptr, (uint16_t *) kc, (uint16_t *) vc, pos, seq, seq_stride, nullptr, nullptr, H, Hkv, n_ctx, scale, RopeP(), nullptr, nullptr, 0, nullptr, 0, 1};
+    const size_t lds = 2 * (size_t) (kpl == 1 ? ShortLds<128, 1>::BYTES : kpl == 2 ? ShortLds<128, 2>::BYTES : ShortLds<128, 4>::BYTES);
+    pm_allow_big_lds((const void *) attn_cached_q8k_kernel, lds);
+    hipLaunchKernelGGL(attn_cached_q8k_kernel, dim3(H / 2, n_tok), dim3(512), lds, st, a, out);
+    return 0;
+}
 
 void pm_launch_rope_table(const pm_rope_cfg & c, const int32_t * pos, const int32_t * seq, const float * freq_factors, float * tab, hipStream_t st, int n_tok, int rows) {
     RopeP r;

@@ -14,6 +14,7 @@
 #include "pm355_dense.h"
 #include "pm355_kernels.h"
 #include "pm355_layer_ops.h"
+#include "pm355_q8k.h"
 
 namespace {
 
@@ -223,8 +224,11 @@ __global__ __launch_bounds__(256, 2) void attn_rowmajor_kernel(PfP p) {
 // exponentials beside them. Against the two-pass form with 4 waves x 32 queries, 32-key tiles through registers: 6001 tokens x 32 heads 870 -> 393 us (752 TFLOP/s), 512 x 64 behind
 // 1024 cached cells 102 -> 38, 101 x 32 behind 300 29.8 -> 11.7, 2048 x 32 144 -> 55.
 // PLAIN: caches that do not start on 16 bytes, by loads and LDS stores instead of DMA
-template <int DH, int QW, int KS, bool MASK, bool PLAIN = false>
-__global__ __launch_bounds__(512, 2) void attn_prompt_kernel(PfP p) {
+// PAIR: tiles of up to 32 queries, the two query waves of a key group are two heads of one KV head; their results leave as Q8_K blocks (the wo product's activations) - no f32 rows and no launch that
+// quantizes them: 8 tokens x 64 heads behind 403 cells 11.3 + 5.0 us, now 13.3
+template <int DH, int QW, int KS, bool MASK, bool PLAIN = false, bool PAIR = false>
+__global__ __launch_bounds__(512, 2) void attn_prompt_kernel(PfP p, pm_q8k_out y) {
+    static_assert(!PAIR || (DH == 128 && QW == 2 && !MASK && !PLAIN), "two heads are a block");
     constexpr int KW = 8 / QW, KT = KS / KW, ST = KT / 32;            // keys per wave and stage, 32-key score tiles
     constexpr int KK = DH / 16, DT = DH / 32, CK = DH / 8, CV = KS / 8;      // k-steps of a score tile, output tiles, 16-byte chunks per K row / V^T row
     constexpr int STAGE = KS * DH * 4, OS = DH + 4;
@@ -238,8 +242,10 @@ __global__ __launch_bounds__(512, 2) void attn_prompt_kernel(PfP p) {
     const int qw = wave % QW, kw = wave / QW;
     // an XCD (blockIdx % 8) keeps to its share of the heads: the query heads of a KV head meet in one L2. Tiles with the most keys first: the short ones fill the tail
     int h, tile;
-    if (p.H % 8 == 0) { const int per = p.H / 8, j = blockIdx.x >> 3; h = (blockIdx.x & 7) * per + j % per; tile = j / per; }
-    else { h = blockIdx.x % p.H; tile = blockIdx.x / p.H; }
+    const int n_h = PAIR ? p.H / 2 : p.H;                         // (heads, or pairs of them)
+    if (n_h % 8 == 0) { const int per = n_h / 8, j = blockIdx.x >> 3; h = (blockIdx.x & 7) * per + j % per; tile = j / per; }
+    else { h = blockIdx.x % n_h; tile = blockIdx.x / n_h; }
+    if (PAIR) h = 2 * h + qw;
     tile = p.n_tiles - 1 - tile;
     const int hk = h / (p.H / p.Hkv);
     int row0 = tile * QW * 32, nq = min(QW * 32, p.T - row0), pos0 = 0, seq = 0;                 // the workgroup's first row, its queries, the first one's position
@@ -248,7 +254,7 @@ __global__ __launch_bounds__(512, 2) void attn_prompt_kernel(PfP p) {
     const long krow = (long) p.Hkv * DH;
     const uint16_t * kc = p.kc + (long) seq * p.seq_stride + (long) hk * DH;                     // K[key][Hkv*DH]
     const uint16_t * vc = p.vc + (long) seq * p.seq_stride + (long) hk * DH * p.n_ctx;           // V^T[hk*DH + e][n_ctx]
-    const int q0 = qw * 32, tq0 = row0 + q0;                                                     // first query of this wave: in the workgroup, and its row
+    const int q0 = PAIR ? 0 : qw * 32, tq0 = row0 + q0;                                                     // first query of this wave: in the workgroup, and its row
     const bool live = q0 < nq;
     const int qi = min(q0 + lr, nq - 1), tq = row0 + qi, qpos = pos0 + qi;
     const int w_first = pos0 + q0, w_last = pos0 + min(q0 + 31, nq - 1);                         // positions of the wave's first and last query
@@ -423,6 +429,20 @@ __global__ __launch_bounds__(512, 2) void attn_prompt_kernel(PfP p) {
         for (int g = 0; g < 4; ++g)
             *(float4 *) (ex + (wave * 32 + lr) * OS + d * 32 + 8 * g + 4 * hf) = float4{o[d][4 * g] * f, o[d][4 * g + 1] * f, o[d][4 * g + 2] * f, o[d][4 * g + 3] * f};
     __syncthreads();
+    if constexpr (PAIR) {                                          // a wave per token: lanes 0 .. 31 the first head, 32 .. 63 the second
+        const int K = p.H * DH;
+        for (int r = wave; r < nq; r += 8) {
+            float4 a = *(const float4 *) (ex + (hf * 32 + r) * OS + 4 * lr);
+#pragma unroll
+            for (int g = 1; g < KW; ++g) {
+                const float4 b = *(const float4 *) (ex + ((g * QW + hf) * 32 + r) * OS + 4 * lr);
+                a.x += b.x; a.y += b.y; a.z += b.z; a.w += b.w;
+            }
+            const float v[4] = {a.x, a.y, a.z, a.w};
+            q8k_block_from_regs(v, lane, y.y + (size_t) (row0 + r) * y.row_bytes, K, (h - qw) / 2, y.tab, row0 + r);
+        }
+        return;
+    }
     constexpr int RL = DH / 4, RP = 64 / RL;                       // lanes per row (4 values each), rows per pass
     for (int r = kw * (32 / KW) + lane / RL; r < (kw + 1) * (32 / KW); r += RP) {
         if (q0 + r >= nq) break;
@@ -438,11 +458,11 @@ __global__ __launch_bounds__(512, 2) void attn_prompt_kernel(PfP p) {
     }
 }
 
-template <int DH, int QW, int KS, bool MASK, bool PLAIN = false> void launch_prompt(PfP p, hipStream_t st) {
+template <int DH, int QW, int KS, bool MASK, bool PLAIN = false, bool PAIR = false> void launch_prompt(PfP p, hipStream_t st, const pm_q8k_out & y = {}) {
     if (!p.tiles) p.n_tiles = (p.T + QW * 32 - 1) / (QW * 32);
     constexpr size_t stages = 2 * (size_t) KS * DH * 4, ex = (size_t) 8 * 32 * (DH + 4) * 4 + 8 * 32 * 2 * 4, lds = stages > ex ? stages : ex;
-    pm_allow_big_lds((const void *) attn_prompt_kernel<DH, QW, KS, MASK, PLAIN>, lds);
-    hipLaunchKernelGGL((attn_prompt_kernel<DH, QW, KS, MASK, PLAIN>), dim3(p.n_tiles * p.H), dim3(512), lds, st, p);
+    pm_allow_big_lds((const void *) attn_prompt_kernel<DH, QW, KS, MASK, PLAIN, PAIR>, lds);
+    hipLaunchKernelGGL((attn_prompt_kernel<DH, QW, KS, MASK, PLAIN, PAIR>), dim3(p.n_tiles * (PAIR ? p.H / 2 : p.H)), dim3(512), lds, st, p, y);
 }
 // Which tile: a CU holds one workgroup. 256 queries share a stage where that still makes two rounds of workgroups (2048 tokens x 64 heads: 102 us, 110 with 128 queries; x 32 heads
 // = one round whose longest tile decides: 80 against 57); 128 queries where they make one (512 x 64 behind 1024 cached: 38 against 50 with 64); below that 64 queries with four key
@@ -482,5 +502,13 @@ int pm_launch_attn_prefill(const float * q, const void * kc, const void * vc, co
     } else {
         if (mask) launch_prompt_dh<64, true>(p, tile_q, st); else launch_prompt_dh<64, false>(p, tile_q, st);
     }
+    return 0;
+}
+
+int pm_launch_attn_prefill_q8k(const float * q, const void * kc, const void * vc, const int32_t * pos0, const int32_t * seq, long seq_stride, int n_tok, int H, int Hkv, int dh, int n_ctx,
+                               float scale, hipStream_t st, const int32_t * tiles, int n_tiles, const pm_q8k_out & out) {
+    if (dh != 128 || n_ctx % 32 || n_tok < 1 || n_tok > 32 || H / Hkv % 2 || (tiles && n_tiles < 1) || (((uintptr_t) kc | (uintptr_t) vc) & 15)) return -1;
+    const PfP p = {q, (const uint16_t *) kc, (const uint16_t *) vc, pos0, seq, seq_stride, nullptr, n_tok, H, Hkv, n_ctx, scale, nullptr, 0, 0, 0, nullptr, tiles, n_tiles};
+    launch_prompt<128, 2, 128, false, false, true>(p, st, out);
     return 0;
 }

@@ -921,7 +921,7 @@ int run_window(pm_window * m, const int32_t * d_tokens, const float * d_x_in, in
         rc |= matmul_small(m, L.t[PM355_T_WV], a, T, m->v, (const float *) L.t[PM355_T_BV].d, nullptr, prepped, st);
         }
         if (rc) return seterr(m, rc, "decode: qkv gemv");
-        bool fused_attn = false;
+        bool fused_attn = false, att_q = false;
         if (T == 1 && !m->no_fuse)
             fused_attn = pm_launch_attn_rope_fused(m->q, m->k, m->v, L.kc, L.vc, m->d_pos, m->d_ctl, kv_stride,
                                                    (const float *) m->rope_freqs.d, m->att, H, Hkv, dh, hp.n_ctx, kq_scale, m->rope, st) == 0;
@@ -930,11 +930,19 @@ int run_window(pm_window * m, const int32_t * d_tokens, const float * d_x_in, in
         // cached cells, one workgroup per (head, token) (attn_cached.hip: one barrier up to 64 cells; 11 -> ~4 us per layer at 2..8 tokens)
         if (!rope_done) rope_store(L, 1);
         const bool mfma = !rg && small_attn_mfma(T, m->h_pos[m->h_seq]);
-        if (rg ? attend_ragged(L) : !(mfma && attend_mfma(L, m->att, nullptr) == 0) && attend_rows(L))
+        if (small && L.t[PM355_T_WO].type != PM_Q8_0 && !m->no_fuse) {          // with the quantization of wo's activations in the launch, where all rows take the same one
+            const pm_q8k_out out = {m->aq_k, pm_q8k_row_bytes(Eq), mmq_tables(m, Eq, T, st)};
+            if (rg && rg->n_rows == T) att_q = pm_launch_attn_cached_q8k(m->q, L.kc, L.vc, d_pos, d_seq, kv_stride, H, Hkv, dh, hp.n_ctx, kq_scale, st, rg->max_cells, T, out) == 0;
+            else if (rg ? rg->n_tiles && !rg->n_rows && !rg->n_long : mfma)
+                att_q = pm_launch_attn_prefill_q8k(m->q, L.kc, L.vc, d_pos, d_seq, kv_stride, T, H, Hkv, dh, hp.n_ctx, kq_scale, st, rg ? rg->tiles : nullptr, rg ? rg->n_tiles : 0, out) == 0;
+            if (att_q) { a = ActQ(); a.k = m->aq_k; a.tab = out.tab.base != nullptr; }
+        }
+        if (att_q) {}
+        else if (rg ? attend_ragged(L) : !(mfma && attend_mfma(L, m->att, nullptr) == 0) && attend_rows(L))
             return seterr(m, PM355_E_RANGE, "decode: n_ctx too large for the decode-attention kernel");
         }
         const Tensor * wo[1] = {&L.t[PM355_T_WO]};
-        a = quantize_for(m, m->att, Eq, T, wo, 1, st);
+        if (!att_q) a = quantize_for(m, m->att, Eq, T, wo, 1, st);
         float * x_mid = (cur == bufs[0]) ? bufs[1] : bufs[0];                 // ffn_inp = wo.att + inpSA
         prepped = false;
         if (matmul_small(m, L.t[PM355_T_WO], a, T, x_mid, nullptr, cur, prepped, st)) return seterr(m, PM355_E_UNSUPPORTED, "decode: wo gemv");

@@ -49,6 +49,8 @@ static inline bool pm_type_is_repacked(int type) { return type == 12 || type == 
 // [super-block][32-value sub-block s][operand lane = 32 * (k / 16 % 2) + row % 32][16 bytes]: one coalesced load per sub-block instead of one
 // cache line per token
 struct pm_q8k_tables { uint8_t * base = nullptr; size_t tab_bytes = 0; int nsb = 0; uint8_t * qbase = nullptr; };
+// Q8_K rows (pm_q8k_row_bytes) and the small-batch mat-mul's tables as a kernel's output
+struct pm_q8k_out { uint8_t * y; size_t row_bytes; pm_q8k_tables tab; };
 // Q8_K activations of up to PM_WIDE_MAX_TOKENS rows for pm_launch_gemm_wide: the 8-bit values as F16 [row][K], sums of 16 as F16 [super-block][ldt][16], scales [super-block][ldt]
 constexpr int PM_WIDE_MAX_TOKENS = 512;
 struct pm_q8k_wide { uint16_t * q = nullptr, * s = nullptr; float * d = nullptr; int ldt = 0; };

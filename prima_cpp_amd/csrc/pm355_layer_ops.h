@@ -62,6 +62,13 @@ int  pm_launch_attn_cached(const float * q, void * kc, void * vc, const int32_t 
                            int H, int Hkv, int dh, int n_ctx, float scale, hipStream_t st, const int32_t * dyn = nullptr,
                            const void * mask = nullptr, int max_keys = 0, int v_rowmajor = 0, int mask_f16 = 0,
                            int n_tok = 1, int rows = 0);    // n_tok > 1 (engine mode): token t of a small batch attends cells [0, pos0 + t] (rows: [0, pos0[t]] of sequence seq[t]), q / out rows t
+// the two launchers of a small batch's attention (rows: every row its own sequence; max_cells: the most cells of a row. tiles or consecutive tokens) with the result quantized to Q8_K where it is made:
+// two heads of 128 are a block. Refused (< 0, nothing launched): other head sizes, more than 256 cells / 32 tokens
+struct pm_q8k_out;
+int  pm_launch_attn_cached_q8k(const float * q, void * kc, void * vc, const int32_t * pos, const int32_t * seq, long seq_stride, int H, int Hkv, int dh, int n_ctx, float scale, hipStream_t st,
+                               int max_cells, int n_tok, const pm_q8k_out & out);
+int  pm_launch_attn_prefill_q8k(const float * q, const void * kc, const void * vc, const int32_t * pos0, const int32_t * seq, long seq_stride, int n_tok, int H, int Hkv, int dh, int n_ctx,
+                                float scale, hipStream_t st, const int32_t * tiles, int n_tiles, const pm_q8k_out & out);
 // ggml-graph mode of the two launchers above: dyn = device int32[2] {cache cell the token is stored in, cells attended}, the RoPE
 // position is pos0[0], mask = additive KQ-mask row [cells attended] (f32, or F16 with mask_f16) or null; v_rowmajor = the V cache is
 // [n_ctx][n_embd_v_gqa] (flash-attention graphs) instead of transposed, with flash-attention rounding points; max_keys (> 0) sizes the fused kernel's LDS score

@@ -636,6 +636,61 @@ def test_batches_of_short_portions_in_wide_passes(E, arch, lens, max_tokens):
     w1.close()
 
 
+def _heads_of_128(E, n_ctx, n_seq, n_head, windows=2):
+    """windows over one model of heads of 128 (two heads are a block of the wo product's activations), with sequences"""
+    d = tiny_model(np.random.default_rng(n_ctx), n_layer=2, n_embd=128 * n_head, n_head=n_head, n_head_kv=2, n_ff=512, n_vocab=320, n_ctx=n_ctx, rope_freqs=True)
+    ws = []
+    for _ in range(windows):
+        w = E.Window(_hp(d), n_ctx=n_ctx)
+        w.load_desc(d)
+        w.finalize_pool(64, n_seq, n_seq * n_ctx)
+        ws.append((w, [w.seq_new() for _ in range(n_seq)]))
+    return ws
+
+
+@pytest.mark.parametrize("lens,n_ctx", [([1, 62, 63, 64, 2, 30], 72), ([63, 126, 127, 128, 1, 64], 136), ([150, 128, 3, 64, 127, 63], 256), ([129, 7], 200)])
+def test_rows_beside_others_keep_their_attention(E, lens, n_ctx):
+    """single tokens of several sequences, heads of 128 quantized where they are made: rows on both sides of 64 and 128 cells, caches of fewer cells than a form takes. The same
+    in whatever company, but for the order of the head's sums."""
+    torch = E.torch
+    (w, s), (w1, s1) = _heads_of_128(E, n_ctx, len(lens), 4)
+    rng = np.random.default_rng(sum(lens))
+    for i, n in enumerate(lens):
+        t = rng.integers(0, 320, n).astype(np.int32)
+        for m, q in ((w, s), (w1, s1)):
+            m.batch([(q[i], t, [n - 1])], logits=torch.empty((1, 320), device="cuda"))
+    for _ in range(2):
+        toks = rng.integers(0, 320, len(lens)).astype(np.int32)
+        lg, lg1 = torch.full((len(lens), 320), float("nan"), device="cuda"), torch.empty((len(lens), 320), device="cuda")
+        w.batch([(q, toks[i:i + 1], [0]) for i, q in enumerate(s)], logits=lg)
+        for i in range(0, len(lens), 2):
+            w1.batch([(s1[j], toks[j:j + 1], [0]) for j in (i, i + 1)], logits=lg1[i:i + 2])
+        assert torch.isfinite(lg).all() and (lg - lg1).abs().max() <= 512 * 2.0 ** -24 * lg1.abs().max()      # (n_embd f32 sums of the head; a turned 8-bit rounding is 1 / 127 of a value)
+    w.close()
+    w1.close()
+
+
+@pytest.mark.parametrize("n_head", [2, 4, 8])
+@pytest.mark.parametrize("past,T", [(200, 2), (191, 5), (130, 31), (255, 32), (250, 33)])
+def test_small_portions_behind_histories_of_heads_of_128(E, past, T, n_head):
+    """a portion of up to 32 tokens on the matrix cores, two heads of a KV head per workgroup (n_head 2: a head each, the launch that quantizes); against the tokens one after the other: the same
+    arithmetic with other summation orders (the bound of the comparisons above)"""
+    torch = E.torch
+    (w, s), (w1, s1) = _heads_of_128(E, 320, 1, n_head)
+    rng = np.random.default_rng(past + T)
+    t, more = rng.integers(0, 320, past).astype(np.int32), rng.integers(0, 320, T).astype(np.int32)
+    lg, lg1 = torch.full((T, 320), float("nan"), device="cuda"), torch.empty((T, 320), device="cuda")
+    for m, q in ((w, s), (w1, s1)):
+        m.batch([(q[0], t, [past - 1])], logits=torch.empty((1, 320), device="cuda"))
+    w.batch([(s[0], more, list(range(T)))], logits=lg)
+    for i in range(T):
+        w1.batch([(s1[0], more[i:i + 1], [0])], logits=lg1[i:i + 1])
+    a, b = lg.double().cpu().numpy(), lg1.double().cpu().numpy()
+    assert (((a - b) ** 2).sum(-1) < 1e-3 * (b ** 2).sum(-1)).all()
+    w.close()
+    w1.close()
+
+
 @pytest.mark.parametrize("n_vocab", [320, 4097, 20011, 140001])
 def test_greedy_token_is_the_first_of_equal_maxima_over_many_workgroups(E, n_vocab):
     """result_norm + lm_head + argmax: rows of the vocabulary are shared by up to 32 workgroups; equal rows of the head (equal logits to the bit) in several of their parts - the first one
