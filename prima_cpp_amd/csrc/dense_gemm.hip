@@ -2,8 +2,8 @@
 // Both operands travel by LDS-DMA as whole 128-byte lines (64 k per stage) into two stages; 16-byte chunks are XOR-swizzled on the source side (chunk c of row r at
 // c ^ ((r >> 1) & 7): the sixteen lanes a ds_read_b128 serves hit sixteen bank groups). One barrier per stage: behind it the stage of the previous step is free and takes
 // the next k-step's DMA, which has this step's MFMAs to land. Tiles of one XCD form compact blocks of the output so that its L2 serves both operands.
-// dense_tile_kernel: one matrix, tiles of 128 .. 256 tokens x 128 or 256 rows, chosen by the time their rounds take. dense_gemm_kernel: two 128 x 128 tiles per CU where that is the quickest; experts
-// (token tiles of 128 or 256 from the routing tables, rows gathered and scattered by pair); latent cache pages into keys and transposed values.
+// dense_tile_kernel: one matrix, tiles of 128 .. 256 tokens x 128 or 256 rows, chosen by the time their rounds take; experts with many pairs. dense_gemm_kernel: two 128 x 128 tiles per CU where
+// that is the quickest; experts (token tiles from the routing tables, rows gathered and scattered by pair); latent cache pages into keys and transposed values.
 #include "pm355_dense.h"
 #include "pm355_kernels.h"
 #include "../../include/prima_mi355.h"
@@ -204,35 +204,44 @@ template <int BM, int BN, int WM, int WN, int STAGES, int KIND> __global__ __lau
     }
 }
 
-// One matrix over many tokens: tiles of 32 MI tokens x 64 NI rows, eight waves of 16 MI x 16 NI, so that tiles can be cut to what a batch has (835 tokens are 3.3 tiles of 256 and 3.7 of 224, and
+// One matrix over many tokens (or experts: sorted pairs, 256 per tile): tiles of 32 MI tokens x 64 NI rows, eight waves of 16 MI x 16 NI, so that tiles can be cut to what a batch has (835 tokens are 3.3 tiles of 256 and 3.7 of 224, and
 // 10240 rows 40 tiles of 256 - 160 workgroups - and 54 of 192). v_mfma_f32_16x16x32_bf16 (the rate of 32 x 32 x 16 per bit of operand): rows of W are the tile's rows, so that a lane holds
-// four neighbouring outputs of a token and stores them together. Both operands by LDS-DMA as in the kernel above, as many stages as fit, up to four.
+// four neighbouring outputs of a token and stores them together. Both operands by LDS-DMA as in the kernel above, as many stages as fit.
 // What bounds it: a step of 64 k of a 256 x 256 tile takes 1.65 us - its products and the LDS reads for them 1.4, its lines from the L2s 1.45 beside that -, in proportion to the tile's area.
-template <int MI, int NI> struct Tile { static constexpr int BM = 32 * MI, BN = 64 * NI, STAGE = (BM + BN) * 128, STAGES = 4 * STAGE <= 160 * 1024 ? 4 : 3 * STAGE <= 160 * 1024 ? 3 : 2; };
-template <int MI, int NI> __global__ __launch_bounds__(512) void dense_tile_kernel(GemmP p) {
+template <int MI, int NI> struct Tile { static constexpr int BM = 32 * MI, BN = 64 * NI, STAGE = (BM + BN) * 128, STAGES = (160 * 1024 - 1) / STAGE; };
+template <int MI, int NI, bool EXP> __global__ __launch_bounds__(512) void dense_tile_kernel(GemmP p) {
     typedef Tile<MI, NI> S;
     constexpr int BM = S::BM, BN = S::BN, STAGE = S::STAGE, STAGES = S::STAGES, ALL = (BM + BN) / 8, PIECES = (ALL + 7) / 8;
     extern __shared__ __attribute__((aligned(1024))) char smem[];
     const int wave = __builtin_amdgcn_readfirstlane((int) threadIdx.x >> 6), lane = threadIdx.x & 63, lr = lane & 15, g = lane >> 4;
     const int wm = wave >> 2, wn = wave & 3;
-    const int tiles = p.nt * p.nn, total = tiles * p.splits, per = (total + 7) / 8;         // (order of the tiles: as above)
+    const int nt = EXP ? __builtin_amdgcn_readfirstlane(ld_g(p.tiles)) : p.nt;               // (the grid has room for the most tiles there can be)
+    const int tiles = nt * p.nn, total = EXP ? tiles : tiles * p.splits, per = (total + 7) / 8;      // (order of the tiles: as above)
     int slot = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
     if (slot >= total || (int) (blockIdx.x >> 3) >= per) return;
-    const int split = slot / tiles;
+    const int split = EXP ? 0 : slot / tiles;
     slot -= split * tiles;
-    const int band = slot / (8 * p.nn), left = p.nt - band * 8, bh = left < 8 ? left : 8, in = slot - band * 8 * p.nn;
-    const int t0 = (band * 8 + in % bh) * BM, n0 = (in / bh) * BN, k0 = split * p.split_steps;
-    const int steps = p.split_steps < (p.K >> 6) - k0 ? p.split_steps : (p.K >> 6) - k0;
+    const int band = slot / (8 * p.nn), left = nt - band * 8, bh = left < 8 ? left : 8, in = slot - band * 8 * p.nn;
+    int t0 = (band * 8 + in % bh) * BM, n_tok = p.T;
+    const int n0 = (in / bh) * BN, k0 = EXP ? 0 : split * p.split_steps;
+    const int steps = !EXP && p.split_steps < (p.K >> 6) - k0 ? p.split_steps : (p.K >> 6) - k0;
+    const uint16_t * W = p.W;
+    if constexpr (EXP) {                                   // t0 .. n_tok: sorted pairs of this tile
+        const int32_t * tt = p.tiles + 1 + 3 * (band * 8 + in % bh);
+        W += (int64_t) __builtin_amdgcn_readfirstlane(ld_g(tt)) * p.e_stride;
+        t0 = __builtin_amdgcn_readfirstlane(ld_g(tt + 1)); n_tok = t0 + __builtin_amdgcn_readfirstlane(ld_g(tt + 2));
+    }
     // pieces of 8 rows x 128 bytes, wave, wave + 8, .. (a wave without a last one brings the last one again: the same bytes to the same place)
-    const char * xb = (const char *) (p.X + (size_t) t0 * p.lda), * wb = (const char *) (p.W + (size_t) n0 * p.K);
-    const int x_last = p.T - 1 - t0, w_last = p.N - 1 - n0;
+    const char * xb = (const char *) (EXP ? p.X : p.X + (size_t) t0 * p.lda), * wb = (const char *) (W + (size_t) n0 * p.K);
+    const int x_last = n_tok - 1 - t0, w_last = p.N - 1 - n0;
     const uint32_t lds0 = (uint32_t) (uintptr_t) (__attribute__((address_space(3))) char *) smem;
     uint32_t off[PIECES];
 #pragma unroll
     for (int i = 0; i < PIECES; ++i) {
         const int q = min(wave + 8 * i, ALL - 1), r = q * 8 + (lane >> 3);
         const bool tok = q < BM / 8;
-        const int row = tok ? min(r, x_last) : min(r - BM, w_last);
+        int row = tok ? min(r, x_last) : min(r - BM, w_last);
+        if constexpr (EXP) if (tok) { row += t0; if (p.gather) row = ld_g(p.order + row) / p.top; }
         off[i] = (uint32_t) row * (uint32_t) (tok ? p.lda : p.K) * 2u + (uint32_t) ((lane & 7) ^ ((r >> 1) & 7)) * 16u;
     }
     auto request = [&](int k, int stage) __attribute__((always_inline)) {
@@ -254,7 +263,9 @@ template <int MI, int NI> __global__ __launch_bounds__(512) void dense_tile_kern
     int stage = 0, next = STAGES - 1;
     for (int k = 0; k < steps; ++k) {
         const int ahead = steps - 1 - k;                   // (as in the kernel above)
+        static_assert(STAGES >= 2 && STAGES <= 5, "the waits are spelled for these");
         if (STAGES > 2 && ahead >= STAGES - 2) vm_wait<PIECES * (STAGES - 2)>();
+        else if (STAGES > 4 && ahead == 2) vm_wait<PIECES * 2>();
         else if (STAGES > 3 && ahead == 1) vm_wait<PIECES>();
         else vm_wait<0>();
         __syncthreads();
@@ -289,13 +300,26 @@ template <int MI, int NI> __global__ __launch_bounds__(512) void dense_tile_kern
         for (int e = 0; e < 4; ++e) { const int col = n0 + (wn * NI + n) * 16 + g * 4 + e; bias[n][e] = p.bias && split == 0 && col < p.n_store ? ld_g(p.bias + col) : 0.0f; }
 #pragma unroll
     for (int n = 0; n < NI; ++n) asm volatile("" : "+v"(bias[n]));
+    int pair[EXP ? MI : 1];
+    float weight[EXP ? MI : 1];
+    if constexpr (EXP) {                                   // what the stores need about their rows
+#pragma unroll
+        for (int m = 0; m < MI; ++m) {
+            const int i = t0 + (wm * MI + m) * 16 + lr;
+            pair[m] = ld_g(p.order + (i < n_tok ? i : n_tok - 1));
+            weight[m] = p.weight ? ld_g(p.weight + pair[m]) : 1.0f;
+        }
+#pragma unroll
+        for (int m = 0; m < MI; ++m) asm volatile("" : "+v"(pair[m]), "+v"(weight[m]));
+    }
     auto put = [&](auto * y, bool whole) __attribute__((always_inline)) {
         typedef std::remove_reference_t<decltype(*y)> Y;
 #pragma unroll
         for (int m = 0; m < MI; ++m) {
-            const int tok = t0 + (wm * MI + m) * 16 + lr;
-            if (tok >= p.T) continue;
-            Y * row = y + (p.rows ? (size_t) tok * p.splits + split : (size_t) split * p.T + tok) * p.ldy + n0 + wn * 16 * NI + g * 4;
+            int tok = t0 + (wm * MI + m) * 16 + lr;
+            if (tok >= n_tok) continue;
+            if constexpr (EXP) { if (p.scatter) tok = pair[m]; }
+            Y * row = y + (EXP ? (size_t) tok : p.rows ? (size_t) tok * p.splits + split : (size_t) split * p.T + tok) * p.ldy + n0 + wn * 16 * NI + g * 4;
 #pragma unroll
             for (int n = 0; n < NI; ++n) {
                 f32x4 v = acc[n][m] + bias[n];
@@ -303,6 +327,7 @@ template <int MI, int NI> __global__ __launch_bounds__(512) void dense_tile_kern
 #pragma unroll
                     for (int e = 0; e < 4; ++e) v[e] = act_apply(p.act_fn, v[e]);
                 }
+                if constexpr (EXP) v *= weight[m];
                 if (whole) {
                     if constexpr (sizeof(Y) == 4) *(PM_G f32x4 *) (row + n * 16) = v;
                     else *(PM_G u32x2 *) (row + n * 16) = u32x2{(uint32_t) f2bf(v[0]) | (uint32_t) f2bf(v[1]) << 16, (uint32_t) f2bf(v[2]) | (uint32_t) f2bf(v[3]) << 16};
@@ -318,13 +343,14 @@ template <int MI, int NI> __global__ __launch_bounds__(512) void dense_tile_kern
     if (p.y_type == PM_BF16) { if (whole) put((uint16_t *) p.y, true); else put((uint16_t *) p.y, false); }
     else { if (whole) put((float *) p.y, true); else put((float *) p.y, false); }
 }
-template <int MI, int NI> int launch_tile(GemmP p, hipStream_t st) {
+template <int MI, int NI, bool EXP = false> int launch_tile(GemmP p, hipStream_t st) {
     typedef Tile<MI, NI> S;
     if (p.splits < 1) { p.splits = 1; p.split_steps = p.K >> 6; }
-    p.nt = (p.T + S::BM - 1) / S::BM; p.nn = (p.n_store + S::BN - 1) / S::BN;
+    if (!EXP) p.nt = (p.T + S::BM - 1) / S::BM;
+    p.nn = (p.n_store + S::BN - 1) / S::BN;
     const size_t lds = (size_t) S::STAGES * S::STAGE;
-    pm_allow_big_lds((const void *) dense_tile_kernel<MI, NI>, lds);
-    hipLaunchKernelGGL((dense_tile_kernel<MI, NI>), dim3((p.nt * p.nn * p.splits + 7) / 8 * 8), dim3(512), lds, st, p);
+    pm_allow_big_lds((const void *) dense_tile_kernel<MI, NI, EXP>, lds);
+    hipLaunchKernelGGL((dense_tile_kernel<MI, NI, EXP>), dim3((p.nt * p.nn * p.splits + 7) / 8 * 8), dim3(512), lds, st, p);
     return 0;
 }
 
@@ -415,7 +441,7 @@ int pm_launch_experts_gemm(const pm_expert_args & a, hipStream_t st) {
     GemmP p = {};
     p.tiles = a.r.tiles; p.order = a.r.order; p.top = a.r.top;
     if (a.r.tile != 128 && a.r.tile != 256) return PM355_E_SHAPE;
-    auto go = [&]() { return a.r.tile == 256 ? launch_stages<256, 256, 128, 64, 2, EXPERTS>(p, st) : launch_128<EXPERTS>(p, st); };
+    auto go = [&]() { return a.r.tile == 256 ? launch_tile<8, 4, true>(p, st) : launch_128<EXPERTS>(p, st); };
     p.nt = (int) (pairs / a.r.tile + (a.r.E < pairs ? a.r.E : pairs));                  // (most tiles there can be: every expert's last one may be short)
     p.W = (const uint16_t *) a.up; p.e_stride = a.up_stride; p.X = (const uint16_t *) a.x; p.lda = a.ldx; p.K = a.width_p; p.N = p.n_store = a.ffp; p.y = a.hid; p.ldy = a.ffp;
     p.y_type = PM_BF16; p.act_fn = a.act_fn; p.gather = 1; p.weight = a.r.w;
