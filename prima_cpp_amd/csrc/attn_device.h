@@ -9,8 +9,12 @@ struct RopeP {
 };
 
 __device__ __forceinline__ void rope_cs(const RopeP & r, float pos, int pair, const float * ff, float & c, float & s) {
+    // (multiplied up step by step, the reference's rounding; eight steps per look at the lanes, a lane that is through multiplies by 1: one by one the loop around them was most of the launch that
+    // makes a step's table, 64 pairs 5.1 us, now 3.4)
     float theta = pos;
-    for (int j = 0; j < pair; ++j) theta *= r.theta_scale;
+    for (int j = 0; __builtin_amdgcn_ballot_w64(j < pair); j += 8)
+#pragma unroll
+        for (int u = 0; u < 8; ++u) theta *= j + u < pair ? r.theta_scale : 1.0f;
     const float f = ff ? ld_g(ff + pair) : 1.0f;
     const float te = theta / f;
     float ti = r.freq_scale * te, th = ti, ms = r.attn_factor;

@@ -109,9 +109,9 @@ __global__ __launch_bounds__(64) void rope_kv_store_kernel(const float * q, cons
         if (pair < half) {
             a = neox ? pair : 2 * pair;
             b = neox ? pair + half : 2 * pair + 1;
+            const float x0 = ld_g(src + a), x1 = ld_g(src + b);      // (on their way while the angle is formed)
             float c, s;
             rope_cs(r, (float) pos, pair, freq_factors, c, s);
-            const float x0 = src[a], x1 = src[b];
             o0 = x0 * c - x1 * s;
             o1 = x0 * s + x1 * c;
         } else {                         // dims beyond n_dims pass through
