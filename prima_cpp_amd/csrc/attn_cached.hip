@@ -42,9 +42,9 @@ template <int DH, int KPL> struct ShortLds {
 // us per launch of 32 heads of 128 over 36 / 100 / 204 cells: a lane's own key and dimension straight from memory 3.3 / 4.4 / 7.0, this 2.8 / 3.7 / 5.7 (multiplied in the registers that the
 // lines arrive in, sums over lanes, 2.6 / 3.1 / 4.5: one other bit here turns 8-bit roundings behind it, 3 % of the logits of eight layers of the 8B shape).
 // Rounding points as everywhere: q, K, V F16, the normalised probabilities rounded to F16, f32 accumulation. n_kv <= 64 * KPL <= n_ctx; DH 64 / 128 (256: KPL = 1).
-// put(d, value): the head's result.
-template <int DH, int KPL, class Put>
-__device__ __forceinline__ void attn_short(const float * q_head, const uint16_t * kc, const uint16_t * vc, Put put, int hk, int Hkv, int n_ctx, int n_kv, float scale, const void * mask,
+// out: the head's result in memory, or a function of (dimension, value).
+template <int DH, int KPL, class Out>
+__device__ __forceinline__ void attn_short(const float * q_head, const uint16_t * kc, const uint16_t * vc, Out out, int hk, int Hkv, int n_ctx, int n_kv, float scale, const void * mask,
                                            int mask_f16, char * smem, int lane, int wave, unsigned long long * ts) {
     unsigned long long tsv[6] = {PM_TS_NOW(), 0, 0, 0, 0, 0};
     typedef ShortLds<DH, KPL> S;
@@ -133,7 +133,10 @@ __device__ __forceinline__ void attn_short(const float * q_head, const uint16_t 
     tsv[4] = PM_TS_NOW();                                      // P.V
     if constexpr (DPW <= 16) o += __builtin_bit_cast(float, other_row(__builtin_bit_cast(uint32_t, o)));
     if constexpr (DPW <= 32) o += __builtin_bit_cast(float, other_half(__builtin_bit_cast(uint32_t, o)));
-    if (lane < DPW) put(DPW * wave + lane, o);
+    if (lane < DPW) {
+        if constexpr (std::is_pointer_v<Out>) st_g(out + DPW * wave + lane, o);
+        else out(DPW * wave + lane, o);
+    }
     tsv[5] = PM_TS_NOW();
     pm_ts_store(ts, 2, tsv);
 }
@@ -160,8 +163,7 @@ __global__ __launch_bounds__(256) void attn_cached_kernel(AttnP a_in) {
         }
         const uint16_t * kc = a.kc + (long) seq * a.seq_stride, * vc = a.vc + (long) seq * a.seq_stride;
         auto go = [&](auto kpl) __attribute__((always_inline)) {
-            float * out = a.out + (long) h * DH;
-            attn_short<DH, decltype(kpl)::value>(a.q + (long) h * DH, kc, vc, [&](int d, float v) __attribute__((always_inline)) { st_g(out + d, v); }, hk, Hkv, n_ctx, n_kv, a.scale, a.mask, a.mask_f16, smem, lane, wave, a.ts);
+            attn_short<DH, decltype(kpl)::value>(a.q + (long) h * DH, kc, vc, a.out + (long) h * DH, hk, Hkv, n_ctx, n_kv, a.scale, a.mask, a.mask_f16, smem, lane, wave, a.ts);
         };
         // (caches that hold fewer cells than the form takes: the general body, as it always was - its sums are in another order)
         if (n_kv <= 64 && n_ctx >= 64) return go(std::integral_constant<int, 1>());
