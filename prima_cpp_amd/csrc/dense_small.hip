@@ -4,7 +4,7 @@
 // block is the one in which a lane's 16-byte loads lie (both operands agree on it).
 // With a few tokens the prologue x + norm(y) runs in every workgroup (one launch less; the residual row is written by the first).
 // The same body serves one matrix per attention head (groups of rows with activations of their own) and experts: with a few tokens one workgroup row per (token, expert)
-// pair, which routes its token in the prologue, and a down product over the concatenation of a token's experts; with more one row per expert that has tokens.
+// pair, which routes its token in the prologue where no launch has, and a down product over the concatenation of a token's experts; with more one row per expert that has tokens.
 #include "pm355_dense.h"
 #include "pm355_kernels.h"
 #include "pm355_route.h"

@@ -1,4 +1,4 @@
-// moe.hip — routing of a step's tokens to experts. Up to 64 tokens: one workgroup scores, selects and sorts (expert by expert, tokens in order). More: a wave per token
+// moe.hip — routing of a step's tokens to experts. Few tokens of few experts: one launch with the norm and the router product, a workgroup per token. Up to 64 tokens: one workgroup scores, selects and sorts (expert by expert, tokens in order). More: a wave per token
 // selects and takes a place in its expert's list, then every workgroup sorts its share of the pairs (the order inside an expert does not enter any sum).
 #include "pm355_route.h"
 #include "pm355_kernels.h"
