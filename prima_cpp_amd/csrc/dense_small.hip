@@ -143,7 +143,7 @@ template <typename T, int NT, int RM, int SRC, int EXP> __global__ __launch_boun
         weight = w[k]; base = blockIdx.y; act += (size_t) t * p.lda; t0 = 0; n_tok = 1;
     }
     if constexpr (EXP == CONCAT) { const int t = blockIdx.y; cat = uniform_const_ptr(p.r.id + t * p.r.top); base = t; act += (size_t) t * p.lda; t0 = 0; n_tok = 1; }
-    __shared__ int local[EXP == SORTED ? 64 : 1];          // SORTED without tables: the expert's pairs
+    __shared__ int local[EXP == SORTED ? PM_ROUTE_PAIRS : 1];          // SORTED without tables: the expert's pairs
     if constexpr (EXP == SORTED) {
         int e;
         if (p.r.logits) {
@@ -151,19 +151,27 @@ template <typename T, int NT, int RM, int SRC, int EXP> __global__ __launch_boun
             e = __builtin_amdgcn_readfirstlane(ld_g(p.r.active + 1 + blockIdx.y));
             base = __builtin_amdgcn_readfirstlane(ld_g(p.r.off + e)); n_tok = __builtin_amdgcn_readfirstlane(ld_g(p.r.off + e + 1)) - base;
         } else {
-            // up to 64 pairs of up to 64 experts: a lane per pair, this workgroup's expert is the blockIdx.y-th that has one. (One load in front of the weights instead of three, one behind the
-            // other, and no launch that sorts; every wave finds the same)
-            const bool pair = lane < p.T * p.r.top;
-            const int mine = pair ? ld_g(p.r.id + lane) : p.r.E;
-            uint32_t has[2] = {pair && mine < 32 ? 1u << mine : 0u, pair && mine >= 32 ? 1u << (mine - 32) : 0u};
+            // up to PM_ROUTE_PAIRS pairs of up to 64 experts: a lane per pair, 64 at a time; this workgroup's expert is the blockIdx.y-th that has one. (One round of loads in front of the weights
+            // instead of three, one behind the other, and no launch that sorts; every wave finds the same)
+            constexpr int G = PM_ROUTE_PAIRS / 64;
+            const int pairs = p.T * p.r.top;
+            int mine[G];
 #pragma unroll
-            for (int i = 0; i < 2; ++i) has[i] = wave_or(has[i]);
-            const uint64_t on = (uint64_t) has[1] << 32 | has[0];
+            for (int i = 0; i < G; ++i) mine[i] = i * 64 + lane < pairs ? ld_g(p.r.id + i * 64 + lane) : 64;       // (64: no expert)
+            uint32_t has[2] = {0, 0};
+#pragma unroll
+            for (int i = 0; i < G; ++i) { has[0] |= mine[i] < 32 ? 1u << mine[i] : 0u; has[1] |= mine[i] >= 32 && mine[i] < 64 ? 1u << (mine[i] - 32) : 0u; }
+            const uint64_t on = (uint64_t) wave_or(has[1]) << 32 | wave_or(has[0]);
             if ((int) blockIdx.y >= __popcll(on)) return;
             e = __builtin_ctzll(__builtin_amdgcn_ballot_w64((on >> lane & 1) && __popcll(on & ((1ull << lane) - 1)) == (int) blockIdx.y));
-            const uint64_t its = __builtin_amdgcn_ballot_w64(mine == e);
-            base = __popcll(__builtin_amdgcn_ballot_w64(mine < e)); n_tok = __popcll(its);
-            if (its >> lane & 1) local[__popcll(its & ((1ull << lane) - 1))] = lane;
+            base = 0; n_tok = 0;
+#pragma unroll
+            for (int i = 0; i < G; ++i) {
+                const uint64_t its = __builtin_amdgcn_ballot_w64(mine[i] == e);
+                base += __popcll(__builtin_amdgcn_ballot_w64(mine[i] < e));
+                if (its >> lane & 1) local[n_tok + __popcll(its & ((1ull << lane) - 1))] = i * 64 + lane;
+                n_tok += __popcll(its);
+            }
             wave_fence();
         }
         W += (size_t) e * p.e_stride; t0 = 0;

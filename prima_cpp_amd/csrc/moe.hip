@@ -1,4 +1,4 @@
-// moe.hip — routing of a step's tokens to experts. Few tokens of few experts: one launch with the norm and the router product, a workgroup per token. Up to 64 tokens: one workgroup scores, selects and sorts (expert by expert, tokens in order). More: a wave per token
+// moe.hip — routing of a step's tokens to experts. Up to 64 tokens of up to 64 experts: one launch with the norm and the router product, a workgroup per token. Up to 64 tokens: one workgroup scores, selects and sorts (expert by expert, tokens in order). More: a wave per token
 // selects and takes a place in its expert's list, then every workgroup sorts its share of the pairs (the order inside an expert does not enter any sum).
 #include "pm355_route.h"
 #include "pm355_kernels.h"
@@ -87,7 +87,7 @@ __global__ __launch_bounds__(1024) void route_one_kernel(pm_route r, int T, int 
     }
 }
 
-// Few tokens of a bf16 model with RMS norms: the residual stream's norm, the router product and the choice of experts, one workgroup per token. Three launches otherwise, whose time is the way to their first
+// Up to 64 tokens of a bf16 model with RMS norms: the residual stream's norm, the router product and the choice of experts, one workgroup per token. Three launches otherwise, whose time is the way to their first
 // byte and from their last one: 5 tokens of 2048 values, 32 experts, 4 each: 4.2 + 4.5 + 7.1 us and the gaps between them, now 8.3 and one gap (all tokens in one workgroup, which then also sorts the
 // pairs: 16.7 us, the vector pipe of one CU; the expert products find their pairs themselves, dense_small.hip). A wave has every 16th 64-value block of the row: it norms those columns and
 // multiplies them, the router's weights of all its blocks on their way from the start (in its registers: that bounds the width and the experts), so that the workgroup meets for the norm's
@@ -221,9 +221,9 @@ void pm_launch_route(const pm_route & r, int T, int want_tiles, hipStream_t st) 
     hipLaunchKernelGGL(route_place_kernel, dim3((pairs + 255) / 256), dim3(256), (size_t) (2 * r.E + 1) * 4, st, r, pairs, want_tiles);
 }
 
-// what a workgroup's registers hold: 64 blocks of 32 experts, 32 of 64; the pairs of the step fit a wave's lanes (dense_small.hip)
+// what a workgroup's registers hold: 64 blocks of 32 experts, 32 of 64; the pairs that the small products find for themselves (dense_small.hip)
 bool pm_route_stream_ok(const pm_route & r, const pm_norm_args & q, int K, int T) {
-    return T * r.top <= 64 && r.E <= 64 && K <= (r.E <= 32 ? 4096 : 2048) && q.width <= K && q.rms && !q.b && !q.parts && q.y_type == PM_F32;
+    return T <= PM_ROUTE_ONE_MAX && T * r.top <= PM_ROUTE_PAIRS && r.E <= 64 && K <= (r.E <= 32 ? 4096 : 2048) && q.width <= K && q.rms && !q.b && !q.parts && q.y_type == PM_F32;
 }
 void pm_launch_route_stream(const pm_route & r, const pm_norm_args & q, float * x, const float * y, const void * W, int K, void * xb, int ld, int T, hipStream_t st) {
     const StreamP p{y, x, (const uint16_t *) W, (uint16_t *) xb, ld, K};

@@ -149,6 +149,7 @@ struct pm_route {
 // 95 pairs each 60 / 67, 114 62 / 68, 118 87 / 70, 125 92 / 70, 156 86 / 71, 207 94 / 72, 256 (every second expert has two large tiles) 112 / 119
 static inline int pm_expert_tile(int64_t pairs, int E) { return pairs >= 384 * (int64_t) E || (pairs >= 116 * (int64_t) E && pairs < 232 * (int64_t) E) ? 256 : 128; }
 constexpr int PM_ROUTE_PAIR_MAX = 4, PM_ROUTE_ONE_MAX = 64;      // tokens up to which the pairs go one by one / one workgroup routes and sorts
+constexpr int PM_ROUTE_PAIRS = 256;                                  // pairs that the products of few tokens find for themselves
 void pm_launch_route(const pm_route & r, int T, int want_tiles, hipStream_t st);
 // few tokens, bf16, RMS: x += norm(y), xb = norm(x) (pm_launch_add_norm), the router product W . xb (rows of K values) and r.id, r.w in one; rows of x, y, xb: ld values. The expert products
 // are then called without logits

@@ -145,13 +145,13 @@ def test_routing_picks_the_same_experts(E, top, count, keep):
 @pytest.mark.parametrize("E,top,count,keep,width", [(1, 1, 1, 1, 60), (5, 3, 1, 1, 130), (32, 4, 1, 1, 2048), (31, 2, 1, 1, 2116), (32, 4, 8, 3, 4096), (33, 7, 11, 4, 1000), (64, 64, 1, 1, 70), (63, 1, 7, 2, 2048),
                                                     (40, 2, 5, 2, 2112), (20, 3, 1, 1, 4160)])
 def test_norm_router_and_choice_in_one_launch(E, top, count, keep, width):
-    """bf16, on both sides of what the launch takes: 32 and 64 experts, rows of 2048 and 4096 values, 64 pairs; rows that end inside a 64-value block, waves without a block"""
+    """bf16, on both sides of what the launch takes: 32 and 64 experts, rows of 2048 and 4096 values, 64 tokens, 64 and 256 pairs; rows that end inside a 64-value block, waves without a block"""
     c = one(scan(inner=64, mlp=moe(E, top, count, keep, 16)), width=width, vocab=200)
     w = silent(weights_for(c, "bfloat16", 3), 0)
     _, _, m = model("route", "bfloat16", c, 3, w, fresh=True, max_tokens=128, n_seq=2, pool_tokens=256)
     toks = tokens(70, 200, 5)
     want = P.run(c, w, toks)
-    for n in sorted({1, 4, 5, 64 // top, 64 // top + 1}):
+    for n in sorted({1, 4, 5, 64 // top, 64 // top + 1, min(256 // top, 64), min(256 // top, 64) + 1}):
         close(alone(m, toks[:n]), want[:n], "bfloat16")
     m.close()
 
