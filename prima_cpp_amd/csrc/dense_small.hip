@@ -459,6 +459,38 @@ template <int RM, int TP> int launch_rows(const SmallP & p, int N, hipStream_t s
     return 0;
 }
 
+// One bf16 matrix per group of rows (attention head) with short rows: NB 64-k blocks, a wave per 16 rows and 16 tokens, everything it needs requested at once and no sums over waves. (Above,
+// eight waves share a row's blocks: of 64 k seven have none. 16384 rows of 64, 5 tokens: 8.4 us, now 3.2 .. 5.0)
+template <int NB> __global__ __launch_bounds__(256) void dense_group_kernel(SmallP p, int rows, int whole) {
+    const int wave = __builtin_amdgcn_readfirstlane((int) threadIdx.x >> 6), lane = threadIdx.x & 63, lr = lane & 15, g = lane >> 4;
+    const int r0 = ((int) blockIdx.x * 4 + wave) * 16, t0 = blockIdx.y * 16;
+    if (r0 >= rows) return;
+    const int h = r0 / p.group, hr = r0 - h * p.group + g * 4, t = t0 + lr;
+    const uint16_t * w = (const uint16_t *) p.W + (size_t) (r0 + lr) * (NB * 64) + g * 8, * x = (const uint16_t *) p.act + (size_t) h * p.g_act + (size_t) (t < p.T ? t : p.T - 1) * p.lda + g * 8;
+    u32x4 a[2 * NB], b[2 * NB];
+#pragma unroll
+    for (int i = 0; i < 2 * NB; ++i) { a[i] = *(const PM_G u32x4 *) (w + i * 32); b[i] = *(const PM_G u32x4 *) (x + i * 32); }
+    f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int i = 0; i < 2 * NB; ++i) acc = Frag<uint16_t>::mma(a[i], b[i], acc);
+    if (t >= p.T) return;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) acc[e] = act_apply(p.act_fn, acc[e]);
+    const size_t at = (size_t) t * p.ldy + h * p.g_out + hr;
+    if (whole) {                                           // (four neighbours of a row of y, wanted and on their boundary)
+        if (p.y_type == PM_F32) *(PM_G f32x4 *) ((float *) p.y + at) = acc;
+        else *(PM_G u32x2 *) ((uint16_t *) p.y + at) = u32x2{(uint32_t) f2bf(acc[0]) | (uint32_t) f2bf(acc[1]) << 16, (uint32_t) f2bf(acc[2]) | (uint32_t) f2bf(acc[3]) << 16};
+        return;
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) if (hr + e < p.g_store && h * p.g_out + hr + e < p.n_store) st_type(p.y, at + e, p.y_type, acc[e]);
+}
+template <int NB> int launch_group(const SmallP & p, int N, hipStream_t st) {
+    const int whole = p.g_store % 16 == 0 && p.g_store == p.group && p.g_out % 4 == 0 && p.ldy % 4 == 0 && ((uintptr_t) p.y & 15) == 0 && (N / p.group - 1) * p.g_out + p.g_store <= p.n_store;
+    hipLaunchKernelGGL(dense_group_kernel<NB>, dim3((N + 63) / 64, (p.T + 15) / 16), dim3(256), 0, st, p, N, whole);
+    return 0;
+}
+
 template <typename T, int NT, int RM, int SRC, int EXP = DENSE> int launch(const SmallP & p, int N, int y, hipStream_t st) {
     constexpr bool LINE = sizeof(T) == 2 && SRC != 0;
     constexpr int rows = (LINE ? 8 : 16) * RM, toks = (LINE ? 8 : 16) * NT;
@@ -481,6 +513,13 @@ template <typename T> int launch_type(const pm_dense_args & a, const SmallP & p,
         if constexpr (sizeof(T) == 2) if (rm == 2) return a.T == 1 ? launch<T, 1, 2, 1>(p, N, 0, st) : a.T == 2 ? launch<T, 1, 2, 2>(p, N, 0, st) : launch<T, 1, 2, 4>(p, N, 0, st);
         return a.T == 1 ? launch<T, 1, 1, 1>(p, N, 0, st) : a.T == 2 ? launch<T, 1, 1, 2>(p, N, 0, st) : launch<T, 1, 1, 4>(p, N, 0, st);
     }
+    // One matrix per group, short rows: up to 256 values a wave's operands fit its registers, and eight waves on a row have at most half a block each
+    if constexpr (sizeof(T) == 2)
+        if (a.group && !a.merge && a.T <= 64 && a.K <= 256 && (((uintptr_t) p.W | (uintptr_t) p.act) & 15) == 0 && p.lda % 8 == 0 && p.g_act % 8 == 0 && N % p.group == 0) {
+            if (a.K == 64) return launch_group<1>(p, N, st);
+            if (a.K == 128) return launch_group<2>(p, N, st);
+            return a.K == 192 ? launch_group<3>(p, N, st) : launch_group<4>(p, N, st);
+        }
     // One matrix, up to 8 tokens: the workgroups that stay, with the activations in LDS where they fit (150 KB: 16 bytes per value for 5..8 tokens, 8 for less), from memory above that
     // (5 tokens of 4096 values, 14336 rows: 22.7 us against 27 from memory). One token of shorter rows stays with a workgroup per tile, which has less to do before its first and after
     // its last weight (32000 x 2048: 23.6 us against 25.1, 4096 x 5120: 10.2 / 10.9; the other way round from 6144 values: 5120 x 6144 16.8 / 15.2, 2048 x 8192 10.3 / 9.0). DMA and buffer loads

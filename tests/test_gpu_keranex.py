@@ -156,6 +156,20 @@ def test_norm_router_and_choice_in_one_launch(E, top, count, keep, width):
     m.close()
 
 
+@pytest.mark.parametrize("heads,dim,kv_rank", [(3, 64, 64), (2, 65, 40), (5, 128, 130), (1, 192, 100), (2, 193, 64), (3, 256, 57)])
+def test_latent_queries_of_short_heads(heads, dim, kv_rank):
+    """bf16: queries into the latents' space, a wave per 16 rows of a head: one to four 64-value blocks, latents that fill their rows and that do not, one and several tiles of 16 tokens"""
+    c = one(latent(heads=heads, dim=dim, rot_dim=16, vdim=24, kv_rank=kv_rank, size=90, scale=dim ** -0.5), width=128, vocab=120)
+    w = weights_for(c, "bfloat16", 4)
+    _, _, m = model("queries", "bfloat16", c, 4, w, fresh=True, max_tokens=64, n_seq=2, pool_tokens=256)
+    toks = tokens(66, 120, 3)
+    want = P.run(c, w, toks)
+    close(alone(m, toks, range(1, 66)), want, "bfloat16")
+    for n in (1, 16, 17, 64):
+        close(alone(m, toks[:n]), want[:n], "bfloat16")
+    m.close()
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("ff,E,top", [(4700, 3, 2), (1030, 5, 1), (576, 2, 2)])
 def test_wide_experts(ff, E, top, dtype):
