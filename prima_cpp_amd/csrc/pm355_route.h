@@ -44,7 +44,7 @@ template <typename Z> __device__ __forceinline__ void route_token(Z z, int E, in
         float wt = 0.0f;                                   // (a row of NaNs has no largest score)
         for (int k = 0; k < top; ++k) {
             const float best = wave_max(m);
-            const uint64_t at = __builtin_amdgcn_ballot_w64(m == best);
+            const uint64_t at = __builtin_amdgcn_ballot_w64(lane < E && m == best);      // (lanes without an expert are the largest where no score compares)
             const int first = at ? __builtin_ctzll(at) : 0;
             if (lane == k && at) { id = first; wt = fmaxf(best, 0.0f); }
             if (lane == first) m = -2.0f;

@@ -156,6 +156,30 @@ def test_norm_router_and_choice_in_one_launch(E, top, count, keep, width):
     m.close()
 
 
+@pytest.mark.parametrize("E,top,count,keep,width", [(5, 3, 1, 1, 130), (32, 4, 1, 1, 2048), (33, 7, 11, 4, 1000), (64, 8, 1, 1, 70), (65, 4, 1, 1, 96), (32, 2, 8, 3, 4160)])
+def test_a_token_without_comparable_scores_stays_alone(E, top, count, keep, width):
+    """bf16: a sequence whose activations are NaN (its router knows no largest score) beside one that is not - pairs one by one, norm and choice in one launch, sorted pairs with and without tables,
+    tiles of a prompt. It names experts that exist, and the other's logits are what they are in finite company, to the bit"""
+    c = one(scan(inner=64, mlp=moe(E, top, count, keep, 16)), width=width, vocab=200)
+    w = weights_for(c, "bfloat16", 3)
+    w["embed"] = w["embed"].copy()
+    w["embed"][0] = np.nan
+    _, _, m = model("route", "bfloat16", c, 3, w, fresh=True, max_tokens=256, n_seq=4, pool_tokens=1024)
+    rng = np.random.default_rng(E)
+    for n, k in ((1, 1), (2, 2), (1, 4), (7, 9), (20, 30), (30, 40), (100, 100)):
+        good = rng.integers(1, 200, n).astype(np.int32)
+        out = []
+        for other in (rng.integers(1, 200, k), np.zeros(k)):
+            lg = torch.empty((n + k, 200), device="cuda")
+            a, b = m.seq_new(), m.seq_new()
+            m.batch([(a, good, list(range(n))), (b, other.astype(np.int32), list(range(k)))], logits=lg)
+            m.seq_free(a)
+            m.seq_free(b)
+            out.append(lg)
+        assert torch.isfinite(out[0]).all() and torch.isnan(out[1][n:]).all() and torch.equal(out[0][:n], out[1][:n]), (n, k)
+    m.close()
+
+
 @pytest.mark.parametrize("heads,dim,kv_rank", [(3, 64, 64), (2, 65, 40), (5, 128, 130), (1, 192, 100), (2, 193, 64), (3, 256, 57)])
 def test_latent_queries_of_short_heads(heads, dim, kv_rank):
     """bf16: queries into the latents' space, a wave per 16 rows of a head: one to four 64-value blocks, latents that fill their rows and that do not, one and several tiles of 16 tokens"""
