@@ -372,6 +372,7 @@ int rgb_log2_for(int nrg) { return nrg >= 5 ? 3 : nrg >= 3 ? 2 : nrg == 2 ? 1 : 
 size_t lds_of(int type, int K) { return type == PM_Q8_0 ? (size_t) NWAVE * MT<PM_Q8_0>::WAVE_LDS : (size_t) (K / 256 + 1) * 128 + NWAVE * MT<PM_Q5_K>::WAVE_LDS; }
 // one matrix of Q5_K or Q8_0 over up to 16 tokens (q: one job)
 int launch_16(const RowsP & q, int type, hipStream_t st) {
+    if (q.T > 16) return -5;
     const int cus = pm_device_cus(), N = q.job[0].N, grid = N / 32 >= cus ? cus : (N + 31) / 32;
     MmqP p = {q.job[0].W, (long) pm_weight_row_stride(type, q.K), N, q.K, q.T, rgb_log2_for(((N + grid - 1) / grid + 31) / 32), q.t_off, type == PM_Q8_0 ? (const uint8_t *) q.dT : q.bsT, q.dT, q.qT,
               q.job[0].y, q.job[0].bias, q.job[0].resid};           // (Q8_0: bsT are the f32 activation scales [blk][32])
@@ -461,6 +462,19 @@ bool one_pass(int type, long N, int K, int T) {
     if (type == PM_Q5_K) return K > 4096;
     return T <= 24 ? K >= 2048 : K > 4096 || groups > 2;
 }
+// One matrix: tokens of the next pass when `left` of a call's T are left (32: up to the end of an activation table, 16: half of one), and its launch. Q4_K and Q6_K always have a form for what is
+// left. Q5_K and Q8_0 have one for more than 16 tokens on some shapes only, and by the number of tokens: a call whose first pass takes 32 may end in one of 17..24 that has none (Q8_0, K < 1024)
+int pass_tokens(int type, long N, int K, int T, int left) {
+    auto whole = [&](int n) { return type == PM_Q4_K || type == PM_Q6_K || one_pass(type, N, K, n) || pm_mmq_rows_takes(type, N, K, n); };
+    const int n = std::min(left, whole(std::min(T, 32)) || whole(32) ? 32 : 16);
+    return n <= 16 || whole(n) ? n : 16;
+}
+int launch_pass(const RowsP & q, int type, hipStream_t st) {
+    const bool k46 = type == PM_Q4_K || type == PM_Q6_K;
+    if (!k46 && one_pass(type, q.job[0].N, q.K, q.T)) return pm_launch_mmq_mid(q, &type, st);
+    if (pm_mmq_rows_takes(type, q.job[0].N, q.K, q.T)) return pm_launch_mmq_rows(q, &type, st);
+    return k46 ? pm_launch_mmq_mid(q, &type, st) : launch_16(q, type, st);
+}
 
 // Q8_0 weights x Q8_0 activations. xq: row-SoA Q8_0 rows (quantize.hip) or null and x_f32 is quantized first. Its tables
 // (operand-ordered values + f32 scales of both 32-slot halves, then a quantized copy of 64 f32 rows) are written by a prologue launch per call.
@@ -501,16 +515,13 @@ int launch_q80(const void * W, const void * xq, const float * x_f32, float * Y, 
         hipLaunchKernelGGL(mmq_prep_q80_kernel, dim3(nb), dim3(64), 0, st, (const uint8_t *) xq + (size_t) t0 * xrow, (long) xrow, K, T - t0 < 32 ? T - t0 : 32,
                            base + c * (qtab + dtab), (float *) (base + c * (qtab + dtab) + qtab));
     }
-    const int tmax = one_pass(PM_Q8_0, N, K, std::min(T, 32)) || pm_mmq_rows_takes(PM_Q8_0, N, K, T) || pm_mmq_rows_takes(PM_Q8_0, N, K, 32) ? 32 : 16;
-    for (int t0 = 0; t0 < T; t0 += tmax) {
-        const int tn = T - t0 < tmax ? T - t0 : tmax;
+    for (int t0 = 0, tn; t0 < T; t0 += tn) {
+        tn = pass_tokens(PM_Q8_0, N, K, T, T - t0);
         uint8_t * tab = base + (t0 / 32) * (qtab + dtab);
         RowsP q = {};
         q.job[0] = {(const uint8_t *) W, Y + (size_t) t0 * N, bias, resid ? resid + (size_t) t0 * N : nullptr, N};
         q.njobs = 1; q.K = K; q.T = tn; q.t_off = t0 % 32; q.qT = tab; q.dT = (const float *) (tab + qtab);
-        const int ty = PM_Q8_0;
-        const bool once = one_pass(PM_Q8_0, N, K, tn);
-        if (!once && pm_mmq_rows_takes(PM_Q8_0, N, K, tn) ? pm_launch_mmq_rows(q, &ty, st) : once ? pm_launch_mmq_mid(q, &ty, st) : launch_16(q, ty, st)) return -3;
+        if (launch_pass(q, PM_Q8_0, st)) return -3;
     }
     return 0;
 }
@@ -571,15 +582,13 @@ int pm_launch_mmq_i8(int type, const void * W, const void * xq, const float * x_
         xq = q;
     }
     if (!reuse_prep) launch_prep(sc, xq, K, T, st);
-    const int tmax = type != PM_Q5_K || one_pass(type, N, K, std::min(T, 32)) || pm_mmq_rows_takes(type, N, K, T) || pm_mmq_rows_takes(type, N, K, 32) ? 32 : 16;
-    for (int t0 = 0, c = 0; t0 < T; t0 += tmax, ++c) {
-        const int tn = T - t0 < tmax ? T - t0 : tmax;
+    for (int t0 = 0, tn; t0 < T; t0 += tn) {
+        tn = pass_tokens(type, N, K, T, T - t0);
         uint8_t * bsT = sc->p + (t0 / 32) * tab; float * dT = (float *) (bsT + (size_t) nsb * 1024);    // tables are per 32 tokens
         RowsP q = {};
         q.job[0] = {(const uint8_t *) W, Y + (size_t) t0 * N, bias, resid ? resid + (size_t) t0 * N : nullptr, N};
         q.njobs = 1; q.K = K; q.T = tn; q.t_off = t0 % 32; q.qT = sc->p + scr_q_off(K) + (size_t) (t0 / 32) * nsb * 8192; q.bsT = bsT; q.dT = dT;
-        const bool once = type != PM_Q5_K || one_pass(type, N, K, tn);
-        if (!(type == PM_Q5_K && once) && pm_mmq_rows_takes(type, N, K, tn) ? pm_launch_mmq_rows(q, &type, st) : once ? pm_launch_mmq_mid(q, &type, st) : launch_16(q, type, st)) return -3;
+        if (launch_pass(q, type, st)) return -3;
     }
     return 0;
 }

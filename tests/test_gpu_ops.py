@@ -1,6 +1,7 @@
 """GPU parity tests (run with -m gpu on an MI355X): every op goes through the C ABI of
 libprima_mi355.so and is compared with the CPU oracle on the same seeded inputs.
 Integer / byte results: bit-exact. Float results: tolerance stated per test."""
+import ctypes as C
 import os
 
 import numpy as np
@@ -1621,3 +1622,24 @@ def test_small_batch_cells_at_their_edges(P, oracle, t):
             ws = [P.upload_weight(t, b.reshape(N, rb)[:n0], K, n0), P.upload_weight(t, b.reshape(N, rb)[n0:], K, N - n0)]
             y3 = np.concatenate([v.cpu().numpy() for v in P.mul_mat_small_multi(ws, xq, T)], axis=1)
             assert np.allclose(y3[:, rows], want, **tol), (K, N, T, np.abs(y3[:, rows] - want).max())
+
+
+@pytest.mark.parametrize("t", [Q4_K, Q5_K, Q6_K, Q8_0])
+def test_small_batches_of_more_than_one_pass(P, oracle, t):
+    """33..64 tokens of one matrix: passes of 32 and of 16, and a last pass of any width, on each of the three kernels (which, by rows, K and tokens: test_host_launches.py). Every token against the
+    oracle, inside the bound of the other small-batch products; rows the oracle has not seen: written."""
+    rng = np.random.default_rng(8200 + t)
+    for K, N, Ts in ((768 if t != Q8_0 else 896, 12288, (33, 48, 49, 52, 56, 57, 64)), (512, 9000, (50, 41)), (2048, 12300, (52, 36)), (4096, 4096, (52, 63)), (4608, 9000, (49, 64)), (1024, 16384, (56, 40))):
+        b = rand_blocks(t, N, K, rng)
+        w = P.upload_weight(t, b, K, N)
+        rows = np.unique(np.concatenate([np.arange(20), np.arange(N - 20, N), rng.integers(0, N, 40)]))                    # (the oracle is a scalar program)
+        x = rng.normal(0, 1, (64, K)).astype(np.float32)
+        want = oracle.mul_mat(t, b.reshape(N, b.size // N)[rows].copy(), K, len(rows), x)
+        for T in Ts:
+            xd, y = _dev(P, x[:T]), _dev(P, np.full((T, N), np.nan, np.float32))
+            f = P.L.load().pm355_mul_mat_q_small
+            f.restype, f.argtypes = C.c_int, [C.c_int, C.c_void_p, C.c_int64, C.c_int64, C.c_void_p, C.c_void_p, C.c_int64, C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p]
+            assert f(w.type, w.data.data_ptr(), K, N, None, xd.data_ptr(), T, y.data_ptr(), None, None, P.stream_ptr()) == 0
+            y = y.cpu().numpy()
+            assert np.isfinite(y).all(), (K, N, T, np.flatnonzero(~np.isfinite(y).all(1)))
+            assert np.allclose(y[:, rows], want[:T], rtol=2e-5, atol=2e-5 * np.sqrt(max(K, 4096) / 4096)), (K, N, T, np.abs(y[:, rows] - want[:T]).max())

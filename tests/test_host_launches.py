@@ -217,3 +217,29 @@ for t, T, K, N, want in ((Q4, 12, 2048, 4096, I), (Q4, 12, 3072, 4096, R), (Q4, 
     assert one(t, N, K, T) == want, (t, T, K, N, one(t, N, K, T))
 print("ok")
 """)
+
+
+def test_passes_of_a_product_hold_all_tokens(run):
+    """1..64 tokens, one matrix: the launched kernels have room for every token (their tiles' tokens are in the names), and only the last pass is not full"""
+    run(COMMON + r"""
+lib = C.CDLL(sys.argv[2])
+f = lib.pm355_mul_mat_q_small
+f.argtypes = [C.c_int, C.c_void_p, C.c_int64, C.c_int64, C.c_void_p, C.c_void_p, C.c_int64, C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p]
+at = C.addressof(C.create_string_buffer(256))
+def room(name):
+    m = re.search(r"mmq_(rows|mid|i8)_kernel<(.*?)>", name)
+    if not m: return 0
+    a = m.group(2).split(", ")
+    return 8 * int(a[2]) if m.group(1) == "rows" else 2 * int(a[2] if len(a) == 4 else a[1])     # groups of 8 tokens; result registers of 2
+short = []
+for t in (12, 13, 14, 8):
+    for N in (17, 4096, 4097, 8192, 8193, 12288, 16384, 32000, 57344, 151936):
+        for K in (512, 768, 1024, 1536, 2048, 3072, 4096, 7168, 14336) + ((544, 896, 992) if t == 8 else ()):
+            for T in range(1, 65):
+                shim.shim_forget()
+                assert f(t, at, K, N, at, None, T, at, None, None, 1) == 0
+                r = [x for x in map(room, (n for _, n, _ in launches())) if x]
+                if sum(r) < T or sum(r[:-1]) >= T or any(x not in (16, 32) for x in r[:-1]): short.append((t, N, K, T, r))
+assert not short, (len(short), short[:20])
+print("ok")
+""")
