@@ -482,10 +482,12 @@ __device__ __forceinline__ void mmq_i8_body(const RowsP & p, const RowsJob & job
         if constexpr (AL) ld.put_a(a, 0, 0);
 #pragma unroll
         for (int f = 0; f < HP<TYPE, NV, AL>; ++f) if (f < HS) ld.put_h(h[f], d[f], 0, (f << ld.kl) + kp);
+        // (up to two steps have no third tile: the products don't wait until its requests, for nothing, are out. Q6_K 10240 x 1536 at 8 tokens 10.5 us, now 9.8)
+        if (total <= 2) meet();
         if constexpr (AL) { PIN; ld.load_a(a); }
         PIN;
         ld.template load<true>(T0);
-        meet();
+        if (total > 2) meet();
         auto step = [&](Tile<TYPE> & T, int s) __attribute__((always_inline)) {     // (s: where the next tile goes)
             PIN;
             ld.template put<true>(T, s);
@@ -496,11 +498,13 @@ __device__ __forceinline__ void mmq_i8_body(const RowsP & p, const RowsJob & job
             meet();
             if (n == 1) meet();
         };
-        for (int s = 0; s < total; s += 2) {
+        for (int s = 1; s < total; s += 2) {
             step(T1, 1);
             if (s + 1 >= total) break;
             step(T0, 0);
         }
+        meet();                                                     // the last tiles' products
+        if (n == 1) meet();
         return;
     }
     // ---- products: wave (cell, half of a pair)
