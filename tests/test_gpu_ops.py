@@ -383,6 +383,20 @@ def test_small_batch_matmul_wv_of_another_type_in_the_same_grid(P, oracle, tv):
         P.mul_mat_small_mixed(ws, xq, 40)
 
 
+@pytest.mark.parametrize("K,Ns,T", [(512, (8192, 1024, 1024), 12), (768, (8192, 1024, 1024), 16), (512, (8160, 1020, 1028), 9), (2304, (8192, 1024, 1030), 3)])
+def test_last_matrix_of_two_types_in_slices_of_whole_row_groups(P, oracle, K, Ns, T):
+    """wv of Q5_K whose share of the workgroups would make slices a row or two longer than 32 (the first matrix gives it some of its own), short rows of one and two steps: the bound of the other
+    mixed launches"""
+    rng = np.random.default_rng(K + T)
+    types = (Q4_K, Q4_K, Q5_K)
+    blocks = [rand_blocks(t, N, K, rng) for t, N in zip(types, Ns)]
+    x = rng.normal(0, 1, (T, K)).astype(np.float32)
+    xq = P.quantize_act(_dev(P, x), P.vec_dot_act_type(Q4_K))
+    ys = P.mul_mat_small_mixed([P.upload_weight(t, b, K, N) for t, b, N in zip(types, blocks, Ns)], xq, T)
+    for t, b, N, y in zip(types, blocks, Ns, ys):
+        assert np.allclose(y.cpu().numpy(), oracle.mul_mat(t, b, K, N, x), rtol=2e-5, atol=2e-5 * np.sqrt(K / 4096)), (t, N)
+
+
 def test_rms_norm_matches_oracle(P, oracle):
     rng = np.random.default_rng(26)
     for K, eps in ((4096, 1e-5), (8192, 1e-6)):
