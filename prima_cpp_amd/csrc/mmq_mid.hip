@@ -5,16 +5,16 @@
 // The loader has two tiles (32 rows x a pair, full 128-byte lines) on their way in its registers and two in LDS, where the others read them in matrix-operand order; the workgroup's twelve waves
 // meet once per step. So no multiplying wave ever waits in the issue of a request (with all waves loading their own tiles, each request held its wave up for 60-260 cycles and the waves' loads,
 // LDS copies and products added up instead of overlapping: of 7 us per step of 72B's ffn_gate | ffn_up at 23 tokens 5 were products), and LDS tiles are turned by XOR, free of padding.
-//   * more than 64 rows a workgroup (AL): a cell is a row group, all four work on the same pair; its activations come into LDS once for all of them (each wave for itself out of L2: 12 of 67 us
+//   * most often more than 64 rows a workgroup (AL): a cell is a row group, all four work on the same pair; its activations come into LDS once for all of them (each wave for itself out of L2: 12 of 67 us
 //     of 57344 x 8192 Q4_K, 20 of 125 of 59136 x 8192 Q6_K)
-//   * up to 64 (32): two (four) cells share a row group and take pairs next to each other; a pair's activations are needed by one wave only, which loads them straight into operand registers
+//   * up to 64 (32), and some others (mmq_i8_rows): two (four) cells share a row group and take pairs next to each other; a pair's activations are needed by one wave only, which loads them straight into operand registers
 // Scales come in blocks of up to four pairs, whole lines of them (32 bytes of a line each time, they were a third of the lines that a CU asks for: 14 of 119 us of Q6_K).
 // An integer product's results are read behind the next one's start, one v_mad_i32_i24 each (mad24), for up to 8, 16, 24 or 32 tokens.
 // Bound by the weights' stream (Q4_K 6.2 TB/s between the first tile, 5 us, and the last sums) and, Q6_K, by vector work (400 instructions per 32 rows x 256 k at 24 tokens).
 // us, the form that it replaced (mmq_i8.hip's of then) / here, at 23 tokens: 59136 x 8192 Q6_K 132 / 97, 10240 x 8192 40 / 30, 8192 x 8192 26 / 21, 8192 x 28672 70 / 57; 57344 x 8192 Q4_K
-// 78 / 57, 10240 x 8192 23 / 18, 8192 x 28672 40 / 33, 28672 x 4096 27 / 20; 128256 x 4096 Q6_K 160 / 107; 8192 x 29568 Q8_0 76 / 55. Weights out of memory, one matrix of 70..57344 rows, K =
-// 512..28672, time here / time there in the geometric mean: Q4_K up to 8 tokens 0.94, 16 0.91, 32 0.88, several matrices 0.87 0.82 0.80; Q6_K 0.98 0.94 0.84, 0.91 0.86 0.77 (slower: K = 512 up
-// to 8192 rows by 0.4 us, and Q6_K 10240 x 5120 at 8 tokens 18.2 / 19.5 us)
+// 78 / 57, 10240 x 8192 23 / 18, 8192 x 28672 40 / 33, 28672 x 4096 27 / 20; 128256 x 4096 Q6_K 160 / 107; 8192 x 29568 Q8_0 76 / 55. Weights out of memory, one matrix of 70..128256 rows, K =
+// 512..28672, time here / time there in the geometric mean: Q4_K up to 8 tokens 0.91, 16 0.87, 32 0.85, several matrices 0.83 0.80 0.77; Q6_K 0.89 0.87 0.81, 0.85 0.82 0.76 (slower: Q6_K
+// 10240 x 5120 up to 8 tokens 17.4 / 18.0 us, Q4_K 57344 x 14336 at 8 tokens 80.5 / 83)
 #include "pm355_device.h"
 #include "pm355_kernels.h"
 #include "pm355_mmq_rows.h"
@@ -607,8 +607,13 @@ __device__ __forceinline__ void mmq_i8_rows(const RowsP & p, const RowsJob & job
     constexpr int STEP = EPI ? 2 : 1;
     const int r0 = STEP * (w * job.each + min(w, job.more)), r1 = STEP * ((w + 1) * job.each + min(w + 1, job.more));
     const int most = STEP * (job.each + (job.more != 0));          // of the matrix' workgroups: one order of the sums for all its rows
-    if (most > 64) mmq_i8_body<TYPE, NV, EPI, true>(p, job, r0, r1, 2, ji, smem);
-    else mmq_i8_body<TYPE, NV, EPI, false>(p, job, r0, r1, most > 32 ? 1 : 0, ji, smem);
+    const int groups = (most + 31) / 32;
+    // five or six: rounds of four leave three or two cells without rows every other round; in rounds of two, us of rounds of four / here: Q4_K 33024 x 5120 at 8 tokens 32.6 / 25.3, 36864 x 14336
+    // 73 / 54, Q6_K 36864 x 8192 at 24 tokens 86 / 73 (the other lengths and numbers of tokens alike). Three: longer rows of Q4_K over up to 8 tokens, which have little to gain from activations in
+    // LDS, one group after the other: 17000 x 14336 34.7 / 31.1, 20480 x 5120 18.7 / 17.2 (512 .. 2048 values 0.84 .. 1.0 of that here, more tokens and Q6_K 0.85 .. 0.95)
+    if (TYPE == PM_Q4_K && NV == 4 && groups == 3 && p.K > 4096) mmq_i8_body<TYPE, NV, EPI, false>(p, job, r0, r1, 0, ji, smem);
+    else if (groups > 2 && groups != 5 && groups != 6) mmq_i8_body<TYPE, NV, EPI, true>(p, job, r0, r1, 2, ji, smem);
+    else mmq_i8_body<TYPE, NV, EPI, false>(p, job, r0, r1, groups > 1 ? 1 : 0, ji, smem);
 }
 
 // (named as mmq_i8.hip's: the form with 32-row groups. TA: the type of all jobs but the last, TB: of the last one; first1, first2: first workgroups of the second and third job)

@@ -1638,6 +1638,19 @@ def test_small_batch_cells_at_their_edges(P, oracle, t):
             assert np.allclose(y3[:, rows], want, **tol), (K, N, T, np.abs(y3[:, rows] - want).max())
 
 
+@pytest.mark.parametrize("t", [Q4_K, Q6_K])
+@pytest.mark.parametrize("K,N,T", [(4352, 16500, 8), (5120, 24500, 5), (9472, 17000, 2), (512, 36000, 3), (768, 33024, 8), (5120, 45000, 8), (4608, 37001, 16), (2304, 49100, 24), (1792, 33100, 32)])
+def test_small_batch_cells_in_rounds(P, oracle, K, N, T, t):
+    """mmq_mid.hip: three, five and six row groups a workgroup, one or two at a time; the last round full, with one group, with a group of a few rows. The bound of the others"""
+    rng = np.random.default_rng(K + N + T)
+    b = rand_blocks(t, N, K, rng)
+    x = rng.normal(0, 1, (T, K)).astype(np.float32)
+    rows = np.unique(np.concatenate([np.arange(200), np.arange(N - 200, N), rng.integers(0, N, 200)]))                     # (the oracle is a scalar program)
+    want = oracle.mul_mat(t, b.reshape(N, b.size // N)[rows].copy(), K, len(rows), x)
+    y = P.mul_mat_small(P.upload_weight(t, b, K, N), x=_dev(P, x)).cpu().numpy()
+    assert np.isfinite(y).all() and np.allclose(y[:, rows], want, rtol=2e-5, atol=2e-5 * np.sqrt(max(K, 4096) / 4096)), np.abs(y[:, rows] - want).max()
+
+
 @pytest.mark.parametrize("t", [Q4_K, Q5_K, Q6_K, Q8_0])
 def test_small_batches_of_more_than_one_pass(P, oracle, t):
     """33..64 tokens of one matrix: passes of 32 and of 16, and a last pass of any width, on each of the three kernels (which, by rows, K and tokens: test_host_launches.py). Every token against the
