@@ -312,6 +312,7 @@ template <int MI, int NI, bool EXP> __global__ __launch_bounds__(512) void dense
 #pragma unroll
         for (int m = 0; m < MI; ++m) asm volatile("" : "+v"(pair[m]), "+v"(weight[m]));
     }
+    const bool four = p.ldy % 4 == 0 && ((uintptr_t) p.y & 15) == 0;      // (four outputs together where rows and their start allow it)
     auto put = [&](auto * y, bool whole) __attribute__((always_inline)) {
         typedef std::remove_reference_t<decltype(*y)> Y;
 #pragma unroll
@@ -328,18 +329,18 @@ template <int MI, int NI, bool EXP> __global__ __launch_bounds__(512) void dense
                     for (int e = 0; e < 4; ++e) v[e] = act_apply(p.act_fn, v[e]);
                 }
                 if constexpr (EXP) v *= weight[m];
-                if (whole) {
+                const int col = n0 + (wn * NI + n) * 16 + g * 4;
+                if (whole || (four && col + 4 <= p.n_store)) {
                     if constexpr (sizeof(Y) == 4) *(PM_G f32x4 *) (row + n * 16) = v;
                     else *(PM_G u32x2 *) (row + n * 16) = u32x2{(uint32_t) f2bf(v[0]) | (uint32_t) f2bf(v[1]) << 16, (uint32_t) f2bf(v[2]) | (uint32_t) f2bf(v[3]) << 16};
                 } else {
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) if (n0 + (wn * NI + n) * 16 + g * 4 + e < p.n_store) st_g(row + n * 16 + e, from_f<Y>(v[e]));
+                    for (int e = 0; e < 4; ++e) if (col + e < p.n_store) st_g(row + n * 16 + e, from_f<Y>(v[e]));
                 }
             }
         }
     };
-    // (four outputs together where rows and their start allow it)
-    const bool whole = n0 + BN <= p.n_store && p.ldy % 4 == 0 && ((uintptr_t) p.y & 15) == 0;
+    const bool whole = four && n0 + BN <= p.n_store;
     if (p.y_type == PM_BF16) { if (whole) put((uint16_t *) p.y, true); else put((uint16_t *) p.y, false); }
     else { if (whole) put((float *) p.y, true); else put((float *) p.y, false); }
 }
@@ -398,31 +399,42 @@ int pm_launch_dense_gemm(const pm_dense_args & a, hipStream_t st) {
     GemmP p = {};
     p.W = (const uint16_t *) a.W; p.X = (const uint16_t *) a.act; p.y = a.y; p.bias = a.bias; p.K = a.K; p.N = a.N; p.T = a.T; p.lda = a.lda; p.ldy = a.ldy; p.y_type = a.y_type;
     p.n_store = a.n_store; p.act_fn = a.act_fn;
-    // The tile whose rounds take the least time: us per 64-k step of a workgroup on a full chip, a CU to itself (two 128 x 128 tiles of the kernel with two stages share one), and what a round
-    // takes besides; half a chip of workgroups runs its steps in 0.77 of that. With too few tiles for the chip ranges of k go to different workgroups; their f32 sums are written and read again.
+    // The tile whose rounds take the least time. With too few tiles for the chip ranges of k go to different workgroups; their f32 sums are written, and added up by a launch of their own or by the
+    // norm behind the product (a workgroup per token, which reads 15 KB of them in a us).
     // Measured on 835 tokens, in a pass between other launches: 10240 x 4096 98 us in 160 tiles of 256 x 256, 79 in 240 of 160 x 256; 14336 x 4096 107 (224 of 256 x 256) / 100 (224 of 224 x
     // 256); 4096 x 14336 135 (224 of 128 x 128, four waves) / 90 and 6 more in the norm behind it (64 of 224 x 256 in four ranges); 4096 x 4096 44 / 41 (128 x 128 tiles by eight waves)
     const int steps = a.K >> 6, ldp = a.parts ? a.ldy : (a.n_store + 3) / 4 * 4;
     const bool may_split = a.split && (!a.parts || a.act_fn == PM355_ACT_NONE);
-    static const struct { int bm, bn, per_cu; float step; } forms[] = {{128, 128, 1, 0.63f}, {160, 256, 1, 1.28f}, {224, 256, 1, 1.62f}, {256, 256, 1, 1.77f}, {128, 128, 2, 1.04f}};
+    auto summed = [&](int s) { return 3.7f + (float) (s + 1) * a.T * ldp * 4.6e-7f; };                                              // us of the launch that adds them up, and
+    auto normed = [&](int s) { return std::max((float) (s - 1) * ldp / 3900, (float) (s - 1) * a.T * ldp * 6.7e-7f); };             // of what the norm takes longer
     int form = 0, splits = 1;
     float best = INFINITY;
-    for (int f = 0; f < 5; ++f) {
-        const int64_t tiles = (int64_t) ((a.T + forms[f].bm - 1) / forms[f].bm) * ((a.n_store + forms[f].bn - 1) / forms[f].bn), room = (int64_t) pm_device_cus() * forms[f].per_cu;
-        for (int s = 1; s == 1 || (f < 4 && may_split && s * tiles <= room && s * 4 <= steps && (size_t) s * a.T * ldp <= a.split_floats); ++s) {
-            const int64_t all = tiles * s, last = all % room;
-            const float rounds = (float) (all / room) + (last ? 0.55f + 0.45f * (float) last / (float) room : 0.0f);      // (in time of a full one's steps)
-            const float t = rounds * (float) ((steps + s - 1) / s) * forms[f].step + (float) ((all + room - 1) / room) * 5.0f + (s > 1 ? (float) s * a.T * ldp * 8 / 4.5e6f + (a.parts ? 0.0f : 5.0f) : 0.0f);
+    for (int f = 0; f < (int) std::size(forms); ++f) {
+        const int nt = (a.T + forms[f].bm - 1) / forms[f].bm;
+        const int64_t tiles = (int64_t) nt * ((a.n_store + forms[f].bn - 1) / forms[f].bn), room = (int64_t) pm_device_cus() * forms[f].per_cu;
+        if (forms[f].per_cu > 1 && tiles <= pm_device_cus()) continue;
+        for (int s = 1; s == 1 || (forms[f].tile && may_split && s * tiles <= room && s * 4 <= steps && (size_t) s * a.T * ldp <= a.split_floats); ++s) {
+            float t = forms[f].us(a.T, nt, tiles * s, room, (steps + s - 1) / s, (float) s * a.T * ldp, s > 1 || a.y_type == PM_F32);
+            if (s > 1) t += a.parts ? std::min(summed(s), normed(s)) : summed(s);
             if (t < best) { best = t; form = f; splits = s; }
         }
     }
-    auto go = [&]() { return form == 0 ? launch_tile<4, 2>(p, st) : form == 1 ? launch_tile<5, 4>(p, st) : form == 2 ? launch_tile<7, 4>(p, st) : form == 3 ? launch_tile<8, 4>(p, st) :
-                             launch_stages<128, 128, 64, 64, 2, DENSE>(p, st); };
+    auto go = [&]() -> int {
+        switch (form) {
+            case 0: return launch_tile<4, 2>(p, st);
+            case 1: return launch_tile<5, 4>(p, st);
+            case 2: return launch_tile<7, 4>(p, st);
+            case 3: return launch_tile<8, 4>(p, st);
+            case 4: return launch_stages<128, 128, 64, 64, 2, DENSE>(p, st);
+            case 5: return launch_stages<256, 256, 128, 64, 2, DENSE>(p, st);
+            default: return launch_stages<128, 128, 64, 64, 4, DENSE>(p, st);
+        }
+    };
     if (a.parts) *a.parts = 0;
     if (splits > 1) {
         p.split_steps = (steps + splits - 1) / splits; p.splits = (steps + p.split_steps - 1) / p.split_steps;
         p.y = a.split; p.ldy = ldp; p.y_type = PM_F32; p.act_fn = PM355_ACT_NONE;
-        if (a.parts) { *a.parts = p.splits; p.rows = 1; return go(); }
+        if (a.parts && normed(p.splits) <= summed(p.splits)) { *a.parts = p.splits; p.rows = 1; return go(); }
         p.bias = nullptr;
         go();
         hipLaunchKernelGGL(reduce_kernel, dim3((unsigned) (((long) a.T * (ldp / 4) + 255) / 256)), dim3(256), 0, st, a.split, p.splits, a.T, ldp, a.bias, a.act_fn, a.y, a.ldy, a.y_type, a.n_store);
