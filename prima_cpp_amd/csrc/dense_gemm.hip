@@ -2,11 +2,13 @@
 // Both operands travel by LDS-DMA as whole 128-byte lines (64 k per stage) into two stages; 16-byte chunks are XOR-swizzled on the source side (chunk c of row r at
 // c ^ ((r >> 1) & 7): the sixteen lanes a ds_read_b128 serves hit sixteen bank groups). One barrier per stage: behind it the stage of the previous step is free and takes
 // the next k-step's DMA, which has this step's MFMAs to land. Tiles of one XCD form compact blocks of the output so that its L2 serves both operands.
-// dense_tile_kernel: one matrix, tiles of 128 .. 256 tokens x 128 or 256 rows, chosen by the time their rounds take; experts with many pairs. dense_gemm_kernel: two 128 x 128 tiles per CU where
-// that is the quickest; experts (token tiles from the routing tables, rows gathered and scattered by pair); latent cache pages into keys and transposed values.
+// dense_tile_kernel: one matrix, tiles of 128 .. 256 tokens x 128 or 256 rows, chosen by the time their rounds take; experts with many pairs. dense_gemm_kernel: 128 x 128 and 256 x 256 tiles where
+// they are the quickest; experts (token tiles from the routing tables, rows gathered and scattered by pair); latent cache pages into keys and transposed values.
 #include "pm355_dense.h"
 #include "pm355_kernels.h"
 #include "../../include/prima_mi355.h"
+#include <algorithm>
+#include <iterator>
 #include <type_traits>
 
 namespace {
@@ -389,6 +391,27 @@ template <int KIND> int launch_128(const GemmP & p, hipStream_t st) {
     if constexpr (KIND != EXPERTS) if ((long) ((p.T + 127) / 128) * ((p.n_store + 127) / 128) <= 256) return launch_stages<128, 128, 64, 64, 4, KIND>(p, st);
     return launch_stages<128, 128, 64, 64, 2, KIND>(p, st);
 }
+
+// Forms of one matrix and the us they take: c per round of workgroups, out32 (out16) per MB of f32 (bf16) results, `rag` where the last token tile is not full, and per 64-k step `step`, of which
+// `fill` also where a workgroup runs alone, and `weights` for lines of W that no other token tile asks for. Least squares of the logarithms over 25 matrices of 512..14336 x 1024..32000, 65..4096
+// tokens, either type of results, up to 32 k ranges, weights out of memory and out of the last-level cache (residuals 5 to 10 %; the last three by 1 .. 3 % less, they are what the choice was between
+// before there were tiles). Choices are 0.5 .. 2 % in the mean from the best form of all; of 1752 products without ranges 30 are more than 3 % (12 % at most) behind the former choice, the mean is
+// 0.95 of its time.
+// The last three are dense_gemm_kernel's: two workgroups per CU, whose stores and steps overlap (257 x 8192 x 14336 out of the cache 92 us, in 160 x 256 tiles 125); 256 x 256 and 128 x 128 tiles of
+// short rows, which it stores in half the time (2048 x 1024 x 14336 68.7 us, dense_tile_kernel's 70.8; 128 x 512 x 8192 8.3 / 9.5)
+struct Form {
+    int bm, bn, per_cu; bool tile; float c, step, fill, weights, out32, out16, rag;
+    float us(int T, int nt, int64_t all, int64_t room, int steps, float values, bool f32) const {
+        const int64_t full = all / room, last = all % room;
+        const float part = (float) last / (float) room;
+        return (float) ((all + room - 1) / room) * c + values * (f32 ? 4e-6f * out32 : 2e-6f * out16) + (T % bm ? rag : 0.0f) +
+               (float) steps * ((float) full * (step + weights / nt) + (last ? step * (fill + (1.0f - fill) * part) + weights * part / nt : 0.0f));
+    }
+};
+constexpr Form forms[] = {{128, 128, 1, true, 4.8f, 0.468f, 0.911f, 0.177f, 0.139f, 0.0f, 0.33f}, {160, 256, 1, true, 7.8f, 0.953f, 0.896f, 0.123f, 0.13f, 0.072f, 0.0f},
+                          {224, 256, 1, true, 3.8f, 1.283f, 0.87f, 0.0f, 0.154f, 0.208f, 4.0f}, {256, 256, 1, true, 8.2f, 1.378f, 0.892f, 0.0f, 0.144f, 0.187f, 0.0f},
+                          {128, 128, 2, false, 1.4f, 0.87f, 0.474f, 0.53f, 0.116f, 0.14f, 1.44f}, {256, 256, 1, false, 5.0f, 1.49f, 0.792f, 0.083f, 0.09f, 0.075f, 1.65f},
+                          {128, 128, 1, false, 3.3f, 0.53f, 0.892f, 0.138f, 0.046f, 0.0f, 1.67f}};
 
 } // namespace
 

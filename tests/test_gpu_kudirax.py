@@ -160,6 +160,40 @@ def test_dense_mul_mat_prompt_tiles(T, K, n_store, pad):
         assert (y[:, n_store:] == 7.0).all()
 
 
+# tokens, values, rows, columns of y behind them: the form that one bf16 matrix takes (test_host_launches.py); last token tiles of a few tokens, rows that end inside a tile, inside four neighbouring
+# outputs and on them, rows of y that start on 16 bytes and that do not
+DENSE_FORMS = {(200, 1024, 4098, 0): "tile_kernel<4,2", (292, 512, 1000, 1): "tile_kernel<4,2", (835, 1024, 10201, 2): "tile_kernel<5,4", (835, 3072, 14281, 0): "tile_kernel<7,4",
+               (1024, 4096, 14340, 0): "tile_kernel<8,4", (1025, 4096, 14338, 3): "gemm_kernel<128,128,64,64,2", (897, 2048, 5001, 0): "gemm_kernel<128,128,64,64,2", (1000, 1024, 16001, 5): "gemm_kernel<256,256,128,64,2",
+               (2048, 1024, 14336, 0): "gemm_kernel<256,256,128,64,2", (128, 512, 8190, 0): "gemm_kernel<128,128,64,64,4", (129, 192, 33, 1): "gemm_kernel<128,128,64,64,4"}
+
+
+@pytest.mark.parametrize("T,K,n_store,pad", sorted(DENSE_FORMS))
+def test_dense_mul_mat_forms(T, K, n_store, pad):
+    import prima_cpp_amd.ops as O
+    N = (n_store + 63) // 64 * 64
+    g = torch.Generator(device="cuda").manual_seed(T + K)
+    w = (torch.randn(N, K, generator=g, device="cuda") / K ** 0.5).bfloat16()
+    x = torch.randn(T, K + 64, generator=g, device="cuda").bfloat16()[:, :K]
+    b = torch.randn(N, generator=g, device="cuda")
+    ref = (x.double() @ w.double().T)[:, :n_store]
+    for ydt, tol in ((torch.float32, 2e-6 * K ** 0.5), (torch.bfloat16, 1e-2)):
+        y = torch.full((T, N + pad), 7.0, dtype=ydt, device="cuda")
+        O.dense_mul_mat(w, x, y, n_store=n_store, bias=b)
+        want = ref + b.double()[:n_store]
+        assert ((y[:, :n_store].double() - want).abs() <= tol * (1 + want.abs())).all()
+        assert (y[:, n_store:] == 7.0).all()
+
+
+@pytest.mark.parametrize("T", [66, 100, 128, 130, 300])
+def test_k_ranges_of_a_wide_model(T):
+    """products whose k ranges the norm adds up and, with few tokens of wide rows, a launch of their own"""
+    c = config(layer(heads=4, kv=1, dim=64, vdim=130, size=400, mix=False, ff=4100), width=4200, vocab=90)
+    _, w, m = model("ranges", "bfloat16", c, 3, fresh=True, max_tokens=320, n_seq=1, pool_tokens=384)
+    toks = tokens(T, 90, T)
+    close(alone(m, toks), P.run(c, w, toks), "bfloat16")
+    m.close()
+
+
 @pytest.mark.parametrize("T,K,off_x,off_w", [(3, 1024, 4, 0), (8, 4096, 1, 0), (1, 8192, 0, 4), (5, 9216, 2, 2)])
 def test_dense_mul_mat_of_operands_that_do_not_start_on_16_bytes(T, K, off_x, off_w):
     import prima_cpp_amd.ops as O

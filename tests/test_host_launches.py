@@ -219,6 +219,26 @@ print("ok")
 """)
 
 
+def test_forms_of_one_dense_matrix(run):
+    """the shapes of test_gpu_kudirax.py's test_dense_mul_mat_forms take the forms that they are there for, of either type of results; every form is among them"""
+    from test_gpu_kudirax import DENSE_FORMS
+    assert len(set(DENSE_FORMS.values())) == 7
+    run(COMMON + "want = " + repr(DENSE_FORMS) + r"""
+lib = C.CDLL(sys.argv[2])
+f = lib.pm355_dense_mul_mat
+f.argtypes = [C.c_int, C.c_void_p, C.c_int64, C.c_int64, C.c_void_p, C.c_int64, C.c_int, C.c_void_p, C.c_int64, C.c_int, C.c_int64, C.c_void_p, C.c_int, C.c_void_p]
+at = (C.addressof(C.create_string_buffer(512)) + 255) // 256 * 256
+for (T, K, n, pad), form in want.items():
+    N = (n + 63) // 64 * 64
+    for y_type in (0, 30):
+        shim.shim_forget()
+        assert f(30, at, K, N, at, K, T, at, N + pad, y_type, n, None, 0, 1) == 0
+        names = [name.replace(" ", "") for _, name, _ in launches()]
+        assert len(names) == 1 and "dense_" + form in names[0], (T, K, n, names)
+print("ok")
+""")
+
+
 def test_passes_of_a_product_hold_all_tokens(run):
     """1..64 tokens, one matrix: the launched kernels have room for every token (their tiles' tokens are in the names), and only the last pass is not full"""
     run(COMMON + r"""
