@@ -8,6 +8,7 @@
 #include "pm355_dense.h"
 #include "pm355_kernels.h"
 #include "pm355_route.h"
+#include <algorithm>
 #include "../../include/prima_mi355.h"
 
 namespace {
@@ -144,38 +145,48 @@ template <typename T, int NT, int RM, int SRC, int EXP> __global__ __launch_boun
     }
     if constexpr (EXP == CONCAT) { const int t = blockIdx.y; cat = uniform_const_ptr(p.r.id + t * p.r.top); base = t; act += (size_t) t * p.lda; t0 = 0; n_tok = 1; }
     __shared__ int local[EXP == SORTED ? PM_ROUTE_PAIRS : 1];          // SORTED without tables: the expert's pairs
+    // SORTED: the workgroup's experts are the blockIdx.y-th, (blockIdx.y + gridDim.y)-th, .. that have pairs
+    constexpr int G = EXP == SORTED ? PM_ROUTE_PAIRS / 64 : 1;
+    int mine_e[G], ye = blockIdx.y, n_on = 0;
+    uint64_t on = 0;
     if constexpr (EXP == SORTED) {
-        int e;
-        if (p.r.logits) {
-            if ((int) blockIdx.y >= ld_g(p.r.active)) return;
-            e = __builtin_amdgcn_readfirstlane(ld_g(p.r.active + 1 + blockIdx.y));
-            base = __builtin_amdgcn_readfirstlane(ld_g(p.r.off + e)); n_tok = __builtin_amdgcn_readfirstlane(ld_g(p.r.off + e + 1)) - base;
-        } else {
-            // up to PM_ROUTE_PAIRS pairs of up to 64 experts: a lane per pair, 64 at a time; this workgroup's expert is the blockIdx.y-th that has one. (One round of loads in front of the weights
-            // instead of three, one behind the other, and no launch that sorts; every wave finds the same)
-            constexpr int G = PM_ROUTE_PAIRS / 64;
+        if (p.r.logits) n_on = __builtin_amdgcn_readfirstlane(ld_g(p.r.active));
+        else {
+            // up to PM_ROUTE_PAIRS pairs of up to 64 experts: a lane per pair, 64 at a time. (One round of loads in front of the weights instead of three, one behind the other, and no launch that
+            // sorts; every wave finds the same)
             const int pairs = p.T * p.r.top;
-            int mine[G];
 #pragma unroll
-            for (int i = 0; i < G; ++i) mine[i] = i * 64 + lane < pairs ? ld_g(p.r.id + i * 64 + lane) : 64;       // (64: no expert)
+            for (int i = 0; i < G; ++i) { mine_e[i] = 64; if (i * 64 < pairs && i * 64 + lane < pairs) mine_e[i] = ld_g(p.r.id + i * 64 + lane); }       // (64: no expert)
             uint32_t has[2] = {0, 0};
 #pragma unroll
-            for (int i = 0; i < G; ++i) { has[0] |= mine[i] < 32 ? 1u << mine[i] : 0u; has[1] |= mine[i] >= 32 && mine[i] < 64 ? 1u << (mine[i] - 32) : 0u; }
-            const uint64_t on = (uint64_t) wave_or(has[1]) << 32 | wave_or(has[0]);
-            if ((int) blockIdx.y >= __popcll(on)) return;
-            e = __builtin_ctzll(__builtin_amdgcn_ballot_w64((on >> lane & 1) && __popcll(on & ((1ull << lane) - 1)) == (int) blockIdx.y));
+            for (int i = 0; i < G; ++i)
+                if (i * 64 < pairs) { has[0] |= mine_e[i] < 32 ? 1u << mine_e[i] : 0u; has[1] |= mine_e[i] >= 32 && mine_e[i] < 64 ? 1u << (mine_e[i] - 32) : 0u; }
+            on = (p.r.E > 32 ? (uint64_t) wave_or(has[1]) << 32 : 0) | wave_or(has[0]);
+            n_on = __popcll(on);
+        }
+        if (ye >= n_on) return;
+    }
+    auto take = [&]() __attribute__((always_inline)) {                  // the ye-th of them
+        int e;
+        if (p.r.logits) {
+            e = __builtin_amdgcn_readfirstlane(ld_g(p.r.active + 1 + ye));
+            base = __builtin_amdgcn_readfirstlane(ld_g(p.r.off + e)); n_tok = __builtin_amdgcn_readfirstlane(ld_g(p.r.off + e + 1)) - base;
+        } else {
+            e = __builtin_ctzll(__builtin_amdgcn_ballot_w64((on >> lane & 1) && __popcll(on & ((1ull << lane) - 1)) == ye));
             base = 0; n_tok = 0;
 #pragma unroll
             for (int i = 0; i < G; ++i) {
-                const uint64_t its = __builtin_amdgcn_ballot_w64(mine[i] == e);
-                base += __popcll(__builtin_amdgcn_ballot_w64(mine[i] < e));
+                if (i * 64 >= p.T * p.r.top) break;
+                const uint64_t its = __builtin_amdgcn_ballot_w64(mine_e[i] == e);
+                base += __popcll(__builtin_amdgcn_ballot_w64(mine_e[i] < e));
                 if (its >> lane & 1) local[n_tok + __popcll(its & ((1ull << lane) - 1))] = i * 64 + lane;
                 n_tok += __popcll(its);
             }
             wave_fence();
         }
-        W += (size_t) e * p.e_stride; t0 = 0;
-    }
+        W = (const T *) p.W + (size_t) e * p.e_stride; t0 = 0;
+    };
+    if constexpr (EXP == SORTED) take();
     // sorted pair base + t
     auto pair_at = [&](int t) __attribute__((always_inline)) -> int { return EXP == SORTED && !p.r.logits ? local[t] : ld_g(p.r.order + base + t); };
     if (EXP == DENSE && p.group) act += (size_t) (r0 / p.group) * p.g_act;
@@ -188,13 +199,13 @@ template <typename T, int NT, int RM, int SRC, int EXP> __global__ __launch_boun
     const int nb1 = p.K >> 6, nblk = EXP == CONCAT ? nb1 * p.r.top : nb1, mine = (nblk - wave + 7) >> 3;      // 64-k blocks wave, wave + 8, ..
     const int koff = (LINE ? (lr >> 3) * 32 : 0) + g * EPL;
     const T * wrow[RM];
-#pragma unroll
-    for (int m = 0; m < RM; ++m) wrow[m] = W + (size_t) (r0 + m * ROWS + lr % ROWS) * p.K + koff;
     auto w_at = [&](int blk) __attribute__((always_inline)) -> int64_t {      // of a 64-k block in a row of W
         if constexpr (EXP == CONCAT) { const int s = blk / nb1; return (int64_t) cat[s] * p.e_stride + ((blk - s * nb1) << 6); }
         return blk << 6;
     };
     do {
+#pragma unroll
+    for (int m = 0; m < RM; ++m) wrow[m] = W + (size_t) (r0 + m * ROWS + lr % ROWS) * p.K + koff;
     const T * arow[NT];
     if (SRC == 0) {
 #pragma unroll
@@ -337,7 +348,11 @@ template <typename T, int NT, int RM, int SRC, int EXP> __global__ __launch_boun
         }
         st_type(p.y, (size_t) tok * p.ldy + col, p.y_type, v);
     }
-    if (EXP == SORTED) { t0 += TOK * NT; __syncthreads(); }
+    if constexpr (EXP == SORTED) {
+        t0 += TOK * NT;
+        __syncthreads();
+        if (t0 >= n_tok && (ye += gridDim.y) < n_on) take();
+    }
     } while (EXP == SORTED && t0 < n_tok);
 }
 
@@ -498,6 +513,9 @@ template <typename T, int NT, int RM, int SRC, int EXP = DENSE> int launch(const
     size_t lds = (size_t) 8 * NT * RM * 1024 + (SRC ? (size_t) here * ((size_t) p.K * (EXP == CONCAT ? p.r.top : 1) * sizeof(T) + 16) : 0);
     if (EXP == PAIR && lds < 8192) lds = 8192;
     pm_allow_big_lds((const void *) dense_small_kernel<T, NT, RM, SRC, EXP>, lds);
+    // Sorted experts: two workgroups per CU, which take their experts in turn. One per row tile and expert that there could be (`y`), most of them without tokens, were 14336 of 512 threads for 8 tokens
+    // of 32 experts of 4096 x 3584: 102 us with tables and 112 without, 96 so; of 2048 x 2048 at 24 tokens 56 and 56, now 47. (768 .. 4096 of them: up to 20 % more, whole rounds or not)
+    if (EXP == SORTED) y = std::min(y, (2 * pm_device_cus() + N / rows - 1) / (N / rows));
     hipLaunchKernelGGL((dense_small_kernel<T, NT, RM, SRC, EXP>), dim3(N / rows, EXP == DENSE ? (p.T + toks - 1) / toks : y), dim3(512), lds, st, p);
     return 0;
 }

@@ -195,6 +195,21 @@ def test_latent_queries_of_short_heads(heads, dim, kv_rank):
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("E,top,ff,width", [(40, 3, 1100, 2048), (20, 2, 2300, 1000), (9, 9, 8300, 70), (70, 4, 1030, 600)])
+def test_experts_in_turn(E, top, ff, width, dtype):
+    """few tokens, more experts with tokens than a product has workgroups per row tile: one, two, three or more in turn, with and without the sorted tables; experts of one pair and of more than a
+    tile's tokens"""
+    c = one(scan(inner=64, mlp=moe(E, top, 1, 1, ff)), width=width, vocab=120)
+    w = silent(weights_for(c, dtype, 6), 0)
+    _, _, m = model("turn", dtype, c, 6, w, fresh=True, max_tokens=64, n_seq=2, pool_tokens=128)
+    toks = tokens(64, 120, 4)
+    want = P.run(c, w, toks)
+    for n in (5, 11, 40, 64):
+        close(alone(m, toks[:n]), want[:n], dtype)
+    m.close()
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("ff,E,top", [(4700, 3, 2), (1030, 5, 1), (576, 2, 2)])
 def test_wide_experts(ff, E, top, dtype):
     """hidden layers too long for the small-batch kernels' on-chip copies, and of block counts that leave some waves without work"""
