@@ -22,7 +22,7 @@ struct pm_add_norm {
 };
 // attention outputs of one head per group that are still split by keys: part [T x head tiles][splits][16 heads][K] sums, ml [..][splits][16][maximum (log2 units), sum]
 struct pm_split_merge { const float * part, * ml; int splits, H; };
-constexpr size_t PM_SPLIT_FLOATS = (size_t) 256 * 224 * 256;
+constexpr size_t PM_SPLIT_FLOATS = (size_t) 256 * 224 * 256, PM_SPLIT_FLOATS_LEAST = (size_t) 256 * 128 * 128;      // 59 MB: a round of 224 x 256 tiles; 17 MB: of 128 x 128
 struct pm_dense_args {
     int type; const void * W; int K, N;                 // N: rows of W that exist (multiple of 64)
     const void * act; int lda; int T;
@@ -32,7 +32,7 @@ struct pm_dense_args {
     // group != 0 (a multiple of 32; the small-batch kernel, any T): one matrix per group of `group` rows (attention heads): group g multiplies the K activations from column
     // g * g_act on, its first g_store rows go to the columns from g * g_out on
     int group, g_act, g_out, g_store;
-    float * split; size_t split_floats;                 // != null: scratch for products whose few tiles are split over k (PM_SPLIT_FLOATS)
+    float * split; size_t split_floats;                 // != null: scratch for products whose few tiles are split over k (up to PM_SPLIT_FLOATS are used)
     int * parts;                                        // != null: the sums of the k ranges may stay where they are, `*parts` rows of ldy values per token (0: y is written)
     const pm_split_merge * merge;                       // != null (pm_dense_merge_ok, bf16, group = a head): the activations are merged from key splits on the way in
 };

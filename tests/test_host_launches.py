@@ -239,6 +239,45 @@ print("ok")
 """)
 
 
+def test_a_dense_model_without_room_for_all_k_ranges_splits_less(run):
+    """59 MB for the sums of k ranges where the device has them, 17 where it does not: prompts are served all the same"""
+    run(COMMON + r"""
+import os
+sys.path.insert(0, os.path.join(os.environ["PYTHONPATH"], "tests"))
+import numpy as np, torch
+torch.cuda.current_device = lambda: 0
+import prima_cpp_amd.engine as E
+E.stream_ptr = lambda: 1
+from prima_cpp_amd import kudirax
+from test_gpu_kudirax import P, config, layer
+c = config(layer(heads=4, kv=1, dim=64, vdim=64, size=400, mix=False, ff=4096), width=2048, vocab=90)
+w = P.random_model(c, 1)
+MOST, LEAST = 256 * 224 * 256 * 4, 256 * 128 * 128 * 4
+def pool(refused):
+    m = kudirax.load_arrays(c, w, "bfloat16")
+    h = shim.shim_held()
+    shim.shim_refuse(refused)
+    try:
+        m.finalize_pool(max_tokens=900, n_seq=1, pool_tokens=1024)
+    finally:
+        shim.shim_refuse(0)
+    return m, shim.shim_held() - h
+def tiles(m, T):                                        # workgroups of a prompt's products
+    s = m.seq_new()
+    shim.shim_forget()
+    m.batch([(s, np.zeros(T, np.int32), (T - 1,))], logits=torch.zeros(1, 90))
+    m.seq_free(s)
+    return [g[0] for _, name, g in launches() if "dense_tile" in name or "dense_gemm" in name]
+m, full = pool(0)
+a = tiles(m, 900); m.close()
+m, less = pool(MOST)
+assert full - less == MOST - LEAST and shim.shim_last() == 0, (full, less)
+b = tiles(m, 900); m.close()
+assert len(a) == len(b) == 4, (a, b)
+print("ok")
+""")
+
+
 def test_passes_of_a_product_hold_all_tokens(run):
     """1..64 tokens, one matrix: the launched kernels have room for every token (their tiles' tokens are in the names), and only the last pass is not full"""
     run(COMMON + r"""
