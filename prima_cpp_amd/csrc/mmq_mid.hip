@@ -7,7 +7,7 @@
 // LDS copies and products added up instead of overlapping: of 7 us per step of 72B's ffn_gate | ffn_up at 23 tokens 5 were products), and LDS tiles are turned by XOR, free of padding.
 //   * most often more than 64 rows a workgroup (AL): a cell is a row group, all four work on the same pair; its activations come into LDS once for all of them (each wave for itself out of L2: 12 of 67 us
 //     of 57344 x 8192 Q4_K, 20 of 125 of 59136 x 8192 Q6_K)
-//   * up to 64 (32), and some others (mmq_i8_rows): two (four) cells share a row group and take pairs next to each other; a pair's activations are needed by one wave only, which loads them straight into operand registers
+//   * up to 64 (32), and some others (mmq_mid_rows): two (four) cells share a row group and take pairs next to each other; a pair's activations are needed by one wave only, which loads them straight into operand registers
 // Scales come in blocks of up to four pairs, whole lines of them (32 bytes of a line each time, they were a third of the lines that a CU asks for: 14 of 119 us of Q6_K).
 // An integer product's results are read behind the next one's start, one v_mad_i32_i24 each (mad24), for up to 8, 16, 24 or 32 tokens.
 // Bound by the weights' stream (Q4_K 6.2 TB/s between the first tile, 5 us, and the last sums) and, Q6_K, by vector work (400 instructions per 32 rows x 256 k at 24 tokens).
@@ -447,7 +447,7 @@ template <bool EPI> __device__ __forceinline__ void store(const RowsP & p, const
 }
 
 template <int TYPE, int NV, bool EPI, bool AL>
-__device__ __forceinline__ void mmq_i8_body(const RowsP & p, const RowsJob & job, int r0, int r1, int rl, int ji, uint8_t * smem) {
+__device__ __forceinline__ void mmq_mid_body(const RowsP & p, const RowsJob & job, int r0, int r1, int rl, int ji, uint8_t * smem) {
     typedef Fmt<TYPE> F;
     typedef Lds<TYPE, NV, AL> L;
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
@@ -460,8 +460,7 @@ __device__ __forceinline__ void mmq_i8_body(const RowsP & p, const RowsJob & job
         // ---- the cell's weights: two tiles on their way in registers, two in LDS
         Loader<TYPE, NV, AL> ld;
         ld.stride = (uint32_t) pm_rows_stride<TYPE>(nb); ld.base = job.W + (long) r0 * ld.stride; ld.dT = p.dT; ld.smem = smem;
-        const uint32_t la = (uint32_t) (32 * (lane >> 5) + min((lane & 31) + p.t_off, 31)) * 16u;      // (slots behind the 32nd are nobody's)
-        ld.qT = p.qT + la; ld.bsT = p.bsT + la; ld.dt0 = min(p.t_off + 4 * (lane & 7), 28);
+        ld.qT = p.qT + lane * 16; ld.bsT = p.bsT + lane * 16; ld.dt0 = 4 * (lane & 7);
         ld.lane = lane; ld.nb = nb; ld.npair = npair; ld.lim = lim; ld.rl = rl; ld.rgi = rgi; ld.kp = kp; ld.cell = cell; ld.n = n; ld.nround = nround; ld.kl = 2 - rl; ld.HS = HS;
         ld.in = {0, 0}; ld.hin = {0, 0}; ld.pa = {0, 0}; ld.hf = ld.at = ld.pf = 0; ld.pb = 1;
         Tile<TYPE> T0, T1;
@@ -518,8 +517,8 @@ __device__ __forceinline__ void mmq_i8_body(const RowsP & p, const RowsJob & job
         as.n = nb;
         as.rq = __builtin_amdgcn_make_buffer_rsrc((void *) p.qT, 0, nb * (Q80 ? 1024 : 8192), 0x00020000);
         as.rb = __builtin_amdgcn_make_buffer_rsrc((void *) p.bsT, 0, Q80 ? 0 : nb * 1024, 0x00020000);
-        as.qo = on ? (uint32_t) (tq * 1024 + (32 * g + tt + p.t_off) * 16) : 0x80000000u;
-        as.bo = on_b ? (uint32_t) ((lane + p.t_off) * 16) : 0x80000000u;
+        as.qo = on ? (uint32_t) (tq * 1024 + (32 * g + tt) * 16) : 0x80000000u;
+        as.bo = on_b ? (uint32_t) (lane * 16) : 0x80000000u;
 #pragma unroll
         for (int k = 0; k < NA<TYPE, NV>; ++k) load_a<TYPE, NV>(A, as, min(kp, npair - 1), par, k);
     }
@@ -603,7 +602,7 @@ __device__ __forceinline__ void mmq_i8_body(const RowsP & p, const RowsJob & job
 }
 // rows of workgroup w: `each`, and one more for the first `more` of them (in pairs for the rotation: they stay inside a workgroup)
 template <int TYPE, int NV, bool EPI>
-__device__ __forceinline__ void mmq_i8_rows(const RowsP & p, const RowsJob & job, int w, int ji, uint8_t * smem) {
+__device__ __forceinline__ void mmq_mid_rows(const RowsP & p, const RowsJob & job, int w, int ji, uint8_t * smem) {
     constexpr int STEP = EPI ? 2 : 1;
     const int r0 = STEP * (w * job.each + min(w, job.more)), r1 = STEP * ((w + 1) * job.each + min(w + 1, job.more));
     const int most = STEP * (job.each + (job.more != 0));          // of the matrix' workgroups: one order of the sums for all its rows
@@ -611,20 +610,20 @@ __device__ __forceinline__ void mmq_i8_rows(const RowsP & p, const RowsJob & job
     // five or six: rounds of four leave three or two cells without rows every other round; in rounds of two, us of rounds of four / here: Q4_K 33024 x 5120 at 8 tokens 32.6 / 25.3, 36864 x 14336
     // 73 / 54, Q6_K 36864 x 8192 at 24 tokens 86 / 73 (the other lengths and numbers of tokens alike). Three: longer rows of Q4_K over up to 8 tokens, which have little to gain from activations in
     // LDS, one group after the other: 17000 x 14336 34.7 / 31.1, 20480 x 5120 18.7 / 17.2 (512 .. 2048 values 0.84 .. 1.0 of that here, more tokens and Q6_K 0.85 .. 0.95)
-    if (TYPE == PM_Q4_K && NV == 4 && groups == 3 && p.K > 4096) mmq_i8_body<TYPE, NV, EPI, false>(p, job, r0, r1, 0, ji, smem);
-    else if (groups > 2 && groups != 5 && groups != 6) mmq_i8_body<TYPE, NV, EPI, true>(p, job, r0, r1, 2, ji, smem);
-    else mmq_i8_body<TYPE, NV, EPI, false>(p, job, r0, r1, groups > 1 ? 1 : 0, ji, smem);
+    if (TYPE == PM_Q4_K && NV == 4 && groups == 3 && p.K > 4096) mmq_mid_body<TYPE, NV, EPI, false>(p, job, r0, r1, 0, ji, smem);
+    else if (groups > 2 && groups != 5 && groups != 6) mmq_mid_body<TYPE, NV, EPI, true>(p, job, r0, r1, 2, ji, smem);
+    else mmq_mid_body<TYPE, NV, EPI, false>(p, job, r0, r1, groups > 1 ? 1 : 0, ji, smem);
 }
 
-// (named as mmq_i8.hip's: the form with 32-row groups. TA: the type of all jobs but the last, TB: of the last one; first1, first2: first workgroups of the second and third job)
+// (TA: the type of all jobs but the last, TB: of the last one; first1, first2: first workgroups of the second and third job)
 template <int TA, int TB, int NV, bool EPI>
-__global__ __launch_bounds__(NT, 3) void mmq_i8_kernel(int first1, int first2, RowsP p) {
+__global__ __launch_bounds__(NT, 3) void mmq_mid_kernel(int first1, int first2, RowsP p) {
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
     const int b = (int) blockIdx.x, ji = (b >= first1) + (b >= first2);
     const RowsJob job = p.job[ji];
     const int w = b - (ji == 0 ? 0 : ji == 1 ? first1 : first2);
-    if (TA == TB || ji < p.njobs - 1) mmq_i8_rows<TA, NV, EPI>(p, job, w, ji, smem);
-    else mmq_i8_rows<TB, NV, EPI>(p, job, w, ji, smem);
+    if (TA == TB || ji < p.njobs - 1) mmq_mid_rows<TA, NV, EPI>(p, job, w, ji, smem);
+    else mmq_mid_rows<TB, NV, EPI>(p, job, w, ji, smem);
 }
 
 template <int TYPE> size_t lds_of(int nv) {
@@ -637,6 +636,7 @@ size_t lds_of(int type, int nv) { return type == PM_Q4_K ? lds_of<PM_Q4_K>(nv) :
 }  // namespace
 
 int pm_launch_mmq_mid(RowsP p, const int * types, hipStream_t st) {
+    if (p.t_off) return -5;                                            // (a pass starts with its tables)
     const int cus = pm_device_cus(), n = p.njobs;
     const int ta = types[0], tb = types[n - 1];
     double bytes[3], all = 0;
@@ -670,20 +670,20 @@ int pm_launch_mmq_mid(RowsP p, const int * types, hipStream_t st) {
         hipLaunchKernelGGL(kern, dim3(at), dim3(NT), lds, st, first[1], first[2], p);
         return 0;
     };
-#define PM_I8_V(TA_, TB_, E_) { return nv == 4 ? go(mmq_i8_kernel<TA_, TB_, 4, E_>) : nv == 8 ? go(mmq_i8_kernel<TA_, TB_, 8, E_>) : nv == 12 ? go(mmq_i8_kernel<TA_, TB_, 12, E_>) : go(mmq_i8_kernel<TA_, TB_, 16, E_>); }
+#define PM_MID_V(TA_, TB_, E_) { return nv == 4 ? go(mmq_mid_kernel<TA_, TB_, 4, E_>) : nv == 8 ? go(mmq_mid_kernel<TA_, TB_, 8, E_>) : nv == 12 ? go(mmq_mid_kernel<TA_, TB_, 12, E_>) : go(mmq_mid_kernel<TA_, TB_, 16, E_>); }
     if (p.e_on) {
-        if (ta == PM_Q4_K && tb == PM_Q4_K) PM_I8_V(PM_Q4_K, PM_Q4_K, true)
-        if (ta == PM_Q6_K && tb == PM_Q6_K) PM_I8_V(PM_Q6_K, PM_Q6_K, true)
-        if (ta == PM_Q4_K && tb == PM_Q6_K) PM_I8_V(PM_Q4_K, PM_Q6_K, true)
-        if (ta == PM_Q4_K && tb == PM_Q5_K) PM_I8_V(PM_Q4_K, PM_Q5_K, true)
+        if (ta == PM_Q4_K && tb == PM_Q4_K) PM_MID_V(PM_Q4_K, PM_Q4_K, true)
+        if (ta == PM_Q6_K && tb == PM_Q6_K) PM_MID_V(PM_Q6_K, PM_Q6_K, true)
+        if (ta == PM_Q4_K && tb == PM_Q6_K) PM_MID_V(PM_Q4_K, PM_Q6_K, true)
+        if (ta == PM_Q4_K && tb == PM_Q5_K) PM_MID_V(PM_Q4_K, PM_Q5_K, true)
         return -5;
     }
-    if (ta == PM_Q4_K && tb == PM_Q4_K) PM_I8_V(PM_Q4_K, PM_Q4_K, false)
-    if (ta == PM_Q6_K && tb == PM_Q6_K) PM_I8_V(PM_Q6_K, PM_Q6_K, false)
-    if (ta == PM_Q5_K && tb == PM_Q5_K) PM_I8_V(PM_Q5_K, PM_Q5_K, false)
-    if (ta == PM_Q8_0 && tb == PM_Q8_0) PM_I8_V(PM_Q8_0, PM_Q8_0, false)
-    if (ta == PM_Q4_K && tb == PM_Q6_K) PM_I8_V(PM_Q4_K, PM_Q6_K, false)
-    if (ta == PM_Q4_K && tb == PM_Q5_K) PM_I8_V(PM_Q4_K, PM_Q5_K, false)
-#undef PM_I8_V
+    if (ta == PM_Q4_K && tb == PM_Q4_K) PM_MID_V(PM_Q4_K, PM_Q4_K, false)
+    if (ta == PM_Q6_K && tb == PM_Q6_K) PM_MID_V(PM_Q6_K, PM_Q6_K, false)
+    if (ta == PM_Q5_K && tb == PM_Q5_K) PM_MID_V(PM_Q5_K, PM_Q5_K, false)
+    if (ta == PM_Q8_0 && tb == PM_Q8_0) PM_MID_V(PM_Q8_0, PM_Q8_0, false)
+    if (ta == PM_Q4_K && tb == PM_Q6_K) PM_MID_V(PM_Q4_K, PM_Q6_K, false)
+    if (ta == PM_Q4_K && tb == PM_Q5_K) PM_MID_V(PM_Q4_K, PM_Q5_K, false)
+#undef PM_MID_V
     return -5;
 }

@@ -16,8 +16,8 @@ template <int TYPE> __device__ __forceinline__ size_t pm_rows_stride(int nb) {
 }
 // one or several matrices of one K (types[0]; only the last may be of another type) over 1..8 tokens, one matrix over more; -5: not served
 enum { PM_ROWS_ONE, PM_ROWS_SEVERAL, PM_ROWS_MIXED };               // one matrix; several of one type; two types
-// whether a pass over T tokens of N rows in all is one for it (else mmq_i8.hip's kernels); type: of the first matrix
+// whether a pass over T tokens of N rows in all is one for it (else mmq_mid.hip's kernel, or mmq_i8.hip's); type: of the first matrix
 bool pm_mmq_rows_takes(int type, long N, int K, int T, int form = PM_ROWS_ONE);
 int pm_launch_mmq_rows(RowsP p, const int * types, hipStream_t st);
-// mmq_mid.hip: one or several matrices of one K (types[0]; only the last may be of another type) over 1..32 tokens; -5: not served
+// mmq_mid.hip: one or several matrices of one K (types[0]; only the last may be of another type) over 1..32 tokens, t_off 0; -5: not served
 int pm_launch_mmq_mid(RowsP p, const int * types, hipStream_t st);

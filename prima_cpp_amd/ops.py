@@ -273,7 +273,7 @@ def mul_mat_vec_fused_ss(ws, x, norm_w=None, eps=0.0, resids=None, want_sumsq=Fa
 
 
 def mul_mat_small(w, x=None, xq=None, n_tokens=None, bias=None, resid=None):
-    """1..32 tokens on the integer matrix cores (mmq_i8.hip): x f32 [T, K] (quantized to Q8_K on device) or pre-quantized xq -> f32 [T, N]."""
+    """1..64 tokens on the integer matrix cores (mmq_i8.hip): x f32 [T, K] (quantized to Q8_K on device) or pre-quantized xq -> f32 [T, N]."""
     import ctypes as C
     lib = L.load()
     lib.pm355_mul_mat_q_small.restype = C.c_int
@@ -288,7 +288,7 @@ def mul_mat_small(w, x=None, xq=None, n_tokens=None, bias=None, resid=None):
 
 
 def mul_mat_small_multi(ws, xq, n_tokens, biases=None):
-    """2 or 3 matrices of one type and K sharing the pre-quantized activations, one launch (mmq_i8.hip multi-job kernels) -> list of f32 [T, N_j]."""
+    """2 or 3 matrices of one type and K sharing the pre-quantized activations, one launch (mmq_mid.hip, mmq_rows.hip) -> list of f32 [T, N_j]."""
     import ctypes as C
     lib = L.load()
     n = len(ws)
@@ -302,7 +302,7 @@ def mul_mat_small_multi(ws, xq, n_tokens, biases=None):
 
 
 def mul_mat_small_mixed(ws, xq, n_tokens, biases=None):
-    """wq | wk of one type and wv of another sharing the pre-quantized activations, one grid (mmq_i8.hip mmq_i8_dual_kernel) -> list of f32 [T, N_j]."""
+    """wq | wk of one type and wv of another sharing the pre-quantized activations, one grid (mmq_mid.hip, mmq_rows.hip) -> list of f32 [T, N_j]."""
     import ctypes as C
     lib = L.load()
     n = len(ws)

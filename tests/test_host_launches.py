@@ -164,15 +164,15 @@ print("ok")
 
 
 def test_which_products_of_few_tokens_take_16_row_operands(run):
-    """mmq_rows.hip where it is the faster form - one group of 16 rows per CU, or steps and passes that are full -, mmq_i8.hip elsewhere, for one matrix, several, and two types."""
+    """mmq_rows.hip where it is the faster form - one group of 16 rows per CU, or steps and passes that are full -, mmq_mid.hip elsewhere, for one matrix, several, and two types; one matrix of Q5_K
+    or Q8_0 over up to 16 tokens: mmq_i8.hip."""
     run(COMMON + r"""
 lib = C.CDLL(sys.argv[2])
 lib.pm355_mul_mat_q_small.argtypes = [C.c_int, C.c_void_p, C.c_int64, C.c_int64, C.c_void_p, C.c_void_p, C.c_int64, C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p]
 at = C.addressof(C.create_string_buffer(256))
 Q4, Q5, Q6, Q8 = 12, 13, 14, 8
 def forms():
-    out = [re.search(r"(mmq_rows|mmq_i8(?:_dual)?)_kernel<(.*?)>", n).groups() for _, n, _ in launches() if re.search("mmq_(rows|i8)(_dual)?_kernel", n)]
-    return [("rows" if a == "mmq_rows" else "i8", b) for a, b in out]
+    return [m.groups() for _, n, _ in launches() for m in [re.search(r"mmq_(rows|mid|i8)_kernel<(.*?)>", n)] if m]
 def one(t, N, K, T):
     shim.shim_forget()
     rc = lib.pm355_mul_mat_q_small(t, at, K, N, at, None, T, at, None, None, 1)
@@ -193,27 +193,28 @@ def several(types, Ns, K, T):
         rc = f(arr(types, C.c_int), n, W, N64, y, None, at, K, T, 1)
     assert rc == 0, (types, Ns, K, T, rc)
     return [f for f, _ in forms()]
-R, I = ["rows"], ["i8"]
+R, M, S = ["rows"], ["mid"], ["i8"]
 for T in (1, 2, 5, 8):
     for t in (Q4, Q5, Q6, Q8):
         for K in (1024, 2048, 4096, 14336):
             assert one(t, 4096, K, T) == R and one(t, 17, K, T) == R, (t, K, T)
         for K in (512, 1024, 1536, 2048):
             for N in (8192, 16384, 32000):
-                assert one(t, N, K, T) == I, (t, N, K, T)
+                assert one(t, N, K, T) == (M if t in (Q4, Q6) else S), (t, N, K, T)
     for t in (Q4, Q6):
         assert one(t, 128256, 4096, T) == one(t, 36864, 8192, T) == one(t, 10240, 4096, T) == one(t, 8001, 3072, T) == R
-        assert one(t, 27648, 5120, T) == one(t, 5120, 5120, T) == one(t, 14336, 14336, T) == one(t, 16384, 3072, T) == I
+        assert one(t, 27648, 5120, T) == one(t, 5120, 5120, T) == one(t, 14336, 14336, T) == one(t, 16384, 3072, T) == M
         assert several([t] * 2, [14336] * 2, 4096, T) == several([t] * 3, [4096, 1024, 1024], 4096, T) == several([t] * 3, [3072, 1024, 1024], 3072, T) == R
-        assert several([t] * 2, [8192] * 2, 2048, T) == several([t] * 3, [5120] * 3, 5120, T) == I
+        assert several([t] * 2, [8192] * 2, 2048, T) == several([t] * 3, [5120] * 3, 5120, T) == M
     for tb in (Q5, Q6):
         assert several([Q4, Q4, tb], [4096, 1024, 1024], 4096, T) == several([Q4, Q4, tb], [8192, 1024, 1024], 8192, T) == several([Q4, Q4, tb], [2048, 512, 512], 2048, T) == R
-        assert several([Q4, Q4, tb], [5120] * 3, 5120, T) == several([Q4, Q4, tb], [8192, 1024, 1024], 2048, T) == I
-    assert one(Q5, 5000, 4096, T) == R and one(Q5, 128256, 4096, T) == one(Q5, 8192, 8192, T) == I
-    assert one(Q8, 10240, 8192, T) == one(Q8, 49152, 2048, T) == R and one(Q8, 8192, 8192, T) == one(Q8, 4096, 512, T) == I
-for t, T, K, N, want in ((Q4, 12, 2048, 4096, I), (Q4, 12, 3072, 4096, R), (Q4, 24, 8192, 4096, R), (Q4, 25, 8192, 4096, I), (Q4, 12, 8192, 4097, I), (Q6, 20, 2048, 4096, R), (Q6, 20, 1024, 4096, I),
-                         (Q5, 9, 512, 4096, R), (Q5, 32, 8192, 4096, R), (Q5, 33, 8192, 4096, R + R), (Q5, 20, 2048, 32000, I + I), (Q5, 20, 4096, 32000, R), (Q5, 16, 4096, 32000, I), (Q5, 25, 4096, 32000, I + I),
-                         (Q8, 12, 4096, 4096, I), (Q8, 12, 8192, 4096, R), (Q8, 17, 512, 4096, R), (Q8, 20, 512, 16384, I + I), (Q8, 20, 1024, 16384, R), (Q8, 32, 4096, 8192, I + I), (Q4, 40, 8192, 4096, I + R)):
+        assert several([Q4, Q4, tb], [5120] * 3, 5120, T) == several([Q4, Q4, tb], [8192, 1024, 1024], 2048, T) == M
+    assert one(Q5, 5000, 4096, T) == R and one(Q5, 128256, 4096, T) == one(Q5, 8192, 8192, T) == S
+    assert one(Q8, 10240, 8192, T) == one(Q8, 49152, 2048, T) == R and one(Q8, 8192, 8192, T) == one(Q8, 4096, 512, T) == S
+for t, T, K, N, want in ((Q4, 12, 2048, 4096, M), (Q4, 12, 3072, 4096, R), (Q4, 24, 8192, 4096, R), (Q4, 25, 8192, 4096, M), (Q4, 12, 8192, 4097, M), (Q6, 20, 2048, 4096, R), (Q6, 20, 1024, 4096, M),
+                         (Q5, 9, 512, 4096, R), (Q5, 32, 8192, 4096, R), (Q5, 33, 8192, 4096, R + R), (Q5, 20, 2048, 32000, S + S), (Q5, 20, 4096, 32000, R), (Q5, 16, 4096, 32000, S), (Q5, 25, 4096, 32000, S + S),
+                         (Q8, 12, 4096, 4096, S), (Q8, 12, 8192, 4096, R), (Q8, 17, 512, 4096, R), (Q8, 20, 512, 16384, S + S), (Q8, 20, 1024, 16384, R), (Q8, 32, 4096, 8192, S + S), (Q4, 40, 8192, 4096, M + R),
+                         (Q5, 17, 4352, 8192, M), (Q5, 40, 8192, 32000, M + S), (Q8, 20, 2048, 8192, M), (Q8, 25, 1024, 16384, M), (Q8, 52, 896, 12288, M + S + S), (Q8, 60, 896, 12288, M + M)):
     assert one(t, N, K, T) == want, (t, T, K, N, one(t, N, K, T))
 print("ok")
 """)
@@ -289,7 +290,7 @@ def room(name):
     m = re.search(r"mmq_(rows|mid|i8)_kernel<(.*?)>", name)
     if not m: return 0
     a = m.group(2).split(", ")
-    return 8 * int(a[2]) if m.group(1) == "rows" else 2 * int(a[2] if len(a) == 4 else a[1])     # groups of 8 tokens; result registers of 2
+    return 8 * int(a[2]) if m.group(1) == "rows" else 2 * int(a[2] if m.group(1) == "mid" else a[1])     # groups of 8 tokens; result registers of 2
 short = []
 for t in (12, 13, 14, 8):
     for N in (17, 4096, 4097, 8192, 8193, 12288, 16384, 32000, 57344, 151936):

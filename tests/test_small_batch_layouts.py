@@ -135,11 +135,12 @@ def test_row_major_v_image_feeds_the_transposing_read(dh):
                     assert got == [(8 * lg + 4 * half + r, 16 * d + col) for r in range(4)], (lg, d, half, col, got)
 
 
-# ---- round 6: the wq | wk | wv epilogue of the small-batch launch (mmq_i8.hip EPI instantiations) and the two-part grid (mmq_i8_dual_kernel)
+# ---- the wq | wk | wv epilogue of the small-batch launches (EPI instantiations) and the division of their workgroups (mmq_mid.hip, mmq_rows.hip)
 
 def epi_slices(N, G):
-    """mmq_i8_body<.., EPI = true>: workgroup w of G owns virtual rows [r0, r1), both forced even."""
-    return [(((N * w) // G) & ~1, ((N * (w + 1)) // G) & ~1) for w in range(G)]
+    """mmq_mid_rows<.., EPI = true>: workgroup w of G owns rows [r0, r1): `each` pairs of rows, and one more for the first `more` of them."""
+    each, more = N // 2 // G, N // 2 % G
+    return [(2 * (w * each + min(w, more)), 2 * ((w + 1) * each + min(w + 1, more))) for w in range(G)]
 
 
 @pytest.mark.parametrize("N,G", [(9216, 224), (9216, 220), (10240, 256), (10240, 255), (1280, 40), (8192 + 1024, 37), (2304, 9)])
@@ -175,22 +176,30 @@ def test_epilogue_thread_finds_its_pair_in_the_neighbouring_lane():
     assert len(seen) == 32 * 32
 
 
-def dual_split(total_a, stride_a, Nb, stride_b, cus=256):
-    """pm_launch_mmq_i8_dual: the device's workgroups divided by weight bytes; neither part gets more workgroups than it has 32-row groups."""
-    ba, bb = total_a * stride_a, Nb * stride_b
-    gb = int(cus * bb / (ba + bb) + 0.5)
-    gb = max(gb, 1)
-    gb = min(gb, (Nb + 31) // 32)
-    ga = min(cus - gb, (total_a + 31) // 32)
-    return ga, gb
+def divide(N, stride, unit, cus=256):
+    """pm_launch_mmq_mid: the device's workgroups divided by weight bytes, at least 32 rows each; slices of the last job that are a little longer than whole groups of 32 rows get some of the first's"""
+    n, total, at, nw = len(N), sum(a * s for a, s in zip(N, stride)), 0, []
+    for j in range(n):
+        want = cus - at if j == n - 1 and n > 1 else int(cus * N[j] * stride[j] / total + 0.5)
+        nw.append(max(1, min(want, cus - at - (n - 1 - j), (N[j] + 31) // 32)))
+        at += nw[-1]
+    groups = lambda j, w: (unit * -(-(N[j] // unit) // w) + 31) // 32
+    g = groups(n - 1, nw[-1]) if n > 1 else 1
+    if g > 1:
+        up = -(-N[-1] // (32 * (g - 1)))
+        more = up - nw[-1]
+        if 16 * more <= nw[-1] and more < nw[0] and groups(0, nw[0] - more) == groups(0, nw[0]) and groups(n - 1, up) < g:
+            nw[0] -= more
+            nw[-1] = up
+    return nw
 
 
-@pytest.mark.parametrize("Na,Nb,K", [(9216, 1024, 8192), (4096 + 1024, 1024, 4096), (5120 + 1024, 1024, 5120), (300 + 70, 75, 1024), (2100 + 260, 300, 2048)])
-def test_two_part_grid_gives_every_part_workgroups_and_whole_row_groups(Na, Nb, K):
-    for stride_b in (K // 256 * 210, K // 256 * 176):                  # Q6_K / Q5_K rows against Q4_K's 144 bytes per super-block
-        ga, gb = dual_split(Na, K // 256 * 144, Nb, stride_b)
-        assert ga >= 1 and gb >= 1 and ga + gb <= 256
-        assert gb <= (Nb + 31) // 32 and ga <= (Na + 31) // 32
-        # the 70B shape: wq | wk take the bulk, wv (1024 rows) about one workgroup per 32 rows (Q6_K: 35.7 by bytes, capped at 32; Q5_K: 31)
-        if (Na, Nb, K) == (9216, 1024, 8192):
-            assert (ga, gb) == ((224, 32) if stride_b == K // 256 * 210 else (225, 31))
+@pytest.mark.parametrize("unit", [1, 2])
+@pytest.mark.parametrize("N,K", [((8192, 1024, 1024), 8192), ((4096, 1024, 1024), 4096), ((5120, 1024, 1024), 5120), ((300, 70, 76), 1024), ((2100, 260, 300), 2048), ((8192, 1024, 1024), 512), ((40, 2, 2), 512)])
+def test_every_matrix_of_a_launch_gets_workgroups_and_no_more_than_it_has_row_groups(N, K, unit):
+    for last in (210, 176, 144):                                       # Q6_K / Q5_K / Q4_K rows beside Q4_K's 144 bytes per super-block
+        nw = divide(N, [K // 256 * b for b in (144, 144, last)], unit)
+        assert min(nw) >= 1 and sum(nw) <= 256
+        assert all(w <= (a + 31) // 32 for w, a in zip(nw, N))
+        if N == (8192, 1024, 1024):                                    # wv of Q5_K: 31 workgroups by its bytes, with slices of 33 and 34 rows
+            assert nw == {210: [196, 24, 32], 176: [199, 25, 32], 144: [205, 26, 25]}[last], (last, nw)

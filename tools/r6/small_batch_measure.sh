@@ -1,7 +1,7 @@
 #!/bin/bash
 # Round 6, small batches: step times of T-token batches through a 16-layer 70B- (and Qwen2.5-72B-) shaped window on the default routing, the prompt-GEMM crossover,
 # and per-kernel tables of 8- / 32- / 64-token steps. A/B partners are separate builds selected with PM355_LIB (python -m prima_cpp_amd.build <tag> -D<FLAG>,
-# -> ab/<tag>.so) or the A/B switches of INTEGRATION.md (PM355_MMQ_DUAL, PM355_MMQ_RGB8_MIN, PM355_SMALL_ATTN_MFMA_MIN, PM355_MMQ_MAX_TOKENS, PM355_GEMM_PF_NT);
+# -> ab/<tag>.so) or the A/B switches of INTEGRATION.md (PM355_MMQ_DUAL, PM355_SMALL_ATTN_MFMA_MIN, PM355_MMQ_MAX_TOKENS, PM355_GEMM_PF_NT);
 # the numbers of the round are in profiles/r06_small_batch.txt.   usage (GPU box): bash tools/r6/small_batch_measure.sh [ab/<tag>.so]
 cd "$(dirname "$0")/../.."
 mkdir -p gpurun_out/r6sb
