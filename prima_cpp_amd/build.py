@@ -26,7 +26,9 @@ SOURCES = DENSE_SOURCES + ["c_api.hip", "quantize.hip", "mmvq.hip", "mmvq_cols.h
 # round 5's measured-slower forms of the decode layer (sum-of-squares partials, attention tail, persistent engine): a library of their own, loaded by their tests
 EXP_LIB = os.path.join(HERE, "libprima_mi355_exp.so")
 EXP_SOURCES = SOURCES + ["decode_engine.hip"]
-PROBE_SOURCES = ["probe.hip", "engine_probe.hip", "probe_api.hip", "overlap_probe.hip"]
+PROBE_SOURCES = ["probe.hip", "engine_probe.hip", "probe_api.hip", "overlap_probe.hip", "attn_blocks.hip"]
+# (and the product objects that attn_blocks.hip launches)
+PROBE_WITH = ["attn_cached.hip", "attn_prefill.hip", "quantize.hip", "c_api_base.hip"]
 # -ffp-contract=off: the quantizers must round exactly like the reference (no fused multiply-add where
 # the reference has a separate multiply and add); FMAs we want are written as fmaf().
 EXTRA = os.environ.get("PM355_EXTRA_FLAGS", "").split()
@@ -66,7 +68,7 @@ def _newer(target, deps):
     return any(os.path.getmtime(d) > t for d in deps)
 
 
-def _compile(srcs, hdrs, objdir, lib, flags, force, verbose):
+def _compile(srcs, hdrs, objdir, lib, flags, force, verbose, objs_with=()):
     hipcc = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
     os.makedirs(objdir, exist_ok=True)
     objs, procs = [], []
@@ -88,6 +90,7 @@ def _compile(srcs, hdrs, objdir, lib, flags, force, verbose):
     for c, pr in procs:
         if pr.wait():
             raise subprocess.CalledProcessError(pr.returncode, c)
+    objs += list(objs_with)
     if force or _newer(lib, objs):
         cmd = [hipcc, "--offload-arch=gfx950", "-shared", "-fPIC", "-o", lib] + objs + ["-ldl", "-lpthread"]
         if verbose:
@@ -125,7 +128,8 @@ def build_probe(force=False, verbose=False):
     d = os.path.join(ROOT, "tools", "csrc")
     srcs = [os.path.join(d, s) for s in PROBE_SOURCES]
     hdrs = _headers() + [os.path.join(d, "pm355_probe.h")]
-    return _compile(srcs, hdrs, os.path.join(d, "obj"), PROBE_LIB, FLAGS + ["-I" + CSRC], force, verbose)
+    _compile([os.path.join(CSRC, s) for s in SOURCES], _headers(), CSRC, LIB, EXTRA + FLAGS, False, verbose)
+    return _compile(srcs, hdrs, os.path.join(d, "obj"), PROBE_LIB, FLAGS + ["-I" + CSRC], force, verbose, [os.path.join(CSRC, s[:-4] + ".o") for s in PROBE_WITH])
 
 
 if __name__ == "__main__":

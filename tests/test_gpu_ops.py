@@ -1184,6 +1184,36 @@ def test_long_context_attention_at_the_70b_head_shape(P, n_kv):
     assert e64 < 2e-3 and e16 < 2e-3 + r1664
 
 
+@pytest.mark.parametrize("H, Hkv, cells", [
+    (2, 1, [1]), (8, 4, [1, 63, 64, 2, 33]), (8, 8, [64, 65, 128, 127, 1]), (16, 2, [129, 256, 255, 8, 64, 200]), (32, 8, list(range(9, 41))),                  # rows: each its own sequence
+    (2, 1, (0, 1)), (4, 2, (0, 32)), (8, 2, (63, 3)), (32, 8, (100, 17)), (16, 2, (480, 32)),                                                             # (first position, consecutive tokens)
+])
+def test_attention_leaves_the_blocks_its_quantizer_would(P, H, Hkv, cells):
+    """A small batch's attention that writes wo's 8-bit activations itself, against the attention stored as f32 rows and quantized by a launch of its own: every byte of the rows and of the tables."""
+    torch = P.torch
+    f = P.L.load_probe().pm355_probe_attn_blocks
+    f.restype, f.argtypes = C.c_int, [C.c_void_p] * 5 + [C.c_int64] + [C.c_int] * 3 + [C.c_float] + [C.c_int] * 3 + [C.c_void_p] * 8
+    rows = isinstance(cells, list)
+    T, dh, n_ctx = (len(cells) if rows else cells[1]), 128, (256 if rows else 512)
+    K, n_seq = H * dh, (T if rows else 1)
+    rng = np.random.default_rng(1000 * H + T)
+    half = lambda a: torch.from_numpy(a.astype(np.float16).view(np.int16)).cuda()
+    kc, vc = (half(rng.normal(0, 1, n_seq * n_ctx * Hkv * dh)) for _ in range(2))
+    q = torch.from_numpy((rng.normal(0, 1.5, (T, K))).astype(np.float16).astype(np.float32)).cuda()
+    pos = torch.tensor([c - 1 for c in cells] if rows else [cells[0] + t for t in range(T)], dtype=torch.int32, device="cuda")
+    seq = torch.tensor(list(range(T))[::-1] if rows else [0] * T, dtype=torch.int32, device="cuda")
+    row = K + K // 256 * 4 + K // 16 * 2
+    out = [[torch.full((n,), 0x5a, dtype=torch.uint8, device="cuda") for n in (T * row + 64, K // 256 * 1152, K // 256 * 8192)] for _ in range(2)]
+    y32 = torch.zeros((T, K), dtype=torch.float32, device="cuda")
+    torch.cuda.synchronize()
+    args = [q, kc, vc, pos, seq, n_ctx * Hkv * dh, H, Hkv, n_ctx, 1.0 / np.sqrt(dh), int(rows), max(cells) if rows else 0, T, *out[0], y32, *out[1]]
+    rc = f(*[a.data_ptr() if isinstance(a, torch.Tensor) else a for a in args], None)
+    torch.cuda.synchronize()
+    assert rc == 0 and bool(torch.isfinite(y32).all()) and bool((y32 != 0).any(dim=1).all())
+    for name, a, b in zip(("rows", "sums", "values"), *out):
+        assert bool((b != 0x5a).any()) and bool((a == b).all()), f"{name}: {int((a != b).sum())} of {a.numel()} bytes differ"
+
+
 def test_long_context_attention_merge_survives_a_starved_chip(P):
     """The in-launch merge of attn_flash_mfma.hip lets the last arrivals of a KV head spin (bounded) for workgroups still behind them. Provoked here:
     a co-running stream-read kernel holds every CU's wave slots while the 8 x 32 attention grid is launched on another stream, so its workgroups
