@@ -453,8 +453,8 @@ void launch_prep(const Scr * sc, const void * xq, int K, int T, hipStream_t st) 
 
 namespace {
 // Q5_K and Q8_0: whether 17..32 tokens go in one pass (else two of up to 16, or mmq_rows.hip). Us, as it was / one pass: Q8_0 20 tokens 8192 x 2048 10.6 / 8.3, 14336 x 4096 24.6 / 17.2,
-// 8192 x 8192 24.9 / 18.3, 8192 x 29568 75 / 55; 28 tokens 16384 x 1024 16.7 / 9.1, 14336 x 4096 33.1 / 18.3, 8192 x 8192 34.3 / 19.2; Q5_K 8192 x 8192 20 tokens 21.0 / 16.8, 28 31.7 / 17.8. On the
-// other side of the lines one pass would be the faster one too (8192 x 4096 at 32 tokens 20.6 / 12.0, Q5_K 14336 x 4096 20.3 / 16.0): there the forms are those that test_host_launches.py has
+// 8192 x 8192 24.9 / 18.3, 8192 x 29568 75 / 55; 28 tokens 16384 x 1024 16.7 / 9.1, 14336 x 4096 33.1 / 18.3, 8192 x 8192 34.3 / 19.2; Q5_K 8192 x 8192 20 tokens 21.0 / 16.8, 28 31.7 / 17.8. The
+// lines are not where the two forms take the same time: on their other side one pass would be the faster one too (8192 x 4096 at 32 tokens 20.6 / 12.0, Q5_K 14336 x 4096 20.3 / 16.0), and is not taken
 bool one_pass(int type, long N, int K, int T) {
     const int cus = pm_device_cus();
     const long groups = ((N + cus - 1) / cus + 15) / 16;

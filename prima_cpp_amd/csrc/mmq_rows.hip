@@ -589,7 +589,7 @@ size_t lds_of(int type, int NG, int R, bool AL, int K) {
 // Where this form is the faster one, by rows per CU (groups of 16) and K. Its workgroup takes all of K at once, eight pairs of super-blocks a step: with one row group the chip is full where
 // 32-row groups fill half of it, with more it pays for the steps' empty pairs (K = 2048: four of eight), for a round of sums over the waves per pass, and for a last pass of few rows (passes of 48
 // rows, of 64 where the activations fit LDS). Weights out of memory, time here / time of mmq_i8.hip's kernel
-// (for Q4_K and Q6_K that was the form before mmq_mid.hip's, which takes 0.94 and 0.98 of its time in the mean):
+// (for Q4_K and Q6_K that was the form before mmq_mid.hip's, which takes 0.91 and 0.89 of its time in the mean up to 8 tokens: divide by these to compare with what a shape not taken here gets now):
 //   8 tokens, one matrix, N = 4096 / 8192 / 12288 / 16384 / 36864 / 128256: Q4_K K = 1024 0.96 1.15 1.23 1.37 1.37 1.51, 2048 0.91 1.07 1.16 1.25 1.14 1.22, 3072 0.84 0.99 1.00 1.11 0.97 0.92,
 //   4096 0.82 0.94 0.94 1.03 0.89 0.87, 5120 0.87 1.13 1.09 1.21 1.07 1.05, 8192 0.86 1.02 0.93 0.98 0.88, 14336 0.92 1.12 0.99 1.24 0.95; Q6_K 1024 0.96 1.24 1.40 1.65 1.60 1.65, 4096 0.74 0.95
 //   0.94 1.07 0.86 0.82, 5120 0.86 1.20 1.13 1.30 1.07, 8192 0.76 1.04 0.90 0.98 0.80, 14336 0.76 1.08 0.93 1.09 0.82; Q5_K 2048 0.89 1.07 1.19 1.36 1.29 1.32, 4096 0.75 1.01 1.03 1.07 1.00,

@@ -1,5 +1,7 @@
-// moe.hip — routing of a step's tokens to experts. Up to 64 tokens of up to 64 experts: one launch with the norm and the router product, a workgroup per token. Up to 64 tokens: one workgroup scores, selects and sorts (expert by expert, tokens in order). More: a wave per token
-// selects and takes a place in its expert's list, then every workgroup sorts its share of the pairs (the order inside an expert does not enter any sum).
+// moe.hip — routing of a step's tokens to experts, in one of three forms:
+// - few pairs of up to 64 experts behind a bf16 model's RMS norm (pm_route_stream_ok): norm, router product and choice in one launch, a workgroup per token; the expert products find their own pairs
+// - up to 64 tokens otherwise: one workgroup scores, selects and sorts (expert by expert, tokens in order)
+// - more: a wave per token selects and takes a place in its expert's list, then every workgroup sorts its share of the pairs (the order inside an expert does not enter any sum)
 #include "pm355_route.h"
 #include "pm355_kernels.h"
 
