@@ -27,6 +27,7 @@
 #include <stdlib.h>
 #include <stdio.h>
 #include <mutex>
+#include <type_traits>
 
 namespace {
 
@@ -36,7 +37,7 @@ typedef _Float16 half2v __attribute__((ext_vector_type(2)));
 typedef float float16v __attribute__((ext_vector_type(16)));
 typedef __attribute__((address_space(3))) void * lds_ptr;
 
-constexpr int PF_NTHR = 512, PF_MAX_JOBS = 4;
+constexpr int PF_NTHR = 512, MID_NTHR = 768, PF_MAX_JOBS = 4;
 
 struct PfJob {
     const uint8_t * W; float * Y; _Float16 * Yh; const float * bias; const float * resid; const float * silu_gate;
@@ -461,15 +462,19 @@ __device__ __forceinline__ void pf_body(const PfP & p, const PfJob & jb, const i
     }
 }
 
-// ---- one round of workgroups (NT = 2 / 4): 128 rows x 32 NT tokens per workgroup, wave (g, kk) = rows [32 g, + 32) x the kk-th 64 k of every 128-k step ----
+// ---- one round of workgroups (NT = 2 / 3 / 4): 128 rows x 32 NT tokens per workgroup, wave (g, kk) = rows [32 g, + 32) x the kk-th 64 k of every 128-k step ----
 // Few tokens leave little to multiply between two barriers. The loop above - 256 rows, two barriers per 16-k slice - spent 860 cycles on a slice of 128 tokens (128 of them in
 // MFMAs), half of them in barriers with nothing else left in it, and a launch had 16-64 tiles whose last K slice then read all slabs and stored 16-byte pieces of 32 token rows
 // by itself (14 of the 34 us of a 4096 x 4096 launch). Here: one barrier per 128 k; both halves of a step are multiplied side by side and added up through LDS at the end (half the
 // slabs of a K split for the same number of workgroups); three activation buffers, weights requested 2 to 4 steps ahead; tiles of 128 rows, so that twice as many
 // workgroups share the reduction; results cross LDS once more and are stored as whole 128-byte pieces of a token row.
-// What bounds it: the DMA of 41 KB of operands per 128 x 128 x 128 products (0.73 of a step's 1.2 us by itself) next to a step's 0.87 us of LDS reads, dequantization and MFMAs.
-// Llama-3-8B's launches at 101 tokens, Q4_K, us before / now: wq | wk | wv 37 / 24, wo 34 / 23, ffn_gate | ffn_up 61 / 50, ffn_down 54 / 36.6. Taken back: 64 rows and a quarter of the
-// k per wave (half the LDS reads: no change, 1-2 us more for the longer merge); two activation buffers instead of three (2-10 % slower).
+// Operands are requested by four waves that do nothing else (mid_load); where a kernel's registers leave no room for them, by the ones that multiply, a quarter of a step's behind each slice's
+// products. 8B shape, Q4_K at 101 tokens, us, requests by the waves that multiply / by their own: ffn_gate | ffn_up 51.9 / 45.6, ffn_down 28.7 / 26.5, wo 18.0 / 17.0, wq | wk | wv 20.0 / 18.7.
+// What bounds it, four layers of that (646 us, 411 without any step): the requests alone 168 of the 235 us of steps - weights 91, whose 32-byte pieces of a line are asked for line by line four
+// times over, activations 41 -, LDS reads, dequantization and MFMAs alone 136. Tiles of 96 tokens cost 0.8 of those of 128: 90 tokens, two layers 287 / 252 us.
+// Llama-3-8B's launches at 101 tokens, Q4_K, us in the general tiles / as these were first: wq | wk | wv 37 / 24, wo 34 / 23, ffn_gate | ffn_up 61 / 50, ffn_down 54 / 36.6. Taken back: 64 rows and
+// a quarter of the k per wave (half the LDS reads: no change, 1-2 us more for the longer merge); two activation buffers instead of three (2-10 % slower); a step's first fragments read in the
+// step before, whose activations then have one step to arrive instead of two (646 -> 680).
 template <int TYPE> constexpr int mid_slot() { return TYPE == PM_Q8_0 ? 4096 : PfT<TYPE>::NSTREAM * 1024; }           // 128 k of 32 rows
 // weights are requested this many steps ahead (what LDS has room for)
 template <int TYPE, bool EX> constexpr int mid_ahead() { return TYPE == PM_Q8_0 || (EX && TYPE == PM_Q5_K) ? 2 : TYPE == PM_Q6_K ? 3 : 4; }
@@ -477,7 +482,129 @@ template <int TYPE, bool EX> constexpr int mid_group_bytes() { return (mid_ahead
 // EX, per super-block: 16 group sums (not for Q6_K: no minima) and a scale of every token, two buffers
 template <int TYPE, int NT> constexpr int mid_sum_bytes() { return TYPE == PM_Q6_K ? 0 : NT * 32 * 32; }
 template <int TYPE, int NT, bool EX> constexpr size_t mid_lds_bytes() { return (size_t) 6 * NT * 32 * 128 + (size_t) 4 * mid_group_bytes<TYPE, EX>() + (EX ? 2 * (mid_sum_bytes<TYPE, NT>() + NT * 32 * 4) : 0); }
+// no waves of their own for the requests: where the kernel's registers leave no room for them (168 a wave). 8B shape, 147 tokens of 8-bit activations, wq | wk | wv with a Q6_K wv: 53 us, with loaders
+// and 12 registers spilled 68
+template <int TA, int TB, int NT, bool EX> constexpr bool mid_self() { return EX && (NT == 4 || TA != TB || TA == PM_Q5_K); }
 template <int N> __device__ __forceinline__ void mid_wait() { asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" : : "n"(N) : "memory"); }
+
+// A tile's requests. Those of weights and of activations are different waves': requests return in order, and weights come from memory (AHEAD steps ahead), activations mostly from L2 (two steps)
+// ... the weights of NG row groups of one wave
+template <int TYPE, int NT, bool EX, int NG> struct MidWeights {
+    static constexpr int SLOT = mid_slot<TYPE>(), W = SLOT / 1024, AHEAD = mid_ahead<TYPE, EX>(), HDR = (AHEAD + 1) * SLOT, XTRA = HDR + 2048, E = TYPE == PM_Q5_K || TYPE == PM_Q6_K ? 2 : 1;
+    const uint8_t * Wg; uint32_t row[NG], ag[NG], sw; int h, K, nsteps, nb;
+    // group g0 + u; row n0 + 32 (r0 + u) of the matrix on
+    __device__ __forceinline__ void init(const PfP & p, const PfJob & jb, int n0, int g0, int r0, uint32_t lds0, int lane) {
+        Wg = jb.W; h = lane >> 5; K = p.K; nsteps = K / 128; nb = (K + 255) / 256; sw = 0;
+#pragma unroll
+        for (int u = 0; u < NG; ++u) {
+            row[u] = (uint32_t) min(n0 + 32 * (r0 + u) + (lane & 31), jb.N - 1) * (uint32_t) jb.row_stride;
+            ag[u] = lds0 + (uint32_t) (6 * NT * 32 * 128 + (g0 + u) * mid_group_bytes<TYPE, EX>());
+        }
+    }
+    // part u (0..3) of step s's requests
+    __device__ __forceinline__ void issue(int s, bool even, int u) const {
+        const uint32_t sc = (uint32_t) min(s, nsteps - 1);
+        const int b = s >> 1;
+        const uint32_t bc = (uint32_t) min(b, nb - 1);
+#pragma unroll
+        for (int i = 0; i < NG; ++i) {
+            if (u < W) {                                        // stream u
+                uint32_t off;
+                if (TYPE == PM_Q8_0) off = (u & 1 ? (uint32_t) K / 2u : 0u) + (4u * sc + 2u * (uint32_t) (u >> 1) + (uint32_t) h) * 16u;       // blocks 2 k + h of k-step k = 2 s + u / 2, stream qa / qb
+                else if (TYPE == PM_Q5_K) off = (sc >> 1) * 176u + 48u + (sc & 1u) * 64u + 32u * (uint32_t) h + 16u * (uint32_t) u;
+                else off = 16u * (uint32_t) h + 32u * sc + (uint32_t) u * (uint32_t) nb * 64u;
+                dma16(Wg, row[i] + off, ag[i] + sw + u * 1024);
+            }
+            if (even && u == 3) {
+                const uint32_t off = TYPE == PM_Q4_K ? (uint32_t) nb * 128u + bc * 16u : TYPE == PM_Q5_K ? bc * 176u : TYPE == PM_Q8_0 ? (uint32_t) K + bc * 16u : pm_q6k_sc_off((uint32_t) nb, bc);
+                if (h == 0) dma16(Wg, row[i] + off, ag[i] + HDR + (b & 3) * 512);
+            }
+            if (even && u == 2) {
+                if (TYPE == PM_Q5_K) dma16(Wg, row[i] + bc * 176u + 16u + 16u * (uint32_t) h, ag[i] + XTRA + (b & 3) * 1024);
+                // (the d's of a group of eight super-blocks: with every one of them, the same bytes again)
+                if (TYPE == PM_Q6_K && h == 0) dma16(Wg, row[i] + pm_q6k_d_off((uint32_t) nb, (uint32_t) (8 * min(b >> 3, (nb - 1) >> 3))), ag[i] + XTRA + ((b >> 3) & 1) * 512);
+            }
+        }
+    }
+    __device__ __forceinline__ void turn() { sw = sw == AHEAD * SLOT ? 0 : sw + SLOT; }
+    // the next step's are there: all but those of the AHEAD - 1 steps behind it
+    static __device__ __forceinline__ void wait(bool even) {
+        if (even) mid_wait<NG * ((AHEAD - 1) * W + AHEAD / 2 * E)>(); else mid_wait<NG * ((AHEAD - 1) * W + (AHEAD - 1) / 2 * E)>();
+    }
+};
+// ... and the activations, every NW-th request of a step by one of NW waves: (64-k half, token rows 8 q .. + 8), lane (row lane / 8, chunk lane % 8 <- chunk ^ swizzle). EX: group sums and scales of
+// every token with an even step, for the next super-block
+template <int TYPE, int NT, bool EX, int NW> struct MidActs {
+    static constexpr int HB = NT * 32 * 128, BBUF = 2 * HB, NQ = 8 * NT / NW, XSUM = mid_sum_bytes<TYPE, NT>(), XB = XSUM + NT * 32 * 4, XS = 3 * BBUF + 4 * mid_group_bytes<TYPE, EX>(),
+                         XP = XSUM / NW, XN = EX ? (XP + 1023) / 1024 + 1 : 0;
+    const uint8_t * Xg, * Xd, * Xs; uint32_t src[NQ], lds, bw; int w, lane, nsteps, nb, ldt, t0;
+    __device__ __forceinline__ void init(const PfP & p, int t0_, int w_, uint32_t lds0, int lane_) {
+        Xg = (const uint8_t *) p.Xh; Xd = p.Xd; Xs = p.Xs; lds = lds0; bw = 0; w = w_; lane = lane_; nsteps = p.K / 128; nb = (p.K + 255) / 256; ldt = p.ldt; t0 = t0_;
+#pragma unroll
+        for (int i = 0; i < NQ; ++i) {
+            const int q = w + NW * i, t = 8 * (q % (4 * NT)) + (lane >> 3);
+            src[i] = (uint32_t) min(t0 + t, p.T - 1) * (uint32_t) (2 * p.K) + 128u * (uint32_t) (q / (4 * NT)) + 16u * (uint32_t) ((lane & 7) ^ ((t >> 1) & 7));
+        }
+    }
+    // requests [from, to) of step s
+    __device__ __forceinline__ void issue(int s, int from, int to) const {
+        const uint32_t at = (uint32_t) min(s, nsteps - 1) * 256u;
+#pragma unroll
+        for (int i = from; i < to; ++i) dma16(Xg, src[i] + at, lds + bw + (uint32_t) ((w + NW * i) * 1024));
+    }
+    __device__ __forceinline__ void issue_x(int b) const {
+        const uint32_t at = (uint32_t) min(b, nb - 1) * (uint32_t) ldt + (uint32_t) t0, dst = lds + (uint32_t) (XS + (b & 1) * XB);
+#pragma unroll
+        for (int o = 0; o < XP; o += 1024) if (o + lane * 16 < XP) dma16(Xs, at * 32u + (uint32_t) (w * XP + o + lane * 16), dst + (uint32_t) (w * XP + o));
+        if (lane < 8 * NT / NW) dma16(Xd, at * 4u + (uint32_t) (w * 128 * NT / NW + lane * 16), dst + (uint32_t) (XSUM + w * 128 * NT / NW));
+    }
+    __device__ __forceinline__ void turn() { bw = bw == 2 * BBUF ? 0 : bw + BBUF; }
+    static __device__ __forceinline__ void wait(bool x) { if (x) mid_wait<NQ + XN>(); else mid_wait<NQ>(); }
+};
+// Four waves of a workgroup that multiply nothing: 0, 1 bring the activations, 2, 3 the weights of two row groups each. (One wave's LDS-DMA moves 61 GB/s, two 119, a CU not much more than
+// that: 143. A request holds its wave up for 60-180 cycles while others are at it.)
+template <int TYPE, int NT, bool EX>
+__device__ __forceinline__ void mid_load(const PfP & p, const PfJob & jb, const int n0, const int t0, uint32_t lds0, const int role, const int b0, const int b1, const int lw, const int lane) {
+    const int n = min(2 * b1, p.K / 128) - 2 * b0;              // steps
+    auto meet = [&] __attribute__((always_inline)) { __builtin_amdgcn_s_barrier(); asm volatile("" ::: "memory"); };
+    if (lw < 2) {
+        typedef MidActs<TYPE, NT, EX, 2> A;
+        A x;
+        x.init(p, t0, lw, lds0, lane);
+        if (EX) x.issue_x(b0);
+        x.issue(2 * b0, 0, A::NQ); x.turn();
+        x.issue(2 * b0 + 1, 0, A::NQ); x.turn();
+        A::wait(false);
+        meet();
+        for (int s = 0; s < n; ++s) {
+            const bool with = EX && !(s & 1);
+            if (with) x.issue_x(b0 + (s >> 1) + 1);
+            x.issue(2 * b0 + s + 2, 0, A::NQ); x.turn();
+            A::wait(with);
+            meet();
+        }
+    } else {
+        typedef MidWeights<TYPE, NT, EX, 2> M;
+        M x;
+        x.init(p, jb, n0, 2 * (lw - 2), role ? 0 : 2 * (lw - 2), lds0, lane);
+        auto step = [&](int s, bool even) __attribute__((always_inline)) {
+#pragma unroll
+            for (int u = 0; u < 4; ++u) x.issue(s, even, u);
+            x.turn();
+        };
+#pragma unroll
+        for (int w = 0; w < M::AHEAD; ++w) step(2 * b0 + w, (w & 1) == 0);
+        M::wait(false);
+        meet();
+        for (int s = 0; s < n; ++s) {
+            const bool even = !(s & 1);
+            step(2 * b0 + s + M::AHEAD, M::AHEAD & 1 ? !even : even);
+            M::wait(even);
+            meet();
+        }
+    }
+    mid_wait<0>();                                              // (the look-ahead of the last steps has landed)
+}
 
 // EX - 8-bit activations (Q8_K blocks): what the matrix cores add up over a wave's 128 k of a super-block are whole numbers, and exact. B = the 8-bit values as F16, A = quant x 6-bit sub-block
 // scale as F16; an f32 accumulator holds whole numbers up to 2^24. Q4_K: at most 945 x 127 x 128, one accumulator. Q5_K: 1953 x 127 x 64 fits, so one accumulator per 64 k, added at the end;
@@ -486,78 +613,70 @@ template <int N> __device__ __forceinline__ void mid_wait() { asm volatile("s_wa
 // 256 k of a super-block at once: here the halves of a super-block meet as f32. Against an integer GEMM: scales per 32 k applied to int32 results cost as much vector work as the products
 // take, and scales inside 8-bit operands two products per sub-block (mmq_big.hip); here scale and quant share the multiply that the F16 form needs anyway.
 // Bound by the LDS-DMA like the F16 form, by the vector work at a super-block's end (3 x 16 instructions per 32 tokens) and, Q6_K, by twice the products; two sets of accumulators beside the
-// running sums leave room for 64 tokens per workgroup. 8B shape, 169 tokens, us with the quantizer's launch: ffn_gate | ffn_up 115 (Q6_K 162; six passes of 28 on mmq_i8.hip 26.6 each), wo 32,
-// ffn_down Q4_K 66, Q6_K 101 (35 each), wq | wk | wv with a Q6_K wv 58. (Q6_K's product and its remainder in ONE accumulator, 128 tokens: 148 and 84, and sums beyond 2^24 rounded 16 times.)
+// running sums leave room for 64 tokens per workgroup, one set and loaders for 96, one set for 128. 8B shape, 147 tokens, us in tiles of 128 / 96 tokens: ffn_gate | ffn_up 112 / 86, wo and ffn_down
+// 32.5 / 25.7, wq | wk | wv 31.5 / 24.9; Q6_K ffn_down without loaders / with 84 / 78; wq | wk | wv with a Q6_K wv 53. (Six passes of 28 on mmq_i8.hip: ffn_gate | ffn_up 26.6 each, ffn_down 35.) (Q6_K's product and its remainder in ONE accumulator, 128 tokens: 148 and 84, and sums beyond 2^24 rounded 16 times.)
 // Distance from 64 bits (2-norm, normal weights) of mmq_i8.hip / this form: Q4_K 4096 x 4096 1.20e-7 / 0.89e-7, x 14336 1.33e-7 / 1.06e-7, Q5_K 1.20e-7 / 0.88e-7, Q6_K 4096 x 14336 0.81e-7 / 0.79e-7,
 // 8192 x 28672 0.92e-7 / 0.86e-7 (running sums over all of a slice's super-blocks: 1.43e-7; minima of a whole super-block by either half in turn: Q4_K x 14336 1.84e-7).
-template <int TYPE, int NT, bool EX>
+template <int TYPE, int NT, bool EX, bool SELF>
 __device__ __forceinline__ void mid_body(const PfP & p, const PfJob & jb, const int n0, const int t0, uint8_t * smem, const int role, const int ks, const int S, const int tile_id) {
     constexpr int HB = NT * 32 * 128, BBUF = 2 * HB;           // activations: 32 NT tokens x 64 halfs, two of them per step
-    constexpr int SLOT = mid_slot<TYPE>(), AG = mid_group_bytes<TYPE, EX>(), NH = NT / 2, AHEAD = mid_ahead<TYPE, EX>(), HDR = (AHEAD + 1) * SLOT, XTRA = HDR + 2048;
-    constexpr int XS = 3 * BBUF + 4 * AG, XSUM = mid_sum_bytes<TYPE, NT>(), XB = XSUM + NT * 32 * 4, XN = EX ? XSUM ? 2 : 1 : 0;      // EX: sums and scales; requests for them per super-block
+    constexpr int SLOT = mid_slot<TYPE>(), AG = mid_group_bytes<TYPE, EX>(), NH = (NT + 1) / 2, AHEAD = mid_ahead<TYPE, EX>(), HDR = (AHEAD + 1) * SLOT, XTRA = HDR + 2048;
+    constexpr int XS = 3 * BBUF + 4 * AG, XSUM = mid_sum_bytes<TYPE, NT>(), XB = XSUM + NT * 32 * 4;      // EX: sums and scales
     constexpr bool K45 = TYPE == PM_Q4_K || TYPE == PM_Q5_K, Q8 = TYPE == PM_Q8_0;
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), g = wave & 3, kk = wave >> 2;       // (waves w and w + 4 share a SIMD)
     const int r = lane & 31, h = lane >> 5;
     const int K = p.K, nsteps = K / 128, nb = (K + 255) / 256;  // (Q8_0 rows may end on half a super-block: one step)
     uint8_t * const ag = smem + 3 * BBUF + g * AG;              // the row group's weights: slots of the steps in turn, header of super-block b % 4
-    const uint32_t lds0 = (uint32_t) (uintptr_t) (__attribute__((address_space(3))) uint8_t *) smem, ag_l = lds0 + 3 * BBUF + g * AG;
-    const uint8_t * const Wg = jb.W;
+    const uint32_t lds0 = (uint32_t) (uintptr_t) (__attribute__((address_space(3))) uint8_t *) smem;
     const int nw = n0 + 32 * (role ? g & 1 : g);                // first row of this wave
-    const uint32_t wrow = (uint32_t) min(nw + r, jb.N - 1) * (uint32_t) jb.row_stride;
-    const uint8_t * const Xg = (const uint8_t *) p.Xh;
-    uint32_t xsrc[2 * NT];                                      // instruction q: 64-k half q / NT, token rows 8 (g + 4 (q % NT)) .. + 8 (swizzled as above)
-#pragma unroll
-    for (int q = 0; q < 2 * NT; ++q) {
-        const int t = 8 * (g + 4 * (q % NT)) + (lane >> 3);
-        xsrc[q] = (uint32_t) min(t0 + t, p.T - 1) * (uint32_t) (2 * K) + 128u * (uint32_t) (q / NT) + 16u * (uint32_t) ((lane & 7) ^ ((t >> 1) & 7));
+    // split K: slice ks of S takes the super-blocks [b0, b1)
+    const int b0 = (int) ((long) ks * nb / S), b1 = (int) ((long) (ks + 1) * nb / S);
+    // the waves meet; what they wrote to LDS, and what a loader waited for, is there
+    auto meet = [&] __attribute__((always_inline)) {
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+    };
+    if (!SELF && wave >= 8) {
+        mid_load<TYPE, NT, EX>(p, jb, n0, t0, lds0, role, b0, b1, wave - 8, lane);
+        meet(); meet(); meet();                                 // the ones behind the loop below
+        if (S == 1 && role) meet();
+        return;
     }
     const uint32_t boff0 = (uint32_t) (kk * HB + r * 128 + ((h ^ ((r >> 1) & 7)) << 4));
     const uint32_t aoff = (uint32_t) (r * 16 + 8 * h);
-
-    // Requests return in order, and weights come from memory, activations mostly from L2: the waves of the first half request the weights, AHEAD steps ahead, those of the
-    // second half the activations, two steps ahead (with both behind one counter every weight was waited for after two steps)
-    // part u (0..3) of step s's requests
-    auto issue_A = [&](int s, uint32_t sl, bool even, int u) __attribute__((always_inline)) {
-        const uint32_t sc = (uint32_t) min(s, nsteps - 1);
-        const int b = s >> 1;
-        const uint32_t bc = (uint32_t) min(b, nb - 1);
-        if (u < SLOT / 1024) {                                  // stream u
-            uint32_t off;
-            if (Q8) off = (u & 1 ? (uint32_t) K / 2u : 0u) + (4u * sc + 2u * (uint32_t) (u >> 1) + (uint32_t) h) * 16u;       // blocks 2 k + h of k-step k = 2 s + u / 2, stream qa / qb
-            else if (TYPE == PM_Q5_K) off = (sc >> 1) * 176u + 48u + (sc & 1u) * 64u + 32u * (uint32_t) h + 16u * (uint32_t) u;
-            else off = 16u * (uint32_t) h + 32u * sc + (uint32_t) u * (uint32_t) nb * 64u;
-            dma16(Wg, wrow + off, ag_l + sl + u * 1024);
-        }
-        if (even && u == 3) {
-            const uint32_t off = TYPE == PM_Q4_K ? (uint32_t) nb * 128u + bc * 16u : TYPE == PM_Q5_K ? bc * 176u : Q8 ? (uint32_t) K + bc * 16u : pm_q6k_sc_off((uint32_t) nb, bc);
-            if (h == 0) dma16(Wg, wrow + off, ag_l + HDR + (b & 3) * 512);
-        }
-        if (even && u == 2) {
-            if (TYPE == PM_Q5_K) dma16(Wg, wrow + bc * 176u + 16u + 16u * (uint32_t) h, ag_l + XTRA + (b & 3) * 1024);
-            // (the d's of a group of eight super-blocks: with every one of them, the same bytes again)
-            if (TYPE == PM_Q6_K && h == 0) dma16(Wg, wrow + pm_q6k_d_off((uint32_t) nb, (uint32_t) (8 * min(b >> 3, (nb - 1) >> 3))), ag_l + XTRA + ((b >> 3) & 1) * 512);
+    // SELF: requests of the first half's waves for the weights of their rows, of the second half's for the activations, a quarter of a step's behind each slice's products
+    struct Own { MidWeights<TYPE, NT, EX, 1> w; MidActs<TYPE, NT, EX, 4> x; };
+    struct None {};
+    std::conditional_t<SELF, Own, None> own_rq;
+    auto request = [&](int s, bool even, int u) __attribute__((always_inline)) {
+        if constexpr (SELF) {
+            constexpr int Q = decltype(own_rq.x)::NQ / 4, AHEAD = decltype(own_rq.w)::AHEAD;
+            if (kk) { if (even && u == 0) own_rq.x.issue_x((s >> 1) + 1); own_rq.x.issue(s + 2, Q * u, Q * u + Q); } else own_rq.w.issue(s + AHEAD, AHEAD & 1 ? !even : even, u);
         }
     };
-    auto issue_B = [&](int s, uint32_t bb, int u) __attribute__((always_inline)) {
-        const uint32_t sc = (uint32_t) min(s, nsteps - 1);
-#pragma unroll
-        for (int v = 0; v < NH; ++v) { const int q = NH * u + v; dma16(Xg, xsrc[q] + sc * 256u, lds0 + bb + (q / NT) * HB + (g + 4 * (q % NT)) * 1024); }
-    };
-    auto issue_X = [&](int b) __attribute__((always_inline)) {     // a quarter of a super-block's sums and scales per wave
-        const uint32_t at = (uint32_t) min(b, nb - 1) * (uint32_t) p.ldt + (uint32_t) t0, dst = lds0 + (uint32_t) (XS + (b & 1) * XB);
-        if (XSUM && lane < 16 * NT) dma16(p.Xs, at * 32u + (uint32_t) (g * 256 * NT + lane * 16), dst + (uint32_t) (g * 256 * NT));
-        if (lane < 2 * NT) dma16(p.Xd, at * 4u + (uint32_t) (g * 32 * NT + lane * 16), dst + (uint32_t) (XSUM + g * 32 * NT));
-    };
-    // end of an even / odd step: the next one's weights (all but those of the AHEAD - 1 steps behind it) and activations are there, this wave's LDS reads are through
+    // the end of a step: the next one's operands are there (a loader waited for them, or this wave), this wave's LDS reads are through
     auto settle = [&](bool even) __attribute__((always_inline)) {
-        constexpr int W = SLOT / 1024, E = TYPE == PM_Q5_K || TYPE == PM_Q6_K ? 2 : 1;
-        if (kk && even) mid_wait<2 * NT + XN>();
-        else if (kk) mid_wait<2 * NT>();
-        else if (even) mid_wait<(AHEAD - 1) * W + AHEAD / 2 * E>();
-        else mid_wait<(AHEAD - 1) * W + (AHEAD - 1) / 2 * E>();
-        __builtin_amdgcn_s_barrier();
+        if constexpr (SELF) { if (kk) { own_rq.x.wait(even); own_rq.x.turn(); } else { own_rq.w.wait(even); own_rq.w.turn(); } }
+        meet();
     };
+    if constexpr (SELF) {
+        if (kk) {
+            own_rq.x.init(p, t0, g, lds0, lane);
+            own_rq.x.issue_x(b0);
+            own_rq.x.issue(2 * b0, 0, 2 * NT); own_rq.x.turn();
+            own_rq.x.issue(2 * b0 + 1, 0, 2 * NT);
+        } else {
+            own_rq.w.init(p, jb, n0, g, role ? g & 1 : g, lds0, lane);
+#pragma unroll
+            for (int w = 0; w < AHEAD; ++w) {
+#pragma unroll
+                for (int u = 0; u < 4; ++u) own_rq.w.issue(2 * b0 + w, (w & 1) == 0, u);
+                if (w + 1 < AHEAD) own_rq.w.turn();
+            }
+        }
+    }
 
     float16v acc[NT];
 #pragma unroll
@@ -575,12 +694,14 @@ __device__ __forceinline__ void mid_body(const PfP & p, const PfJob & jb, const 
 #pragma unroll
             for (int e = 0; e < 16; ++e) { run[jt][e] = 0.0f; if (SUMS) tot[jt][e] = 0.0f; }
     // the 4 slices of this wave's half of the step in buffer bb / slot sl: 128-k half mm of super-block b
-    // a quarter of the step's requests behind each slice's MFMAs (an issue blocks the wave for 60-180 cycles: in front of the step they were 0.4 of its 1.25 us)
-    auto multiply = [&](int b, int mm, uint32_t bb, uint32_t sl, auto && request) __attribute__((always_inline)) {
+    // (addresses that a step or a super-block's end forms anew instead of keeping them in registers, which then spill)
+    auto anew = [](uint32_t v) __attribute__((always_inline)) { if (EX && !SELF) asm volatile("" : "+v"(v)); return v; };
+    auto multiply = [&](int b, int mm, uint32_t bb, uint32_t sl) __attribute__((always_inline)) {
+        const uint32_t bo = anew(boff0);
         half8 bf[2][NT], af[2], al[2];
         auto read_B = [&](int j) __attribute__((always_inline)) {
 #pragma unroll
-            for (int jt = 0; jt < NT; ++jt) bf[j & 1][jt] = *(const half8 *) (smem + bb + jt * 4096 + (boff0 ^ (uint32_t) (j << 5)));
+            for (int jt = 0; jt < NT; ++jt) bf[j & 1][jt] = *(const half8 *) (smem + bb + jt * 4096 + (bo ^ (uint32_t) (j << 5)));
         };
         u32x4 hd = {0, 0, 0, 0};
         uint16_t d6 = 0;
@@ -639,18 +760,20 @@ __device__ __forceinline__ void mid_body(const PfP & p, const PfJob & jb, const 
             if constexpr (TWO && TYPE == PM_Q6_K)
 #pragma unroll
                 for (int jt = 0; jt < NT; ++jt) ac2[jt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(al[j & 1], bf[j & 1][jt], mm + j == 0 ? zero : ac2[jt], 0, 0, 0);
-            request(j);
+            request(2 * b + mm, mm == 0, j);
         }
     };
     // EX: the whole numbers of super-block b (this wave's half of its k, and the minima of that half: without them the halves' sums are twice as large, and their roundings) onto the running sums
     auto fold = [&](int b) __attribute__((always_inline)) {
-        const uint8_t * const xb = smem + XS + (b & 1) * XB;
+        const uint32_t ln = anew((uint32_t) lane), r = ln & 31, h = ln >> 5;
+        const uint8_t * const xs = smem + XS + (b & 1) * XB + r * 32 + 16 * h, * const xd = smem + XS + (b & 1) * XB + XSUM + r * 4;
+        const uint8_t * const gh = ag + HDR + (b & 3) * 512 + h * 64, * const gd = ag + XTRA + ((b >> 3) & 1) * 512 + h * 64 + (b & 7) * 2;      // the half's first row
         uint32_t dd[16];                                        // d, dmin of the rows (F16)
 #pragma unroll
         for (int e = 0; e < 16; ++e) {
-            const int row = (e & 3) + 8 * (e >> 2) + 4 * h;
-            if (K45) dd[e] = *(const uint32_t *) (ag + HDR + (b & 3) * 512 + row * 16);
-            else dd[e] = *(const uint16_t *) (ag + XTRA + ((b >> 3) & 1) * 512 + row * 16 + (b & 7) * 2);
+            const int row = (e & 3) + 8 * (e >> 2);
+            if (K45) dd[e] = *(const uint32_t *) (gh + row * 16);
+            else dd[e] = *(const uint16_t *) (gd + row * 16);
         }
         auto d = [&](int e) __attribute__((always_inline)) { return h2f((uint16_t) dd[e]); };
         auto dm = [&](int e) __attribute__((always_inline)) { return h2f((uint16_t) (dd[e] >> 16)); };
@@ -667,12 +790,12 @@ __device__ __forceinline__ void mid_body(const PfP & p, const PfJob & jb, const 
 #pragma unroll
         for (int jt = 0; jt < NT; ++jt) {
             if (NT == 4) __builtin_amdgcn_sched_barrier(0);     // (the minima of all four token tiles at once: registers spill)
-            const float da = *(const float *) (xb + XSUM + (32 * jt + r) * 4);
+            const float da = *(const float *) (xd + 128 * jt);
             if constexpr (TWO)
 #pragma unroll
                 for (int e = 0; e < 16; ++e) acc[jt][e] = TYPE == PM_Q6_K ? fmaf(64.0f, acc[jt][e], ac2[jt][e]) : acc[jt][e] + ac2[jt][e];
             if (K45) {
-                const float16v am = __builtin_amdgcn_mfma_f32_32x32x16_f16(mo, *(const half8 *) (xb + (32 * jt + r) * 32 + 16 * h), zero, 0, 0, 0);
+                const float16v am = __builtin_amdgcn_mfma_f32_32x32x16_f16(mo, *(const half8 *) (xs + 1024 * jt), zero, 0, 0, 0);
 #pragma unroll
                 for (int e = 0; e < 16; ++e) run[jt][e] = fmaf(da, fmaf(-dm(e), am[e], d(e) * acc[jt][e]), run[jt][e]);
             } else {
@@ -682,27 +805,15 @@ __device__ __forceinline__ void mid_body(const PfP & p, const PfJob & jb, const 
         }
     };
 
-    // split K: slice ks of S takes the super-blocks [b0, b1)
-    const int b0 = (int) ((long) ks * nb / S), b1 = (int) ((long) (ks + 1) * nb / S);
-    uint32_t bb = 0, bn = BBUF, bw = 2 * BBUF, sl = 0, sw = AHEAD * SLOT;       // buffers of steps s, s + 1, s + 2, slots of steps s and s + AHEAD
-    auto request = [&](int s, bool even, int u) __attribute__((always_inline)) { if (kk) { if (EX && even && u == 0) issue_X((s >> 1) + 1); issue_B(s + 2, bw, u); } else issue_A(s + AHEAD, sw, AHEAD & 1 ? !even : even, u); };
-    auto turn = [&] __attribute__((always_inline)) { const uint32_t t = bb; bb = bn; bn = bw; bw = t; sw = sl; sl = sl == AHEAD * SLOT ? 0 : sl + SLOT; };
-#pragma unroll
-    for (int u = 0; u < 8; ++u) if (kk) {
-        if (EX && u == 0) issue_X(b0);
-        issue_B(2 * b0 + (u >> 2), u & 4 ? bn : bb, u & 3);
-    }
-#pragma unroll
-    for (int w = 0; w < AHEAD; ++w)
-#pragma unroll
-        for (int u = 0; u < 4; ++u) if (!kk) issue_A(2 * b0 + w, w * SLOT, (w & 1) == 0, u);
+    uint32_t bb = 0, sl = 0;                                    // buffer and slot of the step
+    auto turn = [&] __attribute__((always_inline)) { bb = bb == 2 * BBUF ? 0 : bb + BBUF; sl = sl == AHEAD * SLOT ? 0 : sl + SLOT; };
     settle(false);
     for (int b = b0; b < b1; ++b) {
-        multiply(b, 0, bb, sl, [&](int u) __attribute__((always_inline)) { request(2 * b, true, u); });
+        multiply(b, 0, bb, sl);
         settle(true);
         turn();
         if (Q8 && 2 * b + 1 >= nsteps) break;
-        multiply(b, 1, bb, sl, [&](int u) __attribute__((always_inline)) { request(2 * b + 1, false, u); });
+        multiply(b, 1, bb, sl);
         if constexpr (EX) fold(b);
         if constexpr (SUMS)
             if (((b - b0) & 3) == 3)
@@ -713,39 +824,44 @@ __device__ __forceinline__ void mid_body(const PfP & p, const PfJob & jb, const 
         settle(false);
         turn();
     }
+    if constexpr (SELF) mid_wait<0>();
     if constexpr (EX)
 #pragma unroll
         for (int jt = 0; jt < NT; ++jt) {
             acc[jt] = run[jt];
             if constexpr (SUMS) acc[jt] += tot[jt];
         }
-    mid_wait<0>();                                             // (the last steps' look-ahead still lands in the buffers)
-    __syncthreads();
-    // ---- the two halves of K: every wave keeps its rows' tokens [32 NH kk, + 32 NH) and takes the partner's sums of them
+    meet();                                                     // (the loaders: their look-ahead has landed)
+    // ---- the two halves of K: every wave keeps its rows' sub-tiles of 32 tokens NH kk, .. (NT = 3: two and one) and takes the partner's sums of them
     f32x4 * const xl = (f32x4 *) smem;
     float16v own[NH];
 #pragma unroll
     for (int i = 0; i < NH; ++i) {
-        const float16v give = kk ? acc[i] : acc[NH + i];
-        own[i] = kk ? acc[NH + i] : acc[i];
+        constexpr int LAST = NT - 1;
+        if (kk || NH + i < NT) {
+            const float16v give = kk ? acc[i] : acc[NH + i < NT ? NH + i : LAST];
 #pragma unroll
-        for (int q = 0; q < 4; ++q) xl[((wave * NH + i) * 4 + q) * 64 + lane] = f32x4{give[4 * q], give[4 * q + 1], give[4 * q + 2], give[4 * q + 3]};
+            for (int q = 0; q < 4; ++q) xl[((wave * NH + i) * 4 + q) * 64 + lane] = f32x4{give[4 * q], give[4 * q + 1], give[4 * q + 2], give[4 * q + 3]};
+        }
+        own[i] = kk ? acc[NH + i < NT ? NH + i : LAST] : acc[i];
     }
-    __syncthreads();
+    meet();
 #pragma unroll
     for (int i = 0; i < NH; ++i)
+        if (!kk || NH + i < NT)
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const f32x4 o = xl[(((wave ^ 4) * NH + i) * 4 + q) * 64 + lane];
+            for (int q = 0; q < 4; ++q) {
+                const f32x4 o = xl[(((wave ^ 4) * NH + i) * 4 + q) * 64 + lane];
 #pragma unroll
-            for (int e = 0; e < 4; ++e) own[i][4 * q + e] += o[e];
-        }
-    __syncthreads();
+                for (int e = 0; e < 4; ++e) own[i][4 * q + e] += o[e];
+            }
+    meet();
     // ---- split K: slabs, as above
     if (S > 1) {
         f32x4 * const mine = (f32x4 *) p.ws + (size_t) (tile_id * S + ks) * (8 * NH * 4 * 64);
 #pragma unroll
         for (int i = 0; i < NH; ++i) {
+            if (kk && NH + i >= NT) break;
             f32x4 o[4];
 #pragma unroll
             for (int q = 0; q < 4; ++q) o[q] = f32x4{own[i][4 * q], own[i][4 * q + 1], own[i][4 * q + 2], own[i][4 * q + 3]};
@@ -761,7 +877,7 @@ __device__ __forceinline__ void mid_body(const PfP & p, const PfJob & jb, const 
 #pragma unroll
                 for (int q = 0; q < 4; ++q) xl[(((2 * kk + (g & 1)) * NH + i) * 4 + q) * 64 + lane] = f32x4{own[i][4 * q], own[i][4 * q + 1], own[i][4 * q + 2], own[i][4 * q + 3]};
         }
-        __syncthreads();
+        meet();
         if (role == 1) return;
 #pragma unroll
         for (int i = 0; i < NH; ++i)
@@ -776,6 +892,7 @@ __device__ __forceinline__ void mid_body(const PfP & p, const PfJob & jb, const 
     uint8_t * const xe = smem + 8 * NH * 4096 + wave * (32 * 144);
 #pragma unroll
     for (int i = 0; i < NH; ++i) {
+        if (kk && NH + i >= NT) break;
 #pragma unroll
         for (int q = 0; q < 4; ++q) *(f32x4 *) (xe + r * 144 + (8 * q + 4 * h) * 4) = f32x4{own[i][4 * q], own[i][4 * q + 1], own[i][4 * q + 2], own[i][4 * q + 3]};
 #pragma unroll
@@ -800,7 +917,7 @@ __device__ __forceinline__ void mid_body(const PfP & p, const PfJob & jb, const 
 // block id -> (row tile, token tile): XCD x = id % 8 takes the row tiles x, x + 8, ..; its consecutive slots sweep the token tiles of one row tile, so the
 // workgroups that run together on an XCD share a few row tiles of weights and the activation k-slices in its L2 (mmq_big.hip's mapping)
 template <int TA, int TB, int NT, bool MID = false, int EXP = 0, bool EX = false>
-__global__ __launch_bounds__(PF_NTHR) void gemm_pf_kernel(PfP p) {
+__global__ __launch_bounds__((MID && !mid_self<TA, TB, NT, EX>() ? MID_NTHR : PF_NTHR)) void gemm_pf_kernel(PfP p) {
     extern __shared__ __attribute__((aligned(1024))) uint8_t pf_smem[];
     const int id = (int) blockIdx.x, x = id & 7;
     // slots [0, full) of an XCD run whole tiles; the slots behind them are split S ways along K, the slices of a tile neighbours on one XCD.
@@ -815,7 +932,8 @@ __global__ __launch_bounds__(PF_NTHR) void gemm_pf_kernel(PfP p) {
     int n0, role = 0;
     constexpr int ROWS = MID ? 128 : 256;
     if (p.pair) {                                              // ROWS / 2-row tiles of job 0 (waves 0-3; mid_body: row groups 0, 1) and job 1
-        role = 1 + __builtin_amdgcn_readfirstlane((int) (MID ? (threadIdx.x >> 7) & 1 : threadIdx.x >> 8));
+        // (of mid_body's loaders wave 10 brings the weights of job 0, wave 11 those of job 1)
+        role = 1 + __builtin_amdgcn_readfirstlane((int) (!MID ? threadIdx.x >> 8 : threadIdx.x < 512 ? (threadIdx.x >> 7) & 1 : (threadIdx.x >> 6) & 1));
         if (role == 2) jb = p.job[1];
         n0 = tile_n * (ROWS / 2);
     } else {
@@ -829,8 +947,9 @@ __global__ __launch_bounds__(PF_NTHR) void gemm_pf_kernel(PfP p) {
         if (TA == TB || jb.type == TA) pf_body<TA, NT, EXP>(p, jb, n0, t0, pf_smem, role, ks, S, tile_id);
         else pf_body<TB, NT, EXP>(p, jb, n0, t0, pf_smem, role, ks, S, tile_id);
     } else {
-        if (TA == TB || jb.type == TA) mid_body<TA, NT, EX>(p, jb, n0, t0, pf_smem, role, ks, S, tile_id);
-        else mid_body<TB, NT, EX>(p, jb, n0, t0, pf_smem, role, ks, S, tile_id);
+        constexpr bool SELF = mid_self<TA, TB, NT, EX>();
+        if (TA == TB || jb.type == TA) mid_body<TA, NT, EX, SELF>(p, jb, n0, t0, pf_smem, role, ks, S, tile_id);
+        else mid_body<TB, NT, EX, SELF>(p, jb, n0, t0, pf_smem, role, ks, S, tile_id);
     }
 }
 
@@ -839,10 +958,11 @@ __global__ __launch_bounds__(PF_NTHR) void gemm_pf_kernel(PfP p) {
 // itself, 48 us behind the last product. us, last arriver (as it was; its loads in fours and the slabs written through) / product + this launch: 512 tokens of 8192 x 8192 Q4_K 107 (102) / 66 + 17,
 // 8192 x 28672 264 (245) / 211 + 17, 10240 x 8192 131 (120) / 91 + 15; 101 tokens (mid_body) of 4096 x 4096 23.0 / 18.3 + 4.8, 4096 x 14336 35.9 / 27.7 + 5.9. (A wave per 32 tokens: 18.7 for 16.8 and
 // 8.1 for 5.9)
-// nti: token sub-tiles of a wave; mid: mid_body's tiles (wave = row group + 4 x token half)
-template <int SMAX> __global__ __launch_bounds__(256) void pf_reduce_kernel(PfP p, int mid, int nti, int units) {
+// nt: sub-tiles of 32 tokens in a tile; mid: mid_body's tiles (wave = row group + 4 x token half)
+template <int SMAX> __global__ __launch_bounds__(256) void pf_reduce_kernel(PfP p, int mid, int nt, int units) {
     const int u4 = (int) blockIdx.x * 4 + __builtin_amdgcn_readfirstlane((int) threadIdx.x >> 6), unit = u4 >> 2, k0 = u4 & 3, lane = threadIdx.x & 63;
     if (unit >= units) return;
+    const int nti = mid ? (nt + 1) / 2 : nt;                    // sub-tiles of a wave
     const int S = p.splitk, per_tile = (p.pair ? 4 : 8) * nti, tile_id = unit / per_tile, wv = unit % per_tile / nti, i = unit % nti;
     const int x = tile_id & 7, slot = p.full + (tile_id >> 3), per_x = (p.nt_n + 7 - x) >> 3;
     if (slot >= per_x * p.nt_t) return;
@@ -858,7 +978,8 @@ template <int SMAX> __global__ __launch_bounds__(256) void pf_reduce_kernel(PfP 
         n0 = (tile_n - jb.tile0) * (mid ? 128 : 256);
         if (mid) { row = wv & 3; half = wv >> 2; }
     }
-    const int t0 = (tile_t * (mid ? 2 : 1) + half) * 32 * nti + 32 * i + 8 * k0, t = t0 + (lane >> 3), n = n0 + 32 * row + (lane & 7) * 4;
+    if (half * nti + i >= nt) return;
+    const int t0 = (tile_t * nt + half * nti + i) * 32 + 8 * k0, t = t0 + (lane >> 3), n = n0 + 32 * row + (lane & 7) * 4;
     if (t0 >= p.T || n >= jb.N) return;                         // (N is a multiple of 4)
     const size_t tile = (size_t) 8 * nti * 256;                 // of f32x4
     const f32x4 * const slab = (const f32x4 *) p.ws + (size_t) tile_id * S * tile + 64 * k0 + lane;
@@ -892,12 +1013,12 @@ template <int SMAX> __global__ __launch_bounds__(256) void pf_reduce_kernel(PfP 
 // The same for one matrix of which every tile is split, a workgroup per token, with the RMS norm of the token's new row (rmsnorm_q8k_kernel's expressions in its order, F16): the row does not
 // travel to memory and back, and a launch goes. Bound by the slabs. us, both launches / this one: 101 tokens x 4096, S = 4 4.8 + 4.6 / 5.3, S = 8 5.9 + 4.6 / 6.3; 512 x 8192, S = 4 16.8 + 9.9 / 20.8 (28.3
 // with 4 waves a token). For up to 512 tokens: beyond, few launches have every tile split
-template <int SMAX> __global__ __launch_bounds__(1024) void pf_reduce_norm_kernel(PfP p, int mid, int nti, const float * w, float eps, _Float16 * yh) {
+template <int SMAX> __global__ __launch_bounds__(1024) void pf_reduce_norm_kernel(PfP p, int mid, int nt, const float * w, float eps, _Float16 * yh) {
     constexpr int NWV = 16, HOLD = 2;
     __shared__ double red[NWV];
     const int t = blockIdx.x, lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane((int) threadIdx.x >> 6), S = p.splitk;
     const PfJob & jb = p.job[0];
-    const int N = jb.N, rows = mid ? 128 : 256, tok = mid ? 64 * nti : 32 * nti;
+    const int N = jb.N, rows = mid ? 128 : 256, tok = 32 * nt, nti = mid ? (nt + 1) / 2 : nt;
     const int tile_t = t / tok, tt = t % tok / 32, half = mid ? tt / nti : 0, i = mid ? tt % nti : tt;
     const size_t tile = (size_t) 8 * nti * 256;                 // of f32x4
     f32x4 f[HOLD], wt[HOLD];
@@ -945,10 +1066,10 @@ template <int SMAX> __global__ __launch_bounds__(1024) void pf_reduce_norm_kerne
 
 // The same for wq | wk | wv, with NORM rope (rope_kv_store_kernel's expressions, cos / sin from the pass's table) and the stores of K and V^T into the cache: the launch behind it and two trips of the
 // rows go. Bound by the chain of its loads. 101 tokens of 32 + 8 + 8 heads of 128, S = 4: 5.1 + 7.3 us as two launches, 6.4 as this one
-template <int SMAX> __global__ __launch_bounds__(1024) void pf_reduce_rope_kernel(PfP p, int mid, int nti, pm_gemm_rope a) {
+template <int SMAX> __global__ __launch_bounds__(1024) void pf_reduce_rope_kernel(PfP p, int mid, int nt, pm_gemm_rope a) {
     constexpr int NWV = 16, HOLD = 3;                           // rows of 256: up to 48
     const int t = blockIdx.x, lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane((int) threadIdx.x >> 6), S = p.splitk;
-    const int Nq = p.job[0].N, Nk = p.job[1].N, rows = mid ? 128 : 256, tok = mid ? 64 * nti : 32 * nti;
+    const int Nq = p.job[0].N, Nk = p.job[1].N, rows = mid ? 128 : 256, tok = 32 * nt, nti = mid ? (nt + 1) / 2 : nt;
     const int tile_t = t / tok, tt = t % tok / 32, half = mid ? tt / nti : 0, i = mid ? tt % nti : tt;
     const size_t tile = (size_t) 8 * nti * 256;                 // of f32x4
     const int seq = a.seq ? a.seq[a.rows ? t : 0] : 0, pos = a.rows ? a.pos[t] : a.pos[seq] + t;
@@ -1044,7 +1165,7 @@ int pm_gemm_pf_check(int type, int K, int N, int T) {
 // every partial tile through memory: 3 x 320 slabs of 256 KB for the qkv launch, 501 us = 685 TFLOP/s against 406 us = 846.
 void pm_gemm_pf_plan(int tiles, int K, int T, int cus, int force_nt, int force_s, int allow_mixed, pm_gemm_pf_plan_t * out) {
     int nt = T <= 64 ? 2 : T <= 128 ? 4 : 8;
-    if (force_nt == 2 || force_nt == 4 || force_nt == 8) nt = force_nt;
+    if ((force_nt >= 2 && force_nt <= 4) || force_nt == 8) nt = force_nt;
     const int nt_t = (T + 32 * nt - 1) / (32 * nt);
     const long wgs = (long) tiles * nt_t;
     const int nb = (K + 255) / 256;
@@ -1088,7 +1209,7 @@ static int launch_pf(const pm_gemm_pf_job * jobs, int njobs, const void * xh, co
     // the 8B shape; their 8-bit roundings turn), although neither is nearer to 64 bits
     bool two = false;                                           // 8-bit activations: tiles of 64 tokens for what needs a second set of accumulators
     for (int j = 0; j < njobs; ++j) two |= wide && jobs[j].type != PM_Q4_K;
-    const int mid_nt = T <= 64 || two ? 2 : 4;
+    const int mid_nt = T <= 64 || two ? 2 : T <= 96 ? 3 : 4;
     long mid_wgs = 0;
     for (int j = 0; j < njobs && !(pair && j); ++j) mid_wgs += (jobs[j].N + (pair ? 63 : 127)) / (pair ? 64 : 128);
     // (8-bit activations: mid_body at any size - its tiles of 128 tokens side by side -, pf_body's registers are its accumulators')
@@ -1119,6 +1240,12 @@ static int launch_pf(const pm_gemm_pf_job * jobs, int njobs, const void * xh, co
     // minimises  rounds of workgroups x (super-blocks per slice + ~3 for prologue, slab traffic and the launch that adds the slices up)
     pm_gemm_pf_plan_t pl;
     pm_gemm_pf_plan(tiles, K, T, cus, mid ? mid_nt : force_nt, force_s, no_mixed ? 0 : 1, &pl);
+    // 8-bit activations of Q4_K: tiles of 96 tokens (with loaders) where they cost less than those of 128 (without: no registers left for them), by rounds of workgroups; the K split stays that of
+    // 128 tokens: the sums in one order. 8B shape, whole passes, us, 128 / 96: 79 tokens 716 / 675, 109 738 / 801, 147 935 / 858, 231 1025 / 1095, 316 1279 / 1260, 459 1498 / 1570
+    if (wide && !two && T > 64 && !pl.full && (T + 95) / 96 * 96 <= wide->ldt) {
+        const auto cost = [&](int nt) { return ((long) tiles * ((T + 32 * nt - 1) / (32 * nt)) * pl.splitk + cus - 1) / cus * (nt + 1); };
+        if (cost(3) < cost(4)) pm_gemm_pf_plan(tiles, K, T, cus, 3, pl.splitk, 0, &pl);
+    }
     const int nt = pl.nt, S = pl.splitk, full = pl.full, maxL = ((tiles + 7) / 8) * pl.nt_t;
     p.nt_t = pl.nt_t;
     p.splitk = S; p.full = full;
@@ -1126,18 +1253,17 @@ static int launch_pf(const pm_gemm_pf_job * jobs, int njobs, const void * xh, co
     std::unique_lock<std::mutex> slabs(g_pf_mu, std::defer_lock);
     if (S > 1) {
         slabs.lock();
-        const size_t slab = (size_t) (mid ? 4 : 8) * nt * 4 * 64 * 16, need = (size_t) 8 * split_slots * S * slab;
+        const size_t slab = (size_t) 8 * (mid ? (nt + 1) / 2 : nt) * 4 * 64 * 16, need = (size_t) 8 * split_slots * S * slab;
         p.ws = (float *) pf_workspace(st, need);
         if (!p.ws) return -3;
     }
     const int slots = full + split_slots * S;
     auto go = [&](auto kern, size_t lds) {
         pf_allow_lds((const void *) kern, lds);
-        hipLaunchKernelGGL(kern, dim3(8 * slots), dim3(PF_NTHR), lds, st, p);
+        hipLaunchKernelGGL(kern, dim3(8 * slots), dim3(mid && !(wide && (nt == 4 || ta != tb || ta == PM_Q5_K)) ? MID_NTHR : PF_NTHR), lds, st, p);
         if (S == 1) return;
-        const int nti = mid ? nt / 2 : nt;
         if (norm && !full && T <= 512 && njobs == 1 && jobs[0].Y && !jobs[0].Yh && !jobs[0].silu_gate && p.job[0].ldy == p.job[0].N && jobs[0].N % 256 == 0 && jobs[0].N <= 8192) {
-            auto fused = [&](auto k) { hipLaunchKernelGGL(k, dim3(T), dim3(1024), 0, st, p, (int) mid, nti, norm->w, norm->eps, (_Float16 *) norm->yh); };
+            auto fused = [&](auto k) { hipLaunchKernelGGL(k, dim3(T), dim3(1024), 0, st, p, (int) mid, nt, norm->w, norm->eps, (_Float16 *) norm->yh); };
             if (S <= 4) fused(pf_reduce_norm_kernel<4>); else fused(pf_reduce_norm_kernel<8>);
             norm->done = true;
             return;
@@ -1146,14 +1272,14 @@ static int launch_pf(const pm_gemm_pf_job * jobs, int njobs, const void * xh, co
         bool roped = rope && !full && T < 256 && njobs == 3 && !p.pair && jobs[1].N == jobs[2].N && jobs[1].N == rope->Hkv * rope->dh && jobs[0].N + 2 * jobs[1].N <= 48 * 256 && rope->dh % 4 == 0 && rope->n_dims % 4 == 0;
         for (int j = 0; j < njobs && roped; ++j) roped = jobs[j].N % 256 == 0 && jobs[j].Y && !jobs[j].Yh && !jobs[j].resid && !jobs[j].silu_gate && p.job[j].ldy == p.job[j].N && jobs[j].N % rope->dh == 0;
         if (roped) {
-            if (S <= 4) hipLaunchKernelGGL(pf_reduce_rope_kernel<4>, dim3(T), dim3(1024), 0, st, p, (int) mid, nti, *rope);
-            else        hipLaunchKernelGGL(pf_reduce_rope_kernel<8>, dim3(T), dim3(1024), 0, st, p, (int) mid, nti, *rope);
+            if (S <= 4) hipLaunchKernelGGL(pf_reduce_rope_kernel<4>, dim3(T), dim3(1024), 0, st, p, (int) mid, nt, *rope);
+            else        hipLaunchKernelGGL(pf_reduce_rope_kernel<8>, dim3(T), dim3(1024), 0, st, p, (int) mid, nt, *rope);
             rope->done = true;
             return;
         }
-        const int units = 8 * split_slots * (p.pair ? 4 : 8) * nti;
-        if (S <= 4) hipLaunchKernelGGL(pf_reduce_kernel<4>, dim3(units), dim3(256), 0, st, p, (int) mid, nti, units);
-        else        hipLaunchKernelGGL(pf_reduce_kernel<8>, dim3(units), dim3(256), 0, st, p, (int) mid, nti, units);
+        const int units = 8 * split_slots * (p.pair ? 4 : 8) * (mid ? (nt + 1) / 2 : nt);
+        if (S <= 4) hipLaunchKernelGGL(pf_reduce_kernel<4>, dim3(units), dim3(256), 0, st, p, (int) mid, nt, units);
+        else        hipLaunchKernelGGL(pf_reduce_kernel<8>, dim3(units), dim3(256), 0, st, p, (int) mid, nt, units);
     };
 #if PM_GEMM_ABLATE
     static const int exp_sw = [] { const char * e = getenv("PM355_GEMM_EXP"); return e ? atoi(e) : 0; }();
@@ -1180,7 +1306,7 @@ static int launch_pf(const pm_gemm_pf_job * jobs, int njobs, const void * xh, co
         return 0;
     }
 #endif
-#define PF_GO(A, B) (wide ? nt == 4 ? go(gemm_pf_kernel<PM_Q4_K, PM_Q4_K, 4, true, 0, true>, pf_lds_bytes<PM_Q4_K, PM_Q4_K, 4, true, true>()) : go(gemm_pf_kernel<A, B, 2, true, 0, A != PM_Q8_0>, pf_lds_bytes<A, B, 2, true, A != PM_Q8_0>()) : mid ? nt == 4 ? go(gemm_pf_kernel<A, B, 4, true>, pf_lds_bytes<A, B, 4, true>()) : go(gemm_pf_kernel<A, B, 2, true>, pf_lds_bytes<A, B, 2, true>()) : nt == 8 ? go(gemm_pf_kernel<A, B, 8>, pf_lds_bytes<A, B, 8>()) : nt == 4 ? go(gemm_pf_kernel<A, B, 4>, pf_lds_bytes<A, B, 4>()) : go(gemm_pf_kernel<A, B, 2>, pf_lds_bytes<A, B, 2>()))
+#define PF_GO(A, B) (wide ? nt == 4 ? go(gemm_pf_kernel<PM_Q4_K, PM_Q4_K, 4, true, 0, true>, pf_lds_bytes<PM_Q4_K, PM_Q4_K, 4, true, true>()) : nt == 3 ? go(gemm_pf_kernel<PM_Q4_K, PM_Q4_K, 3, true, 0, true>, pf_lds_bytes<PM_Q4_K, PM_Q4_K, 3, true, true>()) : go(gemm_pf_kernel<A, B, 2, true, 0, A != PM_Q8_0>, pf_lds_bytes<A, B, 2, true, A != PM_Q8_0>()) : mid ? nt == 4 ? go(gemm_pf_kernel<A, B, 4, true>, pf_lds_bytes<A, B, 4, true>()) : nt == 3 ? go(gemm_pf_kernel<A, B, 3, true>, pf_lds_bytes<A, B, 3, true>()) : go(gemm_pf_kernel<A, B, 2, true>, pf_lds_bytes<A, B, 2, true>()) : nt == 8 ? go(gemm_pf_kernel<A, B, 8>, pf_lds_bytes<A, B, 8>()) : nt == 4 ? go(gemm_pf_kernel<A, B, 4>, pf_lds_bytes<A, B, 4>()) : go(gemm_pf_kernel<A, B, 2>, pf_lds_bytes<A, B, 2>()))
     if (ta == tb) { if (ta == PM_Q4_K) PF_GO(PM_Q4_K, PM_Q4_K); else if (ta == PM_Q5_K) PF_GO(PM_Q5_K, PM_Q5_K); else if (ta == PM_Q8_0) PF_GO(PM_Q8_0, PM_Q8_0); else PF_GO(PM_Q6_K, PM_Q6_K); }
     else if (ta == PM_Q8_0 || tb == PM_Q8_0) return -1;      // (Q8_0 only as a launch of its own: ffn_down of the files whose n_ff is no multiple of 256)
     else if (ta == PM_Q4_K && tb == PM_Q5_K) PF_GO(PM_Q4_K, PM_Q5_K);

@@ -929,6 +929,30 @@ def test_prompt_gemm_tiles_of_128_rows(P, oracle, t, K, N, T):
         assert nm < 1e-6, (at, float(nm))
 
 
+@pytest.mark.parametrize("t", QUANT_TYPES)
+@pytest.mark.parametrize("K,N", [(512, 132), (4096, 260)])
+def test_prompt_tiles_of_96_tokens(P, t, K, N):
+    """Tiles of 96 tokens (65..96 tokens; of 8-bit activations also several side by side) beside those of 64 and 128: a token's sums are the same bits in each. Slices of K (4096) and none, rows that
+    end inside a wave's, several matrices and pairs; the first and last counts of a tile."""
+    rng = np.random.default_rng(K + N + t)
+    if t == Q8_0:
+        K += 128
+    w, w2 = (P.upload_weight(t, rand_blocks(t, N, K, rng), K, N) for _ in range(2))
+    x = _dev(P, rng.normal(0, 0.1, (512, K)).astype(np.float32))
+    full, multi = P.mul_mat_mfma(w, x[:128]), P.mul_mat_mfma_multi([w, w2], x[:128])
+    pair = P.mul_mat_mfma_pair(w, w2, x[:128]) if t != Q8_0 else None
+    for T in (64, 65, 95, 96, 97):
+        assert P.torch.equal(P.mul_mat_mfma(w, x[:T]), full[:T]), T
+        assert all(P.torch.equal(a, b[:T]) for a, b in zip(P.mul_mat_mfma_multi([w, w2], x[:T]), multi)), T
+        assert pair is None or P.torch.equal(P.mul_mat_mfma_pair(w, w2, x[:T]), pair[:T]), T
+    if t == Q8_0:
+        return
+    full, pair = P.mul_mat_wide([w], x)[0], P.mul_mat_wide([w, w2], x, pair=True)[0]
+    for T in (65, 96, 97, 128, 129, 192, 193, 288, 289, 480, 481):
+        assert P.torch.equal(P.mul_mat_wide([w], x[:T])[0], full[:T]), T
+        assert P.torch.equal(P.mul_mat_wide([w, w2], x[:T], pair=True)[0], pair[:T]), T
+
+
 @pytest.mark.parametrize("t", [Q4_K, Q5_K, Q6_K])
 @pytest.mark.parametrize("K,N,T", [(1024, 384, 200), (2048, 132, 64), (512, 256, 257), (8192, 132, 200)])
 def test_prompt_gemm_pair_tiles_silu_gate_times_up(P, oracle, t, K, N, T):
