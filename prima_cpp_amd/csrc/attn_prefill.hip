@@ -213,7 +213,8 @@ __global__ __launch_bounds__(256, 2) void attn_rowmajor_kernel(PfP p) {
 }
 
 // ---- the default graphs' layout: V transposed ---------------------------------------------------------------------------------------------------------------------------------
-// One workgroup = QW * 32 consecutive queries of one head; QW query waves x KW = 8 / QW key groups. Per stage KS keys of K ([KS][DH]) and V^T ([DH][KS]) travel by LDS-DMA
+// One workgroup = QW * 32 consecutive queries of one head; QW query waves x KW = 8 / QW key groups, and four waves that bring the keys and values (a request holds its wave up for 60-180 cycles: a
+// stage's eight per wave were 0.9 of the 1.5 us that a stage of 128 keys took; now 1.2, the requests' own time and their latency). Per stage KS keys of K ([KS][DH]) and V^T ([DH][KS]) travel by LDS-DMA
 // (double-buffered, 16-byte chunks XOR-swizzled on the source side so that the sixteen lanes a fragment read serves hit sixteen bank groups); key group kw multiplies keys
 // kw * KT .. + KT of every stage and keeps an online softmax of its own, the groups are merged through LDS at the end. Rows of a K tile are read with bits 2 and 3 of the row
 // index swapped: the accumulators of S^T then ARE the B operand of the P.V product.
@@ -222,12 +223,13 @@ __global__ __launch_bounds__(256, 2) void attn_rowmajor_kernel(PfP p) {
 // float64 with two passes, 1.6e-4 with one.
 // Bound by the LDS reads of the fragments (32 queries per wave: 32 KiB per 64 keys and wave at ~80 bytes per cycle and CU, about the time of the 32 matrix instructions) and the
 // exponentials beside them. Against the two-pass form with 4 waves x 32 queries, 32-key tiles through registers: 6001 tokens x 32 heads 870 -> 393 us (752 TFLOP/s), 512 x 64 behind
-// 1024 cached cells 102 -> 38, 101 x 32 behind 300 29.8 -> 11.7, 2048 x 32 144 -> 55.
+// 1024 cached cells 102 -> 38, 101 x 32 behind 300 29.8 -> 11.7, 2048 x 32 144 -> 55. Requests by the waves that multiply / by their own, whole passes: 70B shape, three layers, 8 tokens behind 403
+// cells 396 / 391, 8B shape, four layers and head, 101 behind 300 653 / 648, 6001 13330 / 13290. (Both stages asked for at once in front, keys behind the last one left out: no change.)
 // PLAIN: caches that do not start on 16 bytes, by loads and LDS stores instead of DMA
 // PAIR: tiles of up to 32 queries, the two query waves of a key group are two heads of one KV head; their results leave as Q8_K blocks (the wo product's activations) - no f32 rows and no launch that
-// quantizes them: 8 tokens x 64 heads behind 403 cells 11.3 + 5.0 us, now 13.3
+// quantizes them: 8 tokens x 64 heads behind 403 cells 11.3 + 5.0 us, with this ending 13.3, with waves that bring 12.0; 23 tokens and no other cells 11.8 / 9.0
 template <int DH, int QW, int KS, bool MASK, bool PLAIN = false, bool PAIR = false>
-__global__ __launch_bounds__(512, 2) void attn_prompt_kernel(PfP p, pm_q8k_out y) {
+__global__ __launch_bounds__(768, 3) void attn_prompt_kernel(PfP p, pm_q8k_out y) {
     static_assert(!PAIR || (DH == 128 && QW == 2 && !MASK && !PLAIN), "two heads are a block");
     constexpr int KW = 8 / QW, KT = KS / KW, ST = KT / 32;            // keys per wave and stage, 32-key score tiles
     constexpr int KK = DH / 16, DT = DH / 32, CK = DH / 8, CV = KS / 8;      // k-steps of a score tile, output tiles, 16-byte chunks per K row / V^T row
@@ -245,6 +247,7 @@ __global__ __launch_bounds__(512, 2) void attn_prompt_kernel(PfP p, pm_q8k_out y
     const int n_h = PAIR ? p.H / 2 : p.H;                         // (heads, or pairs of them)
     if (n_h % 8 == 0) { const int per = n_h / 8, j = blockIdx.x >> 3; h = (blockIdx.x & 7) * per + j % per; tile = j / per; }
     else { h = blockIdx.x % n_h; tile = blockIdx.x / n_h; }
+    const int pair = h;
     if (PAIR) h = 2 * h + qw;
     tile = p.n_tiles - 1 - tile;
     const int hk = h / (p.H / p.Hkv);
@@ -268,22 +271,49 @@ __global__ __launch_bounds__(512, 2) void attn_prompt_kernel(PfP p, pm_q8k_out y
         if constexpr (PLAIN) { u32x4 v; __builtin_memcpy(&v, base + off, 16); *(u32x4 *) (smem + to + lane * 16) = v; }
         else pm_dma16(base, off, lds0 + to);
     };
+    // a stage: every fourth piece of 1 KiB by each of the loaders
     auto request = [&](int it, int stage) __attribute__((always_inline)) {
         const char * kb = (const char *) (kc + (long) it * KS * krow), * vb = (const char *) vc;
         const int key0 = it * KS, kmax = p.n_ctx - 1 - key0, vmax = p.n_ctx - 8 - key0;          // (cells behind the cache: its last ones, masked)
 #pragma unroll
-        for (int i = 0; i < KS * DH * 2 / 8192; ++i) {
-            const int o = (wave + i * 8) * 64 + lane, row = o / CK, ch = o % CK;
-            bring(kb, (uint32_t) min(row, kmax) * (uint32_t) (krow * 2) + (uint32_t) (ch ^ (CK == 8 ? (row >> 1) & 7 : row & 15)) * 16u, stage * STAGE + (wave + i * 8) * 1024);
+        for (int i = 0; i < KS * DH * 2 / 4096; ++i) {
+            const int o = (wave - 8 + i * 4) * 64 + lane, row = o / CK, ch = o % CK;
+            bring(kb, (uint32_t) min(row, kmax) * (uint32_t) (krow * 2) + (uint32_t) (ch ^ (CK == 8 ? (row >> 1) & 7 : row & 15)) * 16u, stage * STAGE + (wave - 8 + i * 4) * 1024);
         }
 #pragma unroll
-        for (int i = 0; i < KS * DH * 2 / 8192; ++i) {
-            const int o = (wave + i * 8) * 64 + lane, row = o / CV, ch = o % CV;
+        for (int i = 0; i < KS * DH * 2 / 4096; ++i) {
+            const int o = (wave - 8 + i * 4) * 64 + lane, row = o / CV, ch = o % CV;
             const int key = key0 + min((ch ^ (CV == 8 ? (row >> 1) & 7 : row & 15)) * 8, vmax);
-            bring(vb, (uint32_t) row * (uint32_t) (p.n_ctx * 2) + (uint32_t) key * 2u, stage * STAGE + KS * DH * 2 + (wave + i * 8) * 1024);
+            bring(vb, (uint32_t) row * (uint32_t) (p.n_ctx * 2) + (uint32_t) key * 2u, stage * STAGE + KS * DH * 2 + (wave - 8 + i * 4) * 1024);
         }
     };
-    request(0, 0);
+    float * const ex = (float *) smem, * const ml = ex + 8 * 32 * OS;      // behind the loop: [wave][query][DH + 4], [wave][query]{m, l}
+    // PAIR: a wave per token, lanes 0 .. 31 the first head, 32 .. 63 the second
+    auto rows_of_pair = [&] __attribute__((always_inline)) {
+        for (int r = wave; r < nq; r += 12) {
+            float4 a = *(const float4 *) (ex + (hf * 32 + r) * OS + 4 * lr);
+#pragma unroll
+            for (int g = 1; g < KW; ++g) {
+                const float4 b = *(const float4 *) (ex + ((g * QW + hf) * 32 + r) * OS + 4 * lr);
+                a.x += b.x; a.y += b.y; a.z += b.z; a.w += b.w;
+            }
+            const float v[4] = {a.x, a.y, a.z, a.w};
+            q8k_block_from_regs(v, lane, y.y + (size_t) (row0 + r) * y.row_bytes, p.H * DH, pair, y.tab, row0 + r);
+        }
+    };
+    if (wave >= 8) {
+        request(0, 0);
+        for (int it = 0; it < n_it; ++it) {
+            pm_vm_drain();
+            __syncthreads();
+            if (it + 1 < n_it) request(it + 1, (it & 1) ^ 1);
+        }
+        __syncthreads();
+        if (KW > 1) __syncthreads();
+        __syncthreads();
+        if constexpr (PAIR) rows_of_pair();
+        return;
+    }
 
     // Q^T as B operand: lane (query lr, hf) holds q[query][16 kk + 8 hf .. + 8], rounded to F16 like the reference
     half8 q[KK];
@@ -312,9 +342,7 @@ __global__ __launch_bounds__(512, 2) void attn_prompt_kernel(PfP p, pm_q8k_out y
     const int kr = (lr & ~12) | ((lr & 4) << 1) | ((lr & 8) >> 1);
     for (int it = 0; it < n_it; ++it) {
         const int stage = it & 1;
-        pm_vm_drain();
         __syncthreads();
-        if (it + 1 < n_it) request(it + 1, stage ^ 1);
         const int key0 = it * KS + kw * KT;
         if (!live || key0 >= seen) continue;
         // cells behind the last attended one: a probability of 0 does not undo what they hold (0 x NaN), so they become zeros in LDS. Every wave of a key group writes the same bytes and
@@ -410,7 +438,6 @@ __global__ __launch_bounds__(512, 2) void attn_prompt_kernel(PfP p, pm_q8k_out y
     }
     l += __shfl_xor(l, 32);
     __syncthreads();                                              // (the stages become the exchange of the results)
-    float * ex = (float *) smem, * ml = ex + 8 * 32 * OS;         // [wave][query][DH + 4], [wave][query]{m, l}
     float f = 1.0f / l;
     if (KW > 1) {
         if (hf == 0) { ml[(wave * 32 + lr) * 2] = m; ml[(wave * 32 + lr) * 2 + 1] = l; }
@@ -423,26 +450,14 @@ __global__ __launch_bounds__(512, 2) void attn_prompt_kernel(PfP p, pm_q8k_out y
         f = __builtin_amdgcn_exp2f((m - M) * UNIT) / L;
     }
     // O^T[d][query]: queries are columns; through LDS, then a wave stores whole rows
+    if (q0 + lr < nq)
 #pragma unroll
     for (int d = 0; d < DT; ++d)
 #pragma unroll
         for (int g = 0; g < 4; ++g)
             *(float4 *) (ex + (wave * 32 + lr) * OS + d * 32 + 8 * g + 4 * hf) = float4{o[d][4 * g] * f, o[d][4 * g + 1] * f, o[d][4 * g + 2] * f, o[d][4 * g + 3] * f};
     __syncthreads();
-    if constexpr (PAIR) {                                          // a wave per token: lanes 0 .. 31 the first head, 32 .. 63 the second
-        const int K = p.H * DH;
-        for (int r = wave; r < nq; r += 8) {
-            float4 a = *(const float4 *) (ex + (hf * 32 + r) * OS + 4 * lr);
-#pragma unroll
-            for (int g = 1; g < KW; ++g) {
-                const float4 b = *(const float4 *) (ex + ((g * QW + hf) * 32 + r) * OS + 4 * lr);
-                a.x += b.x; a.y += b.y; a.z += b.z; a.w += b.w;
-            }
-            const float v[4] = {a.x, a.y, a.z, a.w};
-            q8k_block_from_regs(v, lane, y.y + (size_t) (row0 + r) * y.row_bytes, K, (h - qw) / 2, y.tab, row0 + r);
-        }
-        return;
-    }
+    if constexpr (PAIR) { rows_of_pair(); return; }
     constexpr int RL = DH / 4, RP = 64 / RL;                       // lanes per row (4 values each), rows per pass
     for (int r = kw * (32 / KW) + lane / RL; r < (kw + 1) * (32 / KW); r += RP) {
         if (q0 + r >= nq) break;
@@ -462,7 +477,7 @@ template <int DH, int QW, int KS, bool MASK, bool PLAIN = false, bool PAIR = fal
     if (!p.tiles) p.n_tiles = (p.T + QW * 32 - 1) / (QW * 32);
     constexpr size_t stages = 2 * (size_t) KS * DH * 4, ex = (size_t) 8 * 32 * (DH + 4) * 4 + 8 * 32 * 2 * 4, lds = stages > ex ? stages : ex;
     pm_allow_big_lds((const void *) attn_prompt_kernel<DH, QW, KS, MASK, PLAIN, PAIR>, lds);
-    hipLaunchKernelGGL((attn_prompt_kernel<DH, QW, KS, MASK, PLAIN, PAIR>), dim3(p.n_tiles * (PAIR ? p.H / 2 : p.H)), dim3(512), lds, st, p, y);
+    hipLaunchKernelGGL((attn_prompt_kernel<DH, QW, KS, MASK, PLAIN, PAIR>), dim3(p.n_tiles * (PAIR ? p.H / 2 : p.H)), dim3(768), lds, st, p, y);
 }
 // Which tile: a CU holds one workgroup. 256 queries share a stage where that still makes two rounds of workgroups (2048 tokens x 64 heads: 102 us, 110 with 128 queries; x 32 heads
 // = one round whose longest tile decides: 80 against 57); 128 queries where they make one (512 x 64 behind 1024 cached: 38 against 50 with 64); below that 64 queries with four key
