@@ -46,13 +46,13 @@ __global__ __launch_bounds__(PM_GEMV_BLOCK, 4) void gemv_q_kernel(GemvP p) {
     extern __shared__ __attribute__((aligned(16))) char smem[];
     __shared__ double nred[PM_GEMV_NW];
 #else
-__global__ __launch_bounds__(PM_GEMV_BLOCK, 4) void gemv_q_kernel(const float * xf, const float * norm_w, const uint8_t * W0, const uint8_t * W0b, long row_stride0,
-                                                                  int K, int xmode, int N0, int U0, GemvP p_in) {
+__global__ __launch_bounds__(PM_GEMV_BLOCK, 4) void gemv_q_kernel(const float * xf, const float * norm_w, const uint8_t * W0, const uint8_t * W0b, int row_stride0,
+                                                                  uint32_t K_xmode /*xmode << 28 | K*/, int U0, int each0, int rest0, uint32_t inv, GemvP p_in) {
     extern __shared__ __attribute__((aligned(16))) char smem[];
     __shared__ double nred[PM_GEMV_NW];
     GemvP p = p_in;
-    p.xf = xf; p.norm_w = norm_w; p.K = K; p.xmode = xmode;
-    p.job[0].W = W0; p.job[0].W2 = W0b; p.job[0].row_stride = row_stride0; p.job[0].N = N0; p.job[0].U = U0;
+    p.xf = xf; p.norm_w = norm_w; p.K = (int) (K_xmode & 0x0fffffffu); p.xmode = (int) (K_xmode >> 28); p.inv = inv;
+    p.job[0].W = W0; p.job[0].W2 = W0b; p.job[0].row_stride = row_stride0; p.job[0].U = U0; p.job[0].each = each0; p.job[0].rest = rest0;
 #endif
     if constexpr (XM >= 0) p.xmode = XM;
     if constexpr (HOT) {
@@ -63,7 +63,7 @@ __global__ __launch_bounds__(PM_GEMV_BLOCK, 4) void gemv_q_kernel(const float * 
             p.job[0].role = 1; p.job[1].role = 2; p.job[2].role = 3;                    // wq, wk, wv in this order (no TA-first swap happened)
             p.job[0].is_b = 0; p.job[1].is_b = 0; p.job[2].is_b = TA != TB ? 1 : 0;     // Q4_K_M: wq / wk of the first type, wv of the second (or all of one)
             p.job[0].split = 0; p.job[0].resid = nullptr; p.job[1].resid = nullptr; p.job[2].resid = nullptr;
-        } else { p.job[1].N = 0; p.job[2].N = 0; p.job[0].split = 0; p.job[0].is_b = 0; p.job[0].role = 0; }
+        } else { p.job[1].N = p.job[1].each = p.job[1].rest = 0; p.job[2].N = p.job[2].each = p.job[2].rest = 0; p.job[0].split = 0; p.job[0].is_b = 0; p.job[0].role = 0; }
         if constexpr (PAIR) p.job[0].resid = nullptr;
         if constexpr (!PAIR && !EPI) __builtin_assume(p.job[0].resid != nullptr);     // wo / ffn_down: always + residual
     }
@@ -78,7 +78,8 @@ int launch_types(const GemvP & p_in, bool pair, int grid, size_t lds, bool dbg, 
 #ifdef PM_NO_PRELOAD_ARGS
         hipLaunchKernelGGL(kern, dim3(grid), dim3(PM_GEMV_BLOCK), lds, st, p);
 #else
-        hipLaunchKernelGGL(kern, dim3(grid), dim3(PM_GEMV_BLOCK), lds, st, p.xf, p.norm_w, p.job[0].W, p.job[0].W2, p.job[0].row_stride, p.K, p.xmode, p.job[0].N, p.job[0].U, p);
+        hipLaunchKernelGGL(kern, dim3(grid), dim3(PM_GEMV_BLOCK), lds, st, p.xf, p.norm_w, p.job[0].W, p.job[0].W2, (int) p.job[0].row_stride, (uint32_t) p.K | (uint32_t) p.xmode << 28, p.job[0].U, p.job[0].each,
+                           p.job[0].rest, p.inv, p);
 #endif
     };
     const bool ss = p.ss_out != nullptr || p.xmode == 3;          // producer or consumer of per-workgroup partial sums of squares
@@ -159,7 +160,7 @@ int pmv::gemv_fill(const pm_gemv_fused & a, int grid_fixed, GemvP & p, int & ta_
     }
     // a Q8_0 job needs Q8_0-quantized activations, the K-quants need Q8_K: one prologue serves only one family
     if ((ta == PM_Q8_0) != (tb == PM_Q8_0)) return -1;
-    if (ta == PM_Q8_0 ? a.K % 32 : a.K % 256) return -2;
+    if ((ta == PM_Q8_0 ? a.K % 32 : a.K % 256) || a.K >= 1 << 28) return -2;
     if (pair && ta != tb) return -1;
     if (ta != tb) {
         if (ta != PM_Q4_K) { const int t = ta; ta = tb; tb = t; }     // canonical order: Q4_K first
@@ -172,12 +173,15 @@ int pmv::gemv_fill(const pm_gemv_fused & a, int grid_fixed, GemvP & p, int & ta_
     int rows_cap = PM_MAX_ROWS_PER_WG;
     if (grid_fixed > 0) rows_cap = (int) ((tot_rows + grid - 1) / grid + 3 > PM_MAX_ROWS_PER_WG ? (tot_rows + grid - 1) / grid + 4 : PM_MAX_ROWS_PER_WG);
     else while ((tot_rows + grid - 1) / grid + 3 > PM_MAX_ROWS_PER_WG) grid *= 2;
+    // (job_slice is exact for a power of two, and for any other number below 2^(32 / 3))
+    if ((int64_t) grid * grid * grid >= (int64_t) 1 << 32) while (grid & (grid - 1)) grid += grid & -grid;
+    p.inv = (uint32_t) ((((uint64_t) 1 << 32) + grid - 1) / grid);
     for (int j = 0; j < 3; ++j) {
         GemvJob & g = p.job[j];
         if (j >= a.njobs) { g.N = 0; continue; }
         const pm_gemv_job & s = a.job[j];
         g.W = (const uint8_t *) s.W; g.W2 = (const uint8_t *) s.W2; g.y = s.y; g.bias = s.bias; g.resid = s.resid;
-        g.N = s.N; g.is_b = (s.type != ta); g.U = a.K / nv_of(s.type);
+        g.N = s.N; g.each = s.N / grid; g.rest = s.N % grid; g.is_b = (s.type != ta); g.U = a.K / nv_of(s.type);
         g.row_stride = (long) pm_weight_row_stride(s.type, a.K);
         g.role = 0; g.split = 0;
         if (a.epi) {

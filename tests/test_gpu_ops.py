@@ -174,6 +174,22 @@ def test_gemv_integer_partials_bitexact_and_float_close(P, oracle, t, K, N):
         assert abs(y[r] - want) <= 4e-6 * mag + 1e-30, (TYPE_NAMES[t], K, r, y[r], want)
 
 
+@pytest.mark.parametrize("t", [Q4_K, Q6_K, Q8_0])
+def test_gemv_rows_whatever_the_slices(P, t):
+    """A row's product is the same bits whatever the number of rows, i.e. the slice that it is in: fewer rows than workgroups, whole slices, slices of unequal length, more rows than 256 workgroups
+    take (one matrix, and pairs)."""
+    K, most, rng = 256, 131077, np.random.default_rng(55)
+    b = rand_blocks(t, 4099, K, rng).reshape(4099, -1)
+    blocks = np.concatenate([b] * (most // 4099 + 1))[:most]
+    x = _dev(P, rng.normal(0, 1, (1, K)).astype(np.float32))
+    w = lambda n, at=0: P.upload_weight(t, np.ascontiguousarray(blocks[at:at + n]).reshape(-1), K, n)
+    y, pair = P.mul_mat_vec(w(most), x=x), P.mul_mat_vec(w(most), x=x, w2=w(most))
+    assert P.torch.equal(y[:, 4099:2 * 4099], y[:, :4099]) and P.torch.equal(y[:, 31 * 4099:], y[:, :most - 31 * 4099])
+    for n in (1, 3, 255, 256, 257, 511, 1000, 4098):
+        assert P.torch.equal(P.mul_mat_vec(w(n, 77), x=x), y[:, 77:77 + n]), n
+        assert P.torch.equal(P.mul_mat_vec(w(n, 77), x=x, w2=w(n, 77)), pair[:, 77:77 + n]), n
+
+
 @pytest.mark.parametrize("C", [2, 3, 4, 5, 7, 8])       # column slots per launch group (mmvq_cols.hip): 2, 4 (one idle), 4, 4+1, 4+4 (one idle), 8; pairs: 2 per launch
 @pytest.mark.parametrize("t", QUANT_TYPES)
 def test_gemv_epilogues_and_columns(P, oracle, t, C):
