@@ -99,7 +99,10 @@ __global__ __launch_bounds__(256) void silu_mul_q80_tab_kernel(const float * __r
 // NWV waves per row: 4 for many rows (prompts: small workgroups, several per CU), 16 while every row has a CU to itself - the launch is then ONE latency chain per row: load, reduce,
 // quantize block after block. us with 4 / 16 waves, K = 4096: 101 rows 5.1 / 3.9, 256 rows 5.3 / 4.2, 300 rows 5.4 / 6.0; K = 8192: 101 rows 7.9 / 4.9, 256 rows 8.2 / 5.4, 512 rows 9.3 / 8.5,
 // 700 rows 11.1 / 11.4. (8 rows 3.8 -> 3.6 with the sum by DPP and the weights asked for with the row.)
-template <int NWV>
+// SPLIT: two workgroups to a row of 17 .. 32 blocks, each adds the whole row up (the same sum) and writes one half of it. Two blocks one after the other in every wave, four waves on a SIMD, were
+// 2.0 of a launch's 3.9 us (stamps, 8 rows of 8192): three layers of the 70B shape at 8 tokens, six such launches, 392 -> 388 us. (One block in every wave, 1.25 of 3.1, in two or four workgroups: no
+// change. A workgroup's share by gridDim.y and a division: 0.6 us more on every launch, the grid's size is another load.)
+template <int NWV, bool SPLIT = false>
 __global__ __launch_bounds__(64 * NWV) void rmsnorm_q8k_kernel(const float * __restrict__ x, const float * __restrict__ w,
                                                           float * __restrict__ ynorm, uint8_t * __restrict__ yq,
                                                           int K, float eps, size_t yq_row_bytes, _Float16 * __restrict__ yh, pm_q8k_tables tb, pm_q8k_wide wd) {
@@ -159,11 +162,13 @@ __global__ __launch_bounds__(64 * NWV) void rmsnorm_q8k_kernel(const float * __r
     };
     if (held) {
 #pragma unroll
-        for (int i = 0; i < HOLD; ++i) if (wv + NWV * i < nblk) emit(f[i], wv + NWV * i, WT ? &wt[i] : nullptr);
+        for (int i = 0; i < HOLD; ++i) if ((!SPLIT || i == (int) blockIdx.y) && wv + NWV * i < nblk) emit(f[i], wv + NWV * i, WT ? &wt[i] : nullptr);
     } else {
         for (int blk = wv; blk < nblk; blk += NWV) emit(((const float4 *) (xr + (size_t) blk * PM_QK_K))[lane], blk);
     }
 }
+
+static bool norm_split(int K, int rows) { return K > 16 * PM_QK_K && K <= 32 * PM_QK_K && 2 * rows <= pm_device_cus(); }
 
 // ---- host launchers -------------------------------------------------------------------------------
 void pm_launch_quantize_q8k(const float * x, void * y, int K, int rows, hipStream_t st, pm_q8k_tables tab) {
@@ -191,10 +196,12 @@ void pm_launch_quantize_q80(const float * x, void * y, int K, int rows, hipStrea
                        x, (uint8_t *) y, K, rows, pm_q80_row_bytes(K));
 }
 void pm_launch_rmsnorm_q8k(const float * x, const float * w, float * ynorm, void * yq, int K, int rows, float eps, hipStream_t st, void * ynorm_f16, pm_q8k_tables tab) {
-    if (rows <= pm_device_cus()) hipLaunchKernelGGL(rmsnorm_q8k_kernel<16>, dim3(rows), dim3(1024), 0, st, x, w, ynorm, (uint8_t *) yq, K, eps, pm_q8k_row_bytes(K), (_Float16 *) ynorm_f16, tab, pm_q8k_wide());
+    if (norm_split(K, rows)) hipLaunchKernelGGL((rmsnorm_q8k_kernel<16, true>), dim3(rows, 2), dim3(1024), 0, st, x, w, ynorm, (uint8_t *) yq, K, eps, pm_q8k_row_bytes(K), (_Float16 *) ynorm_f16, tab, pm_q8k_wide());
+    else if (rows <= pm_device_cus()) hipLaunchKernelGGL(rmsnorm_q8k_kernel<16>, dim3(rows), dim3(1024), 0, st, x, w, ynorm, (uint8_t *) yq, K, eps, pm_q8k_row_bytes(K), (_Float16 *) ynorm_f16, tab, pm_q8k_wide());
     else            hipLaunchKernelGGL(rmsnorm_q8k_kernel<4>, dim3(rows), dim3(256), 0, st, x, w, ynorm, (uint8_t *) yq, K, eps, pm_q8k_row_bytes(K), (_Float16 *) ynorm_f16, tab, pm_q8k_wide());
 }
 void pm_launch_rmsnorm_wide(const float * x, const float * w, const pm_q8k_wide & y, int K, int rows, float eps, hipStream_t st) {
-    if (rows <= pm_device_cus()) hipLaunchKernelGGL(rmsnorm_q8k_kernel<16>, dim3(rows), dim3(1024), 0, st, x, w, (float *) nullptr, (uint8_t *) nullptr, K, eps, 0, (_Float16 *) nullptr, pm_q8k_tables(), y);
+    if (norm_split(K, rows)) hipLaunchKernelGGL((rmsnorm_q8k_kernel<16, true>), dim3(rows, 2), dim3(1024), 0, st, x, w, (float *) nullptr, (uint8_t *) nullptr, K, eps, 0, (_Float16 *) nullptr, pm_q8k_tables(), y);
+    else if (rows <= pm_device_cus()) hipLaunchKernelGGL(rmsnorm_q8k_kernel<16>, dim3(rows), dim3(1024), 0, st, x, w, (float *) nullptr, (uint8_t *) nullptr, K, eps, 0, (_Float16 *) nullptr, pm_q8k_tables(), y);
     else             hipLaunchKernelGGL(rmsnorm_q8k_kernel<4>, dim3(rows), dim3(256), 0, st, x, w, (float *) nullptr, (uint8_t *) nullptr, K, eps, 0, (_Float16 *) nullptr, pm_q8k_tables(), y);
 }

@@ -432,6 +432,17 @@ def test_rms_norm_matches_oracle(P, oracle):
         assert np.abs(y2.view(np.int32).astype(np.int64) - oracle.rms_norm(x, None, eps).view(np.int32).astype(np.int64)).max() <= 1
 
 
+@pytest.mark.parametrize("K", [4352, 5120, 8192])
+def test_rms_norm_rows_of_two_workgroups(P, K):
+    """Rows of 17 .. 32 blocks, two workgroups each up to 128 of them and one beyond: the same bits, f32 and Q8_K."""
+    rng = np.random.default_rng(K)
+    x, w = _dev(P, rng.normal(0, 2, (129, K)).astype(np.float32)), _dev(P, (1 + rng.normal(0, 0.02, K)).astype(np.float32))
+    y, yq = P.rms_norm(x, w, 1e-5, want_q8=True)
+    for rows in (1, 128):
+        a, aq = P.rms_norm(x[:rows], w, 1e-5, want_q8=True)
+        assert P.torch.equal(a, y[:rows]) and P.torch.equal(aq, yq[:aq.numel()]), rows
+
+
 def test_gemv_full_size_linearity(P):
     """BASELINE-size property test (no oracle at this size): W.(a) + W.(b) == W.(a+b) is NOT exact after
     activation quantization, so instead check y(W, x) against dequantize-free structure: scaling x by 2
