@@ -363,14 +363,16 @@ template <typename T, int NT, int RM, int SRC, int EXP> __global__ __launch_boun
 // by the wave that multiplies them (a wave has every 8th 64-k block of all rows: no barrier). TP = 0: they do not fit and ride in the load groups; 16 rows share them, one workgroup
 // per CU with twice the registers. The bias rides there too (loads return in order: one of its own would wait for the weights in flight).
 // Weights from memory, in us before / now: 14336 x 4096 3 tokens 27.9 / 22.5, 6 30.4 / 22.7 (5.2 TB/s); 4096 x 14336 6 tokens 33.2 / 24.3; 32000 x 4096 6 tokens 59 / 45.7 (5.7 TB/s);
-// 28672 x 8192 5 tokens 133 / 77 (6.1 TB/s). Taken back: two sum buffers in turn for one barrier less (spills at RM = 2, 32000 x 2048 25.1 -> 26.6).
-template <int RM, int TP> __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(TP == 0 && RM == 2 ? 2 : 4))) void dense_rows_kernel(SmallP p, int tiles) {
+// 28672 x 8192 5 tokens 133 / 77 (6.1 TB/s). What the first loads need stands first among the arguments (in registers when the launch starts) and the tiles of a
+// workgroup are counted by the host (no division, no grid size from memory): 108 launches of a pass of 6 tokens of 36 layers, 5219 -> 5178 us a pass. Taken back: two sum buffers in turn for one barrier less (spills at RM = 2, 32000 x 2048 25.1 -> 26.6).
+template <int RM, int TP> __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(TP == 0 && RM == 2 ? 2 : 4))) void dense_rows_kernel(const void * W0, const void * act0, int K0, int T0, int lda0, int G, int each, int rest, SmallP p) {
+    p.W = W0; p.act = act0; p.K = K0; p.T = T0; p.lda = lda0;
     constexpr int U = TP ? 8 / RM : 4, NL = U * (RM + (TP ? 0 : 1)) + 1, ROWS = 8 * RM;            // 64-k blocks and loads of a group
     extern __shared__ __attribute__((aligned(16))) char smem[];
     float * red = (float *) smem;                                                                  // [8 waves][RM][16 columns][16 rows]
     const int wave = __builtin_amdgcn_readfirstlane((int) threadIdx.x >> 6), lane = threadIdx.x & 63, lr = lane & 15, g = lane >> 4;
     const int nblk = p.K >> 6, mine = (nblk - wave + 7) >> 3, ng = mine > U ? (mine + U - 1) / U : 1;      // 64-k blocks wave, wave + 8, .. ; load groups per tile
-    const int my_tiles = (tiles - (int) blockIdx.x + (int) gridDim.x - 1) / (int) gridDim.x, total = my_tiles * ng;
+    const int my_tiles = each + ((int) blockIdx.x < rest), total = my_tiles * ng;      // (tiles = each G + rest)
     const uint16_t * W = (const uint16_t *) p.W;
     const uint32_t at = (uint32_t) ((lr >> 3) * 32 + g * 8), tok = (lr & 7) < p.T ? lr & 7 : p.T - 1;
     uint32_t w_off[RM];
@@ -407,7 +409,7 @@ template <int RM, int TP> __global__ __launch_bounds__(512) __attribute__((amdgp
             for (int m = 0; m < RM; ++m) a.w[u][m] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rw, (int) w_off[m], soff, 2));      // (2: streamed past the caches)
         }
         a.bias = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rb, (l_tile * ROWS + o_row) * 4, 0, 0));       // (past n_store, without a bias: 0)
-        if (++l_grp == ng) { l_grp = 0; l_tile += gridDim.x; }
+        if (++l_grp == ng) { l_grp = 0; l_tile += G; }
     };
     Group ga, gb;
     load(ga);
@@ -454,7 +456,7 @@ template <int RM, int TP> __global__ __launch_bounds__(512) __attribute__((amdgp
             for (int w = 0; w < 8; ++w) { const float * q = red + ((w * RM + o_row / 8) * 16 + o_tok) * 16 + o_row % 8; v += q[0]; v += q[8 * 16 + 8]; }
             st_type(p.y, (size_t) o_tok * p.ldy + row, p.y_type, act_apply(p.act_fn, v + bias));
         }
-        c_tile += gridDim.x;
+        c_tile += G;
         __syncthreads();
     };
     if (total == 1) { step(ga); return; }
@@ -470,7 +472,7 @@ template <int RM, int TP> int launch_rows(const SmallP & p, int N, hipStream_t s
     const size_t lds = rows_lds(RM, TP, p.K);
     const int per = (TP == 0 && RM == 2) || lds > 80 * 1024 ? 1 : 2, grid = tiles < per * cus ? tiles : per * cus;
     pm_allow_big_lds((const void *) dense_rows_kernel<RM, TP>, lds);
-    hipLaunchKernelGGL((dense_rows_kernel<RM, TP>), dim3(grid), dim3(512), lds, st, p, tiles);
+    hipLaunchKernelGGL((dense_rows_kernel<RM, TP>), dim3(grid), dim3(512), lds, st, p.W, p.act, p.K, p.T, p.lda, grid, tiles / grid, tiles % grid, p);
     return 0;
 }
 
