@@ -24,11 +24,12 @@ __global__ void fill_kernel(int type, void * dst, int K, long n, int Kp, uint64_
         st_type(dst, (size_t) (i / K) * Kp + i % K, type, mean + amp * ((float) (hash32(seed * 0x9E3779B97F4A7C15ULL + (uint64_t) i) & 0xFFFFFF) / 8388608.0f - 1.0f));
 }
 
-// (NTH: the workgroup's threads, where they are fixed: the waves' sums are then read together. One by one sixteen trips to LDS: a norm of 6 rows of 4096 4.9 us, now 4.7)
+// (NTH: the workgroup's threads, where they are fixed: the waves' sums are then read together, and `red` is this sum's own - no barrier in front of it. One by one sixteen trips to LDS: a norm of
+// 6 rows of 4096 4.9 us, now 4.7)
 template <int NTH = 0> __device__ __forceinline__ float block_sum(float v, float * red) {
     v = wave_sum(v);
-    const int wave = threadIdx.x >> 6, n = blockDim.x >> 6;
-    __syncthreads();
+    const int wave = threadIdx.x >> 6, n = NTH ? NTH / 64 : blockDim.x >> 6;
+    if constexpr (NTH == 0) __syncthreads();
     if ((threadIdx.x & 63) == 0) red[wave] = v;
     __syncthreads();
     float s = 0.0f;
@@ -127,14 +128,24 @@ __global__ void rope_table_kernel(const int32_t * pos, float base, int dims, flo
     }
 }
 
+uint32_t norm_how(int type, const pm_norm_args & q) { return (uint32_t) type | (uint32_t) q.y_type << 7 | (uint32_t) q.parts << 14 | (q.rms ? 1u << 30 : 0u) | (q.b ? 1u << 31 : 0u); }
+__device__ __forceinline__ int norm_take(uint32_t how, const float * w, const float * w2, int width, pm_norm_args & q) {
+    q.w = w; q.w2 = w2; q.width = width; q.y_type = (int) (how >> 7 & 127u); q.parts = (int) (how >> 14 & 0xffffu); q.rms = (int) (how >> 30 & 1u);
+    if (!(how >> 31)) q.b = nullptr;
+    return (int) (how & 127u);
+}
+
 // one row per workgroup. RES: x[row] += norm(y[row]) and out = the sum (or its RMS norm with weight w2) in T; else out[row] = norm(x[rows[row]]) in T. VP > 0: the row and
 // everything that joins it are requested at once, VP values per lane; 0: any width, row in LDS
-template <bool RES, int NTH, int VP> __global__ __launch_bounds__(NTH) void norm_kernel(int type, pm_norm_args q, float * x, const void * y, int ldx, int ldy, const int32_t * rows, void * out,
-                                                                                       int ldo) {
+// What the requests need comes first: these arguments are in registers when the launch starts (norm_how: types, parts, rms and whether there is a bias). A row is a chain of latencies: 6 rows of 4096,
+// 85 such launches of six sequences of the dense design: 5178 -> 5160 us a pass with the barriers that went
+template <bool RES, int NTH, int VP> __global__ __launch_bounds__(NTH) void norm_kernel(float * x, const void * y, const float * w_, const float * w2_, int ldx, int ldy, int width, uint32_t how,
+                                                                                       void * out, pm_norm_args q, const int32_t * rows, int ldo) {
     extern __shared__ __attribute__((aligned(16))) float row[];
-    __shared__ __attribute__((aligned(16))) float red[NTH / 64];
+    __shared__ __attribute__((aligned(16))) float red[3 * (NTH / 64)];
+    const int type = norm_take(how, w_, w2_, width, q);
     constexpr int N = VP ? VP : 1;
-    const int r = blockIdx.x, width = q.width;
+    const int r = blockIdx.x;
     float * xr = x + (size_t) (!RES && rows ? rows[r] : r) * ldx;
     auto value = [&](int c) __attribute__((always_inline)) -> float {        // what is normed
         if (!RES) return ld_g(xr + c);
@@ -186,7 +197,7 @@ template <bool RES, int NTH, int VP> __global__ __launch_bounds__(NTH) void norm
 #pragma unroll
         for (int i = 0; i < N; ++i) { const float d = i * NTH + (int) threadIdx.x < width ? v[i] - mean : 0.0f; s2 = fmaf(d, d, s2); }
     } else for (int c = threadIdx.x; c < width; c += NTH) { const float d = row[c] - mean; s2 = fmaf(d, d, s2); }
-    const float rs = 1.0f / sqrtf(block_sum<NTH>(s2, red) / (float) width + q.eps);
+    const float rs = 1.0f / sqrtf(block_sum<NTH>(s2, red + NTH / 64) / (float) width + q.eps);
     float s3 = 0.0f;
     auto sum = [&](int c, float f, float xo, float wo, float bo) __attribute__((always_inline)) -> float {
         float o = (f - mean) * rs * wo + bo;
@@ -199,7 +210,7 @@ template <bool RES, int NTH, int VP> __global__ __launch_bounds__(NTH) void norm
         for (int i = 0; i < N; ++i) { const int c = i * NTH + threadIdx.x; if (c < width) v[i] = sum(c, v[i], xv[i], wv[i], bv[i]); }
     } else for (int c = threadIdx.x; c < width; c += NTH) row[c] = sum(c, row[c], RES ? xr[c] : 0.0f, q.w[c], q.b ? q.b[c] : 0.0f);
     if (!out) return;
-    const float r2 = RES && q.w2 ? 1.0f / sqrtf(block_sum<NTH>(s3, red) / (float) width + q.eps) : 1.0f;
+    const float r2 = RES && q.w2 ? 1.0f / sqrtf(block_sum<NTH>(s3, red + 2 * (NTH / 64)) / (float) width + q.eps) : 1.0f;
     if (VP) {
 #pragma unroll
         for (int i = 0; i < N; ++i) { const int c = i * NTH + threadIdx.x; if (c < width) st_type(out, (size_t) r * ldo + c, type, v[i] * (r2 * w2v[i])); }
@@ -207,9 +218,10 @@ template <bool RES, int NTH, int VP> __global__ __launch_bounds__(NTH) void norm
 }
 
 // x[row] += norm(y[row]), out = the sum or its RMS norm with weight w2, four consecutive columns per thread and round: rows that are padded to multiples of 4
-template <int NTH, int VP> __global__ __launch_bounds__(NTH) void norm4_kernel(int type, pm_norm_args q, float * x, const void * y, int ldx, int ldy, void * out, int ldo) {
-    __shared__ __attribute__((aligned(16))) float red[NTH / 64];
-    const int r = blockIdx.x, width = q.width;
+template <int NTH, int VP> __global__ __launch_bounds__(NTH) void norm4_kernel(float * x, const void * y, const float * w_, const float * w2_, int ldx, int ldy, int width, uint32_t how, void * out, pm_norm_args q, int ldo) {
+    __shared__ __attribute__((aligned(16))) float red[3 * (NTH / 64)];
+    const int type = norm_take(how, w_, w2_, width, q);
+    const int r = blockIdx.x;
     float * xr = x + (size_t) r * ldx;
     const int parts = q.parts ? q.parts : 1;
     f32x4 v[VP], xv[VP];
@@ -238,7 +250,7 @@ template <int NTH, int VP> __global__ __launch_bounds__(NTH) void norm4_kernel(i
     for (int i = 0; i < VP; ++i)
 #pragma unroll
         for (int e = 0; e < 4; ++e) { const float d = (i * NTH + (int) threadIdx.x) * 4 + e < width ? v[i][e] - mean : 0.0f; s2 = fmaf(d, d, s2); }
-    const float rs = 1.0f / sqrtf(block_sum<NTH>(s2, red) / (float) width + q.eps);
+    const float rs = 1.0f / sqrtf(block_sum<NTH>(s2, red + NTH / 64) / (float) width + q.eps);
     float s3 = 0.0f;
 #pragma unroll
     for (int i = 0; i < VP; ++i) {
@@ -251,7 +263,7 @@ template <int NTH, int VP> __global__ __launch_bounds__(NTH) void norm4_kernel(i
         for (int e = 0; e < 4; ++e) { const float o = xv[i][e] + ((v[i][e] - mean) * rs * w[e] + bias[e]); v[i][e] = c + e < width ? o : 0.0f; s3 = fmaf(v[i][e], v[i][e], s3); }
         *(PM_G f32x4 *) (xr + c) = v[i];
     }
-    const float r2 = q.w2 ? 1.0f / sqrtf(block_sum<NTH>(s3, red) / (float) width + q.eps) : 1.0f;
+    const float r2 = q.w2 ? 1.0f / sqrtf(block_sum<NTH>(s3, red + 2 * (NTH / 64)) / (float) width + q.eps) : 1.0f;
 #pragma unroll
     for (int i = 0; i < VP; ++i) {
         const int c = (i * NTH + threadIdx.x) * 4;
@@ -314,7 +326,7 @@ template <bool RES> static void launch_norm(int type, const pm_norm_args & q, fl
                                             hipStream_t st) {
     auto go = [&](auto kern, int threads, size_t lds) {
         pm_allow_big_lds((const void *) kern, lds);
-        hipLaunchKernelGGL(kern, dim3(n_rows), dim3(threads), lds, st, type, q, x, y, ldx, ldy, rows, out, ldo);
+        hipLaunchKernelGGL(kern, dim3(n_rows), dim3(threads), lds, st, x, y, q.w, q.w2, ldx, ldy, q.width, norm_how(type, q), out, q, rows, ldo);
     };
     if (q.width <= 1024) go(norm_kernel<RES, 256, 4>, 256, 0);
     else if (q.width <= 4096 && n_rows > 512) go(norm_kernel<RES, 256, 16>, 256, 0);
@@ -325,7 +337,7 @@ template <bool RES> static void launch_norm(int type, const pm_norm_args & q, fl
 }
 void pm_launch_add_norm(int type, const pm_norm_args & q, float * x, const void * y, int ldx, int ldy, int n_rows, void * out, int ldo, hipStream_t st) {
     if (q.padded && out && n_rows > 16 && q.width <= 8192 && ldx % 4 == 0 && ldy % 4 == 0 && ldo % 4 == 0) {
-        auto go = [&](auto kern, int threads) { hipLaunchKernelGGL(kern, dim3(n_rows), dim3(threads), 0, st, type, q, x, y, ldx, ldy, out, ldo); };
+        auto go = [&](auto kern, int threads) { hipLaunchKernelGGL(kern, dim3(n_rows), dim3(threads), 0, st, x, y, q.w, q.w2, ldx, ldy, q.width, norm_how(type, q), out, q, ldo); };
         if (q.width <= 1024) go(norm4_kernel<256, 1>, 256);
         else if (q.width <= 2048) go(norm4_kernel<256, 2>, 256);
         else if (q.width <= 4096) go(norm4_kernel<256, 4>, 256);
