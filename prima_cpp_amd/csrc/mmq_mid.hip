@@ -615,15 +615,18 @@ __device__ __forceinline__ void mmq_mid_rows(const RowsP & p, const RowsJob & jo
     else mmq_mid_body<TYPE, NV, EPI, false>(p, job, r0, r1, groups > 1 ? 1 : 0, ji, smem);
 }
 
-// (TA: the type of all jobs but the last, TB: of the last one; first1, first2: first workgroups of the second and third job)
+// (TA: the type of all jobs but the last, TB: of the last one; the leading arguments: pm_rows_args)
 template <int TA, int TB, int NV, bool EPI>
-__global__ __launch_bounds__(NT, 3) void mmq_mid_kernel(int first1, int first2, RowsP p) {
+__global__ __launch_bounds__(NT, 3) void mmq_mid_kernel(const uint8_t * W0, const uint8_t * W1, const uint8_t * W2, const uint8_t * qT, uint32_t first, uint32_t rows0, uint32_t rows1, uint32_t rows2, int K,
+                                                        uint32_t tokens, RowsP args) {
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
-    const int b = (int) blockIdx.x, ji = (b >= first1) + (b >= first2);
-    const RowsJob job = p.job[ji];
-    const int w = b - (ji == 0 ? 0 : ji == 1 ? first1 : first2);
-    if (TA == TB || ji < p.njobs - 1) mmq_mid_rows<TA, NV, EPI>(p, job, w, ji, smem);
-    else mmq_mid_rows<TB, NV, EPI>(p, job, w, ji, smem);
+    const RowsStart s = pm_rows_start(W0, W1, W2, first, rows0, rows1, rows2, (int) blockIdx.x);
+    RowsP p = args;
+    pm_rows_take(p, qT, K, tokens);
+    RowsJob job = args.job[s.ji];
+    job.W = s.W; job.each = s.each; job.more = s.more;
+    if (TA == TB || s.ji < p.njobs - 1) mmq_mid_rows<TA, NV, EPI>(p, job, s.w, s.ji, smem);
+    else mmq_mid_rows<TB, NV, EPI>(p, job, s.w, s.ji, smem);
 }
 
 template <int TYPE> size_t lds_of(int nv) {
@@ -664,10 +667,12 @@ int pm_launch_mmq_mid(RowsP p, const int * types, hipStream_t st) {
         b.each = b.N / unit / nw[j]; b.more = b.N / unit % nw[j];
     }
     const int nv = p.T <= 8 ? 4 : p.T <= 16 ? 8 : p.T <= 24 ? 12 : 16;
+    if (!pm_rows_fit(p)) return -5;
     const size_t lds = std::max(lds_of(ta, nv), lds_of(tb, nv));
     auto go = [&](auto kern) {
         pm_allow_big_lds((const void *) kern, lds);
-        hipLaunchKernelGGL(kern, dim3(at), dim3(NT), lds, st, first[1], first[2], p);
+        const RowsArgs a = pm_rows_args(p, first[1], first[2]);
+        hipLaunchKernelGGL(kern, dim3(at), dim3(NT), lds, st, p.job[0].W, p.job[1].W, p.job[2].W, p.qT, a.first, a.rows[0], a.rows[1], a.rows[2], p.K, a.tokens, p);
         return 0;
     };
 #define PM_MID_V(TA_, TB_, E_) { return nv == 4 ? go(mmq_mid_kernel<TA_, TB_, 4, E_>) : nv == 8 ? go(mmq_mid_kernel<TA_, TB_, 8, E_>) : nv == 12 ? go(mmq_mid_kernel<TA_, TB_, 12, E_>) : go(mmq_mid_kernel<TA_, TB_, 16, E_>); }

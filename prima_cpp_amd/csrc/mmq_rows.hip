@@ -115,30 +115,37 @@ template <int TYPE> struct ALds {
     static constexpr int Q = 2048, B = TYPE == PM_Q8_0 ? 0 : 256, D = TYPE == PM_Q8_0 ? 256 : 32, ZERO = 2048;
     static size_t bytes(int n) { return ZERO + (size_t) n * (Q + B + D); }     // n super-blocks
 };
-template <int TYPE> __device__ __forceinline__ void stage_a(uint8_t * L, const RowsP & p, int n) {
+// (two parts: the pieces of the first round - all of them up to 32 super-blocks - are asked for in front of the first weights and stored behind those requests: loads return in order, so the
+// store waits for the activations alone. Asked for and stored kind by kind before the first weight was, they were three rounds of latency: ffn_gate | ffn_up of the 8B shape at 8 tokens, this and
+// the arguments in registers, 16.7 us, now 15.3; of the 70B shape 44.9 / 44.5, the 8B head 97.1 / 95.5)
+template <int TYPE> struct StageA { u32x4 q[8], b, d; };
+template <int TYPE> __device__ __forceinline__ u32x4 stage_q(const RowsP & p, int lim, int i) {
+    return ld_c16(p.qT + (size_t) min(i >> 4, lim - 1) * 1024 + (32 * ((i >> 3) & 1) + (i & 7) + p.t_off) * 16);
+}
+__device__ __forceinline__ u32x4 stage_b(const RowsP & p, int n, int i) { return ld_c16(p.bsT + (size_t) min(i >> 4, n - 1) * 1024 + (32 * ((i >> 3) & 1) + (i & 7) + p.t_off) * 16); }
+__device__ __forceinline__ u32x4 stage_d(const RowsP & p, int rows, int i) { return ld_c16(p.dT + (size_t) min(i >> 1, rows - 1) * 32 + 4 * (i & 1) + p.t_off); }
+template <int TYPE> __device__ __forceinline__ void load_stage(StageA<TYPE> & a, const RowsP & p, int n) {
+    const int tid = threadIdx.x, lim = TYPE == PM_Q8_0 ? p.K / 32 : n * 8;         // sub-blocks / blocks of the row
+#pragma unroll
+    for (int u = 0; u < 8; ++u) a.q[u] = stage_q<TYPE>(p, lim, min(tid + u * NT, n * 128 - 1));
+    if constexpr (TYPE != PM_Q8_0) a.b = stage_b(p, n, tid);
+    a.d = stage_d(p, TYPE == PM_Q8_0 ? lim : n, tid);
+}
+template <int TYPE> __device__ __forceinline__ void store_stage(uint8_t * L, const StageA<TYPE> & a, const RowsP & p, int n) {
     typedef ALds<TYPE> S;
     const int tid = threadIdx.x;
     const u32x4 z = {0, 0, 0, 0};
-    const int lim = TYPE == PM_Q8_0 ? p.K / 32 : n * 8;                // sub-blocks / blocks of the row
+    const int lim = TYPE == PM_Q8_0 ? p.K / 32 : n * 8, rows = TYPE == PM_Q8_0 ? lim : n;
+    uint8_t * const Lq = L + S::ZERO, * const Lb = Lq + (size_t) n * S::Q, * const Ld = Lb + (size_t) n * S::B;
     for (int i = tid; i < S::ZERO / 16; i += NT) *(u32x4 *) (L + i * 16) = z;
-    L += S::ZERO;
-    for (int i0 = tid; i0 < n * 128; i0 += 8 * NT) {
-        u32x4 v[8];
 #pragma unroll
-        for (int u = 0; u < 8; ++u) {
-            const int i = i0 + u * NT, t = i & 7, half = (i >> 3) & 1, sub = i >> 4;
-            v[u] = sub < lim ? ld_c16(p.qT + (size_t) sub * 1024 + (32 * half + t + p.t_off) * 16) : z;
-        }
-#pragma unroll
-        for (int u = 0; u < 8; ++u) { const int i = i0 + u * NT; if (i < n * 128) *(u32x4 *) (L + (size_t) i * 16) = v[u]; }
-    }
-    L += (size_t) n * S::Q;
-    if constexpr (TYPE != PM_Q8_0) {
-        for (int i = tid; i < n * 16; i += NT) *(u32x4 *) (L + i * 16) = ld_c16(p.bsT + (size_t) (i >> 4) * 1024 + (32 * ((i >> 3) & 1) + (i & 7) + p.t_off) * 16);
-        L += (size_t) n * S::B;
-    }
-    const int rows = TYPE == PM_Q8_0 ? lim : n;
-    for (int i = tid; i < n * S::D / 16; i += NT) *(u32x4 *) (L + i * 16) = (i >> 1) < rows ? ld_c16(p.dT + (size_t) (i >> 1) * 32 + 4 * (i & 1) + p.t_off) : z;
+    for (int u = 0; u < 8; ++u) { const int i = tid + u * NT; if (i < n * 128) *(u32x4 *) (Lq + (size_t) i * 16) = (i >> 4) < lim ? a.q[u] : z; }
+    if constexpr (TYPE != PM_Q8_0) if (tid < n * 16) *(u32x4 *) (Lb + tid * 16) = a.b;
+    if (tid < n * S::D / 16) *(u32x4 *) (Ld + tid * 16) = (tid >> 1) < rows ? a.d : z;
+    // longer rows: the rest
+    for (int i = tid + 8 * NT; i < n * 128; i += NT) *(u32x4 *) (Lq + (size_t) i * 16) = (i >> 4) < lim ? stage_q<TYPE>(p, lim, i) : z;
+    if constexpr (TYPE != PM_Q8_0) for (int i = tid + NT; i < n * 16; i += NT) *(u32x4 *) (Lb + i * 16) = stage_b(p, n, i);
+    for (int i = tid + NT; i < n * S::D / 16; i += NT) *(u32x4 *) (Ld + i * 16) = (i >> 1) < rows ? stage_d(p, rows, i) : z;
 }
 struct ALane { uint32_t q, qi, b, bi, d; };                        // the lane's addresses in it, and what a super-block adds to them (0: an empty row)
 template <int TYPE> __device__ __forceinline__ ALane lane_a(int n, int lr, int kg) {
@@ -439,12 +446,14 @@ __device__ __forceinline__ void rows_body(const RowsP & p, const RowsJob & job, 
     constexpr int NQ = Q80 ? 4 : 8;
     rows_of(0);
     load_scales(0, 0);
-    if constexpr (AL) stage_a<TYPE>(act, p, na);
+    StageA<TYPE> sa;
+    if constexpr (AL) { load_stage<TYPE>(sa, p, na); __builtin_amdgcn_sched_barrier(0); }
 #pragma unroll
     for (int d = 0; d < D; ++d) {
 #pragma unroll
         for (int r = 0; r < R; ++r) W[d][r].load(ws, off[r], kg, wave + KW * wn.it);
         advance();
+        __builtin_amdgcn_sched_barrier(0);
         if constexpr (!AL) if (d == 0) {
 #pragma unroll
             for (int g = 0; g < NG; ++g) {
@@ -455,6 +464,7 @@ __device__ __forceinline__ void rows_body(const RowsP & p, const RowsJob & job, 
         }
     }
     load_end(0);
+    if constexpr (AL) { __builtin_amdgcn_sched_barrier(0); store_stage<TYPE>(act, sa, p, na); }
     store_scales(0);
     __syncthreads();
     ALane al;
@@ -565,15 +575,18 @@ __device__ __forceinline__ void rows_body(const RowsP & p, const RowsJob & job, 
     }
 }
 
-// TA: the type of all jobs but the last, TB: of the last one. first1, first2: first workgroups of the second and third job (in registers when the kernel starts)
+// TA: the type of all jobs but the last, TB: of the last one. What the first loads need leads the arguments and is in registers when the kernel starts (pm_rows_args)
 template <int TA, int TB, int NG, int R, int D, bool AL, bool EPI>
-__global__ __launch_bounds__(NT, 2) void mmq_rows_kernel(int first1, int first2, RowsP p) {
+__global__ __launch_bounds__(NT, 2) void mmq_rows_kernel(const uint8_t * W0, const uint8_t * W1, const uint8_t * W2, const uint8_t * qT, uint32_t first, uint32_t rows0, uint32_t rows1, uint32_t rows2, int K,
+                                                         uint32_t tokens, RowsP args) {
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
-    const int b = (int) blockIdx.x, ji = (b >= first1) + (b >= first2);
-    const RowsJob job = p.job[ji];
-    const int w = b - (ji == 0 ? 0 : ji == 1 ? first1 : first2);
-    if (TA == TB || ji < p.njobs - 1) rows_body<TA, NG, R, D, AL, EPI>(p, job, w, ji, smem);
-    else rows_body<TB, NG, R, D, AL, EPI>(p, job, w, ji, smem);
+    const RowsStart s = pm_rows_start(W0, W1, W2, first, rows0, rows1, rows2, (int) blockIdx.x);
+    RowsP p = args;
+    pm_rows_take(p, qT, K, tokens);
+    RowsJob job = args.job[s.ji];
+    job.W = s.W; job.each = s.each; job.more = s.more;
+    if (TA == TB || s.ji < p.njobs - 1) rows_body<TA, NG, R, D, AL, EPI>(p, job, s.w, s.ji, smem);
+    else rows_body<TB, NG, R, D, AL, EPI>(p, job, s.w, s.ji, smem);
 }
 template <int TYPE> size_t lds_of(int NG, int R, bool AL, int K) {
     const int n = TYPE == PM_Q8_0 ? (K / 32 + 7) / 8 : K / 256;
@@ -644,6 +657,7 @@ int pm_launch_mmq_rows(RowsP p, const int * types, hipStream_t st) {
         const int groups = (unit * (b.each + (b.more != 0)) + 15) / 16;
         if (groups > big) big = groups;
     }
+    if (!pm_rows_fit(p)) return -5;
     // up to 48 rows a workgroup: one pass, activations by the wave that multiplies them; more: passes of 64 rows over activations in LDS where they fit (K up to 9 k: two thirds of it), else
     // again passes of 48
     const auto lds = [&](int g, int r, bool al) { return std::max(lds_of(ta, g, r, al, p.K), lds_of(tb, g, r, al, p.K)); };
@@ -651,7 +665,8 @@ int pm_launch_mmq_rows(RowsP p, const int * types, hipStream_t st) {
     const bool al = ng == 1 && big > 3 && lds(1, 4, true) <= LDS_MOST, deep = p.K > 4096;
     auto go = [&](auto kern, size_t bytes) {
         pm_allow_big_lds((const void *) kern, bytes);
-        hipLaunchKernelGGL(kern, dim3(at), dim3(NT), bytes, st, first[1], first[2], p);
+        const RowsArgs a = pm_rows_args(p, first[1], first[2]);
+        hipLaunchKernelGGL(kern, dim3(at), dim3(NT), bytes, st, p.job[0].W, p.job[1].W, p.job[2].W, p.qT, a.first, a.rows[0], a.rows[1], a.rows[2], p.K, a.tokens, p);
         return 0;
     };
 #define PM_ROWS_GO(TA_, TB_, G_, R_, D_, AL_, E_) go(mmq_rows_kernel<TA_, TB_, G_, R_, D_, AL_, E_>, lds(G_, R_, AL_))

@@ -1637,6 +1637,22 @@ def test_small_batch_rows_kernel_at_its_edges(P, oracle, t):
             assert np.array_equal(one[0], y[T - 1]), (K, N, T)
 
 
+@pytest.mark.parametrize("t", [Q4_K, Q6_K, Q8_0])
+def test_small_batch_activations_staged_behind_weight_requests(P, oracle, t):
+    """mmq_rows.hip with activations in LDS: 32 super-blocks (all asked for in front of the weights), one more and 36 (the rest by loops behind them), a single pair; the bound of the test above."""
+    rng = np.random.default_rng(7200 + t)
+    tail = 32 if t == Q8_0 else 256
+    for K, N, T in ((8192, 16390, 8), (8192 + tail, 16401, 5), (9216, 33000, 7), (1536 + tail, 50001, 1)):
+        b = rand_blocks(t, N, K, rng)
+        x = rng.normal(0, 1, (T, K)).astype(np.float32)
+        w = P.upload_weight(t, b, K, N)
+        rows = np.unique(np.concatenate([np.arange(70), np.arange(N - 70, N), rng.integers(0, N, 100)]))
+        want = oracle.mul_mat(t, b.reshape(N, b.size // N)[rows].copy(), K, len(rows), x)
+        y = P.mul_mat_small(w, x=_dev(P, x)).cpu().numpy()
+        assert np.isfinite(y).all(), (K, N, T)
+        assert np.allclose(y[:, rows], want, rtol=2e-5, atol=2e-5 * np.sqrt(max(K, 4096) / 4096)), (K, N, T, np.abs(y[:, rows] - want).max())
+
+
 @pytest.mark.parametrize("rows,K", [(65, 4096), (256, 8192), (257, 4096), (256, 12288), (2, 256)])
 def test_rms_norm_of_many_rows(P, oracle, rows, K):
     """16 waves per row up to 256 rows, 4 beyond; rows that fit the registers of either form and rows that do not. The bound of the test of few rows: one unit in the last place (the f64 sum's
