@@ -476,6 +476,162 @@ template <int RM, int TP> int launch_rows(const SmallP & p, int N, hipStream_t s
     return 0;
 }
 
+// The same for the experts' products behind pm_launch_route_stream (up to PM_ROUTE_PAIRS pairs of up to 64 experts): a workgroup keeps its rows and takes the experts blockIdx.y, + ny, .. of those
+// that have pairs, up to 8 of an expert's pairs at a time. One by one (dense_small_kernel), an item's 64 KB of weights were asked for when the item in front was stored: nothing was on its way while a
+// workgroup fetched activations, added up and stored. Here the load groups of all items are one sequence, two of them in flight, and the activations of the next item follow the last products
+// of this one, by DMA into the waves' own LDS. 20 pairs of 32 experts of 2048 x 2048: 22.5 us a launch, now 21.2 (5.4 TB/s), a pass of
+// 5 sequences of such layers 6112 -> 5984.
+// The pairs: a lane per pair, 64 at a time, every wave for itself (no launch that sorts, no barrier). inv: 65536 / experts per token + 1. Sums in dense_small_kernel's order.
+template <int RM> __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void dense_experts_kernel(const void * W0, const void * act0, const int32_t * id, const float * pair_w, int64_t e_stride,
+                                                                                                                    int K, int lda, uint32_t pairs_ny, uint32_t inv, SmallP p) {
+    constexpr int U = 8 / RM, ROWS = 8 * RM, G = PM_ROUTE_PAIRS / 64;
+    extern __shared__ __attribute__((aligned(16))) char smem[];
+    __shared__ int list[8][8];
+    __shared__ float weight[PM_ROUTE_PAIRS];
+    float * red = (float *) smem;                                                                  // [8 waves][RM][16 columns][16 rows]
+    const int wave = __builtin_amdgcn_readfirstlane((int) threadIdx.x >> 6), lane = threadIdx.x & 63, lr = lane & 15, g = lane >> 4, pairs = (int) (pairs_ny & 65535), ny = (int) (pairs_ny >> 16);
+    const int nblk = K >> 6, mine = (nblk - wave + 7) >> 3, ng = mine > U ? (mine + U - 1) / U : 1, r0 = (int) blockIdx.x * ROWS;
+    int pe[G];                                                                                     // the experts of pairs lane, 64 + lane, .. (64: no pair)
+    float pw[G];
+#pragma unroll
+    for (int i = 0; i < G; ++i) { pe[i] = 64; pw[i] = 0.0f; if (i * 64 < pairs && i * 64 + lane < pairs) { pe[i] = ld_g(id + i * 64 + lane); pw[i] = ld_g(pair_w + i * 64 + lane); } }
+    uint32_t has[2] = {0, 0};
+#pragma unroll
+    for (int i = 0; i < G; ++i) if (i * 64 < pairs) { has[0] |= pe[i] < 32 ? 1u << pe[i] : 0u; has[1] |= pe[i] >= 32 && pe[i] < 64 ? 1u << (pe[i] - 32) : 0u; }
+    const uint64_t on = (uint64_t) wave_or(has[1]) << 32 | wave_or(has[0]), below = (1ull << lane) - 1;
+    const int n_on = __popcll(on);
+    if ((int) blockIdx.y >= n_on) return;
+    auto nth = [&](int k) __attribute__((always_inline)) { return (int) __builtin_ctzll(__builtin_amdgcn_ballot_w64((on >> lane & 1) && __popcll(on & below) == k)); };
+    auto pairs_of = [&](int e) __attribute__((always_inline)) {
+        int n = 0;
+#pragma unroll
+        for (int i = 0; i < G; ++i) if (i * 64 < pairs) n += __popcll(__builtin_amdgcn_ballot_w64(pe[i] == e));
+        return n;
+    };
+    const uint32_t at = (uint32_t) ((lr >> 3) * 32 + g * 8);
+    uint32_t w_off[RM];
+#pragma unroll
+    for (int m = 0; m < RM; ++m) w_off[m] = ((uint32_t) (m * 8 + (lr & 7)) * (uint32_t) K + at) * 2;
+    const int o_row = threadIdx.x % ROWS, o_tok = threadIdx.x / ROWS;                              // the element of an item that this thread stores
+    // ---- the weights: the next group to be requested
+    struct Group { u32x4 w[U][RM]; };
+    int l_k = blockIdx.y, l_e = nth(l_k), l_left = (pairs_of(l_e) + 7) >> 3, l_grp = 0;             // (l_left 0: no more)
+    auto load = [&](Group & a) __attribute__((always_inline)) {
+        const uint16_t * at_rows = (const uint16_t *) W0 + (size_t) l_e * e_stride + (size_t) r0 * K;
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            // past the end of a row: out of the bounds of an empty buffer, no traffic
+            const int i = l_grp * U + u, in = i < mine, soff = in ? (wave + i * 8) * 128 : 0;
+            const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc((void *) at_rows, 0, in ? ROWS * K * 2 : 0, 0x00020000);
+#pragma unroll
+            for (int m = 0; m < RM; ++m) a.w[u][m] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rw, (int) w_off[m], soff, 2));      // (2: streamed past the caches)
+        }
+        if (++l_grp < ng) return;
+        l_grp = 0;
+        if (--l_left) return;
+        l_k += ny;
+        if (l_k < n_on) { l_e = nth(l_k); l_left = (pairs_of(l_e) + 7) >> 3; }
+    };
+    // ---- the activations: up to 8 pairs of an expert, this wave's blocks of them: [block][8 pairs][8 pieces of 16 bytes, piece p in place p ^ pair / 2]
+    char * const xs = smem + 8 * RM * 1024 + (size_t) wave * ((nblk + 7) >> 3) * 1024;
+    const uint32_t dst = (uint32_t) (uintptr_t) (__attribute__((address_space(3))) char *) xs;
+    struct Item { int at, here, pair; float w; };                                                   // first sorted pair, pairs; this thread's pair and its weight
+    int a_k = blockIdx.y, a_e = l_e, a_n = pairs_of(a_e), a_t = 0;                                  // the next item (a_n 0: no more)
+    auto fetch = [&]() __attribute__((always_inline)) {
+        Item x;
+        int first = 0, seen = -a_t;
+#pragma unroll
+        for (int i = 0; i < G; ++i) {
+            if (i * 64 >= pairs) break;
+            const uint64_t its = __builtin_amdgcn_ballot_w64(pe[i] == a_e);
+            first += __popcll(__builtin_amdgcn_ballot_w64(pe[i] < a_e));
+            const int place = seen + __popcll(its & below);
+            if ((its >> lane & 1) && place >= 0 && place < 8) list[wave][place] = i * 64 + lane;
+            seen += __popcll(its);
+        }
+        wave_fence();
+        x.here = a_n - a_t < 8 ? a_n - a_t : 8; x.at = first + a_t;
+        const int t = lane >> 3, last = x.here - 1;
+        const uint32_t row = p.in_sorted ? (uint32_t) (x.at + t) : (uint32_t) list[wave][t < last ? t : last] * inv >> 16;
+        x.pair = list[wave][o_tok < last ? o_tok : last]; x.w = weight[x.pair];
+        const uint32_t src = (row * (uint32_t) lda + (uint32_t) (((lane & 7) ^ (t >> 1)) * 8)) * 2 + (uint32_t) wave * 128;
+        wave_fence();
+        for (int i = 0; i < mine; ++i) if (t < x.here) pm_dma16(act0, src + (uint32_t) i * 1024, dst + (uint32_t) i * 1024);
+        a_t += 8;
+        if (a_t >= a_n) {
+            a_k += ny; a_t = 0; a_n = 0;
+            if (a_k < n_on) { a_e = nth(a_k); a_n = pairs_of(a_e); }
+        }
+        return x;
+    };
+#pragma unroll
+    for (int i = 0; i < G; ++i) if (i * 64 < pairs) weight[i * 64 + lane] = pw[i];                  // (every wave the same; each reads what it has written itself)
+    wave_fence();
+    Group ga, gb;
+    load(ga);
+    Item now = fetch(), next = now;
+    bool behind = l_left != 0;                                                                     // a group was asked for behind the item's activations
+    if (behind) load(gb);
+    f32x4 acc[RM];
+#pragma unroll
+    for (int m = 0; m < RM; ++m) acc[m] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    int c_grp = 0;
+    auto step = [&](Group & a) __attribute__((always_inline)) -> bool {                             // the next group; false: it was the last one
+        if (c_grp == 0) {
+            if (behind) asm volatile("s_waitcnt vmcnt(8)" : : : "memory"); else asm volatile("s_waitcnt vmcnt(0)" : : : "memory");
+        }
+        const int tok = (lr & 7) < now.here ? lr & 7 : now.here - 1;
+        const char * x_at = xs + tok * 128 + (((lr >> 3) * 4 + g) ^ (tok >> 1)) * 16;
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int i = c_grp * U + u;
+#pragma unroll
+            for (int m = 0; m < RM; ++m) asm volatile("" : : "v"(a.w[u][m]));
+            if (i >= mine) continue;
+            const u32x4 x = *(const u32x4 *) (x_at + i * 1024);
+#pragma unroll
+            for (int m = 0; m < RM; ++m) acc[m] = Frag<uint16_t>::mma(a.w[u][m], x, acc[m]);
+        }
+        const bool end = ++c_grp == ng, more = a_n != 0;
+        if (end && more) next = fetch();
+        behind = l_left != 0;
+        if (behind) load(a);
+        if (!end) return true;
+        c_grp = 0;
+        // (the wait states between a product and the store that reads it, spelled out as in the kernel above)
+#pragma unroll
+        for (int m = 0; m < RM; ++m) asm volatile("" : "+v"(acc[m]));
+        asm volatile("s_nop 15\n\ts_nop 3");
+#pragma unroll
+        for (int m = 0; m < RM; ++m) asm volatile("" : "+v"(acc[m]));
+#pragma unroll
+        for (int m = 0; m < RM; ++m) { *(f32x4 *) (red + ((wave * RM + m) * 16 + lr) * 16 + g * 4) = acc[m]; acc[m] = f32x4{0.0f, 0.0f, 0.0f, 0.0f}; }
+        __syncthreads();
+        const int row = r0 + o_row;
+        if (o_tok < now.here && row < p.n_store) {
+            float v = 0.0f;
+#pragma unroll
+            for (int w = 0; w < 8; ++w) { const float * q = red + ((w * RM + o_row / 8) * 16 + o_tok) * 16 + o_row % 8; v += q[0]; v += q[8 * 16 + 8]; }
+            v = act_apply(p.act_fn, v);
+            if (p.weigh) v *= now.w;
+            st_type(p.y, (size_t) (p.out_sorted ? now.at + o_tok : now.pair) * p.ldy + row, p.y_type, v);
+        }
+        if (!more) return false;
+        now = next;
+        __syncthreads();
+        return true;
+    };
+    while (step(ga) && step(gb)) {}
+}
+template <int RM> int launch_sorted(const SmallP & p, int N, int experts, hipStream_t st) {
+    const int tiles = N / (8 * RM), y = std::min(experts, (2 * pm_device_cus() + tiles - 1) / tiles);      // (two workgroups per CU: the figures at launch() below)
+    const size_t lds = rows_lds(RM, 8, p.K);
+    pm_allow_big_lds((const void *) dense_experts_kernel<RM>, lds);
+    hipLaunchKernelGGL(dense_experts_kernel<RM>, dim3(tiles, y), dim3(512), lds, st, p.W, p.act, (const int32_t *) p.r.id, (const float *) p.r.w, p.e_stride, p.K, p.lda,
+                       (uint32_t) (p.T * p.r.top) | (uint32_t) y << 16, 65536u / (uint32_t) p.r.top + 1, p);
+    return 0;
+}
+
 // One bf16 matrix per group of rows (attention head) with short rows: NB 64-k blocks, a wave per 16 rows and 16 tokens, everything it needs requested at once and no sums over waves. (Above,
 // eight waves share a row's blocks: of 64 k seven have none. 16384 rows of 64, 5 tokens: 8.4 us, now 3.2 .. 5.0)
 template <int NB> __global__ __launch_bounds__(256) void dense_group_kernel(SmallP p, int rows, int whole) {
@@ -564,6 +720,9 @@ template <typename T> int launch_type(const pm_dense_args & a, const SmallP & p,
 template <typename T, int EXP> int launch_experts(const SmallP & p, int N, int y, hipStream_t st) {
     if constexpr (sizeof(T) == 2) {
         const size_t one = (size_t) p.K * (EXP == CONCAT ? p.r.top : 1) * 2 + 16;
+        // (the same line as below; buffer loads and DMA of 16 bytes want operands that start on 16 bytes, 32-bit offsets)
+        if (EXP == SORTED && !p.r.logits && one * 8 <= LDS_ACT && (((uintptr_t) p.W | (uintptr_t) p.act) & 15) == 0 && p.lda % 8 == 0 && p.e_stride % 8 == 0 && (int64_t) p.T * p.r.top * p.lda < (1 << 30))
+            return rows_per_lane(p.K) == 1 ? launch_sorted<1>(p, N, y, st) : launch_sorted<2>(p, N, y, st);
         if (one * (EXP == SORTED ? 8 : 1) <= LDS_ACT) return rows_per_lane(EXP == CONCAT ? p.K * p.r.top : p.K) == 1 ? launch<T, 1, 1, -1, EXP>(p, N, y, st) : launch<T, 1, 2, -1, EXP>(p, N, y, st);
     }
     return launch<T, 1, 1, 0, EXP>(p, N, y, st);

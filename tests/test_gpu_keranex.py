@@ -209,6 +209,20 @@ def test_experts_in_turn(E, top, ff, width, dtype):
     m.close()
 
 
+@pytest.mark.parametrize("E,top,ff,width", [(6, 4, 4160, 260), (64, 4, 520, 600), (33, 1, 64, 2000), (2, 2, 4600, 130)])
+def test_experts_whose_load_groups_are_one_sequence(E, top, ff, width):
+    """bf16, pairs that the products find for themselves: rows of one more block than the waves share (two load groups for one wave, one for the others), of less blocks than waves and up to the longest
+    that fit; 64 experts, one, 256 pairs; experts of one, eight, nine and of 64 pairs"""
+    c = one(scan(inner=64, mlp=moe(E, top, 1, 1, ff)), width=width, vocab=120)
+    w = silent(weights_for(c, "bfloat16", 9), 0)
+    _, _, m = model("sequence", "bfloat16", c, 9, w, fresh=True, max_tokens=64, n_seq=2, pool_tokens=128)
+    toks = tokens(64, 120, 5)
+    want = P.run(c, w, toks)
+    for n in (5, 8, 9, 23, 64):
+        close(alone(m, toks[:n]), want[:n], "bfloat16")
+    m.close()
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("ff,E,top", [(4700, 3, 2), (1030, 5, 1), (576, 2, 2)])
 def test_wide_experts(ff, E, top, dtype):
