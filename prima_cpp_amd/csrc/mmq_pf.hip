@@ -26,6 +26,7 @@
 #include "pm355_kernels.h"
 #include <stdlib.h>
 #include <stdio.h>
+#include <cmath>
 #include <mutex>
 #include <type_traits>
 
@@ -330,12 +331,12 @@ __device__ __forceinline__ void pf_body(const PfP & p, const PfJob & jb, const i
             // reader (slice 3 of step s + 1 reads the fragments of step s + 2's first slice); the weights are the wave's own.
             if (j == 2 && !(exp & 3)) {
                 constexpr int N8[4] = {3, 3, 3, 2}, N4[4] = {2, 2, 2, 1}, Q8N8[4] = {2, 3, 2, 2}, Q8N4[4] = {1, 2, 1, 1};
-                const int n = Q8 ? (NT == 8 ? Q8N8[sq] : Q8N4[sq]) : NT == 8 ? N8[sq] : N4[sq];
+                const int n = Q8 ? (NT >= 6 ? Q8N8[sq] : Q8N4[sq]) : NT >= 6 ? N8[sq] : N4[sq];
                 if (n == 3) asm volatile("s_waitcnt vmcnt(3)" ::: "memory");
                 else if (n == 2) asm volatile("s_waitcnt vmcnt(2)" ::: "memory");
                 else asm volatile("s_waitcnt vmcnt(1)" ::: "memory");
             }
-            if (NT == 8 || (NT == 4 && (j & 1) == 0) || j == 0) issue_B(4 * b + sq + 2, wr, NT == 8 ? j : NT == 4 ? j >> 1 : 0);
+            if (NT == 8 || (NT == 6 && j < 3) || (NT == 4 && (j & 1) == 0) || j == 0) issue_B(4 * b + sq + 2, wr, NT >= 6 ? j : NT == 4 ? j >> 1 : 0);
             // (Q8_0: the 64-k slot of step s is free once its last slice has been read - behind slice 1 - and takes step s + 2's blocks in slices 2 and 3)
             if (Q8) { if (j >= 2) issue_A(4 * b + sq + 2, sq & 1, j - 2); }
             else if ((sq == 0 || sq == 2) && j >= 1 && j - 1 < NSTREAM) issue_A(2 * b + 1 + (sq >> 1), sq == 0 ? 1 : 0, j - 1);
@@ -1165,7 +1166,7 @@ int pm_gemm_pf_check(int type, int K, int N, int T) {
 // every partial tile through memory: 3 x 320 slabs of 256 KB for the qkv launch, 501 us = 685 TFLOP/s against 406 us = 846.
 void pm_gemm_pf_plan(int tiles, int K, int T, int cus, int force_nt, int force_s, int allow_mixed, pm_gemm_pf_plan_t * out) {
     int nt = T <= 64 ? 2 : T <= 128 ? 4 : 8;
-    if ((force_nt >= 2 && force_nt <= 4) || force_nt == 8) nt = force_nt;
+    if ((force_nt >= 2 && force_nt <= 4) || force_nt == 6 || force_nt == 8) nt = force_nt;
     const int nt_t = (T + 32 * nt - 1) / (32 * nt);
     const long wgs = (long) tiles * nt_t;
     const int nb = (K + 255) / 256;
@@ -1246,6 +1247,17 @@ static int launch_pf(const pm_gemm_pf_job * jobs, int njobs, const void * xh, co
         const auto cost = [&](int nt) { return ((long) tiles * ((T + 32 * nt - 1) / (32 * nt)) * pl.splitk + cus - 1) / cus * (nt + 1); };
         if (cost(3) < cost(4)) pm_gemm_pf_plan(tiles, K, T, cus, 3, pl.splitk, 0, &pl);
     }
+    // Tiles of 192 tokens where their rounds of workgroups cost less than those of 256: mostly 129..192, 257..384 and 513..576 tokens, whose rest of a tile of 256 was products of nothing. The K
+    // split stays, so every sum keeps its order; in place of a split of the last tiles only, whole ones. Both by full rounds and, as a last round that is not full runs faster, by the work in them;
+    // one round of 256-token workgroups that leaves CUs idle may become up to a tenth more work.
+    // us, 256 / 192: 8B shape ffn_gate | ffn_up Q4_K 150 tokens 79 / 66, 300 128 / 104 (512 137 / 160, 1000 284 / 317, 6001 1430 / 1475: not taken), 70B shape 300 454 / 376, 513 664 / 559,
+    // Q6_K ffn_down of 8B 380 85 / 72, Q8_0 ffn_down of 72B 513 371 / 319, wq | wk | wv of 8B 150 42 / 36, 1500 120 / 100, 6001 404 / 374 (a split tail before), wo 3000 137 / 122, 6001 285 / 251
+    if (!mid && !force_nt && !force_s && pl.nt == 8) {
+        const int s6 = pl.full ? 1 : pl.splitk, nb = (K + 255) / 256;
+        const auto work = [&](int nt) { return (double) tiles * ((T + 32 * nt - 1) / (32 * nt)) * s6 / cus; };
+        const double tail = pl.full ? pl.cost / nb : 0.0, r8 = pl.full ? tail : std::ceil(work(8)), w8 = pl.full ? tail : work(8);
+        if (7.0 * std::ceil(work(6)) < 0.97 * 9.0 * r8 && 7.0 * work(6) < (r8 == 1.0 ? 1.1 : 0.97) * 9.0 * w8) pm_gemm_pf_plan(tiles, K, T, cus, 6, s6, 0, &pl);
+    }
     const int nt = pl.nt, S = pl.splitk, full = pl.full, maxL = ((tiles + 7) / 8) * pl.nt_t;
     p.nt_t = pl.nt_t;
     p.splitk = S; p.full = full;
@@ -1306,7 +1318,7 @@ static int launch_pf(const pm_gemm_pf_job * jobs, int njobs, const void * xh, co
         return 0;
     }
 #endif
-#define PF_GO(A, B) (wide ? nt == 4 ? go(gemm_pf_kernel<PM_Q4_K, PM_Q4_K, 4, true, 0, true>, pf_lds_bytes<PM_Q4_K, PM_Q4_K, 4, true, true>()) : nt == 3 ? go(gemm_pf_kernel<PM_Q4_K, PM_Q4_K, 3, true, 0, true>, pf_lds_bytes<PM_Q4_K, PM_Q4_K, 3, true, true>()) : go(gemm_pf_kernel<A, B, 2, true, 0, A != PM_Q8_0>, pf_lds_bytes<A, B, 2, true, A != PM_Q8_0>()) : mid ? nt == 4 ? go(gemm_pf_kernel<A, B, 4, true>, pf_lds_bytes<A, B, 4, true>()) : nt == 3 ? go(gemm_pf_kernel<A, B, 3, true>, pf_lds_bytes<A, B, 3, true>()) : go(gemm_pf_kernel<A, B, 2, true>, pf_lds_bytes<A, B, 2, true>()) : nt == 8 ? go(gemm_pf_kernel<A, B, 8>, pf_lds_bytes<A, B, 8>()) : nt == 4 ? go(gemm_pf_kernel<A, B, 4>, pf_lds_bytes<A, B, 4>()) : go(gemm_pf_kernel<A, B, 2>, pf_lds_bytes<A, B, 2>()))
+#define PF_GO(A, B) (wide ? nt == 4 ? go(gemm_pf_kernel<PM_Q4_K, PM_Q4_K, 4, true, 0, true>, pf_lds_bytes<PM_Q4_K, PM_Q4_K, 4, true, true>()) : nt == 3 ? go(gemm_pf_kernel<PM_Q4_K, PM_Q4_K, 3, true, 0, true>, pf_lds_bytes<PM_Q4_K, PM_Q4_K, 3, true, true>()) : go(gemm_pf_kernel<A, B, 2, true, 0, A != PM_Q8_0>, pf_lds_bytes<A, B, 2, true, A != PM_Q8_0>()) : mid ? nt == 4 ? go(gemm_pf_kernel<A, B, 4, true>, pf_lds_bytes<A, B, 4, true>()) : nt == 3 ? go(gemm_pf_kernel<A, B, 3, true>, pf_lds_bytes<A, B, 3, true>()) : go(gemm_pf_kernel<A, B, 2, true>, pf_lds_bytes<A, B, 2, true>()) : nt == 8 ? go(gemm_pf_kernel<A, B, 8>, pf_lds_bytes<A, B, 8>()) : nt == 6 ? go(gemm_pf_kernel<A, B, 6>, pf_lds_bytes<A, B, 6>()) : nt == 4 ? go(gemm_pf_kernel<A, B, 4>, pf_lds_bytes<A, B, 4>()) : go(gemm_pf_kernel<A, B, 2>, pf_lds_bytes<A, B, 2>()))
     if (ta == tb) { if (ta == PM_Q4_K) PF_GO(PM_Q4_K, PM_Q4_K); else if (ta == PM_Q5_K) PF_GO(PM_Q5_K, PM_Q5_K); else if (ta == PM_Q8_0) PF_GO(PM_Q8_0, PM_Q8_0); else PF_GO(PM_Q6_K, PM_Q6_K); }
     else if (ta == PM_Q8_0 || tb == PM_Q8_0) return -1;      // (Q8_0 only as a launch of its own: ffn_down of the files whose n_ff is no multiple of 256)
     else if (ta == PM_Q4_K && tb == PM_Q5_K) PF_GO(PM_Q4_K, PM_Q5_K);

@@ -957,6 +957,26 @@ def test_prompt_gemm_tiles_of_128_rows(P, oracle, t, K, N, T):
 
 
 @pytest.mark.parametrize("t", QUANT_TYPES)
+@pytest.mark.parametrize("K,N", [(512, 132), (4096, 260), (768, 4100)])
+def test_prompt_tiles_of_192_tokens(P, t, K, N):
+    """Tiles of 192 tokens beside those of 256, at the first and last counts of either: a token's sums are the same bits in a batch of another tile. Slices of K (4096) and none, rows that end
+    inside a wave's, several matrices and pairs."""
+    rng = np.random.default_rng(K + N + t)
+    if t == Q8_0:
+        K += 128
+    w = P.upload_weight(t, rand_blocks(t, N, K, rng, scale=1.0), K, N)
+    v = P.upload_weight(t, rand_blocks(t, N, K, rng, scale=1.0), K, N)
+    x = _dev(P, rng.normal(0, 1, (600, K)).astype(np.float32))
+    runs = [lambda a: [P.mul_mat_mfma(w, a)], lambda a: P.mul_mat_mfma_multi([w, v], a), lambda a: [P.mul_mat_mfma_pair(w, v, a)]]
+    for run in runs:
+        for counts in ((129, 192, 193, 256), (257, 384, 385, 512), (513, 576, 577, 600)):      # (as many tiles of 256 tokens, one split of K)
+            full = run(x[:counts[-1]].contiguous())
+            for T in counts[:-1]:
+                for a, b in zip(run(x[:T].contiguous()), full):
+                    assert P.torch.equal(a, b[:T]), (T, counts)
+
+
+@pytest.mark.parametrize("t", QUANT_TYPES)
 @pytest.mark.parametrize("K,N", [(512, 132), (4096, 260)])
 def test_prompt_tiles_of_96_tokens(P, t, K, N):
     """Tiles of 96 tokens (65..96 tokens; of 8-bit activations also several side by side) beside those of 64 and 128: a token's sums are the same bits in each. Slices of K (4096) and none, rows that
