@@ -26,6 +26,7 @@
 #include "pm355_kernels.h"
 #include <stdlib.h>
 #include <stdio.h>
+#include <algorithm>
 #include <cmath>
 #include <mutex>
 #include <type_traits>
@@ -158,7 +159,8 @@ __device__ __forceinline__ void store_slab(const f32x4 (&o)[4], uint8_t * xe, f3
 // the k loop + epilogue of one workgroup tile: rows [n0, n0 + 256) of job jb, tokens [t0, t0 + 32 NT)
 // role: 0 plain; 1 / 2 = the gate / up half of a PAIR tile (waves 0-3 multiply ffn_gate's rows [n0, n0 + 128), waves 4-7 the same rows of ffn_up; the gate
 // accumulators cross over through LDS after the k loop and the up waves store silu(gate) * up: ffn_gate's result never travels to HBM)
-template <int TYPE, int NT, int EXP>
+// NL: sub-tiles of the launch's tiles (its slabs)
+template <int TYPE, int NT, int EXP, int NL>
 __device__ __forceinline__ void pf_body(const PfP & p, const PfJob & jb, const int n0, const int t0, uint8_t * smem, const int role, const int ks, const int S, const int tile_id) {
     constexpr int BBUF = NT * 32 * 128;                       // one activation buffer: 32 NT tokens x 64 halfs
     constexpr int NSTREAM = PfT<TYPE>::NSTREAM, SLOT = NSTREAM * 1024, AW = pf_wave_bytes<TYPE>();   // per wave: two 128-k slots + two 512-byte header slots + EXTRA
@@ -404,13 +406,13 @@ __device__ __forceinline__ void pf_body(const PfP & p, const PfJob & jb, const i
     }
     // ---- split K: every slice leaves its partial tile in a slab for pf_reduce_kernel, 32 rows of a token as one line (turned in a wave-private LDS tile [token][32 rows + 4])
     if (S > 1) {
-        f32x4 * const mine = (f32x4 *) p.ws + (size_t) (tile_id * S + ks) * (8 * NT * 4 * 64);
+        f32x4 * const mine = (f32x4 *) p.ws + (size_t) (tile_id * S + ks) * (8 * NL * 4 * 64);
 #pragma unroll
         for (int jt = 0; jt < NT; ++jt) {
             f32x4 o[4];
 #pragma unroll
             for (int g = 0; g < 4; ++g) o[g] = f32x4{acc[jt][4 * g], acc[jt][4 * g + 1], acc[jt][4 * g + 2], acc[jt][4 * g + 3]};
-            store_slab(o, smem + wave * (32 * 144), mine + (wave * NT + jt) * 256, lane);
+            store_slab(o, smem + wave * (32 * 144), mine + (wave * NL + jt) * 256, lane);
         }
         return;
     }
@@ -945,8 +947,18 @@ __global__ __launch_bounds__((MID && !mid_self<TA, TB, NT, EX>() ? MID_NTHR : PF
     const int t0 = tile_t * 32 * NT;
     const int tile_id = (slot - p.full) * 8 + x;                 // (split tiles only: slab index)
     if constexpr (!MID) {
-        if (TA == TB || jb.type == TA) pf_body<TA, NT, EXP>(p, jb, n0, t0, pf_smem, role, ks, S, tile_id);
-        else pf_body<TB, NT, EXP>(p, jb, n0, t0, pf_smem, role, ks, S, tile_id);
+        auto body = [&](auto nt) __attribute__((always_inline)) {
+            constexpr int N = decltype(nt)::value;
+            if (TA == TB || jb.type == TA) pf_body<TA, N, EXP, NT>(p, jb, n0, t0, pf_smem, role, ks, S, tile_id);
+            else pf_body<TB, N, EXP, NT>(p, jb, n0, t0, pf_smem, role, ks, S, tile_id);
+        };
+        // The batch's last tile of 256 tokens multiplies the 128 or 192 that are left of it only. us of one K split, whole / cut: wo of the 8B shape 640 tokens 50.4 / 47.5, 1400 79.3 / 75.0, 2100 120 / 104,
+        // its Q6_K ffn_down 1400 237 / 225, ffn_gate | ffn_up 1800 515 / 495, Q8_0 ffn_down of 72B 640 404 / 371; nothing left out (1250) the same. (Tiles of 192 with a cut last one: wo 2400
+        // 105 / 110, wq | wk | wv 6001 360 / 379)
+        const int left = p.T - t0;
+        if (NT == 8 && left <= 128) body(std::integral_constant<int, NT == 8 ? 4 : NT>());
+        else if (NT == 8 && left <= 192) body(std::integral_constant<int, NT == 8 ? 6 : NT>());
+        else body(std::integral_constant<int, NT>());
     } else {
         constexpr bool SELF = mid_self<TA, TB, NT, EX>();
         if (TA == TB || jb.type == TA) mid_body<TA, NT, EX, SELF>(p, jb, n0, t0, pf_smem, role, ks, S, tile_id);
@@ -1254,9 +1266,17 @@ static int launch_pf(const pm_gemm_pf_job * jobs, int njobs, const void * xh, co
     // Q6_K ffn_down of 8B 380 85 / 72, Q8_0 ffn_down of 72B 513 371 / 319, wq | wk | wv of 8B 150 42 / 36, 1500 120 / 100, 6001 404 / 374 (a split tail before), wo 3000 137 / 122, 6001 285 / 251
     if (!mid && !force_nt && !force_s && pl.nt == 8) {
         const int s6 = pl.full ? 1 : pl.splitk, nb = (K + 255) / 256;
-        const auto work = [&](int nt) { return (double) tiles * ((T + 32 * nt - 1) / (32 * nt)) * s6 / cus; };
-        const double tail = pl.full ? pl.cost / nb : 0.0, r8 = pl.full ? tail : std::ceil(work(8)), w8 = pl.full ? tail : work(8);
-        if (7.0 * std::ceil(work(6)) < 0.97 * 9.0 * r8 && 7.0 * work(6) < (r8 == 1.0 ? 1.1 : 0.97) * 9.0 * w8) pm_gemm_pf_plan(tiles, K, T, cus, 6, s6, 0, &pl);
+        // workgroups / CUs, rounds and work in them, in sub-tiles of 32 tokens + 1
+        struct Cost { double rounds, work; };
+        const auto cost = [&](int nt) {
+            const int n = (T - 1) / (32 * nt), left = T - 32 * nt * n, last = nt == 6 || !n ? nt : left <= 128 ? 4 : left <= 192 ? 6 : 8;
+            const double w = (double) tiles * s6 / cus;
+            return Cost{std::ceil(w * (n + 1)) * (nt + 1), w * (n * (nt + 1) + last + 1)};
+        };
+        const Cost c6 = cost(6);
+        Cost c8 = cost(8);
+        if (pl.full) c8.rounds = c8.work = 9.0 * pl.cost / nb;
+        if (c6.rounds < 0.97 * c8.rounds && c6.work < (c8.rounds <= 9.0 ? 1.1 : 0.97) * c8.work) pm_gemm_pf_plan(tiles, K, T, cus, 6, s6, 0, &pl);
     }
     const int nt = pl.nt, S = pl.splitk, full = pl.full, maxL = ((tiles + 7) / 8) * pl.nt_t;
     p.nt_t = pl.nt_t;

@@ -969,7 +969,7 @@ def test_prompt_tiles_of_192_tokens(P, t, K, N):
     x = _dev(P, rng.normal(0, 1, (600, K)).astype(np.float32))
     runs = [lambda a: [P.mul_mat_mfma(w, a)], lambda a: P.mul_mat_mfma_multi([w, v], a), lambda a: [P.mul_mat_mfma_pair(w, v, a)]]
     for run in runs:
-        for counts in ((129, 192, 193, 256), (257, 384, 385, 512), (513, 576, 577, 600)):      # (as many tiles of 256 tokens, one split of K)
+        for counts in ((129, 192, 193, 256), (257, 384, 385, 448, 449, 512), (513, 576, 577, 600)):      # (as many tiles of 256 tokens, one split of K; the last one cut to 128 or 192, or whole)
             full = run(x[:counts[-1]].contiguous())
             for T in counts[:-1]:
                 for a, b in zip(run(x[:T].contiguous()), full):
