@@ -141,11 +141,22 @@ __device__ __forceinline__ void attn_short(const float * q_head, const uint16_t 
     pm_ts_store(ts, 2, tsv);
 }
 
+// What leads to the first loads - positions and sequences, queries and caches, the KV head without a division - leads the arguments, in registers when a launch starts: inv = 2^32 / (heads per KV head),
+// rounded up (0: one), how: 1 rows of several sequences, 2 a length from the graph (dyn). us, 8B shape: eight rows of up to 36 cells
+// 5.05 / 4.77, 169 rows of prompts 24.6 / 22.2; a token of eight layers behind 203 cells 428.2 / 426.6 a pass
+struct CachedArgs { uint32_t heads, inv; int how; };
+static CachedArgs cached_args(const AttnP & a) {
+    const uint64_t R = (uint64_t) (a.H / a.Hkv);
+    return CachedArgs{(uint32_t) a.H | (uint32_t) a.Hkv << 16, R == 1 ? 0u : (uint32_t) (((1ull << 32) + R - 1) / R), (a.rows ? 1 : 0) | (a.dyn ? 2 : 0)};
+}
+__device__ __forceinline__ int kv_head(int h, uint32_t inv) { return inv ? (int) __umulhi((uint32_t) h, inv) : h; }      // (exact: heads x heads per KV head < 2^32)
 template <int DH, int VM>
-__global__ __launch_bounds__(256) void attn_cached_kernel(AttnP a_in) {
+__global__ __launch_bounds__(256) void attn_cached_kernel(const float * q0, uint16_t * kc0, uint16_t * vc0, const int32_t * pos0, const int32_t * seq0, uint32_t heads, uint32_t inv, int n_ctx0, int how, AttnP a_in) {
     // grid.y = tokens of a small batch (engine: 2..64-token steps after rope_kv_store has rotated / rounded q and stored every token's K / V):
     // token t attends cells [0, pos0 + t], its q / out rows are t * H * DH further on
+    // (the leading arguments: CachedArgs; the rest, dyn and the output among them, is read behind the first loads)
     AttnP a = a_in;
+    a.q = q0; a.kc = kc0; a.vc = vc0; a.pos0_ptr = pos0; a.seq_ptr = seq0; a.H = (int) (heads & 65535); a.Hkv = (int) (heads >> 16); a.n_ctx = n_ctx0; a.rows = how & 1;
     a.tok = (int) blockIdx.y;
     a.q += (long) a.tok * a.H * DH; a.out += (long) a.tok * a.H * DH;
     extern __shared__ __attribute__((aligned(16))) char smem[];
@@ -154,9 +165,9 @@ __global__ __launch_bounds__(256) void attn_cached_kernel(AttnP a_in) {
     const int h = blockIdx.x;
     if constexpr (VM == 0) {
         const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-        const int Hkv = a.Hkv, hk = h / (a.H / Hkv), n_ctx = a.n_ctx;
+        const int Hkv = a.Hkv, hk = kv_head(h, inv), n_ctx = a.n_ctx;
         int seq = 0, n_kv;
-        if (a.dyn) n_kv = uniform_const_ptr(a.dyn)[1];
+        if (how & 2) n_kv = uniform_const_ptr(a.dyn)[1];
         else {
             seq = a.seq_ptr ? uniform_const_ptr(a.seq_ptr)[a.rows ? a.tok : 0] : 0;
             n_kv = uniform_const_ptr(a.pos0_ptr)[a.rows ? a.tok : seq] + 1 + (a.rows ? 0 : a.tok);
@@ -177,11 +188,13 @@ __global__ __launch_bounds__(256) void attn_cached_kernel(AttnP a_in) {
 
 // The same for rows of up to 256 cells and two heads of 128 per workgroup, whose results meet in LDS and leave as a Q8_K block (the wo product's activations) - no f32 rows and no launch that
 // quantizes them: 8 sequences of the 8B shape, 4.0 + 3.2 us and the gap between them, now 6.4
-__global__ __launch_bounds__(512) void attn_cached_q8k_kernel(AttnP a, pm_q8k_out y) {
+__global__ __launch_bounds__(512) void attn_cached_q8k_kernel(const float * q0, uint16_t * kc0, uint16_t * vc0, const int32_t * pos0, const int32_t * seq0, uint32_t heads, uint32_t inv, int n_ctx0, float scale0, AttnP a,
+                                                              pm_q8k_out y) {
+    a.q = q0; a.kc = kc0; a.vc = vc0; a.pos0_ptr = pos0; a.seq_ptr = seq0; a.H = (int) (heads & 65535); a.Hkv = (int) (heads >> 16); a.n_ctx = n_ctx0; a.scale = scale0;
     extern __shared__ __attribute__((aligned(16))) char smem[];
     __shared__ __attribute__((aligned(16))) float row[256];
     const int tid = threadIdx.x, lane = tid & 63, w8 = __builtin_amdgcn_readfirstlane(tid >> 6), half = w8 >> 2, wave = w8 & 3;
-    const int t = blockIdx.y, blk = blockIdx.x, h = 2 * blk + half, hk = h / (a.H / a.Hkv), seq = uniform_const_ptr(a.seq_ptr)[t], n_kv = uniform_const_ptr(a.pos0_ptr)[t] + 1;
+    const int t = blockIdx.y, blk = blockIdx.x, h = 2 * blk + half, hk = kv_head(h, inv), seq = uniform_const_ptr(a.seq_ptr)[t], n_kv = uniform_const_ptr(a.pos0_ptr)[t] + 1;
     auto go = [&](auto kpl) __attribute__((always_inline)) {     // (chosen by the row's own cells, as above: the sums do not depend on what else is in the batch)
         constexpr int KPL = decltype(kpl)::value;
         attn_short<128, KPL>(a.q + ((long) t * a.H + h) * 128, a.kc + (long) seq * a.seq_stride, a.vc + (long) seq * a.seq_stride, [&](int d, float v) __attribute__((always_inline)) { row[128 * half + d] = v; },
@@ -207,7 +220,8 @@ int pm_launch_attn_cached_q8k(const float * q, void * kc, void * vc, const int32
     AttnP a = {q, nullptr, nullptr, (uint16_t *) kc, (uint16_t *) vc, pos, seq, seq_stride, nullptr, nullptr, H, Hkv, n_ctx, scale, RopeP(), nullptr, nullptr, 0, nullptr, 0, 1};
     const size_t lds = 2 * (size_t) (kpl == 1 ? ShortLds<128, 1>::BYTES : kpl == 2 ? ShortLds<128, 2>::BYTES : ShortLds<128, 4>::BYTES);
     pm_allow_big_lds((const void *) attn_cached_q8k_kernel, lds);
-    hipLaunchKernelGGL(attn_cached_q8k_kernel, dim3(H / 2, n_tok), dim3(512), lds, st, a, out);
+    const CachedArgs c = cached_args(a);
+    hipLaunchKernelGGL(attn_cached_q8k_kernel, dim3(H / 2, n_tok), dim3(512), lds, st, a.q, a.kc, a.vc, a.pos0_ptr, a.seq_ptr, c.heads, c.inv, a.n_ctx, a.scale, a, out);
     return 0;
 }
 
@@ -222,7 +236,7 @@ void pm_launch_rope_table(const pm_rope_cfg & c, const int32_t * pos, const int3
 int pm_launch_attn_cached(const float * q, void * kc, void * vc, const int32_t * pos0, const int32_t * seq, long seq_stride, float * out,
                           int H, int Hkv, int dh, int n_ctx, float scale, hipStream_t st, const int32_t * dyn, const void * mask,
                           int max_keys, int v_rowmajor, int mask_f16, int n_tok, int rows) {
-    if ((dh != 64 && dh != 128 && dh != 256) || n_ctx % 8 || n_tok < 1 || (n_tok > 1 && dyn) || (rows && (dyn || !seq || !pos0))) return -1;
+    if ((dh != 64 && dh != 128 && dh != 256) || n_ctx % 8 || n_tok < 1 || H > 65535 || Hkv > 65535 || (n_tok > 1 && dyn) || (rows && (dyn || !seq || !pos0))) return -1;
     size_t lds = (size_t) (4 * dh + (v_rowmajor ? 2048 : 256) + (max_keys > 0 ? ((max_keys + 7) & ~7) : n_ctx) + 8) * 4;
     if (lds > 150 * 1024) return -1;
     // (two workgroups of the largest short form per CU, as many as their registers allow)
@@ -236,7 +250,8 @@ int pm_launch_attn_cached(const float * q, void * kc, void * vc, const int32_t *
         pm_allow_big_lds((const void *) kern, lds);
         AttnP a = {q, nullptr, nullptr, (uint16_t *) kc, (uint16_t *) vc, pos0, seq, seq_stride, nullptr, out, H, Hkv, n_ctx, scale, r, dyn,
                    (const float *) mask, mask_f16, pm_ts_next_slot(), 0, rows};
-        hipLaunchKernelGGL(kern, dim3(H, n_tok), dim3(256), lds, st, a);
+        const CachedArgs c = cached_args(a);
+        hipLaunchKernelGGL(kern, dim3(H, n_tok), dim3(256), lds, st, a.q, a.kc, a.vc, a.pos0_ptr, a.seq_ptr, c.heads, c.inv, a.n_ctx, c.how, a);
     };
     if (v_rowmajor) {
         if (dh == 64) launch(attn_cached_kernel<64, 1>);
