@@ -17,13 +17,14 @@
 #include "pm355_kernels.h"
 #include "pm355_q8k.h"
 
+// (Grids of rows x groups of four blocks, below of rows x 1024 values: by one index, split into row and block in 64 bits, every launch began with a division of a few hundred instructions in front of
+// its first load. us a pass before / now: eight sequences of the 8B shape, 96 launches of 8 rows of 14336 9056 / 9036;
+// two layers of the 72B shape at 23 tokens, silu_mul_q80_tab_kernel, 451.1 / 449.9)
 __global__ __launch_bounds__(256) void quantize_q8k_kernel(const float * __restrict__ x, uint8_t * __restrict__ y,
-                                                           int K, int rows, size_t y_row_bytes, pm_q8k_tables tb, pm_q8k_wide wd) {
+                                                           int K, size_t y_row_bytes, pm_q8k_tables tb, pm_q8k_wide wd) {
     const int lane = threadIdx.x & 63;
-    const int nblk = K / PM_QK_K;
-    const long wave = (long) blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (wave >= (long) rows * nblk) return;
-    const int row = (int) (wave / nblk), blk = (int) (wave % nblk);
+    const int row = (int) blockIdx.x, blk = (int) blockIdx.y * 4 + __builtin_amdgcn_readfirstlane((int) threadIdx.x >> 6);
+    if (blk >= K / PM_QK_K) return;
     const float4 f = ((const float4 *) (x + (size_t) row * K + (size_t) blk * PM_QK_K))[lane];
     const float v[4] = {f.x, f.y, f.z, f.w};
     q8k_block_from_regs(v, lane, y ? y + (size_t) row * y_row_bytes : nullptr, K, blk, tb, row, wd);
@@ -32,12 +33,10 @@ __global__ __launch_bounds__(256) void quantize_q8k_kernel(const float * __restr
 // silu(gate) * up (ggml_silu + ggml_mul of llm_build_ffn, src/llama.cpp:9804; same f32 expressions as layer_ops.hip's silu_mul_kernel) fused with
 // the Q8_K quantization of the product: the ffn_down activations of a small batch, without the f32 round trip through HBM
 __global__ __launch_bounds__(256) void silu_mul_q8k_kernel(const float * __restrict__ gate, const float * __restrict__ up, uint8_t * __restrict__ y,
-                                                           int K, int rows, size_t y_row_bytes, pm_q8k_tables tb) {
+                                                           int K, size_t y_row_bytes, pm_q8k_tables tb) {
     const int lane = threadIdx.x & 63;
-    const int nblk = K / PM_QK_K;
-    const long wave = (long) blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (wave >= (long) rows * nblk) return;
-    const int row = (int) (wave / nblk), blk = (int) (wave % nblk);
+    const int row = (int) blockIdx.x, blk = (int) blockIdx.y * 4 + __builtin_amdgcn_readfirstlane((int) threadIdx.x >> 6);
+    if (blk >= K / PM_QK_K) return;
     const float4 g = ((const float4 *) (gate + (size_t) row * K + (size_t) blk * PM_QK_K))[lane];
     const float4 u = ((const float4 *) (up + (size_t) row * K + (size_t) blk * PM_QK_K))[lane];
     const float v[4] = {g.x / (1.0f + expf(-g.x)) * u.x, g.y / (1.0f + expf(-g.y)) * u.y, g.z / (1.0f + expf(-g.z)) * u.z, g.w / (1.0f + expf(-g.w)) * u.w};
@@ -46,11 +45,9 @@ __global__ __launch_bounds__(256) void silu_mul_q8k_kernel(const float * __restr
 
 // Q8_0: 32-value blocks, 8 lanes x 4 values; amax over the 8-lane group.
 __global__ __launch_bounds__(256) void quantize_q80_kernel(const float * __restrict__ x, uint8_t * __restrict__ y,
-                                                           int K, int rows, size_t y_row_bytes) {
-    const long t = (long) blockIdx.x * 256 + threadIdx.x;        // one thread = 4 values
-    const long per_row = K / 4;
-    if (t >= (long) rows * per_row) return;
-    const int row = (int) (t / per_row), i4 = (int) (t % per_row);
+                                                           int K, size_t y_row_bytes) {
+    const int row = (int) blockIdx.x, i4 = (int) blockIdx.y * 256 + (int) threadIdx.x;        // one thread = 4 values
+    if (i4 >= K / 4) return;
     const float4 f = ((const float4 *) (x + (size_t) row * K))[i4];
     float amax = fmaxf(fmaxf(fabsf(f.x), fabsf(f.y)), fmaxf(fabsf(f.z), fabsf(f.w)));
     amax = group8_max(amax);
@@ -70,11 +67,9 @@ __global__ __launch_bounds__(256) void quantize_q80_kernel(const float * __restr
 // 256 (Qwen2.5-72B: K = 29568 falls back to Q8_0, src/llama.cpp:19447). Replaces three launches (silu_mul, quantize_q80, the mat-mul's table prologue).
 // Rows T .. 32 * passes - 1 write scale 0 (their values are never loaded).
 __global__ __launch_bounds__(256) void silu_mul_q80_tab_kernel(const float * __restrict__ gate, const float * __restrict__ up, uint8_t * __restrict__ tab,
-                                                               int K, int rows, int rows_padded, size_t pass_bytes, size_t qtab_bytes) {
-    const long t = (long) blockIdx.x * 256 + threadIdx.x;        // one thread = 4 values, 8 lanes = one block
-    const long per_row = K / 4;
-    if (t >= (long) rows_padded * per_row) return;
-    const int row = (int) (t / per_row), i4 = (int) (t % per_row);
+                                                               int K, int rows, size_t pass_bytes, size_t qtab_bytes) {
+    const int row = (int) blockIdx.x, i4 = (int) blockIdx.y * 256 + (int) threadIdx.x;        // one thread = 4 values, 8 lanes = one block
+    if (i4 >= K / 4) return;
     const int blk = i4 >> 3, sub = i4 & 7;
     uint8_t * base = tab + (size_t) (row >> 5) * pass_bytes;
     float * dslot = (float *) (base + qtab_bytes) + ((size_t) blk * 32 + (row & 31));
@@ -170,30 +165,26 @@ __global__ __launch_bounds__(64 * NWV) void rmsnorm_q8k_kernel(const float * __r
 
 static bool norm_split(int K, int rows) { return K > 16 * PM_QK_K && K <= 32 * PM_QK_K && 2 * rows <= pm_device_cus(); }
 
+static dim3 q8k_grid(int K, int rows) { return dim3(rows, (K / PM_QK_K + 3) / 4); }
+
 // ---- host launchers -------------------------------------------------------------------------------
 void pm_launch_quantize_q8k(const float * x, void * y, int K, int rows, hipStream_t st, pm_q8k_tables tab) {
-    const long waves = (long) rows * (K / PM_QK_K);
-    hipLaunchKernelGGL(quantize_q8k_kernel, dim3((unsigned) ((waves + 3) / 4)), dim3(256), 0, st,
-                       x, (uint8_t *) y, K, rows, pm_q8k_row_bytes(K), tab, pm_q8k_wide());
+    hipLaunchKernelGGL(quantize_q8k_kernel, q8k_grid(K, rows), dim3(256), 0, st,
+                       x, (uint8_t *) y, K, pm_q8k_row_bytes(K), tab, pm_q8k_wide());
 }
 void pm_launch_quantize_wide(const float * x, const pm_q8k_wide & y, int K, int rows, hipStream_t st) {
-    const long waves = (long) rows * (K / PM_QK_K);
-    hipLaunchKernelGGL(quantize_q8k_kernel, dim3((unsigned) ((waves + 3) / 4)), dim3(256), 0, st, x, (uint8_t *) nullptr, K, rows, 0, pm_q8k_tables(), y);
+    hipLaunchKernelGGL(quantize_q8k_kernel, q8k_grid(K, rows), dim3(256), 0, st, x, (uint8_t *) nullptr, K, 0, pm_q8k_tables(), y);
 }
 void pm_launch_silu_mul_q8k(const float * gate, const float * up, void * y, int K, int rows, hipStream_t st, pm_q8k_tables tab) {
-    const long waves = (long) rows * (K / PM_QK_K);
-    hipLaunchKernelGGL(silu_mul_q8k_kernel, dim3((unsigned) ((waves + 3) / 4)), dim3(256), 0, st, gate, up, (uint8_t *) y, K, rows, pm_q8k_row_bytes(K), tab);
+    hipLaunchKernelGGL(silu_mul_q8k_kernel, q8k_grid(K, rows), dim3(256), 0, st, gate, up, (uint8_t *) y, K, pm_q8k_row_bytes(K), tab);
 }
 void pm_launch_silu_mul_q80_tab(const float * gate, const float * up, void * tab, size_t qtab_bytes, size_t dtab_bytes, int K, int rows, hipStream_t st) {
-    const int rows_padded = (rows + 31) / 32 * 32;
-    const long n = (long) rows_padded * (K / 4);
-    hipLaunchKernelGGL(silu_mul_q80_tab_kernel, dim3((unsigned) ((n + 255) / 256)), dim3(256), 0, st, gate, up, (uint8_t *) tab, K, rows, rows_padded,
+    hipLaunchKernelGGL(silu_mul_q80_tab_kernel, dim3((rows + 31) / 32 * 32, (K / 4 + 255) / 256), dim3(256), 0, st, gate, up, (uint8_t *) tab, K, rows,
                        qtab_bytes + dtab_bytes, qtab_bytes);
 }
 void pm_launch_quantize_q80(const float * x, void * y, int K, int rows, hipStream_t st) {
-    const long n = (long) rows * (K / 4);
-    hipLaunchKernelGGL(quantize_q80_kernel, dim3((unsigned) ((n + 255) / 256)), dim3(256), 0, st,
-                       x, (uint8_t *) y, K, rows, pm_q80_row_bytes(K));
+    hipLaunchKernelGGL(quantize_q80_kernel, dim3(rows, (K / 4 + 255) / 256), dim3(256), 0, st,
+                       x, (uint8_t *) y, K, pm_q80_row_bytes(K));
 }
 void pm_launch_rmsnorm_q8k(const float * x, const float * w, float * ynorm, void * yq, int K, int rows, float eps, hipStream_t st, void * ynorm_f16, pm_q8k_tables tab) {
     if (norm_split(K, rows)) hipLaunchKernelGGL((rmsnorm_q8k_kernel<16, true>), dim3(rows, 2), dim3(1024), 0, st, x, w, ynorm, (uint8_t *) yq, K, eps, pm_q8k_row_bytes(K), (_Float16 *) ynorm_f16, tab, pm_q8k_wide());
