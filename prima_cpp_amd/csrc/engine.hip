@@ -1546,8 +1546,12 @@ int pm_window::batch_rows(const pm355_batch_entry * e, int n, float * d_logits, 
             else {
                 if (!output.d || !out_norm.d) { rc = seterr(m, PM355_E_UNSUPPORTED, "head: output / output_norm missing"); break; }
                 const Tensor * ow[1] = {&output};
-                pm_launch_gather_rows(rows, d_rows + at_want + w, k, hp.n_embd, x1, st);
-                const ActQ a = norm_quantize_for(m, x1, (const float *) out_norm.d, hp.n_embd, k, ow, 1, st);
+                // (rows that are neighbours in their order, as in every step of single tokens, are normed where they are: a launch of 4.8 us less)
+                float * hx = rows + (size_t) want[w].row * hp.n_embd;
+                bool apart = false;
+                for (int i = 1; i < k; ++i) apart |= want[w + i].row != want[w].row + i;
+                if (apart) { hx = x1; pm_launch_gather_rows(rows, d_rows + at_want + w, k, hp.n_embd, hx, st); }
+                const ActQ a = norm_quantize_for(m, hx, (const float *) out_norm.d, hp.n_embd, k, ow, 1, st);
                 bool prepped = false;
                 if (matmul_small(m, output, a, k, lg, nullptr, nullptr, prepped, st)) rc = seterr(m, PM355_E_UNSUPPORTED, "head: lm_head mat-mul");
                 else if (d_argmax) pm_launch_argmax(lg, V, d_argmax + o, nullptr, st, k, am_part);
