@@ -26,6 +26,7 @@
 //    the rows of every job.
 #include "mmvq_device.h"
 #include <stdlib.h>
+#include <algorithm>
 
 using namespace pmv;
 
@@ -141,7 +142,7 @@ int pm_gemv_units_per_row(int type, int64_t K) { return (int) (K / nv_of(type));
 
 // Validates a fused job list and fills the kernel argument block. ta <= tb are the (at most two) quant types in the
 // canonical order of the instantiated kernels: (Q4_K,Q4_K) (Q5_K,Q5_K) (Q6_K,Q6_K) (Q8_0,Q8_0) (Q4_K,Q6_K) (Q4_K,Q5_K); job 0 is
-// always a `ta` job (the kernel pre-issues it). grid_fixed > 0: the caller's grid (attn_wo.hip), else chosen here.
+// always a `ta` job (the kernel pre-issues it). grid_fixed > 0: the caller's grid, else chosen here (< 0: for a launch of its own).
 int pmv::gemv_fill(const pm_gemv_fused & a, int grid_fixed, GemvP & p, int & ta_out, int & tb_out, bool & pair_out, size_t & lds_out, int & grid_out) {
     if (a.njobs < 1 || a.njobs > 3) return -4;
     p = GemvP{};
@@ -170,6 +171,10 @@ int pmv::gemv_fill(const pm_gemv_fused & a, int grid_fixed, GemvP & p, int & ta_
     int grid = grid_fixed > 0 ? grid_fixed : (1024 / PM_GEMV_BLOCK) * pm_device_cus();
     long tot_rows = 0;
     for (int j = 0; j < a.njobs; ++j) tot_rows += a.job[j].N;
+    // Matrices of less than four rows per CU and 512 KB: workgroups of four rows. The weights are a round of latency anyway, and 4096 waves of which most have no row take longer to start than 1024:
+    // one token of two layers of width 256 64.9 us, now 63.0 (8 rows 63.6, 16 65.9, 32 74.9). (The epilogue's slices hold whole rotation pairs of every matrix, sums of squares are a
+    // workgroup's each, and the phases of one persistent launch have one grid: they stay)
+    if (grid_fixed < 0 && !a.epi && !a.ss_out && tot_rows * (long) pm_weight_row_stride(a.job[0].type, a.K) < 512 * 1024) grid = (int) std::max(1l, std::min((long) grid, (tot_rows + 3) / 4));
     int rows_cap = PM_MAX_ROWS_PER_WG;
     if (grid_fixed > 0) rows_cap = (int) ((tot_rows + grid - 1) / grid + 3 > PM_MAX_ROWS_PER_WG ? (tot_rows + grid - 1) / grid + 4 : PM_MAX_ROWS_PER_WG);
     else while ((tot_rows + grid - 1) / grid + 3 > PM_MAX_ROWS_PER_WG) grid *= 2;
@@ -233,7 +238,7 @@ int pmv::gemv_fill(const pm_gemv_fused & a, int grid_fixed, GemvP & p, int & ta_
 
 int pm_gemv_fused_check(const pm_gemv_fused & a) {
     GemvP p; int ta, tb, grid; bool pair; size_t lds;
-    return gemv_fill(a, 0, p, ta, tb, pair, lds, grid);
+    return gemv_fill(a, -1, p, ta, tb, pair, lds, grid);
 }
 
 int pm_gemv_fused_grid(const pm_gemv_fused & a) {
@@ -245,7 +250,7 @@ int pm_gemv_fused_grid(const pm_gemv_fused & a) {
 // Fused launch: up to 3 matrices sharing one activation row.
 int pm_launch_gemv_fused(const pm_gemv_fused & a, hipStream_t st) {
     GemvP p; int ta, tb, grid; bool pair; size_t lds;
-    const int rc = gemv_fill(a, 0, p, ta, tb, pair, lds, grid);
+    const int rc = gemv_fill(a, -1, p, ta, tb, pair, lds, grid);
     if (rc) return rc;
     p.ts = pm_ts_next_slot();
 #define PM_L(TA_, TB_) return launch_types<TA_, TB_>(p, pair, grid, lds, a.dbg_int != nullptr, st, a.epi != nullptr)
@@ -276,7 +281,7 @@ int pm_launch_gemv(const pm_gemv_args & a, hipStream_t st) {
         int nc = (a.dbg_int || left < 2) ? 1 : pair ? ((a.type == PM_Q4_K || a.type == PM_Q6_K) ? 2 : 1) : (left >= 8 && a.type != PM_Q5_K ? 8 : left >= 3 ? 4 : 2);   // (8 Q5_K columns spill even at 256 VGPRs)
         if (nc > 1) {
             GemvP p; int ta, tb, grid; bool pr; size_t lds1;
-            int rc = gemv_fill(f, 0, p, ta, tb, pr, lds1, grid);
+            int rc = gemv_fill(f, -1, p, ta, tb, pr, lds1, grid);
             if (rc) return rc;
             // LDS: nc activation columns + nc results per row
             const int ablk = ta == PM_Q8_0 ? 32 : 256;
