@@ -133,7 +133,7 @@ PM355_API int pm355_act_to_ggml_blocks(int act_type /*15=Q8_K, 8=Q8_0*/, const v
                                        int64_t K, int64_t rows, pm355_stream_t stream);
 
 /* replaces ggml_compute_forward_rms_norm_f32 (ggml/src/ggml.c:11950) [+ ggml_compute_forward_mul_f32 (:10077)
- * when w != NULL]. y_f32 and/or yq (Q8_K) may be NULL. One pass over x. */
+ * when w != NULL]. y_f32 and/or yq (Q8_K) may be NULL; y_f32 may be x (in place). One pass over x. */
 PM355_API int pm355_rms_norm(const float * x, const float * w, float * y_f32, void * yq, int64_t K, int64_t rows,
                              float eps, pm355_stream_t stream);
 

@@ -163,7 +163,13 @@ __global__ __launch_bounds__(64 * NWV) void rmsnorm_q8k_kernel(const float * __r
     }
 }
 
-static bool norm_split(int K, int rows) { return K > 16 * PM_QK_K && K <= 32 * PM_QK_K && 2 * rows <= pm_device_cus(); }
+// (a row whose results lie on the input is one workgroup's: of two, one may store its half before the other has read the row)
+static bool norm_split(const float * x, const float * ynorm, const void * yq, const void * yh, int K, int rows) {
+    if (K <= 16 * PM_QK_K || K > 32 * PM_QK_K || 2 * rows > pm_device_cus()) return false;
+    const size_t n = (size_t) rows * K;
+    const auto meets = [&](const void * y, size_t bytes) { return y && (uintptr_t) y < (uintptr_t) (x + n) && (uintptr_t) x < (uintptr_t) y + bytes; };
+    return !meets(ynorm, n * 4) && !meets(yq, rows * pm_q8k_row_bytes(K)) && !meets(yh, n * 2);
+}
 
 static dim3 q8k_grid(int K, int rows) { return dim3(rows, (K / PM_QK_K + 3) / 4); }
 
@@ -187,12 +193,12 @@ void pm_launch_quantize_q80(const float * x, void * y, int K, int rows, hipStrea
                        x, (uint8_t *) y, K, pm_q80_row_bytes(K));
 }
 void pm_launch_rmsnorm_q8k(const float * x, const float * w, float * ynorm, void * yq, int K, int rows, float eps, hipStream_t st, void * ynorm_f16, pm_q8k_tables tab) {
-    if (norm_split(K, rows)) hipLaunchKernelGGL((rmsnorm_q8k_kernel<16, true>), dim3(rows, 2), dim3(1024), 0, st, x, w, ynorm, (uint8_t *) yq, K, eps, pm_q8k_row_bytes(K), (_Float16 *) ynorm_f16, tab, pm_q8k_wide());
+    if (norm_split(x, ynorm, yq, ynorm_f16, K, rows)) hipLaunchKernelGGL((rmsnorm_q8k_kernel<16, true>), dim3(rows, 2), dim3(1024), 0, st, x, w, ynorm, (uint8_t *) yq, K, eps, pm_q8k_row_bytes(K), (_Float16 *) ynorm_f16, tab, pm_q8k_wide());
     else if (rows <= pm_device_cus()) hipLaunchKernelGGL(rmsnorm_q8k_kernel<16>, dim3(rows), dim3(1024), 0, st, x, w, ynorm, (uint8_t *) yq, K, eps, pm_q8k_row_bytes(K), (_Float16 *) ynorm_f16, tab, pm_q8k_wide());
     else            hipLaunchKernelGGL(rmsnorm_q8k_kernel<4>, dim3(rows), dim3(256), 0, st, x, w, ynorm, (uint8_t *) yq, K, eps, pm_q8k_row_bytes(K), (_Float16 *) ynorm_f16, tab, pm_q8k_wide());
 }
 void pm_launch_rmsnorm_wide(const float * x, const float * w, const pm_q8k_wide & y, int K, int rows, float eps, hipStream_t st) {
-    if (norm_split(K, rows)) hipLaunchKernelGGL((rmsnorm_q8k_kernel<16, true>), dim3(rows, 2), dim3(1024), 0, st, x, w, (float *) nullptr, (uint8_t *) nullptr, K, eps, 0, (_Float16 *) nullptr, pm_q8k_tables(), y);
+    if (norm_split(x, nullptr, nullptr, nullptr, K, rows)) hipLaunchKernelGGL((rmsnorm_q8k_kernel<16, true>), dim3(rows, 2), dim3(1024), 0, st, x, w, (float *) nullptr, (uint8_t *) nullptr, K, eps, 0, (_Float16 *) nullptr, pm_q8k_tables(), y);
     else if (rows <= pm_device_cus()) hipLaunchKernelGGL(rmsnorm_q8k_kernel<16>, dim3(rows), dim3(1024), 0, st, x, w, (float *) nullptr, (uint8_t *) nullptr, K, eps, 0, (_Float16 *) nullptr, pm_q8k_tables(), y);
     else             hipLaunchKernelGGL(rmsnorm_q8k_kernel<4>, dim3(rows), dim3(256), 0, st, x, w, (float *) nullptr, (uint8_t *) nullptr, K, eps, 0, (_Float16 *) nullptr, pm_q8k_tables(), y);
 }

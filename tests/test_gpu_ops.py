@@ -443,6 +443,21 @@ def test_rms_norm_rows_of_two_workgroups(P, K):
         assert P.torch.equal(a, y[:rows]) and P.torch.equal(aq, yq[:aq.numel()]), rows
 
 
+@pytest.mark.parametrize("K", [4096, 4352, 8192, 8448])
+def test_rms_norm_in_place(P, K):
+    """y_f32 == x: the same bits as into memory of its own, for rows that two workgroups take otherwise and for their neighbours"""
+    import ctypes as C
+    from prima_cpp_amd import lib as L
+    rng = np.random.default_rng(K)
+    f = L.declare("pm355_rms_norm", C.c_int, [C.c_void_p] * 4 + [C.c_int64, C.c_int64, C.c_float, C.c_void_p])
+    for rows in (1, 8, 128):
+        x, w = _dev(P, rng.normal(0, 2, (rows, K)).astype(np.float32)), _dev(P, (1 + rng.normal(0, 0.02, K)).astype(np.float32))
+        want, want_q = P.rms_norm(x, w, 1e-5, want_q8=True)
+        q = P.torch.empty_like(want_q)
+        L.check(f(L.ptr(x), L.ptr(w), L.ptr(x), L.ptr(q), K, rows, 1e-5, L.stream_ptr()), "rms_norm")
+        assert P.torch.equal(x, want) and P.torch.equal(q, want_q), rows
+
+
 def test_gemv_full_size_linearity(P):
     """BASELINE-size property test (no oracle at this size): W.(a) + W.(b) == W.(a+b) is NOT exact after
     activation quantization, so instead check y(W, x) against dequantize-free structure: scaling x by 2

@@ -303,3 +303,26 @@ for t in (12, 13, 14, 8):
 assert not short, (len(short), short[:20])
 print("ok")
 """)
+
+
+def test_a_norm_whose_results_lie_on_its_input_has_one_workgroup_to_a_row(run):
+    """pm355_rms_norm in place (y_f32 == x), or with the Q8_K blocks on the row: of two workgroups to a row (17..32 blocks, up to half the CUs' rows) one could store its half before the other has
+    read the row"""
+    run(COMMON + r"""
+lib = C.CDLL(sys.argv[2])
+f = lib.pm355_rms_norm
+f.argtypes = [C.c_void_p] * 4 + [C.c_int64, C.c_int64, C.c_float, C.c_void_p]
+at = C.addressof(C.create_string_buffer(256)) // 16 * 16 + 16
+def grid(K, rows, y, yq):
+    shim.shim_forget()
+    assert f(at, None, y, yq, K, rows, 1e-5, 1) == 0
+    (_, _, g), = launches()
+    return g[:2]
+for K in (4352, 8192):
+    for rows in (1, 8, 128):
+        n, q = rows * K * 4, rows * (K + K // 256 * 4 + K // 16 * 2)
+        assert grid(K, rows, at + n, None) == grid(K, rows, at - n, None) == grid(K, rows, None, at + n) == grid(K, rows, None, at - q) == grid(K, rows, at + n, at - q) == (rows, 2), (K, rows)
+        assert grid(K, rows, at, None) == grid(K, rows, None, at) == grid(K, rows, at, at + n) == grid(K, rows, at + n, at + n - 16) == grid(K, rows, at - 16, None) == (rows, 1), (K, rows)
+assert grid(4096, 8, at, None) == grid(4096, 8, at + (1 << 20), None) == (8, 1) and grid(8192, 129, at + (1 << 30), None) == (129, 1)
+print("ok")
+""")
