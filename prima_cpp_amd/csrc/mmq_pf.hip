@@ -1214,6 +1214,7 @@ static int launch_pf(const pm_gemm_pf_job * jobs, int njobs, const void * xh, co
     if (njobs < 1 || njobs > PF_MAX_JOBS || !jobs || !xh) return -2;
     if (pair && (njobs != 2 || jobs[0].type != jobs[1].type || jobs[0].N != jobs[1].N || jobs[0].bias || jobs[0].resid || jobs[1].silu_gate)) return -2;
     static const int force_nt = [] { const char * e = getenv("PM355_GEMM_PF_NT"); return e ? atoi(e) : 0; }();
+    const int asked_nt = force_nt == 2 || force_nt == 4 || force_nt == 6 || force_nt == 8 ? force_nt : 0;      // (what the 256-row tiles have kernels for)
     const int cus = pm_device_cus();
     // mid_body for up to 128 tokens where its 128-row tiles are one round of workgroups: there a launch is its fixed costs and its K split. us, pf_body / mid_body, Q4_K: 4096 x 4096
     // 101 tokens 28.9 / 22.0, 4096 x 14336 50.4 / 35.7, 32768 x 4096 (256 tiles) 128 tokens 66 / 52. With more tiles the 256-row tiles' fewer bytes per product win: 40960 x 4096 (320)
@@ -1252,7 +1253,7 @@ static int launch_pf(const pm_gemm_pf_job * jobs, int njobs, const void * xh, co
     // at the reference's default n_ubatch 512 (common/common.h:178) are 64-80 tiles for 256 CUs - are split along K: S slices per tile, the slice count that
     // minimises  rounds of workgroups x (super-blocks per slice + ~3 for prologue, slab traffic and the launch that adds the slices up)
     pm_gemm_pf_plan_t pl;
-    pm_gemm_pf_plan(tiles, K, T, cus, mid ? mid_nt : force_nt, force_s, no_mixed ? 0 : 1, &pl);
+    pm_gemm_pf_plan(tiles, K, T, cus, mid ? mid_nt : asked_nt, force_s, no_mixed ? 0 : 1, &pl);
     // 8-bit activations of Q4_K: tiles of 96 tokens (with loaders) where they cost less than those of 128 (without: no registers left for them), by rounds of workgroups; the K split stays that of
     // 128 tokens: the sums in one order. 8B shape, whole passes, us, 128 / 96: 79 tokens 716 / 675, 109 738 / 801, 147 935 / 858, 231 1025 / 1095, 316 1279 / 1260, 459 1498 / 1570
     if (wide && !two && T > 64 && !pl.full && (T + 95) / 96 * 96 <= wide->ldt) {
@@ -1338,7 +1339,24 @@ static int launch_pf(const pm_gemm_pf_job * jobs, int njobs, const void * xh, co
         return 0;
     }
 #endif
-#define PF_GO(A, B) (wide ? nt == 4 ? go(gemm_pf_kernel<PM_Q4_K, PM_Q4_K, 4, true, 0, true>, pf_lds_bytes<PM_Q4_K, PM_Q4_K, 4, true, true>()) : nt == 3 ? go(gemm_pf_kernel<PM_Q4_K, PM_Q4_K, 3, true, 0, true>, pf_lds_bytes<PM_Q4_K, PM_Q4_K, 3, true, true>()) : go(gemm_pf_kernel<A, B, 2, true, 0, A != PM_Q8_0>, pf_lds_bytes<A, B, 2, true, A != PM_Q8_0>()) : mid ? nt == 4 ? go(gemm_pf_kernel<A, B, 4, true>, pf_lds_bytes<A, B, 4, true>()) : nt == 3 ? go(gemm_pf_kernel<A, B, 3, true>, pf_lds_bytes<A, B, 3, true>()) : go(gemm_pf_kernel<A, B, 2, true>, pf_lds_bytes<A, B, 2, true>()) : nt == 8 ? go(gemm_pf_kernel<A, B, 8>, pf_lds_bytes<A, B, 8>()) : nt == 6 ? go(gemm_pf_kernel<A, B, 6>, pf_lds_bytes<A, B, 6>()) : nt == 4 ? go(gemm_pf_kernel<A, B, 4>, pf_lds_bytes<A, B, 4>()) : go(gemm_pf_kernel<A, B, 2>, pf_lds_bytes<A, B, 2>()))
+    // (an nt that no kernel has stays an error)
+#define PF_GO(A, B) do { \
+        if (wide) { \
+            if (nt == 4)      go(gemm_pf_kernel<PM_Q4_K, PM_Q4_K, 4, true, 0, true>, pf_lds_bytes<PM_Q4_K, PM_Q4_K, 4, true, true>()); \
+            else if (nt == 3) go(gemm_pf_kernel<PM_Q4_K, PM_Q4_K, 3, true, 0, true>, pf_lds_bytes<PM_Q4_K, PM_Q4_K, 3, true, true>()); \
+            else if (nt == 2) go(gemm_pf_kernel<A, B, 2, true, 0, A != PM_Q8_0>, pf_lds_bytes<A, B, 2, true, A != PM_Q8_0>()); \
+            else return -2; \
+        } else if (mid) { \
+            if (nt == 4)      go(gemm_pf_kernel<A, B, 4, true>, pf_lds_bytes<A, B, 4, true>()); \
+            else if (nt == 3) go(gemm_pf_kernel<A, B, 3, true>, pf_lds_bytes<A, B, 3, true>()); \
+            else if (nt == 2) go(gemm_pf_kernel<A, B, 2, true>, pf_lds_bytes<A, B, 2, true>()); \
+            else return -2; \
+        } else if (nt == 8)   go(gemm_pf_kernel<A, B, 8>, pf_lds_bytes<A, B, 8>()); \
+        else if (nt == 6)     go(gemm_pf_kernel<A, B, 6>, pf_lds_bytes<A, B, 6>()); \
+        else if (nt == 4)     go(gemm_pf_kernel<A, B, 4>, pf_lds_bytes<A, B, 4>()); \
+        else if (nt == 2)     go(gemm_pf_kernel<A, B, 2>, pf_lds_bytes<A, B, 2>()); \
+        else return -2; \
+    } while (0)
     if (ta == tb) { if (ta == PM_Q4_K) PF_GO(PM_Q4_K, PM_Q4_K); else if (ta == PM_Q5_K) PF_GO(PM_Q5_K, PM_Q5_K); else if (ta == PM_Q8_0) PF_GO(PM_Q8_0, PM_Q8_0); else PF_GO(PM_Q6_K, PM_Q6_K); }
     else if (ta == PM_Q8_0 || tb == PM_Q8_0) return -1;      // (Q8_0 only as a launch of its own: ffn_down of the files whose n_ff is no multiple of 256)
     else if (ta == PM_Q4_K && tb == PM_Q5_K) PF_GO(PM_Q4_K, PM_Q5_K);

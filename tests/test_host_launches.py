@@ -326,3 +326,33 @@ for K in (4352, 8192):
 assert grid(4096, 8, at, None) == grid(4096, 8, at + (1 << 20), None) == (8, 1) and grid(8192, 129, at + (1 << 30), None) == (129, 1)
 print("ok")
 """)
+
+
+def test_a_tile_that_there_is_no_kernel_for_is_not_forced(run):
+    """PM355_GEMM_PF_NT names the 256-row tiles' sub-tiles of 32 tokens, 2, 4, 6 or 8: with another value a prompt product has the tiles that its tokens ask for (3: grids of 96 tokens in front of the
+    64-token kernel, a third of the tokens never written)"""
+    run(COMMON + r"""
+import os
+def products(nt):
+    r, w = os.pipe()
+    if os.fork() == 0:
+        os.environ["PM355_GEMM_PF_NT"] = nt
+        lib = C.CDLL(sys.argv[2])
+        f = lib.pm355_mul_mat_q_mfma
+        f.argtypes = [C.c_int, C.c_void_p, C.c_int64, C.c_int64, C.c_void_p, C.c_int64, C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p]
+        at = C.addressof(C.create_string_buffer(256))
+        out = []
+        for t, K, N, T in ((12, 4096, 4096, 300), (14, 14336, 4096, 101), (8, 896, 512, 40), (12, 4096, 28672, 1500)):
+            shim.shim_forget()
+            assert f(t, at, K, N, at, T, at, None, None, 1) == 0, (t, K, N, T)
+            out.append([(n, g) for _, n, g in launches() if "gemm_pf" in n or "pf_reduce" in n])
+        os.write(w, repr(out).encode()); os._exit(0)
+    os.close(w)
+    return eval(b"".join(iter(lambda: os.read(r, 65536), b"")).decode())
+plain, three = products("1"), products("3")
+assert len(plain) == 4 and all(len(x) in (1, 2) for x in plain), plain
+assert products("5") == products("9") == plain
+assert three == plain, three
+assert products("4") != plain and all(re.search(r"gemm_pf_kernel<\d+, \d+, 4,", x[0][0]) for x in products("4")), products("4")
+print("ok")
+""")
