@@ -216,7 +216,7 @@ __global__ __launch_bounds__(512) void attn_cached_q8k_kernel(const float * q0, 
 int pm_launch_attn_cached_q8k(const float * q, void * kc, void * vc, const int32_t * pos, const int32_t * seq, long seq_stride, int H, int Hkv, int dh, int n_ctx, float scale, hipStream_t st,
                               int max_cells, int n_tok, const pm_q8k_out & out) {
     const int kpl = max_cells <= 64 ? 1 : max_cells <= 128 ? 2 : 4;
-    if (dh != 128 || H % 2 || n_ctx % 8 || n_tok < 1 || max_cells < 1 || max_cells > 256 || n_ctx < 64 * kpl || !pos || !seq) return -1;
+    if (dh != 128 || Hkv < 1 || H < Hkv || H % 2 || n_ctx % 8 || n_tok < 1 || max_cells < 1 || max_cells > 256 || n_ctx < 64 * kpl || !pos || !seq) return -1;
     AttnP a = {q, nullptr, nullptr, (uint16_t *) kc, (uint16_t *) vc, pos, seq, seq_stride, nullptr, nullptr, H, Hkv, n_ctx, scale, RopeP(), nullptr, nullptr, 0, nullptr, 0, 1};
     const size_t lds = 2 * (size_t) (kpl == 1 ? ShortLds<128, 1>::BYTES : kpl == 2 ? ShortLds<128, 2>::BYTES : ShortLds<128, 4>::BYTES);
     pm_allow_big_lds((const void *) attn_cached_q8k_kernel, lds);
@@ -236,7 +236,7 @@ void pm_launch_rope_table(const pm_rope_cfg & c, const int32_t * pos, const int3
 int pm_launch_attn_cached(const float * q, void * kc, void * vc, const int32_t * pos0, const int32_t * seq, long seq_stride, float * out,
                           int H, int Hkv, int dh, int n_ctx, float scale, hipStream_t st, const int32_t * dyn, const void * mask,
                           int max_keys, int v_rowmajor, int mask_f16, int n_tok, int rows) {
-    if ((dh != 64 && dh != 128 && dh != 256) || n_ctx % 8 || n_tok < 1 || H > 65535 || Hkv > 65535 || (n_tok > 1 && dyn) || (rows && (dyn || !seq || !pos0))) return -1;
+    if ((dh != 64 && dh != 128 && dh != 256) || Hkv < 1 || H < Hkv || n_ctx % 8 || n_tok < 1 || H > 65535 || Hkv > 65535 || (n_tok > 1 && dyn) || (rows && (dyn || !seq || !pos0))) return -1;
     size_t lds = (size_t) (4 * dh + (v_rowmajor ? 2048 : 256) + (max_keys > 0 ? ((max_keys + 7) & ~7) : n_ctx) + 8) * 4;
     if (lds > 150 * 1024) return -1;
     // (two workgroups of the largest short form per CU, as many as their registers allow)

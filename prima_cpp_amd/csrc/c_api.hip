@@ -466,7 +466,7 @@ int pm355_attn_cached(const float * q_rot, void * kc, void * vc, const int32_t *
     if (!q_rot || !kc || !vc || !out || (!d_pos && !d_cell_nkv)) return fail(PM355_E_SHAPE, "attn_cached: null pointer");
     if (pm_launch_attn_cached(q_rot, kc, vc, d_pos, nullptr, 0, out, H, Hkv, dh, n_ctx, kq_scale, S(st), d_cell_nkv, mask, max_keys,
                               flags & PM355_ATTN_V_ROWMAJOR, flags & PM355_ATTN_MASK_F16))
-        return fail(PM355_E_UNSUPPORTED, "attn_cached: head_dim must be 64/128/256, n_ctx % 8 == 0 and max_keys fit LDS");
+        return fail(PM355_E_UNSUPPORTED, "attn_cached: head_dim must be 64/128/256, at least as many heads as KV heads, n_ctx % 8 == 0 and max_keys fit LDS");
     HIP_TRY(hipGetLastError());
     return 0;
 }

@@ -356,3 +356,28 @@ assert three == plain, three
 assert products("4") != plain and all(re.search(r"gemm_pf_kernel<\d+, \d+, 4,", x[0][0]) for x in products("4")), products("4")
 print("ok")
 """)
+
+
+CACHED = COMMON + r"""
+lib = C.CDLL(sys.argv[2])
+f = lib.pm355_attn_cached
+f.argtypes = [C.c_void_p] * 7 + [C.c_int] * 4 + [C.c_float, C.c_int, C.c_int, C.c_void_p]
+at = C.addressof(C.create_string_buffer(256))
+def cached(H, Hkv, dh=64, n_ctx=64):
+    shim.shim_forget()
+    return f(at, at, at, at, None, None, at, H, Hkv, dh, n_ctx, 0.125, 0, 0, 1), [(n, g) for _, n, g in launches()]
+"""
+
+
+def test_cached_attention_of_heads_that_share_nothing_is_refused(run):
+    """no KV heads, or more of them than heads: an error code, no launch, no division by zero on the host"""
+    run(CACHED + r"""
+for H, Hkv in ((8, 0), (8, -1), (4, 8), (0, 0), (0, 8)):
+    for dh in (64, 128, 256):
+        rc, seen = cached(H, Hkv, dh)
+        assert rc and not seen, (H, Hkv, dh, rc, seen)
+for H, Hkv in ((8, 8), (8, 1), (6, 2)):
+    rc, seen = cached(H, Hkv)
+    assert rc == 0 and len(seen) == 1, (H, Hkv, rc, seen)
+print("ok")
+""")
