@@ -150,13 +150,15 @@ static CachedArgs cached_args(const AttnP & a) {
     return CachedArgs{(uint32_t) a.H | (uint32_t) a.Hkv << 16, R == 1 ? 0u : (uint32_t) (((1ull << 32) + R - 1) / R), (a.rows ? 1 : 0) | (a.dyn ? 2 : 0)};
 }
 __device__ __forceinline__ int kv_head(int h, uint32_t inv) { return inv ? (int) __umulhi((uint32_t) h, inv) : h; }      // (exact: heads x heads per KV head < 2^32)
-template <int DH, int VM>
+// MANY: more heads than 16 bits of an argument hold, and the division
+template <int DH, int VM, bool MANY = false>
 __global__ __launch_bounds__(256) void attn_cached_kernel(const float * q0, uint16_t * kc0, uint16_t * vc0, const int32_t * pos0, const int32_t * seq0, uint32_t heads, uint32_t inv, int n_ctx0, int how, AttnP a_in) {
     // grid.y = tokens of a small batch (engine: 2..64-token steps after rope_kv_store has rotated / rounded q and stored every token's K / V):
     // token t attends cells [0, pos0 + t], its q / out rows are t * H * DH further on
     // (the leading arguments: CachedArgs; the rest, dyn and the output among them, is read behind the first loads)
     AttnP a = a_in;
-    a.q = q0; a.kc = kc0; a.vc = vc0; a.pos0_ptr = pos0; a.seq_ptr = seq0; a.H = (int) (heads & 65535); a.Hkv = (int) (heads >> 16); a.n_ctx = n_ctx0; a.rows = how & 1;
+    a.q = q0; a.kc = kc0; a.vc = vc0; a.pos0_ptr = pos0; a.seq_ptr = seq0; a.n_ctx = n_ctx0; a.rows = how & 1;
+    if constexpr (!MANY) { a.H = (int) (heads & 65535); a.Hkv = (int) (heads >> 16); }
     a.tok = (int) blockIdx.y;
     a.q += (long) a.tok * a.H * DH; a.out += (long) a.tok * a.H * DH;
     extern __shared__ __attribute__((aligned(16))) char smem[];
@@ -165,7 +167,7 @@ __global__ __launch_bounds__(256) void attn_cached_kernel(const float * q0, uint
     const int h = blockIdx.x;
     if constexpr (VM == 0) {
         const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-        const int Hkv = a.Hkv, hk = kv_head(h, inv), n_ctx = a.n_ctx;
+        const int Hkv = a.Hkv, hk = MANY ? h / (a.H / Hkv) : kv_head(h, inv), n_ctx = a.n_ctx;
         int seq = 0, n_kv;
         if (how & 2) n_kv = uniform_const_ptr(a.dyn)[1];
         else {
@@ -216,7 +218,7 @@ __global__ __launch_bounds__(512) void attn_cached_q8k_kernel(const float * q0, 
 int pm_launch_attn_cached_q8k(const float * q, void * kc, void * vc, const int32_t * pos, const int32_t * seq, long seq_stride, int H, int Hkv, int dh, int n_ctx, float scale, hipStream_t st,
                               int max_cells, int n_tok, const pm_q8k_out & out) {
     const int kpl = max_cells <= 64 ? 1 : max_cells <= 128 ? 2 : 4;
-    if (dh != 128 || Hkv < 1 || H < Hkv || H % 2 || n_ctx % 8 || n_tok < 1 || max_cells < 1 || max_cells > 256 || n_ctx < 64 * kpl || !pos || !seq) return -1;
+    if (dh != 128 || Hkv < 1 || H < Hkv || H > 65535 || H % 2 || n_ctx % 8 || n_tok < 1 || max_cells < 1 || max_cells > 256 || n_ctx < 64 * kpl || !pos || !seq) return -1;
     AttnP a = {q, nullptr, nullptr, (uint16_t *) kc, (uint16_t *) vc, pos, seq, seq_stride, nullptr, nullptr, H, Hkv, n_ctx, scale, RopeP(), nullptr, nullptr, 0, nullptr, 0, 1};
     const size_t lds = 2 * (size_t) (kpl == 1 ? ShortLds<128, 1>::BYTES : kpl == 2 ? ShortLds<128, 2>::BYTES : ShortLds<128, 4>::BYTES);
     pm_allow_big_lds((const void *) attn_cached_q8k_kernel, lds);
@@ -236,7 +238,7 @@ void pm_launch_rope_table(const pm_rope_cfg & c, const int32_t * pos, const int3
 int pm_launch_attn_cached(const float * q, void * kc, void * vc, const int32_t * pos0, const int32_t * seq, long seq_stride, float * out,
                           int H, int Hkv, int dh, int n_ctx, float scale, hipStream_t st, const int32_t * dyn, const void * mask,
                           int max_keys, int v_rowmajor, int mask_f16, int n_tok, int rows) {
-    if ((dh != 64 && dh != 128 && dh != 256) || Hkv < 1 || H < Hkv || n_ctx % 8 || n_tok < 1 || H > 65535 || Hkv > 65535 || (n_tok > 1 && dyn) || (rows && (dyn || !seq || !pos0))) return -1;
+    if ((dh != 64 && dh != 128 && dh != 256) || Hkv < 1 || H < Hkv || n_ctx % 8 || n_tok < 1 || (n_tok > 1 && dyn) || (rows && (dyn || !seq || !pos0))) return -1;
     size_t lds = (size_t) (4 * dh + (v_rowmajor ? 2048 : 256) + (max_keys > 0 ? ((max_keys + 7) & ~7) : n_ctx) + 8) * 4;
     if (lds > 150 * 1024) return -1;
     // (two workgroups of the largest short form per CU, as many as their registers allow)
@@ -253,12 +255,13 @@ int pm_launch_attn_cached(const float * q, void * kc, void * vc, const int32_t *
         const CachedArgs c = cached_args(a);
         hipLaunchKernelGGL(kern, dim3(H, n_tok), dim3(256), lds, st, a.q, a.kc, a.vc, a.pos0_ptr, a.seq_ptr, c.heads, c.inv, a.n_ctx, c.how, a);
     };
+    auto go = [&](auto few, auto many) { if (H > 65535) launch(many); else launch(few); };
     if (v_rowmajor) {
-        if (dh == 64) launch(attn_cached_kernel<64, 1>);
-        else if (dh == 128) launch(attn_cached_kernel<128, 1>);
-        else launch(attn_cached_kernel<256, 1>);
-    } else if (dh == 64) launch(attn_cached_kernel<64, 0>);
-    else if (dh == 128) launch(attn_cached_kernel<128, 0>);
-    else launch(attn_cached_kernel<256, 0>);
+        if (dh == 64) go(attn_cached_kernel<64, 1>, attn_cached_kernel<64, 1, true>);
+        else if (dh == 128) go(attn_cached_kernel<128, 1>, attn_cached_kernel<128, 1, true>);
+        else go(attn_cached_kernel<256, 1>, attn_cached_kernel<256, 1, true>);
+    } else if (dh == 64) go(attn_cached_kernel<64, 0>, attn_cached_kernel<64, 0, true>);
+    else if (dh == 128) go(attn_cached_kernel<128, 0>, attn_cached_kernel<128, 0, true>);
+    else go(attn_cached_kernel<256, 0>, attn_cached_kernel<256, 0, true>);
     return 0;
 }

@@ -580,6 +580,24 @@ def test_attn_prefill_mfma_vs_exact(P, oracle, n_past, T, dh):
             assert np.abs(out[t, h] - want).max() <= 2e-3 * np.abs(want).max() + 1e-4, (t, h)
 
 
+@pytest.mark.parametrize("H,Hkv,n,rowmajor", [(65538, 32769, 36, False), (65537, 65537, 5, False), (131074, 65537, 40, True), (70000, 7, 300, False)])
+def test_cached_attention_of_more_heads_than_16_bits(P, H, Hkv, n, rowmajor):
+    """the bits of the same heads in calls of fewer"""
+    torch, dh, n_ctx, R = P.torch, 64, 320 if n > 64 else 64, H // Hkv
+    g = torch.Generator(device="cuda").manual_seed(H)
+    q = torch.randn((H, dh), generator=g, device="cuda").half().float()
+    K = torch.randn((n_ctx, Hkv, dh), generator=g, device="cuda").half()
+    V = torch.randn((n_ctx, Hkv, dh) if rowmajor else (Hkv, dh, n_ctx), generator=g, device="cuda").half()
+    pos = torch.tensor([n - 1], dtype=torch.int32, device="cuda")
+    go = lambda q, K, V, H, Hkv: P.attn_cached(q.contiguous(), K.contiguous(), V.contiguous(), pos, H, Hkv, dh, n_ctx, dh ** -0.5, flags=1 if rowmajor else 0)
+    out = go(q, K, V, H, Hkv)
+    c = Hkv // 3
+    for a, b in ((0, c), (c, 2 * c), (2 * c, Hkv)):
+        assert (b - a) * R <= 65535
+        want = go(q[a * R:b * R], K[:, a:b], V[:, a:b] if rowmajor else V[a:b], (b - a) * R, b - a)
+        assert torch.equal(out[a * R:b * R], want), (a, b)
+
+
 @pytest.mark.parametrize("H,Hkv,dh,T,past,mask", [
     (8, 2, 128, 1, 0, None), (8, 2, 64, 31, 1, None), (6, 3, 128, 33, 95, None), (8, 8, 64, 65, 127, None), (8, 1, 128, 130, 30, None),      # 64 queries per workgroup
     (64, 8, 128, 500, 12, None), (256, 32, 64, 128, 1, None),                                                                           # 128

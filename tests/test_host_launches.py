@@ -381,3 +381,13 @@ for H, Hkv in ((8, 8), (8, 1), (6, 2)):
     assert rc == 0 and len(seen) == 1, (H, Hkv, rc, seen)
 print("ok")
 """)
+
+
+def test_cached_attention_of_more_heads_than_16_bits(run):
+    run(CACHED + r"""
+for H, Hkv in ((65535, 65535), (65536, 1), (65536, 65536), (1 << 20, 1 << 10)):
+    for dh in (64, 128, 256):
+        rc, seen = cached(H, Hkv, dh)
+        assert rc == 0 and [g for _, g in seen] == [(H, 1, 1)] and ("true" in seen[0][0]) == (H > 65535), (H, Hkv, dh, rc, seen)
+print("ok")
+""")
