@@ -20,11 +20,18 @@
 // (Grids of rows x groups of four blocks, below of rows x 1024 values: by one index, split into row and block in 64 bits, every launch began with a division of a few hundred instructions in front of
 // its first load. us a pass before / now: eight sequences of the 8B shape, 96 launches of 8 rows of 14336 9056 / 9036;
 // two layers of the 72B shape at 23 tokens, silu_mul_q80_tab_kernel, 451.1 / 449.9)
+// FLAT: rows that fill less than half of a workgroup, by one index all the same (a division of 32 bits). us, rows x groups / flat: Q8_0 200000 rows of 32 45.7 / 6.9,
+// 8192 of 64 3.7 / 2.3, 8192 of 256 4.0 / 3.3, Q8_K 200000 of 256 65.0 / 52.9. From 512 values on rows x groups are faster (Q8_0 8192 of 512 4.6, by one index and 64 bits 5.2). And from 2^24 rows on, where a grid of rows ends
+template <bool FLAT>
 __global__ __launch_bounds__(256) void quantize_q8k_kernel(const float * __restrict__ x, uint8_t * __restrict__ y,
-                                                           int K, size_t y_row_bytes, pm_q8k_tables tb, pm_q8k_wide wd) {
+                                                           int K, int rows, size_t y_row_bytes, pm_q8k_tables tb, pm_q8k_wide wd) {
     const int lane = threadIdx.x & 63;
-    const int row = (int) blockIdx.x, blk = (int) blockIdx.y * 4 + __builtin_amdgcn_readfirstlane((int) threadIdx.x >> 6);
-    if (blk >= K / PM_QK_K) return;
+    int row = (int) blockIdx.x, blk = (int) blockIdx.y * 4 + __builtin_amdgcn_readfirstlane((int) threadIdx.x >> 6);
+    if constexpr (FLAT) {
+        const uint32_t nblk = (uint32_t) K / PM_QK_K, w = blockIdx.x * 4 + (uint32_t) __builtin_amdgcn_readfirstlane((int) threadIdx.x >> 6);
+        row = (int) (w / nblk); blk = (int) (w % nblk);
+        if (row >= rows) return;
+    } else if (blk >= K / PM_QK_K) return;
     const float4 f = ((const float4 *) (x + (size_t) row * K + (size_t) blk * PM_QK_K))[lane];
     const float v[4] = {f.x, f.y, f.z, f.w};
     q8k_block_from_regs(v, lane, y ? y + (size_t) row * y_row_bytes : nullptr, K, blk, tb, row, wd);
@@ -44,10 +51,15 @@ __global__ __launch_bounds__(256) void silu_mul_q8k_kernel(const float * __restr
 }
 
 // Q8_0: 32-value blocks, 8 lanes x 4 values; amax over the 8-lane group.
+template <bool FLAT>
 __global__ __launch_bounds__(256) void quantize_q80_kernel(const float * __restrict__ x, uint8_t * __restrict__ y,
-                                                           int K, size_t y_row_bytes) {
-    const int row = (int) blockIdx.x, i4 = (int) blockIdx.y * 256 + (int) threadIdx.x;        // one thread = 4 values
-    if (i4 >= K / 4) return;
+                                                           int K, int rows, size_t y_row_bytes) {
+    int row = (int) blockIdx.x, i4 = (int) blockIdx.y * 256 + (int) threadIdx.x;        // one thread = 4 values
+    if constexpr (FLAT) {
+        const uint32_t per_row = (uint32_t) K / 4, t = blockIdx.x * 256 + threadIdx.x;
+        row = (int) (t / per_row); i4 = (int) (t % per_row);
+        if (row >= rows) return;
+    } else if (i4 >= K / 4) return;
     const float4 f = ((const float4 *) (x + (size_t) row * K))[i4];
     float amax = fmaxf(fmaxf(fabsf(f.x), fabsf(f.y)), fmaxf(fabsf(f.z), fabsf(f.w)));
     amax = group8_max(amax);
@@ -172,15 +184,17 @@ static bool norm_split(const float * x, const float * ynorm, const void * yq, co
 }
 
 static dim3 q8k_grid(int K, int rows) { return dim3(rows, (K / PM_QK_K + 3) / 4); }
+static bool flat(int K, int rows) { return K < 512 || rows >= 1 << 24; }
 
 // ---- host launchers -------------------------------------------------------------------------------
+static void launch_quantize_q8k(const float * x, void * y, int K, int rows, hipStream_t st, size_t y_row_bytes, const pm_q8k_tables & tab, const pm_q8k_wide & wd) {
+    if (flat(K, rows)) hipLaunchKernelGGL(quantize_q8k_kernel<true>, dim3((unsigned) (((long) rows * (K / PM_QK_K) + 3) / 4)), dim3(256), 0, st, x, (uint8_t *) y, K, rows, y_row_bytes, tab, wd);
+    else               hipLaunchKernelGGL(quantize_q8k_kernel<false>, q8k_grid(K, rows), dim3(256), 0, st, x, (uint8_t *) y, K, rows, y_row_bytes, tab, wd);
+}
 void pm_launch_quantize_q8k(const float * x, void * y, int K, int rows, hipStream_t st, pm_q8k_tables tab) {
-    hipLaunchKernelGGL(quantize_q8k_kernel, q8k_grid(K, rows), dim3(256), 0, st,
-                       x, (uint8_t *) y, K, pm_q8k_row_bytes(K), tab, pm_q8k_wide());
+    launch_quantize_q8k(x, y, K, rows, st, pm_q8k_row_bytes(K), tab, pm_q8k_wide());
 }
-void pm_launch_quantize_wide(const float * x, const pm_q8k_wide & y, int K, int rows, hipStream_t st) {
-    hipLaunchKernelGGL(quantize_q8k_kernel, q8k_grid(K, rows), dim3(256), 0, st, x, (uint8_t *) nullptr, K, 0, pm_q8k_tables(), y);
-}
+void pm_launch_quantize_wide(const float * x, const pm_q8k_wide & y, int K, int rows, hipStream_t st) { launch_quantize_q8k(x, nullptr, K, rows, st, 0, pm_q8k_tables(), y); }
 void pm_launch_silu_mul_q8k(const float * gate, const float * up, void * y, int K, int rows, hipStream_t st, pm_q8k_tables tab) {
     hipLaunchKernelGGL(silu_mul_q8k_kernel, q8k_grid(K, rows), dim3(256), 0, st, gate, up, (uint8_t *) y, K, pm_q8k_row_bytes(K), tab);
 }
@@ -189,8 +203,8 @@ void pm_launch_silu_mul_q80_tab(const float * gate, const float * up, void * tab
                        qtab_bytes + dtab_bytes, qtab_bytes);
 }
 void pm_launch_quantize_q80(const float * x, void * y, int K, int rows, hipStream_t st) {
-    hipLaunchKernelGGL(quantize_q80_kernel, dim3(rows, (K / 4 + 255) / 256), dim3(256), 0, st,
-                       x, (uint8_t *) y, K, pm_q80_row_bytes(K));
+    if (flat(K, rows)) hipLaunchKernelGGL(quantize_q80_kernel<true>, dim3((unsigned) (((long) rows * (K / 4) + 255) / 256)), dim3(256), 0, st, x, (uint8_t *) y, K, rows, pm_q80_row_bytes(K));
+    else               hipLaunchKernelGGL(quantize_q80_kernel<false>, dim3(rows, (K / 4 + 255) / 256), dim3(256), 0, st, x, (uint8_t *) y, K, rows, pm_q80_row_bytes(K));
 }
 void pm_launch_rmsnorm_q8k(const float * x, const float * w, float * ynorm, void * yq, int K, int rows, float eps, hipStream_t st, void * ynorm_f16, pm_q8k_tables tab) {
     if (norm_split(x, ynorm, yq, ynorm_f16, K, rows)) hipLaunchKernelGGL((rmsnorm_q8k_kernel<16, true>), dim3(rows, 2), dim3(1024), 0, st, x, w, ynorm, (uint8_t *) yq, K, eps, pm_q8k_row_bytes(K), (_Float16 *) ynorm_f16, tab, pm_q8k_wide());

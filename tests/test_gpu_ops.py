@@ -73,6 +73,18 @@ def test_quantize_q8_0_bitexact(P, oracle, kind):
         assert np.array_equal(got[r], oracle.quantize_row_q8_0(x[r]))
 
 
+@pytest.mark.parametrize("K,rows", [(32, 1), (32, 1025), (96, 77), (256, 1), (256, 4099), (480, 501), (512, 130), (2080, 9)])
+def test_quantizers_of_short_rows_bitexact(P, oracle, K, rows):
+    """one index over rows and blocks (less than 512 values), rows x groups (the others): first, last and odd rows against the oracle"""
+    x = np.random.default_rng(K + rows).normal(0, 1, (rows, K)).astype(np.float32)
+    for t, row in ((Q8_0, oracle.quantize_row_q8_0), (Q8_K, oracle.quantize_row_q8_K)):
+        if t == Q8_K and K % 256:
+            continue
+        got = P.act_to_ggml_blocks(P.quantize_act(_dev(P, x), t), t, K, rows).reshape(rows, -1)
+        for r in sorted({*range(min(rows, 40)), *range(max(rows - 9, 0), rows), *range(0, rows, 97)}):
+            assert np.array_equal(got[r], row(x[r])), (t, r)
+
+
 @pytest.mark.parametrize("t", QUANT_TYPES)
 @pytest.mark.parametrize("K", [2048, 768])
 def test_repack_roundtrip_bitexact(P, t, K):

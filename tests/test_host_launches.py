@@ -391,3 +391,28 @@ for H, Hkv in ((65535, 65535), (65536, 1), (65536, 65536), (1 << 20, 1 << 10)):
         assert rc == 0 and [g for _, g in seen] == [(H, 1, 1)] and ("true" in seen[0][0]) == (H > 65535), (H, Hkv, dh, rc, seen)
 print("ok")
 """)
+
+
+def test_quantizers_of_short_rows_fill_their_workgroups(run):
+    """rows of less than 512 values, and more rows than a grid of rows has room for, by one index"""
+    run(COMMON + r"""
+lib = C.CDLL(sys.argv[2])
+at = C.addressof(C.create_string_buffer(256))
+def grid(name, K, rows):
+    f = getattr(lib, name)
+    f.argtypes = [C.c_void_p] * 2 + [C.c_int64, C.c_int64, C.c_void_p]
+    shim.shim_forget()
+    assert f(at, at, K, rows, 1) == 0
+    (_, _, g), = launches()
+    return g
+for rows in (1, 7, 200000, 16777215, 16777216, 20000000):
+    for K in (32, 64, 96, 256, 480):
+        assert grid("pm355_quantize_q8_0", K, rows) == (-(-rows * K // 1024), 1, 1), (K, rows)
+    assert grid("pm355_quantize_q8_K", 256, rows) == (-(-rows // 4), 1, 1), rows
+    for K in (512, 768):
+        many = rows >= 1 << 24
+        assert grid("pm355_quantize_q8_0", K, rows) == ((-(-rows * K // 1024), 1, 1) if many else (rows, 1, 1)), (K, rows)
+        assert grid("pm355_quantize_q8_K", K, rows) == ((-(-rows * K // 1024), 1, 1) if many else (rows, 1, 1)), (K, rows)
+assert grid("pm355_quantize_q8_0", 2080, 9) == (9, 3, 1) and grid("pm355_quantize_q8_K", 1280, 9) == (9, 2, 1)
+print("ok")
+""")
