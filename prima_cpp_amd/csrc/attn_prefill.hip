@@ -228,8 +228,10 @@ __global__ __launch_bounds__(256, 2) void attn_rowmajor_kernel(PfP p) {
 // PLAIN: caches that do not start on 16 bytes, by loads and LDS stores instead of DMA
 // PAIR: tiles of up to 32 queries, the two query waves of a key group are two heads of one KV head; their results leave as Q8_K blocks (the wo product's activations) - no f32 rows and no launch that
 // quantizes them: 8 tokens x 64 heads behind 403 cells 11.3 + 5.0 us, with this ending 13.3, with waves that bring 12.0; 23 tokens and no other cells 11.8 / 9.0
-template <int DH, int QW, int KS, bool MASK, bool PLAIN = false, bool PAIR = false>
-__global__ __launch_bounds__(768, 3) void attn_prompt_kernel(PfP p, pm_q8k_out y) {
+// SELF: no waves that bring, each of the eight requests its share of the next stage (launch_prompt says where)
+template <int DH, int QW, int KS, bool MASK, bool PLAIN = false, bool PAIR = false, bool SELF = false>
+__global__ __launch_bounds__(SELF ? 512 : 768, !SELF ? 3 : DH == 64 ? 4 : 2) void attn_prompt_kernel(PfP p, pm_q8k_out y) {
+    static_assert(!PAIR || !SELF, "the waves that bring store rows too");
     static_assert(!PAIR || (DH == 128 && QW == 2 && !MASK && !PLAIN), "two heads are a block");
     constexpr int KW = 8 / QW, KT = KS / KW, ST = KT / 32;            // keys per wave and stage, 32-key score tiles
     constexpr int KK = DH / 16, DT = DH / 32, CK = DH / 8, CV = KS / 8;      // k-steps of a score tile, output tiles, 16-byte chunks per K row / V^T row
@@ -271,20 +273,22 @@ __global__ __launch_bounds__(768, 3) void attn_prompt_kernel(PfP p, pm_q8k_out y
         if constexpr (PLAIN) { u32x4 v; __builtin_memcpy(&v, base + off, 16); *(u32x4 *) (smem + to + lane * 16) = v; }
         else pm_dma16(base, off, lds0 + to);
     };
-    // a stage: every fourth piece of 1 KiB by each of the loaders
+    // a stage: every RW-th piece of 1 KiB by each of the waves that request
+    constexpr int RW = SELF ? 8 : 4;
+    const int rw = SELF ? wave : wave - 8;
     auto request = [&](int it, int stage) __attribute__((always_inline)) {
         const char * kb = (const char *) (kc + (long) it * KS * krow), * vb = (const char *) vc;
         const int key0 = it * KS, kmax = p.n_ctx - 1 - key0, vmax = p.n_ctx - 8 - key0;          // (cells behind the cache: its last ones, masked)
 #pragma unroll
-        for (int i = 0; i < KS * DH * 2 / 4096; ++i) {
-            const int o = (wave - 8 + i * 4) * 64 + lane, row = o / CK, ch = o % CK;
-            bring(kb, (uint32_t) min(row, kmax) * (uint32_t) (krow * 2) + (uint32_t) (ch ^ (CK == 8 ? (row >> 1) & 7 : row & 15)) * 16u, stage * STAGE + (wave - 8 + i * 4) * 1024);
+        for (int i = 0; i < KS * DH * 2 / (1024 * RW); ++i) {
+            const int o = (rw + i * RW) * 64 + lane, row = o / CK, ch = o % CK;
+            bring(kb, (uint32_t) min(row, kmax) * (uint32_t) (krow * 2) + (uint32_t) (ch ^ (CK == 8 ? (row >> 1) & 7 : row & 15)) * 16u, stage * STAGE + (rw + i * RW) * 1024);
         }
 #pragma unroll
-        for (int i = 0; i < KS * DH * 2 / 4096; ++i) {
-            const int o = (wave - 8 + i * 4) * 64 + lane, row = o / CV, ch = o % CV;
+        for (int i = 0; i < KS * DH * 2 / (1024 * RW); ++i) {
+            const int o = (rw + i * RW) * 64 + lane, row = o / CV, ch = o % CV;
             const int key = key0 + min((ch ^ (CV == 8 ? (row >> 1) & 7 : row & 15)) * 8, vmax);
-            bring(vb, (uint32_t) row * (uint32_t) (p.n_ctx * 2) + (uint32_t) key * 2u, stage * STAGE + KS * DH * 2 + (wave - 8 + i * 4) * 1024);
+            bring(vb, (uint32_t) row * (uint32_t) (p.n_ctx * 2) + (uint32_t) key * 2u, stage * STAGE + KS * DH * 2 + (rw + i * RW) * 1024);
         }
     };
     float * const ex = (float *) smem, * const ml = ex + 8 * 32 * OS;      // behind the loop: [wave][query][DH + 4], [wave][query]{m, l}
@@ -301,7 +305,8 @@ __global__ __launch_bounds__(768, 3) void attn_prompt_kernel(PfP p, pm_q8k_out y
             q8k_block_from_regs(v, lane, y.y + (size_t) (row0 + r) * y.row_bytes, p.H * DH, pair, y.tab, row0 + r);
         }
     };
-    if (wave >= 8) {
+    if constexpr (SELF) request(0, 0);
+    else if (wave >= 8) {
         request(0, 0);
         for (int it = 0; it < n_it; ++it) {
             pm_vm_drain();
@@ -342,7 +347,9 @@ __global__ __launch_bounds__(768, 3) void attn_prompt_kernel(PfP p, pm_q8k_out y
     const int kr = (lr & ~12) | ((lr & 4) << 1) | ((lr & 8) >> 1);
     for (int it = 0; it < n_it; ++it) {
         const int stage = it & 1;
+        if constexpr (SELF) pm_vm_drain();
         __syncthreads();
+        if constexpr (SELF) if (it + 1 < n_it) request(it + 1, stage ^ 1);
         const int key0 = it * KS + kw * KT;
         if (!live || key0 >= seen) continue;
         // cells behind the last attended one: a probability of 0 does not undo what they hold (0 x NaN), so they become zeros in LDS. Every wave of a key group writes the same bytes and
@@ -473,11 +480,18 @@ __global__ __launch_bounds__(768, 3) void attn_prompt_kernel(PfP p, pm_q8k_out y
     }
 }
 
+template <int DH, int QW, int KS, bool MASK, bool PLAIN = false, bool PAIR = false, bool SELF = false> void launch_form(const PfP & p, hipStream_t st, const pm_q8k_out & y) {
+    constexpr size_t stages = 2 * (size_t) KS * DH * 4, ex = (size_t) 8 * 32 * (DH + 4) * 4 + 8 * 32 * 2 * 4, lds = stages > ex ? stages : ex;
+    pm_allow_big_lds((const void *) attn_prompt_kernel<DH, QW, KS, MASK, PLAIN, PAIR, SELF>, lds);
+    hipLaunchKernelGGL((attn_prompt_kernel<DH, QW, KS, MASK, PLAIN, PAIR, SELF>), dim3(p.n_tiles * (PAIR ? p.H / 2 : p.H)), dim3(SELF ? 512 : 768), lds, st, p, y);
+}
+// Heads of 64: eight waves of up to 128 registers and half of the LDS leave room for a second workgroup on a CU, eight waves and four that bring do not. Where there are more workgroups than CUs, two
+// at a time win. us, waves that bring / two workgroups: 48 heads x 640 tokens 15.1 / 14.1, 64 x 1000 27.5 / 25.6, 96 x 2048
+// 92.0 / 83.5, with a mask 48 x 512 behind 1024 cells 57.4 / 43.9. With a mask, tiles of 128 and 256 queries took 130 and 136 registers, one workgroup: 64 x 1000 66.2, with waves that bring 65.1
 template <int DH, int QW, int KS, bool MASK, bool PLAIN = false, bool PAIR = false> void launch_prompt(PfP p, hipStream_t st, const pm_q8k_out & y = {}) {
     if (!p.tiles) p.n_tiles = (p.T + QW * 32 - 1) / (QW * 32);
-    constexpr size_t stages = 2 * (size_t) KS * DH * 4, ex = (size_t) 8 * 32 * (DH + 4) * 4 + 8 * 32 * 2 * 4, lds = stages > ex ? stages : ex;
-    pm_allow_big_lds((const void *) attn_prompt_kernel<DH, QW, KS, MASK, PLAIN, PAIR>, lds);
-    hipLaunchKernelGGL((attn_prompt_kernel<DH, QW, KS, MASK, PLAIN, PAIR>), dim3(p.n_tiles * (PAIR ? p.H / 2 : p.H)), dim3(768), lds, st, p, y);
+    if constexpr (DH == 64 && (!MASK || QW == 2)) if ((long) p.n_tiles * p.H > pm_device_cus()) return launch_form<DH, QW, KS, MASK, PLAIN, PAIR, true>(p, st, y);
+    launch_form<DH, QW, KS, MASK, PLAIN, PAIR>(p, st, y);
 }
 // Which tile: a CU holds one workgroup. 256 queries share a stage where that still makes two rounds of workgroups (2048 tokens x 64 heads: 102 us, 110 with 128 queries; x 32 heads
 // = one round whose longest tile decides: 80 against 57); 128 queries where they make one (512 x 64 behind 1024 cached: 38 against 50 with 64); below that 64 queries with four key

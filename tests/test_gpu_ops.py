@@ -648,6 +648,12 @@ def test_attn_prefill_tiles_against_float64(P, H, Hkv, dh, T, past, mask):
         assert bool((off <= bound).all()), (h, float((off / bound).max()))
 
 
+@pytest.mark.parametrize("H,Hkv,T,past,mask", [(40, 8, 400, 33, None), (64, 8, 800, 5, None), (48, 8, 400, 101, "f32"), (96, 8, 200, 0, "f16")])
+def test_attn_prefill_of_64_wide_heads_two_workgroups_to_a_cu(P, H, Hkv, T, past, mask):
+    """more workgroups than CUs: the form whose waves request for themselves, 64 and 128 queries (256: 128 heads x 1000 above)"""
+    test_attn_prefill_tiles_against_float64(P, H, Hkv, 64, T, past, mask)
+
+
 def _masked_attention(P, q, K, V, m, n_kv, H, Hkv, dh, n_ctx, sc):
     import ctypes as C
     from prima_cpp_amd import lib as L
@@ -686,7 +692,8 @@ def test_attn_prefill_does_not_look_behind_the_attended_cells(P, H, Hkv, dh, T, 
 
 
 @pytest.mark.parametrize("off", [1, 4])
-@pytest.mark.parametrize("H,Hkv,dh,T,past,mask", [(8, 2, 128, 40, 60, False), (8, 4, 64, 70, 130, False), (8, 2, 64, 33, 0, True), (8, 2, 128, 130, 0, True)])
+@pytest.mark.parametrize("H,Hkv,dh,T,past,mask", [(8, 2, 128, 40, 60, False), (8, 4, 64, 70, 130, False), (8, 2, 64, 33, 0, True), (8, 2, 128, 130, 0, True),
+                                                    (48, 8, 64, 350, 20, False), (48, 8, 64, 350, 0, True)])
 def test_attn_prefill_of_caches_that_do_not_start_on_16_bytes(P, H, Hkv, dh, T, past, mask, off):
     """views that begin 2 or 8 bytes into a buffer: the same bits as caches that start on 16"""
     torch = P.torch

@@ -416,3 +416,37 @@ for rows in (1, 7, 200000, 16777215, 16777216, 20000000):
 assert grid("pm355_quantize_q8_0", 2080, 9) == (9, 3, 1) and grid("pm355_quantize_q8_K", 1280, 9) == (9, 2, 1)
 print("ok")
 """)
+
+
+PROMPT_ATTENTION = COMMON + r"""
+lib = C.CDLL(sys.argv[2])
+at = C.addressof(C.create_string_buffer(256)) // 16 * 16 + 16
+f, fm = lib.pm355_attn_prefill, lib.pm355_attn_prefill_masked_ex
+f.argtypes = [C.c_void_p] * 5 + [C.c_int] * 5 + [C.c_float, C.c_void_p]
+fm.argtypes = [C.c_void_p] * 4 + [C.c_int64, C.c_void_p] + [C.c_int] * 6 + [C.c_float, C.c_int, C.c_void_p]
+def form(H, dh, T, mask=False, off=0):
+    "(query waves, its waves request themselves, workgroups)"
+    shim.shim_forget()
+    k = at + off
+    rc = fm(at, k, k, at, 4096, at, T, H, 8, dh, 4096, 4096, 0.1, 0, 1) if mask else f(at, k, k, at, at, T, H, 8, dh, 4096, 0.1, 1)
+    assert rc == 0
+    (_, n, g), = launches()
+    a = re.search(r"attn_prompt_kernel<(.*)>", n).group(1).split(", ")
+    assert a[0] == str(dh) and a[3] == str(mask).lower() and a[4] == str(bool(off)).lower() and g[1:] == (1, 1), n
+    return int(a[1]), a[6] == "true", g[0]
+"""
+
+
+def test_heads_of_64_leave_room_for_two_workgroups_where_there_are_more_than_cus(run):
+    run(PROMPT_ATTENTION + r"""
+for H in (8, 24, 40, 48, 64, 96):
+    for T in (40, 400, 640, 1000, 2048, 4000):
+        for off in (0, 8):
+            q, own, n = form(H, 64, T, off=off)
+            assert q == (2 if off else 8 if -(-T // 256) * H >= 512 else 4 if -(-T // 128) * H >= 256 else 2) and n == -(-T // (32 * q)) * H
+            assert own == (n > 256), (H, T, off, q, n)
+            q, own, n = form(H, 64, T, True, off)
+            assert own == (n > 256 and q == 2), (H, T, off, q, n)
+            assert not form(H, 128, T, off=off)[1]
+print("ok")
+""")
