@@ -488,10 +488,12 @@ template <int DH, int QW, int KS, bool MASK, bool PLAIN = false, bool PAIR = fal
 // Heads of 64: eight waves of up to 128 registers and half of the LDS leave room for a second workgroup on a CU, eight waves and four that bring do not. Where there are more workgroups than CUs, two
 // at a time win. us, waves that bring / two workgroups: 48 heads x 640 tokens 15.1 / 14.1, 64 x 1000 27.5 / 25.6, 96 x 2048
 // 92.0 / 83.5, with a mask 48 x 512 behind 1024 cells 57.4 / 43.9. With a mask, tiles of 128 and 256 queries took 130 and 136 registers, one workgroup: 64 x 1000 66.2, with waves that bring 65.1
+// Heads of 128 with a mask, tiles of 128 and 256 queries: 168 registers a wave, what waves that bring leave, are too few (186 and 196 without). us, with them (two spilled) / without: 64 heads
+// x 1000 tokens 85.3 / 87.4, 64 x 512 behind 1024 cells 64.6 / 64.4, 48 x 2500 417 / 406, 64 x 2500 583 / 571, 128 x 2500 1168 / 1013
 template <int DH, int QW, int KS, bool MASK, bool PLAIN = false, bool PAIR = false> void launch_prompt(PfP p, hipStream_t st, const pm_q8k_out & y = {}) {
     if (!p.tiles) p.n_tiles = (p.T + QW * 32 - 1) / (QW * 32);
     if constexpr (DH == 64 && (!MASK || QW == 2)) if ((long) p.n_tiles * p.H > pm_device_cus()) return launch_form<DH, QW, KS, MASK, PLAIN, PAIR, true>(p, st, y);
-    launch_form<DH, QW, KS, MASK, PLAIN, PAIR>(p, st, y);
+    launch_form<DH, QW, KS, MASK, PLAIN, PAIR, DH == 128 && MASK && QW != 2>(p, st, y);
 }
 // Which tile: a CU holds one workgroup. 256 queries share a stage where that still makes two rounds of workgroups (2048 tokens x 64 heads: 102 us, 110 with 128 queries; x 32 heads
 // = one round whose longest tile decides: 80 against 57); 128 queries where they make one (512 x 64 behind 1024 cached: 38 against 50 with 64); below that 64 queries with four key

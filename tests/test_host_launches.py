@@ -1,5 +1,6 @@
 """What the library's host code launches, and in what order, on the CPU: in a process of its own, in front of a HIP runtime that runs nothing (hip_shim.cpp)."""
 import os
+import re
 import subprocess
 import sys
 
@@ -448,5 +449,33 @@ for H in (8, 24, 40, 48, 64, 96):
             q, own, n = form(H, 64, T, True, off)
             assert own == (n > 256 and q == 2), (H, T, off, q, n)
             assert not form(H, 128, T, off=off)[1]
+            q, own, n = form(H, 128, T, True, off)      # (with a mask, tiles of 128 and 256 queries: registers)
+            assert own == (q > 2), (H, T, off, q, n)
 print("ok")
 """)
+
+
+def test_prompt_attention_keeps_its_registers(tmp_path):
+    """no kernel of it has registers spilled: what the compiler wrote beside the kernels of the library built here"""
+    readelf = "/opt/rocm/llvm/bin/llvm-readelf"
+    if not os.path.exists(LIB) or not os.path.exists(readelf):
+        pytest.skip("library not built, or no tool to read it")
+    blob, seen = open(LIB, "rb").read(), {}
+    at = blob.find(b"__CLANG_OFFLOAD_BUNDLE__")
+    while at >= 0:                                          # magic, number of entries, then (offset, size, length of the name, name) of each
+        n, p = int.from_bytes(blob[at + 24:at + 32], "little"), at + 32
+        for _ in range(n):
+            off, size, k = (int.from_bytes(blob[p + 8 * i:p + 8 * i + 8], "little") for i in range(3))
+            name, p = blob[p + 24:p + 24 + k], p + 24 + k
+            obj = blob[at + off:at + off + size]
+            if b"gfx950" in name and b"attn_prompt_kernel" in obj:
+                f = tmp_path / "device.o"
+                f.write_bytes(obj)
+                notes = subprocess.run([readelf, "--notes", str(f)], capture_output=True, text=True, check=True).stdout
+                for kernel in notes.split(".agpr_count")[1:]:
+                    field = lambda key: re.search(key + r":\s+(\S+)", kernel).group(1)  # noqa: E731
+                    seen[field(r"\.name")] = int(field(r"\.vgpr_spill_count")), int(field(r"\.private_segment_fixed_size"))
+        at = blob.find(b"__CLANG_OFFLOAD_BUNDLE__", at + 24)
+    seen = {k: v for k, v in seen.items() if "attn_prompt_kernel" in k}
+    assert len(seen) >= 16, len(seen)
+    assert not any(a or b for a, b in seen.values()), {k: v for k, v in seen.items() if v != (0, 0)}
