@@ -13,25 +13,25 @@ struct RowsP {
 };
 // What a launch's first loads need travels as leading arguments of 14 dwords, which the hardware places in registers before a wave starts; read from memory with the rest they stood in front of every
 // first load. us per launch at 8 tokens, before / now: 8B shape wq | wk | wv 7.9 / 7.0 (with a Q6_K wv 10.1 / 9.0), wo 5.7 / 5.3, ffn_down 12.6 / 10.9 (Q6_K 18.0 / 16.5); 70B shape wo and ffn_down
-// 16.6 / 16.3, wq | wk | wv 15.5 / 14.9. first: first workgroups of the second and third job, 16 bits each (65535: none); rows: each | more << 22; tokens: T | t_off << 8 | njobs << 16
+// 16.6 / 16.3, wq | wk | wv 15.5 / 14.9. first: first workgroups of the second and third job, 16 bits each (65535: none); rows: each | more << 24; tokens: T | t_off << 8 | njobs << 16
 struct RowsArgs { uint32_t first, rows[3], tokens; };
 inline RowsArgs pm_rows_args(const RowsP & p, int first1, int first2) {
     RowsArgs a;
     a.first = (uint32_t) (first1 < 65535 ? first1 : 65535) | (uint32_t) (first2 < 65535 ? first2 : 65535) << 16;
-    for (int j = 0; j < 3; ++j) a.rows[j] = (uint32_t) p.job[j].each | (uint32_t) p.job[j].more << 22;
+    for (int j = 0; j < 3; ++j) a.rows[j] = (uint32_t) p.job[j].each | (uint32_t) p.job[j].more << 24;
     a.tokens = (uint32_t) p.T | (uint32_t) p.t_off << 8 | (uint32_t) p.njobs << 16;
     return a;
 }
-// (a row of a weight is at least 16 bytes: one workgroup's 4 M rows of the smallest job beside its 255 others' would not fit the device; more < workgroups)
+// (more < workgroups of the matrix, at most one per CU. A row is at least 288 bytes, 512 values of Q4_K: a workgroup's 16 M rows, 4.8 GB, beside its 255 others' would be four times the device's memory)
 inline bool pm_rows_fit(const RowsP & p) {
-    for (int j = 0; j < p.njobs; ++j) if (p.job[j].each >= 1 << 22 || p.job[j].more >= 1 << 10) return false;
+    for (int j = 0; j < p.njobs; ++j) if (p.job[j].each >= 1 << 24 || p.job[j].more >= 1 << 8) return false;
     return true;
 }
 struct RowsStart { const uint8_t * W; int ji, w, each, more; };
 __device__ __forceinline__ RowsStart pm_rows_start(const uint8_t * W0, const uint8_t * W1, const uint8_t * W2, uint32_t first, uint32_t rows0, uint32_t rows1, uint32_t rows2, int b) {
     const int first1 = (int) (first & 65535), first2 = (int) (first >> 16), ji = (b >= first1) + (b >= first2);
     const uint32_t rows = ji == 0 ? rows0 : ji == 1 ? rows1 : rows2;
-    return RowsStart{ji == 0 ? W0 : ji == 1 ? W1 : W2, ji, b - (ji == 0 ? 0 : ji == 1 ? first1 : first2), (int) (rows & 0x3FFFFF), (int) (rows >> 22)};
+    return RowsStart{ji == 0 ? W0 : ji == 1 ? W1 : W2, ji, b - (ji == 0 ? 0 : ji == 1 ? first1 : first2), (int) (rows & 0xFFFFFF), (int) (rows >> 24)};
 }
 __device__ __forceinline__ void pm_rows_take(RowsP & p, const uint8_t * qT, int K, uint32_t tokens) { p.qT = qT; p.K = K; p.T = (int) (tokens & 255); p.t_off = (int) (tokens >> 8 & 255); p.njobs = (int) (tokens >> 16); }
 template <int TYPE> __device__ __forceinline__ size_t pm_rows_stride(int nb) {

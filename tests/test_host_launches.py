@@ -479,3 +479,26 @@ def test_prompt_attention_keeps_its_registers(tmp_path):
     seen = {k: v for k, v in seen.items() if "attn_prompt_kernel" in k}
     assert len(seen) >= 16, len(seen)
     assert not any(a or b for a, b in seen.values()), {k: v for k, v in seen.items() if v != (0, 0)}
+
+
+def test_products_of_few_tokens_take_as_many_rows_as_memory_holds(run):
+    """a workgroup of more than 2^22 rows: a small matrix beside one of 220 GB, the longest that the device holds"""
+    run(COMMON + r"""
+lib = C.CDLL(sys.argv[2])
+at = C.addressof(C.create_string_buffer(256))
+one, several = lib.pm355_mul_mat_q_small, lib.pm355_mul_mat_q_small_multi
+one.argtypes = [C.c_int, C.c_void_p, C.c_int64, C.c_int64, C.c_void_p, C.c_void_p, C.c_int64, C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p]
+several.argtypes = [C.c_int, C.c_int] + [C.c_void_p] * 5 + [C.c_int64, C.c_int64, C.c_void_p]
+def products():
+    return [g for _, n, g in launches() if re.search(r"mmq_(rows|mid)_kernel", n)]
+for T in (2, 8, 30):
+    shim.shim_forget()
+    rc = one(12, at, 512, (1 << 30) - 1, at, None, T, at, None, None, 1)
+    assert rc == 0 and products() == [(256, 1, 1)], (T, rc)
+arr = lambda v, ty: (ty * len(v))(*v)
+for Ns in ([760000000, 4250000], [380000000, 380000000, 4250000], [1 << 20, 4250000]):
+    shim.shim_forget()
+    rc = several(12, len(Ns), arr([at] * len(Ns), C.c_void_p), arr(Ns, C.c_int64), arr([at] * len(Ns), C.c_void_p), None, at, 512, 4, 1)
+    assert rc == 0 and products() == [(256, 1, 1)], (Ns, rc)
+print("ok")
+""")
