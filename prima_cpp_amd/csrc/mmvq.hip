@@ -161,7 +161,7 @@ int pmv::gemv_fill(const pm_gemv_fused & a, int grid_fixed, GemvP & p, int & ta_
     }
     // a Q8_0 job needs Q8_0-quantized activations, the K-quants need Q8_K: one prologue serves only one family
     if ((ta == PM_Q8_0) != (tb == PM_Q8_0)) return -1;
-    if ((ta == PM_Q8_0 ? a.K % 32 : a.K % 256) || a.K >= 1 << 28) return -2;
+    if (ta == PM_Q8_0 ? a.K % 32 : a.K % 256) return -2;
     if (pair && ta != tb) return -1;
     if (ta != tb) {
         if (ta != PM_Q4_K) { const int t = ta; ta = tb; tb = t; }     // canonical order: Q4_K first
@@ -231,7 +231,7 @@ int pmv::gemv_fill(const pm_gemv_fused & a, int grid_fixed, GemvP & p, int & ta_
     const int ablk = ta == PM_Q8_0 ? 32 : 256;
     size_t lds = (size_t) ((a.K + 15) & ~15) + (size_t) (a.K / 16) * 4 + (size_t) ((a.K / ablk + 3) & ~3) * 4 + (size_t) rows_cap * 4;
     if (att_lds > lds) lds = att_lds;
-    if (lds > 150 * 1024) return -4;
+    if (lds > 150 * 1024) return -4;                  // (and so K < 2^28: an argument's bits)
     ta_out = ta; tb_out = tb; pair_out = pair; lds_out = lds; grid_out = grid;
     return 0;
 }

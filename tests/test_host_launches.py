@@ -502,3 +502,19 @@ for Ns in ([760000000, 4250000], [380000000, 380000000, 4250000], [1 << 20, 4250
     assert rc == 0 and products() == [(256, 1, 1)], (Ns, rc)
 print("ok")
 """)
+
+
+def test_a_mat_vec_of_rows_beyond_lds_says_so(run):
+    """K a multiple of the block size, however large: PM355_E_RANGE ("K too large"), not the error of a K that is no multiple"""
+    run(COMMON + r"""
+lib = C.CDLL(sys.argv[2])
+f = lib.pm355_mul_mat_vec_q
+f.argtypes = [C.c_int, C.c_void_p, C.c_void_p, C.c_int64, C.c_int64, C.c_void_p, C.c_int, C.c_void_p, C.c_int64, C.c_void_p, C.c_void_p, C.c_void_p]
+at = C.addressof(C.create_string_buffer(256))
+go = lambda t, K: f(t, at, None, K, 64, at, 1, at, 64, None, None, 1)
+for t in (12, 13, 14, 8):
+    assert go(t, 4096) == 0
+    want = go(t, 1 << 20)
+    assert want not in (0, go(t, 4097)) and all(go(t, K) == want for K in (1 << 24, 1 << 28, (1 << 28) + 256, 1 << 30)), (t, want, [go(t, K) for K in (1 << 24, 1 << 28, 1 << 30)])
+print("ok")
+""")
