@@ -269,10 +269,15 @@ int pm355_mul_mat_q_wide(const int * types, int njobs, const void * const * W, c
     HIP_TRY(hipGetLastError());
     return 0;
 }
-int pm355_gemm_plan(int64_t n_row_tiles, int64_t K, int64_t n_tokens, int n_cus, int allow_tail_split, int32_t * out5) {
+int pm355_gemm_plan(int64_t n_row_tiles, int64_t K, int64_t n_tokens, int n_cus, int flags, int32_t * out5) {
     if (n_row_tiles < 1 || K < 256 || n_tokens < 1 || n_cus < 8 || !out5) return fail(PM355_E_RANGE, "gemm_plan: n_row_tiles >= 1, K >= 256, n_tokens >= 1, n_cus >= 8");
+    const int forms[] = {PM355_GEMM_ROWS_256, PM355_GEMM_ROWS_128, PM355_GEMM_WIDE_Q4_K, PM355_GEMM_WIDE}, as[] = {PM_PF_ROWS_256, PM_PF_ROWS_128, PM_PF_WIDE, PM_PF_WIDE_TWO};
+    int form = PM_PF_BY_TOKENS, mixed = flags & 1;
+    for (int i = 0; i < 4; ++i) if (flags & forms[i]) { form = as[i]; mixed = 1; }
+    if (form == PM_PF_ROWS_128 && n_tokens > 128) return fail(PM355_E_RANGE, "gemm_plan: tiles of 128 rows serve up to 128 tokens");
+    if (form >= PM_PF_WIDE && n_tokens > PM_WIDE_MAX_TOKENS) return fail(PM355_E_RANGE, "gemm_plan: 8-bit activations of up to 512 tokens");
     pm_gemm_pf_plan_t pl;
-    pm_gemm_pf_plan((int) n_row_tiles, (int) K, (int) n_tokens, n_cus, 0, 0, allow_tail_split, &pl);
+    pm_gemm_pf_plan({(int) n_row_tiles, (int) K, (int) n_tokens, n_cus, form, PM_WIDE_MAX_TOKENS, 0, 0, mixed}, &pl);
     out5[0] = pl.nt * 32; out5[1] = pl.nt_t; out5[2] = pl.splitk; out5[3] = pl.full; out5[4] = pl.grid;
     return 0;
 }

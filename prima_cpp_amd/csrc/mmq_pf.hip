@@ -1169,16 +1169,14 @@ int pm_gemm_pf_check(int type, int K, int N, int T) {
 }
 
 // The launch geometry of `tiles` row tiles (256 rows, 128 where mid_body runs; pair launches: half of that of each matrix) x T tokens over K on a device of `cus` CUs in 8 XCDs - host
-// arithmetic only (tests/test_gemm_plan.py plans the layer shapes without a device). nt: 32-token sub-tiles per workgroup tile (2 / 4 / 8 = 64 / 128 / 256, 6 on request
-// tokens: a dequantized operand serves nt MFMAs; smaller tiles only where the batch has no more tokens). Few tiles - wo / ffn_down / wq | wk | wv at the
+// arithmetic only (tests/test_gemm_plan.py plans the layer shapes without a device). nt: 32-token sub-tiles per workgroup tile (2, 3, 4, 6, 8 = 64, 96, 128, 192, 256 tokens: a dequantized
+// operand serves nt MFMAs). Few tiles - wo / ffn_down / wq | wk | wv at the
 // reference's default n_ubatch 512 (common/common.h:178) are 64-80 tiles for 256 CUs - are split along K: S slices per tile, the slice count that minimises
 // rounds of workgroups x (super-blocks per slice + ~3 for prologue, slab traffic and the launch that adds the slices up). A launch of R full rounds + a short tail (wq | wk | wv
 // at 2048 tokens: 320 tiles = 256 + 64; Qwen2.5-72B's ffn_gate | ffn_up: 1848 = 7 x 256 + 56) runs whole tiles in the full rounds and splits ONLY the tail's
 // tiles - as many slices as fill the idle CUs of the last round (`full` whole-tile slots per XCD come first in the grid). Splitting every tile instead sends
 // every partial tile through memory: 3 x 320 slabs of 256 KB for the qkv launch, 501 us = 685 TFLOP/s against 406 us = 846.
-void pm_gemm_pf_plan(int tiles, int K, int T, int cus, int force_nt, int force_s, int allow_mixed, pm_gemm_pf_plan_t * out) {
-    int nt = T <= 64 ? 2 : T <= 128 ? 4 : 8;
-    if ((force_nt >= 2 && force_nt <= 4) || force_nt == 6 || force_nt == 8) nt = force_nt;
+static void plan_tiles(int tiles, int K, int T, int cus, int nt, int force_s, int allow_mixed, pm_gemm_pf_plan_t * out) {
     const int nt_t = (T + 32 * nt - 1) / (32 * nt);
     const long wgs = (long) tiles * nt_t;
     const int nb = (K + 255) / 256;
@@ -1203,6 +1201,38 @@ void pm_gemm_pf_plan(int tiles, int K, int T, int cus, int force_nt, int force_s
     if (force_s >= 1 && force_s <= 8 && nb / force_s >= 1) { S = force_s; full = 0; }
     out->nt = nt; out->nt_t = nt_t; out->splitk = S; out->full = full; out->grid = 8 * (full + (maxL - full) * S); out->cost = best;
 }
+void pm_gemm_pf_plan(const pm_gemm_pf_ask & ask, pm_gemm_pf_plan_t * out) {
+    const int tiles = ask.tiles, K = ask.K, T = ask.T, cus = ask.cus, nb = (K + 255) / 256;
+    const bool mid = ask.form == PM_PF_ROWS_128, wide = ask.form == PM_PF_WIDE;
+    const int nt0 = T <= 64 || ask.form == PM_PF_WIDE_TWO ? 2 : T <= 96 && (mid || wide) ? 3 : T <= 128 || mid || wide ? 4 : 8;
+    plan_tiles(tiles, K, T, cus, ask.nt ? ask.nt : nt0, ask.splitk, ask.mixed, out);
+    if (ask.nt) return;
+    // 8-bit activations of Q4_K: tiles of 96 tokens (with loaders) where they cost less than those of 128 (without: no registers left for them), by rounds of workgroups; the K split stays that of
+    // 128 tokens: the sums in one order. 8B shape, whole passes, us, 128 / 96: 79 tokens 716 / 675, 109 738 / 801, 147 935 / 858, 231 1025 / 1095, 316 1279 / 1260, 459 1498 / 1570
+    if (wide && T > 64 && !out->full && (T + 95) / 96 * 96 <= ask.ldt) {
+        const auto cost = [&](int nt) { return ((long) tiles * ((T + 32 * nt - 1) / (32 * nt)) * out->splitk + cus - 1) / cus * (nt + 1); };
+        if (cost(3) < cost(4)) plan_tiles(tiles, K, T, cus, 3, out->splitk, 0, out);
+    }
+    // Tiles of 192 tokens where their rounds of workgroups cost less than those of 256: mostly 129..192, 257..384 and 513..576 tokens, whose rest of a tile of 256 was products of nothing. The K
+    // split stays, so every sum keeps its order; in place of a split of the last tiles only, whole ones. Both by full rounds and, as a last round that is not full runs faster, by the work in them;
+    // one round of 256-token workgroups that leaves CUs idle may become up to a tenth more work.
+    // us, 256 / 192: 8B shape ffn_gate | ffn_up Q4_K 150 tokens 79 / 66, 300 128 / 104 (512 137 / 160, 1000 284 / 317, 6001 1430 / 1475: not taken), 70B shape 300 454 / 376, 513 664 / 559,
+    // Q6_K ffn_down of 8B 380 85 / 72, Q8_0 ffn_down of 72B 513 371 / 319, wq | wk | wv of 8B 150 42 / 36, 1500 120 / 100, 6001 404 / 374 (a split tail before), wo 3000 137 / 122, 6001 285 / 251
+    if (ask.form == PM_PF_ROWS_256 && !ask.splitk && out->nt == 8) {
+        const int s6 = out->full ? 1 : out->splitk;
+        // workgroups / CUs, rounds and work in them, in sub-tiles of 32 tokens + 1
+        struct Cost { double rounds, work; };
+        const auto cost = [&](int nt) {
+            const int n = (T - 1) / (32 * nt), left = T - 32 * nt * n, last = nt == 6 || !n ? nt : left <= 128 ? 4 : left <= 192 ? 6 : 8;
+            const double w = (double) tiles * s6 / cus;
+            return Cost{std::ceil(w * (n + 1)) * (nt + 1), w * (n * (nt + 1) + last + 1)};
+        };
+        const Cost c6 = cost(6);
+        Cost c8 = cost(8);
+        if (out->full) c8.rounds = c8.work = 9.0 * out->cost / nb;
+        if (c6.rounds < 0.97 * c8.rounds && c6.work < (c8.rounds <= 9.0 ? 1.1 : 0.97) * c8.work) plan_tiles(tiles, K, T, cus, 6, s6, 0, out);
+    }
+}
 
 // One launch over njobs <= 4 matrices that share the F16 activations xh [T][K]. Job j: Y_j[t][n] (f32, token stride ldy_j) or Yh_j (F16) =
 // W_j . x (+bias)(+resid)(x silu(gate)). 0, or -1 type / -2 shape
@@ -1221,13 +1251,12 @@ static int launch_pf(const pm_gemm_pf_job * jobs, int njobs, const void * xh, co
     // 101 tokens 65.8 / 70, 128256 x 4096 (Q6_K) 209 / 235. Beyond 128 tokens mid_body is still the faster one (4096 x 4096: 256 tokens 55.8 / 26.6, 512 60 / 36) and not taken for its
     // results: it adds the halves of every 128 k in another order, and tokens decoded behind such a prompt then differ from those behind pf_body's by up to 3 % of their logits (eight layers of
     // the 8B shape; their 8-bit roundings turn), although neither is nearer to 64 bits
-    bool two = false;                                           // 8-bit activations: tiles of 64 tokens for what needs a second set of accumulators
+    bool two = false;                                           // 8-bit activations: tiles of 64 tokens for what needs a second set of accumulators (PM_PF_WIDE_TWO)
     for (int j = 0; j < njobs; ++j) two |= wide && jobs[j].type != PM_Q4_K;
-    const int mid_nt = T <= 64 || two ? 2 : T <= 96 ? 3 : 4;
     long mid_wgs = 0;
     for (int j = 0; j < njobs && !(pair && j); ++j) mid_wgs += (jobs[j].N + (pair ? 63 : 127)) / (pair ? 64 : 128);
     // (8-bit activations: mid_body at any size - its tiles of 128 tokens side by side -, pf_body's registers are its accumulators')
-    const bool mid = wide || (!force_nt && T <= 128 && mid_wgs <= cus);
+    const bool mid = wide || (!asked_nt && T <= 128 && mid_wgs <= cus);
     const int rows = mid ? 128 : 256;
     PfP p = {};
     p.pair = pair ? 1 : 0;
@@ -1249,36 +1278,8 @@ static int launch_pf(const pm_gemm_pf_job * jobs, int njobs, const void * xh, co
     if (wide) { p.Xd = (const uint8_t *) wide->d; p.Xs = (const uint8_t *) wide->s; p.ldt = wide->ldt; }
     static const int force_s = [] { const char * e = getenv("PM355_GEMM_PF_SPLITK"); return e ? atoi(e) : 0; }();
     static const bool no_mixed = [] { const char * e = getenv("PM355_GEMM_PF_MIXED"); return e && e[0] == '0'; }();
-    // 256-token tiles (a dequantized operand serves 8 MFMAs; 128-token tiles only where the batch has no more tokens). Few tiles - wo / ffn_down / wq | wk | wv
-    // at the reference's default n_ubatch 512 (common/common.h:178) are 64-80 tiles for 256 CUs - are split along K: S slices per tile, the slice count that
-    // minimises  rounds of workgroups x (super-blocks per slice + ~3 for prologue, slab traffic and the launch that adds the slices up)
     pm_gemm_pf_plan_t pl;
-    pm_gemm_pf_plan(tiles, K, T, cus, mid ? mid_nt : asked_nt, force_s, no_mixed ? 0 : 1, &pl);
-    // 8-bit activations of Q4_K: tiles of 96 tokens (with loaders) where they cost less than those of 128 (without: no registers left for them), by rounds of workgroups; the K split stays that of
-    // 128 tokens: the sums in one order. 8B shape, whole passes, us, 128 / 96: 79 tokens 716 / 675, 109 738 / 801, 147 935 / 858, 231 1025 / 1095, 316 1279 / 1260, 459 1498 / 1570
-    if (wide && !two && T > 64 && !pl.full && (T + 95) / 96 * 96 <= wide->ldt) {
-        const auto cost = [&](int nt) { return ((long) tiles * ((T + 32 * nt - 1) / (32 * nt)) * pl.splitk + cus - 1) / cus * (nt + 1); };
-        if (cost(3) < cost(4)) pm_gemm_pf_plan(tiles, K, T, cus, 3, pl.splitk, 0, &pl);
-    }
-    // Tiles of 192 tokens where their rounds of workgroups cost less than those of 256: mostly 129..192, 257..384 and 513..576 tokens, whose rest of a tile of 256 was products of nothing. The K
-    // split stays, so every sum keeps its order; in place of a split of the last tiles only, whole ones. Both by full rounds and, as a last round that is not full runs faster, by the work in them;
-    // one round of 256-token workgroups that leaves CUs idle may become up to a tenth more work.
-    // us, 256 / 192: 8B shape ffn_gate | ffn_up Q4_K 150 tokens 79 / 66, 300 128 / 104 (512 137 / 160, 1000 284 / 317, 6001 1430 / 1475: not taken), 70B shape 300 454 / 376, 513 664 / 559,
-    // Q6_K ffn_down of 8B 380 85 / 72, Q8_0 ffn_down of 72B 513 371 / 319, wq | wk | wv of 8B 150 42 / 36, 1500 120 / 100, 6001 404 / 374 (a split tail before), wo 3000 137 / 122, 6001 285 / 251
-    if (!mid && !force_nt && !force_s && pl.nt == 8) {
-        const int s6 = pl.full ? 1 : pl.splitk, nb = (K + 255) / 256;
-        // workgroups / CUs, rounds and work in them, in sub-tiles of 32 tokens + 1
-        struct Cost { double rounds, work; };
-        const auto cost = [&](int nt) {
-            const int n = (T - 1) / (32 * nt), left = T - 32 * nt * n, last = nt == 6 || !n ? nt : left <= 128 ? 4 : left <= 192 ? 6 : 8;
-            const double w = (double) tiles * s6 / cus;
-            return Cost{std::ceil(w * (n + 1)) * (nt + 1), w * (n * (nt + 1) + last + 1)};
-        };
-        const Cost c6 = cost(6);
-        Cost c8 = cost(8);
-        if (pl.full) c8.rounds = c8.work = 9.0 * pl.cost / nb;
-        if (c6.rounds < 0.97 * c8.rounds && c6.work < (c8.rounds <= 9.0 ? 1.1 : 0.97) * c8.work) pm_gemm_pf_plan(tiles, K, T, cus, 6, s6, 0, &pl);
-    }
+    pm_gemm_pf_plan({tiles, K, T, cus, wide ? (two ? PM_PF_WIDE_TWO : PM_PF_WIDE) : mid ? PM_PF_ROWS_128 : PM_PF_ROWS_256, wide ? wide->ldt : 0, mid ? 0 : asked_nt, force_s, no_mixed ? 0 : 1}, &pl);
     const int nt = pl.nt, S = pl.splitk, full = pl.full, maxL = ((tiles + 7) / 8) * pl.nt_t;
     p.nt_t = pl.nt_t;
     p.splitk = S; p.full = full;

@@ -134,7 +134,11 @@ int pm_launch_gemm_q_h(int type, const void * W, const float * X, const void * x
 // go out as ONE launch. Job: Y[t * ldy + n] (f32) or, when Yh != null, Yh[t * ldy + n] (F16) = W . x (+ bias[n]) (+ resid[t * ldy + n]) (* silu(silu_gate[t * ldy + n]));
 // ldy == 0 means N. pm_gemm_pf_check: 0 when (type, K, N, T) is served, -1 type, -2 shape
 struct pm_gemm_pf_plan_t { int nt, nt_t, splitk, full, grid; double cost; };
-void pm_gemm_pf_plan(int tiles, int K, int T, int cus, int force_nt, int force_s, int allow_mixed, pm_gemm_pf_plan_t * out);   // host arithmetic only (mmq_pf.hip)
+// form: 256-row tiles; 128-row ones, up to 128 tokens; 128-row ones of 8-bit activations of Q4_K (ldt: rows that their tables have), of other types. PM_PF_BY_TOKENS: 64, 128 or 256 tokens a tile by
+// the batch, smaller ones not weighed. nt (sub-tiles of 32 tokens), splitk: 0, or what is forced; mixed: the last tiles alone may be split along K
+enum { PM_PF_BY_TOKENS, PM_PF_ROWS_256, PM_PF_ROWS_128, PM_PF_WIDE, PM_PF_WIDE_TWO };
+struct pm_gemm_pf_ask { int tiles, K, T, cus, form, ldt, nt, splitk, mixed; };
+void pm_gemm_pf_plan(const pm_gemm_pf_ask & ask, pm_gemm_pf_plan_t * out);   // host arithmetic only (mmq_pf.hip)
 struct pm_gemm_pf_job { int type; int N; const void * W; float * Y; void * Yh; const float * bias; const float * resid; const float * silu_gate; long ldy; };
 int pm_gemm_pf_check(int type, int K, int N, int T);
 bool pm_gemm_pf_enabled();      // false under PM355_GEMM_KERNEL=1 / 2 (A/B against the older prompt kernels)

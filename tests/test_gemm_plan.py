@@ -94,3 +94,57 @@ def test_bad_arguments_are_refused():
     assert lib.pm355_gemm_plan(0, 8192, 512, CUS, 1, out) != 0
     assert lib.pm355_gemm_plan(4, 8192, 512, CUS, 1, None) != 0
     assert lib.pm355_gemm_plan(4, 128, 512, CUS, 1, out) != 0
+
+
+ROWS_256, ROWS_128, WIDE_Q4_K, WIDE = 2, 4, 8, 16
+
+
+def every_slice_once(tiles, p):
+    cov = coverage(tiles, p)
+    return len(cov) == tiles * p["nt_t"] and all(sorted(sl) == [(k, sl[0][1]) for k in range(sl[0][1])] for sl in cov.values())
+
+
+@pytest.mark.parametrize("tiles,K,T,tile", [
+    (112, 4096, 129, 192), (112, 4096, 192, 192), (112, 4096, 193, 256), (112, 4096, 300, 192), (112, 4096, 384, 192), (112, 4096, 385, 256), (112, 4096, 512, 256),      # ffn_gate | ffn_up of the 8B shape
+    (112, 4096, 128, 128), (112, 4096, 64, 64), (112, 4096, 6001, 256), (224, 8192, 513, 192), (224, 8192, 576, 192), (224, 8192, 577, 256), (32, 29568, 513, 192),
+    (24, 4096, 150, 192), (24, 4096, 1500, 192), (24, 4096, 6001, 192), (16, 4096, 3000, 192), (16, 4096, 6001, 192), (16, 14336, 380, 192), (17, 2048, 4096, 192), (5, 1024, 300, 192)])
+def test_tiles_of_256_rows_as_launched(tiles, K, T, tile):
+    """tiles of 192 tokens beside those of 256, on either side of where they change; the K split stays that of 256 tokens, a split of the last tiles only goes; no tile or slice is left out"""
+    p, by_tokens = plan(tiles, K, T, ROWS_256), plan(tiles, K, T)
+    assert p["tile_tokens"] == tile and p["nt_t"] == -(-T // tile) and every_slice_once(tiles, p)
+    if tile != 192:
+        assert p == by_tokens
+    else:
+        assert p["full"] == 0 and p["S"] == (1 if by_tokens["full"] else by_tokens["S"])
+
+
+def test_tiles_of_192_tokens_over_many_sizes():
+    """every plan covers its tiles, and one of 192 tokens has fewer or as many sub-tiles of 32 tokens in its rounds of workgroups"""
+    taken = 0
+    for tiles in (1, 7, 16, 24, 40, 64, 112, 128, 200, 224, 255, 501):
+        for K in (512, 1024, 4096, 14336):
+            for T in (129, 191, 192, 193, 256, 257, 320, 384, 385, 448, 449, 512, 513, 576, 577, 700, 1000, 1345, 2049, 4000):
+                p, q = plan(tiles, K, T, ROWS_256), plan(tiles, K, T)
+                assert every_slice_once(tiles, p), (tiles, K, T, p)
+                if p["tile_tokens"] == 256:
+                    assert p == q
+                    continue
+                taken += 1
+                rounds = lambda x, tile: -(-tiles * x["nt_t"] * x["S"] // CUS) * (tile // 32 + 1)  # noqa: E731
+                assert p["tile_tokens"] == 192 and (q["full"] or rounds(p, 192) < rounds(q, 256)), (tiles, K, T, p, q)
+    assert taken > 100
+
+
+@pytest.mark.parametrize("tiles,K,T,flags,tile", [(32, 4096, 64, ROWS_128, 64), (32, 4096, 65, ROWS_128, 96), (32, 14336, 96, ROWS_128, 96), (32, 4096, 97, ROWS_128, 128), (224, 4096, 128, ROWS_128, 128),
+                                                  (32, 4096, 40, WIDE_Q4_K, 64), (224, 4096, 79, WIDE_Q4_K, 96), (224, 4096, 147, WIDE_Q4_K, 96), (224, 4096, 128, WIDE_Q4_K, 128), (32, 4096, 500, WIDE_Q4_K, 128),
+                                                  (32, 14336, 40, WIDE, 64), (32, 14336, 147, WIDE, 64), (1, 512, 512, WIDE, 64)])
+def test_tiles_of_128_rows_as_launched(tiles, K, T, flags, tile):
+    """up to 128 tokens 64, 96 or 128 a tile; of 8-bit activations 96 beside 128 by rounds of workgroups, 64 with other types than Q4_K"""
+    p = plan(tiles, K, T, flags)
+    assert p["tile_tokens"] == tile and p["nt_t"] == -(-T // tile) and every_slice_once(tiles, p), p
+
+
+def test_forms_that_have_no_launch_are_refused():
+    lib, out = L.load(), (C.c_int32 * 5)()
+    lib.pm355_gemm_plan.argtypes = [C.c_int64, C.c_int64, C.c_int64, C.c_int, C.c_int, C.c_void_p]
+    assert lib.pm355_gemm_plan(4, 512, 129, CUS, ROWS_128, out) != 0 and lib.pm355_gemm_plan(4, 512, 513, CUS, WIDE, out) != 0 and lib.pm355_gemm_plan(4, 512, 513, CUS, WIDE_Q4_K, out) != 0

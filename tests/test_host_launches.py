@@ -352,7 +352,7 @@ def products(nt):
     return eval(b"".join(iter(lambda: os.read(r, 65536), b"")).decode())
 plain, three = products("1"), products("3")
 assert len(plain) == 4 and all(len(x) in (1, 2) for x in plain), plain
-assert products("5") == products("9") == plain
+assert products("") == products("5") == products("9") == plain
 assert three == plain, three
 assert products("4") != plain and all(re.search(r"gemm_pf_kernel<\d+, \d+, 4,", x[0][0]) for x in products("4")), products("4")
 print("ok")
@@ -516,5 +516,47 @@ for t in (12, 13, 14, 8):
     assert go(t, 4096) == 0
     want = go(t, 1 << 20)
     assert want not in (0, go(t, 4097)) and all(go(t, K) == want for K in (1 << 24, 1 << 28, (1 << 28) + 256, 1 << 30)), (t, want, [go(t, K) for K in (1 << 24, 1 << 28, 1 << 30)])
+print("ok")
+""")
+
+
+def test_prompt_products_are_launched_as_planned(run):
+    """what pm355_gemm_plan answers is the grid that is launched, and its tile the kernel's: tiles of 256 and of 128 rows, one matrix, several and pairs, and 8-bit activations"""
+    run(COMMON + r"""
+lib = C.CDLL(sys.argv[2])
+at = C.addressof(C.create_string_buffer(256)) // 16 * 16 + 16
+lib.pm355_gemm_plan.argtypes = [C.c_int64, C.c_int64, C.c_int64, C.c_int, C.c_int, C.c_void_p]
+lib.pm355_mul_mat_q_mfma.argtypes = [C.c_int, C.c_void_p, C.c_int64, C.c_int64, C.c_void_p, C.c_int64, C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p]
+lib.pm355_mul_mat_q_mfma_pair.argtypes = [C.c_int, C.c_void_p, C.c_void_p, C.c_int64, C.c_int64, C.c_void_p, C.c_int64, C.c_void_p, C.c_void_p]
+lib.pm355_mul_mat_q_wide.argtypes = [C.c_void_p, C.c_int] + [C.c_void_p] * 6 + [C.c_int64, C.c_int64, C.c_int, C.c_void_p, C.c_void_p]
+def plan(tiles, K, T, flags):
+    out = (C.c_int32 * 5)()
+    assert lib.pm355_gemm_plan(tiles, K, T, 256, flags, out) == 0
+    return out[0] // 32, out[4]
+def launched():
+    (n, g), = [(n, g) for _, n, g in launches() if "gemm_pf_kernel" in n]
+    a = re.search(r"gemm_pf_kernel<(.*?)>", n).group(1).split(", ")
+    return (int(a[2]), g[0]), a[3] == "true"
+for t in (12, 13, 14, 8):
+    for K in (512, 4096, 14336):
+        for N in (132, 1024, 4096, 14336, 40960):
+            for T in (33, 65, 96, 97, 128, 129, 192, 193, 300, 384, 385, 513, 576, 700, 1500, 2049):
+                for pair in (False, True):
+                    if pair and t == 8: continue
+                    shim.shim_forget()
+                    rc = lib.pm355_mul_mat_q_mfma_pair(t, at, at, K, N, at, T, at, 1) if pair else lib.pm355_mul_mat_q_mfma(t, at, K, N, at, T, at, None, None, 1)
+                    assert rc == 0, (t, K, N, T, pair, rc)
+                    got, mid = launched()
+                    small, large = (-(-N // 64), -(-N // 128)) if pair else (-(-N // 128), -(-N // 256))
+                    assert mid == (T <= 128 and small <= 256), (t, K, N, T, pair)
+                    assert got == plan(small if mid else large, K, T, 4 if mid else 2), (t, K, N, T, pair, got)
+arr = lambda v, ty: (ty * len(v))(*v)
+for types, Ns, K in (([12], [4096], 4096), ([12, 12], [1024, 14336], 4096), ([12, 14], [4096, 1024], 4096), ([14], [4096], 14336), ([13], [132], 512)):
+    for T in (33, 64, 65, 96, 97, 128, 129, 147, 192, 231, 288, 289, 512):
+        shim.shim_forget()
+        n = len(types)
+        assert lib.pm355_mul_mat_q_wide(arr(types, C.c_int), n, arr([at] * n, C.c_void_p), arr(Ns, C.c_int64), arr([at] * n, C.c_void_p), None, None, at, K, T, 0, at, 1) == 0
+        got, mid = launched()
+        assert mid and got == plan(sum(-(-N // 128) for N in Ns), K, T, 8 if set(types) == {12} else 16), (types, Ns, K, T, got)
 print("ok")
 """)
