@@ -1214,10 +1214,11 @@ void pm_gemm_pf_plan(const pm_gemm_pf_ask & ask, pm_gemm_pf_plan_t * out) {
         if (cost(3) < cost(4)) plan_tiles(tiles, K, T, cus, 3, out->splitk, 0, out);
     }
     // Tiles of 192 tokens where their rounds of workgroups cost less than those of 256: mostly 129..192, 257..384 and 513..576 tokens, whose rest of a tile of 256 was products of nothing. The K
-    // split stays, so every sum keeps its order; in place of a split of the last tiles only, whole ones. Both by full rounds and, as a last round that is not full runs faster, by the work in them;
-    // one round of 256-token workgroups that leaves CUs idle may become up to a tenth more work.
-    // us, 256 / 192: 8B shape ffn_gate | ffn_up Q4_K 150 tokens 79 / 66, 300 128 / 104 (512 137 / 160, 1000 284 / 317, 6001 1430 / 1475: not taken), 70B shape 300 454 / 376, 513 664 / 559,
-    // Q6_K ffn_down of 8B 380 85 / 72, Q8_0 ffn_down of 72B 513 371 / 319, wq | wk | wv of 8B 150 42 / 36, 1500 120 / 100, 6001 404 / 374 (a split tail before), wo 3000 137 / 122, 6001 285 / 251
+    // split stays, so every sum keeps its order; in place of a split of the last tiles only, whole ones. Both by full rounds and, as a last round that is not full runs faster, by the work in them, which
+    // counts what a cut last tile of 256 leaves out: one round of 256-token workgroups that leaves CUs idle may become up to a tenth more work, as many tiles as much (257..384), others have to save some.
+    // us, 256 with the last tile cut / 192: 8B shape ffn_gate | ffn_up Q4_K 150 tokens 64 / 62, 300 110 / 97 (512 129 / 147, 1000 251 / 280, 6001 1425 / 1455: not taken), 70B shape 300 377 / 339, 513
+    // 596 / 508, Q6_K ffn_down of 8B 380 74 / 69, Q8_0 ffn_down of 72B 513 319 / 297, wq | wk | wv of 8B 150 36.2 / 34.6, 1500 105 / 93, 6001 379 / 335 (a split tail before), wo 3000 129 / 115, 6001 259 / 226;
+    // 33 products of 257..384 tokens and more than a round 0.73-0.97, one 1.01. As much work in more tiles, not taken: 5120 x 13824 pairs 1344 tokens 421 / 450, 8192 x 29568 2112 1871 / 1809
     if (ask.form == PM_PF_ROWS_256 && !ask.splitk && out->nt == 8) {
         const int s6 = out->full ? 1 : out->splitk;
         // workgroups / CUs, rounds and work in them, in sub-tiles of 32 tokens + 1
@@ -1230,7 +1231,8 @@ void pm_gemm_pf_plan(const pm_gemm_pf_ask & ask, pm_gemm_pf_plan_t * out) {
         const Cost c6 = cost(6);
         Cost c8 = cost(8);
         if (out->full) c8.rounds = c8.work = 9.0 * out->cost / nb;
-        if (c6.rounds < 0.97 * c8.rounds && c6.work < (c8.rounds <= 9.0 ? 1.1 : 0.97) * c8.work) plan_tiles(tiles, K, T, cus, 6, s6, 0, out);
+        const double most = c8.rounds <= 9.0 ? 1.1 : !out->full && (T + 191) / 192 == out->nt_t ? 1.001 : 0.97;
+        if (c6.rounds < 0.97 * c8.rounds && c6.work < most * c8.work) plan_tiles(tiles, K, T, cus, 6, s6, 0, out);
     }
 }
 

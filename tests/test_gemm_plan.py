@@ -106,7 +106,8 @@ def every_slice_once(tiles, p):
 
 @pytest.mark.parametrize("tiles,K,T,tile", [
     (112, 4096, 129, 192), (112, 4096, 192, 192), (112, 4096, 193, 256), (112, 4096, 300, 192), (112, 4096, 384, 192), (112, 4096, 385, 256), (112, 4096, 512, 256),      # ffn_gate | ffn_up of the 8B shape
-    (112, 4096, 128, 128), (112, 4096, 64, 64), (112, 4096, 6001, 256), (224, 8192, 513, 192), (224, 8192, 576, 192), (224, 8192, 577, 256), (32, 29568, 513, 192),
+    (112, 4096, 128, 128), (112, 4096, 64, 64), (112, 4096, 6001, 256), (224, 8192, 513, 192), (224, 8192, 576, 192), (224, 8192, 577, 256),
+    (224, 8192, 256, 256), (224, 8192, 257, 192), (224, 8192, 384, 192), (224, 8192, 385, 256), (231, 8192, 300, 192), (501, 4096, 320, 192), (501, 4096, 1300, 256), (108, 5120, 1344, 256), (32, 29568, 513, 192),
     (24, 4096, 150, 192), (24, 4096, 1500, 192), (24, 4096, 6001, 192), (16, 4096, 3000, 192), (16, 4096, 6001, 192), (16, 14336, 380, 192), (17, 2048, 4096, 192), (5, 1024, 300, 192)])
 def test_tiles_of_256_rows_as_launched(tiles, K, T, tile):
     """tiles of 192 tokens beside those of 256, on either side of where they change; the K split stays that of 256 tokens, a split of the last tiles only goes; no tile or slice is left out"""
