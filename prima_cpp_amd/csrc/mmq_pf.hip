@@ -919,6 +919,11 @@ __device__ __forceinline__ void mid_body(const PfP & p, const PfJob & jb, const 
 
 // block id -> (row tile, token tile): XCD x = id % 8 takes the row tiles x, x + 8, ..; its consecutive slots sweep the token tiles of one row tile, so the
 // workgroups that run together on an XCD share a few row tiles of weights and the activation k-slices in its L2 (mmq_big.hip's mapping)
+// PF_CUT (a bit of EXP): the batch's last tile of 256 tokens multiplies the 128 or 192 that are left of it only. us, whole / cut: wo of the 8B shape 640 tokens 50.5 / 47.4, 1400 76.8 / 75.7, 2100 113 / 114
+// (in tiles of 192 93), its Q6_K ffn_down 640 114 / 107, 1400 229 / 218, ffn_gate | ffn_up 640 189 / 181, 1800 478 / 471, Q8_0 ffn_down of 72B 640 374 / 345. (Tiles of 192 with a cut last one: wo 2400
+// 105 / 110, wq | wk | wv 6001 360 / 379.) A kernel of its own: with the two smaller bodies beside it a launch that cuts nothing took 0.2-0.9 us more (200 tokens of 1024 x 1024 34.2 -> 34.8, Q8_0
+// 33.8 -> 34.8; now 33.6, 33.7)
+constexpr int PF_CUT = 256;
 template <int TA, int TB, int NT, bool MID = false, int EXP = 0, bool EX = false>
 __global__ __launch_bounds__((MID && !mid_self<TA, TB, NT, EX>() ? MID_NTHR : PF_NTHR)) void gemm_pf_kernel(PfP p) {
     extern __shared__ __attribute__((aligned(1024))) uint8_t pf_smem[];
@@ -949,15 +954,14 @@ __global__ __launch_bounds__((MID && !mid_self<TA, TB, NT, EX>() ? MID_NTHR : PF
     if constexpr (!MID) {
         auto body = [&](auto nt) __attribute__((always_inline)) {
             constexpr int N = decltype(nt)::value;
-            if (TA == TB || jb.type == TA) pf_body<TA, N, EXP, NT>(p, jb, n0, t0, pf_smem, role, ks, S, tile_id);
-            else pf_body<TB, N, EXP, NT>(p, jb, n0, t0, pf_smem, role, ks, S, tile_id);
+            if (TA == TB || jb.type == TA) pf_body<TA, N, EXP & 255, NT>(p, jb, n0, t0, pf_smem, role, ks, S, tile_id);
+            else pf_body<TB, N, EXP & 255, NT>(p, jb, n0, t0, pf_smem, role, ks, S, tile_id);
         };
-        // The batch's last tile of 256 tokens multiplies the 128 or 192 that are left of it only. us of one K split, whole / cut: wo of the 8B shape 640 tokens 50.4 / 47.5, 1400 79.3 / 75.0, 2100 120 / 104,
-        // its Q6_K ffn_down 1400 237 / 225, ffn_gate | ffn_up 1800 515 / 495, Q8_0 ffn_down of 72B 640 404 / 371; nothing left out (1250) the same. (Tiles of 192 with a cut last one: wo 2400
-        // 105 / 110, wq | wk | wv 6001 360 / 379)
+        constexpr bool CUT = (EXP & PF_CUT) != 0;
+        static_assert(!CUT || NT == 8, "tiles of 256 tokens");
         const int left = p.T - t0;
-        if (NT == 8 && left <= 128) body(std::integral_constant<int, NT == 8 ? 4 : NT>());
-        else if (NT == 8 && left <= 192) body(std::integral_constant<int, NT == 8 ? 6 : NT>());
+        if (CUT && left <= 128) body(std::integral_constant<int, CUT ? 4 : NT>());
+        else if (CUT && left <= 192) body(std::integral_constant<int, CUT ? 6 : NT>());
         else body(std::integral_constant<int, NT>());
     } else {
         constexpr bool SELF = mid_self<TA, TB, NT, EX>();
@@ -1342,6 +1346,7 @@ static int launch_pf(const pm_gemm_pf_job * jobs, int njobs, const void * xh, co
         return 0;
     }
 #endif
+    const bool cut = T - 256 * (pl.nt_t - 1) <= 192;            // (of tiles of 256 tokens: the last one)
     // (an nt that no kernel has stays an error)
 #define PF_GO(A, B) do { \
         if (wide) { \
@@ -1354,7 +1359,9 @@ static int launch_pf(const pm_gemm_pf_job * jobs, int njobs, const void * xh, co
             else if (nt == 3) go(gemm_pf_kernel<A, B, 3, true>, pf_lds_bytes<A, B, 3, true>()); \
             else if (nt == 2) go(gemm_pf_kernel<A, B, 2, true>, pf_lds_bytes<A, B, 2, true>()); \
             else return -2; \
-        } else if (nt == 8)   go(gemm_pf_kernel<A, B, 8>, pf_lds_bytes<A, B, 8>()); \
+        } else if (nt == 8) { \
+            if (cut) go(gemm_pf_kernel<A, B, 8, false, PF_CUT>, pf_lds_bytes<A, B, 8>()); else go(gemm_pf_kernel<A, B, 8>, pf_lds_bytes<A, B, 8>()); \
+        } \
         else if (nt == 6)     go(gemm_pf_kernel<A, B, 6>, pf_lds_bytes<A, B, 6>()); \
         else if (nt == 4)     go(gemm_pf_kernel<A, B, 4>, pf_lds_bytes<A, B, 4>()); \
         else if (nt == 2)     go(gemm_pf_kernel<A, B, 2>, pf_lds_bytes<A, B, 2>()); \
