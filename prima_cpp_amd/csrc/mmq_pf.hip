@@ -487,7 +487,11 @@ template <int TYPE, int NT> constexpr int mid_sum_bytes() { return TYPE == PM_Q6
 template <int TYPE, int NT, bool EX> constexpr size_t mid_lds_bytes() { return (size_t) 6 * NT * 32 * 128 + (size_t) 4 * mid_group_bytes<TYPE, EX>() + (EX ? 2 * (mid_sum_bytes<TYPE, NT>() + NT * 32 * 4) : 0); }
 // no waves of their own for the requests: where the kernel's registers leave no room for them (168 a wave). 8B shape, 147 tokens of 8-bit activations, wq | wk | wv with a Q6_K wv: 53 us, with loaders
 // and 12 registers spilled 68
-template <int TA, int TB, int NT, bool EX> constexpr bool mid_self() { return EX && (NT == 4 || TA != TB || TA == PM_Q5_K); }
+// PF_SELF (a bit of EXP): or where a loader's requests are the longer part of a step - Q8_0, four pieces of 1 KiB to a row group and 128 k, up to 64 tokens, where half of the chip is idle anyway: less
+// than 128 workgroups. us at 64 tokens, four loaders / none: 1024 x 512 10.8 / 10.0, 1024 x 1024 14.3 / 13.4, 2048 x 3072 16.8 / 16.0, 512 x 8192 18.9 / 18.1; from 128 workgroups on 6144 x 4096 20.2 /
+// 20.4, 8192 x 8192 29.7 / 30.4. (K = 512 of the other types, 4 steps: 64 tokens 10.3 / 10.0, 128 12.6 / 12.0, from K = 1024 on 0.92-1.00)
+constexpr int PF_SELF = 512;
+template <int TA, int TB, int NT, bool EX, int EXP = 0> constexpr bool mid_self() { return (EXP & PF_SELF) || (EX && (NT == 4 || TA != TB || TA == PM_Q5_K)); }
 template <int N> __device__ __forceinline__ void mid_wait() { asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" : : "n"(N) : "memory"); }
 
 // A tile's requests. Those of weights and of activations are different waves': requests return in order, and weights come from memory (AHEAD steps ahead), activations mostly from L2 (two steps)
@@ -656,7 +660,7 @@ __device__ __forceinline__ void mid_body(const PfP & p, const PfJob & jb, const 
     auto request = [&](int s, bool even, int u) __attribute__((always_inline)) {
         if constexpr (SELF) {
             constexpr int Q = decltype(own_rq.x)::NQ / 4, AHEAD = decltype(own_rq.w)::AHEAD;
-            if (kk) { if (even && u == 0) own_rq.x.issue_x((s >> 1) + 1); own_rq.x.issue(s + 2, Q * u, Q * u + Q); } else own_rq.w.issue(s + AHEAD, AHEAD & 1 ? !even : even, u);
+            if (kk) { if (EX && even && u == 0) own_rq.x.issue_x((s >> 1) + 1); own_rq.x.issue(s + 2, Q * u, Q * u + Q); } else own_rq.w.issue(s + AHEAD, AHEAD & 1 ? !even : even, u);
         }
     };
     // the end of a step: the next one's operands are there (a loader waited for them, or this wave), this wave's LDS reads are through
@@ -667,7 +671,7 @@ __device__ __forceinline__ void mid_body(const PfP & p, const PfJob & jb, const 
     if constexpr (SELF) {
         if (kk) {
             own_rq.x.init(p, t0, g, lds0, lane);
-            own_rq.x.issue_x(b0);
+            if (EX) own_rq.x.issue_x(b0);
             own_rq.x.issue(2 * b0, 0, 2 * NT); own_rq.x.turn();
             own_rq.x.issue(2 * b0 + 1, 0, 2 * NT);
         } else {
@@ -925,7 +929,7 @@ __device__ __forceinline__ void mid_body(const PfP & p, const PfJob & jb, const 
 // 33.8 -> 34.8; now 33.6, 33.7)
 constexpr int PF_CUT = 256;
 template <int TA, int TB, int NT, bool MID = false, int EXP = 0, bool EX = false>
-__global__ __launch_bounds__((MID && !mid_self<TA, TB, NT, EX>() ? MID_NTHR : PF_NTHR)) void gemm_pf_kernel(PfP p) {
+__global__ __launch_bounds__((MID && !mid_self<TA, TB, NT, EX, EXP>() ? MID_NTHR : PF_NTHR)) void gemm_pf_kernel(PfP p) {
     extern __shared__ __attribute__((aligned(1024))) uint8_t pf_smem[];
     const int id = (int) blockIdx.x, x = id & 7;
     // slots [0, full) of an XCD run whole tiles; the slots behind them are split S ways along K, the slices of a tile neighbours on one XCD.
@@ -964,7 +968,7 @@ __global__ __launch_bounds__((MID && !mid_self<TA, TB, NT, EX>() ? MID_NTHR : PF
         else if (CUT && left <= 192) body(std::integral_constant<int, CUT ? 6 : NT>());
         else body(std::integral_constant<int, NT>());
     } else {
-        constexpr bool SELF = mid_self<TA, TB, NT, EX>();
+        constexpr bool SELF = mid_self<TA, TB, NT, EX, EXP>();
         if (TA == TB || jb.type == TA) mid_body<TA, NT, EX, SELF>(p, jb, n0, t0, pf_smem, role, ks, S, tile_id);
         else mid_body<TB, NT, EX, SELF>(p, jb, n0, t0, pf_smem, role, ks, S, tile_id);
     }
@@ -1298,9 +1302,11 @@ static int launch_pf(const pm_gemm_pf_job * jobs, int njobs, const void * xh, co
         if (!p.ws) return -3;
     }
     const int slots = full + split_slots * S;
+    const bool few = mid && !wide && ta == PM_Q8_0 && nt == 2 && (long) tiles * pl.nt_t * S < 128;      // (PF_SELF)
+    const bool self = wide ? nt == 4 || ta != tb || ta == PM_Q5_K : few;                                  // (mid_self of the kernel below)
     auto go = [&](auto kern, size_t lds) {
         pf_allow_lds((const void *) kern, lds);
-        hipLaunchKernelGGL(kern, dim3(8 * slots), dim3(mid && !(wide && (nt == 4 || ta != tb || ta == PM_Q5_K)) ? MID_NTHR : PF_NTHR), lds, st, p);
+        hipLaunchKernelGGL(kern, dim3(8 * slots), dim3(mid && !self ? MID_NTHR : PF_NTHR), lds, st, p);
         if (S == 1) return;
         if (norm && !full && T <= 512 && njobs == 1 && jobs[0].Y && !jobs[0].Yh && !jobs[0].silu_gate && p.job[0].ldy == p.job[0].N && jobs[0].N % 256 == 0 && jobs[0].N <= 8192) {
             auto fused = [&](auto k) { hipLaunchKernelGGL(k, dim3(T), dim3(1024), 0, st, p, (int) mid, nt, norm->w, norm->eps, (_Float16 *) norm->yh); };
@@ -1357,7 +1363,7 @@ static int launch_pf(const pm_gemm_pf_job * jobs, int njobs, const void * xh, co
         } else if (mid) { \
             if (nt == 4)      go(gemm_pf_kernel<A, B, 4, true>, pf_lds_bytes<A, B, 4, true>()); \
             else if (nt == 3) go(gemm_pf_kernel<A, B, 3, true>, pf_lds_bytes<A, B, 3, true>()); \
-            else if (nt == 2) go(gemm_pf_kernel<A, B, 2, true>, pf_lds_bytes<A, B, 2, true>()); \
+            else if (nt == 2) { if (few) go(gemm_pf_kernel<PM_Q8_0, PM_Q8_0, 2, true, PF_SELF>, pf_lds_bytes<PM_Q8_0, PM_Q8_0, 2, true>()); else go(gemm_pf_kernel<A, B, 2, true>, pf_lds_bytes<A, B, 2, true>()); } \
             else return -2; \
         } else if (nt == 8) { \
             if (cut) go(gemm_pf_kernel<A, B, 8, false, PF_CUT>, pf_lds_bytes<A, B, 8>()); else go(gemm_pf_kernel<A, B, 8>, pf_lds_bytes<A, B, 8>()); \

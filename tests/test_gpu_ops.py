@@ -1052,6 +1052,26 @@ def test_prompt_tiles_of_96_tokens(P, t, K, N):
         assert P.torch.equal(P.mul_mat_wide([w, w2], x[:T], pair=True)[0], pair[:T]), T
 
 
+@pytest.mark.parametrize("K", [512, 640, 1664])
+def test_prompt_products_of_few_q8_0_rows(P, oracle, K):
+    """up to 64 tokens and less than 128 workgroups of 128 rows: the kernel without loaders, the bits of the one with them (129 workgroups; no K split at these K, rows that end on half a
+    super-block among them), and the oracle's products of the F16 activations"""
+    N, rng = 129 * 128, np.random.default_rng(K)
+    b = rand_blocks(Q8_0, N, K, rng)
+    x = rng.normal(0, 1, (64, K)).astype(np.float16).astype(np.float32)
+    few, many = b.reshape(N, -1), P.upload_weight(Q8_0, b, K, N)
+    for T in (33, 64):
+        xd = _dev(P, x[:T])
+        want = P.mul_mat_mfma(many, xd)
+        for n in (4, 132, 1024, 127 * 128):
+            got = P.mul_mat_mfma(P.upload_weight(Q8_0, np.ascontiguousarray(few[:n]).reshape(-1), K, n), xd)
+            assert P.torch.equal(got, want[:, :n]), (T, n)
+    w = np.stack([oracle.dequantize_row(Q8_0, np.ascontiguousarray(r), K) for r in few[:132]]).astype(np.float64)
+    y = want[:, :132].cpu().numpy().astype(np.float64)
+    exact = x.astype(np.float64) @ w.T
+    assert np.linalg.norm(y - exact) < 1e-3 * np.linalg.norm(exact)      # (a weight is rounded to F16 once: 2^-11 at most)
+
+
 @pytest.mark.parametrize("t", [Q4_K, Q5_K, Q6_K])
 @pytest.mark.parametrize("K,N,T", [(1024, 384, 200), (2048, 132, 64), (512, 256, 257), (8192, 132, 200)])
 def test_prompt_gemm_pair_tiles_silu_gate_times_up(P, oracle, t, K, N, T):
