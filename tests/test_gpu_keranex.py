@@ -209,10 +209,10 @@ def test_experts_in_turn(E, top, ff, width, dtype):
     m.close()
 
 
-@pytest.mark.parametrize("E,top,ff,width", [(6, 4, 4160, 260), (64, 4, 520, 600), (33, 1, 64, 2000), (2, 2, 4600, 130)])
+@pytest.mark.parametrize("E,top,ff,width", [(6, 4, 4160, 260), (64, 4, 520, 600), (33, 1, 64, 2000), (2, 2, 4544, 130), (2, 2, 4600, 130)])
 def test_experts_whose_load_groups_are_one_sequence(E, top, ff, width):
-    """bf16, pairs that the products find for themselves: rows of one more block than the waves share (two load groups for one wave, one for the others), of less blocks than waves and up to the longest
-    that fit; 64 experts, one, 256 pairs; experts of one, eight, nine and of 64 pairs"""
+    """bf16, pairs that the products find for themselves: rows of one more block than the waves share (two load groups for one wave, one for the others), of less blocks than waves, the longest that
+    fit (71 blocks of 64: nine for seven waves, eight for the last) and the first that do not (72); 64 experts, one, 256 pairs; experts of one, eight, nine and of 64 pairs"""
     c = one(scan(inner=64, mlp=moe(E, top, 1, 1, ff)), width=width, vocab=120)
     w = silent(weights_for(c, "bfloat16", 9), 0)
     _, _, m = model("sequence", "bfloat16", c, 9, w, fresh=True, max_tokens=64, n_seq=2, pool_tokens=128)

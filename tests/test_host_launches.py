@@ -564,3 +564,30 @@ for types, Ns, K in (([12], [4096], 4096), ([12, 12], [1024, 14336], 4096), ([12
         assert mid and got == plan(sum(-(-N // 128) for N in Ns), K, T, 8 if set(types) == {12} else 16), (types, Ns, K, T, got)
 print("ok")
 """)
+
+
+def test_which_experts_products_are_one_sequence_of_load_groups(run):
+    """the shapes of test_gpu_keranex.py's test of dense_experts_kernel reach it: both products of the experts, up to 71 blocks of 64 values; the hidden one of 72 does not"""
+    run(COMMON + r"""
+import os
+sys.path.insert(0, os.path.join(os.environ["PYTHONPATH"], "tests"))
+import numpy as np, torch
+torch.cuda.current_device = lambda: 0
+import prima_cpp_amd.engine as E
+E.stream_ptr = lambda: 1
+from prima_cpp_amd import keranex
+from test_gpu_keranex import moe, one, scan, silent, weights_for
+for (n, top, ff, width), want in (((6, 4, 4160, 260), 2), ((64, 4, 520, 600), 2), ((33, 1, 64, 2000), 2), ((2, 2, 4544, 130), 2), ((2, 2, 4600, 130), 1)):
+    c = one(scan(inner=64, mlp=moe(n, top, 1, 1, ff)), width=width, vocab=120)
+    m = keranex.load_arrays(c, silent(weights_for(c, "bfloat16", 9), 0), "bfloat16")
+    m.finalize_pool(max_tokens=64, n_seq=2, pool_tokens=128)
+    for T in (5, 8, 9, 23, 64):
+        s = m.seq_new()
+        shim.shim_forget()
+        m.batch([(s, np.zeros(T, np.int32), (T - 1,))], logits=torch.zeros(1, 120))
+        m.seq_free(s)
+        got = sum("dense_experts_kernel" in name for _, name, _ in launches())
+        assert got == want, (n, top, ff, width, T, got, [name for _, name, _ in launches()])
+    m.close()
+print("ok")
+""")
