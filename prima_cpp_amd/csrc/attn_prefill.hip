@@ -224,7 +224,7 @@ __global__ __launch_bounds__(256, 2) void attn_rowmajor_kernel(PfP p) {
 // Bound by the LDS reads of the fragments (32 queries per wave: 32 KiB per 64 keys and wave at ~80 bytes per cycle and CU, about the time of the 32 matrix instructions) and the
 // exponentials beside them. Against the two-pass form with 4 waves x 32 queries, 32-key tiles through registers: 6001 tokens x 32 heads 870 -> 393 us (752 TFLOP/s), 512 x 64 behind
 // 1024 cached cells 102 -> 38, 101 x 32 behind 300 29.8 -> 11.7, 2048 x 32 144 -> 55. Requests by the waves that multiply / by their own, whole passes: 70B shape, three layers, 8 tokens behind 403
-// cells 396 / 391, 8B shape, four layers and head, 101 behind 300 653 / 648, 6001 13330 / 13290. (Both stages asked for at once in front, keys behind the last one left out: no change.)
+// cells 408 / 406, 72B shape, two layers, 23 tokens 461 / 459, 8B shape, four layers and head, 6001 13255 / 13215. (Both stages asked for at once in front, keys behind the last one left out: no change.)
 // PLAIN: caches that do not start on 16 bytes, by loads and LDS stores instead of DMA
 // PAIR: tiles of up to 32 queries, the two query waves of a key group are two heads of one KV head; their results leave as Q8_K blocks (the wo product's activations) - no f32 rows and no launch that
 // quantizes them: 8 tokens x 64 heads behind 403 cells 11.3 + 5.0 us, with this ending 13.3, with waves that bring 12.0; 23 tokens and no other cells 11.8 / 9.0

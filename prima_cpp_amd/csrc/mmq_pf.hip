@@ -474,7 +474,8 @@ __device__ __forceinline__ void pf_body(const PfP & p, const PfJob & jb, const i
 // Operands are requested by four waves that do nothing else (mid_load); where a kernel's registers leave no room for them, by the ones that multiply, a quarter of a step's behind each slice's
 // products. 8B shape, Q4_K at 101 tokens, us, requests by the waves that multiply / by their own: ffn_gate | ffn_up 51.9 / 45.6, ffn_down 28.7 / 26.5, wo 18.0 / 17.0, wq | wk | wv 20.0 / 18.7.
 // What bounds it, four layers of that (646 us, 411 without any step): the requests alone 168 of the 235 us of steps - weights 91, whose 32-byte pieces of a line are asked for line by line four
-// times over, activations 41 -, LDS reads, dequantization and MFMAs alone 136. Tiles of 96 tokens cost 0.8 of those of 128: 90 tokens, two layers 287 / 252 us.
+// times over, activations 41 -, LDS reads, dequantization and MFMAs alone 136. Tiles of 96 tokens cost 0.8 of those of 128. Two layers, Q4_K, us, neither / loaders / tiles of 96
+// too: 70 tokens 286 / 264 / 241, 90 tokens 290 / 272 / 250, 101 tokens 293 / 276 / 275; 8-bit activations, eight prompts of up to 12 tokens 498 / 494 / 452, of up to 24 706 / 692 / 624, of up to 30 728 / 714 / 645.
 // Llama-3-8B's launches at 101 tokens, Q4_K, us in the general tiles / as these were first: wq | wk | wv 37 / 24, wo 34 / 23, ffn_gate | ffn_up 61 / 50, ffn_down 54 / 36.6. Taken back: 64 rows and
 // a quarter of the k per wave (half the LDS reads: no change, 1-2 us more for the longer merge); two activation buffers instead of three (2-10 % slower); a step's first fragments read in the
 // step before, whose activations then have one step to arrive instead of two (646 -> 680).
@@ -1265,7 +1266,7 @@ static int launch_pf(const pm_gemm_pf_job * jobs, int njobs, const void * xh, co
     for (int j = 0; j < njobs; ++j) two |= wide && jobs[j].type != PM_Q4_K;
     long mid_wgs = 0;
     for (int j = 0; j < njobs && !(pair && j); ++j) mid_wgs += (jobs[j].N + (pair ? 63 : 127)) / (pair ? 64 : 128);
-    // (8-bit activations: mid_body at any size - its tiles of 128 tokens side by side -, pf_body's registers are its accumulators')
+    // (8-bit activations: mid_body at any size - its tiles side by side -, pf_body's registers are its accumulators')
     const bool mid = wide || (!asked_nt && T <= 128 && mid_wgs <= cus);
     const int rows = mid ? 128 : 256;
     PfP p = {};

@@ -107,7 +107,7 @@ __global__ __launch_bounds__(256) void silu_mul_q80_tab_kernel(const float * __r
 // quantize block after block. us with 4 / 16 waves, K = 4096: 101 rows 5.1 / 3.9, 256 rows 5.3 / 4.2, 300 rows 5.4 / 6.0; K = 8192: 101 rows 7.9 / 4.9, 256 rows 8.2 / 5.4, 512 rows 9.3 / 8.5,
 // 700 rows 11.1 / 11.4. (8 rows 3.8 -> 3.6 with the sum by DPP and the weights asked for with the row.)
 // SPLIT: two workgroups to a row of 17 .. 32 blocks, each adds the whole row up (the same sum) and writes one half of it. Two blocks one after the other in every wave, four waves on a SIMD, were
-// 2.0 of a launch's 3.9 us (stamps, 8 rows of 8192): three layers of the 70B shape at 8 tokens, six such launches, 392 -> 388 us. (One block in every wave, 1.25 of 3.1, in two or four workgroups: no
+// 2.0 of a launch's 3.9 us (stamps, 8 rows of 8192): three layers of the 70B shape at 8 tokens, six such launches, 391 -> 388 us. (One block in every wave, 1.25 of 3.1, in two or four workgroups: no
 // change. A workgroup's share by gridDim.y and a division: 0.6 us more on every launch, the grid's size is another load.)
 template <int NWV, bool SPLIT = false>
 __global__ __launch_bounds__(64 * NWV) void rmsnorm_q8k_kernel(const float * __restrict__ x, const float * __restrict__ w,
