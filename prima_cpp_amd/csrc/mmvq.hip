@@ -281,7 +281,9 @@ int pm_launch_gemv(const pm_gemv_args & a, hipStream_t st) {
         int nc = (a.dbg_int || left < 2) ? 1 : pair ? ((a.type == PM_Q4_K || a.type == PM_Q6_K) ? 2 : 1) : (left >= 8 && a.type != PM_Q5_K ? 8 : left >= 3 ? 4 : 2);   // (8 Q5_K columns spill even at 256 VGPRs)
         if (nc > 1) {
             GemvP p; int ta, tb, grid; bool pr; size_t lds1;
-            int rc = gemv_fill(f, -1, p, ta, tb, pr, lds1, grid);
+            // (eight columns of a small matrix: four rows of them are longer than the workgroups without a row take to start. us, workgroups of four rows / one per CU: 16 rows of 8192 8.6 / 7.2, 64 of 4096
+            // 6.9 / 6.2, 1000 of 1024 6.4 / 6.4; two and four columns 0.90-0.99 with four rows, 16 rows of four 1.02)
+            int rc = gemv_fill(f, nc == 8 ? 0 : -1, p, ta, tb, pr, lds1, grid);
             if (rc) return rc;
             // LDS: nc activation columns + nc results per row
             const int ablk = ta == PM_Q8_0 ? 32 : 256;

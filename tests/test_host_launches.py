@@ -591,3 +591,23 @@ for (n, top, ff, width), want in (((6, 4, 4160, 260), 2), ((64, 4, 520, 600), 2)
     m.close()
 print("ok")
 """)
+
+
+def test_grids_of_small_mat_vecs(run):
+    """a matrix of less than four rows per CU and 512 KB: workgroups of four rows for one, two and four columns, one workgroup per CU for eight and for what is larger"""
+    run(COMMON + r"""
+lib = C.CDLL(sys.argv[2])
+f = lib.pm355_mul_mat_vec_q
+f.argtypes = [C.c_int, C.c_void_p, C.c_void_p, C.c_int64, C.c_int64, C.c_void_p, C.c_int, C.c_void_p, C.c_int64, C.c_void_p, C.c_void_p, C.c_void_p]
+at = C.addressof(C.create_string_buffer(256))
+def grids(K, N, cols):
+    shim.shim_forget()
+    assert f(12, at, None, K, N, at, cols, at, N, None, None, 1) == 0
+    return [g[0] for _, _, g in launches()]
+for K, N in ((256, 16), (1024, 333), (8192, 64), (4096, 200)):
+    assert grids(K, N, 1) == grids(K, N, 2) == grids(K, N, 3) == grids(K, N, 4) == [(N + 3) // 4], (K, N)
+    assert grids(K, N, 8) == [256] and grids(K, N, 5) == [(N + 3) // 4] * 2, (K, N)
+for cols in (1, 2, 4, 8):
+    assert grids(4096, 1024, cols) == grids(8192, 4096, cols) == [256]
+print("ok")
+""")
