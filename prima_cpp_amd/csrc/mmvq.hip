@@ -178,8 +178,9 @@ int pmv::gemv_fill(const pm_gemv_fused & a, int grid_fixed, GemvP & p, int & ta_
     int rows_cap = PM_MAX_ROWS_PER_WG;
     if (grid_fixed > 0) rows_cap = (int) ((tot_rows + grid - 1) / grid + 3 > PM_MAX_ROWS_PER_WG ? (tot_rows + grid - 1) / grid + 4 : PM_MAX_ROWS_PER_WG);
     else while ((tot_rows + grid - 1) / grid + 3 > PM_MAX_ROWS_PER_WG) grid *= 2;
-    // (job_slice is exact for a power of two, and for any other number below 2^(32 / 3))
-    if ((int64_t) grid * grid * grid >= (int64_t) 1 << 32) while (grid & (grid - 1)) grid += grid & -grid;
+    // (job_slice is exact for a power of two up to 65536, and for any other number up to 2^(32 / 3). Plain products of more rows are launched in pieces)
+    if (grid > 65536 && (a.epi || a.ss_out)) return -5;
+    if (grid > 1625) while (grid & (grid - 1)) grid += grid & -grid;
     p.inv = (uint32_t) ((((uint64_t) 1 << 32) + grid - 1) / grid);
     for (int j = 0; j < 3; ++j) {
         GemvJob & g = p.job[j];
@@ -247,11 +248,33 @@ int pm_gemv_fused_grid(const pm_gemv_fused & a) {
     return rc ? (rc < 0 ? rc : -rc) : grid;
 }
 
+// rows that a launch of 65536 workgroups takes: with more of them rest x b of job_slice has more than 32 bits
+constexpr int ROWS_MOST = 65536 * (PM_MAX_ROWS_PER_WG - 3), ROWS_PIECE = 1 << 24;
+static pm_gemv_job rows_from(const pm_gemv_job & j, int K, int64_t r) {
+    pm_gemv_job p = j;
+    const size_t w = (size_t) r * pm_weight_row_stride(j.type, K);
+    p.N = (int) std::min((int64_t) ROWS_PIECE, j.N - r); p.W = (const uint8_t *) j.W + w; if (j.W2) p.W2 = (const uint8_t *) j.W2 + w;
+    p.y = j.y + r; if (j.bias) p.bias = j.bias + r; if (j.resid) p.resid = j.resid + r;
+    return p;
+}
+
 // Fused launch: up to 3 matrices sharing one activation row.
 int pm_launch_gemv_fused(const pm_gemv_fused & a, hipStream_t st) {
     GemvP p; int ta, tb, grid; bool pair; size_t lds;
     const int rc = gemv_fill(a, -1, p, ta, tb, pair, lds, grid);
     if (rc) return rc;
+    if (grid > 65536) {
+        pm_gemv_fused f = a;
+        f.njobs = 1;
+        for (int j = 0; j < a.njobs; ++j)
+            for (int64_t r = 0; r < a.job[j].N; r += ROWS_PIECE) {
+                f.job[0] = rows_from(a.job[j], a.K, r);
+                if (a.dbg_int) f.dbg_int = a.dbg_int + (size_t) r * (a.K / nv_of(a.job[j].type)) * 2;
+                const int piece = pm_launch_gemv_fused(f, st);
+                if (piece) return piece;
+            }
+        return 0;
+    }
     p.ts = pm_ts_next_slot();
 #define PM_L(TA_, TB_) return launch_types<TA_, TB_>(p, pair, grid, lds, a.dbg_int != nullptr, st, a.epi != nullptr)
     if (ta == PM_Q4_K && tb == PM_Q4_K) PM_L(PM_Q4_K, PM_Q4_K);
@@ -268,6 +291,16 @@ int pm_launch_gemv_fused(const pm_gemv_fused & a, hipStream_t st) {
 // weights (gemv_q_cols_kernel), a remaining single column - and pair / debug launches - go one launch per column.
 int pm_launch_gemv(const pm_gemv_args & a, hipStream_t st) {
     const size_t xrow = a.type == PM_Q8_0 ? pm_q80_row_bytes(a.K) : pm_q8k_row_bytes(a.K);
+    if (a.N > ROWS_MOST && a.ncols > 1) {
+        for (int64_t r = 0; r < a.N; r += ROWS_PIECE) {
+            pm_gemv_args g = a;
+            const pm_gemv_job p = rows_from({a.type, a.N, a.W, a.W2, a.y, a.bias, a.resid}, a.K, r);
+            g.N = p.N; g.W = p.W; g.W2 = p.W2; g.y = p.y; g.bias = p.bias; g.resid = p.resid;
+            const int rc = pm_launch_gemv(g, st);
+            if (rc) return rc;
+        }
+        return 0;
+    }
     int c = 0;
     while (c < a.ncols) {
         pm_gemv_fused f = {};

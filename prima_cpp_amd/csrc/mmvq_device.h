@@ -23,9 +23,9 @@ struct GemvJob {
     int nx_s, nx_dh /*log2 head_dim*/, nx_hrot /*n_rot / 2*/;
     int each, rest;                         // N = each * workgroups + rest
 };
-// first row of workgroup b's slice, floor(N b / workgroups), with inv = ceil(2^32 / workgroups) (exact while rest b x (inv workgroups - 2^32) < 2^32, gemv_fill). The division itself, of 64 bits and by a
+// first row of workgroup b's slice, floor(N b / workgroups), with inv = ceil(2^32 / workgroups) (exact while rest b and rest b x (inv workgroups - 2^32) < 2^32, gemv_fill). The division itself, of 64 bits and by a
 // grid size that is one more load, stood in front of every first load of a launch: one token of eight layers of the 8B shape, 33 such launches, 446 -> 429 us without it, three layers of 70B 327 -> 322
-__device__ __forceinline__ int job_slice(int each, int rest, int b, uint32_t inv) { return each * b + (int) __umulhi((uint32_t) (rest * b), inv); }
+__device__ __forceinline__ int job_slice(int each, int rest, int b, uint32_t inv) { return each * b + (int) __umulhi((uint32_t) rest * (uint32_t) b, inv); }
 // logical -> matrix row of a job (wave-uniform arithmetic: shifts and masks, head_dim and the slice size are powers of two)
 __device__ __forceinline__ int job_row(const GemvJob & jb, int L) {
     const int sh = jb.nx_s > 0 ? jb.nx_s : 1, half = 1 << (sh - 1);                // (branch-free: scalar selects, the row loops stay straight-line code)

@@ -202,6 +202,23 @@ def test_gemv_rows_whatever_the_slices(P, t):
         assert P.torch.equal(P.mul_mat_vec(w(n, 77), x=x, w2=w(n, 77)), pair[:, 77:77 + n]), n
 
 
+def test_gemv_of_more_rows_than_a_launch_takes(P):
+    """34 million rows, launched in pieces: the bits of the same rows in a small matrix - with a bias, as a pair, several columns, and beside another matrix"""
+    K, part, N, rng, torch = 32, 10007, 34000001, np.random.default_rng(56), P.torch
+    small = P.upload_weight(Q8_0, rand_blocks(Q8_0, part, K, rng).reshape(-1), K, part)
+    stretch = lambda v: v.repeat((N + part - 1) // part, *[1] * (v.ndim - 1))[:N]
+    large = P.QWeight(Q8_0, K, N, stretch(small.data.view(part, -1)).reshape(-1))
+    b = _dev(P, rng.normal(0, 1, part).astype(np.float32))
+    x = _dev(P, rng.normal(0, 1, (8, K)).astype(np.float32))
+    same = lambda got, want: all(torch.equal(g, stretch(w)) for g, w in zip(got, want))
+    for n in (1, 3, 8):
+        assert same(P.mul_mat_vec(large, x=x[:n], bias=stretch(b)), P.mul_mat_vec(small, x=x[:n], bias=b)), n
+    assert same(P.mul_mat_vec(large, x=x[:1], w2=large), P.mul_mat_vec(small, x=x[:1], w2=small))
+    got, beside = P.mul_mat_vec_fused([large, small], x[0])
+    want = P.mul_mat_vec_fused([small], x[0])[0]
+    assert torch.equal(got, stretch(want)) and torch.equal(beside, want)
+
+
 @pytest.mark.parametrize("C", [2, 3, 4, 5, 7, 8])       # column slots per launch group (mmvq_cols.hip): 2, 4 (one idle), 4, 4+1, 4+4 (one idle), 8; pairs: 2 per launch
 @pytest.mark.parametrize("t", QUANT_TYPES)
 def test_gemv_epilogues_and_columns(P, oracle, t, C):

@@ -611,3 +611,27 @@ for cols in (1, 2, 4, 8):
     assert grids(4096, 1024, cols) == grids(8192, 4096, cols) == [256]
 print("ok")
 """)
+
+
+def test_mat_vecs_of_many_rows_are_launched_in_pieces(run):
+    """33 million rows and more: a launch of more than 65536 workgroups would find its slices with more than 32 bits. One matrix, one column and several, and a fused launch"""
+    run(COMMON + r"""
+lib = C.CDLL(sys.argv[2])
+f = lib.pm355_mul_mat_vec_q
+f.argtypes = [C.c_int, C.c_void_p, C.c_void_p, C.c_int64, C.c_int64, C.c_void_p, C.c_int, C.c_void_p, C.c_int64, C.c_void_p, C.c_void_p, C.c_void_p]
+at = C.addressof(C.create_string_buffer(256))
+grids = lambda: [g for _, _, g in launches()]
+for N, pieces in ((33357824, 1), (33357825, 2), (34000001, 3), ((1 << 31) - 1, 128)):
+    for cols in (1, 2, 4, 8):
+        shim.shim_forget()
+        rc = f(8, at, None, 32, N, at, cols, at, N, at, None, 1)
+        got = grids()
+        assert rc == 0 and len(got) == pieces and all(g[0] <= 65536 for g in got), (N, cols, rc, len(got), got[:4])
+class Job(C.Structure):
+    _fields_ = [("type", C.c_int32), ("pad", C.c_int32), ("N", C.c_int64), ("W", C.c_void_p), ("W2", C.c_void_p), ("y", C.c_void_p), ("bias", C.c_void_p), ("resid", C.c_void_p)]
+jobs = (Job * 2)(Job(12, 0, 34000001, at, None, at, None, None), Job(12, 0, 77, at, None, at, None, None))
+shim.shim_forget()
+assert lib.pm355_mul_mat_vec_fused(jobs, 2, C.c_int64(256), C.c_void_p(at), None, C.c_float(0), C.c_void_p(1)) == 0
+assert len(grids()) == 4 and all(g[0] <= 65536 for g in grids()), grids()
+print("ok")
+""")
