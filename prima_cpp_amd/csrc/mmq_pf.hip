@@ -490,7 +490,8 @@ template <int TYPE, int NT, bool EX> constexpr size_t mid_lds_bytes() { return (
 // and 12 registers spilled 68
 // PF_SELF (a bit of EXP): or where a loader's requests are the longer part of a step - Q8_0, four pieces of 1 KiB to a row group and 128 k, up to 64 tokens, where half of the chip is idle anyway: less
 // than 128 workgroups. us at 64 tokens, four loaders / none: 1024 x 512 10.8 / 10.0, 1024 x 1024 14.3 / 13.4, 2048 x 3072 16.8 / 16.0, 512 x 8192 18.9 / 18.1; from 128 workgroups on 6144 x 4096 20.2 /
-// 20.4, 8192 x 8192 29.7 / 30.4. (K = 512 of the other types, 4 steps: 64 tokens 10.3 / 10.0, 128 12.6 / 12.0, from K = 1024 on 0.92-1.00)
+// 20.4, 8192 x 8192 29.7 / 30.4. Or where a launch is four steps, K = 512 of the other types at 97..128 tokens: us at 128 tokens, four loaders / none, Q4_K 256 rows 11.7 / 11.2, 32768 rows 14.0 / 13.6, Q5_K
+// 4096 rows 12.4 / 12.3, Q6_K 12.6 / 12.1; at 33..64 tokens 0.98-1.00, 1.01-1.05 and 1.00-1.05 of the time, and from K = 1024 on loaders win
 constexpr int PF_SELF = 512;
 template <int TA, int TB, int NT, bool EX, int EXP = 0> constexpr bool mid_self() { return (EXP & PF_SELF) || (EX && (NT == 4 || TA != TB || TA == PM_Q5_K)); }
 template <int N> __device__ __forceinline__ void mid_wait() { asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" : : "n"(N) : "memory"); }
@@ -1303,7 +1304,7 @@ static int launch_pf(const pm_gemm_pf_job * jobs, int njobs, const void * xh, co
         if (!p.ws) return -3;
     }
     const int slots = full + split_slots * S;
-    const bool few = mid && !wide && ta == PM_Q8_0 && nt == 2 && (long) tiles * pl.nt_t * S < 128;      // (PF_SELF)
+    const bool few = mid && !wide && (ta == PM_Q8_0 ? nt == 2 && (long) tiles * pl.nt_t * S < 128 : nt == 4 && K <= 512);      // (PF_SELF)
     const bool self = wide ? nt == 4 || ta != tb || ta == PM_Q5_K : few;                                  // (mid_self of the kernel below)
     auto go = [&](auto kern, size_t lds) {
         pf_allow_lds((const void *) kern, lds);
@@ -1362,7 +1363,8 @@ static int launch_pf(const pm_gemm_pf_job * jobs, int njobs, const void * xh, co
             else if (nt == 2) go(gemm_pf_kernel<A, B, 2, true, 0, A != PM_Q8_0>, pf_lds_bytes<A, B, 2, true, A != PM_Q8_0>()); \
             else return -2; \
         } else if (mid) { \
-            if (nt == 4)      go(gemm_pf_kernel<A, B, 4, true>, pf_lds_bytes<A, B, 4, true>()); \
+            constexpr int OWN4 = A == PM_Q8_0 ? 0 : PF_SELF; \
+            if (nt == 4)      { if (few) go(gemm_pf_kernel<A, B, 4, true, OWN4>, pf_lds_bytes<A, B, 4, true>()); else go(gemm_pf_kernel<A, B, 4, true>, pf_lds_bytes<A, B, 4, true>()); } \
             else if (nt == 3) go(gemm_pf_kernel<A, B, 3, true>, pf_lds_bytes<A, B, 3, true>()); \
             else if (nt == 2) { if (few) go(gemm_pf_kernel<PM_Q8_0, PM_Q8_0, 2, true, PF_SELF>, pf_lds_bytes<PM_Q8_0, PM_Q8_0, 2, true>()); else go(gemm_pf_kernel<A, B, 2, true>, pf_lds_bytes<A, B, 2, true>()); } \
             else return -2; \

@@ -1089,6 +1089,21 @@ def test_prompt_products_of_few_q8_0_rows(P, oracle, K):
     assert np.linalg.norm(y - exact) < 1e-3 * np.linalg.norm(exact)      # (a weight is rounded to F16 once: 2^-11 at most)
 
 
+@pytest.mark.parametrize("types", [(Q4_K, Q6_K), (Q4_K, Q5_K), (Q5_K, Q6_K), (Q4_K,), (Q5_K,), (Q6_K,)])
+def test_prompt_products_of_four_steps(P, types):
+    """K = 512, 97..128 tokens: the kernel without loaders, the bits of the one with them (the first 96 tokens, tiles of 96), one type and two in a launch; one row tile, several, and the most"""
+    K, rng = 512, np.random.default_rng(sum(types))
+    x = _dev(P, rng.normal(0, 1, (128, K)).astype(np.float32))
+    for N in (4, 132, 16384):
+        ws = [P.upload_weight(t, rand_blocks(t, N, K, rng), K, N) for t in types]
+        run = lambda a: P.mul_mat_mfma_multi(ws, a) if len(ws) > 1 else [P.mul_mat_mfma(ws[0], a)]
+        want = run(x[:96].contiguous())
+        late = run(x[32:].contiguous())
+        for T in (97, 128):
+            for a, b, c in zip(run(x[:T].contiguous()), want, late):
+                assert P.torch.equal(a[:96], b) and P.torch.equal(a[32:], c[:T - 32]), (N, T)
+
+
 @pytest.mark.parametrize("t", [Q4_K, Q5_K, Q6_K])
 @pytest.mark.parametrize("K,N,T", [(1024, 384, 200), (2048, 132, 64), (512, 256, 257), (8192, 132, 200)])
 def test_prompt_gemm_pair_tiles_silu_gate_times_up(P, oracle, t, K, N, T):

@@ -550,7 +550,7 @@ for t in (12, 13, 14, 8):
                     small, large = (-(-N // 64), -(-N // 128)) if pair else (-(-N // 128), -(-N // 256))
                     assert mid == (T <= 128 and small <= 256), (t, K, N, T, pair)
                     assert got == plan(small if mid else large, K, T, 4 if mid else 2), (t, K, N, T, pair, got)
-                    own = mid and t == 8 and T <= 64 and got[1] < 128    # (few workgroups of Q8_0: no loaders)
+                    own = mid and (T <= 64 and got[1] < 128 if t == 8 else K == 512 and T > 96)    # (few workgroups of Q8_0, four steps: no loaders)
                     assert any("gemm_pf_kernel" in n and ", 512, " in n for _, n, _ in launches()) == own, (t, K, N, T, pair)
                     cut = got[0] == 8 and (T - 1) % 256 < 192       # (the last tile of 256 tokens: the kernel that multiplies what is left of it)
                     assert any("gemm_pf_kernel" in n and ", 256, " in n for _, n, _ in launches()) == cut, (t, K, N, T, pair)
