@@ -928,7 +928,8 @@ __device__ __forceinline__ void mid_body(const PfP & p, const PfJob & jb, const 
 // PF_CUT (a bit of EXP): the batch's last tile of 256 tokens multiplies the 128 or 192 that are left of it only. us, whole / cut: wo of the 8B shape 640 tokens 50.5 / 47.4, 1400 76.8 / 75.7, 2100 113 / 114
 // (in tiles of 192 93), its Q6_K ffn_down 640 114 / 107, 1400 229 / 218, ffn_gate | ffn_up 640 189 / 181, 1800 478 / 471, Q8_0 ffn_down of 72B 640 374 / 345. (Tiles of 192 with a cut last one: wo 2400
 // 105 / 110, wq | wk | wv 6001 360 / 379.) A kernel of its own: with the two smaller bodies beside it a launch that cuts nothing took 0.2-0.9 us more (200 tokens of 1024 x 1024 34.2 -> 34.8, Q8_0
-// 33.8 -> 34.8; now 33.6, 33.7)
+// 33.8 -> 34.8; now 33.6, 33.7). The kernel that cuts nothing has no such choice in its source either: with one of a single body the compiler laid its blocks out otherwise, Q8_0 256 tokens of 512 values
+// x 4096 rows 26.9 -> 27.4, of 1024 x 16384 39.0 -> 40.4
 constexpr int PF_CUT = 256;
 template <int TA, int TB, int NT, bool MID = false, int EXP = 0, bool EX = false>
 __global__ __launch_bounds__((MID && !mid_self<TA, TB, NT, EX, EXP>() ? MID_NTHR : PF_NTHR)) void gemm_pf_kernel(PfP p) {
@@ -957,18 +958,20 @@ __global__ __launch_bounds__((MID && !mid_self<TA, TB, NT, EX, EXP>() ? MID_NTHR
     }
     const int t0 = tile_t * 32 * NT;
     const int tile_id = (slot - p.full) * 8 + x;                 // (split tiles only: slab index)
-    if constexpr (!MID) {
+    if constexpr (!MID && (EXP & PF_CUT)) {
+        static_assert(NT == 8, "tiles of 256 tokens");
         auto body = [&](auto nt) __attribute__((always_inline)) {
             constexpr int N = decltype(nt)::value;
             if (TA == TB || jb.type == TA) pf_body<TA, N, EXP & 255, NT>(p, jb, n0, t0, pf_smem, role, ks, S, tile_id);
             else pf_body<TB, N, EXP & 255, NT>(p, jb, n0, t0, pf_smem, role, ks, S, tile_id);
         };
-        constexpr bool CUT = (EXP & PF_CUT) != 0;
-        static_assert(!CUT || NT == 8, "tiles of 256 tokens");
         const int left = p.T - t0;
-        if (CUT && left <= 128) body(std::integral_constant<int, CUT ? 4 : NT>());
-        else if (CUT && left <= 192) body(std::integral_constant<int, CUT ? 6 : NT>());
-        else body(std::integral_constant<int, NT>());
+        if (left <= 128) body(std::integral_constant<int, 4>());
+        else if (left <= 192) body(std::integral_constant<int, 6>());
+        else body(std::integral_constant<int, 8>());
+    } else if constexpr (!MID) {
+        if (TA == TB || jb.type == TA) pf_body<TA, NT, EXP, NT>(p, jb, n0, t0, pf_smem, role, ks, S, tile_id);
+        else pf_body<TB, NT, EXP, NT>(p, jb, n0, t0, pf_smem, role, ks, S, tile_id);
     } else {
         constexpr bool SELF = mid_self<TA, TB, NT, EX, EXP>();
         if (TA == TB || jb.type == TA) mid_body<TA, NT, EX, SELF>(p, jb, n0, t0, pf_smem, role, ks, S, tile_id);
