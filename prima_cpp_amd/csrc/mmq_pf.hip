@@ -1234,17 +1234,18 @@ void pm_gemm_pf_plan(const pm_gemm_pf_ask & ask, pm_gemm_pf_plan_t * out) {
     // 33 products of 257..384 tokens and more than a round 0.73-0.97, one 1.01. As much work in more tiles, not taken: 5120 x 13824 pairs 1344 tokens 421 / 450, 8192 x 29568 2112 1871 / 1809
     if (ask.form == PM_PF_ROWS_256 && !ask.splitk && out->nt == 8) {
         const int s6 = out->full ? 1 : out->splitk;
-        // workgroups / CUs, rounds and work in them, in sub-tiles of 32 tokens + 1
-        struct Cost { double rounds, work; };
+        // rounds of workgroups and work in them, in sub-tiles of 32 tokens + 1; the rounds are those of the XCD with the most row tiles. Counted over the chip, launches whose row tiles do not
+        // divide by eight took a round more than with tiles of 256. us, 256 / 192: 1024 rows of 8192, 777 tokens 53 / 62, 2304 of 4096, 4096 tokens 135 / 172, 4352 of 4096, 2100 tokens 115 / 166
+        struct Cost { double rounds, work; bool one; };
         const auto cost = [&](int nt) {
             const int n = (T - 1) / (32 * nt), left = T - 32 * nt * n, last = nt == 6 || !n ? nt : left <= 128 ? 4 : left <= 192 ? 6 : 8;
-            const double w = (double) tiles * s6 / cus;
-            return Cost{std::ceil(w * (n + 1)) * (nt + 1), w * (n * (nt + 1) + last + 1)};
+            const double w = (double) tiles * s6 / cus, x = (double) ((tiles + 7) / 8) * s6 / (cus / 8);
+            return Cost{std::ceil(x * (n + 1)) * (nt + 1), w * (n * (nt + 1) + last + 1), w * (n + 1) <= 1.0};
         };
         const Cost c6 = cost(6);
         Cost c8 = cost(8);
-        if (out->full) c8.rounds = c8.work = 9.0 * out->cost / nb;
-        const double most = c8.rounds <= 9.0 ? 1.1 : !out->full && (T + 191) / 192 == out->nt_t ? 1.001 : 0.97;
+        if (out->full) { c8.rounds = c8.work = 9.0 * out->cost / nb; c8.one = false; }
+        const double most = c8.one ? 1.1 : !out->full && (T + 191) / 192 == out->nt_t ? 1.001 : 0.97;
         if (c6.rounds < 0.97 * c8.rounds && c6.work < most * c8.work) plan_tiles(tiles, K, T, cus, 6, s6, 0, out);
     }
 }

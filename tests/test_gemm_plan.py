@@ -108,9 +108,11 @@ def every_slice_once(tiles, p):
     (112, 4096, 129, 192), (112, 4096, 192, 192), (112, 4096, 193, 256), (112, 4096, 300, 192), (112, 4096, 384, 192), (112, 4096, 385, 256), (112, 4096, 512, 256),      # ffn_gate | ffn_up of the 8B shape
     (112, 4096, 128, 128), (112, 4096, 64, 64), (112, 4096, 6001, 256), (224, 8192, 513, 192), (224, 8192, 576, 192), (224, 8192, 577, 256),
     (224, 8192, 256, 256), (224, 8192, 257, 192), (224, 8192, 384, 192), (224, 8192, 385, 256), (231, 8192, 300, 192), (501, 4096, 320, 192), (501, 4096, 1300, 256), (108, 5120, 1344, 256), (32, 29568, 513, 192),
-    (24, 4096, 150, 192), (24, 4096, 1500, 192), (24, 4096, 6001, 192), (16, 4096, 3000, 192), (16, 4096, 6001, 192), (16, 14336, 380, 192), (17, 2048, 4096, 192), (5, 1024, 300, 192)])
+    (24, 4096, 150, 192), (24, 4096, 1500, 192), (24, 4096, 6001, 192), (16, 4096, 3000, 192), (16, 4096, 6001, 192), (16, 14336, 380, 192), (17, 2048, 4096, 256), (5, 1024, 300, 192),
+    (4, 8192, 777, 256), (4, 8192, 1100, 192), (9, 4096, 4096, 256), (9, 4096, 300, 192), (17, 4096, 2100, 256), (25, 4096, 777, 256), (50, 8192, 777, 256), (8, 8192, 777, 256)])
 def test_tiles_of_256_rows_as_launched(tiles, K, T, tile):
-    """tiles of 192 tokens beside those of 256, on either side of where they change; the K split stays that of 256 tokens, a split of the last tiles only goes; no tile or slice is left out"""
+    """tiles of 192 tokens beside those of 256, on either side of where they change; the K split stays that of 256 tokens, a split of the last tiles only goes; no tile or slice is left out. Where row
+    tiles do not divide by eight, the XCDs that own one more decide"""
     p, by_tokens = plan(tiles, K, T, ROWS_256), plan(tiles, K, T)
     assert p["tile_tokens"] == tile and p["nt_t"] == -(-T // tile) and every_slice_once(tiles, p)
     if tile != 192:
@@ -131,7 +133,7 @@ def test_tiles_of_192_tokens_over_many_sizes():
                     assert p == q
                     continue
                 taken += 1
-                rounds = lambda x, tile: -(-tiles * x["nt_t"] * x["S"] // CUS) * (tile // 32 + 1)  # noqa: E731
+                rounds = lambda x, tile: -(-(-(-tiles // 8)) * x["nt_t"] * x["S"] // (CUS // 8)) * (tile // 32 + 1)  # noqa: E731      (of the XCD with the most row tiles)
                 assert p["tile_tokens"] == 192 and (q["full"] or rounds(p, 192) < rounds(q, 256)), (tiles, K, T, p, q)
     assert taken > 100
 
