@@ -928,7 +928,7 @@ __device__ __forceinline__ void mid_body(const PfP & p, const PfJob & jb, const 
 // PF_CUT (a bit of EXP): the batch's last tile of 256 tokens multiplies the 128 or 192 that are left of it only. us, whole / cut: wo of the 8B shape 640 tokens 50.5 / 47.4, 1400 76.8 / 75.7, 2100 113 / 114
 // (in tiles of 192 93), its Q6_K ffn_down 640 114 / 107, 1400 229 / 218, ffn_gate | ffn_up 640 189 / 181, 1800 478 / 471, Q8_0 ffn_down of 72B 640 374 / 345. (Tiles of 192 with a cut last one: wo 2400
 // 105 / 110, wq | wk | wv 6001 360 / 379.) A kernel of its own: with the two smaller bodies beside it a launch that cuts nothing took 0.2-0.9 us more (200 tokens of 1024 x 1024 34.2 -> 34.8, Q8_0
-// 33.8 -> 34.8; now 33.6, 33.7). The kernel that cuts nothing has no such choice in its source either: with one of a single body the compiler laid its blocks out otherwise, Q8_0 256 tokens of 512 values
+// 33.8 -> 34.8; now 33.6, 33.7). Where it is taken: cut_pays. The kernel that cuts nothing has no such choice in its source either: with one of a single body the compiler laid its blocks out otherwise, Q8_0 256 tokens of 512 values
 // x 4096 rows 26.9 -> 27.4, of 1024 x 16384 39.0 -> 40.4
 constexpr int PF_CUT = 256;
 template <int TA, int TB, int NT, bool MID = false, int EXP = 0, bool EX = false>
@@ -1214,6 +1214,14 @@ static void plan_tiles(int tiles, int K, int T, int cus, int nt, int force_s, in
     if (force_s >= 1 && force_s <= 8 && nb / force_s >= 1) { S = force_s; full = 0; }
     out->nt = nt; out->nt_t = nt_t; out->splitk = S; out->full = full; out->grid = 8 * (full + (maxL - full) * S); out->cost = best;
 }
+// Does a launch whose last tile of 256 tokens is cut gain by it? It saves that tile's part of the steps; what it costs is the same for any K, some 7 us a round of workgroups: two loops of tens of KB
+// side by side do not fit the instruction cache that two CUs share. us, whole / cut, by K x sub-tiles saved of 9 / token tiles: 19 (25600 rows of 1024, 3000 tokens) 260 / 294, 76 (8448 of 4096, 3000)
+// 243 / 254, 114 (16384 of 1024, 777) 57.0 / 56.5, 152 (8448 of 2048, 1400) 78 / 81, 202 (2100 tokens, 14336 of 4096) 281 / 285, (12800) 261 / 267, 228 (16384 of 2048, 400) 62 / 58, (14336 of 4096, 900)
+// 131 / 131, 303 (14336 of 4096, 1400) 206 / 203, 364 (1100) 178 / 172. Where every tile is split along K a cut one has smaller slabs too: 0.89-1.01
+static bool cut_pays(int K, int T, int S, int full) {
+    const int n = (T + 255) / 256, left = T - 256 * (n - 1), saved = left <= 128 ? 4 : left <= 192 ? 2 : 0;
+    return saved && (n == 1 || (S > 1 && !full) || (long) saved * K > 215L * 9 * n);
+}
 void pm_gemm_pf_plan(const pm_gemm_pf_ask & ask, pm_gemm_pf_plan_t * out) {
     const int tiles = ask.tiles, K = ask.K, T = ask.T, cus = ask.cus, nb = (K + 255) / 256;
     const bool mid = ask.form == PM_PF_ROWS_128, wide = ask.form == PM_PF_WIDE;
@@ -1238,7 +1246,7 @@ void pm_gemm_pf_plan(const pm_gemm_pf_ask & ask, pm_gemm_pf_plan_t * out) {
         // divide by eight took a round more than with tiles of 256. us, 256 / 192: 1024 rows of 8192, 777 tokens 53 / 62, 2304 of 4096, 4096 tokens 135 / 172, 4352 of 4096, 2100 tokens 115 / 166
         struct Cost { double rounds, work; bool one; };
         const auto cost = [&](int nt) {
-            const int n = (T - 1) / (32 * nt), left = T - 32 * nt * n, last = nt == 6 || !n ? nt : left <= 128 ? 4 : left <= 192 ? 6 : 8;
+            const int n = (T - 1) / (32 * nt), left = T - 32 * nt * n, last = nt == 6 || !n || !cut_pays(K, T, s6, out->full) ? nt : left <= 128 ? 4 : 6;
             const double w = (double) tiles * s6 / cus, x = (double) ((tiles + 7) / 8) * s6 / (cus / 8);
             return Cost{std::ceil(x * (n + 1)) * (nt + 1), w * (n * (nt + 1) + last + 1), w * (n + 1) <= 1.0};
         };
@@ -1358,7 +1366,7 @@ static int launch_pf(const pm_gemm_pf_job * jobs, int njobs, const void * xh, co
         return 0;
     }
 #endif
-    const bool cut = T - 256 * (pl.nt_t - 1) <= 192;            // (of tiles of 256 tokens: the last one)
+    const bool cut = nt == 8 && cut_pays(K, T, S, full);
     // (an nt that no kernel has stays an error)
 #define PF_GO(A, B) do { \
         if (wide) { \

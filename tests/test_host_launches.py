@@ -532,11 +532,14 @@ lib.pm355_mul_mat_q_wide.argtypes = [C.c_void_p, C.c_int] + [C.c_void_p] * 6 + [
 def plan(tiles, K, T, flags):
     out = (C.c_int32 * 5)()
     assert lib.pm355_gemm_plan(tiles, K, T, 256, flags, out) == 0
+    global split
+    split = out[2], out[3]
     return out[0] // 32, out[4]
 def launched():
     (n, g), = [(n, g) for _, n, g in launches() if "gemm_pf_kernel" in n]
     a = re.search(r"gemm_pf_kernel<(.*?)>", n).group(1).split(", ")
     return (int(a[2]), g[0]), a[3] == "true"
+seen = set()
 for t in (12, 13, 14, 8):
     for K in (512, 4096, 14336):
         for N in (132, 1024, 4096, 14336, 40960):
@@ -552,8 +555,12 @@ for t in (12, 13, 14, 8):
                     assert got == plan(small if mid else large, K, T, 4 if mid else 2), (t, K, N, T, pair, got)
                     own = mid and (T <= 64 and got[1] < 128 if t == 8 else K == 512 and T > 96)    # (few workgroups of Q8_0, four steps: no loaders)
                     assert any("gemm_pf_kernel" in n and ", 512, " in n for _, n, _ in launches()) == own, (t, K, N, T, pair)
-                    cut = got[0] == 8 and (T - 1) % 256 < 192       # (the last tile of 256 tokens: the kernel that multiplies what is left of it)
+                    tiles, left = -(-T // 256), (T - 1) % 256 + 1            # (the last tile of 256 tokens: the kernel that multiplies what is left of it, where that is enough or every tile is split)
+                    saved = 4 if left <= 128 else 2 if left <= 192 else 0
+                    cut = got[0] == 8 and saved > 0 and ((split[0] > 1 and not split[1]) or saved * K > 215 * 9 * tiles)
+                    seen.add((got[0], cut))
                     assert any("gemm_pf_kernel" in n and ", 256, " in n for _, n, _ in launches()) == cut, (t, K, N, T, pair)
+assert seen >= {(8, False), (8, True), (6, False)}
 arr = lambda v, ty: (ty * len(v))(*v)
 for types, Ns, K in (([12], [4096], 4096), ([12, 12], [1024, 14336], 4096), ([12, 14], [4096, 1024], 4096), ([14], [4096], 14336), ([13], [132], 512)):
     for T in (33, 64, 65, 96, 97, 128, 129, 147, 192, 231, 288, 289, 512):
