@@ -1231,7 +1231,10 @@ void pm_gemm_pf_plan(const pm_gemm_pf_ask & ask, pm_gemm_pf_plan_t * out) {
     // 8-bit activations of Q4_K: tiles of 96 tokens (with loaders) where they cost less than those of 128 (without: no registers left for them), by rounds of workgroups; the K split stays that of
     // 128 tokens: the sums in one order. 8B shape, whole passes, us, 128 / 96: 79 tokens 716 / 675, 109 738 / 801, 147 935 / 858, 231 1025 / 1095, 316 1279 / 1260, 459 1498 / 1570
     if (wide && T > 64 && !out->full && (T + 95) / 96 * 96 <= ask.ldt) {
-        const auto cost = [&](int nt) { return ((long) tiles * ((T + 32 * nt - 1) / (32 * nt)) * out->splitk + cus - 1) / cus * (nt + 1); };
+        // (rounds of the XCD with the most row tiles. Counted over the chip: 83 row tiles of 2048 values, 231 tokens 31.6 / 45.2, 18 of 4096 27.6 / 36.1, 99 of 8192, 385 tokens 190 / 210 - and 128 where 96 are
+        // faster: 84 of 8192, 300 tokens 186 / 141)
+        const int cpx = cus / 8;
+        const auto cost = [&](int nt) { return ((long) ((tiles + 7) / 8) * ((T + 32 * nt - 1) / (32 * nt)) * out->splitk + cpx - 1) / cpx * (nt + 1); };
         if (cost(3) < cost(4)) plan_tiles(tiles, K, T, cus, 3, out->splitk, 0, out);
     }
     // Tiles of 192 tokens where their rounds of workgroups cost less than those of 256: mostly 129..192, 257..384 and 513..576 tokens, whose rest of a tile of 256 was products of nothing. The K

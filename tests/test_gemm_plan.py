@@ -140,9 +140,10 @@ def test_tiles_of_192_tokens_over_many_sizes():
 
 @pytest.mark.parametrize("tiles,K,T,flags,tile", [(32, 4096, 64, ROWS_128, 64), (32, 4096, 65, ROWS_128, 96), (32, 14336, 96, ROWS_128, 96), (32, 4096, 97, ROWS_128, 128), (224, 4096, 128, ROWS_128, 128),
                                                   (32, 4096, 40, WIDE_Q4_K, 64), (224, 4096, 79, WIDE_Q4_K, 96), (224, 4096, 147, WIDE_Q4_K, 96), (224, 4096, 128, WIDE_Q4_K, 128), (32, 4096, 500, WIDE_Q4_K, 128),
+                                                  (83, 2048, 231, WIDE_Q4_K, 128), (18, 4096, 231, WIDE_Q4_K, 128), (99, 8192, 385, WIDE_Q4_K, 128), (84, 8192, 300, WIDE_Q4_K, 96), (11, 4096, 459, WIDE_Q4_K, 128),
                                                   (32, 14336, 40, WIDE, 64), (32, 14336, 147, WIDE, 64), (1, 512, 512, WIDE, 64)])
 def test_tiles_of_128_rows_as_launched(tiles, K, T, flags, tile):
-    """up to 128 tokens 64, 96 or 128 a tile; of 8-bit activations 96 beside 128 by rounds of workgroups, 64 with other types than Q4_K"""
+    """up to 128 tokens 64, 96 or 128 a tile; of 8-bit activations 96 beside 128 by rounds of workgroups (of the XCD with the most row tiles), 64 with other types than Q4_K"""
     p = plan(tiles, K, T, flags)
     assert p["tile_tokens"] == tile and p["nt_t"] == -(-T // tile) and every_slice_once(tiles, p), p
 
